@@ -209,6 +209,47 @@ int msd_conv_relu_backward_kb_static(int dtype, int ndim, int64_t batch, int64_t
                                      const void *input, const int64_t *input_strides,
                                      void *grad_kernel, void *grad_bias, void *stream);
 
+/* All gradients of one layer as a differentiated function of its own returns them: grad_input,
+ * grad_kernel and grad_bias (each may be NULL) are OVERWRITTEN, so the caller neither clears
+ * them nor are they read.  `relu` selects the mask of the conv_relu operators (`output` may be
+ * NULL without it); the workspace is msd_workspace_bytes'.  No counterpart in the reference,
+ * where an autograd function clears three buffers and calls three operators (conv2d.py:100-123). */
+int msd_conv_layer_backward(int relu, int dtype, int ndim, int64_t batch, int64_t c_in, int64_t c_out,
+                            const int64_t *spatial, int dilation,
+                            const void *output, const int64_t *output_strides,
+                            const void *grad_output, const int64_t *grad_output_strides,
+                            const void *input, const int64_t *input_strides, const void *kernel,
+                            void *grad_input, const int64_t *grad_input_strides,
+                            void *grad_kernel, void *grad_bias,
+                            void *workspace, int64_t workspace_bytes, void *stream);
+
+/* One update of Adam (no weight decay) for n contiguous parameters of one type.  With
+ * device_step the count of updates is read from there and incremented (a float on the device,
+ * as torch's capturable form keeps it), otherwise `step` is the count that this update makes.
+ * The reference leaves the optimiser to torch (msd_model.py:118-121). */
+typedef struct msd_adam_param {
+    void *param;
+    const void *grad;
+    void *exp_avg, *exp_avg_sq;
+    float *device_step;
+    double step;
+    int64_t count;
+} msd_adam_param;
+int msd_adam_step(int dtype, int n, const msd_adam_param *params, double lr, double beta1, double beta2, double eps,
+                  void *stream);
+
+/* A frozen c_out x c_out scaling S (+ shift) behind a 1x1 layer W, b: folded_weight = S W and
+ * folded_bias = S b + shift.  With shift == NULL the transposed product S^T W, S^T b, which
+ * takes gradients of the folded layer back to those of W and b.  No counterpart in the reference. */
+int msd_scale_fold(int dtype, int64_t c_out, int64_t c_in, const void *scale, const void *shift, const void *weight,
+                   const void *bias, void *folded_weight, void *folded_bias, void *stream);
+
+/* Labels on the device, checked without waiting for it: clamped = labels limited to
+ * [0, num_labels), range[0] = min(range[0], labels), range[1] = max(range[1], labels).
+ * The reference checks on the host (msd_segmentation_model.py:105-119). */
+int msd_label_check(int64_t count, int64_t num_labels, const int64_t *labels, int64_t *clamped, int64_t *range,
+                    void *stream);
+
 /* msd_conv_backward_k and msd_conv_backward_bias in one pass (no ReLU mask).
  * grad_bias may be NULL.  No counterpart in the reference. */
 int msd_conv_backward_kb(int dtype, int ndim, int64_t batch, int64_t c_in, int64_t c_out,

@@ -45,6 +45,11 @@ PROTOTYPES = {
     "msd_conv_relu_backward_kb_static": (_c_int, _HEAD + _VIEW + _VIEW + _VIEW + [_ptr, _ptr, _ptr]),
     "msd_conv_backward_kb": (_c_int, _HEAD + _VIEW + _VIEW + [_ptr, _ptr] + _WS + [_ptr]),
     "msd_conv_backward_xkb": (_c_int, _HEAD + _VIEW + _VIEW + [_ptr] + _VIEW + [_ptr, _ptr] + _WS + [_ptr]),
+    "msd_conv_layer_backward": (_c_int, [_c_int] + _HEAD + _VIEW + _VIEW + _VIEW + [_ptr] + _VIEW + [_ptr, _ptr] + _WS
+                                + [_ptr]),
+    "msd_adam_step": (_c_int, [_c_int, _c_int, _ptr] + [ctypes.c_double] * 4 + [_ptr]),
+    "msd_scale_fold": (_c_int, [_c_int, _c_i64, _c_i64] + [_ptr] * 7),
+    "msd_label_check": (_c_int, [_c_i64, _c_i64] + [_ptr] * 4),
     "msd_relu_mask_gradient": (_c_int, [_c_int, _c_int, _c_i64, _c_i64, _i64p] + _VIEW + _VIEW + [_ptr]),
     "msd_block_workspace_bytes": (_c_i64, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p]),
     "msd_block_forward": (_c_int, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p, _i64p] + _VIEW
@@ -85,6 +90,21 @@ def load():
         raise ImportError(f"{LIB_PATH}: ABI version {lib.msd_abi_version()}, expected {ABI_VERSION}")
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The C++ host path (``_msd_host``, csrc/host/msd_host.cpp) on top of the library.  Built
+    with it; missing, it is an ImportError like the library itself."""
+    global _host
+    if _host is None:
+        from . import _msd_host
+        load()
+        _msd_host.bind(LIB_PATH)
+        _host = _msd_host
+    return _host
 
 
 def last_error():

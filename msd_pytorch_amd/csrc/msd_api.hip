@@ -177,6 +177,7 @@ int make_geom(const char *fn, int dtype, int ndim, int64_t batch, int64_t c_in, 
     }
     g->ndim = ndim;
     g->reverse = 0;
+    g->fresh = 0;
     g->B = (int)batch;
     g->C = (int)c_in;
     g->Wd = (int)c_out;
@@ -323,6 +324,7 @@ int backward_x_t(const char *fn, bool relu, const msd::Geom &g, int ndim, const 
                     msd::Geom g2;
                     msd::View<const float> o2, gy2;
                     group(co, &g2, &o2, &gy2);
+                    g2.fresh = g.fresh && co == 0;
                     e = msd::fast_backward_x(g2, relu, o2, gy2, (const float *)kernel + (int64_t)co * g.C * taps, gx,
                                              none, s);
                     if (e != hipSuccess) return hip_fail(fn, e);
@@ -355,7 +357,8 @@ int backward_x_t(const char *fn, bool relu, const msd::Geom &g, int ndim, const 
 int backward_x(const char *fn, bool relu, int dtype, int ndim, int64_t batch, int64_t c_in, int64_t c_out,
                const int64_t *spatial, int dilation, const void *output, const int64_t *os, const void *grad_output,
                const int64_t *gs, const void *kernel, void *grad_input, const int64_t *xs, void *stream,
-               int mask_from = 0, const void *act = nullptr, const int64_t *as = nullptr, bool *masked = nullptr)
+               int mask_from = 0, const void *act = nullptr, const int64_t *as = nullptr, bool *masked = nullptr,
+               bool fresh = false)
 {
     // act/as/mask_from: optional ReLU mask applied to grad_input channels >= mask_from on the
     // way out (dense block only); *masked reports whether the kernel that ran did it.
@@ -363,6 +366,7 @@ int backward_x(const char *fn, bool relu, int dtype, int ndim, int64_t batch, in
     MSD_TRY(make_geom(fn, dtype, ndim, batch, c_in, c_out, spatial, dilation, true, &g));
     if (c_in <= 0) return fail(MSD_ERR_INVALID, "%s: c_in must be positive", fn);
     if (masked) *masked = false;
+    g.fresh = fresh;
     return dtype == MSD_F32 ? backward_x_t<float>(fn, relu, g, ndim, output, os, grad_output, gs, kernel, grad_input,
                                                   xs, (hipStream_t)stream, mask_from, act, as, masked)
                             : backward_x_t<double>(fn, relu, g, ndim, output, os, grad_output, gs, kernel, grad_input,
@@ -396,12 +400,13 @@ int backward_kb_t(const char *fn, bool relu, const msd::Geom &g, int ndim, const
 int backward_kb(const char *fn, bool relu, bool need_k, int dtype, int ndim, int64_t batch, int64_t c_in,
                 int64_t c_out, const int64_t *spatial, int dilation, const void *output, const int64_t *os,
                 const void *grad_output, const int64_t *gs, const void *input, const int64_t *xs, void *grad_kernel,
-                void *grad_bias, void *ws, int64_t ws_bytes, void *stream)
+                void *grad_bias, void *ws, int64_t ws_bytes, void *stream, bool fresh = false)
 {
     msd::Geom g;
     MSD_TRY(make_geom(fn, dtype, ndim, batch, c_in, c_out, spatial, dilation, need_k, &g));
     if (need_k && c_in <= 0) return fail(MSD_ERR_INVALID, "%s: c_in must be positive", fn);
     if (need_k && !grad_kernel) return fail(MSD_ERR_INVALID, "%s: grad_kernel is NULL", fn);
+    g.fresh = fresh;
     return dtype == MSD_F32 ? backward_kb_t<float>(fn, relu, g, ndim, output, os, grad_output, gs, input, xs,
                                                    grad_kernel, grad_bias, ws, ws_bytes, (hipStream_t)stream)
                             : backward_kb_t<double>(fn, relu, g, ndim, output, os, grad_output, gs, input, xs,
@@ -596,6 +601,66 @@ int msd_conv_relu_backward_kb(int dtype, int ndim, int64_t batch, int64_t c_in, 
                        workspace, workspace_bytes, stream);
 }
 
+
+int msd_conv_layer_backward(int relu, int dtype, int ndim, int64_t batch, int64_t c_in, int64_t c_out,
+                            const int64_t *spatial, int dilation, const void *output, const int64_t *output_strides,
+                            const void *grad_output, const int64_t *grad_output_strides, const void *input,
+                            const int64_t *input_strides, const void *kernel, void *grad_input,
+                            const int64_t *grad_input_strides, void *grad_kernel, void *grad_bias, void *workspace,
+                            int64_t workspace_bytes, void *stream)
+{
+    const char *fn = "conv_layer_backward";
+    if (!grad_input && !grad_kernel && !grad_bias) return fail(MSD_ERR_INVALID, "%s: no gradient buffer given", fn);
+    if (grad_input)
+        MSD_TRY(backward_x(fn, relu != 0, dtype, ndim, batch, c_in, c_out, spatial, dilation, output, output_strides,
+                           grad_output, grad_output_strides, kernel, grad_input, grad_input_strides, stream, 0, nullptr,
+                           nullptr, nullptr, true));
+    if (grad_kernel || grad_bias)
+        MSD_TRY(backward_kb(fn, relu != 0, grad_kernel != nullptr, dtype, ndim, batch, c_in, c_out, spatial, dilation,
+                            output, output_strides, grad_output, grad_output_strides, input, input_strides,
+                            grad_kernel, grad_bias, workspace, workspace_bytes, stream, true));
+    return MSD_OK;
+}
+
+// ---------------------------------------------------------------------------
+// What a training step does around the network: the optimiser, the frozen output scaling folded
+// into the final layer, the check of the labels (kernels in msd_step.hip).
+// ---------------------------------------------------------------------------
+
+int msd_adam_step(int dtype, int n, const msd_adam_param *params, double lr, double beta1, double beta2, double eps,
+                  void *stream)
+{
+    const char *fn = "adam_step";
+    if (dtype != MSD_F32 && dtype != MSD_F64) return fail(MSD_ERR_INVALID, "%s: dtype must be MSD_F32 or MSD_F64", fn);
+    if (n < 0 || (n > 0 && !params)) return fail(MSD_ERR_INVALID, "%s: no parameters given", fn);
+    for (int i = 0; i < n; i++)
+        if (params[i].count < 0 || !params[i].param || !params[i].grad || !params[i].exp_avg || !params[i].exp_avg_sq)
+            return fail(MSD_ERR_INVALID, "%s: parameter %d: NULL tensor or negative size", fn, i);
+    const hipError_t e = msd::adam_step(dtype == MSD_F64, n, params, lr, beta1, beta2, eps, (hipStream_t)stream);
+    return e == hipSuccess ? MSD_OK : hip_fail(fn, e);
+}
+
+int msd_scale_fold(int dtype, int64_t c_out, int64_t c_in, const void *scale, const void *shift, const void *weight,
+                   const void *bias, void *folded_weight, void *folded_bias, void *stream)
+{
+    const char *fn = "scale_fold";
+    if (dtype != MSD_F32 && dtype != MSD_F64) return fail(MSD_ERR_INVALID, "%s: dtype must be MSD_F32 or MSD_F64", fn);
+    if (c_out <= 0 || c_in <= 0 || c_out * c_in > INT32_MAX) return fail(MSD_ERR_INVALID, "%s: channel counts out of range", fn);
+    if (!scale || !weight || !bias || !folded_weight || !folded_bias) return fail(MSD_ERR_INVALID, "%s: NULL argument", fn);
+    const hipError_t e = msd::scale_fold(dtype == MSD_F64, (int)c_out, (int)c_in, scale, shift, weight, bias,
+                                         folded_weight, folded_bias, (hipStream_t)stream);
+    return e == hipSuccess ? MSD_OK : hip_fail(fn, e);
+}
+
+int msd_label_check(int64_t count, int64_t num_labels, const int64_t *labels, int64_t *clamped, int64_t *range,
+                    void *stream)
+{
+    const char *fn = "label_check";
+    if (count <= 0 || num_labels <= 0) return fail(MSD_ERR_INVALID, "%s: counts must be positive", fn);
+    if (!labels || !clamped || !range) return fail(MSD_ERR_INVALID, "%s: NULL argument", fn);
+    const hipError_t e = msd::label_check(count, num_labels, labels, clamped, range, (hipStream_t)stream);
+    return e == hipSuccess ? MSD_OK : hip_fail(fn, e);
+}
 
 // ---------------------------------------------------------------------------
 // msd_conv_relu_backward_kb for callers that cannot allocate: the partial sums go through

@@ -39,8 +39,16 @@ __device__ __forceinline__ void bwdx_rows_body(const Geom &g, const RowTeams &rt
     // behind the gather's (lanes outside the image ask for a valid address and drop the values)
     float *gp = gx.p + (int64_t)b * gx.sb + (int64_t)z * gx.sz + (int64_t)y * gx.sy + min(x0, g.W - V);
     float first[U][V];
+    auto load_old = [&](int ci, float (&v)[V]) {
+        if (g.fresh) {                           // uniform: nothing to add to
 #pragma unroll
-    for (int u = 0; u < U; u++) load_vec<V>(gp + (int64_t)min(c0 + u, c1 - 1) * gx.sc, first[u]);
+            for (int i = 0; i < V; i++) v[i] = 0.f;
+        } else {
+            load_vec<V>(gp + (int64_t)ci * gx.sc, v);
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < U; u++) load_old(min(c0 + u, c1 - 1), first[u]);
 
     // adjoint gather, kept in registers for the whole channel loop
     float A[WOUT][K][V];
@@ -72,7 +80,7 @@ __device__ __forceinline__ void bwdx_rows_body(const Geom &g, const RowTeams &rt
 #pragma unroll
                 for (int i = 0; i < V; i++) cur[u][i] = first[u][i];
             } else {
-                load_vec<V>(gp + (int64_t)cu[u] * gx.sc, cur[u]);
+                load_old(cu[u], cur[u]);
             }
         }
 #pragma unroll

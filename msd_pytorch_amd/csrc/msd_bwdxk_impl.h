@@ -949,7 +949,8 @@ hipError_t launch(const Geom &g, const View<const float> &gy, const View<const f
         return hipSuccess;
     }
     if (group) return reduce_columns_batch(&job, 1, s);   // (adds in the same order)
-    hipLaunchKernelGGL(bwdk::reduce_columns, dim3((ncols + 3) / 4), dim3(256), 0, s, part, rows, nk, ncols, gk, gb);
+    hipLaunchKernelGGL(bwdk::reduce_columns, dim3((ncols + 3) / 4), dim3(256), 0, s, part, rows, nk, ncols, gk, gb,
+                       g.fresh);
     return hipGetLastError();
 }
 

@@ -33,6 +33,8 @@ struct Geom {
     int nvox;           // D * H * W, checked on the host to fit in 31 bits
     int reverse;        // walk the input channels from the last to the first (same sums, other order);
                         // set by the dense block's layer loops for every second layer
+    int fresh;          // gradients overwrite their buffers instead of being added to them (a single
+                        // layer's backward pass: no zero fill before it, no read of the old values)
 };
 
 // Strided view: element strides {batch, channel, z, y, x}.

@@ -96,7 +96,7 @@ __global__ __launch_bounds__(kBlock) void bwdx_generic(Geom g, int cch, View<con
             T s = T(0);
 #pragma unroll
             for (int t = 0; t < K; t++) s += kc[t] * A[t];
-            gxp[(int64_t)ci * gx.sc] += s;
+            gxp[(int64_t)ci * gx.sc] = g.fresh && co == 0 ? s : gxp[(int64_t)ci * gx.sc] + s;
         }
     }
 }
@@ -187,16 +187,17 @@ __global__ __launch_bounds__(kBlock) void bwdk_generic_partial(Geom g, View<cons
     }
 }
 
-// dst[i] += sum over rows of part[row][first + i], rows in increasing order.
+// dst[i] += (fresh: =) sum over rows of part[row][first + i], rows in increasing order.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void reduce_partials(const T *__restrict__ part, int rows, int64_t nout,
-                                                          int64_t first, int64_t count, T *__restrict__ dst)
+                                                          int64_t first, int64_t count, T *__restrict__ dst,
+                                                          int fresh)
 {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= count) return;
     T s = T(0);
     for (int r = 0; r < rows; r++) s += part[(int64_t)r * nout + first + i];
-    dst[i] += s;
+    dst[i] = fresh ? s : dst[i] + s;
 }
 
 // gy = gy * [0 < out], in place, over batch * Wd * nvox elements.
@@ -270,11 +271,11 @@ hipError_t launch_bwdk(const Geom &g, View<const T> out, View<const T> gy, View<
     if (want_k) {
         const int64_t cnt = (int64_t)g.Wd * g.C * K;
         hipLaunchKernelGGL((reduce_partials<T>), dim3((cnt + kBlock - 1) / kBlock), dim3(kBlock), 0, s, ws, rows, nout,
-                           (int64_t)0, cnt, gk);
+                           (int64_t)0, cnt, gk, g.fresh);
     }
     if (want_bias) {
         hipLaunchKernelGGL((reduce_partials<T>), dim3(1), dim3(kBlock), 0, s, ws, rows, nout,
-                           (int64_t)g.Wd * g.C * K, (int64_t)g.Wd, gb);
+                           (int64_t)g.Wd * g.C * K, (int64_t)g.Wd, gb, g.fresh);
     }
     return hipGetLastError();
 }

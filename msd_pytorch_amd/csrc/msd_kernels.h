@@ -3,6 +3,8 @@
 
 #include "msd_common.h"
 
+struct msd_adam_param;
+
 namespace msd {
 
 // Upper bound on the number of partial-sum rows of the weight/bias gradient
@@ -54,6 +56,14 @@ hipError_t final_forward_loss(int kind, int64_t batch, int c_in, int c_out, int6
                               int64_t xsc, const T *w, const T *bias, const void *target, int64_t tsb, int64_t tsc,
                               T *out, int64_t osb, int64_t osc, T *gout, int64_t gsb, int64_t gsc, T *gw, T *gb,
                               T *loss, T *ws, hipStream_t s);
+
+// msd_step.hip: see the C ABI.
+hipError_t adam_step(bool f64, int n, const msd_adam_param *params, double lr, double beta1, double beta2, double eps,
+                     hipStream_t s);
+hipError_t scale_fold(bool f64, int c_out, int c_in, const void *scale, const void *shift, const void *weight,
+                      const void *bias, void *folded_weight, void *folded_bias, hipStream_t s);
+hipError_t label_check(int64_t count, int64_t num_labels, const int64_t *labels, int64_t *clamped, int64_t *range,
+                       hipStream_t s);
 
 // Launch-shape knobs (msd_set_tuning in the C ABI).  A value < 0 means "library default".
 enum Knob {
