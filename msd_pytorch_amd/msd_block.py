@@ -104,6 +104,7 @@ class MSDBlock(torch.nn.Module):
         depth = len(dilations)
         self.bias = torch.nn.Parameter(torch.empty(depth * width))
         self.weights = []
+        self.weight_names = tuple(f"weight{i}" for i in range(depth))
         for i in range(depth):
             weight = torch.nn.Parameter(torch.empty(width, in_channels + width * i, *self.kernel_size))
             self.register_parameter(f"weight{i}", weight)
@@ -117,6 +118,11 @@ class MSDBlock(torch.nn.Module):
         fan_in, _ = torch.nn.init._calculate_fan_in_and_fan_out(self.weights[0])
         bound = 1 / math.sqrt(fan_in)
         torch.nn.init.uniform_(self.bias, -bound, bound)
+
+    def own_weights(self):
+        """The registered weights, in order, for the native calls (None where one is not a
+        parameter of this module at the moment)."""
+        return list(map(self._parameters.get, self.weight_names))
 
     def forward(self, input):
         # Look the weights up by attribute on every call: after a device move,

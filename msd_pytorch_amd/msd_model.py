@@ -1,11 +1,15 @@
 """Training wrapper shared by the regression and segmentation models
 (reference msd_model.py:8-342): frozen 1x1 input/output scaling layers, Adam
 on the trainable part, normalisation from a data loader, save/load."""
+import operator
+
 import numpy as np
 import torch
 import torch.nn as nn
 import torch.optim as optim
+import torch.optim.optimizer as optimizer_base
 
+from . import _native
 from . import msd_custom_convolutions as cc
 from .msd_module import MSDFinalFunction, MSDModule
 
@@ -246,10 +250,72 @@ class MSDModel:
             return "nll"
         return None
 
-    def _fused_forward_loss(self):
-        """(loss, output) through the fused node, or None when the model is not the plain
-        scale_in -> msd [-> scale_out | -> LogSoftmax] -> criterion chain on the GPU."""
+    def _fused_parts(self):
+        """(loss kind, scale_out or None) when the model is the plain
+        scale_in -> msd [-> scale_out | -> LogSoftmax] -> criterion chain, else None."""
         return None
+
+    def _fused_forward_loss(self):
+        """(loss, output) through the fused node, or None where that does not apply."""
+        parts = self._fused_parts()
+        if parts is None:
+            return None
+        kind, scale_out = parts
+        return self.msd.forward_loss(self.net[0](self.input), self.target, kind, scale=scale_out)
+
+    def _native_step(self):
+        """Forward, zero_grad and backward as one native call (MSDModule.train_step).  False, with
+        nothing done, where the model or the optimiser is not the plain one."""
+        if not self.fuse_loss or not torch.is_grad_enabled() or not self.input.is_cuda:
+            return False
+        parts = self._fused_parts()
+        if parts is None or type(self.net[0]) not in (ScalingConv2d, ScalingConv3d) or self._net_hooked():
+            return False
+        # the gradients are replaced, which is zero_grad() and backward() for the optimiser of
+        # exactly these parameters
+        linear, block = self.msd.final_layer.linear, self.msd.msd_block
+        own = [block.bias, *block.own_weights(), linear.weight, linear.bias]
+        held = [p for group in self.optimizer.param_groups for p in group["params"]]
+        if len(own) != len(held) or not all(map(operator.is_, own, held)):
+            return False
+        kind, scale_out = parts
+        result = self.msd.train_step(self.input, self.target, kind, self.net[0], scale_out)
+        if result is None:
+            return False
+        self.loss, self.output = result
+        return True
+
+    def _optimizer_step(self):
+        """``self.optimizer.step()``; for a plain Adam all parameters in one launch."""
+        if not self._native_adam():
+            self.optimizer.step()
+
+    _adam_states = None                           # (optimiser state, parameters, their entries)
+
+    def _native_adam(self):
+        opt = self.optimizer
+        # (a learning-rate scheduler puts a step of its own on the instance)
+        if type(opt) is not optim.Adam or "step" in opt.__dict__ or opt._optimizer_step_pre_hooks \
+                or opt._optimizer_step_post_hooks or optimizer_base._global_optimizer_pre_hooks \
+                or optimizer_base._global_optimizer_post_hooks or len(opt.param_groups) != 1:
+            return False
+        group = opt.param_groups[0]
+        if group["weight_decay"] or group["amsgrad"] or group["maximize"] or group["foreach"] is False \
+                or group["differentiable"] or group["fused"] or type(group["lr"]) is not float \
+                or not all(type(b) is float for b in group["betas"]):
+            return False
+        params, state = group["params"], opt.state
+        if not params or not params[0].is_cuda:
+            return False
+        if not group["capturable"] and torch.cuda.is_current_stream_capturing():
+            return False                          # torch's step raises
+        seen = self._adam_states
+        if seen is None or seen[0] is not state or seen[1] is not params or len(state) != len(seen[2]) \
+                or len(params) != len(seen[2]):
+            if len(state) != len(params) or not all(p in state for p in params):
+                return False                      # the first step makes the state
+            seen = self._adam_states = (state, params, [state[p] for p in params])
+        return _native.host().adam_step(params, seen[2], group["lr"], *group["betas"], group["eps"])
 
     def forward(self, input=None, target=None):
         """Loss of one (input, target) pair; arguments left out keep their last value."""
@@ -260,11 +326,16 @@ class MSDModel:
         """Launch forward, zero_grad, backward and (``update``) the optimiser step of
         msd_model.py:225-244 without waiting for the GPU.  Nothing is returned: ``get_loss()``
         reads the loss when it is wanted, and waits then."""
-        self._launch_forward(input, target)
-        self.optimizer.zero_grad()
-        self.loss.backward()
+        if input is not None:
+            self.set_input(input)
+        if target is not None:
+            self.set_target(target)
+        if not self._native_step():
+            self._launch_forward()
+            self.optimizer.zero_grad()
+            self.loss.backward()
         if update:
-            self.optimizer.step()
+            self._optimizer_step()
 
     def gradients(self, input=None, target=None):
         """forward + zero_grad + backward: what ``learn`` does short of the optimiser step.

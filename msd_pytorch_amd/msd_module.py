@@ -3,6 +3,7 @@ from math import sqrt
 
 import torch
 
+from . import _native
 from . import msd_custom_convolutions as cc
 from .msd_block import MSDBlock, block_stack_backward, block_stack_forward
 
@@ -222,9 +223,38 @@ class MSDModule(torch.nn.Module):
                 and linear.bias is not None and not self._hooked():
             # block + final layer as one autograd node (no copy of the stack's gradient)
             block = self.msd_block
+            if not torch.is_grad_enabled() and self.plain_dilations():
+                output = _native.host().net_forward(input, block.bias, block.own_weights(), block.dilations,
+                                                    linear.weight, linear.bias)
+                if output is not None:
+                    return output
             weights = (getattr(block, f"weight{i}") for i in range(len(block.weights)))
             return MSDNetFunction.apply(input, block.dilations, block.bias, linear.weight, linear.bias, *weights)
         return self.final_layer(self.msd_block(input))
+
+    def plain_dilations(self):
+        """True when the dilations are a list of ints, which the native calls take as it is."""
+        d = self.msd_block.dilations
+        return type(d) is list and set(map(type, d)) == {int}
+
+    def train_step(self, input, target, kind, scale_in, scale_out=None):
+        """One training step short of the optimiser, without autograd: ``scale_in`` (frozen 1x1
+        layer), this network, optionally ``scale_out`` (frozen as well) and the loss ``kind``; the
+        gradients of this module's parameters REPLACE their ``.grad``.  The launches are those of
+        the scaling layer and of MSDNetLossFunction, forward and backward, without the autograd
+        graph in between.  Returns (loss, output), neither differentiable, or None (nothing has
+        been done) where the native step does not apply: see csrc/host/msd_host.cpp."""
+        linear, block = self.final_layer.linear, self.msd_block
+        if linear.bias is None or scale_in.bias is None or not self.plain_dilations() or self._hooked():
+            return None
+        sw = sb = None
+        if scale_out is not None:
+            if scale_out.bias is None:
+                return None
+            sw, sb = scale_out.weight, scale_out.bias
+        return _native.host().train_step(input, scale_in.weight, scale_in.bias, block.bias, block.own_weights(),
+                                         block.dilations, linear.weight, linear.bias, sw, sb, target,
+                                         cc.LOSS_KINDS[kind])
 
     def forward_loss(self, input, target, kind, scale=None):
         """(loss, output) of the network followed by an optional frozen 1x1 ``scale`` layer and

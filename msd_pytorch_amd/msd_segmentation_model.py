@@ -2,6 +2,7 @@
 import torch
 import torch.nn as nn
 
+from . import _native
 from .msd_model import MSDModel, _moments, scaling_module_set_bias, scaling_module_set_scale
 
 
@@ -39,31 +40,39 @@ class MSDSegmentationModel(MSDModel):
         # NLLLoss takes (B, *spatial) class indices: drop the channel axis
         self.target = target.squeeze(1).cuda()
 
+    _label_range = None
+
     def _set_target_deferred(self, target):
         if not target.is_cuda:
             return self.set_target(target)      # a host tensor is checked on the host: no device wait
-        target = target.long()
         # lowest and highest label seen since the last verdict, kept on the device; the step
         # itself runs on labels clamped into range, so no loss kernel ever sees an invalid one
-        lo, hi = target.min(), target.max()
-        seen = getattr(self, "_label_range", None)
-        self._label_range = (lo, hi) if seen is None else (torch.minimum(seen[0], lo), torch.maximum(seen[1], hi))
-        self.target = target.squeeze(1).clamp(0, self.num_labels - 1)
+        target = target.long().contiguous()
+        seen = self._label_range
+        if seen is None:
+            limits = torch.iinfo(torch.int64)
+            seen = torch.full((2,), limits.min, dtype=torch.int64, device=target.device)
+            seen[0] = limits.max
+        clamped = _native.host().label_check(target, self.num_labels, seen)
+        if clamped is None:                     # an empty batch, another device than the batch before
+            return self.set_target(target)
+        self._label_range = seen
+        self.target = clamped.squeeze(1)
 
     def _raise_deferred_target_error(self):
-        seen, self._label_range = getattr(self, "_label_range", None), None
+        seen, self._label_range = self._label_range, None
         if seen is None:
             return
-        lo, hi = int(seen[0]), int(seen[1])
+        lo, hi = seen.tolist()
         if lo < 0 or self.num_labels <= hi:
             raise ValueError(
                 f"Target invalid: expected values in range {[0, self.num_labels - 1]}, but got {[lo, hi]}")
 
-    def _fused_forward_loss(self):
+    def _fused_parts(self):
         if self._loss_kind() != "nll" or not isinstance(self.net, nn.Sequential) or len(self.net) != 2:
             return None
         trained = self.net[1]
         if not isinstance(trained, nn.Sequential) or len(trained) != 2 or trained[0] is not self.msd \
                 or type(trained[1]) is not nn.LogSoftmax or trained[1].dim != 1:
             return None
-        return self.msd.forward_loss(self.net[0](self.input), self.target, "nll")
+        return "nll", None

@@ -1,0 +1,150 @@
+"""The native host path (csrc/host/msd_host.cpp) against the Python path it stands in for: the
+same launches, so the same bits where nothing but the route differs."""
+import pytest
+import torch
+
+from parity import bias_close, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ndim,size,c_in,c_out,dilation,dtype", [
+    (2, (1, 5), 1, 1, 1, torch.float32),           # rows too short for the row kernels
+    (2, (96, 96), 12, 1, 3, torch.float32),
+    (2, (33, 130), 17, 2, 10, torch.float32),
+    (2, (40, 64), 5, 5, 2, torch.float32),         # output channels two at a time
+    (3, (8, 9, 33), 3, 1, 2, torch.float32),
+    (3, (6, 7, 64), 16, 3, 1, torch.float32),
+    (2, (9, 11), 2, 2, 4, torch.float64),
+    (3, (5, 6, 7), 2, 1, 2, torch.float64),
+])
+@pytest.mark.parametrize("relu", [True, False])
+def test_a_layer_overwrites_what_the_operators_add_to_zeros(ndim, size, c_in, c_out, dilation, dtype, relu):
+    from msd_pytorch_amd import conv2d, conv3d
+    function = {(2, True): conv2d.Conv2dReluFunction, (2, False): conv2d.Conv2dFunction,
+                (3, True): conv3d.Conv3DReluFunction, (3, False): conv3d.Conv3DFunction}[ndim, relu]
+    native = {(2, True): conv2d.conv2d_relu, (2, False): conv2d.conv2d,
+              (3, True): conv3d.conv3d_relu, (3, False): conv3d.conv3d}[ndim, relu]
+    gen = torch.Generator().manual_seed(7)
+    x = torch.randn(2, c_in, *size, generator=gen, dtype=dtype).cuda().requires_grad_()
+    w = torch.randn(c_out, c_in, *([3] * ndim), generator=gen, dtype=dtype).cuda().requires_grad_()
+    b = torch.randn(c_out, generator=gen, dtype=dtype).cuda().requires_grad_()
+    g = torch.randn(2, c_out, *size, generator=gen, dtype=dtype).cuda()
+    results = []
+    for apply in (native, function.apply):
+        # memory that the gradients will be allocated from holds something else than zeros
+        dirty = [torch.full_like(t, 7.0) for t in (x, w, b)]
+        del dirty
+        out = torch.empty_like(g)
+        y = apply(x, w, b, out, 1, dilation)
+        assert y.data_ptr() == out.data_ptr()
+        results.append([y.detach().clone(), *torch.autograd.grad(y, (x, w, b), g)])
+    for got, want in zip(*results):
+        # one rounding more or less where a gradient is added to a zero that was stored before
+        assert rel_err(got, want) <= (1e-6 if dtype == torch.float32 else 1e-14)
+    # only what is asked for
+    y = native(x.detach(), w, b, torch.empty_like(g), 1, dilation)
+    only = torch.autograd.grad(y, (b,), g)
+    # (the bias gradient alone is summed by another kernel, in another order)
+    terms = g * (y.detach() > 0) if relu else g
+    assert bias_close(only[0], results[1][3].cpu(), terms.cpu(), tol=1e-4 if dtype == torch.float32 else 1e-12)
+
+
+def test_a_layer_raises_like_the_operators():
+    from msd_pytorch_amd.conv2d import conv2d_relu
+    x, w, b = torch.zeros(1, 2, 4, 4).cuda(), torch.zeros(1, 2, 3, 3).cuda(), torch.zeros(1).cuda()
+    with pytest.raises(RuntimeError, match="Dilation cannot be greater"):
+        conv2d_relu(x, w, b, torch.zeros(1, 1, 4, 4).cuda(), 1, 5)
+    with pytest.raises(RuntimeError, match="same type"):
+        conv2d_relu(x, w.double(), b, torch.zeros(1, 1, 4, 4).cuda(), 1, 1)
+
+
+def _models(task, ndim, depth, width, c_out, count):
+    from msd_pytorch_amd import MSDRegressionModel, MSDSegmentationModel
+    models = []
+    for _ in range(count):
+        torch.manual_seed(3)
+        if task == "labels":
+            m = MSDSegmentationModel(2, c_out, depth, width, dilations=[1, 2, 3], ndim=ndim)
+        else:
+            m = MSDRegressionModel(2, c_out, depth, width, dilations=[1, 2, 3], loss=task, ndim=ndim)
+            m.scale_out.weight.data += 0.3 * torch.randn_like(m.scale_out.weight)
+            m.scale_out.bias.data += 0.7
+        m.scale_in.weight.data *= 1.7
+        m.scale_in.bias.data -= 0.2
+        m.msd.final_layer.linear.weight.data.normal_(0, 0.2)
+        models.append(m)
+    return models
+
+
+@pytest.mark.parametrize("task,ndim,size,depth,width,c_out", [
+    ("L2", 2, (20, 65), 4, 1, 1), ("L1", 2, (32, 64), 5, 2, 3), ("labels", 2, (31, 40), 6, 1, 4),
+    ("L2", 3, (6, 9, 36), 4, 1, 2), ("labels", 3, (5, 7, 33), 3, 2, 2),
+    ("L2", 2, (16, 64), 62, 1, 1),                 # more parameters than one launch of the optimiser takes
+])
+def test_training_steps_follow_the_autograd_path(task, ndim, size, depth, width, c_out):
+    native, general = _models(task, ndim, depth, width, c_out, 2)
+    general._native_step = lambda: False
+    general._native_adam = lambda: False
+    gen = torch.Generator().manual_seed(5)
+    for step in range(3):
+        x = torch.randn(2, 2, *size, generator=gen).cuda()
+        t = torch.randint(0, c_out, (2, 1, *size), generator=gen).cuda() if task == "labels" \
+            else torch.randn(2, c_out, *size, generator=gen).cuda()
+        losses = [m.learn(x, t) for m in (native, general)]
+        assert abs(losses[0] - losses[1]) <= 1e-5 * abs(losses[1])
+        assert native.loss.grad_fn is None and general.loss.grad_fn is not None
+        assert rel_err(native.output, general.output) <= 1e-4
+        for p, q in zip(native.msd.parameters(), general.msd.parameters()):
+            # Adam's first steps are lr * sign(gradient): a rounding of a gradient near zero may
+            # move its parameter by up to lr, so the parameters are copied over for the next step
+            assert p.grad.shape == q.grad.shape and rel_err(p.grad, q.grad) <= 1e-4
+            state, want = native.optimizer.state[p], general.optimizer.state[q]
+            assert float(state["step"]) == float(want["step"]) == step + 1
+            assert rel_err(state["exp_avg"], want["exp_avg"]) <= 1e-4
+            assert rel_err(state["exp_avg_sq"], want["exp_avg_sq"]) <= 2e-4
+            assert float((p.detach() - q.detach()).abs().max()) <= 2.1e-3
+            p.data.copy_(q.data)
+
+
+def test_what_the_native_step_leaves_to_the_general_path():
+    (model,) = _models("L2", 2, 3, 1, 1, 1)
+    x, t = torch.rand(1, 2, 24, 40).cuda(), torch.rand(1, 1, 24, 40).cuda()
+    model.learn(x, t)
+    assert model.loss.grad_fn is None
+    seen = []
+    handle = model.msd.msd_block.weight1.register_hook(lambda g: seen.append(tuple(g.shape)))
+    model.learn(x, t)                              # a watched parameter
+    assert seen == [(1, 3, 3, 3)] and model.loss.grad_fn is not None
+    handle.remove()
+    model.optimizer = torch.optim.SGD(list(model.msd.parameters())[:2], lr=0.1)
+    before = model.msd.final_layer.linear.weight.detach().clone()
+    model.learn(x, t)                              # an optimiser of some of the parameters
+    assert model.loss.grad_fn is not None and torch.equal(before, model.msd.final_layer.linear.weight)
+    model.optimizer = torch.optim.Adam(model.msd.parameters(), weight_decay=0.1)
+    model.learn(x, t)
+    scheduler = torch.optim.lr_scheduler.StepLR(model.optimizer, 1)
+    assert not model._native_adam()                # weight decay, and a scheduler's own step
+    model.learn(x, t)
+    scheduler.step()
+
+
+@pytest.mark.parametrize("count", [1, 63, 1000, 300001])
+def test_label_check(count):
+    from msd_pytorch_amd import _native
+    gen = torch.Generator().manual_seed(count)
+    labels = torch.randint(-3, 9, (count,), generator=gen).cuda()
+    seen = torch.tensor([2, 4]).cuda()
+    out = _native.host().label_check(labels, 6, seen)
+    assert torch.equal(out, labels.clamp(0, 5))
+    assert seen.tolist() == [min(2, int(labels.min())), max(4, int(labels.max()))]
+
+
+@pytest.mark.parametrize("ndim,size", [(2, (30, 70)), (3, (5, 8, 40))])
+def test_prediction_without_gradients_equals_the_differentiable_pass(ndim, size):
+    (model,) = _models("L2", ndim, 5, 1, 3, 1)
+    x = torch.rand(2, 2, *size).cuda()
+    with torch.no_grad():
+        got = model.net(x)
+    want = model.net(x)
+    assert want.requires_grad and torch.equal(got, want.detach())
