@@ -313,6 +313,15 @@ int msd_block_forward(int dtype, int ndim, int64_t batch, int64_t c_in, int dept
                       const int64_t *spatial, const int64_t *dilations,
                       void *stack, const int64_t *stack_strides,
                       const void *const *weights, const void *bias, void *stream);
+/* The same with a workspace (msd_block_forward_workspace_bytes; less, or none, is accepted):
+ * groups of layers then take the channels in front of them in one pass (2D, fp32; same sums in
+ * another order). */
+int64_t msd_block_forward_workspace_bytes(int dtype, int ndim, int64_t batch, int64_t c_in, int depth,
+                                          const int64_t *widths, const int64_t *spatial);
+int msd_block_forward_ws(int dtype, int ndim, int64_t batch, int64_t c_in, int depth, const int64_t *widths,
+                         const int64_t *spatial, const int64_t *dilations, void *stack, const int64_t *stack_strides,
+                         const void *const *weights, const void *bias, void *workspace, int64_t workspace_bytes,
+                         void *stream);
 
 int msd_block_backward(int dtype, int ndim, int64_t batch, int64_t c_in, int depth, const int64_t *widths,
                        const int64_t *spatial, const int64_t *dilations,

@@ -54,6 +54,9 @@ PROTOTYPES = {
     "msd_block_workspace_bytes": (_c_i64, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p]),
     "msd_block_forward": (_c_int, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p, _i64p] + _VIEW
                           + [ctypes.POINTER(ctypes.c_void_p), _ptr, _ptr]),
+    "msd_block_forward_workspace_bytes": (_c_i64, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p]),
+    "msd_block_forward_ws": (_c_int, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p, _i64p] + _VIEW
+                             + [ctypes.POINTER(ctypes.c_void_p), _ptr] + _WS + [_ptr]),
     "msd_block_backward": (_c_int, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p, _i64p] + _VIEW + _VIEW
                            + [ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_void_p), _ptr, _c_int]
                            + _WS + [_ptr]),

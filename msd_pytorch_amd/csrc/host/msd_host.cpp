@@ -28,7 +28,7 @@ namespace py = pybind11;
 // The entry points, looked up in the library that the package has loaded.
 #define MSD_ENTRIES(X)                                                                                              \
     X(msd_last_error) X(msd_conv_forward) X(msd_conv_relu_forward) X(msd_conv_layer_backward) X(msd_workspace_bytes)  \
-    X(msd_block_forward) X(msd_block_backward) X(msd_block_workspace_bytes) X(msd_final_forward)                     \
+    X(msd_block_forward_ws) X(msd_block_forward_workspace_bytes) X(msd_block_backward) X(msd_block_workspace_bytes) X(msd_final_forward)                     \
     X(msd_final_backward) X(msd_final_forward_loss) X(msd_final_workspace_bytes) X(msd_scale_fold) X(msd_adam_step)   \
     X(msd_label_check)
 struct Entries {
@@ -217,9 +217,14 @@ struct Block {
 
     void forward(const Tensor &stack, const Tensor &bias, void *stream) const
     {
-        check(lib.msd_block_forward(dtype_of(stack), (int)stack.dim() - 2, stack.size(0), c_in, (int)widths.size(),
-                                    widths.data(), stack.sizes().data() + 2, dilations.data(), stack.data_ptr(),
-                                    stack.strides().data(), weights.data(), bias.data_ptr(), stream));
+        const int64_t need = lib.msd_block_forward_workspace_bytes(dtype_of(stack), (int)stack.dim() - 2,
+                                                                   stack.size(0), c_in, (int)widths.size(),
+                                                                   widths.data(), stack.sizes().data() + 2);
+        const Tensor ws = need ? workspace(need, stack) : Tensor();
+        check(lib.msd_block_forward_ws(dtype_of(stack), (int)stack.dim() - 2, stack.size(0), c_in, (int)widths.size(),
+                                       widths.data(), stack.sizes().data() + 2, dilations.data(), stack.data_ptr(),
+                                       stack.strides().data(), weights.data(), bias.data_ptr(),
+                                       need ? ws.data_ptr() : nullptr, need, stream));
     }
 };
 

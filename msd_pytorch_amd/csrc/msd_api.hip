@@ -2,6 +2,7 @@
 // the kernels.  Nothing here touches the device before the checks pass, so
 // every MSD_ERR_INVALID path can be exercised on a machine without a GPU.
 #include "../../include/msd_hip.h"
+#include "msd_group.h"
 #include "msd_kernels.h"
 
 #include <cstdarg>
@@ -18,8 +19,9 @@ const char *const kKnobNames[kKnobCount] = {
     "fwd.vec2d", "fwd.vec3d", "fwd.split", "fwd.rows2d", "bwdk.rows", "block.fuse",
     "block.defer", "bwdk.interleave", "block.snake", "fwd.class3d", "fwd.lattice3d",
     "block.pair", "block.triple", "final.tiled", "block.split3d", "block.chainpair", "bwdk.fused3d", "bwdx.lean1",
+    "fwd.group",
 };
-static_assert(kKnobBwdxLean1 + 1 == kKnobCount, "one name per knob, in the order of the enum");
+static_assert(kKnobFwdGroup + 1 == kKnobCount, "one name per knob, in the order of the enum");
 int g_knobs[kKnobCount];
 // every knob starts at "library default"
 const bool g_knobs_ready = [] {
@@ -1268,9 +1270,123 @@ int64_t msd_block_workspace_bytes(int dtype, int ndim, int64_t batch, int64_t c_
     return need + (regions < kDeferBudgetBytes ? regions : kDeferBudgetBytes);
 }
 
+namespace {
+
+// Layers of a 2D block are taken together (msd_group.h) where this many channels lie in front of
+// the first of them.  At 1024 x 1024 and at 512 x 512 a start at 4, 6, 9, 12 or 16 channels times
+// within 2 %, with one channel per layer; below that the pass costs more than the layers' own
+// kernels, which read few channels from the caches.  With two channels per layer those kernels
+// are slower (64 registers of sums) and the pass pays at once.  Small images gain as well (100 layers at
+// 64 x 64: 854 -> 535 us): the last launch of a group reads 10 planes, not 100.
+constexpr int64_t kGroupChannels = 12, kGroupChannelsWide = 6;
+
+// Number of layers from layer i on that form a group of the forward pass (0: none).
+int forward_group(const BlockArgs &a, int i, int64_t first)
+{
+    const int from = msd::knob(msd::kKnobFwdGroup, -1);
+    if (a.dtype != MSD_F32 || a.ndim != 2 || g_kernel_path != 0 || from == 0) return 0;
+    if (first < (from > 0 ? from : a.widths[i] > 1 ? kGroupChannelsWide : kGroupChannels)) return 0;
+    int n = 0;
+    int64_t outputs = 0;
+    while (i + n < a.depth && a.widths[i + n] <= 2 && outputs + a.widths[i + n] <= msd::group2d::kMaxOut)
+        outputs += a.widths[i + n++];
+    return n >= 2 ? n : 0;
+}
+
+int64_t forward_group_bytes(const BlockArgs &a)
+{
+    int64_t first = a.c_in;
+    for (int i = 0; i < a.depth; i++) {
+        if (forward_group(a, i, first))
+            return 3 * msd::group2d::kMaxOut * a.batch * a.spatial[0] * a.spatial[1] * (int64_t)sizeof(float);
+        first += a.widths[i];
+    }
+    return 0;
+}
+
+// Layers i .. i + n - 1: one pass over the channels [0, first) for all of them, then each layer
+// over the few channels that the group itself adds.  *done is false (and nothing was launched)
+// where a kernel does not take the shape.
+int block_group_forward(const char *fn, const BlockArgs &a, int i, int n, int64_t first, void *stack,
+                        const int64_t *stack_strides, const void *const *weights, const float *bias, float *z,
+                        hipStream_t s, bool *done)
+{
+    *done = false;
+    msd::View<float> st;
+    MSD_TRY(make_view(fn, "stack", a.ndim, stack, stack_strides, &st));
+    const msd::View<const float> x{st.p, st.sb, st.sc, st.sz, st.sy, st.sx};
+    msd::group2d::Outputs out;
+    out.n = 0;
+    int dmax = 0;
+    int64_t added = 0;
+    std::vector<msd::Geom> geoms(n);
+    for (int j = 0; j < n; j++) {
+        const int64_t w = a.widths[i + j];
+        const int d = (int)a.dilations[i + j];
+        dmax = d > dmax ? d : dmax;
+        for (int co = 0; co < w; co++) {
+            out.dil[out.n] = d;
+            out.k[out.n++] = (const float *)weights[i + j] + co * (first + added) * msd::group2d::kTaps;
+        }
+        MSD_TRY(make_geom(fn, a.dtype, a.ndim, a.batch, added, w, a.spatial, d, true, &geoms[j]));
+        const msd::View<float> y{st.p + (first + added) * st.sc, st.sb, st.sc, st.sz, st.sy, st.sx};
+        const msd::View<const float> xn{st.p + first * st.sc, st.sb, st.sc, st.sz, st.sy, st.sx};
+        if (!msd::group_finish_supported_2d(geoms[j], xn, y) && !msd::fast_forward_supported_2d(geoms[j], xn, y))
+            return MSD_OK;
+        added += w;
+    }
+    for (int o = out.n; o < msd::group2d::kMaxOut; o++) {
+        out.dil[o] = 0;
+        out.k[o] = nullptr;
+    }
+    msd::Geom shared;
+    MSD_TRY(make_geom(fn, a.dtype, a.ndim, a.batch, first, out.n, a.spatial, dmax, true, &shared));
+    if (!msd::group_push_supported_2d(shared, x, dmax)) return MSD_OK;
+    ProfileScope scope(0, s);
+    hipError_t e = msd::group_push_2d(shared, x, out, z, s);
+    if (e != hipSuccess) return hip_fail(fn, e);
+    const int64_t plane = a.spatial[0] * a.spatial[1];
+    added = 0;
+    for (int j = 0; j < n; j++) {
+        const msd::View<float> y{st.p + (first + added) * st.sc, st.sb, st.sc, st.sz, st.sy, st.sx};
+        const msd::View<const float> xn{st.p + first * st.sc, st.sb, st.sc, st.sz, st.sy, st.sx};
+        const int64_t per_output = (first + added) * msd::group2d::kTaps;
+        const msd::ForwardSums sums{z + 3 * added * plane, 3 * (int64_t)out.n * plane, per_output};
+        const float *kn = (const float *)weights[i + j] + first * msd::group2d::kTaps;
+        e = msd::group_finish_supported_2d(geoms[j], xn, y)
+                ? msd::group_finish_2d(geoms[j], xn, kn, bias + added, y, sums, s)
+                : msd::fast_forward_sums_2d(geoms[j], xn, kn, bias + added, y, s, sums);
+        if (e != hipSuccess) return hip_fail(fn, e);
+        added += a.widths[i + j];
+    }
+    *done = true;
+    return MSD_OK;
+}
+
+}  // namespace
+
+int64_t msd_block_forward_workspace_bytes(int dtype, int ndim, int64_t batch, int64_t c_in, int depth,
+                                          const int64_t *widths, const int64_t *spatial)
+{
+    if (!widths || !spatial || depth <= 0 || (ndim != 2 && ndim != 3) || batch <= 0 || c_in <= 0) return -1;
+    for (int i = 0; i < depth; i++)
+        if (widths[i] <= 0) return -1;
+    const BlockArgs a{dtype, ndim, depth, batch, c_in, 0, widths, spatial, nullptr, dtype == MSD_F32 ? 4u : 8u};
+    return forward_group_bytes(a);
+}
+
 int msd_block_forward(int dtype, int ndim, int64_t batch, int64_t c_in, int depth, const int64_t *widths,
                       const int64_t *spatial, const int64_t *dilations, void *stack, const int64_t *stack_strides,
                       const void *const *weights, const void *bias, void *stream)
+{
+    return msd_block_forward_ws(dtype, ndim, batch, c_in, depth, widths, spatial, dilations, stack, stack_strides, weights,
+                                bias, nullptr, 0, stream);
+}
+
+int msd_block_forward_ws(int dtype, int ndim, int64_t batch, int64_t c_in, int depth, const int64_t *widths,
+                         const int64_t *spatial, const int64_t *dilations, void *stack, const int64_t *stack_strides,
+                         const void *const *weights, const void *bias, void *workspace, int64_t workspace_bytes,
+                         void *stream)
 {
     const char *fn = "block_forward";
     BlockArgs a;
@@ -1280,6 +1396,20 @@ int msd_block_forward(int dtype, int ndim, int64_t batch, int64_t c_in, int dept
     ProfileBatch profile_runs((hipStream_t)stream);
     int64_t first = c_in, b0 = 0;
     for (int i = 0; i < depth; i++) {
+        const int n = workspace ? forward_group(a, i, first) : 0;
+        if (n && workspace_bytes >= forward_group_bytes(a)) {
+            bool done = false;
+            MSD_TRY(block_group_forward(fn, a, i, n, first, stack, stack_strides, weights, (const float *)bias + b0,
+                                        (float *)workspace, (hipStream_t)stream, &done));
+            if (done) {
+                for (int j = 0; j < n; j++) {
+                    first += widths[i + j];
+                    b0 += widths[i + j];
+                }
+                i += n - 1;
+                continue;
+            }
+        }
         char *out = (char *)stack + first * stack_strides[1] * a.elem;
         // Every second layer walks its input channels from the last to the first: what the
         // layer before touched last is then read first, while it is still in the caches

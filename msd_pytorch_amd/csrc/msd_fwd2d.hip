@@ -14,4 +14,10 @@ hipError_t fast_forward_2d(const Geom &g, bool relu, const View<const float> &x,
     return fwd::run_nd<2>(g, relu, x, k, bias, out, s);
 }
 
+hipError_t fast_forward_sums_2d(const Geom &g, const View<const float> &x, const float *k, const float *bias,
+                                const View<float> &out, hipStream_t s, const ForwardSums &sums)
+{
+    return fwd::run_nd<2>(g, true, x, k, bias, out, s, &sums);
+}
+
 }  // namespace msd

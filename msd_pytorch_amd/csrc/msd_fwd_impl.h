@@ -39,6 +39,9 @@ struct Lattice {
     int tiles_z;    // dil * segs_z (1 in 2D)
     int ntiles;
     int by_class;   // 3D: tiles numbered residue class by residue class (2: a class row by row, no blocks)
+    int64_t kco;    // distance between the weights of two output channels
+    const float *zin;   // 2D: planes (3 per output channel, one per tap row) that are added to the output,
+    int64_t zsb;        // row y +- dil of each: what a group's pass over the shared channels left (or null)
 };
 
 // First output row (y0, z0) of the lattice this workgroup computes; false for the padding
@@ -139,6 +142,24 @@ __global__ __launch_bounds__(NDIM == 3 ? 512 : 1024, (NDIM == 3 && V == 1 && WOU
                 for (int r = 0; r < 3; r++)
 #pragma unroll
                     for (int i = 0; i < V; i++) acc[co][jz][jy][r][i] = 0.f;
+    if constexpr (NDIM == 2) {
+        if (lt.zin && kg == 0) {                 // uniform over the wave
+            // already shifted along x: they start the centre sum of the first channel group
+            const float *zp = lt.zin + (int64_t)b * lt.zsb + x0;
+#pragma unroll
+            for (int co = 0; co < WOUT; co++)
+#pragma unroll
+                for (int ky = 0; ky < 3; ky++)
+#pragma unroll
+                    for (int jy = 0; jy < RY; jy++) {
+                        const int y = min(y0 + jy * g.dil, g.H - 1);
+                        float v[V];
+                        load_vec<V>(zp + ((int64_t)(3 * co + ky) * g.H + min(reflect_idx(y + (ky - 1) * g.dil, g.H), g.H - 1)) * g.W, v);
+#pragma unroll
+                        for (int i = 0; i < V; i++) acc[co][0][jy][1][i] += v[i];
+                    }
+        }
+    }
 
     const char *xb = reinterpret_cast<const char *>(x.p + (int64_t)b * x.sb);
     for (int cn = kg; cn < g.C; cn += lt.ks) {
@@ -148,7 +169,7 @@ __global__ __launch_bounds__(NDIM == 3 ? 512 : 1024, (NDIM == 3 && V == 1 && WOU
 #pragma unroll
         for (int co = 0; co < WOUT; co++)
 #pragma unroll
-            for (int t = 0; t < K; t++) w[co][t] = k[((int64_t)co * g.C + ci) * K + t];
+            for (int t = 0; t < K; t++) w[co][t] = k[co * lt.kco + (int64_t)ci * K + t];
         // (redefining the lane offsets here keeps their widening to 64 bits inside the loop, next
         // to the loads, where it costs nothing; hoisted, it would turn them into register pairs
         // and every load address into a 64-bit vector addition)
@@ -283,10 +304,13 @@ inline bool make_lattice(const Geom &g, int V, int rz, int ry, int ks_wanted, La
 
 template <int NDIM, bool RELU, int WOUT, int V, int RZ, int RY>
 hipError_t launch(const Geom &g, const View<const float> &x, const float *k, const float *bias,
-                  const View<float> &out, hipStream_t s)
+                  const View<float> &out, hipStream_t s, const ForwardSums *sums)
 {
     Lattice lt;
     if (!make_lattice(g, V, RZ, RY, knob(kKnobFwdSplit, 2), &lt)) return hipErrorInvalidConfiguration;
+    lt.kco = sums ? sums->kco : (int64_t)g.C * Taps<NDIM>::K;
+    lt.zin = sums ? sums->z : nullptr;
+    lt.zsb = sums ? sums->zsb : 0;
     const int remap = knob(kKnobXcdRemap, 1);
     const dim3 grid(remap ? xcd_grid(lt.ntiles) : lt.ntiles, g.B, 1);
     const size_t lds = (size_t)lt.ks * 3 * V * lt.lpr * sizeof(float);
@@ -321,20 +345,20 @@ bool supported_nd(const Geom &g, const View<const float> &x, const View<float> &
 // 2D, one output channel: the instance with `ry` output rows per tile (2 to 6; 4 otherwise).
 template <bool RELU, int V>
 hipError_t launch_rows_2d(int ry, const Geom &g, const View<const float> &x, const float *k, const float *bias,
-                          const View<float> &out, hipStream_t s)
+                          const View<float> &out, hipStream_t s, const ForwardSums *sums)
 {
     switch (ry) {
-    case 2: return launch<2, RELU, 1, V, 1, 2>(g, x, k, bias, out, s);
-    case 3: return launch<2, RELU, 1, V, 1, 3>(g, x, k, bias, out, s);
-    case 5: return launch<2, RELU, 1, V, 1, 5>(g, x, k, bias, out, s);
-    case 6: return launch<2, RELU, 1, V, 1, 6>(g, x, k, bias, out, s);
-    default: return launch<2, RELU, 1, V, 1, 4>(g, x, k, bias, out, s);
+    case 2: return launch<2, RELU, 1, V, 1, 2>(g, x, k, bias, out, s, sums);
+    case 3: return launch<2, RELU, 1, V, 1, 3>(g, x, k, bias, out, s, sums);
+    case 5: return launch<2, RELU, 1, V, 1, 5>(g, x, k, bias, out, s, sums);
+    case 6: return launch<2, RELU, 1, V, 1, 6>(g, x, k, bias, out, s, sums);
+    default: return launch<2, RELU, 1, V, 1, 4>(g, x, k, bias, out, s, sums);
     }
 }
 
 template <int NDIM, bool RELU, int WOUT>
 hipError_t pick(const Geom &g, const View<const float> &x, const float *k, const float *bias, const View<float> &out,
-                hipStream_t s)
+                hipStream_t s, const ForwardSums *sums)
 {
     int vmax = knob(NDIM == 3 ? kKnobFwdVec3d : kKnobFwdVec2d, NDIM == 3 ? 1 : 4);
     const bool resident = (int64_t)g.B * g.C * x.sc * (int64_t)sizeof(float) <= kCacheResidentBytes;
@@ -342,8 +366,8 @@ hipError_t pick(const Geom &g, const View<const float> &x, const float *k, const
     int v = choose_vec(g, vmax, x, out);
     if (v == 0) v = choose_vec(g, 4, x, out);
     if constexpr (NDIM == 3) {
-        if (v == 4) return launch<3, RELU, WOUT, 4, 2, 2>(g, x, k, bias, out, s);
-        if (v == 2) return launch<3, RELU, WOUT, 2, 2, 4>(g, x, k, bias, out, s);
+        if (v == 4) return launch<3, RELU, WOUT, 4, 2, 2>(g, x, k, bias, out, s, sums);
+        if (v == 2) return launch<3, RELU, WOUT, 2, 2, 4>(g, x, k, bias, out, s, sums);
         if (v == 1) {
             if constexpr (WOUT == 1) {
                 // Lattices of 3 x 3 rows instead of 2 x 4 where they cover the residue classes
@@ -358,13 +382,13 @@ hipError_t pick(const Geom &g, const View<const float> &x, const float *k, const
                 // two workgroups fewer share a CU.
                 const long t44 = (long)((rows_z + 3) / 4) * ((rows_y + 3) / 4);
                 const int forced = knob(kKnobFwdLattice3d, 0);
-                if (forced == 44) return launch<3, RELU, 1, 1, 4, 4>(g, x, k, bias, out, s);
-                if (forced == 33) return launch<3, RELU, 1, 1, 3, 3>(g, x, k, bias, out, s);
-                if (forced == 24) return launch<3, RELU, 1, 1, 2, 4>(g, x, k, bias, out, s);
+                if (forced == 44) return launch<3, RELU, 1, 1, 4, 4>(g, x, k, bias, out, s, sums);
+                if (forced == 33) return launch<3, RELU, 1, 1, 3, 3>(g, x, k, bias, out, s, sums);
+                if (forced == 24) return launch<3, RELU, 1, 1, 2, 4>(g, x, k, bias, out, s, sums);
                 (void)t44;
-                if (g.dil >= 3 && t33 * 16 < t24 * 15) return launch<3, RELU, 1, 1, 3, 3>(g, x, k, bias, out, s);
+                if (g.dil >= 3 && t33 * 16 < t24 * 15) return launch<3, RELU, 1, 1, 3, 3>(g, x, k, bias, out, s, sums);
             }
-            return launch<3, RELU, WOUT, 1, 2, 4>(g, x, k, bias, out, s);
+            return launch<3, RELU, WOUT, 1, 2, 4>(g, x, k, bias, out, s, sums);
         }
     } else {
         if constexpr (WOUT == 1) {
@@ -384,14 +408,14 @@ hipError_t pick(const Geom &g, const View<const float> &x, const float *k, const
                 if (ry == first || cost < best_cost) { best = ry; best_cost = cost; }
             }
             best = knob(kKnobFwdRows2d, best);
-            if (v == 4) return launch_rows_2d<RELU, 4>(best, g, x, k, bias, out, s);
-            if (v == 2) return launch_rows_2d<RELU, 2>(best, g, x, k, bias, out, s);
-            if (v == 1) return launch_rows_2d<RELU, 1>(best, g, x, k, bias, out, s);
+            if (v == 4) return launch_rows_2d<RELU, 4>(best, g, x, k, bias, out, s, sums);
+            if (v == 2) return launch_rows_2d<RELU, 2>(best, g, x, k, bias, out, s, sums);
+            if (v == 1) return launch_rows_2d<RELU, 1>(best, g, x, k, bias, out, s, sums);
         } else {
             // two output channels double the accumulators: three rows per tile keep them in registers
-            if (v == 4) return launch<2, RELU, 2, 4, 1, 3>(g, x, k, bias, out, s);
-            if (v == 2) return launch<2, RELU, 2, 2, 1, 4>(g, x, k, bias, out, s);
-            if (v == 1) return launch<2, RELU, 2, 1, 1, 4>(g, x, k, bias, out, s);
+            if (v == 4) return launch<2, RELU, 2, 4, 1, 3>(g, x, k, bias, out, s, sums);
+            if (v == 2) return launch<2, RELU, 2, 2, 1, 4>(g, x, k, bias, out, s, sums);
+            if (v == 1) return launch<2, RELU, 2, 1, 1, 4>(g, x, k, bias, out, s, sums);
         }
     }
     return hipErrorInvalidConfiguration;
@@ -399,11 +423,11 @@ hipError_t pick(const Geom &g, const View<const float> &x, const float *k, const
 
 template <int NDIM>
 hipError_t run_nd(const Geom &g, bool relu, const View<const float> &x, const float *k, const float *bias,
-                  const View<float> &out, hipStream_t s)
+                  const View<float> &out, hipStream_t s, const ForwardSums *sums = nullptr)
 {
     if (g.Wd == 1)
-        return relu ? pick<NDIM, true, 1>(g, x, k, bias, out, s) : pick<NDIM, false, 1>(g, x, k, bias, out, s);
-    return relu ? pick<NDIM, true, 2>(g, x, k, bias, out, s) : pick<NDIM, false, 2>(g, x, k, bias, out, s);
+        return relu ? pick<NDIM, true, 1>(g, x, k, bias, out, s, sums) : pick<NDIM, false, 1>(g, x, k, bias, out, s, sums);
+    return relu ? pick<NDIM, true, 2>(g, x, k, bias, out, s, sums) : pick<NDIM, false, 2>(g, x, k, bias, out, s, sums);
 }
 
 }  // namespace fwd

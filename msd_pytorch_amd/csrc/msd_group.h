@@ -1,0 +1,72 @@
+// Groups of consecutive layers of a dense block on the matrix cores (2D, fp32).
+//
+// The layers i, i + 1, ... of a group read the same channels [0, c) of the stack, c the number
+// of channels in front of the first of them.  Taken together they are one matrix product over
+// those channels: with one row per (output, tap) a group of seven one-channel layers is a
+// 63 x c weight matrix, which fills four 16-row tiles of v_mfma_f32_16x16x4 to 98 %, and every
+// channel is read once for seven layers instead of once (three rows at a time) per layer.
+#pragma once
+#include "msd_kernels.h"
+#include "msd_rows.h"
+
+namespace msd {
+namespace group2d {
+
+constexpr int kTaps = 9;
+constexpr int kMaxOut = 7;                        // outputs of a group: 7 * 9 = 63 of 64 matrix rows
+constexpr int kRows = 64;                         // matrix rows
+constexpr int kTiles = kRows / 16;
+constexpr int kChunk = 128;                       // channels whose weights are in LDS at a time
+
+// The outputs of a group: dilation, and weights of the channels from 0 on, of each.
+struct Outputs {
+    int n;
+    int dil[kMaxOut];
+    const float *k[kMaxOut];
+};
+
+// How the rows of an image are spread over waves: a team of `waves` waves owns one row (or one
+// segment of a long row: 64 * waves voxels of which `inner` are its own, the rest overlap with its
+// neighbours), `rpw` teams form a workgroup.
+struct Teams {
+    int waves, rpw, segs, inner;
+};
+
+// Chosen so that as few waves as possible work in all, counted with those that find no room: up
+// to 16 waves share a compute unit, as one workgroup or as two of at most 8 (which also lets one
+// work while the other finishes a row).
+inline Teams make_teams(int W, int halo)
+{
+    Teams best{0, 0, 0, 0};
+    double best_cost = 0;
+    for (int w = 1; w <= 16; w++) {
+        int inner = W, segs = 1;
+        if (w * kWave < W) {
+            inner = (w * kWave - 2 * halo) & ~3;
+            if (inner < kWave) continue;
+            segs = (W + inner - 1) / inner;
+        }
+        const int rpw = w <= 8 ? 8 / w : 1;
+        const double cost = (double)segs * w * 16 / (w <= 8 ? 2 * rpw * w : w);
+        if (best.waves == 0 || cost < best_cost) {
+            best = Teams{w, rpw, segs, inner};
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+}  // namespace group2d
+
+// z[b][3 o + ky][y][x] = sum over the g.C channels and kx of k[o][c][ky][kx] * x[c][y][fold(x + dil_o (kx - 1))]:
+// what row y of the channels contributes to the output rows that read it through tap row ky.
+bool group_push_supported_2d(const Geom &g, const View<const float> &x, int dmax);
+hipError_t group_push_2d(const Geom &g, const View<const float> &x, const group2d::Outputs &out, float *z, hipStream_t s);
+
+
+// One layer of the group from its planes and the g.C channels that the group has added (with ReLU).
+bool group_finish_supported_2d(const Geom &g, const View<const float> &x, const View<float> &out);
+hipError_t group_finish_2d(const Geom &g, const View<const float> &x, const float *k, const float *bias,
+                           const View<float> &out, const ForwardSums &sums, hipStream_t s);
+
+}  // namespace msd

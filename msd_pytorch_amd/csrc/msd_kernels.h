@@ -3,9 +3,28 @@
 
 #include "msd_common.h"
 
+#include <atomic>
+
 struct msd_adam_param;
 
 namespace msd {
+
+// A kernel that asks for more than 64 KB of LDS needs an attribute set once per device (it
+// stays); launches after the first, also ones recorded into a graph, go without the call.
+struct LargeLds {
+    std::atomic<uint64_t> asked{0};
+    hipError_t allow(const void *kernel, int bytes)
+    {
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess) return e;
+        const uint64_t bit = dev >= 0 && dev < 64 ? (uint64_t)1 << dev : 0;
+        if (asked.load(std::memory_order_acquire) & bit) return hipSuccess;
+        e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+        if (e == hipSuccess) asked.fetch_or(bit, std::memory_order_release);
+        return e;
+    }
+};
 
 // Upper bound on the number of partial-sum rows of the weight/bias gradient
 // reduction (one row per workgroup of the first pass).
@@ -72,6 +91,7 @@ enum Knob {
     kKnobFwdVec2d, kKnobFwdVec3d, kKnobFwdSplit, kKnobFwdRows2d, kKnobBwdkRows, kKnobBlockFuse,
     kKnobBlockDefer, kKnobBwdkInterleave, kKnobBlockSnake, kKnobFwdClass3d, kKnobFwdLattice3d,
     kKnobBlockPair, kKnobBlockTriple, kKnobFinalTiled, kKnobBlockSplit3d, kKnobBlockChainPair, kKnobBwdkFused3d, kKnobBwdxLean1,
+    kKnobFwdGroup,
     kKnobCount
 };
 int knob(Knob k, int dflt);
@@ -116,6 +136,17 @@ hipError_t fast_forward_2d(const Geom &g, bool relu, const View<const float> &x,
                            const View<float> &out, hipStream_t s);
 hipError_t fast_forward_3d(const Geom &g, bool relu, const View<const float> &x, const float *k, const float *bias,
                            const View<float> &out, hipStream_t s);
+
+// The 2D forward pass (with ReLU) of a layer whose sums over most of its channels lie ready: z
+// holds three planes [H][W] per output channel, one per row of taps, shifted along x (batch
+// stride zsb); plane ky counts for output row y from its row y + (ky - 1) dil.  g.C channels
+// (possibly none) are left, whose weights follow k with kco between output channels.
+struct ForwardSums {
+    const float *z;
+    int64_t zsb, kco;
+};
+hipError_t fast_forward_sums_2d(const Geom &g, const View<const float> &x, const float *k, const float *bias,
+                                const View<float> &out, hipStream_t s, const ForwardSums &sums);
 
 inline bool fast_forward_supported(const Geom &g, const View<const float> &x, const View<float> &out)
 {

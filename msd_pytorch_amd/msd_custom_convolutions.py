@@ -413,8 +413,13 @@ def block_forward(stack, c_in, dilations, bias, weights):
     fn = "block_forward"
     dilations = _check_block(fn, stack, c_in, dilations, bias, weights)
     bias = bias.contiguous()
-    _call("msd_block_forward", stack.device, *_block_head(stack, c_in, dilations, weights), *_view(stack),
-          _ptr_array(weights), ctypes.c_void_p(bias.data_ptr()), _stream(stack))
+    head = _block_head(stack, c_in, dilations, weights)
+    need = _native.load().msd_block_forward_workspace_bytes(head[0], head[1], head[2], c_in, head[4], head[5], head[6])
+    if need < 0:
+        _fail(fn, "invalid block geometry")
+    ws = torch.empty(max(int(need), 8), dtype=torch.uint8, device=stack.device) if need else None
+    _call("msd_block_forward_ws", stack.device, *head, *_view(stack), _ptr_array(weights),
+          ctypes.c_void_p(bias.data_ptr()), ctypes.c_void_p(ws.data_ptr() if need else 0), int(need), _stream(stack))
 
 
 def block_backward(stack, grads, c_in, dilations, weights, grad_weights, grad_bias, need_input_grad):

@@ -1,0 +1,36 @@
+"""Groups of layers of a 2D block on the matrix cores, forced on small images, against the oracle."""
+import pytest
+
+from parity import check_block
+from test_knobs_gpu import tuning
+
+pytestmark = pytest.mark.gpu
+
+# Edges: rows of less than a wave, of whole waves, of every tail length, of 16 waves, cut into
+# segments (also short last ones), several teams in a workgroup; a last group of one to seven
+# layers; channels in front that are a multiple of four, one more, one less, more than the 128
+# whose weights fit the table at once; dilations up to the image, folds on both sides; two
+# channels per layer; several images.
+BLOCKS = [
+    # (size, c_in, width, depth, batch, dilations)
+    ((33, 64), 1, 1, 15, 1, None),
+    ((10, 40), 4, 1, 9, 2, [1, 10, 3]),
+    ((12, 129), 2, 1, 8, 1, [7, 1, 12, 2]),
+    ((9, 131), 3, 1, 14, 2, [9, 3, 1]),
+    ((7, 1021), 1, 1, 9, 1, [7, 1, 2]),
+    ((11, 1024), 5, 1, 16, 1, [11, 10, 1, 5]),
+    ((6, 1500), 1, 1, 8, 1, [6, 1, 3]),
+    ((130, 1100), 2, 1, 3, 1, [128, 1, 100]),
+    ((5, 2048), 2, 2, 6, 1, [5, 1, 2, 3]),
+    ((13, 333), 2, 2, 8, 2, [1, 10, 4]),
+    ((8, 70), 127, 1, 9, 1, [1, 2, 8]),
+    ((8, 64), 140, 2, 4, 1, [1, 2]),
+]
+
+
+@pytest.mark.parametrize("case", BLOCKS, ids=lambda c: "x".join(map(str, c[0])) + "-c%d-w%d-d%d-B%d" % c[1:5])
+def test_block_in_layer_groups(case):
+    size, c_in, width, depth, batch, dilations = case
+    dilations = [(dilations or range(1, 11))[i % len(dilations or range(1, 11))] for i in range(depth)]
+    with tuning({"fwd.group": 1}):
+        check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=41)
