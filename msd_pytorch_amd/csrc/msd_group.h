@@ -69,4 +69,19 @@ bool group_finish_supported_2d(const Geom &g, const View<const float> &x, const 
 hipError_t group_finish_2d(const Geom &g, const View<const float> &x, const float *k, const float *bias,
                            const View<float> &out, const ForwardSums &sums, hipStream_t s);
 
+// Backward pass of a group over the channels [0, g.C) of the stack x: the first `update` channels of
+// grads get grad_input (masked with their activations from `mask_from` on), gk[o] the weight gradients
+// of output o's channels[o] input channels, gb the bias gradients.  The outputs' gradients are the
+// channels from `first` on.  ws: group_pull_floats_2d floats.
+int64_t group_pull_floats_2d(int64_t batch, int64_t H, int64_t W, int64_t channels);
+bool group_pull_supported_2d(const Geom &g, const View<const float> &x, const View<float> &gx);
+hipError_t group_pull_2d(const Geom &g, const View<const float> &x, const group2d::Outputs &out, int update, int mask_from,
+                         const View<float> &grads, int first, const int *channels, float *const *gk, float *gb,
+                         float *ws, bool reverse, hipStream_t s);
+
+// Completes the gradient of the `width` channels from `channel` on: adds what the outputs right
+// above them (`above`, their weights of these channels) contribute, and applies the ReLU mask.
+hipError_t group_finish_back_2d(const Geom &g, const View<const float> &x, const View<float> &grads, int channel, int width,
+                                const group2d::Outputs &above, hipStream_t s);
+
 }  // namespace msd

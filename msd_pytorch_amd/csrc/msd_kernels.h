@@ -92,6 +92,7 @@ enum Knob {
     kKnobBlockDefer, kKnobBwdkInterleave, kKnobBlockSnake, kKnobFwdClass3d, kKnobFwdLattice3d,
     kKnobBlockPair, kKnobBlockTriple, kKnobFinalTiled, kKnobBlockSplit3d, kKnobBlockChainPair, kKnobBwdkFused3d, kKnobBwdxLean1,
     kKnobFwdGroup,
+    kKnobBwdGroup,
     kKnobCount
 };
 int knob(Knob k, int dflt);

@@ -34,3 +34,31 @@ def test_block_in_layer_groups(case):
     dilations = [(dilations or range(1, 11))[i % len(dilations or range(1, 11))] for i in range(depth)]
     with tuning({"fwd.group": 1}):
         check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=41)
+
+
+# The backward pass works in tiles of 32 voxels (the last one of a row moved left), blocks of 16
+# channels and chunks of at most 112: rows of one tile, of one voxel more, of every remainder modulo
+# four; channels below, at and past a block and a chunk; three groups and a rest; dilations up to
+# the image (both mirrors at once); more tiles than waves.
+BACKWARD = [
+    ((33, 32), 1, 1, 15, 1, None),
+    ((5, 33), 4, 1, 9, 2, [1, 5, 3]),
+    ((12, 66), 9, 1, 8, 1, [7, 1, 12, 2]),
+    ((9, 95), 3, 1, 24, 2, [9, 3, 1]),
+    ((40, 132), 16, 1, 7, 1, [40, 33, 1, 16]),
+    ((32, 35), 2, 1, 8, 1, [32, 31, 30]),
+    ((7, 1021), 105, 1, 14, 1, [7, 1, 2]),
+    ((6, 64), 226, 1, 8, 1, [6, 1, 3]),
+    ((13, 333), 2, 2, 8, 2, [1, 10, 4]),
+    ((5, 40), 122, 2, 4, 1, [1, 2]),
+    ((300, 320), 1, 1, 9, 1, None),
+]
+
+
+@pytest.mark.parametrize("case", BACKWARD, ids=lambda c: "x".join(map(str, c[0])) + "-c%d-w%d-d%d-B%d" % c[1:5])
+@pytest.mark.parametrize("input_grad", [True, False])
+def test_block_backward_in_layer_groups(case, input_grad):
+    size, c_in, width, depth, batch, dilations = case
+    dilations = [(dilations or range(1, 11))[i % len(dilations or range(1, 11))] for i in range(depth)]
+    with tuning({"bwd.group": 1}):
+        check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=43, input_grad=input_grad)
