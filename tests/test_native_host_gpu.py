@@ -148,3 +148,22 @@ def test_prediction_without_gradients_equals_the_differentiable_pass(ndim, size)
         got = model.net(x)
     want = model.net(x)
     assert want.requires_grad and torch.equal(got, want.detach())
+
+
+@pytest.mark.parametrize("ndim,size,depth,width", [(2, (512, 512), 9, 1), (2, (256, 1024), 4, 2), (3, (64, 64, 64), 4, 1)])
+def test_planes_of_whole_64_kilobytes(ndim, size, depth, width):
+    """The native calls keep the channels of such stacks a little apart; the general path does not.
+    The launches and their order of summation are the same."""
+    native, general = _models("L2", ndim, depth, width, 2, 2)
+    general._native_step = lambda: False
+    gen = torch.Generator().manual_seed(11)
+    x, t = torch.randn(2, 2, *size, generator=gen).cuda(), torch.randn(2, 2, *size, generator=gen).cuda()
+    with torch.no_grad():
+        got = native.net(x)
+    assert torch.equal(got, general.net(x).detach())
+    for m in (native, general):
+        m.learn(x, t)
+    assert native.loss.grad_fn is None and general.loss.grad_fn is not None
+    assert rel_err(native.output, general.output) <= 1e-5
+    for p, q in zip(native.msd.parameters(), general.msd.parameters()):
+        assert rel_err(p.grad, q.grad) <= 1e-4
