@@ -133,7 +133,28 @@ def make_model(name, torch):
     return model
 
 
-def algorithmic_work(name, fused, paired=False, triple_from=32, kpairs=False, chainpairs=False):
+def grouped_layers(c_in, depth, width):
+    """The layers that the library takes in groups of up to seven outputs on the matrix cores (2D,
+    one or two channels per layer): {first layer: layers} of the forward pass (from the bottom, where
+    at least 12 channels, 6 with two per layer, lie in front) and of the backward pass (from the
+    top, over at least 4 channels)."""
+    most, forward, backward = 7 // width, {}, {}
+    i = 0
+    while i < depth:
+        n = min(most, depth - i) if c_in + width * i >= (6 if width > 1 else 12) else 0
+        if n >= 2:
+            forward[i] = n
+        i += n if n >= 2 else 1
+    i = depth - 1
+    while i >= 0:
+        n = sum(1 for j in range(min(most, i + 1)) if c_in + width * (i - j) >= 4)
+        if n >= 2:
+            backward[i - n + 1] = n
+        i -= n if n >= 2 else 1
+    return forward, backward
+
+
+def algorithmic_work(name, fused, paired=False, triple_from=32, kpairs=False, chainpairs=False, groups=({}, {})):
     """Per-step algorithmic bytes and flops of each kernel class, fp32, per layer with C input
     and w output channels over N voxels and K = 9 or 27 taps:
     bytes: forward (C + w) N 4, backward_x (2C + 2w) N 4, backward_k+bias (C + 2w) N 4, the fused
@@ -149,6 +170,11 @@ def algorithmic_work(name, fused, paired=False, triple_from=32, kpairs=False, ch
     one pass over the c channels below all n layers with the layers as its n output channels,
     (3c + 2n) N 4 bytes: what that algorithm has to move, a half to a third of the per-layer
     figure.  The per-layer figure is returned as well, under "backward_xkb_per_layer".
+    `groups` (grouped_layers): the forward pass of n layers over the c channels in front of them is
+    one read of these and three planes per output, (c + 3 n w) N 4 bytes, then per layer its planes, the
+    j w channels that the group has added and its outputs, (4 + j) w N 4; the backward pass is per
+    layer but the top one its channels' gradient (read, written, activation) and the outputs above,
+    (3 + j) w N 4, then one pass (3 c + (2 n - 1) w) N 4.
     `kpairs`: the library runs a 3D block of width 1 as a chain of backward_x launches with the
     weight and bias gradients of two layers per pass over x beside it (layers depth-1 and depth-2,
     ... down to 1 and 0; an odd lowest layer alone): a pair reads the C input channels of its
@@ -166,9 +192,18 @@ def algorithmic_work(name, fused, paired=False, triple_from=32, kpairs=False, ch
     nbytes = {"forward": 0, "backward_x": 3 * width * n * 4, "backward_kb": 0, "backward_xkb": 0,
               "backward_xkb_per_layer": 0}
     flops = {"forward": 0, "backward_x": 0, "backward_kb": 0, "backward_xkb": 0}
-    in_pair = set()
+    in_pair, in_group = set(), set()
+    for i, m in groups[0].items():
+        c = c_in + width * i
+        in_group.update(range(i, i + m))
+        nbytes["forward"] += (c + 3 * m * width + sum((4 + j) * width for j in range(m))) * n * 4 + m * width * c * K * 4
+    for i, m in groups[1].items():
+        c = c_in + width * i
+        in_pair.update(range(i, i + m))
+        nbytes["backward_xkb"] += (3 * c + (2 * m - 1) * width + sum((3 + j) * width for j in range(1, m))) * n * 4 \
+            + 2 * m * width * c * K * 4
     if fused and paired:
-        i = depth - 1
+        i = min(groups[1], default=depth) - 1
         while i - 1 > 0:
             first = c_in + width * i             # channels that layer i reads
             m = 3 if triple_from is not None and i - 2 > 0 and first - 2 >= max(triple_from, 1) else 2
@@ -182,7 +217,8 @@ def algorithmic_work(name, fused, paired=False, triple_from=32, kpairs=False, ch
         C = c_in + width * i
         wts = width * C * K * 4
         op = 2 * C * width * K * n
-        nbytes["forward"] += (C + width) * n * 4 + wts
+        if i not in in_group:
+            nbytes["forward"] += (C + width) * n * 4 + wts
         flops["forward"] += op
         if i > 0 and fused:
             per_layer = (3 * C + 2 * width) * n * 4 + 2 * wts
@@ -328,7 +364,8 @@ def measure(name, args, lib, torch, steps=None, warmup=None, cpu=True):
 
     if not args.no_kernel_timing:
         totals = kernel_times(lib, torch, lambda: [eager_step() for _ in range(args.steps)])
-        # 2D blocks of width 1 run their layers two or three at a time in the backward pass
+        # 2D blocks run their layers in groups of up to seven outputs (fwd.group, bwd.group: 0 never); what
+        # is left, or without groups all layers of width 1, two or three at a time in the backward pass
         # (block.pair; block.triple: from how many shared channels three, 0 never, 32 by default)
         tuned = dict(kv.replace(" ", "").split("=") for kv in args.tune)
         paired = ndim == 2 and width == 1 and tuned.get("block.pair") != "0" and tuned.get("block.fuse") != "0"
@@ -339,7 +376,14 @@ def measure(name, args, lib, torch, steps=None, warmup=None, cpu=True):
         # on one stream, so the classes' times add up to more than the step's backward pass
         split3d = ndim == 3 and width == 1 and totals["backward_xkb"][1] == 0 and \
             0 < totals["backward_kb"][1] // args.steps < depth
+        forward, backward = grouped_layers(c_in, depth, width) if ndim == 2 and width <= 2 else ({}, {})
+        if tuned.get("fwd.group") == "0":
+            forward = {}
+        if tuned.get("bwd.group") == "0" or tuned.get("block.fuse") == "0" or "block.pair" in tuned \
+                or "block.triple" in tuned:
+            backward = {}
         bytes_per_step, flops_per_step, _ = algorithmic_work(name, totals["backward_xkb"][1] > 0, paired, triple_from,
+                                                             groups=(forward, backward),
                                                              kpairs=split3d,
                                                              chainpairs=split3d and tuned.get("block.chainpair") != "0")
         kernels = {}
