@@ -25,10 +25,11 @@ HBM_PEAK_GBS = 8000.0
 # fp32 peak of MI355X (matrix cores, or packed vector instructions); plain (non-packed) vector
 # fp32, which the build rules leave to the forward kernel's multiply-adds, peaks at half of it
 FP32_PEAK_TFLOPS = 157.3
-PIPE = {"forward": "fp32 VALU, non-packed (78.6 TFLOP/s of the 157.3 peak)",
+PIPE = {"forward": "fp32 VALU, non-packed (78.6 TFLOP/s of the 157.3 peak); 2D layer groups: fp32 MFMA 16x16x4",
         "backward_x": "fp32 VALU, non-packed (78.6 TFLOP/s of the 157.3 peak)",
         "backward_kb": "fp32 MFMA 16x16x4",
-        "backward_xkb": "fp32 MFMA 16x16x4 (weight gradient) + fp32 VALU (input gradient), half of the flops each"}
+        "backward_xkb": "fp32 MFMA 16x16x4 (weight gradient) + fp32 VALU (input gradient), half of the flops each; "
+                        "2D layer groups: both on the MFMA"}
 
 # kernel families (as named in the profile summaries) whose HBM traffic belongs to a class
 FAMILIES = {"forward": ("fwd_lattice",), "backward_xkb": ("bwd_rows_fused", "bwd_one_channel", "reduce_columns"),

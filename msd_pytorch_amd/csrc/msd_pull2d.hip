@@ -14,10 +14,11 @@
 // Bound by the matrix cores and by memory about alike: per channel and voxel 128 multiply-adds
 // (30 us per 16 channels at 1024 x 1024 and the clock they run at) and 12 bytes (40 us at the rate of
 // a device copy), for seven layers at once, where passes of three layers move 28.  Seven layers at
-// 1024 x 1024: 120 us over 20 channels, 186 over 48, 455 over 104 (2.9 TB/s); three layers per pass
-// of bwd_rows_fused took 112 (32 channels), 157 (64) and 305 (over 96), two and a third of them for seven.
-// A step at 1024 x 1024, depth 100: 8.5 -> 6.7 ms; 4 x 512 x 512: 8.0 -> 6.2; 2048 x 2048, two
-// channels per layer, depth 200: 509 -> 319.
+// 1024 x 1024: 120 us over 20 channels, 186 over 48, 455 over 104 (2.9 TB/s; 118, 164 and 372 with the
+// planes kept apart as the models do, csrc/host); three layers per pass of bwd_rows_fused took 112 (32
+// channels), 157 (64) and 305 (over 96), two and a third of them for seven.
+// A step at 1024 x 1024, depth 100: 8.5 -> 6.7 ms (6.3 with the planes apart); 4 x 512 x 512: 8.0 -> 6.2;
+// 2048 x 2048, two channels per layer, depth 200: 509 -> 319 (274).
 //
 // What it took to get there: a workgroup holds at most 64 channels (their sums, and a set of
 // registers for x and grad_input of each block, asked for a whole tile ahead; 112 channels with two
@@ -281,8 +282,14 @@ __global__ __launch_bounds__(kPullWaves *kWave, 2) void pull_rows(const PullArgs
         const Place next = locate(tile + stride);
         const int skip = here.own0 - here.x0;     // voxels of the tile that belong to the one before
         f32x4_t acc[kTiles];
-        auto compute = [&](int cb, const f32x4_t(&xv)[2], f32x4_t(&gv)[2]) {
+        auto compute = [&](int cb, f32x4_t(&xv)[2], f32x4_t(&gv)[2]) {
             const int ch0 = c0 + cb * 16;
+            if (skip > 0) {                       // uniform: an infinity there belongs to the other tile
+#pragma unroll
+                for (int s = 0; s < 2; s++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) xv[s][e] = 16 * s + 4 * q + e >= skip ? xv[s][e] : 0.f;
+            }
 #pragma unroll
             for (int t = 0; t < kTiles; t++) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
             if (cb < blocks) {                    // uniform

@@ -1,5 +1,6 @@
 """Groups of layers of a 2D block on the matrix cores, forced on small images, against the oracle."""
 import pytest
+import torch
 
 from parity import check_block
 from test_knobs_gpu import tuning
@@ -62,3 +63,23 @@ def test_block_backward_in_layer_groups(case, input_grad):
     dilations = [(dilations or range(1, 11))[i % len(dilations or range(1, 11))] for i in range(depth)]
     with tuning({"bwd.group": 1}):
         check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=43, input_grad=input_grad)
+
+
+def test_an_infinity_meets_its_own_voxels_only():
+    """The last tile of a row repeats voxels of the one before (here 8 to 31): what they hold counts once."""
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator().manual_seed(3)
+    c_in, depth, size = 4, 8, (6, 40)
+    stack = torch.rand(1, c_in + depth, *size, generator=gen).cuda() + 0.1     # every ReLU open
+    stack[0, 1, 3, 20] = float("inf")
+    gradient = torch.randn(1, c_in + depth, *size, generator=gen).cuda()
+    weights = [torch.randn(1, c_in + i, 3, 3, generator=gen).cuda() for i in range(depth)]
+    found = []
+    for setting in (0, 1):
+        gk, gb = [torch.zeros_like(w) for w in weights], torch.zeros(depth).cuda()
+        with tuning({"bwd.group": setting}):
+            cc.block_backward(stack, gradient.clone(), c_in, [1, 2, 3, 1, 2, 3, 1, 2], weights, gk, gb, True)
+        found.append(torch.cat([k.flatten() for k in gk]))
+    assert torch.isinf(found[0]).any()
+    assert torch.equal(torch.isnan(found[0]), torch.isnan(found[1]))
+    assert torch.equal(torch.isinf(found[0]), torch.isinf(found[1]))
