@@ -305,6 +305,9 @@ __global__ __launch_bounds__(kPullWaves *kWave, 2) void pull_rows(const PullArgs
                         for (int t = 0; t < kTiles; t++)
                             acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[t][e], xv[s][e], acc[t], 0, 0, 0);
                 }
+                // Added to grad_input in two halves: a chain of 63 products that started from it would round
+                // each of them to its size (2.7 times the error of passes of three layers, now 0.8 times).
+                f32x4_t d[2];
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
                     const f32x4_t w = table[(cb * 4 + j) * kWave + lane];
@@ -314,10 +317,16 @@ __global__ __launch_bounds__(kPullWaves *kWave, 2) void pull_rows(const PullArgs
 #pragma unroll
                         for (int e = 0; e < 4; e++) av[s][e] = T[(16 * j + 4 * q + e) * kRowFloats + 16 * s + n];
 #pragma unroll
+                    for (int s = 0; s < 2; s++)
+                        if (j % 2 == 0) d[s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
                     for (int e = 0; e < 4; e++)
 #pragma unroll
                         for (int s = 0; s < 2; s++)
-                            gv[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s][e], w[e], gv[s], 0, 0, 0);
+                            d[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s][e], w[e], d[s], 0, 0, 0);
+#pragma unroll
+                    for (int s = 0; s < 2; s++)
+                        if (j % 2 == 1) gv[s] += d[s];
                 }
                 if (ch0 + 16 > a.mask_from) {     // uniform
                     int nn = n;
@@ -440,15 +449,25 @@ __global__ __launch_bounds__(1024) void sum_group(const SumArgs a, const float *
         p = part + (int64_t)a.chunks.first_wg(chunk) * a.stride + (blk - a.chunks.first_block(chunk)) * 1024 + col % 1024;
         stride = a.stride;
     }
-    float s = 0.f;
-#pragma unroll 8
-    for (int r = wave; r < rows; r += 16) s += p[r * stride];
-    lds[wave * kWave + lane] = s;
+    float part_sum[4] = {0.f, 0.f, 0.f, 0.f};     // (short chains, then trees: these are the largest sums)
+    for (int r = wave; r < rows; r += 128) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = p[min(r + 16 * i, rows - 1) * stride];
+#pragma unroll
+        for (int i = 0; i < 8; i++) part_sum[i % 4] += r + 16 * i < rows ? v[i] : 0.f;
+    }
+    lds[wave * kWave + lane] = (part_sum[0] + part_sum[1]) + (part_sum[2] + part_sum[3]);
     __syncthreads();
     if (wave != 0) return;
-    s = 0.f;
+    float tree[16];
 #pragma unroll
-    for (int w = 0; w < 16; w++) s += lds[w * kWave + lane];
+    for (int w = 0; w < 16; w++) tree[w] = lds[w * kWave + lane];
+#pragma unroll
+    for (int w = 8; w > 0; w /= 2)
+#pragma unroll
+        for (int i = 0; i < w; i++) tree[i] += tree[i + w];
+    const float s = tree[0];
     if (bias) {
         if (lane < a.n) a.gb[lane] += s;
         return;
@@ -530,10 +549,15 @@ __global__ __launch_bounds__(256) void finish_back(const FinishArgs a, const flo
     }
 #pragma unroll
     for (int c = 0; c < NOUT; c++) {
+        float all = 0.f;                          // (output by output, and added to grad_input last: see pull_rows)
 #pragma unroll
-        for (int o = 0; o < NQ; o++)
+        for (int o = 0; o < NQ; o++) {
+            float one = 0.f;
 #pragma unroll
-            for (int t = 0; t < kTaps; t++) sum[c] += a.k[o][c * kTaps + t] * A[o][t];
+            for (int t = 0; t < kTaps; t++) one += a.k[o][c * kTaps + t] * A[o][t];
+            all += one;
+        }
+        sum[c] += all;
         const float v[1] = {0.f < m[c] ? sum[c] : 0.f};
         if (u0 < a.W) store_global_vec<1>(img, (uint32_t)c * plane + here, v);
     }
