@@ -423,8 +423,8 @@ std::optional<std::pair<Tensor, Tensor>> train_step(const Tensor &x, const Tenso
 // False (and nothing has happened) for a state that the kernel does not take.
 // ---------------------------------------------------------------------------
 
-bool adam_step(const std::vector<Tensor> &params, const std::vector<py::dict> &states, double lr, double beta1,
-               double beta2, double eps)
+bool adam_step(const std::vector<Tensor> &params, const py::list &states, double lr, double beta1, double beta2,
+               double eps)
 {
     static PyObject *const k_step = PyUnicode_InternFromString("step");
     static PyObject *const k_avg = PyUnicode_InternFromString("exp_avg");
@@ -440,8 +440,9 @@ bool adam_step(const std::vector<Tensor> &params, const std::vector<py::dict> &s
         const Tensor &p = params[i];
         const Tensor &g = p.grad();
         if (!g.defined()) continue;               // torch's optimiser passes it over as well
-        PyObject *ps = PyDict_GetItem(states[i].ptr(), k_step), *pa = PyDict_GetItem(states[i].ptr(), k_avg),
-                 *pq = PyDict_GetItem(states[i].ptr(), k_sq);
+        PyObject *const entry = PyList_GET_ITEM(states.ptr(), i);
+        if (!PyDict_Check(entry)) return false;
+        PyObject *ps = PyDict_GetItem(entry, k_step), *pa = PyDict_GetItem(entry, k_avg), *pq = PyDict_GetItem(entry, k_sq);
         if (!ps || !pa || !pq || !THPVariable_Check(ps) || !THPVariable_Check(pa) || !THPVariable_Check(pq)) return false;
         const Tensor &step = THPVariable_Unpack(ps), &avg = THPVariable_Unpack(pa), &sq = THPVariable_Unpack(pq);
         for (const Tensor *t : {&p, &g, &avg, &sq})

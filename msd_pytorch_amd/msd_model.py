@@ -290,8 +290,6 @@ class MSDModel:
         if not self._native_adam():
             self.optimizer.step()
 
-    _adam_states = None                           # (optimiser state, parameters, their entries)
-
     def _native_adam(self):
         opt = self.optimizer
         # (a learning-rate scheduler puts a step of its own on the instance)
@@ -309,13 +307,16 @@ class MSDModel:
             return False
         if not group["capturable"] and torch.cuda.is_current_stream_capturing():
             return False                          # torch's step raises
-        seen = self._adam_states
-        if seen is None or seen[0] is not state or seen[1] is not params or len(state) != len(seen[2]) \
-                or len(params) != len(seen[2]):
-            if len(state) != len(params) or not all(p in state for p in params):
-                return False                      # the first step makes the state
-            seen = self._adam_states = (state, params, [state[p] for p in params])
-        return _native.host().adam_step(params, seen[2], group["lr"], *group["betas"], group["eps"])
+        # the entries that the optimiser holds now: they may be dropped or replaced between two steps
+        if len(state) != len(params):
+            return False                          # the first step makes the state
+        if all(map(operator.is_, state, params)):   # (in order, as torch makes them: no tensor is hashed)
+            entries = list(state.values())
+        elif all(p in state for p in params):
+            entries = [state[p] for p in params]
+        else:
+            return False
+        return _native.host().adam_step(params, entries, group["lr"], *group["betas"], group["eps"])
 
     def forward(self, input=None, target=None):
         """Loss of one (input, target) pair; arguments left out keep their last value."""

@@ -293,3 +293,62 @@ def test_package_exports():
     for name in ("MSDRegressionModel", "MSDSegmentationModel", "MSDModule", "MSDBlock2d", "MSDBlock3d",
                  "ImageDataset", "ImageStack", "InputError"):
         assert hasattr(msd_pytorch_amd, name)
+
+
+class _OnGpu(torch.nn.Parameter):
+    is_cuda = True                                 # (what the step asks before it hands the tensors on)
+
+
+def _one_launch_adam(monkeypatch):
+    """A model that is an Adam over three parameters, with the launch replaced by a record of its states."""
+    from msd_pytorch_amd import _native
+    from msd_pytorch_amd.msd_model import MSDModel
+    calls = []
+
+    class Host:
+        @staticmethod
+        def adam_step(params, states, *settings):
+            calls.append(list(states))
+            return True
+
+    monkeypatch.setattr(_native, "host", lambda: Host)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    params = [_OnGpu(torch.full((n,), 0.5)) for n in (1, 3, 4)]
+    model = MSDModel.__new__(MSDModel)
+    model.optimizer = torch.optim.Adam(params)
+
+    def step():
+        for p in params:
+            p.grad = torch.ones_like(p)
+        before = len(calls)
+        model._optimizer_step()
+        return len(calls) > before
+
+    return model.optimizer, params, calls, step
+
+
+def test_optimiser_step_uses_the_state_that_is_there_now(monkeypatch):
+    opt, params, calls, step = _one_launch_adam(monkeypatch)
+    assert not step()                              # the first step makes the state
+    assert step() and step()
+
+    def emptied():
+        opt.state.clear()
+
+    def one_less():
+        del opt.state[params[1]]
+
+    def one_replaced():
+        opt.state[params[0]] = {k: v.clone() for k, v in opt.state[params[0]].items()}
+
+    def reloaded():
+        opt.load_state_dict(opt.state_dict())
+
+    def another():
+        opt.state = type(opt.state)(opt.state.default_factory, reversed(list(opt.state.items())))
+
+    for change in (emptied, one_less, one_replaced, reloaded, another):
+        change()
+        step()
+        assert step(), change.__name__
+        assert all(a is opt.state[p] for a, p in zip(calls[-1], params)), change.__name__

@@ -167,3 +167,69 @@ def test_planes_of_whole_64_kilobytes(ndim, size, depth, width):
     assert rel_err(native.output, general.output) <= 1e-5
     for p, q in zip(native.msd.parameters(), general.msd.parameters()):
         assert rel_err(p.grad, q.grad) <= 1e-4
+
+
+def _optimised(dtype, capturable, count, seed):
+    """A model that is nothing but an Adam over `count` parameters, a thousand steps old."""
+    from msd_pytorch_amd.msd_model import MSDModel
+    gen = torch.Generator().manual_seed(seed)
+    sizes = [1, 3, 63, 64, 65, 257, 1000, 4099]
+
+    def draw(n):
+        return torch.randn(n, generator=gen, dtype=dtype).cuda()
+
+    params = [torch.nn.Parameter(0.01 * draw(sizes[i % len(sizes)])) for i in range(count)]
+    model = MSDModel.__new__(MSDModel)
+    model.optimizer = torch.optim.Adam(params, lr=2e-3, betas=(0.8, 0.99), eps=1e-6, capturable=capturable)
+    for p in params:
+        step = torch.tensor(1000.0)
+        model.optimizer.state[p] = {"step": step.cuda() if capturable else step, "exp_avg": 1e-3 * draw(p.numel()),
+                                    "exp_avg_sq": 1e-6 * (0.1 + draw(p.numel()).abs())}
+    return model, params, [[1e-3 * draw(p.numel()) for p in params] for _ in range(5)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("capturable", [False, True])
+@pytest.mark.parametrize("count", [1, 13, 130])    # 130: more than one launch takes
+def test_the_optimiser_in_one_launch_is_torchs(dtype, capturable, count):
+    """Moments of a thousand steps, so that an update is a value and not a sign; then the state is
+    dropped, replaced in part and as a whole.  Both sides do the same arithmetic in some order, so
+    that they are a few roundings apart; but torch forms 1 - beta ** step of a step on the device in 32
+    bits whatever the type, which is 6e-8 of the 0.01 of a first step, or 6e-6 of the update."""
+    tol = 1e-6 if dtype == torch.float32 else 1e-14
+    update_tol = max(tol, 1e-5 if capturable else 0.0)
+    native, ours, grads = _optimised(dtype, capturable, count, 9)
+    torchs, theirs, _ = _optimised(dtype, capturable, count, 9)
+    launched = []
+
+    def drop(model, params, which):
+        state = model.optimizer.state
+        if which == 2:
+            state.clear()
+        elif which == 3:
+            del state[params[0]]
+        elif which == 4:
+            state[params[-1]] = {k: v.clone() for k, v in state[params[-1]].items()}
+
+    for i, step in enumerate(grads):
+        for model, params in ((native, ours), (torchs, theirs)):
+            drop(model, params, i)
+            before = [p.detach().clone() for p in params]
+            for p, g in zip(params, step):
+                p.grad = g.clone()
+            if model is native:
+                launched.append(model._native_adam())
+                if not launched[-1]:
+                    model.optimizer.step()
+            else:
+                model.optimizer.step()
+        for p, q, old in zip(ours, theirs, before):
+            state, want = native.optimizer.state[p], torchs.optimizer.state[q]
+            assert float(state["step"]) == float(want["step"])
+            assert rel_err(state["exp_avg"], want["exp_avg"]) <= tol
+            assert rel_err(state["exp_avg_sq"], want["exp_avg_sq"]) <= tol
+            moved = float((q.detach() - old).abs().max())
+            assert float((p - q).detach().abs().max()) <= tol * float(q.detach().abs().max()) + update_tol * moved
+            assert moved > 0
+    # torch makes what is missing
+    assert launched == [True, True, False, False, True]
