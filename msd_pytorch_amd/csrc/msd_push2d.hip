@@ -85,7 +85,7 @@ __global__ __launch_bounds__(kMaxWaves *kWave) void push_rows(PushArgs a, const 
         return p;
     };
     // Step st of the chunk of cn channels from c0 on stands for the channels c0 + 4 st + q; past the
-    // last channel the lanes repeat it (its weights are zero there, its values are finite).
+    // last channel the lanes repeat it, and its repetitions are cleared before they are used.
     auto request = [&](const Place &p, int c0, int cn, int st, float (&d)[4]) {
         const int s = min(st, (cn + 3) / 4 - 1);
         const uint64_t cb = p.base + (uint64_t)(c0 + 4 * s) * (uint64_t)a.xsc * 4u;
@@ -146,6 +146,11 @@ __global__ __launch_bounds__(kMaxWaves *kWave) void push_rows(PushArgs a, const 
 #pragma unroll
                     for (int u = 0; u < kAhead; u++) {
                         if (s0 + u >= steps) break;                 // uniform
+                        if (4 * (s0 + u) + 4 > cn) {                // uniform: an infinity times a weight of zero is NaN
+                            const bool past = 4 * (s0 + u) + q >= cn;
+#pragma unroll
+                            for (int j = 0; j < 4; j++) set[half][u][j] = past ? 0.f : set[half][u][j];
+                        }
                         const f32x4_t w = table[(s0 + u) * kWave + lane];
 #pragma unroll
                         for (int j = 0; j < 4; j++)

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from parity import check_block
+from parity import check_block, rel_err
 from test_knobs_gpu import tuning
 
 pytestmark = pytest.mark.gpu
@@ -83,3 +83,26 @@ def test_an_infinity_meets_its_own_voxels_only():
     assert torch.isinf(found[0]).any()
     assert torch.equal(torch.isnan(found[0]), torch.isnan(found[1]))
     assert torch.equal(torch.isinf(found[0]), torch.isinf(found[1]))
+
+
+@pytest.mark.parametrize("c_in", [4, 5, 6, 7, 129])
+def test_an_infinity_in_front_of_a_forward_group_stays_one(c_in):
+    """A step of the pass takes four channels; the last one's repetitions must not meet it."""
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator().manual_seed(5)
+    depth, size = 9, (6, 40)
+    image = torch.rand(1, c_in, *size, generator=gen).cuda()
+    image[0, c_in - 1, 2, 17] = float("inf")
+    weights = [(torch.rand(1, c_in + i, 3, 3, generator=gen) * 0.1 + 0.01).cuda() for i in range(depth)]
+    found = []
+    for setting in (0, 1):
+        stack = torch.empty(1, c_in + depth, *size, device="cuda")
+        stack[:, :c_in] = image
+        with tuning({"fwd.group": setting}):
+            cc.block_forward(stack, c_in, [1, 2, 3, 1, 2, 3, 1, 2, 3], torch.zeros(depth, device="cuda"), weights)
+        found.append(stack)
+    assert torch.isinf(found[0][:, c_in:]).any() and not torch.isnan(found[0]).any()
+    finite = torch.isfinite(found[0])
+    assert torch.equal(torch.isinf(found[0]), torch.isinf(found[1]))
+    assert torch.equal(finite, torch.isfinite(found[1]))
+    assert rel_err(found[1][finite], found[0][finite]) <= 1e-5
