@@ -120,9 +120,11 @@ class MSDBlock(torch.nn.Module):
         torch.nn.init.uniform_(self.bias, -bound, bound)
 
     def own_weights(self):
-        """The registered weights, in order, for the native calls (None where one is not a
-        parameter of this module at the moment)."""
-        return list(map(self._parameters.get, self.weight_names))
+        """The registered weights, in order, for the native calls; None where one is no parameter
+        of this module at the moment (replicas of nn.DataParallel hold plain tensors, parametrized
+        weights are computed when they are asked for)."""
+        own = list(map(self._parameters.get, self.weight_names))
+        return own if all(w is not None for w in own) else None
 
     def forward(self, input):
         # Look the weights up by attribute on every call: after a device move,

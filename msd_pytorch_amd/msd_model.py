@@ -274,7 +274,10 @@ class MSDModel:
         # the gradients are replaced, which is zero_grad() and backward() for the optimiser of
         # exactly these parameters
         linear, block = self.msd.final_layer.linear, self.msd.msd_block
-        own = [block.bias, *block.own_weights(), linear.weight, linear.bias]
+        weights = block.own_weights()
+        if weights is None:
+            return False
+        own = [block.bias, *weights, linear.weight, linear.bias]
         held = [p for group in self.optimizer.param_groups for p in group["params"]]
         if len(own) != len(held) or not all(map(operator.is_, own, held)):
             return False

@@ -223,9 +223,9 @@ class MSDModule(torch.nn.Module):
                 and linear.bias is not None and not self._hooked():
             # block + final layer as one autograd node (no copy of the stack's gradient)
             block = self.msd_block
-            if not torch.is_grad_enabled() and self.plain_dilations():
-                output = _native.host().net_forward(input, block.bias, block.own_weights(), block.dilations,
-                                                    linear.weight, linear.bias)
+            own = None if torch.is_grad_enabled() or not self.plain_dilations() else block.own_weights()
+            if own is not None:
+                output = _native.host().net_forward(input, block.bias, own, block.dilations, linear.weight, linear.bias)
                 if output is not None:
                     return output
             weights = (getattr(block, f"weight{i}") for i in range(len(block.weights)))
@@ -245,16 +245,16 @@ class MSDModule(torch.nn.Module):
         graph in between.  Returns (loss, output), neither differentiable, or None (nothing has
         been done) where the native step does not apply: see csrc/host/msd_host.cpp."""
         linear, block = self.final_layer.linear, self.msd_block
-        if linear.bias is None or scale_in.bias is None or not self.plain_dilations() or self._hooked():
+        own = block.own_weights()
+        if linear.bias is None or scale_in.bias is None or own is None or not self.plain_dilations() or self._hooked():
             return None
         sw = sb = None
         if scale_out is not None:
             if scale_out.bias is None:
                 return None
             sw, sb = scale_out.weight, scale_out.bias
-        return _native.host().train_step(input, scale_in.weight, scale_in.bias, block.bias, block.own_weights(),
-                                         block.dilations, linear.weight, linear.bias, sw, sb, target,
-                                         cc.LOSS_KINDS[kind])
+        return _native.host().train_step(input, scale_in.weight, scale_in.bias, block.bias, own, block.dilations,
+                                         linear.weight, linear.bias, sw, sb, target, cc.LOSS_KINDS[kind])
 
     def forward_loss(self, input, target, kind, scale=None):
         """(loss, output) of the network followed by an optional frozen 1x1 ``scale`` layer and

@@ -352,3 +352,11 @@ def test_optimiser_step_uses_the_state_that_is_there_now(monkeypatch):
         step()
         assert step(), change.__name__
         assert all(a is opt.state[p] for a, p in zip(calls[-1], params)), change.__name__
+
+
+def test_weights_that_are_not_parameters_are_left_to_the_general_path():
+    block = MSDBlock(2, [1, 2, 3])
+    assert [w is getattr(block, f"weight{i}") for i, w in enumerate(block.own_weights())] == [True] * 3
+    replica = block._replicate_for_data_parallel()
+    replica.weight0 = replica.weight1 = replica.weight2 = torch.zeros(1, 2, 3, 3)
+    assert replica.own_weights() is None

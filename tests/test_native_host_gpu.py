@@ -233,3 +233,32 @@ def test_the_optimiser_in_one_launch_is_torchs(dtype, capturable, count):
             assert moved > 0
     # torch makes what is missing
     assert launched == [True, True, False, False, True]
+
+
+def test_prediction_where_a_weight_is_not_a_parameter_of_its_module():
+    """Replicas of nn.DataParallel hold plain tensors, parametrized modules compute theirs."""
+    (model,) = _models("L2", 2, 4, 1, 2, 1)
+    x, t = torch.rand(2, 2, 24, 40).cuda(), torch.rand(2, 2, 24, 40).cuda()
+    with torch.no_grad():
+        want = model.net(x)
+        replica = torch.nn.parallel.replicate(model.net, [torch.device("cuda", 0)], detach=True)[0]
+        copy = replica[1].msd_block
+        assert copy is not model.msd.msd_block
+        for name in copy.weight_names:             # (a replica on the module's own device keeps its parameters)
+            tensor = copy._parameters.pop(name).detach().clone()
+            setattr(copy, name, tensor)
+        assert torch.equal(replica(x), want)
+
+    class Half(torch.nn.Module):
+        def forward(self, w):
+            return 0.5 * w
+
+    block = model.msd.msd_block
+    original = block.weight1.detach().clone()
+    torch.nn.utils.parametrize.register_parametrization(block, "weight1", Half())
+    with torch.no_grad():
+        block.parametrizations.weight1.original.mul_(2)
+        assert torch.equal(model.net(x), want)
+    model.learn(x, t)                              # (the parameter behind the weight is the one that is trained)
+    assert model.loss.grad_fn is not None
+    assert not torch.equal(0.5 * block.parametrizations.weight1.original.detach(), original)
