@@ -4,8 +4,8 @@
 // whole training step up to the gradients, and the optimiser.
 //
 // Every entry checks its arguments and returns None for whatever it does not take (other types,
-// strides, hooks, tensor subclasses ...); the Python modules then go their general way, which
-// also raises the errors.  Nothing is kept between calls.
+// strides, hooks, tensor subclasses, forward mode, a tracer that is running ...); the Python modules then go
+// their general way, which also raises the errors.  Nothing is kept between calls.
 #include <torch/extension.h>
 
 #include <ATen/core/grad_mode.h>
@@ -14,6 +14,7 @@
 #include <dlfcn.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <string>
 #include <vector>
@@ -54,14 +55,19 @@ int dtype_of(const Tensor &t) { return t.scalar_type() == at::kFloat ? MSD_F32 :
 
 void *stream_on(const at::Device &d) { return c10::hip::getCurrentHIPStream(d.index()).stream(); }
 
-// A dense tensor on the GPU that nothing dispatches on.
+// A dense tensor on the GPU that nothing dispatches on and that carries no tangent of forward mode.
 bool plain(const Tensor &t)
 {
     return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.is_neg() && !t.is_conj() &&
+           !t._fw_grad(0).defined() &&
            !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
                                                      c10::DispatchKey::FuncTorchGradWrapper,
                                                      c10::DispatchKey::Functionalize}));
 }
+// A tracer records autograd functions as calls of their own; it cannot see the calls made here, and
+// their results would become constants of the trace.
+bool traced() { return torch::jit::tracer::isTracing(); }
+
 bool floating(const Tensor &t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kDouble; }
 bool like(const Tensor &t, const Tensor &first)
 {
@@ -171,7 +177,7 @@ class ConvLayer : public torch::autograd::Function<ConvLayer> {
 std::optional<Tensor> conv_layer(const Tensor &x, const Tensor &w, const Tensor &b, const Tensor &out,
                                  int64_t dilation, bool relu)
 {
-    if (!plain(x) || !floating(x) || (x.dim() != 4 && x.dim() != 5) || !like(w, x) || !like(b, x) || !like(out, x) ||
+    if (traced() || !plain(x) || !floating(x) || (x.dim() != 4 && x.dim() != 5) || !like(w, x) || !like(b, x) || !like(out, x) ||
         !kernel_ok(w, x.dim()) || w.size(1) != x.size(1) || b.dim() != 1 || !b.is_contiguous() ||
         b.size(0) != w.size(0) || out.dim() != x.dim() || out.size(0) != x.size(0) || out.size(1) != w.size(0) ||
         out.sizes().slice(2) != x.sizes().slice(2) || !dilation_ok(x, dilation) || x.numel() == 0)
@@ -267,7 +273,7 @@ void pointwise(const Tensor &x, const Tensor &w, const Tensor &b, const Tensor &
 std::optional<Tensor> net_forward(const Tensor &x, const Tensor &bias, const std::vector<Tensor> &weights,
                                   const std::vector<int64_t> &dilations, const Tensor &fw, const Tensor &fb)
 {
-    if (!plain(x) || !floating(x) || (x.dim() != 4 && x.dim() != 5) || x.numel() == 0) return std::nullopt;
+    if (traced() || !plain(x) || !floating(x) || (x.dim() != 4 && x.dim() != 5) || x.numel() == 0) return std::nullopt;
     Block block;
     if (!block.set(x, bias, weights, dilations) || !final_ok(block, x, fw, fb)) return std::nullopt;
     const c10::DeviceGuard guard(x.device());
@@ -314,7 +320,7 @@ std::optional<std::pair<Tensor, Tensor>> train_step(const Tensor &x, const Tenso
                                                     const Tensor &fb, const std::optional<Tensor> &osw,
                                                     const std::optional<Tensor> &osb, const Tensor &target, int kind)
 {
-    if (!plain(x) || !floating(x) || (x.dim() != 4 && x.dim() != 5) || !planes_ok(x) || x.requires_grad())
+    if (traced() || !plain(x) || !floating(x) || (x.dim() != 4 && x.dim() != 5) || !planes_ok(x) || x.requires_grad())
         return std::nullopt;
     Block block;
     if (!block.set(x, bias, weights, dilations) || !final_ok(block, x, fw, fb)) return std::nullopt;

@@ -262,3 +262,41 @@ def test_prediction_where_a_weight_is_not_a_parameter_of_its_module():
     model.learn(x, t)                              # (the parameter behind the weight is the one that is trained)
     assert model.loss.grad_fn is not None
     assert not torch.equal(0.5 * block.parametrizations.weight1.original.detach(), original)
+
+
+def test_a_trace_does_not_hold_the_example_output():
+    """A layer is recorded as a call; a network cannot be traced (sizes are tensors then) and says so."""
+    from msd_pytorch_amd.conv2d import conv2d_relu
+    (model,) = _models("L2", 2, 3, 1, 1, 1)
+    x, other = torch.rand(1, 2, 24, 40).cuda(), torch.rand(1, 2, 24, 40).cuda()
+    w, b = torch.randn(1, 2, 3, 3).cuda(), torch.randn(1).cuda()
+
+    def layer(x):
+        return conv2d_relu(x, w, b, torch.empty(1, 1, 24, 40, device="cuda"), 1, 2)
+
+    with torch.no_grad():
+        traced = torch.jit.trace(layer, (x,), check_trace=False)
+        assert torch.equal(traced(other), layer(other))
+        with pytest.raises(RuntimeError):
+            torch.jit.trace(model.net, (x,), check_trace=False)
+
+
+def test_a_tangent_is_not_dropped():
+    """No forward mode: the autograd functions say so, and so do the calls that stand in for them."""
+    import torch.autograd.forward_ad as fwd
+    from msd_pytorch_amd.conv2d import conv2d_relu
+    (model,) = _models("L2", 2, 3, 1, 1, 1)
+    x, w, b = torch.rand(1, 2, 24, 40).cuda(), torch.randn(1, 2, 3, 3).cuda(), torch.randn(1).cuda()
+    out = torch.empty(1, 1, 24, 40).cuda()
+    with fwd.dual_level(), torch.no_grad():
+        for i in range(3):
+            args = [x, w, b]
+            args[i] = fwd.make_dual(args[i], torch.ones_like(args[i]))
+            with pytest.raises(NotImplementedError):
+                conv2d_relu(*args, out, 1, 2)
+        with pytest.raises(NotImplementedError):
+            model.msd(fwd.make_dual(x, torch.ones_like(x)))
+        weights = dict(model.msd.named_parameters())
+        weights["msd_block.weight1"] = fwd.make_dual(weights["msd_block.weight1"], torch.ones(1, 3, 3, 3).cuda())
+        with pytest.raises(NotImplementedError):
+            torch.func.functional_call(model.msd, weights, (x,))
