@@ -271,14 +271,15 @@ class MSDModel:
         parts = self._fused_parts()
         if parts is None or type(self.net[0]) not in (ScalingConv2d, ScalingConv3d) or self._net_hooked():
             return False
-        # the gradients are replaced, which is zero_grad() and backward() for the optimiser of
+        # the gradients are replaced, which is torch's zero_grad() and backward() for the optimiser of
         # exactly these parameters
         linear, block = self.msd.final_layer.linear, self.msd.msd_block
-        weights = block.own_weights()
-        if weights is None:
+        weights, opt = block.own_weights(), self.optimizer
+        if weights is None or not isinstance(opt, optim.Optimizer) or "zero_grad" in opt.__dict__ \
+                or type(opt).zero_grad is not optim.Optimizer.zero_grad:
             return False
         own = [block.bias, *weights, linear.weight, linear.bias]
-        held = [p for group in self.optimizer.param_groups for p in group["params"]]
+        held = [p for group in opt.param_groups for p in group["params"]]
         if len(own) != len(held) or not all(map(operator.is_, own, held)):
             return False
         kind, scale_out = parts

@@ -300,3 +300,42 @@ def test_a_tangent_is_not_dropped():
         weights["msd_block.weight1"] = fwd.make_dual(weights["msd_block.weight1"], torch.ones(1, 3, 3, 3).cuda())
         with pytest.raises(NotImplementedError):
             torch.func.functional_call(model.msd, weights, (x,))
+
+
+def test_an_optimiser_with_a_zero_grad_of_its_own():
+    class Accumulating(torch.optim.Adam):
+        def zero_grad(self, set_to_none=True):
+            pass
+
+    (model,) = _models("L2", 2, 3, 1, 1, 1)
+    x, t = torch.rand(1, 2, 24, 40).cuda(), torch.rand(1, 1, 24, 40).cuda()
+    model.gradients(x, t)
+    once = [p.grad.clone() for p in model.msd.parameters()]
+    plain = model.optimizer
+
+    def replaced():
+        model.optimizer = torch.optim.Adam(model.msd.parameters())
+        model.optimizer.zero_grad = lambda set_to_none=True: None
+
+    def subclass():
+        model.optimizer = Accumulating(model.msd.parameters())
+
+    class Wrapper:                                 # zero_grad and step are all that a step needs
+        def zero_grad(self):
+            plain.zero_grad()
+
+        def step(self):
+            plain.step()
+
+    for change in (replaced, subclass):
+        plain.zero_grad()
+        change()
+        for _ in range(2):
+            model.gradients(x, t)
+        for p, g in zip(model.msd.parameters(), once):
+            assert rel_err(p.grad, 2 * g) <= 1e-5
+    model.optimizer = Wrapper()
+    before = model.msd.msd_block.bias.detach().clone()
+    model.learn(x, t)
+    assert not torch.equal(before, model.msd.msd_block.bias)
+    assert rel_err(model.msd.msd_block.weight1.grad, once[2]) <= 1e-5
