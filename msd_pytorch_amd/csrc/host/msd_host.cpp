@@ -8,10 +8,12 @@
 // their general way, which also raises the errors.  Nothing is kept between calls.
 #include <torch/extension.h>
 
+#include <ATen/SavedTensorHooks.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
+#include <torch/csrc/autograd/anomaly_mode.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -290,6 +292,13 @@ std::optional<Tensor> net_forward(const Tensor &x, const Tensor &bias, const std
     return out;
 }
 
+// Somebody looks at the graph that a training step would make: hooks on what it saves, or a check of
+// every gradient for NaN.
+bool watched()
+{
+    return !at::SavedTensorDefaultHooks::get_tls_state().stack.empty() || torch::autograd::AnomalyMode::is_enabled();
+}
+
 // A parameter whose gradient can be set without autograd: a leaf that nobody watches.
 bool settable(const Tensor &p)
 {
@@ -320,7 +329,8 @@ std::optional<std::pair<Tensor, Tensor>> train_step(const Tensor &x, const Tenso
                                                     const Tensor &fb, const std::optional<Tensor> &osw,
                                                     const std::optional<Tensor> &osb, const Tensor &target, int kind)
 {
-    if (traced() || !plain(x) || !floating(x) || (x.dim() != 4 && x.dim() != 5) || !planes_ok(x) || x.requires_grad())
+    if (traced() || watched() || !plain(x) || !floating(x) || (x.dim() != 4 && x.dim() != 5) || !planes_ok(x) ||
+        x.requires_grad())
         return std::nullopt;
     Block block;
     if (!block.set(x, bias, weights, dilations) || !final_ok(block, x, fw, fb)) return std::nullopt;

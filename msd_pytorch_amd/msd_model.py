@@ -6,6 +6,7 @@ import operator
 import numpy as np
 import torch
 import torch.nn as nn
+import torch.nn.modules.module as module_base
 import torch.optim as optim
 import torch.optim.optimizer as optimizer_base
 
@@ -266,7 +267,9 @@ class MSDModel:
     def _native_step(self):
         """Forward, zero_grad and backward as one native call (MSDModule.train_step).  False, with
         nothing done, where the model or the optimiser is not the plain one."""
-        if not self.fuse_loss or not torch.is_grad_enabled() or not self.input.is_cuda:
+        # (hooks on all modules see the scaling layer's call)
+        if not self.fuse_loss or not torch.is_grad_enabled() or not self.input.is_cuda \
+                or module_base._has_any_global_hook():
             return False
         parts = self._fused_parts()
         if parts is None or type(self.net[0]) not in (ScalingConv2d, ScalingConv3d) or self._net_hooked():

@@ -339,3 +339,22 @@ def test_an_optimiser_with_a_zero_grad_of_its_own():
     model.learn(x, t)
     assert not torch.equal(before, model.msd.msd_block.bias)
     assert rel_err(model.msd.msd_block.weight1.grad, once[2]) <= 1e-5
+
+
+def test_a_training_step_under_watch_goes_through_autograd():
+    """Saved-tensor hooks and anomaly detection see the autograd graph, so there has to be one."""
+    (model,) = _models("L2", 2, 3, 1, 1, 1)
+    x, t = torch.rand(1, 2, 24, 40).cuda(), torch.rand(1, 1, 24, 40).cuda()
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda s: packed.append(s.shape) or s, lambda s: s):
+        model.learn(x, t)
+    assert packed
+    with torch.autograd.detect_anomaly(check_nan=True), pytest.raises(RuntimeError, match="nan"):
+        model.learn(torch.full_like(x, float("nan")), t)
+    seen = []
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, i, o: seen.append(m))
+    try:
+        model.learn(x, t)
+    finally:
+        handle.remove()
+    assert model.scale_in in seen
