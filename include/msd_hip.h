@@ -315,7 +315,8 @@ int msd_block_forward(int dtype, int ndim, int64_t batch, int64_t c_in, int dept
                       const void *const *weights, const void *bias, void *stream);
 /* The same with a workspace (msd_block_forward_workspace_bytes; less, or none, is accepted):
  * groups of layers then take the channels in front of them in one pass (2D, fp32; same sums in
- * another order). */
+ * another order).  It holds three planes per output channel of a group, so up to 21 channels of the
+ * stack's size, while the call runs. */
 int64_t msd_block_forward_workspace_bytes(int dtype, int ndim, int64_t batch, int64_t c_in, int depth,
                                           const int64_t *widths, const int64_t *spatial);
 int msd_block_forward_ws(int dtype, int ndim, int64_t batch, int64_t c_in, int depth, const int64_t *widths,

@@ -1401,15 +1401,25 @@ int forward_group(const BlockArgs &a, int i, int64_t first)
     return n >= 2 ? n : 0;
 }
 
+// Bytes of the three planes per output that the n layers from layer i on leave to their finishing launches.
+int64_t group_planes_bytes(const BlockArgs &a, int i, int n)
+{
+    int64_t outputs = 0;
+    for (int j = 0; j < n; j++) outputs += a.widths[i + j];
+    return 3 * outputs * a.batch * a.spatial[0] * a.spatial[1] * (int64_t)sizeof(float);
+}
+
+// Of the largest group that a block can form, whichever layer its groups start at.
 int64_t forward_group_bytes(const BlockArgs &a)
 {
-    int64_t first = a.c_in;
+    if (a.ndim != 2 || !msd::group_rows_supported_2d(a.spatial[1])) return 0;
+    int64_t first = a.c_in, most = 0;
     for (int i = 0; i < a.depth; i++) {
-        if (forward_group(a, i, first))
-            return 3 * msd::group2d::kMaxOut * a.batch * a.spatial[0] * a.spatial[1] * (int64_t)sizeof(float);
+        const int64_t n = group_planes_bytes(a, i, forward_group(a, i, first));
+        most = n > most ? n : most;
         first += a.widths[i];
     }
-    return 0;
+    return most;
 }
 
 // Layers i .. i + n - 1: one pass over the channels [0, first) for all of them, then each layer
@@ -1505,7 +1515,7 @@ int msd_block_forward_ws(int dtype, int ndim, int64_t batch, int64_t c_in, int d
     int64_t first = c_in, b0 = 0;
     for (int i = 0; i < depth; i++) {
         const int n = workspace ? forward_group(a, i, first) : 0;
-        if (n && workspace_bytes >= forward_group_bytes(a)) {
+        if (n && workspace_bytes >= group_planes_bytes(a, i, n)) {
             bool done = false;
             MSD_TRY(block_group_forward(fn, a, i, n, first, stack, stack_strides, weights, (const float *)bias + b0,
                                         (float *)workspace, (hipStream_t)stream, &done));

@@ -58,6 +58,9 @@ inline Teams make_teams(int W, int halo)
 
 }  // namespace group2d
 
+// Rows of W voxels that the launches of a forward group take where their alignment allows it.
+bool group_rows_supported_2d(int64_t W);
+
 // z[b][3 o + ky][y][x] = sum over the g.C channels and kx of k[o][c][ky][kx] * x[c][y][fold(x + dil_o (kx - 1))]:
 // what row y of the channels contributes to the output rows that read it through tap row ky.
 bool group_push_supported_2d(const Geom &g, const View<const float> &x, int dmax);

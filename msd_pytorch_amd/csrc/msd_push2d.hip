@@ -338,10 +338,16 @@ int finish_vec(const Geom &g, const View<const float> &x, const View<float> &out
 }  // namespace
 }  // namespace group2d
 
+bool group_rows_supported_2d(int64_t W)
+{
+    // (the longer rows: fwd_lattice with a workgroup of 1024 lanes, two or four voxels each)
+    return W >= 32 && (W <= 1024 || (W % 2 == 0 && W <= 2048) || (W % 4 == 0 && W <= 4096));
+}
+
 bool group_push_supported_2d(const Geom &g, const View<const float> &x, int dmax)
 {
     using namespace group2d;
-    return g.ndim == 2 && x.sx == 1 && g.W >= 32 && dmax <= 128 && g.C >= 1 && x.sc < ((int64_t)1 << 28) &&
+    return g.ndim == 2 && x.sx == 1 && group_rows_supported_2d(g.W) && dmax <= 128 && g.C >= 1 && x.sc < ((int64_t)1 << 28) &&
            (int64_t)g.B * g.H * ((g.W + kWave - 1) / kWave) < ((int64_t)1 << 30);
 }
 

@@ -121,3 +121,27 @@ def test_tuning_hook_rejects_unknown_key():
         assert lib.msd_set_tuning(key.encode(), -1) == _native.MSD_OK, key
     assert lib.msd_set_kernel_path(2) == _native.MSD_ERR_INVALID
     assert lib.msd_set_kernel_path(0) == _native.MSD_OK
+
+
+@pytest.mark.parametrize("size,c_in,width,depth,outputs", [
+    ((64, 64), 1, 1, 100, 7),
+    ((64, 64), 12, 1, 3, 3),                       # one short group
+    ((64, 64), 12, 1, 8, 7),                       # a layer is left over
+    ((64, 64), 1, 1, 12, 0),                       # fewer channels in front than a group needs
+    ((64, 64), 1, 2, 20, 6),                       # three layers of two channels
+    ((64, 64), 12, 3, 20, 0),                      # wider layers form no groups
+    ((9, 31), 12, 1, 8, 0),                        # rows that no pass takes: short, odd and long, longer
+    ((9, 1024), 12, 1, 8, 7),
+    ((9, 1025), 12, 1, 8, 0),
+    ((9, 1026), 12, 1, 8, 7),
+    ((9, 2050), 12, 1, 8, 0),
+    ((9, 2052), 12, 1, 8, 7),
+    ((9, 4096), 12, 1, 8, 7),
+    ((9, 4100), 12, 1, 8, 0),
+])
+def test_forward_workspace_holds_the_planes_of_the_largest_group(size, c_in, width, depth, outputs):
+    lib = _native.load()
+    for batch in (1, 3):
+        need = lib.msd_block_forward_workspace_bytes(0, 2, batch, c_in, depth, i64(*[width] * depth), i64(*size))
+        assert need == 3 * outputs * batch * size[0] * size[1] * 4
+    assert lib.msd_block_forward_workspace_bytes(1, 2, 1, c_in, depth, i64(*[width] * depth), i64(*size)) == 0

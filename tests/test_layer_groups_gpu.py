@@ -106,3 +106,18 @@ def test_an_infinity_in_front_of_a_forward_group_stays_one(c_in):
     assert torch.equal(torch.isinf(found[0]), torch.isinf(found[1]))
     assert torch.equal(finite, torch.isfinite(found[1]))
     assert rel_err(found[1][finite], found[0][finite]) <= 1e-5
+
+
+# Rows that the finishing launch does not take (more than 1024 voxels that are not whole groups of
+# four, more than 2048): fwd_lattice adds the planes, with no channel of the group's own and with some.
+@pytest.mark.parametrize("case", [
+    ((7, 1030), 12, 1, 9, 2, [7, 1, 2]),
+    ((6, 2046), 12, 1, 8, 1, [1, 6, 3]),
+    ((5, 2052), 13, 1, 9, 1, [5, 1, 2]),
+    ((5, 1026), 6, 2, 4, 1, [1, 2, 5]),
+    ((4, 4096), 8, 2, 5, 1, [1, 2, 4]),
+], ids=lambda c: "x".join(map(str, c[0])) + "-c%d-w%d-d%d-B%d" % c[1:5])
+def test_forward_groups_of_long_rows(case):
+    size, c_in, width, depth, batch, dilations = case
+    dilations = [dilations[i % len(dilations)] for i in range(depth)]
+    check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=47)
