@@ -244,11 +244,16 @@ struct Block {
         const int64_t need = lib.msd_block_forward_workspace_bytes(dtype_of(stack), (int)stack.dim() - 2,
                                                                    stack.size(0), c_in, (int)widths.size(),
                                                                    widths.data(), stack.sizes().data() + 2);
-        const Tensor ws = need ? workspace(need, stack) : Tensor();
+        Tensor ws;
+        try {
+            if (need) ws = workspace(need, stack);
+        } catch (const c10::OutOfMemoryError &) {
+            // the block needs none: its layers then run one by one
+        }
         check(lib.msd_block_forward_ws(dtype_of(stack), (int)stack.dim() - 2, stack.size(0), c_in, (int)widths.size(),
                                        widths.data(), stack.sizes().data() + 2, dilations.data(), stack.data_ptr(),
                                        stack.strides().data(), weights.data(), bias.data_ptr(),
-                                       need ? ws.data_ptr() : nullptr, need, stream));
+                                       ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? need : 0, stream));
     }
 };
 

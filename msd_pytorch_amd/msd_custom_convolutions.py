@@ -417,7 +417,12 @@ def block_forward(stack, c_in, dilations, bias, weights):
     need = _native.load().msd_block_forward_workspace_bytes(head[0], head[1], head[2], c_in, head[4], head[5], head[6])
     if need < 0:
         _fail(fn, "invalid block geometry")
-    ws = torch.empty(max(int(need), 8), dtype=torch.uint8, device=stack.device) if need else None
+    ws = None
+    if need:
+        try:
+            ws = torch.empty(int(need), dtype=torch.uint8, device=stack.device)
+        except torch.cuda.OutOfMemoryError:
+            need = 0                # the block needs none: its layers then run one by one
     _call("msd_block_forward_ws", stack.device, *head, *_view(stack), _ptr_array(weights),
           ctypes.c_void_p(bias.data_ptr()), ctypes.c_void_p(ws.data_ptr() if need else 0), int(need), _stream(stack))
 

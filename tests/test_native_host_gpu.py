@@ -358,3 +358,25 @@ def test_a_training_step_under_watch_goes_through_autograd():
     finally:
         handle.remove()
     assert model.scale_in in seen
+
+
+@pytest.mark.parametrize("gradients", [False, True])
+def test_a_forward_pass_that_has_no_room_for_the_planes_of_its_groups(gradients):
+    """Up to 21 channels of the stack's size for a while; without them the layers run one by one."""
+    (model,) = _models("L2", 2, 20, 1, 1, 1)
+    x = torch.rand(1, 2, 1024, 1024).cuda()
+    with torch.set_grad_enabled(gradients):
+        want = model.net(x).detach().clone()
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        plane = x.numel() // 2 * 4
+        # stack, scaled input, output and half the planes
+        room = torch.cuda.memory_reserved() + plane * (22 + 2 + 2 + 10)
+        total = torch.cuda.get_device_properties(0).total_memory
+        torch.cuda.set_per_process_memory_fraction(room / total)
+        try:
+            got = model.net(x).detach()
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+    assert not torch.equal(got, want)              # (another order of summation)
+    assert rel_err(got, want) <= 1e-5
