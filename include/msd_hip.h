@@ -303,8 +303,9 @@ int msd_relu_mask_gradient(int dtype, int ndim, int64_t batch, int64_t c_out, co
  * Replaces the loop of msd_block.py:89-130.  Workspace: msd_block_workspace_bytes,
  * which is the largest msd_workspace_bytes of the layers plus room (at most 1 GiB) for
  * the partial weight-gradient sums of many layers at once, so that one launch can
- * reduce up to 16 layers; the largest msd_workspace_bytes of the layers alone is
- * accepted too (every layer then reduces its sums right away; same results).
+ * reduce up to 16 layers, or what the partial sums of a group of 2D layers take where
+ * that is more.  The largest msd_workspace_bytes of the layers alone is accepted too
+ * (layers are then taken one at a time and reduced right away; same sums, in another order).
  */
 int64_t msd_block_workspace_bytes(int dtype, int ndim, int64_t batch, int64_t c_in, int depth,
                                   const int64_t *widths, const int64_t *spatial);

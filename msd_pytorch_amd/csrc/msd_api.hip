@@ -207,6 +207,11 @@ int make_view(const char *fn, const char *name, int ndim, const void *p, const i
     return MSD_OK;
 }
 
+bool workspace_holds(const msd::Geom &g, size_t elem, const void *ws, int64_t bytes)
+{
+    return ws && bytes >= msd::generic_workspace_elems(g) * (int64_t)elem;
+}
+
 int check_workspace(const char *fn, const msd::Geom &g, size_t elem, const void *ws, int64_t bytes)
 {
     const int64_t need = msd::generic_workspace_elems(g) * (int64_t)elem;
@@ -978,7 +983,7 @@ int block_group_fused(const char *fn, const BlockArgs &a, int i, int n, int64_t 
         st.gy = msd::View<const float>{gx.p + gy_ch * gx.sc, gx.sb, gx.sc, gx.sz, gx.sy, gx.sx};
         st.lean = !shared && msd::fast_backward_one_channel_supported_2d(st.g, st.gy, st.x, st.gx);
         if (!st.lean && !msd::fast_backward_xkb_supported(st.g, st.gy, st.x, st.gx)) return MSD_OK;
-        MSD_TRY(check_workspace(fn, st.g, sizeof(float), ws, ws_bytes));
+        if (!workspace_holds(st.g, sizeof(float), ws, ws_bytes)) return MSD_OK;     // (enough for single layers)
     }
     for (int j = 1; j <= n; j++) {
         Step &st = steps[j - 1];
@@ -1162,7 +1167,7 @@ int block_backward_split3d(const char *fn, const BlockArgs &a, int64_t c_in, con
             p.group.max_workgroups = 0;
             p.gy = gy;                            // channels first (layer i) and first + 1 (layer i + 1)
             if (!msd::fast_backward_k_pair_supported_3d(p.g, p.gy, x)) return MSD_OK;
-            MSD_TRY(check_workspace(fn, p.g, sizeof(float), workspace, workspace_bytes));
+            if (!workspace_holds(p.g, sizeof(float), workspace, workspace_bytes)) return MSD_OK;
         }
     }
     // a profiled run keeps to one stream: its per-class event pairs time one stream's work

@@ -121,3 +121,56 @@ def test_forward_groups_of_long_rows(case):
     size, c_in, width, depth, batch, dilations = case
     dilations = [dilations[i % len(dilations)] for i in range(depth)]
     check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=47)
+
+
+@pytest.mark.parametrize("size", [(256, 256), (9, 20, 64)], ids=str)
+def test_blocks_with_less_workspace_than_the_groups_ask_for(size):
+    """Callers of the C interface choose the workspace: down to what the layers ask for one by one."""
+    import ctypes
+    import oracle
+    from msd_pytorch_amd import _native, msd_custom_convolutions as cc
+    from parity import block_problem
+    lib = _native.load()
+    ndim, c_in, depth = len(size), 17, 15
+    x, dil, bias, ws, g = block_problem(ndim, size, c_in, 1, depth, 1, seed=3)
+    want = oracle.block_forward(x.double(), dil, bias.double(), [w.double() for w in ws])
+    weights, bias_d = [w.cuda() for w in ws], bias.cuda()
+    stack = torch.empty(1, c_in + depth, *size, device="cuda")
+    stack[:, :c_in] = x.cuda()
+    head = cc._block_head(stack, c_in, dil, weights)
+    query = (head[0], head[1], head[2], c_in, depth, head[5], head[6])
+    pointers, stream = cc._ptr_array(weights), cc._stream(stack)
+
+    def scratch(need):
+        # what lies behind the workspace has to stay as it is
+        buffer = torch.full((need + 1024,), 0x5a, dtype=torch.uint8, device="cuda")
+        return buffer, ctypes.c_void_p(buffer.data_ptr())
+
+    need = lib.msd_block_forward_workspace_bytes(*query)
+    assert need == (3 * 7 * size[0] * size[1] * 4 if ndim == 2 else 0)
+    if need:
+        need -= 4                                  # (the second group, of the last layer alone, is none)
+        buffer, at = scratch(need)
+        assert lib.msd_block_forward_ws(*head, *cc._view(stack), pointers, ctypes.c_void_p(bias_d.data_ptr()), at, need,
+                                        stream) == 0, _native.last_error()
+        assert rel_err(stack, want) <= 1e-5
+        assert bool((buffer[need:] == 0x5a).all())
+    else:
+        stack.copy_(want)
+
+    layers = [lib.msd_workspace_bytes(head[0], ndim, 1, c_in + i, 1, head[6]) for i in range(depth)]
+    pairs = [lib.msd_workspace_bytes(head[0], ndim, 1, c_in + i, 2, head[6]) for i in range(depth - 1)]
+    need = max(layers)
+    # (a 2D group over 17 to 32 channels asks for 4.2 MB here)
+    assert need < max(pairs) and (ndim == 3 or need < 4_200_000) and need < lib.msd_block_workspace_bytes(*query)
+    buffer, at = scratch(need)
+    grads = g.cuda()
+    gk, gb = [torch.zeros_like(w) for w in weights], torch.zeros_like(bias_d)
+    assert lib.msd_block_backward(*head, *cc._view(stack), *cc._view(grads), pointers, cc._ptr_array(gk),
+                                  ctypes.c_void_p(gb.data_ptr()), 1, at, need, stream) == 0, _native.last_error()
+    want_gx, want_gb, want_gw = oracle.block_backward(stack.double().cpu(), g.double(), dil, bias.double(),
+                                                      [w.double() for w in ws])
+    assert rel_err(grads[:, :c_in], want_gx) <= 1e-4 and rel_err(gb, want_gb) <= 1e-4
+    for a, c in zip(gk, want_gw):
+        assert rel_err(a, c) <= 1e-4
+    assert bool((buffer[need:] == 0x5a).all())
