@@ -343,7 +343,8 @@ std::optional<std::pair<Tensor, Tensor>> train_step(const Tensor &x, const Tenso
     if (c_out > 8 || !scale_ok(sw, sb, x, c_in)) return std::nullopt;
     const bool scaled = osw.has_value();
     if (scaled != osb.has_value() || (scaled && !scale_ok(*osw, *osb, x, c_out))) return std::nullopt;
-    if (!plain(target) || target.device() != x.device() || target.requires_grad() || target.size(0) != x.size(0))
+    if (!plain(target) || target.device() != x.device() || target.requires_grad() || target.dim() == 0 ||
+        target.size(0) != x.size(0))
         return std::nullopt;
     if (kind == MSD_LOSS_NLL) {
         if (target.scalar_type() != at::kLong || target.dim() != x.dim() - 1 || !target.is_contiguous() ||

@@ -380,3 +380,13 @@ def test_a_forward_pass_that_has_no_room_for_the_planes_of_its_groups(gradients)
             torch.cuda.set_per_process_memory_fraction(1.0)
     assert not torch.equal(got, want)              # (another order of summation)
     assert rel_err(got, want) <= 1e-5
+
+
+@pytest.mark.filterwarnings("ignore:Using a target size")
+def test_a_target_of_another_shape_is_left_to_the_criterion():
+    (model,) = _models("L2", 2, 3, 1, 1, 1)
+    model.set_input(torch.rand(2, 2, 24, 40).cuda())
+    for target in (torch.tensor(0.5), torch.rand(40), torch.rand(1, 1, 24, 40)):
+        model.target = target.cuda()
+        loss = model.learn()
+        assert abs(loss - float(((model.output - model.target) ** 2).mean())) <= 1e-5 * loss
