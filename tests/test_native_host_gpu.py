@@ -390,3 +390,36 @@ def test_a_target_of_another_shape_is_left_to_the_criterion():
         model.target = target.cuda()
         loss = model.learn()
         assert abs(loss - float(((model.output - model.target) ** 2).mean())) <= 1e-5 * loss
+
+
+@pytest.mark.parametrize("path", ["layer", "prediction", "step"])
+def test_native_calls_run_on_the_current_stream(path):
+    """The input arrives late on a stream of its own: work on any other stream would miss it."""
+    from msd_pytorch_amd.conv2d import conv2d_relu
+    (model,) = _models("L2", 2, 9, 1, 1, 1)
+    value, t = torch.rand(1, 2, 64, 96).cuda(), torch.rand(1, 1, 64, 96).cuda()
+    w, b = torch.randn(1, 2, 3, 3).cuda().requires_grad_(), torch.randn(1).cuda().requires_grad_()
+
+    def run(x):
+        if path == "layer":
+            leaf = x.requires_grad_()
+            y = conv2d_relu(leaf, w, b, torch.empty_like(t), 1, 3)
+            return [y.detach(), *torch.autograd.grad(y, (leaf, w, b), t)]
+        if path == "prediction":
+            with torch.no_grad():
+                return [model.net(x)]
+        model.step_async(x, t, update=False)
+        assert model.loss.grad_fn is None
+        return [model.loss, model.output, *(p.grad for p in model.msd.parameters())]
+
+    want = [r.clone() for r in run(value.clone())]
+    side, late = torch.cuda.Stream(), torch.zeros_like(value)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(50_000_000)              # some 20 ms
+        late.copy_(value)
+        got = run(late)
+        assert not side.query()                    # (nothing has waited)
+    side.synchronize()
+    for a, c in zip(got, want):
+        assert torch.equal(a, c)
