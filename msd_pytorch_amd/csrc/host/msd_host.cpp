@@ -445,8 +445,8 @@ std::optional<std::pair<Tensor, Tensor>> train_step(const Tensor &x, const Tenso
 // False (and nothing has happened) for a state that the kernel does not take.
 // ---------------------------------------------------------------------------
 
-bool adam_step(const std::vector<Tensor> &params, const py::list &states, double lr, double beta1, double beta2,
-               double eps)
+bool adam_step(const std::vector<Tensor> &params, const py::list &states, bool capturable, double lr, double beta1,
+               double beta2, double eps)
 {
     static PyObject *const k_step = PyUnicode_InternFromString("step");
     static PyObject *const k_avg = PyUnicode_InternFromString("exp_avg");
@@ -474,7 +474,7 @@ bool adam_step(const std::vector<Tensor> &params, const py::list &states, double
         if (step.is_cuda()) {
             if (step.device() != first.device()) return false;
             e.device_step = step.data_ptr<float>();
-        } else if (step.is_cpu()) {
+        } else if (step.is_cpu() && !capturable) {   // (torch refuses a capturable step counted on the host)
             float *s = step.data_ptr<float>();
             e.step = (double)*s + 1.0;
             host_steps.push_back(s);

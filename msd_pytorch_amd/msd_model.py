@@ -323,7 +323,8 @@ class MSDModel:
             entries = [state[p] for p in params]
         else:
             return False
-        return _native.host().adam_step(params, entries, group["lr"], *group["betas"], group["eps"])
+        return _native.host().adam_step(params, entries, bool(group["capturable"]), group["lr"], *group["betas"],
+                                        group["eps"])
 
     def forward(self, input=None, target=None):
         """Loss of one (input, target) pair; arguments left out keep their last value."""

@@ -423,3 +423,13 @@ def test_native_calls_run_on_the_current_stream(path):
     side.synchronize()
     for a, c in zip(got, want):
         assert torch.equal(a, c)
+
+
+def test_a_capturable_optimiser_with_its_counts_on_the_host_is_refused():
+    (model,) = _models("L2", 2, 3, 1, 1, 1)
+    x, t = torch.rand(1, 2, 24, 40).cuda(), torch.rand(1, 1, 24, 40).cuda()
+    model.learn(x, t)
+    model.learn(x, t)
+    model.optimizer.param_groups[0]["capturable"] = True
+    with pytest.raises(AssertionError, match="capturable"):
+        model.learn(x, t)
