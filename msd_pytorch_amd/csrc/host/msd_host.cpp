@@ -9,6 +9,7 @@
 #include <torch/extension.h>
 
 #include <ATen/SavedTensorHooks.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -297,11 +298,13 @@ std::optional<Tensor> net_forward(const Tensor &x, const Tensor &bias, const std
     return out;
 }
 
-// Somebody looks at the graph that a training step would make: hooks on what it saves, or a check of
-// every gradient for NaN.
+// Somebody looks at the graph that a training step would make: hooks on what it saves, a check of
+// every gradient for NaN, or autocast, which acts on the products with the output scaling (and which the
+// general path refuses for that).
 bool watched()
 {
-    return !at::SavedTensorDefaultHooks::get_tls_state().stack.empty() || torch::autograd::AnomalyMode::is_enabled();
+    return !at::SavedTensorDefaultHooks::get_tls_state().stack.empty() || torch::autograd::AnomalyMode::is_enabled() ||
+           at::autocast::is_autocast_enabled(at::kCUDA);
 }
 
 // A parameter whose gradient can be set without autograd: a leaf that nobody watches.

@@ -433,3 +433,15 @@ def test_a_capturable_optimiser_with_its_counts_on_the_host_is_refused():
     model.optimizer.param_groups[0]["capturable"] = True
     with pytest.raises(AssertionError, match="capturable"):
         model.learn(x, t)
+
+
+def test_autocast_acts_as_on_the_autograd_path():
+    (model,) = _models("L2", 2, 3, 1, 1, 1)
+    (labels,) = _models("labels", 2, 3, 1, 4, 1)
+    x, t = torch.rand(1, 2, 24, 40).cuda(), torch.rand(1, 1, 24, 40).cuda()
+    y = torch.randint(0, 4, (1, 1, 24, 40)).cuda()
+    want = labels.gradients(x, y)
+    with torch.autocast("cuda", dtype=torch.float16):
+        with pytest.raises(RuntimeError, match="same type"):
+            model.learn(x, t)
+        assert abs(labels.gradients(x, y) - want) <= 1e-5 * want and labels.loss.grad_fn is not None
