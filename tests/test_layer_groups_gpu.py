@@ -174,3 +174,45 @@ def test_blocks_with_less_workspace_than_the_groups_ask_for(size):
     for a, c in zip(gk, want_gw):
         assert rel_err(a, c) <= 1e-4
     assert bool((buffer[need:] == 0x5a).all())
+
+
+# Layers of one and of two channels in one block: groups of five to seven outputs whose layers start
+# at odd outputs, with an odd number of channels in front and above.
+@pytest.mark.parametrize("widths", [
+    [1, 2, 1, 2, 1, 2, 2, 1, 2, 1],
+    [2, 2, 2, 1, 2, 2, 2, 1],
+    [2, 1, 2, 2, 2, 2, 1, 1, 2],
+    [2, 2, 1, 1, 1, 2, 1, 1, 1, 1, 2],
+], ids=lambda w: "".join(map(str, w)))
+@pytest.mark.parametrize("size,c_in", [((18, 64), 4), ((9, 77), 13)])
+def test_groups_of_layers_of_one_and_two_channels(widths, size, c_in):
+    import oracle
+    from msd_pytorch_amd.msd_block import msd_block
+    gen = torch.Generator().manual_seed(19)
+    weights, channels = [], c_in
+    for w in widths:
+        weights.append(torch.randn(w, channels, 3, 3, generator=gen) * (2.0 / (9 * channels)) ** 0.5)
+        channels += w
+    dilations = [1 + i % 4 for i in range(len(widths))]
+    x, bias = torch.rand(2, c_in, *size, generator=gen), torch.randn(channels - c_in, generator=gen) * 0.05
+    g = torch.randn(2, channels, *size, generator=gen)
+    leaves = [t.cuda().requires_grad_() for t in (x, bias, *weights)]
+    with tuning({"fwd.group": 1, "bwd.group": 1}):
+        got = msd_block(leaves[0], dilations, leaves[1], *leaves[2:])
+        grads = torch.autograd.grad(got, leaves, g.cuda())
+    w64 = [w.double() for w in weights]
+    assert rel_err(got, oracle.block_forward(x.double(), dilations, bias.double(), w64)) <= 1e-5
+    want_gx, want_gb, want_gw = oracle.block_backward(got.detach().double().cpu(), g.double(), dilations, bias.double(), w64)
+    for a, b in zip(grads, (want_gx, want_gb, *want_gw)):
+        assert rel_err(a, b) <= 1e-4
+
+
+# What passes of two layers run where the groups do not apply, at sizes that a block takes in groups by default.
+@pytest.mark.parametrize("case", [
+    ((40, 67), 20, 1, 6, 1, None),                 # odd rows, 17 to 32 channels
+    ((64, 128), 50, 1, 4, 1, None),                # whole rows, 33 to 64
+], ids=lambda c: "x".join(map(str, c[0])) + "-c%d-w%d-d%d-B%d" % c[1:5])
+def test_pairs_of_layers_where_groups_would_run(case):
+    size, c_in, width, depth, batch, dilations = case
+    with tuning({"block.pair": 1, "block.triple": 0}):
+        check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=53)

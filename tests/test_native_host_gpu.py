@@ -448,3 +448,21 @@ def test_autocast_acts_as_on_the_autograd_path():
         with pytest.raises(RuntimeError, match="same type"):
             model.learn(x, t)
         assert abs(labels.gradients(x, y) - want) <= 1e-5 * want and labels.loss.grad_fn is not None
+
+
+@pytest.mark.parametrize("task,ndim,size,c_out", [("L2", 2, (20, 33), 3), ("labels", 3, (5, 7, 9), 2)])
+def test_a_training_step_in_double_precision(task, ndim, size, c_out):
+    native, general = _models(task, ndim, 5, 1, c_out, 2)
+    general._native_step = lambda: False
+    gen = torch.Generator().manual_seed(6)
+    x = torch.randn(2, 2, *size, generator=gen, dtype=torch.float64).cuda()
+    t = torch.randint(0, c_out, (2, 1, *size), generator=gen).cuda() if task == "labels" \
+        else torch.randn(2, c_out, *size, generator=gen, dtype=torch.float64).cuda()
+    for m in (native, general):
+        m.net.double()
+        m.gradients(x, t)
+    assert native.loss.grad_fn is None and general.loss.grad_fn is not None
+    assert abs(float(native.loss) - float(general.loss)) <= 1e-13 * float(general.loss)
+    assert rel_err(native.output, general.output) <= 1e-13
+    for p, q in zip(native.msd.parameters(), general.msd.parameters()):
+        assert rel_err(p.grad, q.grad) <= 1e-12
