@@ -32,10 +32,11 @@ PIPE = {"forward": "fp32 VALU, non-packed (78.6 TFLOP/s of the 157.3 peak); 2D l
                         "2D layer groups: both on the MFMA"}
 
 # kernel families (as named in the profile summaries) whose HBM traffic belongs to a class
-FAMILIES = {"forward": ("fwd_lattice",), "backward_xkb": ("bwd_rows_fused", "bwd_one_channel", "reduce_columns"),
+FAMILIES = {"forward": ("fwd_lattice", "push_rows", "finish_rows"),
+            "backward_xkb": ("bwd_rows_fused", "bwd_one_channel", "pull_rows", "finish_back", "sum_group", "reduce_columns"),
             "backward_kb": ("bwdk_rows", "bwdk_mfma"), "backward_x": ("relu_mask", "bwdx_rows", "bwdx_one_channel")}
-# families that are the second pass of an operator call, not a call of their own
-SECOND_PASS = ("reduce_columns",)
+# families that are the further passes of an operator call or of a group of layers, not a call of their own
+SECOND_PASS = ("reduce_columns", "finish_rows", "finish_back", "sum_group")
 
 
 def profiled_traffic(name, split3d=False):
