@@ -18,6 +18,7 @@
 // together.  1024 x 1024, 7 layers: 35 us + 1.1 us per channel (0.95 us are the matrix instructions
 // at the clock they run at), 139 us at 94 channels where seven launches of fwd_lattice took 520;
 // output by output, with the voxels as columns, it was 45 us + 1.1 us.
+// Counters over the 13 launches of a forward pass of depth 100 there: 4.1 GB in 1.14 ms, matrix cores busy 52 %.
 #include "msd_group.h"
 
 #include <algorithm>
