@@ -216,3 +216,36 @@ def test_pairs_of_layers_where_groups_would_run(case):
     size, c_in, width, depth, batch, dilations = case
     with tuning({"block.pair": 1, "block.triple": 0}):
         check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=53)
+
+
+@pytest.mark.parametrize("pitch,gap,offset", [(80, 0, 0), (83, 5, 3), (96, 64, 1)])
+def test_groups_on_views_with_gaps(pitch, gap, offset):
+    """Rows and planes apart, and not on 16 bytes: a view of a larger buffer, what lies between is left alone."""
+    import oracle
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    from parity import block_problem
+    size, c_in, depth, batch = (11, 77), 13, 9, 2
+    x, dil, bias, ws, g = block_problem(2, size, c_in, 1, depth, batch, seed=23)
+    channels, plane = c_in + depth, size[0] * pitch + gap
+
+    def view():
+        buffer = torch.full((offset + batch * channels * plane,), 7.0, device="cuda")
+        strides = (channels * plane, plane, pitch, 1)
+        return buffer, buffer.as_strided((batch, channels, *size), strides, offset)
+
+    (sbuf, stack), (gbuf, grads) = view(), view()
+    stack[:, :c_in] = x.cuda()
+    grads.copy_(g)
+    weights, gk, gb = [w.cuda() for w in ws], [torch.zeros_like(w).cuda() for w in ws], torch.zeros(depth).cuda()
+    with tuning({"fwd.group": 1, "bwd.group": 1}):
+        cc.block_forward(stack, c_in, dil, bias.cuda(), weights)
+        cc.block_backward(stack, grads, c_in, dil, weights, gk, gb, True)
+    w64 = [w.double() for w in ws]
+    assert rel_err(stack, oracle.block_forward(x.double(), dil, bias.double(), w64)) <= 1e-5
+    want_gx, want_gb, want_gw = oracle.block_backward(stack.double().cpu().contiguous(), g.double(), dil, bias.double(), w64)
+    assert rel_err(grads[:, :c_in], want_gx) <= 1e-4 and rel_err(gb, want_gb) <= 1e-4
+    for a, b in zip(gk, want_gw):
+        assert rel_err(a, b) <= 1e-4
+    for buffer, inner in ((sbuf, stack), (gbuf, grads)):
+        inner.fill_(7.0)
+        assert bool((buffer == 7.0).all())
