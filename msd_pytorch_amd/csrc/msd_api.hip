@@ -1256,12 +1256,14 @@ int block_backward_split3d(const char *fn, const BlockArgs &a, int64_t c_in, con
 }
 
 // ---------------------------------------------------------------------------
-// Groups of layers of the 2D backward pass on the matrix cores (msd_pull2d.hip).
+// Groups of layers of the 2D backward pass on the matrix cores (msd_pull.hip).
 // ---------------------------------------------------------------------------
 
 // Channels below the lowest layer of a group from which on it is taken.  The pass works in blocks of
 // 16 channels, but already over the four below the layers of a depth of ten (256 x 256, recorded step)
-// it is faster than pairs of layers: 157 -> 150 us; 3 x 333 x 477, depth 30: 1.84 -> 0.97 ms per step.
+// it is faster than pairs of layers: 157 -> 150 us; 3 x 333 x 477, depth 30: 1.84 -> 0.97 ms per step.  A group takes
+// up to 14 outputs wherever there are that many: at 1024 x 1024 a pass and the upper half's share of the lower (49 us)
+// are as fast as two groups of seven over 20 channels (266 us both), 332 against 371 us over 48, 552 against 860 over 95.
 constexpr int64_t kGroupBackChannels = 4;
 
 // Number of layers from layer i down that form a group of the backward pass (0: none); `first` is
@@ -1340,15 +1342,26 @@ int block_group_backward(const char *fn, const BlockArgs &a, int i, int n, int64
     if (!msd::group_pull_supported_2d(g, x, gx)) return MSD_OK;
     if (ws_bytes < msd::group_pull_floats_2d(g.B, g.H, g.W, first) * (int64_t)sizeof(float)) return MSD_OK;
     ProfileScope scope(3, s);
+    // The layers whose outputs are the upper slab (the last seven outputs or fewer) complete one another;
+    // what they add to the channels below them in the group is added to all of these at once.
+    int top = i;                                  // lowest layer of the upper half
+    while (top > lo && out.n - start[top - 1 - lo] <= msd::group2d::kSlabOut) top--;
+    auto above = [&](int from, int to, int ch) {
+        msd::group2d::Outputs up{};
+        for (int o = from; o < to; o++) {
+            up.dil[up.n] = out.dil[o];
+            up.k[up.n++] = out.k[o] + (int64_t)ch * msd::group2d::kTaps;
+        }
+        return up;
+    };
     for (int j = i - 1; j >= lo; j--) {
         const int ch = (int)c + start[j - lo], from = start[j - lo] + (int)a.widths[j];
-        msd::group2d::Outputs above{};
-        for (int o = from; o < out.n; o++) {
-            above.dil[above.n] = out.dil[o];
-            above.k[above.n++] = out.k[o] + (int64_t)ch * msd::group2d::kTaps;
-        }
         // a layer of two channels: the second one's weights follow the first's in each output's kernel
-        const hipError_t e = msd::group_finish_back_2d(g, x, gx, ch, (int)a.widths[j], above, s);
+        const hipError_t e = j == top - 1
+                                 ? msd::group_spread_back_2d(g, x, gx, (int)c, start[top - lo], (int)a.widths[j],
+                                                             above(start[top - lo], out.n, (int)c), s)
+                                 : msd::group_finish_back_2d(g, x, gx, ch, (int)a.widths[j],
+                                                             above(from, j < top ? start[top - lo] : out.n, ch), s);
         if (e != hipSuccess) return hip_fail(fn, e);
     }
     const bool update = lo > 0 || need_input_grad;
@@ -1401,7 +1414,7 @@ int forward_group(const BlockArgs &a, int i, int64_t first)
     if (first < (from > 0 ? from : a.widths[i] > 1 ? kGroupChannelsWide : kGroupChannels)) return 0;
     int n = 0;
     int64_t outputs = 0;
-    while (i + n < a.depth && a.widths[i + n] <= 2 && outputs + a.widths[i + n] <= msd::group2d::kMaxOut)
+    while (i + n < a.depth && a.widths[i + n] <= 2 && outputs + a.widths[i + n] <= msd::group2d::kSlabOut)
         outputs += a.widths[i + n++];
     return n >= 2 ? n : 0;
 }

@@ -2,9 +2,9 @@
 //
 // The layers i, i + 1, ... of a group read the same channels [0, c) of the stack, c the number
 // of channels in front of the first of them.  Taken together they are one matrix product over
-// those channels: with one row per (output, tap) a group of seven one-channel layers is a
-// 63 x c weight matrix, which fills four 16-row tiles of v_mfma_f32_16x16x4 to 98 %, and every
-// channel is read once for seven layers instead of once (three rows at a time) per layer.
+// those channels: with one row per (output, tap) seven one-channel layers are a 63 x c weight
+// matrix, which fills a slab of 64 rows to 98 %, and every channel is read once for seven layers
+// (the backward pass: for up to fourteen, two slabs) instead of once (three rows at a time) per layer.
 #pragma once
 #include "msd_kernels.h"
 #include "msd_rows.h"
@@ -13,8 +13,11 @@ namespace msd {
 namespace group2d {
 
 constexpr int kTaps = 9;
-constexpr int kMaxOut = 7;                        // outputs of a group: 7 * 9 = 63 of 64 matrix rows
-constexpr int kRows = 64;                         // matrix rows
+constexpr int kSlabOut = 7;                       // outputs of a slab: 7 * 9 = 63 of 64 matrix rows
+constexpr int kRows = 64;                         // matrix rows of a slab
+constexpr int kMaxOut = 14;                       // outputs of a group: one or two slabs
+constexpr int kMaxAbove = 7;                      // outputs that complete a channel of the group in one launch
+constexpr int kMaxLower = 8;                      // channels of a group's lower half
 constexpr int kTiles = kRows / 16;
 constexpr int kChunk = 128;                       // channels whose weights are in LDS at a time
 
@@ -86,5 +89,10 @@ hipError_t group_pull_2d(const Geom &g, const View<const float> &x, const group2
 // above them (`above`, their weights of these channels) contribute, and applies the ReLU mask.
 hipError_t group_finish_back_2d(const Geom &g, const View<const float> &x, const View<float> &grads, int channel, int width,
                                 const group2d::Outputs &above, hipStream_t s);
+
+// Adds to the gradients of the `channels` channels from `channel` on what the outputs right above
+// them (at most kSlabOut) contribute, and completes the last `width` of them.
+hipError_t group_spread_back_2d(const Geom &g, const View<const float> &x, const View<float> &grads, int channel, int channels,
+                                int width, const group2d::Outputs &above, hipStream_t s);
 
 }  // namespace msd

@@ -1,0 +1,1239 @@
+// Backward pass of a group of layers over the channels they share (msd_group.h).
+//
+// With A[m][v], m = (output o, tap t), the adjoint-form gather of the masked output gradients at
+// voxel v, both gradients are matrix products with the same matrix:
+//     grad_input[c][v]  += sum_m k[m][c] * A[m][v],
+//     grad_kernel[c][m] += sum_v x[c][v] * A[m][v].
+// fp32 values are taken in three bf16 parts and six products (msd_split.h).  A workgroup of eight
+// waves owns a tile of eight segments of 32 voxels (four where a group has more than seven outputs) and
+// the 64 rows m of one slab (128 of two).  Each wave gathers a segment's A of one slab, splits it and
+// leaves it in LDS as [part][voxel][m]: the grad_input product reads it as it lies (lane = voxel, eight
+// rows m), the grad_kernel product through the transposing LDS read (ds_read_b64_tr_b16).  Behind a
+// barrier each wave takes its own block of 16 channels through both products, 64 voxels at a time; its
+// weights and its sums of grad_kernel stay in registers over all tiles, the sums leave as one row of
+// partial sums per workgroup.  x and grad_input go through a transposition in the wave's own part of LDS:
+// in the layout of the matrix cores a load touches 64 bytes of each of 16 channels, which memory
+// serves at 2.6-3.0 TB/s whatever else happens, four channels of 256 bytes at 4.0 (probed with loads and
+// stores alone, 64 channels of 1024 x 1024).
+//
+// 1024 x 1024, 14 outputs, us over the channels below: 4: 167, 20: 217, 45: 283, 70: 448, 95: 503, where two passes of
+// seven outputs on the fp32 instruction took 236 (20), 328 (48) and about 700 (95); seven outputs: 105 over 20 (118),
+// 411 over 100 (448).  Bound by the vector and matrix pipes together below about 60 channels (the split of A and
+// x is a third of the vector instructions; the waves of a workgroup are in the same phase, so that the two
+// pipes overlap little), above by memory (2.7 TB/s of channels that are read, and read and written).
+// A training step at 1024 x 1024, depth 100: 6.35 -> 5.33 ms; 4 x 512 x 512: 6.25 -> 4.99; 2048 x 2048, two
+// channels per layer, depth 200: 275 -> 194.
+//
+// Tried on the way: waves that walk the channels on their own tile (weights in LDS, loads in the matrix layout): 650 us
+// over 95 channels, 320 over 45; two workgroups of four waves per compute unit: 604 and 293; for 5 to 8 blocks
+// two chunks of at most 4: 588.  Any register spilt in the loop costs 10 % (its reload waits for all loads and stores).
+#include "msd_group.h"
+#include "msd_split.h"
+
+#include <algorithm>
+
+
+namespace msd {
+namespace group2d {
+namespace {
+
+constexpr int kWaves = 8;                         // of a workgroup; one workgroup per compute unit
+constexpr int kSegment = 32;                      // voxels of a row whose A a wave gathers
+constexpr int kVoxelBytes = 2 * 64;               // of a voxel's rows of a slab in LDS
+constexpr int kPartBytes = kSegment * kVoxelBytes;
+constexpr int kSlabBytes = 3 * kPartBytes;
+constexpr int kBiasColumns = 8;                   // per slab
+
+
+// LDS of a wave for a unit of voxels: 16 channels of x in three parts (the sums for grad_input take less)
+constexpr int unit_bytes(int voxels) { return 3 * 16 * (2 * voxels + 16); }
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
+
+// Row m of a slab's 64: the halves of 32 belong to the lanes h = 0 and 1 of the gather.  A lane holds
+// whole outputs (the folds at the image's edges move values between an output's rows): three of nine
+// taps each, and of the seventh output, which both gather, five or four taps.
+struct Slot {
+    int output, tap;                              // tap < 0: a row of zeros
+};
+__host__ __device__ __forceinline__ Slot slot_of(int m)
+{
+    const int h = m / 32 % 2, s = m % 32, first = m / kRows * kSlabOut;
+    if (s < 27) return Slot{first + 3 * h + s / kTaps, s % kTaps};
+    const int tap = 5 * h + s - 27;
+    return Slot{first + 6, tap < kTaps ? tap : -1};
+}
+
+// A voxel's rows lie in eight pieces of 16 bytes, piece i at i ^ turn(voxel): the 16 lanes that read one
+// piece of 16 consecutive voxels, the 16 that write it and the 32 that read 16 rows of two times 4 voxels,
+// 8 apart, transposed all meet the 64 banks once.
+__device__ __forceinline__ uint32_t turn(uint32_t voxel) { return voxel / 2 % 2 * 2 + voxel / 8 % 2 * 4 + voxel / 4 % 2; }
+
+// The channels' blocks of 16 are cut into n chunks: `large` chunks of `blocks` blocks, then chunks
+// of one less.  A chunk has `wgs` workgroups (the smaller ones: `wgs_small`).
+struct Chunks {
+    int n, large, blocks, wgs, wgs_small;
+    __host__ __device__ int size(int i) const { return i < large ? blocks : blocks - 1; }
+    __host__ __device__ int rows(int i) const { return i < large ? wgs : wgs_small; }
+    __host__ __device__ int first_block(int i) const { return i * blocks - (i > large ? i - large : 0); }
+    __host__ __device__ int first_wg(int i) const { return i <= large ? i * wgs : large * wgs + (i - large) * wgs_small; }
+};
+
+// n / d for 0 <= n < 2^31 without a division.
+struct Divisor {
+    uint32_t magic;
+    int shift;
+    __host__ explicit Divisor(uint32_t d = 1) : shift(0)
+    {
+        while (((uint64_t)1 << shift) < d) shift++;
+        magic = (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << shift) - d)) / d + 1);
+    }
+    __device__ __forceinline__ int of(int n) const { return (int)((__umulhi((uint32_t)n, magic) + (uint32_t)n) >> shift); }
+};
+
+struct PullArgs {
+    int C, update;                                // channels of x; the first `update` of them have grad_input
+    int mask_from;                                // channels from here on are masked with their activation
+    int H, W, segs, items;                        // items: segments of an image
+    int tiles, image_tiles;                       // of all images, of one
+    Divisor by_segs, by_tiles;
+    int reverse;                                  // walk the tiles from the last to the first
+    int dmax;
+    Chunks chunks;
+    int64_t sb, sc, sy;                           // strides of x and of the gradients
+    Outputs out;
+};
+
+__device__ __forceinline__ float load1(uint64_t base, uint32_t off)
+{
+    float d[1];
+    load_global_vec<1>(base, off, d);
+    return d[0];
+}
+
+// Between LDS accesses of one wave: LDS executes them in order, only the compiler has to be kept from
+// reordering them.
+__device__ __forceinline__ void own_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// Between the LDS accesses of a workgroup (of LDS only: the loads and stores of the units stay in flight).
+__device__ __forceinline__ void tile_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+__device__ __forceinline__ float part_value(const char *p)        // one bf16 in LDS
+{
+    return (float)*reinterpret_cast<const __bf16 *>(p);
+}
+
+// The sources of one voxel (or row) u of an axis of n through the outer taps of dilation d
+// (adjoint_sources): `up` is read by tap 0 where it lies inside and is otherwise the mirrored source of
+// tap 2, `down` the other way round, so that two loads hold all of them.
+struct Sides {
+    int up, down;
+    bool up_in, down_in;
+};
+__device__ __forceinline__ Sides sides(int u, int n, int d)
+{
+    Sides s;
+    s.up_in = u + d < n;
+    s.down_in = u >= d;
+    s.up = s.up_in ? u + d : 2 * n - 1 - d - u;
+    s.down = s.down_in ? u - d : d - 1 - u;
+    return s;
+}
+__device__ __forceinline__ void fold(const Sides &s, float &tap0, float &tap2)
+{
+    const float up = tap0, down = tap2;
+    tap0 = (s.up_in ? up : 0.f) + (s.down_in ? 0.f : down);
+    tap2 = (s.down_in ? down : 0.f) + (s.up_in ? 0.f : up);
+}
+
+// What a workgroup of pull_rows keeps in LDS besides A and the waves' own space.
+struct Source {                                   // an output's place in bytes: its dilation in rows and in voxels, its plane
+    uint32_t rows, voxels, plane, pad;
+};
+struct PullShared {
+    Source sources[kMaxOut];
+    int bad_again, bad_tile[kWaves];
+    f32x4_t bias_sums[kWaves * kWave];                // of the lanes' outputs at their voxels (not in registers: there are none left)
+};
+
+// G slabs of rows; P waves share a block of 16 channels (the tile's voxels in as many parts).
+template <int G, int P> struct PullShape {
+    static constexpr int kSegs = kWaves / G;             // segments of a tile
+    static constexpr int kSteps = 2 * G;                 // of 32 rows m
+    static constexpr int kTiles = 4 * G;                 // of 16 rows m
+    static constexpr int kUnit = kSegs * kSegment / P < 64 ? 32 : 64;      // voxels that a wave takes through the products at a time
+    static constexpr int kUnits = kSegs * kSegment / P / kUnit;
+    static constexpr int kVec = kUnit / 16;              // 16-byte accesses per lane for a unit of 16 channels
+    static constexpr int kLanes = kUnit / 4;             // lanes of a channel in one of them
+    static constexpr int kOwnBytes = unit_bytes(kUnit);
+    static constexpr int kLaneOut = 4;                   // outputs that a lane of the gather holds
+};
+
+// What the kernel keeps for its life: the weights of rows 32 step + 8 q .. of channel n in parts, the sums of
+// grad_kernel.
+template <int G> struct PullState {
+    bf16x8_t w[2 * G][3];
+    bool weights_split;
+    f32x4_t sums[4 * G];
+};
+
+// The tiles of a workgroup.  True where units were left out that hold values which cannot be split: the second
+// run (WHOLE) takes these, with the fp32 instruction.  Apart, so that it keeps no registers in the first.
+template <int G, int P, bool WHOLE>
+__device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__restrict__ x, const float *gy, float *gx, float *row,
+                                           char *lds, PullShared &shared, int tid, int wave, int blocks, int c0, int wgs, int wg,
+                                           PullState<G> &state)
+{
+    using S = PullShape<G, P>;
+    constexpr int kSegs = S::kSegs, kSteps = S::kSteps, kTiles = S::kTiles, kUnit = S::kUnit, kUnits = S::kUnits, kVec = S::kVec;
+    constexpr int kLanes = S::kLanes, kOwnBytes = S::kOwnBytes, kLaneOut = S::kLaneOut;
+    const int lane = tid % kWave;
+    const int cb = wave / P, ch0 = c0 + cb * 16;  // the wave's block
+    const bool active = cb < blocks, update = ch0 < a.update;       // uniform
+    char *const A = lds;
+    char *const own = lds + kSegs * G * kSlabBytes + wave * kOwnBytes;
+    bf16x8_t(&w)[kSteps][3] = state.w;
+    f32x4_t(&sums)[kTiles] = state.sums;
+
+    struct Tile {
+        int first;                                // segment of its image
+        int64_t img;                              // byte offset of the image
+        uint32_t sign;                            // of x in this tile
+    };
+    struct Place {
+        int x0, skip, y;                          // first voxel, voxels that belong to the segment before, row
+        bool valid;
+    };
+    // (past the last tile that one again)
+    auto tile_of = [&](int tile) {
+        Tile t;
+        const int it0 = min(tile, a.tiles - 1), it = a.reverse ? a.tiles - 1 - it0 : it0;
+        const int b = a.by_tiles.of(it);
+        t.first = (it - b * a.image_tiles) * kSegs;
+        t.img = (int64_t)b * a.sb * 4;
+        t.sign = (uint32_t)it << 31;
+        return t;
+    };
+    auto locate = [&](const Tile &t, int segment) {
+        Place p;
+        p.valid = t.first + segment < a.items;
+        const int it = min(t.first + segment, a.items - 1);
+        p.y = a.by_segs.of(it);
+        const int own0 = (it - p.y * a.segs) * kSegment;
+        p.x0 = min(own0, a.W - kSegment);         // (the last segment of a row overlaps the one before)
+        p.skip = p.valid ? own0 - p.x0 : kSegment;
+        return p;
+    };
+    const uint32_t plane = (uint32_t)a.sc * 4u;
+
+    // The tiles: kSegs consecutive segments of an image each; every workgroup of an XCD works on neighbouring ones.
+    const int lb = block_for_xcd(wg, wgs, wgs % kXcds == 0);
+
+    // ---- x and grad_input of a unit: lane (channel lane / kLanes of kVec x .., four voxels lane % kLanes)
+    const int lv = lane % kLanes, lc = lane / kLanes;               // voxels 4 lv .., channels lc + kRows4 i
+    constexpr int kChannels = kWave / kLanes;     // channels of one access
+    const uint32_t lane_plane = (uint32_t)lc * plane;
+    struct Unit {
+        int64_t img;                              // byte offset of the image
+        uint32_t at;                              // the lane's of (row, voxel)
+        int skip;                                 // first of its four voxels that is its segment's own (0: all, 4: none)
+    };
+    auto unit_of = [&](const Tile &t, int u) {
+        const int first = ((wave % P) * kUnits + u) * (kUnit / kSegment);
+        const Place p0 = locate(t, first), p1 = locate(t, first + kUnit / kSegment - 1);
+        const int sel = lv / (kSegment / 4), v4 = lv % (kSegment / 4) * 4;
+        const uint32_t at0 = 4u * (uint32_t)(p0.y * (int)a.sy + p0.x0), at1 = 4u * (uint32_t)(p1.y * (int)a.sy + p1.x0);
+        Unit un;
+        un.img = t.img;
+        un.at = (sel ? at1 : at0) + 4u * (uint32_t)v4;
+        un.skip = min(max((sel ? p1.skip : p0.skip) - v4, 0), 4);
+        return un;
+    };
+    // channels from `limit` on: that channel before it again
+    auto request = [&](const float *from, int limit, const Unit &un, f32x4_t (&d)[kVec]) {
+        uint64_t base = reinterpret_cast<uint64_t>(from) + (uint64_t)un.img + (uint64_t)min(ch0, limit - 1) * plane;
+        asm volatile("" : "+s"(base));           // (scalar base, 32-bit lane offsets)
+        const uint32_t last = (uint32_t)min(max(limit - 1 - ch0, 0), 15) * plane;
+        uint32_t at = lane_plane;
+        asm volatile("" : "+v"(at));             // (nothing of this is kept over the tiles)
+#pragma unroll
+        for (int i = 0; i < kVec; i++) {
+            float v4[4];
+            load_global_vec4_unaligned(base, min(at + (uint32_t)(kChannels * i) * plane, last) + un.at, v4);
+            d[i] = f32x4_t{v4[0], v4[1], v4[2], v4[3]};
+        }
+    };
+    const int g_limit = max(a.update, 1);
+
+    f32x4_t xs[kVec], gs[kVec];
+
+    // ---- the gather: lane (v, h) takes its outputs at voxel v of the wave's segment, 36 values for 32 rows
+    // m.  Its loads are issued in the tile before, in front of that tile's last stores and requests (all of
+    // them retire in order: behind those it would wait for memory).
+    const int segment = wave / G, slab = wave % G;
+    const int v = lane % kSegment, h = lane / kSegment;
+    const uint32_t bias = 4u * (uint32_t)(a.dmax * (int)a.sy);
+    auto source = [&](int j) {
+        int o = j < 3 ? 3 * h + j : 6;
+        asm volatile("" : "+v"(o));
+        return shared.sources[slab * kSlabOut + o];
+    };
+    auto away = [&](const Place &p) {             // uniform: from all edges
+        return p.x0 >= a.dmax && p.x0 + kSegment + a.dmax <= a.W && p.y >= a.dmax && p.y + a.dmax < a.H;
+    };
+    float val[kLaneOut][3][3];
+    auto gather = [&](const Tile &t, const Place &p) {
+        const uint32_t u = (uint32_t)(p.x0 + v);
+        if (away(p)) {
+            const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)(t.img + (int64_t)p.y * a.sy * 4) - bias;
+#pragma unroll
+            for (int j = 0; j < kLaneOut; j++) {
+                const Source o = source(j);
+                const uint32_t c = o.plane + bias + 4u * u;
+#pragma unroll
+                for (int ky = 0; ky < 3; ky++) {
+                    const uint32_t r = ky == 0 ? c + o.rows : ky == 1 ? c : c - o.rows;
+                    val[j][ky][0] = load1(base, r + o.voxels);
+                    val[j][ky][1] = load1(base, r);
+                    val[j][ky][2] = load1(base, r - o.voxels);
+                }
+                __builtin_amdgcn_sched_barrier(0);    // (an output's addresses at a time: registers)
+            }
+        } else {
+            const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)t.img;
+#pragma unroll
+            for (int j = 0; j < kLaneOut; j++) {
+                const Source o = source(j);
+                const int d = (int)(o.voxels / 4u);
+                const Sides sx = sides((int)u, a.W, d), sy = sides(p.y, a.H, d);
+#pragma unroll
+                for (int ky = 0; ky < 3; ky++) {
+                    const int y = ky == 0 ? sy.up : ky == 1 ? p.y : sy.down;
+                    const uint32_t r = o.plane + 4u * (uint32_t)(y * (int)a.sy);
+                    val[j][ky][0] = load1(base, r + 4u * (uint32_t)sx.up);
+                    val[j][ky][1] = load1(base, r + 4u * u);
+                    val[j][ky][2] = load1(base, r + 4u * (uint32_t)sx.down);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    auto gathered = [&](const Place &p, bool count) {
+        if (!away(p)) {
+#pragma unroll
+            for (int j = 0; j < kLaneOut; j++) {
+                const int d = (int)(source(j).voxels / 4u);
+                const Sides sx = sides(p.x0 + v, a.W, d), sy = sides(p.y, a.H, d);
+#pragma unroll
+                for (int ky = 0; ky < 3; ky++) fold(sx, val[j][ky][0], val[j][ky][2]);
+#pragma unroll
+                for (int r = 0; r < 3; r++) fold(sy, val[j][0][r], val[j][2][r]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (p.skip > 0 || a.out.n < G * kSlabOut) {                 // uniform
+#pragma unroll
+            for (int j = 0; j < kLaneOut; j++) {
+                const bool ok = v >= p.skip && slab * kSlabOut + (j < 3 ? 3 * h + j : 6) < a.out.n;
+#pragma unroll
+                for (int t = 0; t < kTaps; t++) val[j][t / 3][t % 3] = ok ? val[j][t / 3][t % 3] : 0.f;
+            }
+        }
+        if (count) shared.bias_sums[tid] += f32x4_t{val[0][1][1], val[1][1][1], val[2][1][1], val[3][1][1]};
+        // -A at every second voxel: the sums of the bf16 instruction are cut off towards minus infinity, which adds up
+        // over an image where the gradients themselves cancel (bias gradients: an error of 2e-6 instead of 1.2e-7).
+        // For the same reason x changes its sign with the voxel and from tile to tile.
+        const uint32_t odd = (uint32_t)v << 31;
+#pragma unroll
+        for (int j = 0; j < kLaneOut; j++)
+#pragma unroll
+            for (int t = 0; t < kTaps; t++)
+                val[j][t / 3][t % 3] = __uint_as_float(__float_as_uint(val[j][t / 3][t % 3]) ^ odd);
+        // rows m of the lane (slot_of), eight at a time
+        auto eight = [&](int i, float (&e8)[8]) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const int s = 8 * i + e;
+                if (s < 27) {
+                    e8[e] = val[s / 9][s % 9 / 3][s % 3];
+                } else {
+                    const int t0 = s - 27, t1 = s - 22;
+                    e8[e] = h ? (t1 < kTaps ? val[3][t1 / 3 % 3][t1 % 3] : 0.f) : val[3][t0 / 3][t0 % 3];
+                }
+            }
+        };
+        char *const at = A + (segment * G + slab) * kSlabBytes + v * kVoxelBytes;
+        const uint32_t piece = 16 * (4 * (uint32_t)h ^ turn((uint32_t)v));
+        float bad = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float e8[8];
+            eight(i, e8);
+            Split8 s;
+            bad += split8(e8, s);
+#pragma unroll
+            for (int k = 0; k < 3; k++) *reinterpret_cast<bf16x8_t *>(at + k * kPartBytes + (piece ^ 16 * i)) = s.p[k];
+        }
+        const bool any = __any(bad != bad);
+        if (any) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float e8[8];
+                eight(i, e8);
+                Split8 s;
+                split_any(e8, s);
+#pragma unroll
+                for (int k = 0; k < 3; k++) *reinterpret_cast<bf16x8_t *>(at + k * kPartBytes + (piece ^ 16 * i)) = s.p[k];
+            }
+        }
+        if (lane == 0) shared.bad_tile[wave] = any;
+    };
+
+    // ---- the products of a unit.  The wave's own space holds x as [part][channel][voxel], then what is added to
+    // grad_input as [channel][voxel]: loads and stores go by channel in whole lines, the matrix cores take 16
+    // channels at once (loaded in that form, 64 bytes of 16 channels at a time, memory gives 2.6 to 3.0 TB/s instead of 4).
+    constexpr int kXRow = 2 * kUnit + 16, kDRow = 4 * kUnit + 16;   // bytes of a channel (16 apart in the banks)
+    const int first_seg = (wave % P) * kUnits * (kUnit / kSegment); // of the wave's first unit
+    auto clear_skipped = [&](const Unit &un) {    // an infinity there belongs to the other segment
+        if (__any(un.skip > 0)) {
+#pragma unroll
+            for (int i = 0; i < kVec; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) xs[i][e] = e >= un.skip ? xs[i][e] : 0.f;
+        }
+    };
+    // bit 4 i + e: the channel's gradient at voxel e is kept
+    auto mask_of = [&]() {
+        uint32_t bits = 0xffffu;
+        if (ch0 + 16 > a.mask_from) {             // uniform
+            bits = 0;
+#pragma unroll
+            for (int i = 0; i < kVec; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    bits |= ch0 + lc + kChannels * i < a.mask_from || 0.f < xs[i][e] ? 1u << (4 * i + e) : 0u;
+        }
+        return bits;
+    };
+    // x in parts to the wave's own space; NaN where a value cannot be split
+    auto signed_x = [&](int i, int e, uint32_t sign) {
+        return __uint_as_float(__float_as_uint(xs[i][e]) ^ (sign ^ (uint32_t)(e % 2) << 31));
+    };
+    auto put_x = [&](uint32_t sign) {
+        float rest = 0.f;
+#pragma unroll
+        for (int i = 0; i < kVec; i += 2) {
+            float x8[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) x8[e] = signed_x(i + e / 4, e % 4, sign);
+            Split8 s;
+            rest += split8(x8, s);
+            typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+#pragma unroll
+            for (int p = 0; p < 3; p++) {
+                char *const at = own + (p * 16 + lc + kChannels * i) * kXRow + 8 * lv;
+                *reinterpret_cast<bf16x4_t *>(at) = __builtin_shufflevector(s.p[p], s.p[p], 0, 1, 2, 3);
+                *reinterpret_cast<bf16x4_t *>(at + kChannels * kXRow) = __builtin_shufflevector(s.p[p], s.p[p], 4, 5, 6, 7);
+            }
+        }
+        return rest;
+    };
+    // what the wave's own space holds for grad_input, added to it and masked
+    auto add_d = [&](uint32_t bits) {
+#pragma unroll
+        for (int i = 0; i < kVec; i++) {
+            const f32x4_t d = *reinterpret_cast<const f32x4_t *>(own + (lc + kChannels * i) * kDRow + 16 * lv);
+#pragma unroll
+            for (int e = 0; e < 4; e++) gs[i][e] += e % 2 ? -d[e] : d[e];
+        }
+        if (ch0 + 16 > a.mask_from) {             // uniform
+#pragma unroll
+            for (int i = 0; i < kVec; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) gs[i][e] = bits & 1u << (4 * i + e) ? gs[i][e] : 0.f;
+        }
+    };
+    constexpr int kK = kUnit / 32;                // steps of 32 voxels: the segments of the unit
+    // False where a value cannot be split (and nothing is computed).
+    auto compute = [&](int u, bool split, uint32_t sign_bit, const Unit &un, const Unit &next) {
+        const float sign = __uint_as_float(sign_bit | 0x3f800000u);
+        uint32_t ll = (uint32_t)lane;
+        if (G > 1 && P < 4) asm volatile("" : "+v"(ll));            // (no LDS addresses are kept over the tiles: registers)
+        const uint32_t nn = ll % 16, qq = ll / 16 % 4;
+        const char *const Au = A + (first_seg + u * kK) * G * kSlabBytes;
+        // rows 16 t + n, voxels 8 q .. of segment j (the lane's address is that of voxel 8 q + n / 4 (+ 4), rows
+        // 4 (n % 4) .., which the read transposes)
+        const uint32_t tr_voxel = 8 * qq + nn / 4;
+        const char *const tr = Au + tr_voxel * kVoxelBytes + nn % 2 * 8;
+        const uint32_t tr_piece = 16 * (nn % 4 / 2 ^ turn(tr_voxel)), tr_next = 16 * (nn % 4 / 2 ^ turn(tr_voxel + 4));
+        auto read_rows = [&](int j, int t, bf16x8_t(&to)[3]) {
+            typedef short s16x4_t __attribute__((ext_vector_type(4)));
+            typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+            typedef __attribute__((address_space(3))) s16x4_t *lds_tr_t;
+#pragma unroll
+            for (int p = 0; p < 3; p++) {
+                const char *const at = tr + (j * G + t / 4) * kSlabBytes + p * kPartBytes;
+                const bf16x4_t lo = __builtin_bit_cast(
+                    bf16x4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)(at + (tr_piece ^ (uint32_t)(t % 4 * 32)))));
+                const bf16x4_t hi = __builtin_bit_cast(
+                    bf16x4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)(at + 4 * kVoxelBytes + (tr_next ^ (uint32_t)(t % 4 * 32)))));
+                to[p] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+            }
+        };
+        // voxels 16 s + n of the unit, rows 32 i + 8 q ..
+        const char *const vox = Au + nn * kVoxelBytes;
+        const uint32_t vox_piece = 16 * (qq ^ turn(nn));
+        auto read_voxels = [&](int s, int i, bf16x8_t(&to)[3]) {
+#pragma unroll
+            for (int p = 0; p < 3; p++)
+                to[p] = *reinterpret_cast<const bf16x8_t *>(vox + (s / 2 * G + i / 2) * kSlabBytes + p * kPartBytes +
+                                                            s % 2 * 16 * kVoxelBytes + (vox_piece ^ (uint32_t)(i % 2 * 64)));
+        };
+        clear_skipped(un);
+        const uint32_t bits = mask_of();
+        const float rest = put_x(sign_bit);
+        const bool done = split && !__any(rest != rest);            // uniform
+        __builtin_amdgcn_sched_barrier(0);        // (the scheduler would move the loads to where they are used)
+        request(x, a.C, next, xs);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!done) return false;
+        own_sync();
+        // Both products in stages of two chains of six matrix instructions, whose operands are read from LDS a
+        // stage ahead (where there are registers for it).
+        constexpr bool kAhead = G == 1 || P > 1;
+        bf16x8_t op[2][2][3], xp[kK][3];
+        constexpr int kRowStages = kTiles * kK / 2, kVoxelStages = kSteps * kK;
+        // stage r: tiles 2 (r / kK) and the next at segment r % kK
+        auto stage_rows = [&](int r, bf16x8_t(&to)[2][3]) {
+#pragma unroll
+            for (int o = 0; o < 2; o++) read_rows(r % kK, r / kK * 2 + o, to[o]);
+        };
+        // stage r: step r % kSteps at the voxels of segment r / kSteps
+        auto stage_voxels = [&](int r, bf16x8_t(&to)[2][3]) {
+#pragma unroll
+            for (int s = 0; s < 2; s++) read_voxels(r / kSteps * 2 + s, r % kSteps, to[s]);
+        };
+        f32x4_t acc[2];
+        bf16x8_t high[2];
+        stage_rows(0, op[0]);
+#pragma unroll
+        for (int j = 0; j < kK; j++)
+#pragma unroll
+            for (int p = 0; p < 3; p++)
+                xp[j][p] = *reinterpret_cast<const bf16x8_t *>(own + (p * 16 + nn) * kXRow + (32 * j + 8 * qq) * 2);
+#pragma unroll
+        for (int r = 0; r < kRowStages; r++) {
+            if (!kAhead && r > 0) stage_rows(r, op[r % 2]);
+            if (kAhead && r + 1 < kRowStages) stage_rows(r + 1, op[(r + 1) % 2]);
+            if (kAhead && r + 1 == kRowStages) stage_voxels(0, op[(r + 1) % 2]);
+            __builtin_amdgcn_sched_barrier(0);
+            // (the products of the high parts of both segments last: each instruction cuts its sum off at the size
+            // that it has reached)
+#pragma unroll
+            for (int k = 0; k < 5; k++)
+#pragma unroll
+                for (int o = 0; o < 2; o++)
+                    acc[o] = mfma_split(op[r % 2][o], xp[r % kK], k == 0 && r % kK == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[o], k);
+            if (r % kK == kK - 1) {
+#pragma unroll
+                for (int j = 0; j < kK; j++)
+#pragma unroll
+                    for (int o = 0; o < 2; o++)
+                        acc[o] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j == kK - 1 ? op[r % 2][o][0] : high[o], xp[j][0], acc[o], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int o = 0; o < 2; o++) high[o] = op[r % 2][o][0];
+            }
+            if (r % kK == kK - 1) {
+#pragma unroll
+                for (int o = 0; o < 2; o++) {
+                    sums[r / kK * 2 + o] += sign * acc[o];
+                    asm volatile("" : "+v"(sums[r / kK * 2 + o]));  // (here and not at the end of the tile: registers)
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (update) {                             // uniform
+            // (x has been read: the wave's space is free for the sums)
+            f32x4_t d[2], all[2];
+#pragma unroll
+            for (int r = 0; r < kVoxelStages; r++) {
+                const int i = r % kSteps;
+                if (!kAhead) stage_voxels(r, op[(kRowStages + r) % 2]);
+                if (kAhead && r + 1 < kVoxelStages) stage_voxels(r + 1, op[(kRowStages + r + 1) % 2]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int k = 0; k < 5; k++)
+#pragma unroll
+                    for (int s = 0; s < 2; s++)
+                        d[s] = mfma_split(op[(kRowStages + r) % 2][s], w[i], k == 0 && i % 2 == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : d[s], k);
+                if (i % 2 == 0) {
+#pragma unroll
+                    for (int s = 0; s < 2; s++) high[s] = op[(kRowStages + r) % 2][s][0];
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+#pragma unroll
+                        for (int s = 0; s < 2; s++)
+                            d[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j ? op[(kRowStages + r) % 2][s][0] : high[s], w[i - 1 + j][0], d[s], 0, 0, 0);
+                }
+                // Summed slab by slab from zero and added to grad_input last: a chain of products that started from it
+                // would round each of them to its size.
+                if (i % 2 == 1) {
+#pragma unroll
+                    for (int s = 0; s < 2; s++) {
+                        all[s] = i == 1 ? d[s] : all[s] + d[s];
+                        if (i == kSteps - 1)
+                            *reinterpret_cast<f32x4_t *>(own + nn * kDRow + (16 * (r / kSteps * 2 + s) + 4 * qq) * 4) = all[s];
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            own_sync();
+            add_d(bits);
+            own_sync();
+        }
+        return true;
+    };
+    // The same with the fp32 instruction, for values that cannot be split among x, A or the weights.
+    auto compute_whole = [&](int u, uint32_t sign_bit, const Unit &un) {
+        const float sign = __uint_as_float(sign_bit | 0x3f800000u);
+        clear_skipped(un);
+        const uint32_t bits = mask_of();
+        uint32_t ll = (uint32_t)lane;
+        asm volatile("" : "+v"(ll));
+        const uint32_t nn = ll % 16, qq = ll / 16 % 4;
+        const char *const Au = A + (first_seg + u * kK) * G * kSlabBytes;
+        auto value = [&](uint32_t voxel, uint32_t m) {
+            const char *const at = Au + (voxel / kSegment * G + m / kRows) * kSlabBytes + voxel % kSegment * kVoxelBytes +
+                                   16 * (m % kRows / 8 ^ turn(voxel)) + m % 8 * 2;
+            return part_value(at) + part_value(at + kPartBytes) + part_value(at + 2 * kPartBytes);
+        };
+        own_sync();
+#pragma unroll
+        for (int i = 0; i < kVec; i++)
+            *reinterpret_cast<f32x4_t *>(own + (lc + kChannels * i) * kDRow + 16 * lv) =
+                f32x4_t{signed_x(i, 0, sign_bit), signed_x(i, 1, sign_bit), signed_x(i, 2, sign_bit), signed_x(i, 3, sign_bit)};
+        own_sync();
+#pragma unroll
+        for (int t = 0; t < kTiles; t++)
+#pragma unroll
+            for (int j = 0; j < kK; j++) {
+                f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+                for (int e = 0; e < 8; e++) {
+                    const uint32_t voxel = 32 * j + 8 * qq + (uint32_t)e;
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(value(voxel, 16 * t + nn),
+                                                               *reinterpret_cast<const float *>(own + nn * kDRow + 4 * voxel), acc, 0, 0, 0);
+                }
+                sums[t] += sign * acc;
+            }
+        if (update) {
+            own_sync();
+#pragma unroll 1
+            for (int s = 0; s < kUnit / 16; s++) {
+                f32x4_t all = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < kSteps; i++) {
+                    f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        const float we = (float)w[i][0][e] + (float)w[i][1][e] + (float)w[i][2][e];
+                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(value(16 * s + nn, 32 * i + 8 * qq + e), we, d, 0, 0, 0);
+                    }
+                    all += d;
+                }
+                *reinterpret_cast<f32x4_t *>(own + nn * kDRow + (16 * s + 4 * qq) * 4) = all;
+            }
+            own_sync();
+            add_d(bits);
+        }
+        own_sync();
+    };
+    auto store = [&](const Unit &un, bool all) {
+        // Buffer stores, whose lanes past the end of the buffer store nothing: there is no branch around
+        // them.  (Loads and stores retire through one in-order counter, and a store that may be skipped turns the
+        // wait for the next unit's values, requested before it, into one for the store itself.)
+        const uint64_t base = reinterpret_cast<uint64_t>(gx) + (uint64_t)un.img + (uint64_t)ch0 * plane;
+        uint32_t at = lane_plane;
+        asm volatile("" : "+v"(at));
+        const int end = un.skip == 0 && all ? a.update - ch0 : 0;
+        const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(base), 0, 0xfffffff0u, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < kVec; i++) {
+            typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+            const uint32_t plane_at = at + (uint32_t)(kChannels * i) * plane;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, gs[i]), buffer,
+                                                   lc + kChannels * i < end ? plane_at + un.at : 0xffffffffu, 0, 0);
+        }
+        if (__any(un.skip % 4 != 0)) {            // some lanes own the last of their four voxels only
+#pragma unroll
+            for (int i = 0; i < kVec; i++)
+#pragma unroll
+                for (int e = 1; e < 4; e++)
+                    if (all && lc + kChannels * i < a.update - ch0 && un.skip > 0 && e >= un.skip)
+                        reinterpret_cast<__attribute__((address_space(1))) float *>(base + (uint64_t)(lane_plane + (uint32_t)(kChannels * i) * plane) + un.at)[e] = gs[i][e];
+        }
+    };
+    // values of the tile at hand that can be split: A and the weights
+    auto tile_split = [&]() {
+        int bad = 0;
+#pragma unroll
+        for (int i = 0; i < kWaves; i++) bad |= shared.bad_tile[i];
+        return state.weights_split && __builtin_amdgcn_readfirstlane(bad) == 0;
+    };
+
+    if constexpr (WHOLE) {
+#pragma unroll 1
+        for (int tile = lb; tile < a.tiles; tile += wgs) {
+            const Tile t = tile_of(tile);
+            const Place here = locate(t, segment);
+            gather(t, here);
+            gathered(here, false);
+            __syncthreads();
+            if (active) {
+                const bool split = tile_split();
+#pragma unroll 1
+                for (int u = 0; u < kUnits; u++) {
+                    const Unit un = unit_of(t, u);
+                    request(x, a.C, un, xs);
+                    request(gx, g_limit, un, gs);
+                    clear_skipped(un);
+                    const float rest = put_x(t.sign);
+                    if (split && !__any(rest != rest)) continue;    // (the first run has done it)
+                    compute_whole(u, t.sign, un);
+                    store(un, true);
+                }
+            }
+            __syncthreads();
+        }
+        return false;
+    } else {
+        Tile now = tile_of(lb);
+        Unit un = unit_of(now, 0);
+        request(x, a.C, un, xs);
+        request(gx, g_limit, un, gs);
+        bool again = false;                       // units were left to the second run
+        Place here = locate(now, segment);
+        gather(now, here);
+        for (int tile = lb; tile < a.tiles; tile += wgs) {          // uniform over the workgroup
+            gathered(here, true);
+            tile_sync();
+            const Tile then = tile_of(tile + wgs);
+            here = locate(then, segment);
+            if (active) {
+                const bool split = tile_split();
+#pragma unroll
+                for (int u = 0; u < kUnits; u++) {
+                    const Unit next = u + 1 < kUnits ? unit_of(now, u + 1) : unit_of(then, 0);
+                    const bool done = compute(u, split, now.sign, un, next);
+                    again = again || !done;
+                    if (u + 1 == kUnits) gather(then, here);
+                    store(un, done);
+                    __builtin_amdgcn_sched_barrier(0);
+                    request(gx, g_limit, next, gs);
+                    __builtin_amdgcn_sched_barrier(0);
+                    un = next;
+                }
+            } else {
+                gather(then, here);
+            }
+            now = then;
+            tile_sync();
+        }
+        return again;
+    }
+}
+
+template <int G, int P>
+__global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, const float *__restrict__ x, const float *gy,
+                                                             float *gx, float *__restrict__ part, float *__restrict__ bias_part)
+{
+    constexpr int kSegs = PullShape<G, P>::kSegs, kTiles = PullShape<G, P>::kTiles, kLaneOut = PullShape<G, P>::kLaneOut;
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
+    const int n = lane % 16, q = lane / 16;
+    const int bid = blockIdx.x, big = a.chunks.large * a.chunks.wgs;
+    const int chunk = bid < big ? bid / a.chunks.wgs : a.chunks.large + (bid - big) / a.chunks.wgs_small;
+    const int blocks = a.chunks.size(chunk), c0 = a.chunks.first_block(chunk) * 16;
+    const int wgs = a.chunks.rows(chunk), wg = bid - a.chunks.first_wg(chunk);
+    const int cb = wave / P, ch0 = c0 + cb * 16;  // the wave's block
+    __shared__ PullShared shared;
+    PullState<G> state;
+
+    if (tid == 0) shared.bad_again = 0;
+    if (tid < G * kSlabOut) {
+        const int o = min(tid, a.out.n - 1), d = a.out.dil[o];
+        shared.sources[tid] = Source{4u * (uint32_t)(d * (int)a.sy), 4u * (uint32_t)d, (uint32_t)o * ((uint32_t)a.sc * 4u), 0};
+    }
+    state.weights_split = true;
+#pragma unroll
+    for (int step = 0; step < 2 * G; step++) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const Slot m = slot_of(32 * step + 8 * q + i);
+            const bool ok = m.tap >= 0 && m.output < a.out.n && ch0 + n < a.update;
+            const float k = a.out.k[ok ? m.output : 0][ok ? (int64_t)(ch0 + n) * kTaps + m.tap : 0];
+            v[i] = ok ? k : 0.f;
+        }
+        Split8 s;
+        const float bad = split8(v, s);
+        if (__any(bad != bad)) {
+            split_any(v, s);
+            state.weights_split = false;
+        }
+#pragma unroll
+        for (int p = 0; p < 3; p++) state.w[step][p] = s.p[p];
+    }
+    __syncthreads();
+
+    float *const row = part + (int64_t)bid * (a.chunks.blocks * 1024 * G);
+#pragma unroll
+    for (int t = 0; t < kTiles; t++) state.sums[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    shared.bias_sums[tid] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const bool again = pull_tiles<G, P, false>(a, x, gy, gx, row, lds, shared, tid, wave, blocks, c0, wgs, wg, state);
+    if (lane == 0 && again) shared.bad_again = 1;
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(shared.bad_again) != 0) {    // uniform over the workgroup
+        int tid2 = tid;
+        asm volatile("" : "+v"(tid2));           // (nothing of the first run is kept for the second)
+        pull_tiles<G, P, true>(a, x, gy, gx, row, lds, shared, tid2, wave, blocks, c0, wgs, wg, state);
+    }
+
+    // the sums, of the waves that share a block through LDS
+    constexpr int kBlock = 1024 * G;              // sums of a block of channels
+    if constexpr (P == 1) {
+        if (cb < blocks) {
+#pragma unroll
+            for (int t = 0; t < kTiles; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) row[cb * kBlock + (t * 4 + r) * kWave + lane] = state.sums[t][r];
+        }
+    } else {
+        float *const red = reinterpret_cast<float *>(lds);
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < kTiles; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) red[wave * kBlock + (t * 4 + r) * kWave + lane] = state.sums[t][r];
+        __syncthreads();
+        for (int i = tid; i < kWaves / P * kBlock; i += kWaves * kWave) {
+            const int b = i / kBlock;
+            const float *const r = red + b * P * kBlock + i % kBlock;
+            if (b < blocks) row[i] = P == 2 ? r[0] + r[kBlock] : (r[0] + r[kBlock]) + (r[2 * kBlock] + r[3 * kBlock]);
+        }
+    }
+    if (chunk != 0) return;
+    const int v = lane % kSegment, h = lane / kSegment;
+    // the bias gradients: the centre taps, over the lanes' voxels and the segments
+    f32x4_t bias_sum = shared.bias_sums[tid];
+#pragma unroll
+    for (int j = 0; j < kLaneOut; j++)
+#pragma unroll
+        for (int off = kSegment / 2; off > 0; off >>= 1) bias_sum[j] += __shfl_down(bias_sum[j], off, kSegment);
+    float *const red = reinterpret_cast<float *>(lds);
+    __syncthreads();
+    if (v == 0) {
+#pragma unroll
+        for (int j = 0; j < kLaneOut; j++)
+            if (j < 3 || h == 0) red[wave * kBiasColumns + (j < 3 ? 3 * h + j : 6)] = bias_sum[j];
+    }
+    __syncthreads();
+    if (tid < G * kBiasColumns && tid % kBiasColumns < kSlabOut) {
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < kSegs; i++) s += red[i * G * kBiasColumns + tid];
+        bias_part[wg * (G * kBiasColumns) + tid] = s;
+    }
+}
+
+struct SumArgs {
+    Chunks chunks;
+    int columns;                                  // weight columns in all (a multiple of 1024 slabs)
+    int slabs;
+    int stride;                                   // of the rows of partial sums
+    int n;
+    int channels[kMaxOut];                        // input channels of each output
+    float *gk[kMaxOut];
+    float *gb;
+};
+
+// Adds the rows of partial sums, 64 columns per workgroup: 16 waves take every 16th row, their
+// sums are added in order.  The last workgroup takes the biases.
+__global__ __launch_bounds__(1024) void sum_group(const SumArgs a, const float *__restrict__ part,
+                                                  const float *__restrict__ bias_part)
+{
+    __shared__ float lds[16 * kWave];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int col = blockIdx.x * kWave + lane, block = 1024 * a.slabs;
+    const bool bias = (int)blockIdx.x * kWave >= a.columns;
+    const int blk = col / block, big = a.chunks.large * a.chunks.blocks;
+    const int chunk = blk < big ? blk / a.chunks.blocks
+                                : (a.chunks.blocks > 1 ? a.chunks.large + (blk - big) / (a.chunks.blocks - 1) : 0);
+    const int rows = a.chunks.rows(bias ? 0 : chunk);
+    const float *p;
+    int64_t stride;
+    if (bias) {
+        stride = a.slabs * kBiasColumns;
+        p = bias_part + lane % (a.slabs * kBiasColumns);
+    } else {
+        p = part + (int64_t)a.chunks.first_wg(chunk) * a.stride + (blk - a.chunks.first_block(chunk)) * block + col % block;
+        stride = a.stride;
+    }
+    float part_sum[4] = {0.f, 0.f, 0.f, 0.f};     // (short chains, then trees: these are the largest sums)
+    for (int r = wave; r < rows; r += 128) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = p[min(r + 16 * i, rows - 1) * stride];
+#pragma unroll
+        for (int i = 0; i < 8; i++) part_sum[i % 4] += r + 16 * i < rows ? v[i] : 0.f;
+    }
+    lds[wave * kWave + lane] = (part_sum[0] + part_sum[1]) + (part_sum[2] + part_sum[3]);
+    __syncthreads();
+    if (wave != 0) return;
+    float tree[16];
+#pragma unroll
+    for (int w = 0; w < 16; w++) tree[w] = lds[w * kWave + lane];
+#pragma unroll
+    for (int w = 8; w > 0; w /= 2)
+#pragma unroll
+        for (int i = 0; i < w; i++) tree[i] += tree[i + w];
+    const float s = tree[0];
+    if (bias) {
+        const int o = lane / kBiasColumns * kSlabOut + lane % kBiasColumns;
+        if (lane < a.slabs * kBiasColumns && lane % kBiasColumns < kSlabOut && o < a.n) a.gb[o] += s;
+        return;
+    }
+    // column (tile of 16 rows, r, lane (channel, q)) of a block: row 16 tile + 4 q + r
+    const int i = col % block, l = i % kWave;
+    const Slot m = slot_of(i / 256 * 16 + l / 16 * 4 + i / kWave % 4);
+    const int ch = blk * 16 + l % 16;
+    if (m.tap >= 0 && m.output < a.n && ch < a.channels[m.output]) a.gk[m.output][(int64_t)ch * kTaps + m.tap] += s;
+}
+
+// grad_input of the channels that layers of a group wrote, from the outputs of the layers above them
+// in the group.
+//
+// One voxel per lane; the nine values of each output come straight from the caches (a group's planes
+// were written or read by the launches before), with no LDS and no barrier: the launches are bound by
+// their ramp and by the vector cache.
+struct FinishArgs {
+    int H, W, segs, items, dmax;
+    int n, channels, masked;                      // spread_back: outputs above, channels, first one to mask
+    int64_t sb, sc, sy;
+    int dil[kMaxAbove];
+    const float *k[kMaxAbove];                    // of the first of the channels
+};
+
+// The lane's place, and the adjoint gather there.
+struct FinishPlace {
+    int y, u, own;                                // row, voxel, whether the voxel is the lane's own
+    bool away;                                    // uniform: from all edges
+    int64_t img;
+    uint32_t here;
+};
+__device__ __forceinline__ FinishPlace finish_place(const FinishArgs &a, int it)
+{
+    FinishPlace p;
+    const int row = it / a.segs, xw = (it - row * a.segs) * kWave;
+    const int b = row / a.H;
+    p.y = row - b * a.H;
+    const int u0 = xw + threadIdx.x % kWave;
+    p.u = min(u0, a.W - 1);
+    p.own = u0 < a.W;
+    p.away = xw >= a.dmax && xw + kWave + a.dmax <= a.W && p.y >= a.dmax && p.y + a.dmax < a.H;
+    p.img = (int64_t)b * a.sb * 4;
+    p.here = 4u * (uint32_t)(p.y * (int)a.sy + p.u);
+    return p;
+}
+__device__ __forceinline__ void finish_gather(const FinishArgs &a, const FinishPlace &p, uint64_t output, int d, float (&A)[3][3])
+{
+    Sides sx = {p.u + d, p.u - d, true, true}, sy = {p.y + d, p.y - d, true, true};      // y: uniform
+    if (!p.away) {
+        sx = sides(p.u, a.W, d);
+        sy = sides(p.y, a.H, d);
+    }
+#pragma unroll
+    for (int ky = 0; ky < 3; ky++) {
+        const int y = ky == 0 ? sy.up : ky == 1 ? p.y : sy.down;
+        const uint64_t base = output + (uint64_t)(4 * (int64_t)y * a.sy);
+        A[ky][0] = load1(base, 4u * (uint32_t)sx.up);
+        A[ky][1] = load1(base, 4u * (uint32_t)p.u);
+        A[ky][2] = load1(base, 4u * (uint32_t)sx.down);
+    }
+}
+__device__ __forceinline__ void finish_fold(const FinishArgs &a, const FinishPlace &p, int d, float (&A)[3][3])
+{
+    const Sides sx = sides(p.u, a.W, d), sy = sides(p.y, a.H, d);
+#pragma unroll
+    for (int ky = 0; ky < 3; ky++) fold(sx, A[ky][0], A[ky][2]);
+#pragma unroll
+    for (int r = 0; r < 3; r++) fold(sy, A[0][r], A[2][r]);
+}
+
+// The NOUT channels of one layer from the NQ outputs right above, and the channels' ReLU mask: with it
+// they are complete.
+template <int NQ, int NOUT>
+__global__ __launch_bounds__(256) void finish_back(const FinishArgs a, const float *__restrict__ act, float *g)
+{
+    const int lb = block_for_xcd(blockIdx.x, gridDim.x, true);
+    const int it = lb * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    if (it >= a.items) return;                    // uniform over the wave
+    const FinishPlace p = finish_place(a, it);
+    const uint64_t img = reinterpret_cast<uint64_t>(g) + (uint64_t)p.img;
+    const uint64_t ximg = reinterpret_cast<uint64_t>(act) + (uint64_t)p.img;
+    const uint32_t plane = (uint32_t)a.sc * 4u;
+    float sum[NOUT], m[NOUT];
+#pragma unroll
+    for (int c = 0; c < NOUT; c++) {
+        sum[c] = load1(img, (uint32_t)c * plane + p.here);
+        m[c] = load1(ximg, (uint32_t)c * plane + p.here);
+    }
+    float A[NQ][3][3];
+#pragma unroll
+    for (int o = 0; o < NQ; o++) finish_gather(a, p, img + (uint64_t)(NOUT + o) * plane, a.dil[o], A[o]);
+    if (!p.away) {
+#pragma unroll
+        for (int o = 0; o < NQ; o++) finish_fold(a, p, a.dil[o], A[o]);
+    }
+#pragma unroll
+    for (int c = 0; c < NOUT; c++) {
+        float all = 0.f;                          // (output by output, and added to grad_input last: see pull_rows)
+#pragma unroll
+        for (int o = 0; o < NQ; o++) {
+            float one = 0.f;
+#pragma unroll
+            for (int t = 0; t < kTaps; t++) one += a.k[o][c * kTaps + t] * A[o][t / 3][t % 3];
+            all += one;
+        }
+        sum[c] += all;
+        const float v[1] = {0.f < m[c] ? sum[c] : 0.f};
+        if (p.own) store_global_vec<1>(img, (uint32_t)c * plane + p.here, v);
+    }
+}
+
+// What the upper half of a group's outputs adds to all channels that its lower half wrote, before
+// those are completed one layer after the other; the last of them, from `masked` on, are with it.
+__global__ __launch_bounds__(256) void spread_back(const FinishArgs a, const float *__restrict__ act, float *g)
+{
+    const int lb = block_for_xcd(blockIdx.x, gridDim.x, true);
+    const int it = lb * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    if (it >= a.items) return;                    // uniform over the wave
+    const FinishPlace p = finish_place(a, it);
+    const uint64_t img = reinterpret_cast<uint64_t>(g) + (uint64_t)p.img;
+    const uint64_t ximg = reinterpret_cast<uint64_t>(act) + (uint64_t)p.img;
+    const uint32_t plane = (uint32_t)a.sc * 4u;
+    float sum[kMaxLower], m[2];                   // (a layer has one or two channels)
+#pragma unroll
+    for (int c = 0; c < 2; c++) m[c] = load1(ximg, (uint32_t)min(a.masked + c, a.channels - 1) * plane + p.here);
+#pragma unroll
+    for (int c = 0; c < kMaxLower; c++) sum[c] = load1(img, (uint32_t)min(c, a.channels - 1) * plane + p.here);
+    // output by output, the next one's values requested before this one's products: few registers, so that the
+    // waves of a SIMD hide each other's scalar loads of the weights
+    float all[kMaxLower] = {}, A[2][3][3];
+    auto gather = [&](int o, float(&to)[3][3]) { finish_gather(a, p, img + (uint64_t)(a.channels + o) * plane, a.dil[o], to); };
+    auto add = [&](int o, float(&from)[3][3]) {
+        if (!p.away) finish_fold(a, p, a.dil[o], from);
+        const float *const k = a.k[o];
+#pragma unroll
+        for (int c = 0; c < kMaxLower; c++) {
+            float one = 0.f;
+            const int cc = min(c, a.channels - 1);                  // (what the rest sums is not used)
+#pragma unroll
+            for (int t = 0; t < kTaps; t++) one += k[cc * kTaps + t] * from[t / 3][t % 3];
+            all[c] += one;
+        }
+    };
+    gather(0, A[0]);
+#pragma unroll 1
+    for (int o = 0; o < a.n; o += 2) {
+        gather(min(o + 1, a.n - 1), A[1]);
+        add(o, A[0]);
+        if (o + 1 >= a.n) break;
+        gather(min(o + 2, a.n - 1), A[0]);
+        add(o + 1, A[1]);
+    }
+#pragma unroll
+    for (int c = 0; c < kMaxLower; c++) {
+        if (c >= a.channels) break;               // uniform
+        const float act_c = c == a.masked ? m[0] : m[1];
+        const float v[1] = {c < a.masked || 0.f < act_c ? sum[c] + all[c] : 0.f};
+        if (p.own) store_global_vec<1>(img, (uint32_t)c * plane + p.here, v);
+    }
+}
+
+template <int NQ, int NOUT>
+hipError_t finish_back_launch(const FinishArgs &a, const float *act, float *g, hipStream_t s)
+{
+    hipLaunchKernelGGL((finish_back<NQ, NOUT>), dim3(xcd_grid((a.items + 3) / 4)), dim3(256), 0, s, a, act, g);
+    return hipGetLastError();
+}
+
+FinishArgs finish_args(const Geom &g, const View<const float> &x, const group2d::Outputs &above)
+{
+    const int segs = (g.W + kWave - 1) / kWave;
+    FinishArgs a{g.H, g.W, segs, g.B * g.H * segs, 0, above.n, 0, 0, x.sb, x.sc, x.sy, {}, {}};
+    for (int o = 0; o < above.n; o++) {
+        a.dil[o] = above.dil[o];
+        a.k[o] = above.k[o];
+        a.dmax = std::max(a.dmax, above.dil[o]);
+    }
+    return a;
+}
+
+template <int G, int P>
+hipError_t pull_launch(const PullArgs &a, int wgs, const float *x, const float *gy, float *gx, float *part, float *bias_part,
+                       hipStream_t s)
+{
+    constexpr int kLds = kWaves * (kSlabBytes + PullShape<G, P>::kOwnBytes);
+    static LargeLds large;
+    const hipError_t e = large.allow(reinterpret_cast<const void *>(&pull_rows<G, P>), kLds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((pull_rows<G, P>), dim3(wgs), dim3(kWaves * kWave), kLds, s, a, x, gy, gx, part, bias_part);
+    return hipGetLastError();
+}
+
+// As many workgroups as are resident, shared out over the chunks by their size.
+struct PullPlan {
+    Chunks chunks;
+    int segs, wgs, image_tiles, tiles;
+};
+
+PullPlan pull_plan(int64_t batch, int64_t H, int64_t W, int64_t channels, int slabs)
+{
+    PullPlan p;
+    const int nb = (int)((channels + 15) / 16);
+    Chunks &c = p.chunks;
+    const int most = slabs == 1 ? 4 : kWaves;     // blocks of a chunk (one slab: 411 us over 100 channels, 463 with 8)
+    c.n = (nb + most - 1) / most;
+    c.blocks = (nb + c.n - 1) / c.n;
+    c.large = nb - c.n * (c.blocks - 1);
+    p.segs = (int)((W + kSegment - 1) / kSegment);
+    const int per_tile = kWaves / slabs;
+    p.image_tiles = (int)((H * p.segs + per_tile - 1) / per_tile);
+    p.tiles = (int)batch * p.image_tiles;
+    auto share = [&](int blocks) {
+        return (int)std::min<int64_t>(p.tiles, std::max(kXcds, 256 * blocks / nb / kXcds * kXcds));
+    };
+    c.wgs = share(c.blocks);
+    c.wgs_small = share(std::max(1, c.blocks - 1));
+    p.wgs = c.first_wg(c.n);
+    return p;
+}
+
+int64_t pull_floats(const PullPlan &p, int slabs)
+{
+    return (int64_t)p.wgs * slabs * (p.chunks.blocks * 1024 + kBiasColumns);
+}
+
+}  // namespace
+}  // namespace group2d
+
+int64_t group_pull_floats_2d(int64_t batch, int64_t H, int64_t W, int64_t channels)
+{
+    using namespace group2d;
+    return std::max(pull_floats(pull_plan(batch, H, W, channels, 1), 1), pull_floats(pull_plan(batch, H, W, channels, 2), 2));
+}
+
+bool group_pull_supported_2d(const Geom &g, const View<const float> &x, const View<float> &gx)
+{
+    return g.ndim == 2 && x.sx == 1 && gx.sx == 1 && x.sb == gx.sb && x.sc == gx.sc && x.sy == gx.sy && g.W >= group2d::kSegment &&
+           x.sc < ((int64_t)1 << 26) && (int64_t)(g.H - 1) * x.sy + g.W < ((int64_t)1 << 26) &&
+           (int64_t)g.B * g.H * ((g.W + group2d::kSegment - 1) / group2d::kSegment) < ((int64_t)1 << 30);
+}
+
+hipError_t group_pull_2d(const Geom &g, const View<const float> &x, const group2d::Outputs &out, int update, int mask_from,
+                         const View<float> &grads, int first, const int *channels, float *const *gk, float *gb,
+                         float *ws, bool reverse, hipStream_t s)
+{
+    using namespace group2d;
+    if (out.n < 1 || out.n > kMaxOut || !group_pull_supported_2d(g, x, grads)) return hipErrorInvalidValue;
+    const int slabs = out.n > kSlabOut ? 2 : 1;
+    const PullPlan p = pull_plan(g.B, g.H, g.W, g.C, slabs);
+    PullArgs a{g.C, update, mask_from, g.H, g.W, p.segs, g.H * p.segs, p.tiles, p.image_tiles, Divisor((uint32_t)p.segs),
+               Divisor((uint32_t)p.image_tiles), reverse, 0, p.chunks, x.sb, x.sc, x.sy, out};
+    SumArgs sum;
+    for (int o = 0; o < kMaxOut; o++) {
+        if (o < out.n) a.dmax = std::max(a.dmax, out.dil[o]);
+        sum.channels[o] = o < out.n ? channels[o] : 0;
+        sum.gk[o] = o < out.n ? gk[o] : nullptr;
+    }
+    float *const bias_part = ws + (int64_t)p.wgs * slabs * p.chunks.blocks * 1024;
+    const float *const gy = grads.p + (int64_t)first * grads.sc;
+    hipError_t e = hipErrorInvalidConfiguration;
+    // waves to a block: 4, 2 or 1
+    const int share = p.chunks.blocks <= 2 ? 4 : p.chunks.blocks <= 4 ? 2 : 1;
+    switch (slabs * 10 + share) {
+    case 14: e = pull_launch<1, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 12: e = pull_launch<1, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 24: e = pull_launch<2, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 22: e = pull_launch<2, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 21: e = pull_launch<2, 1>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    }
+    if (e != hipSuccess) return e;
+    sum.chunks = p.chunks;
+    sum.slabs = slabs;
+    sum.columns = p.chunks.first_block(p.chunks.n) * 1024 * slabs;
+    sum.stride = p.chunks.blocks * 1024 * slabs;
+    sum.n = out.n;
+    sum.gb = gb;
+    hipLaunchKernelGGL(sum_group, dim3(sum.columns / kWave + 1), dim3(1024), 0, s, sum, ws, bias_part);
+    return hipGetLastError();
+}
+
+hipError_t group_finish_back_2d(const Geom &g, const View<const float> &x, const View<float> &grads, int channel, int width,
+                                const group2d::Outputs &above, hipStream_t s)
+{
+    using namespace group2d;
+    const FinishArgs a = finish_args(g, x, above);
+    const float *const act = x.p + (int64_t)channel * x.sc;
+    float *const gp = grads.p + (int64_t)channel * grads.sc;
+    if (width == 1) {
+        switch (above.n) {
+        case 1: return finish_back_launch<1, 1>(a, act, gp, s);
+        case 2: return finish_back_launch<2, 1>(a, act, gp, s);
+        case 3: return finish_back_launch<3, 1>(a, act, gp, s);
+        case 4: return finish_back_launch<4, 1>(a, act, gp, s);
+        case 5: return finish_back_launch<5, 1>(a, act, gp, s);
+        case 6: return finish_back_launch<6, 1>(a, act, gp, s);
+        case 7: return finish_back_launch<7, 1>(a, act, gp, s);
+        }
+    } else if (width == 2) {
+        switch (above.n) {
+        case 1: return finish_back_launch<1, 2>(a, act, gp, s);
+        case 2: return finish_back_launch<2, 2>(a, act, gp, s);
+        case 3: return finish_back_launch<3, 2>(a, act, gp, s);
+        case 4: return finish_back_launch<4, 2>(a, act, gp, s);
+        case 5: return finish_back_launch<5, 2>(a, act, gp, s);
+        case 6: return finish_back_launch<6, 2>(a, act, gp, s);
+        }
+    }
+    return hipErrorInvalidConfiguration;
+}
+
+hipError_t group_spread_back_2d(const Geom &g, const View<const float> &x, const View<float> &grads, int channel, int channels,
+                                int width, const group2d::Outputs &above, hipStream_t s)
+{
+    using namespace group2d;
+    if (above.n < 1 || above.n > kSlabOut || channels > kMaxLower || width < 1 || width > 2 || channels < width) return hipErrorInvalidValue;
+    FinishArgs a = finish_args(g, x, above);
+    a.channels = channels;
+    a.masked = channels - width;
+    hipLaunchKernelGGL(spread_back, dim3(xcd_grid((a.items + 3) / 4)), dim3(256), 0, s, a, x.p + (int64_t)channel * x.sc,
+                       grads.p + (int64_t)channel * grads.sc);
+    return hipGetLastError();
+}
+
+}  // namespace msd

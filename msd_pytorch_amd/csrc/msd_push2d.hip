@@ -117,7 +117,7 @@ __global__ __launch_bounds__(kMaxWaves *kWave) void push_rows(PushArgs a, const 
                 __syncthreads();
                 // a thread's entries are one column of the product, every blockDim / 64 channels;
                 // eight loads at a time
-                const int t = tid % kTiles, i = tid / kTiles % 16, tri = triple_of(t, i), o = min(tri / 3, kMaxOut - 1);
+                const int t = tid % kTiles, i = tid / kTiles % 16, tri = triple_of(t, i), o = min(tri / 3, kSlabOut - 1);
                 const bool column = o < a.out.n && !(i == 15 && t == 3);
                 const float *const k = a.out.k[column ? o : 0] + (int64_t)c0 * kTaps + (tri % 3) * 3 + kx_of(t, i);
                 const int stride = blockDim.x / kWave, end = 4 * steps;
@@ -357,7 +357,7 @@ hipError_t group_push_2d(const Geom &g, const View<const float> &x, const group2
     using namespace group2d;
     int dmax = 0;
     for (int o = 0; o < out.n; o++) dmax = std::max(dmax, out.dil[o]);
-    if (out.n < 1 || out.n > kMaxOut || !group_push_supported_2d(g, x, dmax)) return hipErrorInvalidValue;
+    if (out.n < 1 || out.n > kSlabOut || !group_push_supported_2d(g, x, dmax)) return hipErrorInvalidValue;
     const int halo = (dmax + 3) & ~3;
     const Teams t = make_teams(g.W, halo);
     PushArgs a{g.C, g.H, g.W, g.B * g.H * t.segs, t.segs, x.sb, x.sc, x.sy, t.waves, t.rpw, t.inner, halo, out};
@@ -376,7 +376,7 @@ hipError_t group_push_2d(const Geom &g, const View<const float> &x, const group2
 bool group_finish_supported_2d(const Geom &g, const View<const float> &x, const View<float> &out)
 {
     return g.ndim == 2 && x.sx == 1 && out.sx == 1 && group2d::finish_vec(g, x, out) != 0 &&
-           ((g.Wd == 1 && g.C < group2d::kMaxOut) || (g.Wd == 2 && g.C < 6 && g.C % 2 == 0));
+           ((g.Wd == 1 && g.C < group2d::kSlabOut) || (g.Wd == 2 && g.C < 6 && g.C % 2 == 0));
 }
 
 hipError_t group_finish_2d(const Geom &g, const View<const float> &x, const float *k, const float *bias,

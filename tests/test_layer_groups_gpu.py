@@ -65,6 +65,66 @@ def test_block_backward_in_layer_groups(case, input_grad):
         check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=43, input_grad=input_grad)
 
 
+# Groups of eight to fourteen outputs: two slabs of 64 matrix rows, the upper outputs' share of the lower
+# channels in one launch.  Blocks of 16 channels shared by four, two or one waves (1, 2 | 3, 4 | 5 to 8 blocks),
+# two chunks; tiles of four segments that end inside an image, also between two images; halves of 7 + 7, 7 + 1,
+# 6 + 8 and 6 + 2 outputs.
+FOURTEEN = [
+    ((5, 33), 1, 1, 8, 2, [1, 5, 3]),
+    ((7, 95), 3, 1, 14, 2, [7, 2]),
+    ((9, 66), 4, 1, 13, 1, None),
+    ((6, 130), 19, 1, 14, 1, [6, 1, 4]),
+    ((11, 64), 20, 1, 14, 3, [3, 11]),
+    ((5, 127), 52, 1, 14, 1, [5, 1]),
+    ((4, 97), 115, 1, 14, 1, [1, 4]),
+    ((4, 40), 116, 1, 14, 2, [2, 3]),
+    ((6, 70), 5, 2, 7, 1, [1, 6, 2]),
+    ((13, 35), 3, 2, 4, 2, [13, 1]),
+    ((40, 160), 2, 1, 28, 1, None),
+]
+
+
+@pytest.mark.parametrize("case", FOURTEEN, ids=lambda c: "x".join(map(str, c[0])) + "-c%d-w%d-d%d-B%d" % c[1:5])
+def test_block_backward_in_groups_of_up_to_fourteen(case):
+    size, c_in, width, depth, batch, dilations = case
+    dilations = [min(size[0], (dilations or range(1, 11))[i % len(dilations or range(1, 11))]) for i in range(depth)]
+    with tuning({"bwd.group": 1}):
+        check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=59)
+
+
+# What is no sum of three bf16 values takes the fp32 instruction: the same infinities and NaNs as from the
+# layers' own kernels, and the largest finite values (which round to an infinity in bf16) stay finite.
+@pytest.mark.parametrize("where", ["stack", "gradient", "weight"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38, -3.4028234e38])
+@pytest.mark.parametrize("depth", [6, 14])
+def test_values_without_bf16_parts(where, value, depth):
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator().manual_seed(29)
+    c_in, size = 4, (9, 71)
+    stack = torch.rand(1, c_in + depth, *size, generator=gen).cuda() + 0.1     # every ReLU open
+    gradient = torch.rand(1, c_in + depth, *size, generator=gen).cuda() * 1e-3
+    weights = [(torch.rand(1, c_in + i, 3, 3, generator=gen) * 1e-3 + 1e-4).cuda() for i in range(depth)]
+    if where == "stack":
+        stack[0, 2, 4, 65] = value
+    elif where == "gradient":
+        gradient[0, c_in + 1, 4, 66] = value
+    else:
+        weights[depth - 2][0, 1, 1, 2] = value
+    found = []
+    for setting in (0, 1):
+        gk, gb, grads = [torch.zeros_like(w) for w in weights], torch.zeros(depth).cuda(), gradient.clone()
+        with tuning({"bwd.group": setting}):
+            cc.block_backward(stack, grads, c_in, [1 + i % 4 for i in range(depth)], weights, gk, gb, True)
+        found.append(torch.cat([grads[:, :c_in].flatten(), gb, *(k.flatten() for k in gk)]))
+    assert torch.equal(torch.isnan(found[0]), torch.isnan(found[1]))
+    assert torch.equal(torch.isinf(found[0]), torch.isinf(found[1]))
+    finite = torch.isfinite(found[0])
+    assert bool(finite.any())
+    # (sums of up to 639 terms of one sign in another order, relative to the largest)
+    a, b = found[0][finite].double(), found[1][finite].double()
+    assert float(((a - b).abs() / a.abs().clamp_min(1e-30)).max()) <= 1e-4
+
+
 def test_an_infinity_meets_its_own_voxels_only():
     """The last tile of a row repeats voxels of the one before (here 8 to 31): what they hold counts once."""
     from msd_pytorch_amd import msd_custom_convolutions as cc
