@@ -77,16 +77,27 @@ __global__ __launch_bounds__(kThreads) void scale_fold_kernel(int c_out, int c_i
         ob[o] = shift ? acc + shift[o] : acc;
 }
 
-__global__ __launch_bounds__(kThreads) void label_check_kernel(int64_t n, long long num_labels,
-                                                               const int64_t *__restrict__ labels,
-                                                               int64_t *__restrict__ clamped, long long *range)
+// Bound by the two atomics of each workgroup, which all go to one line (7 ns each): one workgroup of 16
+// waves per compute unit and four labels per lane in flight.  Back to back, launch included: 1024 x 1024 labels 180 us
+// with the atomics of 4096 waves, 11 us so; 476 523 labels 144 and 11, 65 536 labels 40 and 6.
+constexpr int kLabelThreads = 1024, kLabelGroups = 256, kLabelUnroll = 4;
+__global__ __launch_bounds__(kLabelThreads) void label_check_kernel(int64_t n, long long num_labels,
+                                                                    const int64_t *__restrict__ labels,
+                                                                    int64_t *__restrict__ clamped, long long *range)
 {
+    __shared__ long long ends[2][kLabelThreads / kWave];
     long long lo = INT64_MAX, hi = INT64_MIN;
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
-        const long long v = labels[i];
-        lo = v < lo ? v : lo;
-        hi = v > hi ? v : hi;
-        clamped[i] = v < 0 ? 0 : (v >= num_labels ? num_labels - 1 : v);
+    const int64_t stride = (int64_t)gridDim.x * kLabelThreads;
+    for (int64_t i = (int64_t)blockIdx.x * kLabelThreads + threadIdx.x; i < n; i += kLabelUnroll * stride) {
+        long long v[kLabelUnroll];
+#pragma unroll
+        for (int u = 0; u < kLabelUnroll; u++) v[u] = labels[i + u * stride < n ? i + u * stride : i];
+#pragma unroll
+        for (int u = 0; u < kLabelUnroll; u++) {
+            lo = v[u] < lo ? v[u] : lo;
+            hi = v[u] > hi ? v[u] : hi;
+            if (i + u * stride < n) clamped[i + u * stride] = v[u] < 0 ? 0 : (v[u] >= num_labels ? num_labels - 1 : v[u]);
+        }
     }
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) {
@@ -95,10 +106,18 @@ __global__ __launch_bounds__(kThreads) void label_check_kernel(int64_t n, long l
         hi = h2 > hi ? h2 : hi;
     }
     if (threadIdx.x % kWave == 0) {
-        // (read first: after the first few waves hardly any has something to add)
-        if (lo < range[0]) atomicMin(&range[0], lo);
-        if (hi > range[1]) atomicMax(&range[1], hi);
+        ends[0][threadIdx.x / kWave] = lo;
+        ends[1][threadIdx.x / kWave] = hi;
     }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int w = 1; w < kLabelThreads / kWave; w++) {
+        lo = ends[0][w] < lo ? ends[0][w] : lo;
+        hi = ends[1][w] > hi ? ends[1][w] : hi;
+    }
+    // (read first: after the first few workgroups hardly any has something to add)
+    if (lo < range[0]) atomicMin(&range[0], lo);
+    if (hi > range[1]) atomicMax(&range[1], hi);
 }
 
 }  // namespace
@@ -150,8 +169,8 @@ hipError_t scale_fold(bool f64, int c_out, int c_in, const void *scale, const vo
 hipError_t label_check(int64_t count, int64_t num_labels, const int64_t *labels, int64_t *clamped, int64_t *range,
                        hipStream_t s)
 {
-    const unsigned blocks = (unsigned)std::min<int64_t>((count + kThreads - 1) / kThreads, 1024);
-    hipLaunchKernelGGL(label_check_kernel, dim3(blocks), dim3(kThreads), 0, s, count, (long long)num_labels, labels,
+    const unsigned blocks = (unsigned)std::min<int64_t>((count + kLabelThreads - 1) / kLabelThreads, kLabelGroups);
+    hipLaunchKernelGGL(label_check_kernel, dim3(blocks), dim3(kLabelThreads), 0, s, count, (long long)num_labels, labels,
                        clamped, (long long *)range);
     return hipGetLastError();
 }

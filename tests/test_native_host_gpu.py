@@ -140,6 +140,17 @@ def test_label_check(count):
     assert seen.tolist() == [min(2, int(labels.min())), max(4, int(labels.max()))]
 
 
+@pytest.mark.parametrize("count", [(1 << 18) - 1, (1 << 18) + 1, (1 << 20) + 1])
+def test_label_check_of_whole_images(count):
+    """A grid of labels less and more one, and one more than the grid takes in one round."""
+    from msd_pytorch_amd import _native
+    labels = torch.randint(0, 5, (count,), generator=torch.Generator().manual_seed(count))
+    labels[count - 1], labels[count // 2] = -7, 12
+    seen = torch.tensor([2, 4]).cuda()
+    out = _native.host().label_check(labels.cuda(), 5, seen)
+    assert torch.equal(out.cpu(), labels.clamp(0, 4)) and seen.tolist() == [-7, 12]
+
+
 @pytest.mark.parametrize("ndim,size", [(2, (30, 70)), (3, (5, 8, 40))])
 def test_prediction_without_gradients_equals_the_differentiable_pass(ndim, size):
     (model,) = _models("L2", ndim, 5, 1, 3, 1)
