@@ -1259,12 +1259,12 @@ int block_backward_split3d(const char *fn, const BlockArgs &a, int64_t c_in, con
 // Groups of layers of the 2D backward pass on the matrix cores (msd_pull.hip).
 // ---------------------------------------------------------------------------
 
-// Channels below the lowest layer of a group from which on it is taken.  The pass works in blocks of
-// 16 channels, but already over the four below the layers of a depth of ten (256 x 256, recorded step)
-// it is faster than pairs of layers: 157 -> 150 us; 3 x 333 x 477, depth 30: 1.84 -> 0.97 ms per step.  A group takes
-// up to 14 outputs wherever there are that many: at 1024 x 1024 a pass and the upper half's share of the lower (49 us)
-// are as fast as two groups of seven over 20 channels (266 us both), 332 against 371 us over 48, 552 against 860 over 95.
-constexpr int64_t kGroupBackChannels = 4;
+// Channels below the lowest layer of a group from which on it is taken: always.  256 x 256, depth 10, recorded step:
+// all ten layers in one group 132 us, seven over four channels and the rest in pairs 140, pairs alone 157; neutral
+// at depth 30 and 100 (3 x 333 x 477, 1024 x 1024).  A group takes up to 14 outputs wherever there are that many: at
+// 1024 x 1024 a pass and the upper half's share of the lower (49 us) are as fast as two groups of seven over
+// 20 channels (266 us both), 332 against 371 us over 48, 552 against 860 over 95.
+constexpr int64_t kGroupBackChannels = 1;
 
 // Number of layers from layer i down that form a group of the backward pass (0: none); `first` is
 // the output channel of layer i.
