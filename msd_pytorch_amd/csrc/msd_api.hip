@@ -1405,39 +1405,60 @@ namespace {
 // are slower (64 registers of sums) and the pass pays at once.  Small images gain as well (100 layers at
 // 64 x 64: 854 -> 535 us): the last launch of a group reads 10 planes, not 100.
 constexpr int64_t kGroupChannels = 12, kGroupChannelsWide = 6;
+// Up to fourteen outputs instead of seven where the channels in front are at least this many voxels in all.  The pass
+// then moves them once and not twice (two channels per layer: 2.3 times, since sevens take six outputs), but the
+// upper layers of the group find up to 13 channels to add, and passes of seven have twice the waves.  Push and finish of
+// 14 outputs, us, sevens and fourteens: two channels per layer 1024 x 1024 over 60: 323, 339; over 180: 707, 613;
+// 2048 x 2048 over 24: 967, 959; over 60: 1426, 1185; over 120: 2180, 1663; one channel 1536 x 1536 over 80: 928, 913;
+// 2048 x 2048 over 45: 1127, 1253; over 90: 1657, 1507.
+constexpr int64_t kFourteenVoxels = (int64_t)1 << 28, kFourteenVoxelsWide = (int64_t)1 << 27;
 
-// Number of layers from layer i on that form a group of the forward pass (0: none).
-int forward_group(const BlockArgs &a, int i, int64_t first)
+// Number of layers from layer i on that form a group of the forward pass (0: none), of at most `most` outputs.
+// Knob: n > 0 from n channels on, in sevens; n < -1 from -n channels on, in fourteens.
+int forward_group(const BlockArgs &a, int i, int64_t first, int most)
 {
     const int from = msd::knob(msd::kKnobFwdGroup, -1);
     if (a.dtype != MSD_F32 || a.ndim != 2 || g_kernel_path != 0 || from == 0) return 0;
-    if (first < (from > 0 ? from : a.widths[i] > 1 ? kGroupChannelsWide : kGroupChannels)) return 0;
+    const bool wide = a.widths[i] > 1;
+    if (first < (from > 0 ? from : from < -1 ? -from : wide ? kGroupChannelsWide : kGroupChannels)) return 0;
     int n = 0;
-    int64_t outputs = 0;
-    while (i + n < a.depth && a.widths[i + n] <= 2 && outputs + a.widths[i + n] <= msd::group2d::kSlabOut)
+    int64_t outputs = 0, dmax = 0;
+    while (i + n < a.depth && a.widths[i + n] <= 2 && outputs + a.widths[i + n] <= most) {
+        // (a query of the workspace does not know the dilations)
+        if (a.dilations) dmax = a.dilations[i + n] > dmax ? a.dilations[i + n] : dmax;
         outputs += a.widths[i + n++];
+    }
+    if (outputs > msd::group2d::kSlabOut) {
+        const bool large = a.batch * a.spatial[0] * a.spatial[1] >= ((wide ? kFourteenVoxelsWide : kFourteenVoxels) + first - 1) / first;
+        if (from > 0 || (from == -1 && !large) || !msd::group_split_supported_2d(a.spatial[1], (int)dmax)) return 0;
+    }
     return n >= 2 ? n : 0;
 }
 
-// Bytes of the three planes per output that the n layers from layer i on leave to their finishing launches.
-int64_t group_planes_bytes(const BlockArgs &a, int i, int n)
+// Bytes of the three planes per output that the n layers from layer i on leave to their finishing launches, and of
+// the table of weights of a pass of more than seven outputs.
+int64_t group_planes_bytes(const BlockArgs &a, int i, int n, int64_t first)
 {
     int64_t outputs = 0;
     for (int j = 0; j < n; j++) outputs += a.widths[i + j];
-    return 3 * outputs * a.batch * a.spatial[0] * a.spatial[1] * (int64_t)sizeof(float);
+    const int64_t planes = 3 * outputs * a.batch * a.spatial[0] * a.spatial[1];
+    if (outputs <= msd::group2d::kSlabOut) return planes * (int64_t)sizeof(float);
+    return ((planes + 3) / 4 * 4 + msd::group_table_floats_2d(first)) * (int64_t)sizeof(float);
 }
 
 // Of the largest group that a block can form, whichever layer its groups start at.
 int64_t forward_group_bytes(const BlockArgs &a)
 {
     if (a.ndim != 2 || !msd::group_rows_supported_2d(a.spatial[1])) return 0;
-    int64_t first = a.c_in, most = 0;
+    int64_t first = a.c_in, bytes = 0;
     for (int i = 0; i < a.depth; i++) {
-        const int64_t n = group_planes_bytes(a, i, forward_group(a, i, first));
-        most = n > most ? n : most;
+        for (const int most : {msd::group2d::kSlabOut, msd::group2d::kMaxOut}) {
+            const int64_t n = group_planes_bytes(a, i, forward_group(a, i, first, most), first);
+            bytes = n > bytes ? n : bytes;
+        }
         first += a.widths[i];
     }
-    return most;
+    return bytes;
 }
 
 // Layers i .. i + n - 1: one pass over the channels [0, first) for all of them, then each layer
@@ -1479,9 +1500,11 @@ int block_group_forward(const char *fn, const BlockArgs &a, int i, int n, int64_
     MSD_TRY(make_geom(fn, a.dtype, a.ndim, a.batch, first, out.n, a.spatial, dmax, true, &shared));
     if (!msd::group_push_supported_2d(shared, x, dmax)) return MSD_OK;
     ProfileScope scope(0, s);
-    hipError_t e = msd::group_push_2d(shared, x, out, z, s);
-    if (e != hipSuccess) return hip_fail(fn, e);
     const int64_t plane = a.spatial[0] * a.spatial[1];
+    hipError_t e = out.n > msd::group2d::kSlabOut
+                       ? msd::group_push_split_2d(shared, x, out, z, z + (3 * out.n * a.batch * plane + 3) / 4 * 4, s)
+                       : msd::group_push_2d(shared, x, out, z, s);
+    if (e != hipSuccess) return hip_fail(fn, e);
     added = 0;
     for (int j = 0; j < n; j++) {
         const msd::View<float> y{st.p + (first + added) * st.sc, st.sb, st.sc, st.sz, st.sy, st.sx};
@@ -1532,8 +1555,16 @@ int msd_block_forward_ws(int dtype, int ndim, int64_t batch, int64_t c_in, int d
     ProfileBatch profile_runs((hipStream_t)stream);
     int64_t first = c_in, b0 = 0;
     for (int i = 0; i < depth; i++) {
-        const int n = workspace ? forward_group(a, i, first) : 0;
-        if (n && workspace_bytes >= group_planes_bytes(a, i, n)) {
+        // the largest group that there is room for
+        int n = 0;
+        if (workspace) {
+            for (const int most : {msd::group2d::kSlabOut, msd::group2d::kMaxOut}) {
+                const int m = forward_group(a, i, first, most);
+                if (m && workspace_bytes >= group_planes_bytes(a, i, m, first)) n = m;
+            }
+            if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0 && n) n = forward_group(a, i, first, msd::group2d::kSlabOut);
+        }
+        if (n) {
             bool done = false;
             MSD_TRY(block_group_forward(fn, a, i, n, first, stack, stack_strides, weights, (const float *)bias + b0,
                                         (float *)workspace, (hipStream_t)stream, &done));

@@ -69,6 +69,11 @@ bool group_rows_supported_2d(int64_t W);
 bool group_push_supported_2d(const Geom &g, const View<const float> &x, int dmax);
 hipError_t group_push_2d(const Geom &g, const View<const float> &x, const group2d::Outputs &out, float *z, hipStream_t s);
 
+// The same for up to kMaxOut outputs, more than kSlabOut.  table: group_table_floats_2d floats (their address a multiple of 16 bytes).
+bool group_split_supported_2d(int64_t W, int dmax);
+int64_t group_table_floats_2d(int64_t channels);
+hipError_t group_push_split_2d(const Geom &g, const View<const float> &x, const group2d::Outputs &out, float *z, float *table,
+                               hipStream_t s);
 
 // One layer of the group from its planes and the g.C channels that the group has added (with ReLU).
 bool group_finish_supported_2d(const Geom &g, const View<const float> &x, const View<float> &out);

@@ -20,6 +20,7 @@
 // output by output, with the voxels as columns, it was 45 us + 1.1 us.
 // Counters over the 13 launches of a forward pass of depth 100 there: 4.1 GB in 1.14 ms, matrix cores busy 52 %.
 #include "msd_group.h"
+#include "msd_split.h"
 
 #include <algorithm>
 
@@ -207,6 +208,350 @@ __global__ __launch_bounds__(kMaxWaves *kWave) void push_rows(PushArgs a, const 
     }
 }
 
+// ---- More than seven outputs: two slabs of columns, fp32 values in bf16 parts (msd_split.h).
+//
+// A wave walks a row, or a part of one, in segments of 64 voxels and forms the columns of one slab; no
+// wave waits for another.  x arrives by channel in 256-byte pieces, is split and goes through the wave's
+// own part of LDS: the matrix cores take 16 voxels x 32 channels at once, read transposed
+// (ds_read_b64_tr_b16).  The shifts along x are taken as in push_rows, tile by tile of the columns, through the same
+// space; what a segment's outputs need of the segment before stays in registers, so that nothing is formed
+// twice.  Every channel is read once for up to fourteen outputs.
+//
+// Bound by latencies: eight waves per compute unit (their registers), each a chain of loads, split, LDS and matrix
+// instructions; the matrix part is a quarter of the time.  14 outputs at 2048 x 2048 over 20 / 45 / 90 / 120 channels: 512, 696,
+// 958, 1223 us, where two passes of push_rows take 485, 803, 1335 and 1526.  At 1024 x 1024 over 50: 206 (matrix
+// instructions cut to a sixth 200, x from the caches 163, without the shifts 112).  With a workgroup per row, its waves
+// side by side and barriers around each tile of the shifts: 194 there, but 2.3 ms at 2048 x 2048 over 120.
+constexpr int kSlabs = 2;
+constexpr int kPushWaves = 8;                     // of a workgroup; one workgroup per compute unit
+constexpr int kPushTeams = kPushWaves / kSlabs;   // rows that a workgroup works on
+constexpr int kHalo = 16;                         // dilations up to here
+constexpr int kStepChannels = 32;
+constexpr int kTileBytes = 3 * kWave * 16;        // weights of 16 columns, a step
+constexpr int kTableSteps = 4;                    // steps whose weights are in LDS at a time
+constexpr int kTableBytes = kTableSteps * kSlabs * kTiles * kTileBytes;
+constexpr int kLine = 2 * kHalo + kWave + 4;      // floats of a staged row (16 bytes apart in the banks)
+constexpr int kOwnBytes = kStaged * kLine * 4 + 16;                 // of a wave: staged rows, or 16 channels of x in parts
+static_assert(kOwnBytes >= 3 * 16 * 2 * kWave && kOwnBytes % 16 == 0, "x lies over the staged rows");
+constexpr int kSplitLds = kTableBytes + kPushWaves * kOwnBytes;
+
+struct SplitArgs {
+    int C, H, W, items, parts, length;            // items: parts of all rows; outputs of a part
+    int64_t xsb, xsc, xsy;                        // strides of x
+    Outputs out;
+};
+
+// Channel (of the step's 32) that value e of the lanes q stands for: the first half of a step's channels
+// is split, put and read before the second.
+__host__ __device__ __forceinline__ int channel_of(int q, int e) { return e < 4 ? 4 * q + e : 16 + 4 * q + e - 4; }
+
+// [step][tile of columns][part][lane (column n, q)]: eight channels each; bad[step]: weights without parts
+// among them.
+__global__ __launch_bounds__(kSlabs *kTiles *kWave) void push_table(const SplitArgs a, bf16x8_t *__restrict__ table, int *__restrict__ bad)
+{
+    const int step = blockIdx.x, t = threadIdx.x / kWave, lane = threadIdx.x % kWave, i = lane % 16, q = lane / 16;
+    const int tri = triple_of(t % kTiles, i), o = t / kTiles * kSlabOut + tri / 3;
+    const bool column = o < a.out.n && !(i == 15 && t % kTiles == 3);
+    const float *const k = a.out.k[column ? o : 0] + (tri % 3) * 3 + kx_of(t % kTiles, i);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const int c = step * kStepChannels + channel_of(q, e);
+        const float w = k[min(c, a.C - 1) * kTaps];
+        v[e] = column && c < a.C ? w : 0.f;
+    }
+    Split8 s;
+    const float rest = split8(v, s);
+    const int any = __syncthreads_or(rest != rest);
+    if (any) split_any(v, s);
+    if (threadIdx.x == 0) bad[step] = any;
+#pragma unroll
+    for (int p = 0; p < 3; p++) table[((step * kSlabs * kTiles + t) * 3 + p) * kWave + lane] = s.p[p];
+}
+
+// LDS accesses of one wave: executed in order, only the compiler has to be kept from reordering them.
+__device__ __forceinline__ void own_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// Of a workgroup (of LDS only: the loads of x and the stores of z stay in flight).
+__device__ __forceinline__ void all_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+// A row of 16 bytes pieces lies at piece ^ turn(row): what is read transposed meets all banks once.
+__device__ __forceinline__ uint32_t turn(uint32_t row) { return row / 2 % 4 * 2 + row / 8 % 2; }
+
+__global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitArgs a, const float *__restrict__ x,
+                                                                  const bf16x8_t *__restrict__ table, const int *__restrict__ bad,
+                                                                  float *__restrict__ z)
+{
+    constexpr int kStepEntries = kSlabs * kTiles * 3 * kWave;
+    extern __shared__ __attribute__((aligned(16))) char split_lds[];
+    const int tid = threadIdx.x, lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), slab = wave % kSlabs, team = wave / kSlabs;
+    bf16x8_t *const weights = reinterpret_cast<bf16x8_t *>(split_lds);
+    char *const own = split_lds + kTableBytes + wave * kOwnBytes;
+    const int steps = (a.C + kStepChannels - 1) / kStepChannels;
+    bool weights_split = true;
+    for (int s = 0; s < steps; s++) weights_split = weights_split && bad[s] == 0;
+    const uint32_t plane = (uint32_t)(a.xsc * 4);
+    // (a lane's place, formed anew where it is used: nothing of the addresses is kept over a row)
+    struct Lane {
+        uint32_t id, n, q;
+    };
+    auto fresh = [&]() {
+        uint32_t id = (uint32_t)lane;
+        asm volatile("" : "+v"(id));
+        return Lane{id, id % 16, id / 16 % 4};
+    };
+
+    // an item: outputs [from, to) of a row, formed from the voxels [start, end)
+    struct Item {
+        int b, y, from, to, start, end;
+        bool valid;
+    };
+    auto locate = [&](int it0) {
+        Item p;
+        p.valid = it0 < a.items;
+        const int it = min(it0, a.items - 1), row = it / a.parts, part = it - row * a.parts;
+        p.b = row / a.H;
+        p.y = row - p.b * a.H;
+        p.from = min(part * a.length, a.W);
+        p.to = min(p.from + a.length, a.W);
+        p.start = max(p.from - kHalo, 0);
+        p.end = min(p.to + kHalo, a.W);
+        return p;
+    };
+    // Loads: lane (channel q of four, voxels 4 n ..) of 64 voxels; past the row end its last four voxels, past
+    // the last channel that one again (its weights are zero).
+    f32x4_t xv[8];
+    auto request = [&](const Item &p, int first, int step) {
+        const Lane l = fresh();
+        const uint32_t at = 4u * (uint32_t)min(first + 4 * (int)l.n, a.W - 4), lane_plane = l.q * plane;
+        const uint64_t image = reinterpret_cast<uint64_t>(x) + (uint64_t)(((int64_t)p.b * a.xsb + (int64_t)p.y * a.xsy) * 4);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int c = min(step * kStepChannels + 4 * i, a.C - 1);              // uniform
+            uint64_t base = image + (uint64_t)c * (uint64_t)(a.xsc * 4);
+            asm volatile("" : "+s"(base));
+            float v[4];
+            load_global_vec4_unaligned(base, min(lane_plane, (uint32_t)min(a.C - 1 - c, 3) * plane) + at, v);
+            xv[i] = f32x4_t{v[0], v[1], v[2], v[3]};
+        }
+    };
+    const bool resident = steps <= kTableSteps;   // the weights are in LDS once and for all
+    if (resident) {
+        for (int i = tid; i < steps * kStepEntries; i += kPushWaves * kWave) weights[i] = table[i];
+        __syncthreads();
+    }
+    // (workgroups whose table does not hold all weights meet at each part of it: all their waves take as many segments)
+    const int most = (a.length + 2 * kHalo + kWave - 1) / kWave;
+    const int stride = gridDim.x * kPushTeams;
+    int it = blockIdx.x * kPushTeams + team;
+    Item here = locate(it);
+    request(here, here.start, 0);
+    for (int it0 = blockIdx.x * kPushTeams; it0 < a.items; it0 += stride, it += stride) {
+        const Item next = locate(it + stride);
+        f32x4_t before[2][kTiles];                // the last 32 voxels of the segment before
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int t = 0; t < kTiles; t++) before[j][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        const int segs = resident ? (here.end - here.start + kWave - 1) / kWave : most;
+        for (int seg = 0; seg < segs; seg++) {
+            const int first = here.start + seg * kWave;
+            const bool real = here.valid && first < here.end;                      // uniform
+            f32x4_t acc[4][kTiles];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int t = 0; t < kTiles; t++) acc[j][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            float rest = 0.f;
+            for (int step = 0; step < steps; step++) {
+                if (!resident && step % kTableSteps == 0) {                        // uniform over the workgroup
+                    all_sync();
+                    const int count = min(kTableSteps, steps - step) * kStepEntries;
+                    for (int i = tid; i < count; i += kPushWaves * kWave) weights[i] = table[step * kStepEntries + i];
+                    all_sync();
+                }
+                const auto [id, n, q] = fresh();
+                // the lane at the row end has loaded voxels further left
+                const int over = first + 4 * (int)n - (a.W - 4);
+                if (first + kWave > a.W && (a.W - first) % 4 != 0) {               // uniform
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const f32x4_t v = xv[i];
+                        xv[i][0] = over == 1 ? v[1] : over == 2 ? v[2] : over == 3 ? v[3] : v[0];
+                        xv[i][1] = over == 1 ? v[2] : over == 2 ? v[3] : v[1];
+                        xv[i][2] = over == 1 ? v[3] : v[2];
+                    }
+                }
+                bf16x8_t xa[4][3];                // [16 voxels][part]: voxel n, channels channel_of(q, ..)
+                const uint32_t tr_row = 4 * q + n / 4;
+                const char *const tr = own + tr_row * (2 * kWave) + n % 2 * 8;
+                const uint32_t tr_piece = 16 * (n % 4 / 2 ^ turn(tr_row));
+                typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+                bf16x4_t low[4][3];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    own_sync();                   // (what was there has been read)
+#pragma unroll
+                    for (int i = 4 * h; i < 4 * h + 4; i += 2) {
+                        // -x at every second voxel: the sums of the bf16 instruction are cut off towards minus infinity
+                        const float v[8] = {xv[i][0], -xv[i][1], xv[i][2], -xv[i][3], xv[i + 1][0], -xv[i + 1][1], xv[i + 1][2], -xv[i + 1][3]};
+                        Split8 s;
+                        rest += split8(v, s);
+#pragma unroll
+                        for (int k = 0; k < 2; k++) {
+                            const uint32_t channel = q + 4 * (uint32_t)(i % 4 + k);
+                            char *const at = own + channel * (2 * kWave) + 16 * (n / 2 ^ turn(channel)) + n % 2 * 8;
+#pragma unroll
+                            for (int p = 0; p < 3; p++)
+                                *reinterpret_cast<bf16x4_t *>(at + p * (16 * 2 * kWave)) =
+                                    k ? __builtin_shufflevector(s.p[p], s.p[p], 4, 5, 6, 7) : __builtin_shufflevector(s.p[p], s.p[p], 0, 1, 2, 3);
+                        }
+                    }
+                    own_sync();
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+#pragma unroll
+                        for (int p = 0; p < 3; p++) {
+                            typedef short s16x4_t __attribute__((ext_vector_type(4)));
+                            typedef __attribute__((address_space(3))) s16x4_t *lds_tr_t;
+                            const bf16x4_t r = __builtin_bit_cast(
+                                bf16x4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                              (lds_tr_t)(tr + p * (16 * 2 * kWave) + (tr_piece ^ (uint32_t)(32 * j)))));
+                            if (h == 0) low[j][p] = r;
+                            else xa[j][p] = __builtin_shufflevector(low[j][p], r, 0, 1, 2, 3, 4, 5, 6, 7);
+                        }
+                }
+                __builtin_amdgcn_sched_barrier(0);    // (the scheduler would move the loads to where they are used)
+                if (step + 1 < steps) request(here, first, step + 1);
+                else if (seg + 1 < segs) request(here, first + kWave, 0);
+                else request(next, next.start, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (real) {
+                    const bf16x8_t *const wt = weights + ((resident ? step : step % kTableSteps) * kSlabs + slab) * (kTiles * 3 * kWave) + id;
+                    bf16x8_t w[2][3];
+#pragma unroll
+                    for (int p = 0; p < 3; p++) w[0][p] = wt[p * kWave];
+#pragma unroll
+                    for (int t = 0; t < kTiles; t++) {
+                        if (t + 1 < kTiles) {
+#pragma unroll
+                            for (int p = 0; p < 3; p++) w[(t + 1) % 2][p] = wt[((t + 1) * 3 + p) * kWave];
+                        }
+                        f32x4_t one[4];               // (summed from zero and then added: the instruction cuts its sums off)
+#pragma unroll
+                        for (int k = 0; k < 6; k++)
+#pragma unroll
+                            for (int j = 0; j < 4; j++)
+                                one[j] = mfma_split(xa[j], w[t % 2], k == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : one[j], k);
+#pragma unroll
+                        for (int j = 0; j < 4; j++) acc[j][t] += one[j];
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+            if (!real) continue;
+            if (!weights_split || __any(rest != rest)) {                           // uniform
+                // values without parts: all of the segment's sums again, with the fp32 instruction
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int t = 0; t < kTiles; t++) acc[j][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                const float *const image = x + (int64_t)here.b * a.xsb + (int64_t)here.y * a.xsy;
+                const auto [id, n, q] = fresh();
+#pragma unroll 1
+                for (int c0 = 0; c0 < a.C; c0 += 4) {
+                    const int c = c0 + (int)q;
+                    const int r = c % kStepChannels, at = (int)n + r % 16 / 4 * 16, e = r % 4 + r / 16 * 4;
+                    float xj[4], wj[kTiles];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float v = image[(int64_t)min(c, a.C - 1) * a.xsc + min(first + 16 * j + (int)n, a.W - 1)];
+                        xj[j] = c < a.C ? (n % 2 ? -v : v) : 0.f;
+                    }
+#pragma unroll
+                    for (int t = 0; t < kTiles; t++) {
+                        const __bf16 *const k = reinterpret_cast<const __bf16 *>(
+                            table + ((int64_t)(min(c, a.C - 1) / kStepChannels * kSlabs + slab) * kTiles + t) * (3 * kWave) + at) + e;
+                        wj[t] = c < a.C ? (float)k[0] + (float)k[8 * kWave] + (float)k[16 * kWave] : 0.f;
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+#pragma unroll
+                        for (int t = 0; t < kTiles; t++) acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xj[j], wj[t], acc[j][t], 0, 0, 0);
+                }
+            }
+
+            // The shifts along x: the staged rows hold the voxels first - 32 .., the outputs are first - 16 .. (at the row end
+            // all that are left, which is a second round of a few lanes).
+            const auto [id, n, q] = fresh();
+            float *const T = reinterpret_cast<float *>(own);
+            const int zero = first - 2 * kHalo;       // voxel of the staged rows' first value
+            const int rounds = first + kWave >= a.W && here.to > first + kWave - kHalo ? 2 : 1;
+            const bool folds = first - 2 * kHalo < 0 || first + kWave + kHalo > a.W;                  // uniform
+            const uint64_t zb = reinterpret_cast<uint64_t>(z + ((int64_t)here.b * 3 * a.out.n * a.H + here.y) * a.W);
+            const int triples_in = 3 * min(max(a.out.n - slab * kSlabOut, 0), kSlabOut);
+#pragma unroll
+            for (int t = 0; t < kTiles; t++) {
+                if (kTriples * t >= triples_in) break;                             // uniform
+                float *const put = T + n * kLine + 4 * q + (n == 15 ? t * kLine : 0);                // (the last columns keep rows of their own)
+                auto stage = [&](int at, const f32x4_t &v) { *reinterpret_cast<f32x4_t *>(put + at) = f32x4_t{v[0], -v[1], v[2], -v[3]}; };
+                own_sync();                           // (x, or the tile before, has been read)
+#pragma unroll
+                for (int j = 0; j < 2; j++) stage(16 * j, before[j][t]);
+#pragma unroll
+                for (int j = 0; j < 4; j++) stage(2 * kHalo + 16 * j, acc[j][t]);
+                own_sync();
+                constexpr int kMost = kTriples + 1;
+                const int triples = t == kTiles - 1 ? kMost : kTriples;
+                for (int round = 0; round < rounds; round++) {
+                    const int xx = first - kHalo + round * kWave + (int)id;
+                    if (round > 0 && id >= kHalo) break;
+                    const bool store = xx >= here.from && xx < here.to;
+                    const int xc = min(max(xx, 0), a.W - 1) - zero;
+                    float sum[kMost][3];
+#pragma unroll
+                    for (int i = 0; i < kMost; i++) {
+                        if (i >= triples) break;
+                        const float *const r = T + 3 * i * kLine;
+                        const int d = a.out.dil[min(slab * kSlabOut + (kTriples * t + i) / 3, a.out.n - 1)];
+                        int lo = xc - d, hi = xc + d;
+                        if (folds) {                  // fold(x - d), fold(x + d)
+                            lo = max(lo, -1 - 2 * zero - lo);
+                            hi = min(hi, 2 * (a.W - zero) - 1 - hi);
+                        }
+                        sum[i][0] = r[lo];
+                        sum[i][1] = r[kLine + xc];
+                        sum[i][2] = r[2 * kLine + hi];
+                    }
+#pragma unroll
+                    for (int i = 0; i < kMost; i++) {
+                        const int tri = kTriples * t + i;
+                        if (i >= triples || tri >= triples_in) break;              // uniform
+                        const float v[1] = {sum[i][0] + sum[i][1] + sum[i][2]};
+                        if (store)
+                            store_global_vec<1>(zb + (uint64_t)(3 * slab * kSlabOut + tri) * (uint64_t)((int64_t)a.H * a.W * 4),
+                                                4u * (uint32_t)xx, v);
+                    }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int t = 0; t < kTiles; t++) before[j][t] = acc[2 + j][t];
+        }
+        here = next;
+    }
+}
+
 // Finishes one layer of a group: the planes that push_rows left, plus NC channels that the group
 // itself has written since, bias and ReLU.
 //
@@ -232,36 +577,50 @@ __global__ __launch_bounds__(V == 1 ? 1024 : 512) void finish_rows(Geom g, RowTe
     int rows[3];
 #pragma unroll
     for (int ky = 0; ky < 3; ky++) rows[ky] = reflect_idx(y + (ky - 1) * g.dil, g.H);
-    float zv[WOUT][3][V], xv[NC > 0 ? NC : 1][3][V];
+    // (channels in batches of at most seven: registers)
+    constexpr int kBatch = NC <= 7 ? (NC > 0 ? NC : 1) : (NC + 1) / 2;
+    float zv[WOUT][3][V], xv[kBatch][3][V];
 #pragma unroll
     for (int co = 0; co < WOUT; co++)
 #pragma unroll
         for (int ky = 0; ky < 3; ky++)
             load_vec<V>(sums.z + (int64_t)b * sums.zsb + ((int64_t)(3 * co + ky) * g.H + rows[ky]) * g.W + x0, zv[co][ky]);
+    auto load = [&](int c0) {
 #pragma unroll
-    for (int c = 0; c < NC; c++)
+        for (int c = 0; c < kBatch; c++)
 #pragma unroll
-        for (int ky = 0; ky < 3; ky++)
-            load_vec<V>(x.p + (int64_t)b * x.sb + c * x.sc + rows[ky] * x.sy + x0, xv[c][ky]);
+            for (int ky = 0; ky < 3; ky++)
+                if (c0 + c < NC) load_vec<V>(x.p + (int64_t)b * x.sb + (c0 + c) * x.sc + rows[ky] * x.sy + x0, xv[c][ky]);
+    };
+    load(0);
 
     float acc[WOUT][3][V];
 #pragma unroll
-    for (int co = 0; co < WOUT; co++) {
+    for (int co = 0; co < WOUT; co++)
 #pragma unroll
         for (int i = 0; i < V; i++) {
             acc[co][0][i] = acc[co][2][i] = 0.f;
             acc[co][1][i] = bias[co] + (zv[co][0][i] + zv[co][1][i] + zv[co][2][i]);
         }
 #pragma unroll
-        for (int c = 0; c < NC; c++)
+    for (int c0 = 0; c0 < NC; c0 += kBatch) {
+        if (c0 > 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            load(c0);
+        }
 #pragma unroll
-            for (int ky = 0; ky < 3; ky++)
+        for (int co = 0; co < WOUT; co++)
 #pragma unroll
-                for (int r = 0; r < 3; r++) {
-                    const float wv = k[co * sums.kco + c * kTaps + ky * 3 + r];
+            for (int c = 0; c < kBatch; c++)
 #pragma unroll
-                    for (int i = 0; i < V; i++) acc[co][r][i] += xv[c][ky][i] * wv;
-                }
+                for (int ky = 0; ky < 3; ky++)
+#pragma unroll
+                    for (int r = 0; r < 3; r++) {
+                        if (c0 + c >= NC) continue;
+                        const float wv = k[co * sums.kco + (c0 + c) * kTaps + ky * 3 + r];
+#pragma unroll
+                        for (int i = 0; i < V; i++) acc[co][r][i] += xv[c][ky][i] * wv;
+                    }
     }
     const int rowlen = V * rt.lpr;
     float *const T = lds + (size_t)team * WOUT * 2 * rowlen;
@@ -317,12 +676,23 @@ hipError_t finish_pick(const Geom &g, const View<const float> &x, const float *k
         case 4: return finish_launch<V, 4, 1>(g, x, k, bias, out, sums, s);
         case 5: return finish_launch<V, 5, 1>(g, x, k, bias, out, sums, s);
         case 6: return finish_launch<V, 6, 1>(g, x, k, bias, out, sums, s);
+        case 7: return finish_launch<V, 7, 1>(g, x, k, bias, out, sums, s);
+        case 8: return finish_launch<V, 8, 1>(g, x, k, bias, out, sums, s);
+        case 9: return finish_launch<V, 9, 1>(g, x, k, bias, out, sums, s);
+        case 10: return finish_launch<V, 10, 1>(g, x, k, bias, out, sums, s);
+        case 11: return finish_launch<V, 11, 1>(g, x, k, bias, out, sums, s);
+        case 12: return finish_launch<V, 12, 1>(g, x, k, bias, out, sums, s);
+        case 13: return finish_launch<V, 13, 1>(g, x, k, bias, out, sums, s);
         }
     } else if (g.Wd == 2) {
         switch (g.C) {
         case 0: return finish_launch<V, 0, 2>(g, x, k, bias, out, sums, s);
         case 2: return finish_launch<V, 2, 2>(g, x, k, bias, out, sums, s);
         case 4: return finish_launch<V, 4, 2>(g, x, k, bias, out, sums, s);
+        case 6: return finish_launch<V, 6, 2>(g, x, k, bias, out, sums, s);
+        case 8: return finish_launch<V, 8, 2>(g, x, k, bias, out, sums, s);
+        case 10: return finish_launch<V, 10, 2>(g, x, k, bias, out, sums, s);
+        case 12: return finish_launch<V, 12, 2>(g, x, k, bias, out, sums, s);
         }
     }
     return hipErrorInvalidConfiguration;
@@ -352,6 +722,50 @@ bool group_push_supported_2d(const Geom &g, const View<const float> &x, int dmax
            (int64_t)g.B * g.H * ((g.W + kWave - 1) / kWave) < ((int64_t)1 << 30);
 }
 
+bool group_split_supported_2d(int64_t W, int dmax) { return W >= 32 && dmax <= group2d::kHalo; }
+
+int64_t group_table_floats_2d(int64_t channels)
+{
+    using namespace group2d;
+    const int64_t steps = (channels + kStepChannels - 1) / kStepChannels;
+    return steps * (kSlabs * kTiles * kTileBytes / 4) + (steps + 3) / 4 * 4;
+}
+
+hipError_t group_push_split_2d(const Geom &g, const View<const float> &x, const group2d::Outputs &out, float *z, float *table,
+                               hipStream_t s)
+{
+    using namespace group2d;
+    int dmax = 0;
+    for (int o = 0; o < out.n; o++) dmax = std::max(dmax, out.dil[o]);
+    if (out.n <= kSlabOut || out.n > kMaxOut || !group_push_supported_2d(g, x, dmax) || !group_split_supported_2d(g.W, dmax))
+        return hipErrorInvalidValue;
+    const int steps = (g.C + kStepChannels - 1) / kStepChannels;
+    SplitArgs a{g.C, g.H, g.W, 0, 1, 0, x.sb, x.sc, x.sy, out};
+    // Parts of a row: the waves that are resident take as few segments one after the other as can be.
+    const int64_t rows = (int64_t)g.B * g.H, slots = 256 * kPushTeams;
+    int64_t best = INT64_MAX;
+    for (int parts = 1; parts <= 32; parts++) {
+        const int length = ((g.W + parts - 1) / parts + 3) & ~3;
+        if (parts > 1 && length < kWave) break;
+        const int64_t cost = (rows * parts + slots - 1) / slots * ((std::min(g.W, length + (parts > 1 ? 2 * kHalo : 0)) + kWave - 1) / kWave);
+        if (cost < best) {
+            best = cost;
+            a.parts = parts;
+            a.length = length;
+        }
+    }
+    a.items = (int)(rows * a.parts);
+    const int blocks = (int)std::min<int64_t>(256, (a.items + kPushTeams - 1) / kPushTeams);
+    bf16x8_t *const weights = reinterpret_cast<bf16x8_t *>(table);
+    int *const bad = reinterpret_cast<int *>(table + (int64_t)steps * (kSlabs * kTiles * kTileBytes / 4));
+    hipLaunchKernelGGL(push_table, dim3(steps), dim3(kSlabs * kTiles * kWave), 0, s, a, weights, bad);
+    static LargeLds large;
+    const hipError_t e = large.allow(reinterpret_cast<const void *>(&push_split), kSplitLds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(push_split, dim3(blocks), dim3(kPushWaves * kWave), kSplitLds, s, a, x.p, weights, bad, z);
+    return hipGetLastError();
+}
+
 hipError_t group_push_2d(const Geom &g, const View<const float> &x, const group2d::Outputs &out, float *z, hipStream_t s)
 {
     using namespace group2d;
@@ -376,7 +790,7 @@ hipError_t group_push_2d(const Geom &g, const View<const float> &x, const group2
 bool group_finish_supported_2d(const Geom &g, const View<const float> &x, const View<float> &out)
 {
     return g.ndim == 2 && x.sx == 1 && out.sx == 1 && group2d::finish_vec(g, x, out) != 0 &&
-           ((g.Wd == 1 && g.C < group2d::kSlabOut) || (g.Wd == 2 && g.C < 6 && g.C % 2 == 0));
+           ((g.Wd == 1 && g.C < group2d::kMaxOut) || (g.Wd == 2 && g.C < group2d::kMaxOut - 1 && g.C % 2 == 0));
 }
 
 hipError_t group_finish_2d(const Geom &g, const View<const float> &x, const float *k, const float *bias,

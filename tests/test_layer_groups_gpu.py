@@ -168,6 +168,60 @@ def test_an_infinity_in_front_of_a_forward_group_stays_one(c_in):
     assert rel_err(found[1][finite], found[0][finite]) <= 1e-5
 
 
+# Forward groups of eight to fourteen outputs (forced; dilations up to 16): one segment of 64 voxels, several, a last
+# one of a single voxel or of less than a halo, of odd lengths; rows in parts; one step of 32 channels, whole
+# steps, one channel more, more than the table of weights holds at once; two channels per layer; dilations
+# above 16, which go in sevens; rows that the finishing launches take one voxel at a time.
+FORWARD_FOURTEEN = [
+    ((40, 64), 2, 1, 14, 1, [1, 16, 5]),
+    ((33, 65), 3, 1, 9, 2, [16, 3]),
+    ((20, 520), 32, 1, 14, 1, None),
+    ((17, 111), 33, 1, 14, 3, [12, 7, 1]),
+    ((9, 1021), 12, 1, 16, 1, [9, 2]),
+    ((1100, 35), 130, 1, 14, 1, [1, 2, 4, 8]),
+    ((12, 1024), 7, 2, 7, 1, None),
+    ((27, 499), 6, 2, 7, 1, [3, 12]),
+    ((30, 32), 65, 1, 14, 1, [16, 15]),
+    ((20, 96), 5, 1, 15, 1, [17, 1]),
+    ((5, 2048), 30, 2, 5, 1, [5, 1]),
+]
+
+
+@pytest.mark.parametrize("case", FORWARD_FOURTEEN, ids=lambda c: "x".join(map(str, c[0])) + "-c%d-w%d-d%d-B%d" % c[1:5])
+def test_block_in_forward_groups_of_up_to_fourteen(case):
+    size, c_in, width, depth, batch, dilations = case
+    dilations = [(dilations or range(1, 11))[i % len(dilations or range(1, 11))] for i in range(depth)]
+    with tuning({"fwd.group": -2}):
+        check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=61)
+
+
+@pytest.mark.parametrize("where", ["input", "weight"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
+def test_values_without_bf16_parts_in_front_of_a_forward_group(where, value):
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator().manual_seed(37)
+    c_in, depth, size = 45, 9, (22, 513)
+    image = torch.rand(1, c_in, *size, generator=gen).cuda()
+    # (small weights of one sign: what a layer makes of the largest finite value is finite)
+    weights = [(torch.rand(1, c_in + i, 3, 3, generator=gen) * 1e-3 + 1e-4).cuda() for i in range(depth)]
+    if where == "input":
+        image[0, c_in - 1, 17, 511] = value
+    else:
+        weights[2][0, 40, 1, 2] = value
+        image[0, 40] = image[0, 40] * 1e-3 + 1e-4
+    found = []
+    for setting in (0, -2):
+        stack = torch.empty(1, c_in + depth, *size, device="cuda")
+        stack[:, :c_in] = image
+        with tuning({"fwd.group": setting}):
+            cc.block_forward(stack, c_in, [1, 12, 3, 1, 2, 3, 1, 2, 3], torch.zeros(depth, device="cuda"), weights)
+        found.append(stack[:, c_in:])
+    assert torch.equal(torch.isnan(found[0]), torch.isnan(found[1]))
+    assert torch.equal(torch.isinf(found[0]), torch.isinf(found[1]))
+    finite = torch.isfinite(found[0])
+    assert bool(finite.any()) and rel_err(found[1][finite], found[0][finite]) <= 1e-5
+
+
 # Rows that the finishing launch does not take (more than 1024 voxels that are not whole groups of
 # four, more than 2048): fwd_lattice adds the planes, with no channel of the group's own and with some.
 @pytest.mark.parametrize("case", [
