@@ -1018,7 +1018,8 @@ int block_group_fused(const char *fn, const BlockArgs &a, int i, int n, int64_t 
 }
 
 // ---------------------------------------------------------------------------
-// 3D blocks of one-channel layers: the reverse loop as two streams of work.
+// 3D blocks of one-channel layers: the reverse loop as two streams of work, where the groups of
+// msd_pull.hip do not apply (rows of fewer than 32 voxels, channels 2^26 values apart, no room).
 //
 // Only the input gradient makes the reverse loop a chain (layer i's masked output gradient
 // is complete once every layer above has added its share to that channel); the weight and
@@ -1079,9 +1080,9 @@ int block_backward_split3d(const char *fn, const BlockArgs &a, int64_t c_in, con
                            bool *done)
 {
     *done = false;
-    // By default wherever the kernels take the shapes: the two streams gain what the launches'
-    // ramps and tails leave idle (about 15 to 30 microseconds per launch) and the chain moves half
-    // the bytes of grad_input (128^3, depth 50: 6.8 against 8.2 ms for the backward pass; 256^3,
+    // Against one layer at a time the two streams gain what the launches' ramps and tails leave
+    // idle (about 15 to 30 microseconds per launch), and the chain moves half the bytes of
+    // grad_input (128^3, depth 50: 6.8 against 8.2 ms for the backward pass; 256^3,
     // depth 30: 35.0 against 35.9 ms per step; 160 x 160 x 256, depth 50: 30.7 against 34.0 ms).
     const int mode = msd::knob(msd::kKnobBlockSplit3d, 1);
     if (mode == 0 || a.dtype != MSD_F32 || a.ndim != 3 || g_kernel_path != 0 || !grad_bias || a.depth < 2 ||
@@ -1256,7 +1257,7 @@ int block_backward_split3d(const char *fn, const BlockArgs &a, int64_t c_in, con
 }
 
 // ---------------------------------------------------------------------------
-// Groups of layers of the 2D backward pass on the matrix cores (msd_pull.hip).
+// Groups of layers of the backward pass on the matrix cores (msd_pull.hip).
 // ---------------------------------------------------------------------------
 
 // Channels below the lowest layer of a group from which on it is taken: always.  256 x 256, depth 10, recorded step:
@@ -1264,6 +1265,10 @@ int block_backward_split3d(const char *fn, const BlockArgs &a, int64_t c_in, con
 // at depth 30 and 100 (3 x 333 x 477, 1024 x 1024).  A group takes up to 14 outputs wherever there are that many: at
 // 1024 x 1024 a pass and the upper half's share of the lower (49 us) are as fast as two groups of seven over
 // 20 channels (266 us both), 332 against 371 us over 48, 552 against 860 over 95.
+// Volumes: up to four outputs (two slabs of 54 of 64 rows), at every size; backward pass of the whole block, us, one layer
+// at a time or the two streams of block_backward_split3d, and groups: 16 x 16 x 32, depth 10: 207, 110; 61 x 93 x 75, depth 20: 891, 622
+// (groups of two outputs 684); 96 x 101 x 160, depth 30: 3268, 2152; 127^3, depth 50: 9761, 5337 (6396); 128^3: 6846, 5350 (5904);
+// 192^3, depth 10: 3209, 2564; two channels per layer, 128^3, depth 25: 7393, 4936.
 constexpr int64_t kGroupBackChannels = 1;
 
 // Number of layers from layer i down that form a group of the backward pass (0: none); `first` is
@@ -1271,13 +1276,15 @@ constexpr int64_t kGroupBackChannels = 1;
 int backward_group(const BlockArgs &a, int i, int64_t first)
 {
     const int from = msd::knob(msd::kKnobBwdGroup, -1);
-    if (a.dtype != MSD_F32 || a.ndim != 2 || g_kernel_path != 0 || from == 0 || !msd::knob(msd::kKnobBlockFuse, 1)) return 0;
-    // (a caller who sets how layers are paired gets the pairs)
-    if (from < 0 && (msd::knob(msd::kKnobBlockPair, -1) >= 0 || msd::knob(msd::kKnobBlockTriple, -1) >= 0)) return 0;
+    if (a.dtype != MSD_F32 || g_kernel_path != 0 || from == 0 || !msd::knob(msd::kKnobBlockFuse, 1)) return 0;
+    // (a caller who sets how layers are paired gets the pairs, who sets how the two streams are used gets these)
+    if (from < 0 && a.ndim == 2 && (msd::knob(msd::kKnobBlockPair, -1) >= 0 || msd::knob(msd::kKnobBlockTriple, -1) >= 0)) return 0;
+    if (from < 0 && a.ndim == 3 && (msd::knob(msd::kKnobBlockSplit3d, -1) >= 0 || msd::knob(msd::kKnobBlockChainPair, -1) >= 0)) return 0;
     const int64_t least = from > 0 ? from : kGroupBackChannels;
     int n = 0;
     int64_t outputs = 0, c = first + a.widths[i];
-    while (i - n >= 0 && a.widths[i - n] <= 2 && outputs + a.widths[i - n] <= msd::group2d::kMaxOut &&
+    const int most = a.ndim == 3 ? 2 * msd::group2d::kSlabOut3d : msd::group2d::kMaxOut;
+    while (i - n >= 0 && a.widths[i - n] <= 2 && outputs + a.widths[i - n] <= most &&
            c - a.widths[i - n] >= least) {
         outputs += a.widths[i - n];
         c -= a.widths[i - n++];
@@ -1289,8 +1296,8 @@ int64_t backward_group_bytes(const BlockArgs &a)
 {
     int64_t total = a.c_in, most = 0;
     for (int i = 0; i < a.depth; i++) {
-        if (a.ndim == 2 && a.dtype == MSD_F32 && a.widths[i] <= 2) {
-            const int64_t n = msd::group_pull_floats_2d(a.batch, a.spatial[0], a.spatial[1], total);
+        if (a.dtype == MSD_F32 && a.widths[i] <= 2) {
+            const int64_t n = msd::group_pull_floats(a.batch, a.ndim == 3 ? a.spatial[0] * a.spatial[1] : a.spatial[0], a.spatial[a.ndim - 1], total);
             most = n > most ? n : most;
         }
         total += a.widths[i];
@@ -1302,8 +1309,8 @@ int64_t backward_group_bytes(const BlockArgs &a)
 // that the layers of the group wrote are completed one layer after the other, then one pass over
 // the channels of the stack adds what all of them contribute to the channels below the group and
 // forms all their weight and bias gradients.  *done is false (and nothing was launched) where a
-// kernel does not take the shape.
-int block_group_backward(const char *fn, const BlockArgs &a, int i, int n, int64_t first, bool need_input_grad,
+// kernel does not take the shape.  ask: launch nothing, set *done only.
+int block_group_backward(const char *fn, const BlockArgs &a, int i, int n, int64_t first, bool ask, bool need_input_grad,
                          const void *stack, const int64_t *stack_strides, void *grads, const int64_t *grads_strides,
                          const void *const *weights, void *const *grad_weights, float *gb_lowest, float *ws,
                          int64_t ws_bytes, hipStream_t s, int pass_no, bool *masked, bool *done)
@@ -1325,22 +1332,27 @@ int block_group_backward(const char *fn, const BlockArgs &a, int i, int n, int64
     msd::group2d::Outputs out{};
     int channels[msd::group2d::kMaxOut];
     float *gk[msd::group2d::kMaxOut];
+    const int64_t taps = a.ndim == 3 ? 27 : msd::group2d::kTaps;
     int start[msd::group2d::kMaxOut];             // first output of the group's layers
     int64_t read = c;                             // channels that the layer at hand reads
     for (int j = lo; j <= i; j++) {
         start[j - lo] = out.n;
         for (int co = 0; co < a.widths[j]; co++) {
             out.dil[out.n] = (int)a.dilations[j];
-            out.k[out.n] = (const float *)weights[j] + co * read * msd::group2d::kTaps;
-            gk[out.n] = (float *)grad_weights[j] + co * read * msd::group2d::kTaps;
+            out.k[out.n] = (const float *)weights[j] + co * read * taps;
+            gk[out.n] = (float *)grad_weights[j] + co * read * taps;
             channels[out.n++] = (int)read;
         }
         read += a.widths[j];
     }
     msd::Geom g;
     MSD_TRY(make_geom(fn, a.dtype, a.ndim, a.batch, first, out.n, a.spatial, dmax, true, &g));
-    if (!msd::group_pull_supported_2d(g, x, gx)) return MSD_OK;
-    if (ws_bytes < msd::group_pull_floats_2d(g.B, g.H, g.W, first) * (int64_t)sizeof(float)) return MSD_OK;
+    if (!msd::group_pull_supported(g, x, gx)) return MSD_OK;
+    if (ws_bytes < msd::group_pull_floats(g.B, (int64_t)g.D * g.H, g.W, first) * (int64_t)sizeof(float)) return MSD_OK;
+    if (ask) {
+        *done = true;
+        return MSD_OK;
+    }
     ProfileScope scope(3, s);
     // The layers whose outputs are the upper slab (the last seven outputs or fewer) complete one another;
     // what they add to the channels below them in the group is added to all of these at once.
@@ -1350,7 +1362,7 @@ int block_group_backward(const char *fn, const BlockArgs &a, int i, int n, int64
         msd::group2d::Outputs up{};
         for (int o = from; o < to; o++) {
             up.dil[up.n] = out.dil[o];
-            up.k[up.n++] = out.k[o] + (int64_t)ch * msd::group2d::kTaps;
+            up.k[up.n++] = out.k[o] + ch * taps;
         }
         return up;
     };
@@ -1360,14 +1372,13 @@ int block_group_backward(const char *fn, const BlockArgs &a, int i, int n, int64
         const hipError_t e = j == top - 1
                                  ? msd::group_spread_back_2d(g, x, gx, (int)c, start[top - lo], (int)a.widths[j],
                                                              above(start[top - lo], out.n, (int)c), s)
-                                 : msd::group_finish_back_2d(g, x, gx, ch, (int)a.widths[j],
-                                                             above(from, j < top ? start[top - lo] : out.n, ch), s);
+                                 : msd::group_finish_back(g, x, gx, ch, (int)a.widths[j],
+                                                          above(from, j < top ? start[top - lo] : out.n, ch), s);
         if (e != hipSuccess) return hip_fail(fn, e);
     }
     const bool update = lo > 0 || need_input_grad;
     const int mask_from = lo > 0 ? (int)(c - a.widths[lo - 1]) : (int)first;
-    const hipError_t e = msd::group_pull_2d(g, x, out, update ? (int)c : 0, mask_from, gx, (int)c, channels, gk, gb_lowest,
-                                            ws, msd::knob(msd::kKnobBlockSnake, 1) && (pass_no & 1), s);
+    const hipError_t e = msd::group_pull(g, x, out, update ? (int)c : 0, mask_from, gx, (int)c, channels, gk, gb_lowest, ws, msd::knob(msd::kKnobBlockSnake, 1) && (pass_no & 1), s);
     if (e != hipSuccess) return hip_fail(fn, e);
     *masked = lo > 0;
     *done = true;
@@ -1611,7 +1622,12 @@ int msd_block_backward(int dtype, int ndim, int64_t batch, int64_t c_in, int dep
         pending.base = (float *)((char *)workspace + layer_ws);
         pending.capacity = (workspace_bytes - layer_ws) / (int64_t)sizeof(float);
     }
-    {
+    bool grouped = false;                         // volumes: the uppermost layers form a group
+    if (const int n = ndim == 3 ? backward_group(a, depth - 1, last - widths[depth - 1]) : 0)
+        MSD_TRY(block_group_backward(fn, a, depth - 1, n, last - widths[depth - 1], true, need_input_grad != 0, stack, stack_strides,
+                                     grads, grads_strides, weights, grad_weights, (float *)grad_bias, (float *)workspace,
+                                     workspace_bytes, (hipStream_t)stream, 0, &grouped, &grouped));
+    if (!grouped) {
         bool done = false;
         MSD_TRY(block_backward_split3d(fn, a, c_in, stack, stack_strides, grads, grads_strides, weights, grad_weights,
                                        grad_bias, need_input_grad != 0, workspace, workspace_bytes, (hipStream_t)stream,
@@ -1640,7 +1656,7 @@ int msd_block_backward(int dtype, int ndim, int64_t batch, int64_t c_in, int dep
             for (int j = 1; j < n; j++) below += widths[i - j];
             MSD_TRY(pending.flush(fn));           // (its regions and the group's partial sums share the workspace)
             bool done = false;
-            MSD_TRY(block_group_backward(fn, a, i, n, first, need_input_grad != 0, stack, stack_strides, grads, grads_strides,
+            MSD_TRY(block_group_backward(fn, a, i, n, first, false, need_input_grad != 0, stack, stack_strides, grads, grads_strides,
                                          weights, grad_weights, gb ? (float *)gb - below : nullptr, (float *)workspace,
                                          workspace_bytes, (hipStream_t)stream, groups_done, &masked, &done));
             if (done) {

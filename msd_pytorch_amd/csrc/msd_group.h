@@ -1,4 +1,4 @@
-// Groups of consecutive layers of a dense block on the matrix cores (2D, fp32).
+// Groups of consecutive layers of a dense block on the matrix cores (fp32; 3D: the backward pass).
 //
 // The layers i, i + 1, ... of a group read the same channels [0, c) of the stack, c the number
 // of channels in front of the first of them.  Taken together they are one matrix product over
@@ -14,6 +14,7 @@ namespace group2d {
 
 constexpr int kTaps = 9;
 constexpr int kSlabOut = 7;                       // outputs of a slab: 7 * 9 = 63 of 64 matrix rows
+constexpr int kSlabOut3d = 2;                     // 3D: 2 * 27 = 54
 constexpr int kRows = 64;                         // matrix rows of a slab
 constexpr int kMaxOut = 14;                       // outputs of a group: one or two slabs
 constexpr int kMaxAbove = 7;                      // outputs that complete a channel of the group in one launch
@@ -83,17 +84,17 @@ hipError_t group_finish_2d(const Geom &g, const View<const float> &x, const floa
 // Backward pass of a group over the channels [0, g.C) of the stack x: the first `update` channels of
 // grads get grad_input (masked with their activations from `mask_from` on), gk[o] the weight gradients
 // of output o's channels[o] input channels, gb the bias gradients.  The outputs' gradients are the
-// channels from `first` on.  ws: group_pull_floats_2d floats.
-int64_t group_pull_floats_2d(int64_t batch, int64_t H, int64_t W, int64_t channels);
-bool group_pull_supported_2d(const Geom &g, const View<const float> &x, const View<float> &gx);
-hipError_t group_pull_2d(const Geom &g, const View<const float> &x, const group2d::Outputs &out, int update, int mask_from,
-                         const View<float> &grads, int first, const int *channels, float *const *gk, float *gb,
-                         float *ws, bool reverse, hipStream_t s);
+// channels from `first` on.  ws: group_pull_floats floats (rows: of an image, or of all slices of a volume).
+int64_t group_pull_floats(int64_t batch, int64_t rows, int64_t W, int64_t channels);
+bool group_pull_supported(const Geom &g, const View<const float> &x, const View<float> &gx);
+hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::Outputs &out, int update, int mask_from,
+                      const View<float> &grads, int first, const int *channels, float *const *gk, float *gb,
+                      float *ws, bool reverse, hipStream_t s);
 
 // Completes the gradient of the `width` channels from `channel` on: adds what the outputs right
 // above them (`above`, their weights of these channels) contribute, and applies the ReLU mask.
-hipError_t group_finish_back_2d(const Geom &g, const View<const float> &x, const View<float> &grads, int channel, int width,
-                                const group2d::Outputs &above, hipStream_t s);
+hipError_t group_finish_back(const Geom &g, const View<const float> &x, const View<float> &grads, int channel, int width,
+                             const group2d::Outputs &above, hipStream_t s);
 
 // Adds to the gradients of the `channels` channels from `channel` on what the outputs right above
 // them (at most kSlabOut) contribute, and completes the last `width` of them.

@@ -24,6 +24,11 @@
 // A training step at 1024 x 1024, depth 100: 6.35 -> 5.33 ms; 4 x 512 x 512: 6.25 -> 4.99; 2048 x 2048, two
 // channels per layer, depth 200: 275 -> 194.
 //
+// Volumes (N = 3): two outputs of 27 taps in a slab's 64 rows, up to four in a group, the same tiles over the rows of all
+// slices.  128^3 over 1 to 46 channels: 338 us on average for four layers, and 140 for completing their own
+// channels, where the two streams of one and two layers per pass took 1060; 61 x 93 x 75: 79 and 33 (336).  Bound as above; every
+// tile lies at an edge there (27 values folded along three axes instead of 63 along two).
+//
 // Tried on the way: waves that walk the channels on their own tile (weights in LDS, loads in the matrix layout): 650 us
 // over 95 channels, 320 over 45; two workgroups of four waves per compute unit: 604 and 293; for 5 to 8 blocks
 // two chunks of at most 4: 588.  Any register spilt in the loop costs 10 % (its reload waits for all loads and stores).
@@ -51,14 +56,22 @@ constexpr int unit_bytes(int voxels) { return 3 * 16 * (2 * voxels + 16); }
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
 
+template <int N> struct Gather {
+    static constexpr int kTaps = N == 3 ? 27 : group2d::kTaps;
+    static constexpr int kLines = kTaps / 3;             // taps along x apart
+    static constexpr int kOutputs = N == 3 ? kSlabOut3d : kSlabOut;        // of a slab
+    static constexpr int kLaneOut = N == 3 ? 1 : 4;      // that a lane holds
+};
+
 // Row m of a slab's 64: the halves of 32 belong to the lanes h = 0 and 1 of the gather.  A lane holds
-// whole outputs (the folds at the image's edges move values between an output's rows): three of nine
-// taps each, and of the seventh output, which both gather, five or four taps.
+// whole outputs (the folds at the image's edges move values between an output's rows).  2D: three of nine
+// taps each, and of the seventh output, which both gather, five or four taps.  3D: one of 27.
 struct Slot {
     int output, tap;                              // tap < 0: a row of zeros
 };
-__host__ __device__ __forceinline__ Slot slot_of(int m)
+template <int N> __host__ __device__ __forceinline__ Slot slot_of(int m)
 {
+    if (N == 3) return Slot{m / 32, m % 32 < 27 ? m % 32 : -1};
     const int h = m / 32 % 2, s = m % 32, first = m / kRows * kSlabOut;
     if (s < 27) return Slot{first + 3 * h + s / kTaps, s % kTaps};
     const int tap = 5 * h + s - 27;
@@ -95,13 +108,13 @@ struct Divisor {
 struct PullArgs {
     int C, update;                                // channels of x; the first `update` of them have grad_input
     int mask_from;                                // channels from here on are masked with their activation
-    int H, W, segs, items;                        // items: segments of an image
+    int D, H, W, segs, items;                     // items: segments of an image
     int tiles, image_tiles;                       // of all images, of one
-    Divisor by_segs, by_tiles;
+    Divisor by_segs, by_tiles, by_rows;           // by_rows: rows of a slice (3D)
     int reverse;                                  // walk the tiles from the last to the first
     int dmax;
     Chunks chunks;
-    int64_t sb, sc, sy;                           // strides of x and of the gradients
+    int64_t sb, sc, sz, sy;                       // strides of x and of the gradients
     Outputs out;
 };
 
@@ -157,8 +170,8 @@ __device__ __forceinline__ void fold(const Sides &s, float &tap0, float &tap2)
 }
 
 // What a workgroup of pull_rows keeps in LDS besides A and the waves' own space.
-struct Source {                                   // an output's place in bytes: its dilation in rows and in voxels, its plane
-    uint32_t rows, voxels, plane, pad;
+struct Source {                                   // an output's place in bytes: its dilation in slices, rows and voxels, its plane
+    uint32_t slices, rows, voxels, plane;
 };
 struct PullShared {
     Source sources[kMaxOut];
@@ -176,7 +189,6 @@ template <int G, int P> struct PullShape {
     static constexpr int kVec = kUnit / 16;              // 16-byte accesses per lane for a unit of 16 channels
     static constexpr int kLanes = kUnit / 4;             // lanes of a channel in one of them
     static constexpr int kOwnBytes = unit_bytes(kUnit);
-    static constexpr int kLaneOut = 4;                   // outputs that a lane of the gather holds
 };
 
 // What the kernel keeps for its life: the weights of rows 32 step + 8 q .. of channel n in parts, the sums of
@@ -189,14 +201,15 @@ template <int G> struct PullState {
 
 // The tiles of a workgroup.  True where units were left out that hold values which cannot be split: the second
 // run (WHOLE) takes these, with the fp32 instruction.  Apart, so that it keeps no registers in the first.
-template <int G, int P, bool WHOLE>
+template <int N, int G, int P, bool WHOLE>
 __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__restrict__ x, const float *gy, float *gx, float *row,
                                            char *lds, PullShared &shared, int tid, int wave, int blocks, int c0, int wgs, int wg,
                                            PullState<G> &state)
 {
     using S = PullShape<G, P>;
     constexpr int kSegs = S::kSegs, kSteps = S::kSteps, kTiles = S::kTiles, kUnit = S::kUnit, kUnits = S::kUnits, kVec = S::kVec;
-    constexpr int kLanes = S::kLanes, kOwnBytes = S::kOwnBytes, kLaneOut = S::kLaneOut;
+    constexpr int kLanes = S::kLanes, kOwnBytes = S::kOwnBytes;
+    constexpr int kTaps = Gather<N>::kTaps, kLines = Gather<N>::kLines, kLaneOut = Gather<N>::kLaneOut, kSlabOut = Gather<N>::kOutputs;
     const int lane = tid % kWave;
     const int cb = wave / P, ch0 = c0 + cb * 16;  // the wave's block
     const bool active = cb < blocks, update = ch0 < a.update;       // uniform
@@ -211,7 +224,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         uint32_t sign;                            // of x in this tile
     };
     struct Place {
-        int x0, skip, y;                          // first voxel, voxels that belong to the segment before, row
+        int x0, skip, y, z;                       // first voxel, voxels that belong to the segment before, row, slice
         bool valid;
     };
     // (past the last tile that one again)
@@ -230,11 +243,14 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         const int it = min(t.first + segment, a.items - 1);
         p.y = a.by_segs.of(it);
         const int own0 = (it - p.y * a.segs) * kSegment;
+        p.z = N == 3 ? a.by_rows.of(p.y) : 0;
+        p.y -= N == 3 ? p.z * a.H : 0;
         p.x0 = min(own0, a.W - kSegment);         // (the last segment of a row overlaps the one before)
         p.skip = p.valid ? own0 - p.x0 : kSegment;
         return p;
     };
     const uint32_t plane = (uint32_t)a.sc * 4u;
+    auto row_at = [&](int z, int y) { return (N == 3 ? z * (int)a.sz : 0) + y * (int)a.sy; };
 
     // The tiles: kSegs consecutive segments of an image each; every workgroup of an XCD works on neighbouring ones.
     const int lb = block_for_xcd(wg, wgs, wgs % kXcds == 0);
@@ -252,7 +268,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         const int first = ((wave % P) * kUnits + u) * (kUnit / kSegment);
         const Place p0 = locate(t, first), p1 = locate(t, first + kUnit / kSegment - 1);
         const int sel = lv / (kSegment / 4), v4 = lv % (kSegment / 4) * 4;
-        const uint32_t at0 = 4u * (uint32_t)(p0.y * (int)a.sy + p0.x0), at1 = 4u * (uint32_t)(p1.y * (int)a.sy + p1.x0);
+        const uint32_t at0 = 4u * (uint32_t)(row_at(p0.z, p0.y) + p0.x0), at1 = 4u * (uint32_t)(row_at(p1.z, p1.y) + p1.x0);
         Unit un;
         un.img = t.img;
         un.at = (sel ? at1 : at0) + 4u * (uint32_t)v4;
@@ -277,35 +293,38 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
 
     f32x4_t xs[kVec], gs[kVec];
 
-    // ---- the gather: lane (v, h) takes its outputs at voxel v of the wave's segment, 36 values for 32 rows
+    // ---- the gather: lane (v, h) takes its outputs at voxel v of the wave's segment, 36 (27) values for 32 rows
     // m.  Its loads are issued in the tile before, in front of that tile's last stores and requests (all of
     // them retire in order: behind those it would wait for memory).
     const int segment = wave / G, slab = wave % G;
     const int v = lane % kSegment, h = lane / kSegment;
-    const uint32_t bias = 4u * (uint32_t)(a.dmax * (int)a.sy);
+    const uint32_t bias = 4u * (uint32_t)row_at(a.dmax, a.dmax);
+    auto output_of = [&](int j) { return N == 3 ? h : j < 3 ? 3 * h + j : 6; };
     auto source = [&](int j) {
-        int o = j < 3 ? 3 * h + j : 6;
+        int o = output_of(j);
         asm volatile("" : "+v"(o));
         return shared.sources[slab * kSlabOut + o];
     };
     auto away = [&](const Place &p) {             // uniform: from all edges
-        return p.x0 >= a.dmax && p.x0 + kSegment + a.dmax <= a.W && p.y >= a.dmax && p.y + a.dmax < a.H;
+        return p.x0 >= a.dmax && p.x0 + kSegment + a.dmax <= a.W && p.y >= a.dmax && p.y + a.dmax < a.H &&
+               (N == 2 || (p.z >= a.dmax && p.z + a.dmax < a.D));
     };
-    float val[kLaneOut][3][3];
+    float val[kLaneOut][kLines][3];
     auto gather = [&](const Tile &t, const Place &p) {
         const uint32_t u = (uint32_t)(p.x0 + v);
         if (away(p)) {
-            const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)(t.img + (int64_t)p.y * a.sy * 4) - bias;
+            const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)(t.img + (int64_t)row_at(p.z, p.y) * 4) - bias;
 #pragma unroll
             for (int j = 0; j < kLaneOut; j++) {
                 const Source o = source(j);
                 const uint32_t c = o.plane + bias + 4u * u;
 #pragma unroll
-                for (int ky = 0; ky < 3; ky++) {
-                    const uint32_t r = ky == 0 ? c + o.rows : ky == 1 ? c : c - o.rows;
-                    val[j][ky][0] = load1(base, r + o.voxels);
-                    val[j][ky][1] = load1(base, r);
-                    val[j][ky][2] = load1(base, r - o.voxels);
+                for (int l = 0; l < kLines; l++) {
+                    const uint32_t s = N == 2 || l / 3 == 1 ? c : l / 3 == 0 ? c + o.slices : c - o.slices;
+                    const uint32_t r = l % 3 == 0 ? s + o.rows : l % 3 == 1 ? s : s - o.rows;
+                    val[j][l][0] = load1(base, r + o.voxels);
+                    val[j][l][1] = load1(base, r);
+                    val[j][l][2] = load1(base, r - o.voxels);
                 }
                 __builtin_amdgcn_sched_barrier(0);    // (an output's addresses at a time: registers)
             }
@@ -315,14 +334,15 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             for (int j = 0; j < kLaneOut; j++) {
                 const Source o = source(j);
                 const int d = (int)(o.voxels / 4u);
-                const Sides sx = sides((int)u, a.W, d), sy = sides(p.y, a.H, d);
+                const Sides sx = sides((int)u, a.W, d), sy = sides(p.y, a.H, d), sz = sides(p.z, N == 3 ? a.D : 1, N == 3 ? d : 0);
 #pragma unroll
-                for (int ky = 0; ky < 3; ky++) {
-                    const int y = ky == 0 ? sy.up : ky == 1 ? p.y : sy.down;
-                    const uint32_t r = o.plane + 4u * (uint32_t)(y * (int)a.sy);
-                    val[j][ky][0] = load1(base, r + 4u * (uint32_t)sx.up);
-                    val[j][ky][1] = load1(base, r + 4u * u);
-                    val[j][ky][2] = load1(base, r + 4u * (uint32_t)sx.down);
+                for (int l = 0; l < kLines; l++) {
+                    const int y = l % 3 == 0 ? sy.up : l % 3 == 1 ? p.y : sy.down;
+                    const int z = N == 2 || l / 3 == 1 ? p.z : l / 3 == 0 ? sz.up : sz.down;
+                    const uint32_t r = o.plane + 4u * (uint32_t)row_at(z, y);
+                    val[j][l][0] = load1(base, r + 4u * (uint32_t)sx.up);
+                    val[j][l][1] = load1(base, r + 4u * u);
+                    val[j][l][2] = load1(base, r + 4u * (uint32_t)sx.down);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -333,23 +353,34 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
 #pragma unroll
             for (int j = 0; j < kLaneOut; j++) {
                 const int d = (int)(source(j).voxels / 4u);
-                const Sides sx = sides(p.x0 + v, a.W, d), sy = sides(p.y, a.H, d);
+                const Sides sx = sides(p.x0 + v, a.W, d), sy = sides(p.y, a.H, d), sz = sides(p.z, N == 3 ? a.D : 1, N == 3 ? d : 0);
 #pragma unroll
-                for (int ky = 0; ky < 3; ky++) fold(sx, val[j][ky][0], val[j][ky][2]);
+                for (int l = 0; l < kLines; l++) fold(sx, val[j][l][0], val[j][l][2]);
 #pragma unroll
-                for (int r = 0; r < 3; r++) fold(sy, val[j][0][r], val[j][2][r]);
+                for (int l = 0; l < kLines; l += 3)
+#pragma unroll
+                    for (int r = 0; r < 3; r++) fold(sy, val[j][l][r], val[j][l + 2][r]);
+                if constexpr (N == 3) {
+#pragma unroll
+                    for (int l = 0; l < 3; l++)
+#pragma unroll
+                        for (int r = 0; r < 3; r++) fold(sz, val[j][l][r], val[j][l + 6][r]);
+                }
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
         if (p.skip > 0 || a.out.n < G * kSlabOut) {                 // uniform
 #pragma unroll
             for (int j = 0; j < kLaneOut; j++) {
-                const bool ok = v >= p.skip && slab * kSlabOut + (j < 3 ? 3 * h + j : 6) < a.out.n;
+                const bool ok = v >= p.skip && slab * kSlabOut + output_of(j) < a.out.n;
 #pragma unroll
                 for (int t = 0; t < kTaps; t++) val[j][t / 3][t % 3] = ok ? val[j][t / 3][t % 3] : 0.f;
             }
         }
-        if (count) shared.bias_sums[tid] += f32x4_t{val[0][1][1], val[1][1][1], val[2][1][1], val[3][1][1]};
+        if (count) {
+            if constexpr (N == 3) shared.bias_sums[tid][0] += val[0][4][1];
+            else shared.bias_sums[tid] += f32x4_t{val[0][1][1], val[1][1][1], val[2][1][1], val[3][1][1]};
+        }
         // -A at every second voxel: the sums of the bf16 instruction are cut off towards minus infinity, which adds up
         // over an image where the gradients themselves cancel (bias gradients: an error of 2e-6 instead of 1.2e-7).
         // For the same reason x changes its sign with the voxel and from tile to tile.
@@ -365,7 +396,9 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             for (int e = 0; e < 8; e++) {
                 const int s = 8 * i + e;
                 if (s < 27) {
-                    e8[e] = val[s / 9][s % 9 / 3][s % 3];
+                    e8[e] = val[s / kTaps][s % kTaps / 3][s % 3];
+                } else if constexpr (N == 3) {
+                    e8[e] = 0.f;
                 } else {
                     const int t0 = s - 27, t1 = s - 22;
                     e8[e] = h ? (t1 < kTaps ? val[3][t1 / 3 % 3][t1 % 3] : 0.f) : val[3][t0 / 3][t0 % 3];
@@ -755,11 +788,12 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
     }
 }
 
-template <int G, int P>
+template <int N, int G, int P>
 __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, const float *__restrict__ x, const float *gy,
                                                              float *gx, float *__restrict__ part, float *__restrict__ bias_part)
 {
-    constexpr int kSegs = PullShape<G, P>::kSegs, kTiles = PullShape<G, P>::kTiles, kLaneOut = PullShape<G, P>::kLaneOut;
+    constexpr int kSegs = PullShape<G, P>::kSegs, kTiles = PullShape<G, P>::kTiles;
+    constexpr int kTaps = Gather<N>::kTaps, kLaneOut = Gather<N>::kLaneOut, kSlabOut = Gather<N>::kOutputs;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), lane = tid % kWave;
@@ -775,7 +809,7 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
     if (tid == 0) shared.bad_again = 0;
     if (tid < G * kSlabOut) {
         const int o = min(tid, a.out.n - 1), d = a.out.dil[o];
-        shared.sources[tid] = Source{4u * (uint32_t)(d * (int)a.sy), 4u * (uint32_t)d, (uint32_t)o * ((uint32_t)a.sc * 4u), 0};
+        shared.sources[tid] = Source{N == 3 ? 4u * (uint32_t)(d * (int)a.sz) : 0u, 4u * (uint32_t)(d * (int)a.sy), 4u * (uint32_t)d, (uint32_t)o * ((uint32_t)a.sc * 4u)};
     }
     state.weights_split = true;
 #pragma unroll
@@ -783,7 +817,7 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
         float v[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const Slot m = slot_of(32 * step + 8 * q + i);
+            const Slot m = slot_of<N>(32 * step + 8 * q + i);
             const bool ok = m.tap >= 0 && m.output < a.out.n && ch0 + n < a.update;
             const float k = a.out.k[ok ? m.output : 0][ok ? (int64_t)(ch0 + n) * kTaps + m.tap : 0];
             v[i] = ok ? k : 0.f;
@@ -803,13 +837,13 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
 #pragma unroll
     for (int t = 0; t < kTiles; t++) state.sums[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     shared.bias_sums[tid] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    const bool again = pull_tiles<G, P, false>(a, x, gy, gx, row, lds, shared, tid, wave, blocks, c0, wgs, wg, state);
+    const bool again = pull_tiles<N, G, P, false>(a, x, gy, gx, row, lds, shared, tid, wave, blocks, c0, wgs, wg, state);
     if (lane == 0 && again) shared.bad_again = 1;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(shared.bad_again) != 0) {    // uniform over the workgroup
         int tid2 = tid;
         asm volatile("" : "+v"(tid2));           // (nothing of the first run is kept for the second)
-        pull_tiles<G, P, true>(a, x, gy, gx, row, lds, shared, tid2, wave, blocks, c0, wgs, wg, state);
+        pull_tiles<N, G, P, true>(a, x, gy, gx, row, lds, shared, tid2, wave, blocks, c0, wgs, wg, state);
     }
 
     // the sums, of the waves that share a block through LDS
@@ -848,7 +882,7 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
     if (v == 0) {
 #pragma unroll
         for (int j = 0; j < kLaneOut; j++)
-            if (j < 3 || h == 0) red[wave * kBiasColumns + (j < 3 ? 3 * h + j : 6)] = bias_sum[j];
+            if (N == 3 || j < 3 || h == 0) red[wave * kBiasColumns + (N == 3 ? h : j < 3 ? 3 * h + j : 6)] = bias_sum[j];
     }
     __syncthreads();
     if (tid < G * kBiasColumns && tid % kBiasColumns < kSlabOut) {
@@ -872,9 +906,11 @@ struct SumArgs {
 
 // Adds the rows of partial sums, 64 columns per workgroup: 16 waves take every 16th row, their
 // sums are added in order.  The last workgroup takes the biases.
+template <int N>
 __global__ __launch_bounds__(1024) void sum_group(const SumArgs a, const float *__restrict__ part,
                                                   const float *__restrict__ bias_part)
 {
+    constexpr int kTaps = Gather<N>::kTaps, kSlabOut = Gather<N>::kOutputs;
     __shared__ float lds[16 * kWave];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int col = blockIdx.x * kWave + lane, block = 1024 * a.slabs;
@@ -918,7 +954,7 @@ __global__ __launch_bounds__(1024) void sum_group(const SumArgs a, const float *
     }
     // column (tile of 16 rows, r, lane (channel, q)) of a block: row 16 tile + 4 q + r
     const int i = col % block, l = i % kWave;
-    const Slot m = slot_of(i / 256 * 16 + l / 16 * 4 + i / kWave % 4);
+    const Slot m = slot_of<N>(i / 256 * 16 + l / 16 * 4 + i / kWave % 4);
     const int ch = blk * 16 + l % 16;
     if (m.tap >= 0 && m.output < a.n && ch < a.channels[m.output]) a.gk[m.output][(int64_t)ch * kTaps + m.tap] += s;
 }
@@ -926,72 +962,89 @@ __global__ __launch_bounds__(1024) void sum_group(const SumArgs a, const float *
 // grad_input of the channels that layers of a group wrote, from the outputs of the layers above them
 // in the group.
 //
-// One voxel per lane; the nine values of each output come straight from the caches (a group's planes
+// One voxel per lane; the nine (27) values of each output come straight from the caches (a group's planes
 // were written or read by the launches before), with no LDS and no barrier: the launches are bound by
 // their ramp and by the vector cache.
 struct FinishArgs {
-    int H, W, segs, items, dmax;
+    int D, H, W, segs, items, dmax;
     int n, channels, masked;                      // spread_back: outputs above, channels, first one to mask
-    int64_t sb, sc, sy;
+    int64_t sb, sc, sz, sy;
     int dil[kMaxAbove];
     const float *k[kMaxAbove];                    // of the first of the channels
 };
 
 // The lane's place, and the adjoint gather there.
 struct FinishPlace {
-    int y, u, own;                                // row, voxel, whether the voxel is the lane's own
+    int z, y, u, own;                             // slice, row, voxel, whether the voxel is the lane's own
     bool away;                                    // uniform: from all edges
     int64_t img;
     uint32_t here;
 };
-__device__ __forceinline__ FinishPlace finish_place(const FinishArgs &a, int it)
+template <int N> __device__ __forceinline__ FinishPlace finish_place(const FinishArgs &a, int it)
 {
     FinishPlace p;
     const int row = it / a.segs, xw = (it - row * a.segs) * kWave;
-    const int b = row / a.H;
-    p.y = row - b * a.H;
+    const int slice = row / a.H, b = N == 3 ? slice / a.D : slice;
+    p.y = row - slice * a.H;
+    p.z = slice - b * (N == 3 ? a.D : 1);
     const int u0 = xw + threadIdx.x % kWave;
     p.u = min(u0, a.W - 1);
     p.own = u0 < a.W;
-    p.away = xw >= a.dmax && xw + kWave + a.dmax <= a.W && p.y >= a.dmax && p.y + a.dmax < a.H;
+    p.away = xw >= a.dmax && xw + kWave + a.dmax <= a.W && p.y >= a.dmax && p.y + a.dmax < a.H &&
+             (N == 2 || (p.z >= a.dmax && p.z + a.dmax < a.D));
     p.img = (int64_t)b * a.sb * 4;
-    p.here = 4u * (uint32_t)(p.y * (int)a.sy + p.u);
+    p.here = 4u * (uint32_t)((N == 3 ? p.z * (int)a.sz : 0) + p.y * (int)a.sy + p.u);
     return p;
 }
-__device__ __forceinline__ void finish_gather(const FinishArgs &a, const FinishPlace &p, uint64_t output, int d, float (&A)[3][3])
+template <int N>
+__device__ __forceinline__ void finish_gather(const FinishArgs &a, const FinishPlace &p, uint64_t output, int d, float (&A)[Gather<N>::kLines][3])
 {
-    Sides sx = {p.u + d, p.u - d, true, true}, sy = {p.y + d, p.y - d, true, true};      // y: uniform
+    Sides sx = {p.u + d, p.u - d, true, true}, sy = {p.y + d, p.y - d, true, true};      // y, z: uniform
+    Sides sz = {p.z + d, p.z - d, true, true};
     if (!p.away) {
         sx = sides(p.u, a.W, d);
         sy = sides(p.y, a.H, d);
+        if (N == 3) sz = sides(p.z, a.D, d);
     }
 #pragma unroll
-    for (int ky = 0; ky < 3; ky++) {
-        const int y = ky == 0 ? sy.up : ky == 1 ? p.y : sy.down;
-        const uint64_t base = output + (uint64_t)(4 * (int64_t)y * a.sy);
-        A[ky][0] = load1(base, 4u * (uint32_t)sx.up);
-        A[ky][1] = load1(base, 4u * (uint32_t)p.u);
-        A[ky][2] = load1(base, 4u * (uint32_t)sx.down);
+    for (int l = 0; l < Gather<N>::kLines; l++) {
+        const int y = l % 3 == 0 ? sy.up : l % 3 == 1 ? p.y : sy.down;
+        const int z = l / 3 == 0 ? sz.up : l / 3 == 1 ? p.z : sz.down;
+        const uint64_t base = output + (uint64_t)(4 * ((N == 3 ? (int64_t)z * a.sz : 0) + (int64_t)y * a.sy));
+        A[l][0] = load1(base, 4u * (uint32_t)sx.up);
+        A[l][1] = load1(base, 4u * (uint32_t)p.u);
+        A[l][2] = load1(base, 4u * (uint32_t)sx.down);
     }
 }
-__device__ __forceinline__ void finish_fold(const FinishArgs &a, const FinishPlace &p, int d, float (&A)[3][3])
+template <int N>
+__device__ __forceinline__ void finish_fold(const FinishArgs &a, const FinishPlace &p, int d, float (&A)[Gather<N>::kLines][3])
 {
     const Sides sx = sides(p.u, a.W, d), sy = sides(p.y, a.H, d);
 #pragma unroll
-    for (int ky = 0; ky < 3; ky++) fold(sx, A[ky][0], A[ky][2]);
+    for (int l = 0; l < Gather<N>::kLines; l++) fold(sx, A[l][0], A[l][2]);
 #pragma unroll
-    for (int r = 0; r < 3; r++) fold(sy, A[0][r], A[2][r]);
+    for (int l = 0; l < Gather<N>::kLines; l += 3)
+#pragma unroll
+        for (int r = 0; r < 3; r++) fold(sy, A[l][r], A[l + 2][r]);
+    if constexpr (N == 3) {
+        const Sides sz = sides(p.z, a.D, d);
+#pragma unroll
+        for (int l = 0; l < 3; l++)
+#pragma unroll
+            for (int r = 0; r < 3; r++) fold(sz, A[l][r], A[l + 6][r]);
+    }
 }
 
 // The NOUT channels of one layer from the NQ outputs right above, and the channels' ReLU mask: with it
 // they are complete.
-template <int NQ, int NOUT>
+template <int N, int NQ, int NOUT>
 __global__ __launch_bounds__(256) void finish_back(const FinishArgs a, const float *__restrict__ act, float *g)
 {
+    constexpr int kTaps = Gather<N>::kTaps;
     const int lb = block_for_xcd(blockIdx.x, gridDim.x, true);
     const int it = lb * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (it >= a.items) return;                    // uniform over the wave
-    const FinishPlace p = finish_place(a, it);
+    const FinishPlace p = finish_place<N>(a, it);
     const uint64_t img = reinterpret_cast<uint64_t>(g) + (uint64_t)p.img;
     const uint64_t ximg = reinterpret_cast<uint64_t>(act) + (uint64_t)p.img;
     const uint32_t plane = (uint32_t)a.sc * 4u;
@@ -1001,12 +1054,12 @@ __global__ __launch_bounds__(256) void finish_back(const FinishArgs a, const flo
         sum[c] = load1(img, (uint32_t)c * plane + p.here);
         m[c] = load1(ximg, (uint32_t)c * plane + p.here);
     }
-    float A[NQ][3][3];
+    float A[NQ][Gather<N>::kLines][3];
 #pragma unroll
-    for (int o = 0; o < NQ; o++) finish_gather(a, p, img + (uint64_t)(NOUT + o) * plane, a.dil[o], A[o]);
+    for (int o = 0; o < NQ; o++) finish_gather<N>(a, p, img + (uint64_t)(NOUT + o) * plane, a.dil[o], A[o]);
     if (!p.away) {
 #pragma unroll
-        for (int o = 0; o < NQ; o++) finish_fold(a, p, a.dil[o], A[o]);
+        for (int o = 0; o < NQ; o++) finish_fold<N>(a, p, a.dil[o], A[o]);
     }
 #pragma unroll
     for (int c = 0; c < NOUT; c++) {
@@ -1031,7 +1084,7 @@ __global__ __launch_bounds__(256) void spread_back(const FinishArgs a, const flo
     const int lb = block_for_xcd(blockIdx.x, gridDim.x, true);
     const int it = lb * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (it >= a.items) return;                    // uniform over the wave
-    const FinishPlace p = finish_place(a, it);
+    const FinishPlace p = finish_place<2>(a, it);
     const uint64_t img = reinterpret_cast<uint64_t>(g) + (uint64_t)p.img;
     const uint64_t ximg = reinterpret_cast<uint64_t>(act) + (uint64_t)p.img;
     const uint32_t plane = (uint32_t)a.sc * 4u;
@@ -1043,9 +1096,9 @@ __global__ __launch_bounds__(256) void spread_back(const FinishArgs a, const flo
     // output by output, the next one's values requested before this one's products: few registers, so that the
     // waves of a SIMD hide each other's scalar loads of the weights
     float all[kMaxLower] = {}, A[2][3][3];
-    auto gather = [&](int o, float(&to)[3][3]) { finish_gather(a, p, img + (uint64_t)(a.channels + o) * plane, a.dil[o], to); };
+    auto gather = [&](int o, float(&to)[3][3]) { finish_gather<2>(a, p, img + (uint64_t)(a.channels + o) * plane, a.dil[o], to); };
     auto add = [&](int o, float(&from)[3][3]) {
-        if (!p.away) finish_fold(a, p, a.dil[o], from);
+        if (!p.away) finish_fold<2>(a, p, a.dil[o], from);
         const float *const k = a.k[o];
 #pragma unroll
         for (int c = 0; c < kMaxLower; c++) {
@@ -1074,17 +1127,17 @@ __global__ __launch_bounds__(256) void spread_back(const FinishArgs a, const flo
     }
 }
 
-template <int NQ, int NOUT>
+template <int N, int NQ, int NOUT>
 hipError_t finish_back_launch(const FinishArgs &a, const float *act, float *g, hipStream_t s)
 {
-    hipLaunchKernelGGL((finish_back<NQ, NOUT>), dim3(xcd_grid((a.items + 3) / 4)), dim3(256), 0, s, a, act, g);
+    hipLaunchKernelGGL((finish_back<N, NQ, NOUT>), dim3(xcd_grid((a.items + 3) / 4)), dim3(256), 0, s, a, act, g);
     return hipGetLastError();
 }
 
 FinishArgs finish_args(const Geom &g, const View<const float> &x, const group2d::Outputs &above)
 {
     const int segs = (g.W + kWave - 1) / kWave;
-    FinishArgs a{g.H, g.W, segs, g.B * g.H * segs, 0, above.n, 0, 0, x.sb, x.sc, x.sy, {}, {}};
+    FinishArgs a{g.D, g.H, g.W, segs, g.B * g.D * g.H * segs, 0, above.n, 0, 0, x.sb, x.sc, x.sz, x.sy, {}, {}};
     for (int o = 0; o < above.n; o++) {
         a.dil[o] = above.dil[o];
         a.k[o] = above.k[o];
@@ -1093,15 +1146,15 @@ FinishArgs finish_args(const Geom &g, const View<const float> &x, const group2d:
     return a;
 }
 
-template <int G, int P>
+template <int N, int G, int P>
 hipError_t pull_launch(const PullArgs &a, int wgs, const float *x, const float *gy, float *gx, float *part, float *bias_part,
                        hipStream_t s)
 {
     constexpr int kLds = kWaves * (kSlabBytes + PullShape<G, P>::kOwnBytes);
     static LargeLds large;
-    const hipError_t e = large.allow(reinterpret_cast<const void *>(&pull_rows<G, P>), kLds);
+    const hipError_t e = large.allow(reinterpret_cast<const void *>(&pull_rows<N, G, P>), kLds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((pull_rows<G, P>), dim3(wgs), dim3(kWaves * kWave), kLds, s, a, x, gy, gx, part, bias_part);
+    hipLaunchKernelGGL((pull_rows<N, G, P>), dim3(wgs), dim3(kWaves * kWave), kLds, s, a, x, gy, gx, part, bias_part);
     return hipGetLastError();
 }
 
@@ -1111,7 +1164,7 @@ struct PullPlan {
     int segs, wgs, image_tiles, tiles;
 };
 
-PullPlan pull_plan(int64_t batch, int64_t H, int64_t W, int64_t channels, int slabs)
+PullPlan pull_plan(int64_t batch, int64_t rows, int64_t W, int64_t channels, int slabs)
 {
     PullPlan p;
     const int nb = (int)((channels + 15) / 16);
@@ -1122,7 +1175,7 @@ PullPlan pull_plan(int64_t batch, int64_t H, int64_t W, int64_t channels, int sl
     c.large = nb - c.n * (c.blocks - 1);
     p.segs = (int)((W + kSegment - 1) / kSegment);
     const int per_tile = kWaves / slabs;
-    p.image_tiles = (int)((H * p.segs + per_tile - 1) / per_tile);
+    p.image_tiles = (int)((rows * p.segs + per_tile - 1) / per_tile);
     p.tiles = (int)batch * p.image_tiles;
     auto share = [&](int blocks) {
         return (int)std::min<int64_t>(p.tiles, std::max(kXcds, 256 * blocks / nb / kXcds * kXcds));
@@ -1141,29 +1194,32 @@ int64_t pull_floats(const PullPlan &p, int slabs)
 }  // namespace
 }  // namespace group2d
 
-int64_t group_pull_floats_2d(int64_t batch, int64_t H, int64_t W, int64_t channels)
+int64_t group_pull_floats(int64_t batch, int64_t rows, int64_t W, int64_t channels)
 {
     using namespace group2d;
-    return std::max(pull_floats(pull_plan(batch, H, W, channels, 1), 1), pull_floats(pull_plan(batch, H, W, channels, 2), 2));
+    return std::max(pull_floats(pull_plan(batch, rows, W, channels, 1), 1), pull_floats(pull_plan(batch, rows, W, channels, 2), 2));
 }
 
-bool group_pull_supported_2d(const Geom &g, const View<const float> &x, const View<float> &gx)
+bool group_pull_supported(const Geom &g, const View<const float> &x, const View<float> &gx)
 {
-    return g.ndim == 2 && x.sx == 1 && gx.sx == 1 && x.sb == gx.sb && x.sc == gx.sc && x.sy == gx.sy && g.W >= group2d::kSegment &&
-           x.sc < ((int64_t)1 << 26) && (int64_t)(g.H - 1) * x.sy + g.W < ((int64_t)1 << 26) &&
-           (int64_t)g.B * g.H * ((g.W + group2d::kSegment - 1) / group2d::kSegment) < ((int64_t)1 << 30);
+    const int64_t plane = (int64_t)(g.D - 1) * x.sz + (int64_t)(g.H - 1) * x.sy + g.W;
+    return x.sx == 1 && gx.sx == 1 && x.sb == gx.sb && x.sc == gx.sc && (g.ndim == 2 || x.sz == gx.sz) && x.sy == gx.sy &&
+           g.W >= group2d::kSegment && x.sc < ((int64_t)1 << 26) && (g.ndim == 2 || x.sz < ((int64_t)1 << 26)) &&
+           x.sy < ((int64_t)1 << 26) && plane < ((int64_t)1 << 26) &&
+           (int64_t)g.B * g.D * g.H * ((g.W + group2d::kSegment - 1) / group2d::kSegment) < ((int64_t)1 << 30);
 }
 
-hipError_t group_pull_2d(const Geom &g, const View<const float> &x, const group2d::Outputs &out, int update, int mask_from,
-                         const View<float> &grads, int first, const int *channels, float *const *gk, float *gb,
-                         float *ws, bool reverse, hipStream_t s)
+hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::Outputs &out, int update, int mask_from,
+                      const View<float> &grads, int first, const int *channels, float *const *gk, float *gb,
+                      float *ws, bool reverse, hipStream_t s)
 {
     using namespace group2d;
-    if (out.n < 1 || out.n > kMaxOut || !group_pull_supported_2d(g, x, grads)) return hipErrorInvalidValue;
-    const int slabs = out.n > kSlabOut ? 2 : 1;
-    const PullPlan p = pull_plan(g.B, g.H, g.W, g.C, slabs);
-    PullArgs a{g.C, update, mask_from, g.H, g.W, p.segs, g.H * p.segs, p.tiles, p.image_tiles, Divisor((uint32_t)p.segs),
-               Divisor((uint32_t)p.image_tiles), reverse, 0, p.chunks, x.sb, x.sc, x.sy, out};
+    const int per_slab = g.ndim == 3 ? kSlabOut3d : kSlabOut, rows = g.D * g.H;
+    if (out.n < 1 || out.n > 2 * per_slab || !group_pull_supported(g, x, grads)) return hipErrorInvalidValue;
+    const int slabs = out.n > per_slab ? 2 : 1;
+    const PullPlan p = pull_plan(g.B, rows, g.W, g.C, slabs);
+    PullArgs a{g.C, update, mask_from, g.D, g.H, g.W, p.segs, rows * p.segs, p.tiles, p.image_tiles, Divisor((uint32_t)p.segs),
+               Divisor((uint32_t)p.image_tiles), Divisor((uint32_t)g.H), reverse, 0, p.chunks, x.sb, x.sc, x.sz, x.sy, out};
     SumArgs sum;
     for (int o = 0; o < kMaxOut; o++) {
         if (o < out.n) a.dmax = std::max(a.dmax, out.dil[o]);
@@ -1175,12 +1231,17 @@ hipError_t group_pull_2d(const Geom &g, const View<const float> &x, const group2
     hipError_t e = hipErrorInvalidConfiguration;
     // waves to a block: 4, 2 or 1
     const int share = p.chunks.blocks <= 2 ? 4 : p.chunks.blocks <= 4 ? 2 : 1;
-    switch (slabs * 10 + share) {
-    case 14: e = pull_launch<1, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 12: e = pull_launch<1, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 24: e = pull_launch<2, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 22: e = pull_launch<2, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 21: e = pull_launch<2, 1>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    switch (g.ndim * 100 + slabs * 10 + share) {
+    case 214: e = pull_launch<2, 1, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 212: e = pull_launch<2, 1, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 224: e = pull_launch<2, 2, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 222: e = pull_launch<2, 2, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 221: e = pull_launch<2, 2, 1>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 314: e = pull_launch<3, 1, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 312: e = pull_launch<3, 1, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 324: e = pull_launch<3, 2, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 322: e = pull_launch<3, 2, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    case 321: e = pull_launch<3, 2, 1>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
     }
     if (e != hipSuccess) return e;
     sum.chunks = p.chunks;
@@ -1189,35 +1250,43 @@ hipError_t group_pull_2d(const Geom &g, const View<const float> &x, const group2
     sum.stride = p.chunks.blocks * 1024 * slabs;
     sum.n = out.n;
     sum.gb = gb;
-    hipLaunchKernelGGL(sum_group, dim3(sum.columns / kWave + 1), dim3(1024), 0, s, sum, ws, bias_part);
+    hipLaunchKernelGGL(g.ndim == 3 ? sum_group<3> : sum_group<2>, dim3(sum.columns / kWave + 1), dim3(1024), 0, s, sum, ws, bias_part);
     return hipGetLastError();
 }
 
-hipError_t group_finish_back_2d(const Geom &g, const View<const float> &x, const View<float> &grads, int channel, int width,
-                                const group2d::Outputs &above, hipStream_t s)
+hipError_t group_finish_back(const Geom &g, const View<const float> &x, const View<float> &grads, int channel, int width,
+                             const group2d::Outputs &above, hipStream_t s)
 {
     using namespace group2d;
     const FinishArgs a = finish_args(g, x, above);
     const float *const act = x.p + (int64_t)channel * x.sc;
     float *const gp = grads.p + (int64_t)channel * grads.sc;
-    if (width == 1) {
+    if (g.ndim == 3) {
+        switch (width * 10 + above.n) {
+        case 11: return finish_back_launch<3, 1, 1>(a, act, gp, s);
+        case 12: return finish_back_launch<3, 2, 1>(a, act, gp, s);
+        case 13: return finish_back_launch<3, 3, 1>(a, act, gp, s);
+        case 21: return finish_back_launch<3, 1, 2>(a, act, gp, s);
+        case 22: return finish_back_launch<3, 2, 2>(a, act, gp, s);
+        }
+    } else if (width == 1) {
         switch (above.n) {
-        case 1: return finish_back_launch<1, 1>(a, act, gp, s);
-        case 2: return finish_back_launch<2, 1>(a, act, gp, s);
-        case 3: return finish_back_launch<3, 1>(a, act, gp, s);
-        case 4: return finish_back_launch<4, 1>(a, act, gp, s);
-        case 5: return finish_back_launch<5, 1>(a, act, gp, s);
-        case 6: return finish_back_launch<6, 1>(a, act, gp, s);
-        case 7: return finish_back_launch<7, 1>(a, act, gp, s);
+        case 1: return finish_back_launch<2, 1, 1>(a, act, gp, s);
+        case 2: return finish_back_launch<2, 2, 1>(a, act, gp, s);
+        case 3: return finish_back_launch<2, 3, 1>(a, act, gp, s);
+        case 4: return finish_back_launch<2, 4, 1>(a, act, gp, s);
+        case 5: return finish_back_launch<2, 5, 1>(a, act, gp, s);
+        case 6: return finish_back_launch<2, 6, 1>(a, act, gp, s);
+        case 7: return finish_back_launch<2, 7, 1>(a, act, gp, s);
         }
     } else if (width == 2) {
         switch (above.n) {
-        case 1: return finish_back_launch<1, 2>(a, act, gp, s);
-        case 2: return finish_back_launch<2, 2>(a, act, gp, s);
-        case 3: return finish_back_launch<3, 2>(a, act, gp, s);
-        case 4: return finish_back_launch<4, 2>(a, act, gp, s);
-        case 5: return finish_back_launch<5, 2>(a, act, gp, s);
-        case 6: return finish_back_launch<6, 2>(a, act, gp, s);
+        case 1: return finish_back_launch<2, 1, 2>(a, act, gp, s);
+        case 2: return finish_back_launch<2, 2, 2>(a, act, gp, s);
+        case 3: return finish_back_launch<2, 3, 2>(a, act, gp, s);
+        case 4: return finish_back_launch<2, 4, 2>(a, act, gp, s);
+        case 5: return finish_back_launch<2, 5, 2>(a, act, gp, s);
+        case 6: return finish_back_launch<2, 6, 2>(a, act, gp, s);
         }
     }
     return hipErrorInvalidConfiguration;

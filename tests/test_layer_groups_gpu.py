@@ -92,6 +92,35 @@ def test_block_backward_in_groups_of_up_to_fourteen(case):
         check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=59)
 
 
+# Volumes: groups of up to four outputs, the same tiles over the rows of all slices.  Slices and rows
+# whose outer taps lie outside on both sides, dilations up to the volume, tiles that end inside a volume and between
+# two, every remainder modulo four, groups of 2, 3 and 4 outputs and a layer left over, two channels per layer, blocks
+# shared by four, two and one waves, two chunks.
+VOLUMES = [
+    ((5, 6, 33), 1, 1, 5, 2, [1, 5, 3]),
+    ((9, 5, 32), 2, 1, 4, 1, [5, 2, 1]),
+    ((3, 11, 67), 9, 1, 7, 2, [3, 1, 2]),
+    ((12, 13, 38), 14, 1, 6, 1, [1, 12, 7]),
+    ((4, 4, 101), 30, 1, 4, 3, [4, 1]),
+    ((6, 3, 64), 52, 1, 9, 1, [3, 2, 1]),
+    ((2, 5, 45), 100, 1, 4, 1, [2, 1]),
+    ((3, 2, 35), 125, 1, 3, 2, [1, 2]),
+    ((24, 30, 75), 1, 1, 9, 1, None),
+    ((5, 7, 33), 1, 2, 2, 2, [5, 1]),
+    ((4, 6, 130), 15, 2, 5, 1, [3, 1, 4]),
+    ((25, 23, 65), 2, 2, 4, 1, [10, 9, 1]),
+]
+
+
+@pytest.mark.parametrize("case", VOLUMES, ids=lambda c: "x".join(map(str, c[0])) + "-c%d-w%d-d%d-B%d" % c[1:5])
+@pytest.mark.parametrize("input_grad", [True, False])
+def test_block_backward_of_volumes_in_groups(case, input_grad):
+    size, c_in, width, depth, batch, dilations = case
+    dilations = [(dilations or range(1, 11))[i % len(dilations or range(1, 11))] for i in range(depth)]
+    with tuning({"bwd.group": 1}):
+        check_block(3, size, c_in, width, depth, batch, dilations=dilations, seed=67, input_grad=input_grad)
+
+
 # What is no sum of three bf16 values takes the fp32 instruction: the same infinities and NaNs as from the
 # layers' own kernels, and the largest finite values (which round to an infinity in bf16) stay finite.
 @pytest.mark.parametrize("where", ["stack", "gradient", "weight"])
