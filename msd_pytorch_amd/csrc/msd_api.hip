@@ -1425,13 +1425,15 @@ constexpr int64_t kGroupChannels = 12, kGroupChannelsWide = 6;
 constexpr int64_t kFourteenVoxels = (int64_t)1 << 28, kFourteenVoxelsWide = (int64_t)1 << 27;
 
 // Number of layers from layer i on that form a group of the forward pass (0: none), of at most `most` outputs.
-// Knob: n > 0 from n channels on, in sevens; n < -1 from -n channels on, in fourteens.
+// Knob: 0 < n < kFourteenKnob from n channels on, in sevens; from kFourteenKnob on: from n - kFourteenKnob channels on, in fourteens.
+constexpr int kFourteenKnob = 1024;
 int forward_group(const BlockArgs &a, int i, int64_t first, int most)
 {
-    const int from = msd::knob(msd::kKnobFwdGroup, -1);
-    if (a.dtype != MSD_F32 || a.ndim != 2 || g_kernel_path != 0 || from == 0) return 0;
+    const int set = msd::knob(msd::kKnobFwdGroup, -1), from = set % kFourteenKnob;
+    const bool force = set >= kFourteenKnob;
+    if (a.dtype != MSD_F32 || a.ndim != 2 || g_kernel_path != 0 || set == 0) return 0;
     const bool wide = a.widths[i] > 1;
-    if (first < (from > 0 ? from : from < -1 ? -from : wide ? kGroupChannelsWide : kGroupChannels)) return 0;
+    if (first < (set > 0 ? from : wide ? kGroupChannelsWide : kGroupChannels)) return 0;
     int n = 0;
     int64_t outputs = 0, dmax = 0;
     while (i + n < a.depth && a.widths[i + n] <= 2 && outputs + a.widths[i + n] <= most) {
@@ -1441,7 +1443,7 @@ int forward_group(const BlockArgs &a, int i, int64_t first, int most)
     }
     if (outputs > msd::group2d::kSlabOut) {
         const bool large = a.batch * a.spatial[0] * a.spatial[1] >= ((wide ? kFourteenVoxelsWide : kFourteenVoxels) + first - 1) / first;
-        if (from > 0 || (from == -1 && !large) || !msd::group_split_supported_2d(a.spatial[1], (int)dmax)) return 0;
+        if (!(set < 0 ? large : force) || !msd::group_split_supported_2d(a.spatial[1], (int)dmax)) return 0;
     }
     return n >= 2 ? n : 0;
 }
