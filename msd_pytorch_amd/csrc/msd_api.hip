@@ -1019,7 +1019,7 @@ int block_group_fused(const char *fn, const BlockArgs &a, int i, int n, int64_t 
 
 // ---------------------------------------------------------------------------
 // 3D blocks of one-channel layers: the reverse loop as two streams of work, where the groups of
-// msd_pull.hip do not apply (rows of fewer than 32 voxels, channels 2^26 values apart, no room).
+// msd_pull.hip do not apply (channels 2^26 values apart, gaps between rows of fewer than 32 voxels, no room).
 //
 // Only the input gradient makes the reverse loop a chain (layer i's masked output gradient
 // is complete once every layer above has added its share to that channel); the weight and
@@ -1266,9 +1266,9 @@ int block_backward_split3d(const char *fn, const BlockArgs &a, int64_t c_in, con
 // 1024 x 1024 a pass and the upper half's share of the lower (49 us) are as fast as two groups of seven over
 // 20 channels (266 us both), 332 against 371 us over 48, 552 against 860 over 95.
 // Volumes: up to four outputs (two slabs of 54 of 64 rows), at every size; backward pass of the whole block, us, one layer
-// at a time or the two streams of block_backward_split3d, and groups: 16 x 16 x 32, depth 10: 207, 110; 61 x 93 x 75, depth 20: 891, 622
-// (groups of two outputs 684); 96 x 101 x 160, depth 30: 3268, 2152; 127^3, depth 50: 9761, 5337 (6396); 128^3: 6846, 5350 (5904);
-// 192^3, depth 10: 3209, 2564; two channels per layer, 128^3, depth 25: 7393, 4936.
+// at a time or the two streams of block_backward_split3d, and groups: 16 x 16 x 32, depth 10: 207, 110; 61 x 93 x 75, depth 20: 891, 499;
+// 40 x 45 x 47, depth 30: 549, 354; 128^3, depth 50: 6846, 5290 (groups of two outputs 5904); 192^3, depth 10: 3209, 2564; two
+// channels per layer, 128^3, depth 25: 7393, 4890.
 constexpr int64_t kGroupBackChannels = 1;
 
 // Number of layers from layer i down that form a group of the backward pass (0: none); `first` is

@@ -25,9 +25,10 @@
 // channels per layer, depth 200: 275 -> 194.
 //
 // Volumes (N = 3): two outputs of 27 taps in a slab's 64 rows, up to four in a group, the same tiles over the rows of all
-// slices.  128^3 over 1 to 46 channels: 338 us on average for four layers, and 140 for completing their own
-// channels, where the two streams of one and two layers per pass took 1060; 61 x 93 x 75: 79 and 33 (336).  Bound as above; every
-// tile lies at an edge there (27 values folded along three axes instead of 63 along two).
+// slices or over a volume as one row.  128^3 over 1 to 46 channels: 335 us on average for four layers, and 80 for completing
+// their own channels, where the two streams of one and two layers per pass took 530; 61 x 93 x 75: 60 and 27
+// (168 one layer per pass).  Bound as above; every tile is taken to lie at an edge there (27 values folded along three axes
+// instead of 63 along two).
 //
 // Tried on the way: waves that walk the channels on their own tile (weights in LDS, loads in the matrix layout): 650 us
 // over 95 channels, 320 over 45; two workgroups of four waves per compute unit: 604 and 293; for 5 to 8 blocks
@@ -56,11 +57,15 @@ constexpr int unit_bytes(int voxels) { return 3 * 16 * (2 * voxels + 16); }
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
 
+// What the kernels run over.  kFlat: a volume whose voxels lie without gaps, as one row: segments cross the
+// ends of the rows, every lane has a row of its own.
+enum Form { kImage = 2, kVolume = 3, kFlat = 4 };
 template <int N> struct Gather {
-    static constexpr int kTaps = N == 3 ? 27 : group2d::kTaps;
+    static constexpr bool kIsVolume = N != kImage;
+    static constexpr int kTaps = kIsVolume ? 27 : group2d::kTaps;
     static constexpr int kLines = kTaps / 3;             // taps along x apart
-    static constexpr int kOutputs = N == 3 ? kSlabOut3d : kSlabOut;        // of a slab
-    static constexpr int kLaneOut = N == 3 ? 1 : 4;      // that a lane holds
+    static constexpr int kOutputs = kIsVolume ? kSlabOut3d : kSlabOut;     // of a slab
+    static constexpr int kLaneOut = kIsVolume ? 1 : 4;   // that a lane holds
 };
 
 // Row m of a slab's 64: the halves of 32 belong to the lanes h = 0 and 1 of the gather.  A lane holds
@@ -71,7 +76,7 @@ struct Slot {
 };
 template <int N> __host__ __device__ __forceinline__ Slot slot_of(int m)
 {
-    if (N == 3) return Slot{m / 32, m % 32 < 27 ? m % 32 : -1};
+    if (N != kImage) return Slot{m / 32, m % 32 < 27 ? m % 32 : -1};
     const int h = m / 32 % 2, s = m % 32, first = m / kRows * kSlabOut;
     if (s < 27) return Slot{first + 3 * h + s / kTaps, s % kTaps};
     const int tap = 5 * h + s - 27;
@@ -108,9 +113,9 @@ struct Divisor {
 struct PullArgs {
     int C, update;                                // channels of x; the first `update` of them have grad_input
     int mask_from;                                // channels from here on are masked with their activation
-    int D, H, W, segs, items;                     // items: segments of an image
+    int D, H, W, span, segs, items;               // voxels of a row of segments (kFlat: of all); segments of one, of an image
     int tiles, image_tiles;                       // of all images, of one
-    Divisor by_segs, by_tiles, by_rows;           // by_rows: rows of a slice (3D)
+    Divisor by_segs, by_tiles, by_rows, by_voxels;        // by_rows: rows of a slice; by_voxels: of a row
     int reverse;                                  // walk the tiles from the last to the first
     int dmax;
     Chunks chunks;
@@ -243,14 +248,14 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         const int it = min(t.first + segment, a.items - 1);
         p.y = a.by_segs.of(it);
         const int own0 = (it - p.y * a.segs) * kSegment;
-        p.z = N == 3 ? a.by_rows.of(p.y) : 0;
-        p.y -= N == 3 ? p.z * a.H : 0;
-        p.x0 = min(own0, a.W - kSegment);         // (the last segment of a row overlaps the one before)
+        p.z = N == kVolume ? a.by_rows.of(p.y) : 0;
+        p.y -= N == kVolume ? p.z * a.H : 0;
+        p.x0 = min(own0, a.span - kSegment);         // (the last segment of a row overlaps the one before)
         p.skip = p.valid ? own0 - p.x0 : kSegment;
         return p;
     };
     const uint32_t plane = (uint32_t)a.sc * 4u;
-    auto row_at = [&](int z, int y) { return (N == 3 ? z * (int)a.sz : 0) + y * (int)a.sy; };
+    auto row_at = [&](int z, int y) { return (Gather<N>::kIsVolume ? z * (int)a.sz : 0) + y * (int)a.sy; };
 
     // The tiles: kSegs consecutive segments of an image each; every workgroup of an XCD works on neighbouring ones.
     const int lb = block_for_xcd(wg, wgs, wgs % kXcds == 0);
@@ -299,20 +304,34 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
     const int segment = wave / G, slab = wave % G;
     const int v = lane % kSegment, h = lane / kSegment;
     const uint32_t bias = 4u * (uint32_t)row_at(a.dmax, a.dmax);
-    auto output_of = [&](int j) { return N == 3 ? h : j < 3 ? 3 * h + j : 6; };
+    auto output_of = [&](int j) { return Gather<N>::kIsVolume ? h : j < 3 ? 3 * h + j : 6; };
     auto source = [&](int j) {
         int o = output_of(j);
         asm volatile("" : "+v"(o));
         return shared.sources[slab * kSlabOut + o];
     };
+    // the lane's voxel (kImage, kVolume: y and z are uniform)
+    struct Voxel {
+        int x, y, z;
+    };
+    auto voxel_of = [&](const Place &p) {
+        Voxel vx{p.x0 + v, p.y, p.z};
+        if constexpr (N == kFlat) {
+            const int row = a.by_voxels.of(vx.x);
+            vx.x -= row * a.W;
+            vx.z = a.by_rows.of(row);
+            vx.y = row - vx.z * a.H;
+        }
+        return vx;
+    };
     auto away = [&](const Place &p) {             // uniform: from all edges
-        return p.x0 >= a.dmax && p.x0 + kSegment + a.dmax <= a.W && p.y >= a.dmax && p.y + a.dmax < a.H &&
-               (N == 2 || (p.z >= a.dmax && p.z + a.dmax < a.D));
+        return N != kFlat && p.x0 >= a.dmax && p.x0 + kSegment + a.dmax <= a.W && p.y >= a.dmax && p.y + a.dmax < a.H &&
+               (N == kImage || (p.z >= a.dmax && p.z + a.dmax < a.D));
     };
     float val[kLaneOut][kLines][3];
     auto gather = [&](const Tile &t, const Place &p) {
-        const uint32_t u = (uint32_t)(p.x0 + v);
         if (away(p)) {
+            const uint32_t u = (uint32_t)(p.x0 + v);
             const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)(t.img + (int64_t)row_at(p.z, p.y) * 4) - bias;
 #pragma unroll
             for (int j = 0; j < kLaneOut; j++) {
@@ -320,7 +339,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                 const uint32_t c = o.plane + bias + 4u * u;
 #pragma unroll
                 for (int l = 0; l < kLines; l++) {
-                    const uint32_t s = N == 2 || l / 3 == 1 ? c : l / 3 == 0 ? c + o.slices : c - o.slices;
+                    const uint32_t s = N == kImage || l / 3 == 1 ? c : l / 3 == 0 ? c + o.slices : c - o.slices;
                     const uint32_t r = l % 3 == 0 ? s + o.rows : l % 3 == 1 ? s : s - o.rows;
                     val[j][l][0] = load1(base, r + o.voxels);
                     val[j][l][1] = load1(base, r);
@@ -330,18 +349,19 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             }
         } else {
             const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)t.img;
+            const Voxel vx = voxel_of(p);
 #pragma unroll
             for (int j = 0; j < kLaneOut; j++) {
                 const Source o = source(j);
                 const int d = (int)(o.voxels / 4u);
-                const Sides sx = sides((int)u, a.W, d), sy = sides(p.y, a.H, d), sz = sides(p.z, N == 3 ? a.D : 1, N == 3 ? d : 0);
+                const Sides sx = sides(vx.x, a.W, d), sy = sides(vx.y, a.H, d), sz = sides(vx.z, N == kImage ? 1 : a.D, N == kImage ? 0 : d);
 #pragma unroll
                 for (int l = 0; l < kLines; l++) {
-                    const int y = l % 3 == 0 ? sy.up : l % 3 == 1 ? p.y : sy.down;
-                    const int z = N == 2 || l / 3 == 1 ? p.z : l / 3 == 0 ? sz.up : sz.down;
+                    const int y = l % 3 == 0 ? sy.up : l % 3 == 1 ? vx.y : sy.down;
+                    const int z = N == kImage || l / 3 == 1 ? vx.z : l / 3 == 0 ? sz.up : sz.down;
                     const uint32_t r = o.plane + 4u * (uint32_t)row_at(z, y);
                     val[j][l][0] = load1(base, r + 4u * (uint32_t)sx.up);
-                    val[j][l][1] = load1(base, r + 4u * u);
+                    val[j][l][1] = load1(base, r + 4u * (uint32_t)vx.x);
                     val[j][l][2] = load1(base, r + 4u * (uint32_t)sx.down);
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -350,17 +370,18 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
     };
     auto gathered = [&](const Place &p, bool count) {
         if (!away(p)) {
+            const Voxel vx = voxel_of(p);
 #pragma unroll
             for (int j = 0; j < kLaneOut; j++) {
                 const int d = (int)(source(j).voxels / 4u);
-                const Sides sx = sides(p.x0 + v, a.W, d), sy = sides(p.y, a.H, d), sz = sides(p.z, N == 3 ? a.D : 1, N == 3 ? d : 0);
+                const Sides sx = sides(vx.x, a.W, d), sy = sides(vx.y, a.H, d), sz = sides(vx.z, N == kImage ? 1 : a.D, N == kImage ? 0 : d);
 #pragma unroll
                 for (int l = 0; l < kLines; l++) fold(sx, val[j][l][0], val[j][l][2]);
 #pragma unroll
                 for (int l = 0; l < kLines; l += 3)
 #pragma unroll
                     for (int r = 0; r < 3; r++) fold(sy, val[j][l][r], val[j][l + 2][r]);
-                if constexpr (N == 3) {
+                if constexpr (N != kImage) {
 #pragma unroll
                     for (int l = 0; l < 3; l++)
 #pragma unroll
@@ -378,7 +399,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             }
         }
         if (count) {
-            if constexpr (N == 3) shared.bias_sums[tid][0] += val[0][4][1];
+            if constexpr (N != kImage) shared.bias_sums[tid][0] += val[0][4][1];
             else shared.bias_sums[tid] += f32x4_t{val[0][1][1], val[1][1][1], val[2][1][1], val[3][1][1]};
         }
         // -A at every second voxel: the sums of the bf16 instruction are cut off towards minus infinity, which adds up
@@ -397,7 +418,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                 const int s = 8 * i + e;
                 if (s < 27) {
                     e8[e] = val[s / kTaps][s % kTaps / 3][s % 3];
-                } else if constexpr (N == 3) {
+                } else if constexpr (N != kImage) {
                     e8[e] = 0.f;
                 } else {
                     const int t0 = s - 27, t1 = s - 22;
@@ -809,7 +830,7 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
     if (tid == 0) shared.bad_again = 0;
     if (tid < G * kSlabOut) {
         const int o = min(tid, a.out.n - 1), d = a.out.dil[o];
-        shared.sources[tid] = Source{N == 3 ? 4u * (uint32_t)(d * (int)a.sz) : 0u, 4u * (uint32_t)(d * (int)a.sy), 4u * (uint32_t)d, (uint32_t)o * ((uint32_t)a.sc * 4u)};
+        shared.sources[tid] = Source{N == kVolume ? 4u * (uint32_t)(d * (int)a.sz) : 0u, 4u * (uint32_t)(d * (int)a.sy), 4u * (uint32_t)d, (uint32_t)o * ((uint32_t)a.sc * 4u)};
     }
     state.weights_split = true;
 #pragma unroll
@@ -882,7 +903,7 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
     if (v == 0) {
 #pragma unroll
         for (int j = 0; j < kLaneOut; j++)
-            if (N == 3 || j < 3 || h == 0) red[wave * kBiasColumns + (N == 3 ? h : j < 3 ? 3 * h + j : 6)] = bias_sum[j];
+            if (N != kImage || j < 3 || h == 0) red[wave * kBiasColumns + (N != kImage ? h : j < 3 ? 3 * h + j : 6)] = bias_sum[j];
     }
     __syncthreads();
     if (tid < G * kBiasColumns && tid % kBiasColumns < kSlabOut) {
@@ -966,7 +987,8 @@ __global__ __launch_bounds__(1024) void sum_group(const SumArgs a, const float *
 // were written or read by the launches before), with no LDS and no barrier: the launches are bound by
 // their ramp and by the vector cache.
 struct FinishArgs {
-    int D, H, W, segs, items, dmax;
+    int D, H, W, span, segs, items, dmax;         // (as in PullArgs, segments of 64)
+    Divisor by_rows, by_voxels;
     int n, channels, masked;                      // spread_back: outputs above, channels, first one to mask
     int64_t sb, sc, sz, sy;
     int dil[kMaxAbove];
@@ -984,16 +1006,26 @@ template <int N> __device__ __forceinline__ FinishPlace finish_place(const Finis
 {
     FinishPlace p;
     const int row = it / a.segs, xw = (it - row * a.segs) * kWave;
-    const int slice = row / a.H, b = N == 3 ? slice / a.D : slice;
-    p.y = row - slice * a.H;
-    p.z = slice - b * (N == 3 ? a.D : 1);
-    const int u0 = xw + threadIdx.x % kWave;
-    p.u = min(u0, a.W - 1);
-    p.own = u0 < a.W;
-    p.away = xw >= a.dmax && xw + kWave + a.dmax <= a.W && p.y >= a.dmax && p.y + a.dmax < a.H &&
-             (N == 2 || (p.z >= a.dmax && p.z + a.dmax < a.D));
-    p.img = (int64_t)b * a.sb * 4;
-    p.here = 4u * (uint32_t)((N == 3 ? p.z * (int)a.sz : 0) + p.y * (int)a.sy + p.u);
+    const int u0 = xw + threadIdx.x % kWave, at = min(u0, a.span - 1);
+    p.own = u0 < a.span;
+    if constexpr (N == kFlat) {                   // (a row is a volume)
+        const int line = a.by_voxels.of(at);
+        p.u = at - line * a.W;
+        p.z = a.by_rows.of(line);
+        p.y = line - p.z * a.H;
+        p.away = false;
+        p.img = (int64_t)row * a.sb * 4;
+        p.here = 4u * (uint32_t)at;
+    } else {
+        const int slice = row / a.H, b = N == kVolume ? slice / a.D : slice;
+        p.u = at;
+        p.y = row - slice * a.H;
+        p.z = slice - b * (N == kVolume ? a.D : 1);
+        p.away = xw >= a.dmax && xw + kWave + a.dmax <= a.W && p.y >= a.dmax && p.y + a.dmax < a.H &&
+                 (N == kImage || (p.z >= a.dmax && p.z + a.dmax < a.D));
+        p.img = (int64_t)b * a.sb * 4;
+        p.here = 4u * (uint32_t)((N == kVolume ? p.z * (int)a.sz : 0) + p.y * (int)a.sy + p.u);
+    }
     return p;
 }
 template <int N>
@@ -1004,13 +1036,22 @@ __device__ __forceinline__ void finish_gather(const FinishArgs &a, const FinishP
     if (!p.away) {
         sx = sides(p.u, a.W, d);
         sy = sides(p.y, a.H, d);
-        if (N == 3) sz = sides(p.z, a.D, d);
+        if (N != kImage) sz = sides(p.z, a.D, d);
     }
 #pragma unroll
     for (int l = 0; l < Gather<N>::kLines; l++) {
         const int y = l % 3 == 0 ? sy.up : l % 3 == 1 ? p.y : sy.down;
         const int z = l / 3 == 0 ? sz.up : l / 3 == 1 ? p.z : sz.down;
-        const uint64_t base = output + (uint64_t)(4 * ((N == 3 ? (int64_t)z * a.sz : 0) + (int64_t)y * a.sy));
+        // (kFlat: an offset of the lane's, else a uniform base)
+        const int64_t line = 4 * ((N != kImage ? (int64_t)z * a.sz : 0) + (int64_t)y * a.sy);
+        if constexpr (N == kFlat) {
+            const uint32_t at = (uint32_t)line;
+            A[l][0] = load1(output, at + 4u * (uint32_t)sx.up);
+            A[l][1] = load1(output, at + 4u * (uint32_t)p.u);
+            A[l][2] = load1(output, at + 4u * (uint32_t)sx.down);
+            continue;
+        }
+        const uint64_t base = output + (uint64_t)line;
         A[l][0] = load1(base, 4u * (uint32_t)sx.up);
         A[l][1] = load1(base, 4u * (uint32_t)p.u);
         A[l][2] = load1(base, 4u * (uint32_t)sx.down);
@@ -1026,7 +1067,7 @@ __device__ __forceinline__ void finish_fold(const FinishArgs &a, const FinishPla
     for (int l = 0; l < Gather<N>::kLines; l += 3)
 #pragma unroll
         for (int r = 0; r < 3; r++) fold(sy, A[l][r], A[l + 2][r]);
-    if constexpr (N == 3) {
+    if constexpr (N != kImage) {
         const Sides sz = sides(p.z, a.D, d);
 #pragma unroll
         for (int l = 0; l < 3; l++)
@@ -1084,7 +1125,7 @@ __global__ __launch_bounds__(256) void spread_back(const FinishArgs a, const flo
     const int lb = block_for_xcd(blockIdx.x, gridDim.x, true);
     const int it = lb * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     if (it >= a.items) return;                    // uniform over the wave
-    const FinishPlace p = finish_place<2>(a, it);
+    const FinishPlace p = finish_place<kImage>(a, it);
     const uint64_t img = reinterpret_cast<uint64_t>(g) + (uint64_t)p.img;
     const uint64_t ximg = reinterpret_cast<uint64_t>(act) + (uint64_t)p.img;
     const uint32_t plane = (uint32_t)a.sc * 4u;
@@ -1096,9 +1137,9 @@ __global__ __launch_bounds__(256) void spread_back(const FinishArgs a, const flo
     // output by output, the next one's values requested before this one's products: few registers, so that the
     // waves of a SIMD hide each other's scalar loads of the weights
     float all[kMaxLower] = {}, A[2][3][3];
-    auto gather = [&](int o, float(&to)[3][3]) { finish_gather<2>(a, p, img + (uint64_t)(a.channels + o) * plane, a.dil[o], to); };
+    auto gather = [&](int o, float(&to)[3][3]) { finish_gather<kImage>(a, p, img + (uint64_t)(a.channels + o) * plane, a.dil[o], to); };
     auto add = [&](int o, float(&from)[3][3]) {
-        if (!p.away) finish_fold<2>(a, p, a.dil[o], from);
+        if (!p.away) finish_fold<kImage>(a, p, a.dil[o], from);
         const float *const k = a.k[o];
 #pragma unroll
         for (int c = 0; c < kMaxLower; c++) {
@@ -1127,6 +1168,15 @@ __global__ __launch_bounds__(256) void spread_back(const FinishArgs a, const flo
     }
 }
 
+// Wherever the voxels lie without gaps.  Backward pass of a block, us, as rows and as one row: 61 x 93 x 75, depth 20: 639, 499;
+// 80 x 81 x 65, depth 30: 1051, 732; 127^3, depth 30: 2784, 2732; and with whole segments (no fold is ever skipped, but the
+// lanes' rows cost no scalar work) 64^3, depth 30: 548, 529; 128^3: 2800, 2757.
+Form form_of(const Geom &g, const View<const float> &x)
+{
+    if (g.ndim == 2) return kImage;
+    return x.sy == g.W && x.sz == (int64_t)g.H * g.W ? kFlat : kVolume;
+}
+
 template <int N, int NQ, int NOUT>
 hipError_t finish_back_launch(const FinishArgs &a, const float *act, float *g, hipStream_t s)
 {
@@ -1136,8 +1186,9 @@ hipError_t finish_back_launch(const FinishArgs &a, const float *act, float *g, h
 
 FinishArgs finish_args(const Geom &g, const View<const float> &x, const group2d::Outputs &above)
 {
-    const int segs = (g.W + kWave - 1) / kWave;
-    FinishArgs a{g.D, g.H, g.W, segs, g.B * g.D * g.H * segs, 0, above.n, 0, 0, x.sb, x.sc, x.sz, x.sy, {}, {}};
+    const int span = form_of(g, x) == kFlat ? g.nvox : g.W, segs = (span + kWave - 1) / kWave;
+    FinishArgs a{g.D, g.H, g.W, span, segs, g.nvox / span * g.B * segs, 0, Divisor((uint32_t)g.H), Divisor((uint32_t)g.W),
+                 above.n, 0, 0, x.sb, x.sc, x.sz, x.sy, {}, {}};
     for (int o = 0; o < above.n; o++) {
         a.dil[o] = above.dil[o];
         a.k[o] = above.k[o];
@@ -1164,7 +1215,7 @@ struct PullPlan {
     int segs, wgs, image_tiles, tiles;
 };
 
-PullPlan pull_plan(int64_t batch, int64_t rows, int64_t W, int64_t channels, int slabs)
+PullPlan pull_plan(int64_t batch, int64_t rows, int64_t span, int64_t channels, int slabs)
 {
     PullPlan p;
     const int nb = (int)((channels + 15) / 16);
@@ -1173,7 +1224,7 @@ PullPlan pull_plan(int64_t batch, int64_t rows, int64_t W, int64_t channels, int
     c.n = (nb + most - 1) / most;
     c.blocks = (nb + c.n - 1) / c.n;
     c.large = nb - c.n * (c.blocks - 1);
-    p.segs = (int)((W + kSegment - 1) / kSegment);
+    p.segs = (int)((span + kSegment - 1) / kSegment);
     const int per_tile = kWaves / slabs;
     p.image_tiles = (int)((rows * p.segs + per_tile - 1) / per_tile);
     p.tiles = (int)batch * p.image_tiles;
@@ -1197,16 +1248,19 @@ int64_t pull_floats(const PullPlan &p, int slabs)
 int64_t group_pull_floats(int64_t batch, int64_t rows, int64_t W, int64_t channels)
 {
     using namespace group2d;
+    // (volumes without gaps have fewer segments, and so no more workgroups)
     return std::max(pull_floats(pull_plan(batch, rows, W, channels, 1), 1), pull_floats(pull_plan(batch, rows, W, channels, 2), 2));
 }
 
 bool group_pull_supported(const Geom &g, const View<const float> &x, const View<float> &gx)
 {
+    using namespace group2d;
     const int64_t plane = (int64_t)(g.D - 1) * x.sz + (int64_t)(g.H - 1) * x.sy + g.W;
+    const int span = form_of(g, x) == kFlat ? g.nvox : g.W;
     return x.sx == 1 && gx.sx == 1 && x.sb == gx.sb && x.sc == gx.sc && (g.ndim == 2 || x.sz == gx.sz) && x.sy == gx.sy &&
-           g.W >= group2d::kSegment && x.sc < ((int64_t)1 << 26) && (g.ndim == 2 || x.sz < ((int64_t)1 << 26)) &&
+           span >= kSegment && x.sc < ((int64_t)1 << 26) && (g.ndim == 2 || x.sz < ((int64_t)1 << 26)) &&
            x.sy < ((int64_t)1 << 26) && plane < ((int64_t)1 << 26) &&
-           (int64_t)g.B * g.D * g.H * ((g.W + group2d::kSegment - 1) / group2d::kSegment) < ((int64_t)1 << 30);
+           (int64_t)g.B * g.D * g.H * ((g.W + kSegment - 1) / kSegment) < ((int64_t)1 << 30);
 }
 
 hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::Outputs &out, int update, int mask_from,
@@ -1214,12 +1268,15 @@ hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::
                       float *ws, bool reverse, hipStream_t s)
 {
     using namespace group2d;
-    const int per_slab = g.ndim == 3 ? kSlabOut3d : kSlabOut, rows = g.D * g.H;
+    const int per_slab = g.ndim == 3 ? kSlabOut3d : kSlabOut;
     if (out.n < 1 || out.n > 2 * per_slab || !group_pull_supported(g, x, grads)) return hipErrorInvalidValue;
     const int slabs = out.n > per_slab ? 2 : 1;
-    const PullPlan p = pull_plan(g.B, rows, g.W, g.C, slabs);
-    PullArgs a{g.C, update, mask_from, g.D, g.H, g.W, p.segs, rows * p.segs, p.tiles, p.image_tiles, Divisor((uint32_t)p.segs),
-               Divisor((uint32_t)p.image_tiles), Divisor((uint32_t)g.H), reverse, 0, p.chunks, x.sb, x.sc, x.sz, x.sy, out};
+    const Form form = form_of(g, x);
+    const int span = form == kFlat ? g.nvox : g.W, rows = g.nvox / span;
+    const PullPlan p = pull_plan(g.B, rows, span, g.C, slabs);
+    PullArgs a{g.C, update, mask_from, g.D, g.H, g.W, span, p.segs, rows * p.segs, p.tiles, p.image_tiles, Divisor((uint32_t)p.segs),
+               Divisor((uint32_t)p.image_tiles), Divisor((uint32_t)g.H), Divisor((uint32_t)g.W), reverse, 0, p.chunks,
+               x.sb, x.sc, x.sz, x.sy, out};
     SumArgs sum;
     for (int o = 0; o < kMaxOut; o++) {
         if (o < out.n) a.dmax = std::max(a.dmax, out.dil[o]);
@@ -1231,17 +1288,21 @@ hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::
     hipError_t e = hipErrorInvalidConfiguration;
     // waves to a block: 4, 2 or 1
     const int share = p.chunks.blocks <= 2 ? 4 : p.chunks.blocks <= 4 ? 2 : 1;
-    switch (g.ndim * 100 + slabs * 10 + share) {
-    case 214: e = pull_launch<2, 1, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 212: e = pull_launch<2, 1, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 224: e = pull_launch<2, 2, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 222: e = pull_launch<2, 2, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 221: e = pull_launch<2, 2, 1>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 314: e = pull_launch<3, 1, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 312: e = pull_launch<3, 1, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 324: e = pull_launch<3, 2, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 322: e = pull_launch<3, 2, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
-    case 321: e = pull_launch<3, 2, 1>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s); break;
+    auto launch = [&](auto f) {
+        constexpr int N = decltype(f)::value;
+        switch (slabs * 10 + share) {
+        case 14: return pull_launch<N, 1, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
+        case 12: return pull_launch<N, 1, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
+        case 24: return pull_launch<N, 2, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
+        case 22: return pull_launch<N, 2, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
+        case 21: return pull_launch<N, 2, 1>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
+        }
+        return hipErrorInvalidConfiguration;
+    };
+    switch (form) {
+    case kImage: e = launch(std::integral_constant<int, kImage>{}); break;
+    case kVolume: e = launch(std::integral_constant<int, kVolume>{}); break;
+    case kFlat: e = launch(std::integral_constant<int, kFlat>{}); break;
     }
     if (e != hipSuccess) return e;
     sum.chunks = p.chunks;
@@ -1250,7 +1311,7 @@ hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::
     sum.stride = p.chunks.blocks * 1024 * slabs;
     sum.n = out.n;
     sum.gb = gb;
-    hipLaunchKernelGGL(g.ndim == 3 ? sum_group<3> : sum_group<2>, dim3(sum.columns / kWave + 1), dim3(1024), 0, s, sum, ws, bias_part);
+    hipLaunchKernelGGL(g.ndim == 3 ? sum_group<kVolume> : sum_group<kImage>, dim3(sum.columns / kWave + 1), dim3(1024), 0, s, sum, ws, bias_part);
     return hipGetLastError();
 }
 
@@ -1262,31 +1323,36 @@ hipError_t group_finish_back(const Geom &g, const View<const float> &x, const Vi
     const float *const act = x.p + (int64_t)channel * x.sc;
     float *const gp = grads.p + (int64_t)channel * grads.sc;
     if (g.ndim == 3) {
-        switch (width * 10 + above.n) {
-        case 11: return finish_back_launch<3, 1, 1>(a, act, gp, s);
-        case 12: return finish_back_launch<3, 2, 1>(a, act, gp, s);
-        case 13: return finish_back_launch<3, 3, 1>(a, act, gp, s);
-        case 21: return finish_back_launch<3, 1, 2>(a, act, gp, s);
-        case 22: return finish_back_launch<3, 2, 2>(a, act, gp, s);
-        }
+        auto launch = [&](auto form) {
+            constexpr int N = decltype(form)::value;
+            switch (width * 10 + above.n) {
+            case 11: return finish_back_launch<N, 1, 1>(a, act, gp, s);
+            case 12: return finish_back_launch<N, 2, 1>(a, act, gp, s);
+            case 13: return finish_back_launch<N, 3, 1>(a, act, gp, s);
+            case 21: return finish_back_launch<N, 1, 2>(a, act, gp, s);
+            case 22: return finish_back_launch<N, 2, 2>(a, act, gp, s);
+            }
+            return hipErrorInvalidConfiguration;
+        };
+        return form_of(g, x) == kFlat ? launch(std::integral_constant<int, kFlat>{}) : launch(std::integral_constant<int, kVolume>{});
     } else if (width == 1) {
         switch (above.n) {
-        case 1: return finish_back_launch<2, 1, 1>(a, act, gp, s);
-        case 2: return finish_back_launch<2, 2, 1>(a, act, gp, s);
-        case 3: return finish_back_launch<2, 3, 1>(a, act, gp, s);
-        case 4: return finish_back_launch<2, 4, 1>(a, act, gp, s);
-        case 5: return finish_back_launch<2, 5, 1>(a, act, gp, s);
-        case 6: return finish_back_launch<2, 6, 1>(a, act, gp, s);
-        case 7: return finish_back_launch<2, 7, 1>(a, act, gp, s);
+        case 1: return finish_back_launch<kImage, 1, 1>(a, act, gp, s);
+        case 2: return finish_back_launch<kImage, 2, 1>(a, act, gp, s);
+        case 3: return finish_back_launch<kImage, 3, 1>(a, act, gp, s);
+        case 4: return finish_back_launch<kImage, 4, 1>(a, act, gp, s);
+        case 5: return finish_back_launch<kImage, 5, 1>(a, act, gp, s);
+        case 6: return finish_back_launch<kImage, 6, 1>(a, act, gp, s);
+        case 7: return finish_back_launch<kImage, 7, 1>(a, act, gp, s);
         }
     } else if (width == 2) {
         switch (above.n) {
-        case 1: return finish_back_launch<2, 1, 2>(a, act, gp, s);
-        case 2: return finish_back_launch<2, 2, 2>(a, act, gp, s);
-        case 3: return finish_back_launch<2, 3, 2>(a, act, gp, s);
-        case 4: return finish_back_launch<2, 4, 2>(a, act, gp, s);
-        case 5: return finish_back_launch<2, 5, 2>(a, act, gp, s);
-        case 6: return finish_back_launch<2, 6, 2>(a, act, gp, s);
+        case 1: return finish_back_launch<kImage, 1, 2>(a, act, gp, s);
+        case 2: return finish_back_launch<kImage, 2, 2>(a, act, gp, s);
+        case 3: return finish_back_launch<kImage, 3, 2>(a, act, gp, s);
+        case 4: return finish_back_launch<kImage, 4, 2>(a, act, gp, s);
+        case 5: return finish_back_launch<kImage, 5, 2>(a, act, gp, s);
+        case 6: return finish_back_launch<kImage, 6, 2>(a, act, gp, s);
         }
     }
     return hipErrorInvalidConfiguration;

@@ -109,6 +109,9 @@ VOLUMES = [
     ((5, 7, 33), 1, 2, 2, 2, [5, 1]),
     ((4, 6, 130), 15, 2, 5, 1, [3, 1, 4]),
     ((25, 23, 65), 2, 2, 4, 1, [10, 9, 1]),
+    ((4, 3, 5), 2, 1, 4, 2, [3, 1]),
+    ((2, 4, 4), 17, 1, 3, 1, [2, 1]),
+    ((19, 9, 7), 3, 2, 3, 3, [7, 2]),
 ]
 
 
@@ -119,6 +122,33 @@ def test_block_backward_of_volumes_in_groups(case, input_grad):
     dilations = [(dilations or range(1, 11))[i % len(dilations or range(1, 11))] for i in range(depth)]
     with tuning({"bwd.group": 1}):
         check_block(3, size, c_in, width, depth, batch, dilations=dilations, seed=67, input_grad=input_grad)
+
+
+# A volume without gaps is taken as one row, any other by its rows (of 32 voxels at least): the same gradients from
+# rows with gaps, from slices with gaps and from slices and rows in the other order.
+@pytest.mark.parametrize("layout", ["rows", "slices", "transposed"])
+@pytest.mark.parametrize("c_in,width,depth", [(3, 1, 4), (33, 1, 3), (66, 1, 4), (5, 1, 2), (40, 1, 2), (2, 2, 2), (1, 2, 5), (3, 1, 5)])
+def test_volumes_in_other_layouts(c_in, width, depth, layout):
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator().manual_seed(71)
+    size, channels = (4, 5, 45), c_in + depth * width
+    stack, gradient = (torch.randn(2, channels, *size, generator=gen).cuda() for _ in range(2))
+    weights = [torch.randn(width, c_in + i * width, 3, 3, 3, generator=gen).cuda() * 0.1 for i in range(depth)]
+
+    def view(t):
+        d, h, w = size
+        big = {"rows": (d, h, w + 3), "slices": (d, h + 2, w), "transposed": (h, d, w)}[layout]
+        big = torch.full((2, channels, *big), float("nan"), device="cuda")
+        big = big.transpose(2, 3) if layout == "transposed" else big[..., :h, :w]
+        return big.copy_(t)
+
+    found = []
+    for s, g in ((stack, gradient.clone()), (view(stack), view(gradient))):
+        gk, gb = [torch.zeros_like(w) for w in weights], torch.zeros(depth * width).cuda()
+        cc.block_backward(s, g, c_in, [1 + i % 4 for i in range(depth)], weights, gk, gb, True)
+        found.append((g[:, :c_in], gb, *gk))
+    for a, b in zip(*found):
+        assert rel_err(b, a) <= 1e-5
 
 
 # What is no sum of three bf16 values takes the fp32 instruction: the same infinities and NaNs as from the
