@@ -91,8 +91,15 @@ __device__ __forceinline__ bool tile_origin(const Geom &g, const Lattice &lt, in
     return y0 < g.H && z0 < g.D;                 // false: empty tail of a residue class
 }
 
-template <int NDIM, bool RELU, int WOUT, int V, int RZ, int RY>
-__global__ __launch_bounds__(NDIM == 3 ? 512 : 1024, (NDIM == 3 && V == 1 && WOUT == 1) ? (RZ * RY > 9 ? 4 : 8) : 1) void fwd_lattice(Geom g, Lattice lt, int remap, View<const float> x,
+// Output rows of a tile of `rows` that are finished together.  3D with one voxel per lane: the rows of half a tile take at
+// most 30 KB, which costs no resident workgroup (61 x 93 x 75, depth 20: 364 -> 358 us; 40 x 45 x 47, depth 30, in four groups:
+// 366 -> 323).  2D: one at a time (256 x 256, depth 10: half tiles are 3 us slower).
+constexpr int finish_batch(int ndim, int V, int rows) { return ndim == 2 || V > 1 ? 1 : rows <= 10 ? (rows + 1) / 2 : 6; }
+
+// ONE (3D): all channels in one group.  A channel's nine products are summed before they are added: in one chain over
+// all channels the error would be a third larger than with two groups (as it is, it is a fifth smaller).
+template <int NDIM, bool RELU, int WOUT, int V, int RZ, int RY, bool ONE = false>
+__global__ __launch_bounds__(NDIM == 3 ? 512 : 1024, (NDIM == 3 && V == 1 && WOUT == 1) ? (RZ * RY > 9 ? 4 : ONE ? 7 : 8) : 1) void fwd_lattice(Geom g, Lattice lt, int remap, View<const float> x,
                                                     const float *__restrict__ k, const float *__restrict__ bias,
                                                     View<float> out)
 {
@@ -192,6 +199,16 @@ __global__ __launch_bounds__(NDIM == 3 ? 512 : 1024, (NDIM == 3 && V == 1 && WOU
 #pragma unroll
             for (int jy = 0; jy < RY; jy++) {
                 if (jy >= nyv) break;
+                if constexpr (ONE) {
+#pragma unroll
+                    for (int r = 0; r < 3; r++) {
+                        float one = xv[jz][jy][0] * w[0][r];
+#pragma unroll
+                        for (int t = 1; t < 9; t++) one += xv[jz + t / 3][jy + t % 3][0] * w[0][t * 3 + r];
+                        acc[0][jz][jy][r][0] += one;
+                    }
+                    continue;
+                }
 #pragma unroll
                 for (int p = 0; p < NZ; p++)
 #pragma unroll
@@ -209,49 +226,71 @@ __global__ __launch_bounds__(NDIM == 3 ? 512 : 1024, (NDIM == 3 && V == 1 && WOU
         }
     }
 
-    // Finish the rows one at a time.  LDS holds T_r of the current row for every
-    // channel group: T[kg][r][staged x]; group (row counter % KS) adds the groups
-    // up at the three shifted positions and writes the row.
+    // Finish the rows, `batch` at a time.  LDS holds T_r of these rows for every channel group, T[kg][row][r][staged x];
+    // the groups take turns in adding them up at the three shifted positions and writing the row.
+    constexpr int R = RZ * RY, batch = finish_batch(NDIM, V, R);
     const int rowlen = V * lt.lpr;
     float *T = lds;
+    // the row staged at t (and `group` floats on for each further group)
+    auto write_row = [&](int co, float bv, const float *t, int group, int z, int y) {
+        float o[V];
+#pragma unroll
+        for (int i = 0; i < V; i++) {
+            const int xx = x0 + i;
+            const int i0 = staged_index<V>(reflect_idx(xx - g.dil, g.W), lt.lpr);
+            const int i1 = i * lt.lpr + lane;
+            const int i2 = staged_index<V>(reflect_idx(xx + g.dil, g.W), lt.lpr);
+            float s = bv;
+            for (int kk = 0; kk < lt.ks; kk++) {
+                const float *tk = t + (size_t)kk * group;
+                s += tk[i0] + tk[rowlen + i1] + tk[2 * rowlen + i2];
+            }
+            o[i] = RELU ? (s > 0.f ? s : 0.f) : s;
+        }
+        store_vec<V>(out.p + (int64_t)b * out.sb + (int64_t)co * out.sc + (int64_t)z * out.sz +
+                         (int64_t)y * out.sy + x0,
+                     o);
+    };
+    auto stage_row = [&](float *t, const float (&a)[3][V]) {
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+#pragma unroll
+            for (int i = 0; i < V; i++) t[r * rowlen + i * lt.lpr + lane] = act ? a[r][i] : 0.f;
+    };
     int counter = 0;
 #pragma unroll
     for (int co = 0; co < WOUT; co++) {
         const float bv = bias[co];
+        if constexpr (batch > 1) {
 #pragma unroll
-        for (int jz = 0; jz < RZ; jz++)
+            for (int r0 = 0; r0 < R; r0 += batch) {
+                if (co > 0 || r0 > 0) __syncthreads();
 #pragma unroll
-            for (int jy = 0; jy < RY; jy++) {
-                const int z = z0 + jz * g.dil, y = y0 + jy * g.dil;
-                if (z >= g.D || y >= g.H) continue;             // uniform over the workgroup
-#pragma unroll
-                for (int r = 0; r < 3; r++)
-#pragma unroll
-                    for (int i = 0; i < V; i++)
-                        T[(kg * 3 + r) * rowlen + i * lt.lpr + lane] = act ? acc[co][jz][jy][r][i] : 0.f;
-                __syncthreads();
-                if (kg == counter % lt.ks && act) {
-                    float o[V];
-#pragma unroll
-                    for (int i = 0; i < V; i++) {
-                        const int xx = x0 + i;
-                        const int i0 = staged_index<V>(reflect_idx(xx - g.dil, g.W), lt.lpr);
-                        const int i1 = i * lt.lpr + lane;
-                        const int i2 = staged_index<V>(reflect_idx(xx + g.dil, g.W), lt.lpr);
-                        float s = bv;
-                        for (int kk = 0; kk < lt.ks; kk++) {
-                            const float *tk = T + (size_t)kk * 3 * rowlen;
-                            s += tk[i0] + tk[rowlen + i1] + tk[2 * rowlen + i2];
-                        }
-                        o[i] = RELU ? (s > 0.f ? s : 0.f) : s;
-                    }
-                    store_vec<V>(out.p + (int64_t)b * out.sb + (int64_t)co * out.sc + (int64_t)z * out.sz +
-                                     (int64_t)y * out.sy + x0,
-                                 o);
+                for (int j = 0; j < batch; j++) {
+                    const int jz = (r0 + j) / RY, jy = (r0 + j) % RY;
+                    if (r0 + j < R && jz < nzv && jy < nyv) stage_row(T + (kg * batch + j) * 3 * rowlen, acc[co][jz][jy]);  // uniform
                 }
-                counter++;
                 __syncthreads();
+                for (int j = kg; j < min(batch, R - r0); j += lt.ks) {      // uniform over the wave
+                    const int jz = (r0 + j) / RY, jy = (r0 + j) % RY;
+                    if (jz < nzv && jy < nyv && act)
+                        write_row(co, bv, T + j * 3 * rowlen, batch * 3 * rowlen, z0 + jz * g.dil, y0 + jy * g.dil);
+                }
             }
+        } else {
+#pragma unroll
+            for (int jz = 0; jz < RZ; jz++)
+#pragma unroll
+                for (int jy = 0; jy < RY; jy++) {
+                    const int z = z0 + jz * g.dil, y = y0 + jy * g.dil;
+                    if (z >= g.D || y >= g.H) continue;             // uniform over the workgroup
+                    stage_row(T + kg * 3 * rowlen, acc[co][jz][jy]);
+                    __syncthreads();
+                    if (kg == counter % lt.ks && act) write_row(co, bv, T, 3 * rowlen, z, y);
+                    counter++;
+                    __syncthreads();
+                }
+        }
     }
 }
 
@@ -276,7 +315,7 @@ inline bool make_lattice(const Geom &g, int V, int rz, int ry, int ks_wanted, La
     if (lpr > max_threads) return false;
     int ks = ks_wanted;
     while (ks > 1 && (ks * lpr > max_threads || ks > g.C)) ks /= 2;
-    if ((size_t)ks * 3 * V * lpr * sizeof(float) > kMaxLds) return false;
+    if ((size_t)ks * finish_batch(g.ndim, V, rz * ry) * 3 * V * lpr * sizeof(float) > kMaxLds) return false;
     lt->lpr = lpr;
     lt->ks = ks;
     lt->segs_y = ((g.H + g.dil - 1) / g.dil + ry - 1) / ry;
@@ -302,19 +341,19 @@ inline bool make_lattice(const Geom &g, int V, int rz, int ry, int ks_wanted, La
     return true;
 }
 
-template <int NDIM, bool RELU, int WOUT, int V, int RZ, int RY>
+template <int NDIM, bool RELU, int WOUT, int V, int RZ, int RY, bool ONE = false>
 hipError_t launch(const Geom &g, const View<const float> &x, const float *k, const float *bias,
-                  const View<float> &out, hipStream_t s, const ForwardSums *sums)
+                  const View<float> &out, hipStream_t s, const ForwardSums *sums, int groups = 2)
 {
     Lattice lt;
-    if (!make_lattice(g, V, RZ, RY, knob(kKnobFwdSplit, 2), &lt)) return hipErrorInvalidConfiguration;
+    if (!make_lattice(g, V, RZ, RY, ONE ? 1 : knob(kKnobFwdSplit, groups), &lt)) return hipErrorInvalidConfiguration;
     lt.kco = sums ? sums->kco : (int64_t)g.C * Taps<NDIM>::K;
     lt.zin = sums ? sums->z : nullptr;
     lt.zsb = sums ? sums->zsb : 0;
     const int remap = knob(kKnobXcdRemap, 1);
     const dim3 grid(remap ? xcd_grid(lt.ntiles) : lt.ntiles, g.B, 1);
-    const size_t lds = (size_t)lt.ks * 3 * V * lt.lpr * sizeof(float);
-    hipLaunchKernelGGL((fwd_lattice<NDIM, RELU, WOUT, V, RZ, RY>), grid, dim3(lt.ks * lt.lpr), lds, s, g, lt, remap, x,
+    const size_t lds = (size_t)lt.ks * finish_batch(NDIM, V, RZ * RY) * 3 * V * lt.lpr * sizeof(float);
+    hipLaunchKernelGGL((fwd_lattice<NDIM, RELU, WOUT, V, RZ, RY, ONE>), grid, dim3(lt.ks * lt.lpr), lds, s, g, lt, remap, x,
                        k, bias, out);
     return hipGetLastError();
 }
@@ -370,23 +409,42 @@ hipError_t pick(const Geom &g, const View<const float> &x, const float *k, const
         if (v == 2) return launch<3, RELU, WOUT, 2, 2, 4>(g, x, k, bias, out, s, sums);
         if (v == 1) {
             if constexpr (WOUT == 1) {
-                // Lattices of 3 x 3 rows instead of 2 x 4 where they cover the residue classes
-                // with at least 1/16 fewer tiles (a partly filled lattice costs as much time as a
-                // full one): at 128^3 dilations 3, 5, 9, 10, by 2 to 12 %.  Not at dilations 1
-                // and 2, where the nine rows per tile cost more than the fewer tiles save.
+                // Times are means over dilations 1 to 10, us.
                 const int rows_y = (g.H + g.dil - 1) / g.dil, rows_z = (g.D + g.dil - 1) / g.dil;
                 const long t24 = (long)((rows_z + 1) / 2) * ((rows_y + 3) / 4);
                 const long t33 = (long)((rows_z + 2) / 3) * ((rows_y + 2) / 3);
-                // Lattices of 4 x 4 rows read 36 input rows for 16 output rows (2.25 per row
-                // instead of 3) and halve the number of tiles; they take twice the registers, so
-                // two workgroups fewer share a CU.
                 const long t44 = (long)((rows_z + 3) / 4) * ((rows_y + 3) / 4);
+                const long waves = (long)g.dil * g.dil * g.B * ((g.W + kWave - 1) / kWave);     // per tile of a residue class
                 const int forced = knob(kKnobFwdLattice3d, 0);
-                if (forced == 44) return launch<3, RELU, 1, 1, 4, 4>(g, x, k, bias, out, s, sums);
+                if (forced == 44) return launch<3, RELU, 1, 1, 4, 4, true>(g, x, k, bias, out, s, sums);
                 if (forced == 33) return launch<3, RELU, 1, 1, 3, 3>(g, x, k, bias, out, s, sums);
                 if (forced == 24) return launch<3, RELU, 1, 1, 2, 4>(g, x, k, bias, out, s, sums);
-                (void)t44;
-                if (g.dil >= 3 && t33 * 16 < t24 * 15) return launch<3, RELU, 1, 1, 3, 3>(g, x, k, bias, out, s, sums);
+                // Lattices of 4 x 4 rows read 36 input rows for 16 output rows (2.25 per row
+                // instead of 3) but take twice the registers: where the input comes from memory and not
+                // from the 256 MB cache, the tiles of all channels at once fill the chip (four waves per SIMD) and are
+                // hardly more than half as many.  256^3 over 16 / 30 channels: 317, 297 / 602, 555; 192^3 over
+                // 20 / 45: 169, 165 / 403, 364; 128^3 over 30 (2048 waves): 69, 89.
+                const bool streams = (double)g.B * g.C * g.nvox * sizeof(float) > 1.5 * kCacheResidentBytes;
+                if (streams && t44 * waves >= 4096 && t44 * 32 <= t24 * 17)
+                    return launch<3, RELU, 1, 1, 4, 4, true>(g, x, k, bias, out, s, sums);
+                // The channels in one group where few of them leave the finishing step a large part and the tiles fill
+                // the chip without more waves (192^3 over 5 / 8 / 12 channels: 64, 50 / 80, 67 / 107, 99; over 20:
+                // 169, 175), in four where the tiles leave most of it idle (64^3 over 20 / 45: 18, 16 / 33, 23;
+                // 40 x 45 x 47 over 45: 27, 17; 61 x 93 x 75, 1500 waves, over 20: 25, 25; over 12: 18, 19).
+                const bool full = t24 * waves >= 7000;
+                const bool one = (full && g.C <= 12 && knob(kKnobFwdSplit, -1) < 0) || knob(kKnobFwdSplit, -1) == 1;
+                const int groups = t24 * waves <= 1100 && g.C >= 12 ? 4 : 2;
+                // Lattices of 3 x 3 rows instead of 2 x 4 where they cover the residue classes
+                // with at least 1/16 fewer tiles (a partly filled lattice costs as much time as a
+                // full one): at 128^3 dilations 3, 5, 9, 10, by 2 to 12 %.  Not at dilations 1
+                // and 2 of volumes that do not fill the chip, where the nine rows per tile cost more than the
+                // fewer tiles save.
+                const bool square = (g.dil >= 3 || full) && t33 * 16 < t24 * 15;
+                if (one)
+                    return square ? launch<3, RELU, 1, 1, 3, 3, true>(g, x, k, bias, out, s, sums)
+                                  : launch<3, RELU, 1, 1, 2, 4, true>(g, x, k, bias, out, s, sums);
+                return square ? launch<3, RELU, 1, 1, 3, 3>(g, x, k, bias, out, s, sums, groups)
+                              : launch<3, RELU, 1, 1, 2, 4>(g, x, k, bias, out, s, sums, groups);
             }
             return launch<3, RELU, WOUT, 1, 2, 4>(g, x, k, bias, out, s, sums);
         }

@@ -202,6 +202,21 @@ def test_operators_under_a_forced_setting(cc, case):
         check_operator_problem(cc, shape, seed=3)
 
 
+# 3D forward with all channels in one group (a channel's products first) and in four, tiles of 2 x 4, 3 x 3 and
+# 4 x 4 rows: whole ones, ones cut off in y, in z and in both, rows of one voxel over a wave, the longest rows.
+GROUPS_3D = [({"fwd.split": 1}, s) for s in ((1, 7, 1, (9, 9, 40), 3), (2, 13, 1, (7, 10, 65), 1), (1, 1, 1, (5, 3, 512), 2),
+                                            (1, 5, 1, (20, 19, 33), 3))]
+GROUPS_3D += [({"fwd.lattice3d": 44}, s) for s in ((1, 7, 1, (9, 11, 40), 2), (2, 3, 1, (4, 4, 130), 1), (1, 30, 1, (15, 13, 64), 5))]
+GROUPS_3D += [({}, s) for s in ((1, 12, 1, (9, 9, 40), 3), (1, 13, 1, (8, 11, 65), 1), (1, 15, 1, (4, 5, 300), 2))]
+
+
+@pytest.mark.parametrize("case", GROUPS_3D, ids=_id)
+def test_channel_groups_of_the_3d_forward(cc, case):
+    settings, shape = case
+    with tuning(settings):
+        check_operator_problem(cc, shape, seed=5)
+
+
 BLOCK_SETTINGS = [{"block.snake": 0}, {"block.snake": 1}, {"block.fuse": 0}, {"block.defer": 0},
                   {"xcd_remap": 0}, {"bwdk.interleave": 0}, {"fwd.class3d": 0}, {"fwd.lattice3d": 44},
                   {"block.pair": 0}, {"block.pair": 1}, {"block.pair": 1, "block.defer": 0},
