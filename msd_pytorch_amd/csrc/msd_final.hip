@@ -305,9 +305,28 @@ constexpr int kTiledWaves = 8;
 constexpr int kTiledThreads = kTiledWaves * kWave;
 constexpr int kTiledMaxChannels = 128;
 
+// V floats at any multiple of four bytes (images of odd size: every channel begins elsewhere).  3 x 333 x 477, 35
+// channels, three labels: 66 us with one voxel per lane, the widest aligned access, 42 with four; 61 x 93 x 75, 21 channels: 35 and 15.
+template <int V> __device__ __forceinline__ void load_unaligned(uint64_t base, uint32_t byte_offset, float (&d)[V])
+{
+    typedef float vec_t __attribute__((ext_vector_type(V), aligned(4)));
+    typedef const __attribute__((address_space(1))) char *gbytes_t;
+    const vec_t v = *reinterpret_cast<const __attribute__((address_space(1))) vec_t *>(reinterpret_cast<gbytes_t>(base) + byte_offset);
+#pragma unroll
+    for (int i = 0; i < V; i++) d[i] = v[i];
+}
+template <int V> __device__ __forceinline__ void store_unaligned(float *p, const float (&d)[V])
+{
+    typedef float vec_t __attribute__((ext_vector_type(V), aligned(4)));
+    vec_t v;
+#pragma unroll
+    for (int i = 0; i < V; i++) v[i] = d[i];
+    *reinterpret_cast<vec_t *>(p) = v;
+}
+
 template <int V, int MAXO, int KIND, int CC>
 __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
-    int64_t nvec, int tiles_per_image, int total_tiles, int C, int c_out, const float *__restrict__ x, int64_t xsb,
+    int64_t nvox, int tiles_per_image, int total_tiles, int C, int c_out, const float *__restrict__ x, int64_t xsb,
     int64_t xsc, const float *__restrict__ w, const float *__restrict__ bias, const void *__restrict__ target,
     int64_t tsb, int64_t tsc, float *__restrict__ out, int64_t osb, int64_t osc, float *__restrict__ gout, int64_t gsb,
     int64_t gsc, float inv_n, int want_sums, float *__restrict__ part, int64_t rows)
@@ -336,11 +355,15 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
         asm volatile("" : "+s"(xsc), "+s"(C));
         const int b = tile / tiles_per_image;
         const int64_t i = (int64_t)(tile - b * tiles_per_image) * kWave + lane;
+        const int64_t nvec = (nvox + V - 1) / V;
         const bool active = i < nvec;
-        const int64_t ic = active ? i : nvec - 1;             // lanes past the end work on a valid voxel, contribute zeros
+        // lanes past the end work on valid voxels and contribute zeros; the last lane's are moved left where there are fewer
+        // than V, those below `skip` are the lane's before it
+        const int64_t iv = min((active ? i : nvec - 1) * V, nvox - V);
+        const int skip = active ? (int)(i * V - iv) : 0;
         // a uniform base per channel plus one 32-bit lane offset: no address registers per request
         const uint64_t xbase = reinterpret_cast<uint64_t>(x + (int64_t)b * xsb);
-        const uint32_t xoff = (uint32_t)(ic * V) * 4u;
+        const uint32_t xoff = (uint32_t)iv * 4u;
         float acc[MAXO][V];
 #pragma unroll
         for (int o = 0; o < MAXO; o++)
@@ -354,7 +377,7 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
             float v[G][V];
 #pragma unroll
             for (int j = 0; j < G; j++)
-                load_global_vec<V>(xbase + (uint64_t)((int64_t)min((c0 + j) * kTiledWaves + wave, C - 1) * xsc * 4), xoff,
+                load_unaligned<V>(xbase + (uint64_t)((int64_t)min((c0 + j) * kTiledWaves + wave, C - 1) * xsc * 4), xoff,
                                    v[j]);
 #pragma unroll
             for (int j = 0; j < G; j++) {
@@ -394,7 +417,7 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
         if constexpr (KIND == 2) {
             // the softmax is the expensive part: wave q forms it for element q of every lane's
             // voxels only, and the waves exchange the results through LDS below
-            const int64_t *lab = static_cast<const int64_t *>(target) + (int64_t)b * tsb + ic * V;
+            const int64_t *lab = static_cast<const int64_t *>(target) + (int64_t)b * tsb + iv;
 #pragma unroll
             for (int e = 0; e < V; e++) {
                 if (wave != e) continue;                      // uniform
@@ -415,7 +438,7 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
                     acc[o][e] -= lse;                         // log-probability
                     const float pr = o < c_out ? exp(acc[o][e]) : 0.f;
                     g[o][e] = active && o < c_out ? (pr - (t == o ? 1.f : 0.f)) * inv_n : 0.f;
-                    if (active && t == o) tile_loss -= acc[o][e];
+                    if (active && e >= skip && t == o) tile_loss -= acc[o][e];
                 }
             }
         } else {
@@ -423,8 +446,8 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
             for (int o = 0; o < MAXO; o++) {
                 const bool keep = active && o < c_out;
                 float t[V];
-                load_elems<float, V>(static_cast<const float *>(target) + (int64_t)b * tsb +
-                                         (int64_t)min(o, c_out - 1) * tsc + ic * V, t);
+                load_unaligned<V>(reinterpret_cast<uint64_t>(static_cast<const float *>(target) + (int64_t)b * tsb +
+                                                             (int64_t)min(o, c_out - 1) * tsc), xoff, t);
                 const float bv = bias && o < c_out ? bk[o] : 0.f;
 #pragma unroll
                 for (int e = 0; e < V; e++) {
@@ -432,10 +455,10 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
                     const float diff = acc[o][e] - t[e];
                     if (KIND == 0) {
                         g[o][e] = keep ? 2.f * diff * inv_n : 0.f;
-                        tile_loss += keep ? diff * diff : 0.f;
+                        tile_loss += keep && e >= skip ? diff * diff : 0.f;
                     } else {
                         g[o][e] = keep ? (diff > 0.f ? inv_n : (diff < 0.f ? -inv_n : 0.f)) : 0.f;
-                        tile_loss += keep ? (diff < 0.f ? -diff : diff) : 0.f;
+                        tile_loss += keep && e >= skip ? (diff < 0.f ? -diff : diff) : 0.f;
                     }
                 }
             }
@@ -469,10 +492,19 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
 #pragma unroll
                 for (int o = 0; o < MAXO; o++) {
                     if (o >= c_out) break;
-                    store_elems<float, V>(out + (int64_t)b * osb + (int64_t)o * osc + i * V, acc[o]);
-                    store_elems<float, V>(gout + (int64_t)b * gsb + (int64_t)o * gsc + i * V, g[o]);
+                    // (the voxels below `skip` get the same values twice)
+                    store_unaligned<V>(out + (int64_t)b * osb + (int64_t)o * osc + iv, acc[o]);
+                    store_unaligned<V>(gout + (int64_t)b * gsb + (int64_t)o * gsc + iv, g[o]);
                 }
             }
+        }
+        if (__any(skip > 0)) {
+#pragma unroll
+            for (int o = 0; o < MAXO; o++)
+#pragma unroll
+                for (int e = 0; e < V; e++) g[o][e] = e >= skip ? g[o][e] : 0.f;
+        }
+        if (wave == 0) {
 #pragma unroll
             for (int o = 0; o < MAXO; o++)
 #pragma unroll
@@ -674,8 +706,7 @@ hipError_t launch_tiled(int64_t batch, int c_in, int c_out, int64_t nvox, const 
                         int64_t osb, int64_t osc, float *gout, int64_t gsb, int64_t gsc, float inv_n, int want,
                         float *ws, int64_t *rows, hipStream_t s)
 {
-    const int64_t nvec = nvox / V;
-    const int64_t tiles_per_image = (nvec + kWave - 1) / kWave;
+    const int64_t tiles_per_image = ((nvox + V - 1) / V + kWave - 1) / kWave;
     const int64_t total = tiles_per_image * batch;
     if (total > INT32_MAX) return hipErrorInvalidConfiguration;
     const size_t lds = ((size_t)c_in * kWave * V + (size_t)kTiledWaves * MAXO * V * kWave) * sizeof(float);
@@ -686,23 +717,10 @@ hipError_t launch_tiled(int64_t batch, int c_in, int c_out, int64_t nvox, const 
     }
     const int grid = (int)std::min<int64_t>(total, 512);      // two workgroups per CU, each walks its tiles
     *rows = grid;
-    hipLaunchKernelGGL((final_forward_loss_tiled<V, MAXO, KIND, CC>), dim3(grid), dim3(kTiledThreads), lds, s, nvec,
+    hipLaunchKernelGGL((final_forward_loss_tiled<V, MAXO, KIND, CC>), dim3(grid), dim3(kTiledThreads), lds, s, nvox,
                        (int)tiles_per_image, (int)total, c_in, c_out, x, xsb, xsc, w, bias, target, tsb, tsc, out, osb,
                        osc, gout, gsb, gsc, inv_n, want, ws, (int64_t)grid);
     return hipGetLastError();
-}
-
-// V-wide accesses at multiples of V are aligned in every view given.
-inline bool vec_aligned(int v, int64_t nvox, std::initializer_list<std::pair<const void *, std::pair<int64_t, int64_t>>> views)
-{
-    if (nvox % v != 0) return false;
-    for (const auto &vw : views) {
-        if (!vw.first) continue;
-        if (reinterpret_cast<uintptr_t>(vw.first) % (v * sizeof(float)) != 0 || vw.second.first % v != 0 ||
-            vw.second.second % v != 0)
-            return false;
-    }
-    return true;
 }
 
 // The tiled kernel where it applies (fp32, up to 128 input and 4 output channels, a tile that
@@ -717,12 +735,9 @@ hipError_t final_forward_loss_tiled_try(int kind, int64_t batch, int c_in, int c
     if (c_in > kTiledMaxChannels || c_out > 4 || !knob(kKnobFinalTiled, 1)) return hipSuccess;
     const int mo = c_out > 2 ? 4 : (c_out > 1 ? 2 : 1);
     int v = 0;
-    for (int cand = 4; cand >= 1; cand /= 2) {
-        const bool aligned =
-            kind == 2 ? vec_aligned(cand, nvox, {{x, {xsb, xsc}}, {out, {osb, osc}}, {gout, {gsb, gsc}}})
-                      : vec_aligned(cand, nvox, {{x, {xsb, xsc}}, {out, {osb, osc}}, {gout, {gsb, gsc}}, {target, {tsb, tsc}}});
+    for (int cand = 4; cand >= 2; cand /= 2) {
         const size_t lds = ((size_t)c_in * kWave * cand + (size_t)kTiledWaves * mo * cand * kWave) * sizeof(float);
-        if (aligned && lds <= kTiledLdsLimit && (cand < 4 || c_in <= 64)) {
+        if (nvox >= cand && lds <= kTiledLdsLimit && (cand < 4 || c_in <= 64)) {
             v = cand;
             break;
         }
@@ -745,7 +760,7 @@ hipError_t final_forward_loss_tiled_try(int kind, int64_t batch, int c_in, int c
     do {                                                                                        \
         if (mo == 4) MSD_TILED_K(VV, 4); else if (mo == 2) MSD_TILED_K(VV, 2); else MSD_TILED_K(VV, 1); \
     } while (0)
-    if (v == 4) MSD_TILED_O(4); else if (v == 2) MSD_TILED_O(2); else MSD_TILED_O(1);
+    if (v == 4) MSD_TILED_O(4); else MSD_TILED_O(2);
 #undef MSD_TILED_O
 #undef MSD_TILED_K
 #undef MSD_TILED_C
