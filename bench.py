@@ -14,6 +14,7 @@ kernels) on a bounded sample of the same network.
 """
 import argparse
 import json
+import math
 import os
 import sys
 import time
@@ -32,11 +33,12 @@ PIPE = {"forward": "fp32 VALU, non-packed (78.6 TFLOP/s of the 157.3 peak); 2D l
                         "2D layer groups: both on the MFMA"}
 
 # kernel families (as named in the profile summaries) whose HBM traffic belongs to a class
-FAMILIES = {"forward": ("fwd_lattice", "push_rows", "finish_rows"),
-            "backward_xkb": ("bwd_rows_fused", "bwd_one_channel", "pull_rows", "finish_back", "sum_group", "reduce_columns"),
+FAMILIES = {"forward": ("fwd_lattice", "push_rows", "push_table", "push_split", "finish_rows"),
+            "backward_xkb": ("bwd_rows_fused", "bwd_one_channel", "pull_rows", "finish_back", "spread_back", "sum_group",
+                             "reduce_columns"),
             "backward_kb": ("bwdk_rows", "bwdk_mfma"), "backward_x": ("relu_mask", "bwdx_rows", "bwdx_one_channel")}
 # families that are the further passes of an operator call or of a group of layers, not a call of their own
-SECOND_PASS = ("reduce_columns", "finish_rows", "finish_back", "sum_group")
+SECOND_PASS = ("reduce_columns", "push_table", "finish_rows", "finish_back", "spread_back", "sum_group")
 
 
 def profiled_traffic(name, split3d=False):
@@ -135,21 +137,24 @@ def make_model(name, torch):
     return model
 
 
-def grouped_layers(c_in, depth, width):
-    """The layers that the library takes in groups of up to seven outputs on the matrix cores (2D,
-    one or two channels per layer): {first layer: layers} of the forward pass (from the bottom, where
-    at least 12 channels, 6 with two per layer, lie in front) and of the backward pass (from the
-    top, over at least 4 channels)."""
-    most, forward, backward = 7 // width, {}, {}
+def grouped_layers(ndim, c_in, depth, width, voxels):
+    """The layers that the library takes in groups on the matrix cores (one or two channels per
+    layer): {first layer: layers} of the forward pass (2D; from the bottom, where at least 12
+    channels, 6 with two per layer, lie in front: up to seven outputs, fourteen where these channels are
+    2^28 voxels in all, 2^27 with two per layer; no dilation above 16) and of the backward pass (from the
+    top, down to the first layer: up to fourteen outputs, four in 3D)."""
+    forward, backward = {}, {}
     i = 0
-    while i < depth:
-        n = min(most, depth - i) if c_in + width * i >= (6 if width > 1 else 12) else 0
+    while ndim == 2 and i < depth:
+        c = c_in + width * i
+        most = (14 if c * voxels >= 1 << (27 if width > 1 else 28) else 7) // width
+        n = min(most, depth - i) if c >= (6 if width > 1 else 12) else 0
         if n >= 2:
             forward[i] = n
         i += n if n >= 2 else 1
     i = depth - 1
     while i >= 0:
-        n = sum(1 for j in range(min(most, i + 1)) if c_in + width * (i - j) >= 4)
+        n = min((14 if ndim == 2 else 4) // width, i + 1)
         if n >= 2:
             backward[i - n + 1] = n
         i -= n if n >= 2 else 1
@@ -175,8 +180,9 @@ def algorithmic_work(name, fused, paired=False, triple_from=32, kpairs=False, ch
     `groups` (grouped_layers): the forward pass of n layers over the c channels in front of them is
     one read of these and three planes per output, (c + 3 n w) N 4 bytes, then per layer its planes, the
     j w channels that the group has added and its outputs, (4 + j) w N 4; the backward pass is per
-    layer but the top one its channels' gradient (read, written, activation) and the outputs above,
-    (3 + j) w N 4, then one pass (3 c + (2 n - 1) w) N 4.
+    layer but the top one its channels' gradient (read, written, activation) and the j layers above it,
+    (3 + j) w N 4, then one pass (3 c + (2 n - 1) w) N 4.  Above seven outputs (2D) the upper seven add what they
+    owe the m layers below them at once, (7 + (2 m + 1) w) N 4, and j counts within each half.
     `kpairs`: the library runs a 3D block of width 1 as a chain of backward_x launches with the
     weight and bias gradients of two layers per pass over x beside it (layers depth-1 and depth-2,
     ... down to 1 and 0; an odd lowest layer alone): a pair reads the C input channels of its
@@ -202,8 +208,11 @@ def algorithmic_work(name, fused, paired=False, triple_from=32, kpairs=False, ch
     for i, m in groups[1].items():
         c = c_in + width * i
         in_pair.update(range(i, i + m))
-        nbytes["backward_xkb"] += (3 * c + (2 * m - 1) * width + sum((3 + j) * width for j in range(1, m))) * n * 4 \
-            + 2 * m * width * c * K * 4
+        upper = min(m, 7 // width) if ndim == 2 else m
+        finish = sum((3 + j) * width for j in range(1, upper))
+        if m > upper:                         # the lower half's top layer is complete with the upper half's share
+            finish += upper * width + (2 * (m - upper) + 1) * width + sum((3 + j) * width for j in range(1, m - upper))
+        nbytes["backward_xkb"] += (3 * c + (2 * m - 1) * width + finish) * n * 4 + 2 * m * width * c * K * 4
     if fused and paired:
         i = min(groups[1], default=depth) - 1
         while i - 1 > 0:
@@ -228,6 +237,9 @@ def algorithmic_work(name, fused, paired=False, triple_from=32, kpairs=False, ch
             if i not in in_pair:
                 nbytes["backward_xkb"] += per_layer
             flops["backward_xkb"] += 2 * op
+            continue
+        if fused and i in in_pair:            # layer 0 of a group: weight gradients only
+            flops["backward_xkb"] += op
             continue
         upper, lower = (depth - 1 - i) % 2 == 0 and i > 0, (depth - 1 - i) % 2 == 1
         if chainpairs and (upper or lower):
@@ -366,23 +378,24 @@ def measure(name, args, lib, torch, steps=None, warmup=None, cpu=True):
 
     if not args.no_kernel_timing:
         totals = kernel_times(lib, torch, lambda: [eager_step() for _ in range(args.steps)])
-        # 2D blocks run their layers in groups of up to seven outputs (fwd.group, bwd.group: 0 never); what
-        # is left, or without groups all layers of width 1, two or three at a time in the backward pass
-        # (block.pair; block.triple: from how many shared channels three, 0 never, 32 by default)
+        # blocks run their layers in groups (fwd.group, bwd.group: 0 never); without groups the 2D
+        # layers of width 1 go two or three at a time in the backward pass (block.pair; block.triple: from how
+        # many shared channels three, 0 never, 32 by default)
         tuned = dict(kv.replace(" ", "").split("=") for kv in args.tune)
         paired = ndim == 2 and width == 1 and tuned.get("block.pair") != "0" and tuned.get("block.fuse") != "0"
         triple = int(tuned.get("block.triple", -1))
         triple_from = None if triple == 0 else (32 if triple < 0 else triple)
-        # 3D blocks of width 1 may run as a chain of backward_x launches with the weight gradients
+        # without groups 3D blocks of width 1 may run as a chain of backward_x launches with the weight gradients
         # two layers per pass on a second stream (block.split3d); the instrumented repeat runs both
         # on one stream, so the classes' times add up to more than the step's backward pass
         split3d = ndim == 3 and width == 1 and totals["backward_xkb"][1] == 0 and \
             0 < totals["backward_kb"][1] // args.steps < depth
-        forward, backward = grouped_layers(c_in, depth, width) if ndim == 2 and width <= 2 else ({}, {})
+        voxels = batch * math.prod(spatial)
+        forward, backward = grouped_layers(ndim, c_in, depth, width, voxels) if width <= 2 else ({}, {})
         if tuned.get("fwd.group") == "0":
             forward = {}
-        if tuned.get("bwd.group") == "0" or tuned.get("block.fuse") == "0" or "block.pair" in tuned \
-                or "block.triple" in tuned:
+        if tuned.get("bwd.group") == "0" or tuned.get("block.fuse") == "0" or any(
+                k in tuned for k in (("block.pair", "block.triple") if ndim == 2 else ("block.split3d", "block.chainpair"))):
             backward = {}
         bytes_per_step, flops_per_step, _ = algorithmic_work(name, totals["backward_xkb"][1] > 0, paired, triple_from,
                                                              groups=(forward, backward),
@@ -402,7 +415,7 @@ def measure(name, args, lib, torch, steps=None, warmup=None, cpu=True):
                             "algorithmic_GFLOP_per_step": round(flops_per_step[cls] / 1e9, 2),
                             "TFLOPs": round(tfl, 2), "frac_fp32": round(tfl / FP32_PEAK_TFLOPS, 4),
                             "Mvoxel_per_s": round(nvox / per_step_s / 1e6, 2)}
-            if cls == "backward_xkb" and paired:
+            if cls == "backward_xkb" and (paired or backward):
                 # the same time priced with the bytes of one fused pass per layer, for comparison
                 per_layer = bytes_per_step["backward_xkb_per_layer"]
                 kernels[cls]["layers_in_groups"] = True

@@ -303,7 +303,7 @@ int msd_relu_mask_gradient(int dtype, int ndim, int64_t batch, int64_t c_out, co
  * Replaces the loop of msd_block.py:89-130.  Workspace: msd_block_workspace_bytes,
  * which is the largest msd_workspace_bytes of the layers plus room (at most 1 GiB) for
  * the partial weight-gradient sums of many layers at once, so that one launch can
- * reduce up to 16 layers, or what the partial sums of a group of 2D layers take where
+ * reduce up to 16 layers, or what the partial sums of a group of layers take where
  * that is more.  The largest msd_workspace_bytes of the layers alone is accepted too
  * (layers are then taken one at a time and reduced right away; same sums, in another order).
  */
@@ -317,7 +317,8 @@ int msd_block_forward(int dtype, int ndim, int64_t batch, int64_t c_in, int dept
 /* The same with a workspace (msd_block_forward_workspace_bytes; less, or none, is accepted):
  * groups of layers then take the channels in front of them in one pass (2D, fp32; same sums in
  * another order).  It holds three planes per output channel of a group, so up to 21 channels of the
- * stack's size, while the call runs. */
+ * stack's size (large stacks: 42, and 13 KB per 32 channels; these groups take a workspace that begins at a multiple of
+ * 16 bytes), while the call runs. */
 int64_t msd_block_forward_workspace_bytes(int dtype, int ndim, int64_t batch, int64_t c_in, int depth,
                                           const int64_t *widths, const int64_t *spatial);
 int msd_block_forward_ws(int dtype, int ndim, int64_t batch, int64_t c_in, int depth, const int64_t *widths,
