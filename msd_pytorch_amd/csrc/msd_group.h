@@ -91,6 +91,12 @@ hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::
                       const View<float> &grads, int first, const int *channels, float *const *gk, float *gb,
                       float *ws, bool reverse, hipStream_t s);
 
+// All three gradients of a single layer (g.Wd <= 2 outputs of dilation g.dil) over a volume without gaps, written and not added
+// to.  gy: the masked output gradient, without gaps in an image.  ws: group_pull_floats floats.
+bool layer_pull_supported_3d(const Geom &g, const View<const float> &x, const View<const float> &gy, const View<float> &gx);
+hipError_t layer_pull_3d(const Geom &g, const View<const float> &x, const View<const float> &gy, const float *k, const View<float> &gx,
+                         float *gk, float *gb, float *ws, hipStream_t s);
+
 // Completes the gradient of the `width` channels from `channel` on: adds what the outputs right
 // above them (`above`, their weights of these channels) contribute, and applies the ReLU mask.
 hipError_t group_finish_back(const Geom &g, const View<const float> &x, const View<float> &grads, int channel, int width,

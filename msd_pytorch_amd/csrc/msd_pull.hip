@@ -119,7 +119,8 @@ struct PullArgs {
     int reverse;                                  // walk the tiles from the last to the first
     int dmax;
     Chunks chunks;
-    int64_t sb, sc, sz, sy;                       // strides of x and of the gradients
+    int64_t sb, sc, sz, sy;                       // strides of x and of grad_input
+    int64_t gsb, gsc;                             // of the outputs' gradients (their rows lie as those of x)
     Outputs out;
 };
 
@@ -206,7 +207,7 @@ template <int G> struct PullState {
 
 // The tiles of a workgroup.  True where units were left out that hold values which cannot be split: the second
 // run (WHOLE) takes these, with the fp32 instruction.  Apart, so that it keeps no registers in the first.
-template <int N, int G, int P, bool WHOLE>
+template <int N, int G, int P, bool FRESH, bool WHOLE>
 __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__restrict__ x, const float *gy, float *gx, float *row,
                                            char *lds, PullShared &shared, int tid, int wave, int blocks, int c0, int wgs, int wg,
                                            PullState<G> &state)
@@ -225,7 +226,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
 
     struct Tile {
         int first;                                // segment of its image
-        int64_t img;                              // byte offset of the image
+        int64_t img, gimg;                        // byte offsets of the image, of the outputs' gradients
         uint32_t sign;                            // of x in this tile
     };
     struct Place {
@@ -239,6 +240,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         const int b = a.by_tiles.of(it);
         t.first = (it - b * a.image_tiles) * kSegs;
         t.img = (int64_t)b * a.sb * 4;
+        t.gimg = (int64_t)b * a.gsb * 4;
         t.sign = (uint32_t)it << 31;
         return t;
     };
@@ -294,9 +296,15 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             d[i] = f32x4_t{v4[0], v4[1], v4[2], v4[3]};
         }
     };
-    const int g_limit = max(a.update, 1);
-
     f32x4_t xs[kVec], gs[kVec];
+    auto request_g = [&](const Unit &un) {
+        if constexpr (FRESH) {
+#pragma unroll
+            for (int i = 0; i < kVec; i++) gs[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        } else {
+            request(gx, max(a.update, 1), un, gs);
+        }
+    };
 
     // ---- the gather: lane (v, h) takes its outputs at voxel v of the wave's segment, 36 (27) values for 32 rows
     // m.  Its loads are issued in the tile before, in front of that tile's last stores and requests (all of
@@ -332,7 +340,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
     auto gather = [&](const Tile &t, const Place &p) {
         if (away(p)) {
             const uint32_t u = (uint32_t)(p.x0 + v);
-            const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)(t.img + (int64_t)row_at(p.z, p.y) * 4) - bias;
+            const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)(t.gimg + (int64_t)row_at(p.z, p.y) * 4) - bias;
 #pragma unroll
             for (int j = 0; j < kLaneOut; j++) {
                 const Source o = source(j);
@@ -348,7 +356,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                 __builtin_amdgcn_sched_barrier(0);    // (an output's addresses at a time: registers)
             }
         } else {
-            const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)t.img;
+            const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)t.gimg;
             const Voxel vx = voxel_of(p);
 #pragma unroll
             for (int j = 0; j < kLaneOut; j++) {
@@ -368,7 +376,8 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             }
         }
     };
-    auto gathered = [&](const Place &p, bool count) {
+    // round: number of the tile among the workgroup's, below 0 where its biases have been counted
+    auto gathered = [&](const Place &p, int round) {
         if (!away(p)) {
             const Voxel vx = voxel_of(p);
 #pragma unroll
@@ -398,8 +407,9 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                 for (int t = 0; t < kTaps; t++) val[j][t / 3][t % 3] = ok ? val[j][t / 3][t % 3] : 0.f;
             }
         }
-        if (count) {
-            if constexpr (N != kImage) shared.bias_sums[tid][0] += val[0][4][1];
+        if (round >= 0) {
+            // (volumes: one value per lane, four chains of a quarter of the tiles)
+            if constexpr (N != kImage) reinterpret_cast<float *>(&shared.bias_sums[tid])[round % 4] += val[0][4 * (kLines / 9)][1];
             else shared.bias_sums[tid] += f32x4_t{val[0][1][1], val[1][1][1], val[2][1][1], val[3][1][1]};
         }
         // -A at every second voxel: the sums of the bf16 instruction are cut off towards minus infinity, which adds up
@@ -753,7 +763,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             const Tile t = tile_of(tile);
             const Place here = locate(t, segment);
             gather(t, here);
-            gathered(here, false);
+            gathered(here, -1);
             __syncthreads();
             if (active) {
                 const bool split = tile_split();
@@ -761,7 +771,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                 for (int u = 0; u < kUnits; u++) {
                     const Unit un = unit_of(t, u);
                     request(x, a.C, un, xs);
-                    request(gx, g_limit, un, gs);
+                    request_g(un);
                     clear_skipped(un);
                     const float rest = put_x(t.sign);
                     if (split && !__any(rest != rest)) continue;    // (the first run has done it)
@@ -776,12 +786,13 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         Tile now = tile_of(lb);
         Unit un = unit_of(now, 0);
         request(x, a.C, un, xs);
-        request(gx, g_limit, un, gs);
+        request_g(un);
         bool again = false;                       // units were left to the second run
         Place here = locate(now, segment);
         gather(now, here);
+        int round = 0;
         for (int tile = lb; tile < a.tiles; tile += wgs) {          // uniform over the workgroup
-            gathered(here, true);
+            gathered(here, round++);
             tile_sync();
             const Tile then = tile_of(tile + wgs);
             here = locate(then, segment);
@@ -795,7 +806,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                     if (u + 1 == kUnits) gather(then, here);
                     store(un, done);
                     __builtin_amdgcn_sched_barrier(0);
-                    request(gx, g_limit, next, gs);
+                    request_g(next);
                     __builtin_amdgcn_sched_barrier(0);
                     un = next;
                 }
@@ -809,7 +820,8 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
     }
 }
 
-template <int N, int G, int P>
+// FRESH: grad_input is written, not added to.
+template <int N, int G, int P, bool FRESH = false>
 __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, const float *__restrict__ x, const float *gy,
                                                              float *gx, float *__restrict__ part, float *__restrict__ bias_part)
 {
@@ -830,7 +842,7 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
     if (tid == 0) shared.bad_again = 0;
     if (tid < G * kSlabOut) {
         const int o = min(tid, a.out.n - 1), d = a.out.dil[o];
-        shared.sources[tid] = Source{N == kVolume ? 4u * (uint32_t)(d * (int)a.sz) : 0u, 4u * (uint32_t)(d * (int)a.sy), 4u * (uint32_t)d, (uint32_t)o * ((uint32_t)a.sc * 4u)};
+        shared.sources[tid] = Source{N == kVolume ? 4u * (uint32_t)(d * (int)a.sz) : 0u, 4u * (uint32_t)(d * (int)a.sy), 4u * (uint32_t)d, (uint32_t)o * ((uint32_t)a.gsc * 4u)};
     }
     state.weights_split = true;
 #pragma unroll
@@ -858,13 +870,13 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
 #pragma unroll
     for (int t = 0; t < kTiles; t++) state.sums[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     shared.bias_sums[tid] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    const bool again = pull_tiles<N, G, P, false>(a, x, gy, gx, row, lds, shared, tid, wave, blocks, c0, wgs, wg, state);
+    const bool again = pull_tiles<N, G, P, FRESH, false>(a, x, gy, gx, row, lds, shared, tid, wave, blocks, c0, wgs, wg, state);
     if (lane == 0 && again) shared.bad_again = 1;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(shared.bad_again) != 0) {    // uniform over the workgroup
         int tid2 = tid;
         asm volatile("" : "+v"(tid2));           // (nothing of the first run is kept for the second)
-        pull_tiles<N, G, P, true>(a, x, gy, gx, row, lds, shared, tid2, wave, blocks, c0, wgs, wg, state);
+        pull_tiles<N, G, P, FRESH, true>(a, x, gy, gx, row, lds, shared, tid2, wave, blocks, c0, wgs, wg, state);
     }
 
     // the sums, of the waves that share a block through LDS
@@ -894,6 +906,7 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
     const int v = lane % kSegment, h = lane / kSegment;
     // the bias gradients: the centre taps, over the lanes' voxels and the segments
     f32x4_t bias_sum = shared.bias_sums[tid];
+    if constexpr (N != kImage) bias_sum[0] = (bias_sum[0] + bias_sum[1]) + (bias_sum[2] + bias_sum[3]);
 #pragma unroll
     for (int j = 0; j < kLaneOut; j++)
 #pragma unroll
@@ -919,7 +932,7 @@ struct SumArgs {
     int columns;                                  // weight columns in all (a multiple of 1024 slabs)
     int slabs;
     int stride;                                   // of the rows of partial sums
-    int n;
+    int n, fresh;                                 // outputs; gradients are written, not added to
     int channels[kMaxOut];                        // input channels of each output
     float *gk[kMaxOut];
     float *gb;
@@ -970,14 +983,17 @@ __global__ __launch_bounds__(1024) void sum_group(const SumArgs a, const float *
     const float s = tree[0];
     if (bias) {
         const int o = lane / kBiasColumns * kSlabOut + lane % kBiasColumns;
-        if (lane < a.slabs * kBiasColumns && lane % kBiasColumns < kSlabOut && o < a.n) a.gb[o] += s;
+        if (lane < a.slabs * kBiasColumns && lane % kBiasColumns < kSlabOut && o < a.n) a.gb[o] = a.fresh ? s : a.gb[o] + s;
         return;
     }
     // column (tile of 16 rows, r, lane (channel, q)) of a block: row 16 tile + 4 q + r
     const int i = col % block, l = i % kWave;
     const Slot m = slot_of<N>(i / 256 * 16 + l / 16 * 4 + i / kWave % 4);
     const int ch = blk * 16 + l % 16;
-    if (m.tap >= 0 && m.output < a.n && ch < a.channels[m.output]) a.gk[m.output][(int64_t)ch * kTaps + m.tap] += s;
+    if (m.tap >= 0 && m.output < a.n && ch < a.channels[m.output]) {
+        float &k = a.gk[m.output][(int64_t)ch * kTaps + m.tap];
+        k = a.fresh ? s : k + s;
+    }
 }
 
 // grad_input of the channels that layers of a group wrote, from the outputs of the layers above them
@@ -1197,15 +1213,15 @@ FinishArgs finish_args(const Geom &g, const View<const float> &x, const group2d:
     return a;
 }
 
-template <int N, int G, int P>
+template <int N, int G, int P, bool FRESH = false>
 hipError_t pull_launch(const PullArgs &a, int wgs, const float *x, const float *gy, float *gx, float *part, float *bias_part,
                        hipStream_t s)
 {
     constexpr int kLds = kWaves * (kSlabBytes + PullShape<G, P>::kOwnBytes);
     static LargeLds large;
-    const hipError_t e = large.allow(reinterpret_cast<const void *>(&pull_rows<N, G, P>), kLds);
+    const hipError_t e = large.allow(reinterpret_cast<const void *>(&pull_rows<N, G, P, FRESH>), kLds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((pull_rows<N, G, P>), dim3(wgs), dim3(kWaves * kWave), kLds, s, a, x, gy, gx, part, bias_part);
+    hipLaunchKernelGGL((pull_rows<N, G, P, FRESH>), dim3(wgs), dim3(kWaves * kWave), kLds, s, a, x, gy, gx, part, bias_part);
     return hipGetLastError();
 }
 
@@ -1263,20 +1279,25 @@ bool group_pull_supported(const Geom &g, const View<const float> &x, const View<
            (int64_t)g.B * g.D * g.H * ((g.W + kSegment - 1) / kSegment) < ((int64_t)1 << 30);
 }
 
-hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::Outputs &out, int update, int mask_from,
-                      const View<float> &grads, int first, const int *channels, float *const *gk, float *gb,
-                      float *ws, bool reverse, hipStream_t s)
+namespace {
+
+// gy: the outputs' gradients, channels gsc apart, rows as in x.  fresh: the gradients are written, not added to (volumes
+// without gaps, at most two outputs).
+hipError_t pull(const Geom &g, const View<const float> &x, const float *gy, int64_t gsb, int64_t gsc, const group2d::Outputs &out,
+                int update, int mask_from, const View<float> &grads, const int *channels, float *const *gk, float *gb, float *ws,
+                bool reverse, bool fresh, hipStream_t s)
 {
     using namespace group2d;
     const int per_slab = g.ndim == 3 ? kSlabOut3d : kSlabOut;
-    if (out.n < 1 || out.n > 2 * per_slab || !group_pull_supported(g, x, grads)) return hipErrorInvalidValue;
-    const int slabs = out.n > per_slab ? 2 : 1;
     const Form form = form_of(g, x);
+    if (out.n < 1 || out.n > 2 * per_slab || !group_pull_supported(g, x, grads) || (fresh && (form != kFlat || out.n > kSlabOut3d)))
+        return hipErrorInvalidValue;
+    const int slabs = out.n > per_slab ? 2 : 1;
     const int span = form == kFlat ? g.nvox : g.W, rows = g.nvox / span;
     const PullPlan p = pull_plan(g.B, rows, span, g.C, slabs);
     PullArgs a{g.C, update, mask_from, g.D, g.H, g.W, span, p.segs, rows * p.segs, p.tiles, p.image_tiles, Divisor((uint32_t)p.segs),
                Divisor((uint32_t)p.image_tiles), Divisor((uint32_t)g.H), Divisor((uint32_t)g.W), reverse, 0, p.chunks,
-               x.sb, x.sc, x.sz, x.sy, out};
+               x.sb, x.sc, x.sz, x.sy, gsb, gsc, out};
     SumArgs sum;
     for (int o = 0; o < kMaxOut; o++) {
         if (o < out.n) a.dmax = std::max(a.dmax, out.dil[o]);
@@ -1284,12 +1305,15 @@ hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::
         sum.gk[o] = o < out.n ? gk[o] : nullptr;
     }
     float *const bias_part = ws + (int64_t)p.wgs * slabs * p.chunks.blocks * 1024;
-    const float *const gy = grads.p + (int64_t)first * grads.sc;
     hipError_t e = hipErrorInvalidConfiguration;
     // waves to a block: 4, 2 or 1
     const int share = p.chunks.blocks <= 2 ? 4 : p.chunks.blocks <= 4 ? 2 : 1;
     auto launch = [&](auto f) {
         constexpr int N = decltype(f)::value;
+        if constexpr (N == kFlat) {
+            if (fresh) return share == 4 ? pull_launch<N, 1, 4, true>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s)
+                                         : pull_launch<N, 1, 2, true>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
+        }
         switch (slabs * 10 + share) {
         case 14: return pull_launch<N, 1, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
         case 12: return pull_launch<N, 1, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
@@ -1310,9 +1334,42 @@ hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::
     sum.columns = p.chunks.first_block(p.chunks.n) * 1024 * slabs;
     sum.stride = p.chunks.blocks * 1024 * slabs;
     sum.n = out.n;
+    sum.fresh = fresh;
     sum.gb = gb;
     hipLaunchKernelGGL(g.ndim == 3 ? sum_group<kVolume> : sum_group<kImage>, dim3(sum.columns / kWave + 1), dim3(1024), 0, s, sum, ws, bias_part);
     return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::Outputs &out, int update, int mask_from,
+                      const View<float> &grads, int first, const int *channels, float *const *gk, float *gb,
+                      float *ws, bool reverse, hipStream_t s)
+{
+    return pull(g, x, grads.p + (int64_t)first * grads.sc, grads.sb, grads.sc, out, update, mask_from, grads, channels, gk, gb, ws,
+                reverse, false, s);
+}
+
+bool layer_pull_supported_3d(const Geom &g, const View<const float> &x, const View<const float> &gy, const View<float> &gx)
+{
+    using namespace group2d;
+    return g.ndim == 3 && g.Wd <= kSlabOut3d && form_of(g, x) == kFlat && form_of(g, gy) == kFlat && gy.sx == 1 &&
+           gy.sc < ((int64_t)1 << 26) && group_pull_supported(g, x, gx);
+}
+
+hipError_t layer_pull_3d(const Geom &g, const View<const float> &x, const View<const float> &gy, const float *k, const View<float> &gx,
+                         float *gk, float *gb, float *ws, hipStream_t s)
+{
+    group2d::Outputs out{};
+    int channels[group2d::kSlabOut3d];
+    float *gks[group2d::kSlabOut3d];
+    for (; out.n < g.Wd; out.n++) {
+        out.dil[out.n] = g.dil;
+        out.k[out.n] = k + (int64_t)out.n * g.C * 27;
+        gks[out.n] = gk + (int64_t)out.n * g.C * 27;
+        channels[out.n] = g.C;
+    }
+    return pull(g, x, gy.p, gy.sb, gy.sc, out, g.C, g.C, gx, channels, gks, gb, ws, false, true, s);
 }
 
 hipError_t group_finish_back(const Geom &g, const View<const float> &x, const View<float> &grads, int channel, int width,

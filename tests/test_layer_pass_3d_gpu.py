@@ -1,0 +1,73 @@
+"""All gradients of a 3D layer of one or two outputs in one pass over its input."""
+import pytest
+import torch
+
+from parity import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def gradients(x, w, b, g, dilation, relu):
+    from msd_pytorch_amd import conv3d
+    leaves = [t.detach().clone().requires_grad_() for t in (x, w, b)]
+    out = torch.empty_like(g)
+    y = (conv3d.conv3d_relu if relu else conv3d.conv3d)(*leaves, out, 1, dilation)
+    return torch.autograd.grad(y, leaves, g)
+
+
+def problem(size, batch, c_in, c_out, seed=11):
+    gen = torch.Generator().manual_seed(seed)
+    x = torch.randn(batch, c_in, *size, generator=gen).cuda()
+    w = (torch.randn(c_out, c_in, 3, 3, 3, generator=gen) * (2.0 / (27 * c_in)) ** 0.5).cuda()
+    return x, w, (torch.randn(c_out, generator=gen) * 0.1).cuda(), torch.randn(batch, c_out, *size, generator=gen).cuda()
+
+
+# Blocks of 16 channels that four or two waves share, one and two chunks of the grid, channels at, below and past a
+# block; volumes of one segment of 32 voxels, of one more, of fewer than a tile, rows shorter than a segment; a
+# dilation of the volume's extent; images that end inside a tile.  Two outputs at any number of channels.
+CASES = [
+    ((2, 4, 4), 1, 12, 1, 1),
+    ((3, 1, 11), 2, 16, 1, 1),
+    ((5, 7, 9), 3, 33, 1, 5),
+    ((4, 6, 32), 1, 16, 1, 4),
+    ((6, 5, 45), 2, 64, 1, 2),
+    ((3, 4, 33), 1, 80, 1, 3),
+    ((9, 11, 13), 2, 1, 2, 9),
+    ((4, 5, 70), 1, 17, 2, 1),
+    ((7, 6, 40), 2, 40, 2, 3),
+    ((3, 5, 37), 1, 130, 2, 2),
+    ((40, 33, 35), 1, 20, 2, 10),
+]
+
+
+@pytest.mark.parametrize("relu", [True, False], ids=["relu", "plain"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[0])) + "-B%d-c%d-w%d-d%d" % c[1:])
+def test_layer_gradients(case, relu):
+    size, batch, c_in, c_out, dilation = case
+    tensors = problem(size, batch, c_in, c_out)
+    got = gradients(*tensors, dilation, relu)
+    # (double precision goes through the shape-generic kernels; a ReLU that is open in one precision only would show)
+    want = gradients(*(t.double() for t in tensors), dilation, relu)
+    for a, b in zip(got, want):
+        assert rel_err(a, b) <= 1e-5
+
+
+@pytest.mark.parametrize("where", ["input", "gradient", "weight"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
+def test_values_without_bf16_parts(where, value):
+    from msd_pytorch_amd import _native
+    lib = _native.load()
+    x, w, b, g = problem((5, 6, 37), 2, 33, 2, seed=13)
+    x, w, g = x.abs() * 1e-3 + 1e-3, w.abs() * 1e-3 + 1e-4, g.abs() * 1e-3 + 1e-4      # (every ReLU open, sums of one sign)
+    {"input": x, "gradient": g, "weight": w}[where].view(-1)[777 % (w.numel() if where == "weight" else g.numel())] = value
+    found = []
+    for path in (1, 0):
+        assert lib.msd_set_kernel_path(path) == 0
+        try:
+            found.append(gradients(x, w, b + 1, g, 2, True))
+        finally:
+            lib.msd_set_kernel_path(0)
+    for want, got in zip(*found):
+        assert torch.equal(torch.isnan(want), torch.isnan(got)) and torch.equal(torch.isinf(want), torch.isinf(got))
+        finite = torch.isfinite(want)
+        assert not bool(finite.any()) or rel_err(got[finite], want[finite]) <= 1e-4
