@@ -31,7 +31,7 @@ namespace py = pybind11;
 
 // The entry points, looked up in the library that the package has loaded.
 #define MSD_ENTRIES(X)                                                                                              \
-    X(msd_last_error) X(msd_conv_forward) X(msd_conv_relu_forward) X(msd_conv_layer_backward) X(msd_workspace_bytes)  \
+    X(msd_last_error) X(msd_conv_forward) X(msd_conv_relu_forward) X(msd_conv_layer_backward) X(msd_conv_layer_workspace_bytes)  \
     X(msd_block_forward_ws) X(msd_block_forward_workspace_bytes) X(msd_block_backward) X(msd_block_workspace_bytes) X(msd_final_forward)                     \
     X(msd_final_backward) X(msd_final_forward_loss) X(msd_final_workspace_bytes) X(msd_scale_fold) X(msd_adam_step)   \
     X(msd_label_check)
@@ -161,8 +161,8 @@ class ConvLayer : public torch::autograd::Function<ConvLayer> {
             Tensor ws;
             int64_t need = 0;
             if (gw.defined() || gb.defined()) {
-                need = lib.msd_workspace_bytes(dtype_of(x), (int)x.dim() - 2, x.size(0), x.size(1), w.size(0),
-                                               x.sizes().data() + 2);
+                need = lib.msd_conv_layer_workspace_bytes(dtype_of(x), (int)x.dim() - 2, x.size(0), x.size(1), w.size(0),
+                                                          x.sizes().data() + 2);
                 ws = workspace(need, x);
             }
             check(lib.msd_conv_layer_backward(

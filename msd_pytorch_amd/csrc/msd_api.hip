@@ -450,11 +450,19 @@ int64_t msd_workspace_bytes(int dtype, int ndim, int64_t batch, int64_t c_in, in
 {
     msd::Geom g;
     if (make_geom("msd_workspace_bytes", dtype, ndim, batch, c_in, c_out, spatial, 1, false, &g) != MSD_OK) return -1;
-    int64_t elems = msd::generic_workspace_elems(g);
+    return msd::generic_workspace_elems(g) * (dtype == MSD_F32 ? 4 : 8);
+}
+
+int64_t msd_conv_layer_workspace_bytes(int dtype, int ndim, int64_t batch, int64_t c_in, int64_t c_out, const int64_t *spatial)
+{
+    const int64_t need = msd_workspace_bytes(dtype, ndim, batch, c_in, c_out, spatial);
+    msd::Geom g;
+    if (need < 0 || dtype != MSD_F32 || ndim != 3 || c_in <= 0 || c_out > msd::group2d::kSlabOut3d ||
+        make_geom("msd_conv_layer_workspace_bytes", dtype, ndim, batch, c_in, c_out, spatial, 1, false, &g) != MSD_OK)
+        return need;
     // (the pass of volume_layer_backward)
-    if (dtype == MSD_F32 && ndim == 3 && c_out <= msd::group2d::kSlabOut3d)
-        elems = std::max(elems, msd::backward_k_mask_floats(g) + msd::group_pull_floats(g.B, (int64_t)g.D * g.H, g.W, g.C));
-    return elems * (dtype == MSD_F32 ? 4 : 8);
+    const int64_t pass = msd::backward_k_mask_floats(g) + msd::group_pull_floats(g.B, (int64_t)g.D * g.H, g.W, g.C);
+    return std::max(need, pass * (int64_t)sizeof(float));
 }
 
 int msd_conv_forward(int dtype, int ndim, int64_t batch, int64_t c_in, int64_t c_out, const int64_t *spatial,
