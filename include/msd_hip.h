@@ -212,8 +212,8 @@ int msd_conv_relu_backward_kb_static(int dtype, int ndim, int64_t batch, int64_t
 /* All gradients of one layer as a differentiated function of its own returns them: grad_input,
  * grad_kernel and grad_bias (each may be NULL) are OVERWRITTEN, so the caller neither clears
  * them nor are they read.  `relu` selects the mask of the conv_relu operators (`output` may be
- * NULL without it); the workspace is msd_conv_layer_workspace_bytes', with which a 3D layer of one or two
- * outputs takes all three in one pass, or msd_workspace_bytes', with which it may take them one after the other.
+ * NULL without it); the workspace is msd_conv_layer_workspace_bytes', with which a layer of up to seven outputs
+ * (3D: two) may take all three in one pass, or msd_workspace_bytes', with which it may take them one after the other.
  * No counterpart in the reference, where an autograd function clears three buffers and calls three
  * operators (conv2d.py:100-123). */
 int64_t msd_conv_layer_workspace_bytes(int dtype, int ndim, int64_t batch, int64_t c_in, int64_t c_out,

@@ -457,10 +457,10 @@ int64_t msd_conv_layer_workspace_bytes(int dtype, int ndim, int64_t batch, int64
 {
     const int64_t need = msd_workspace_bytes(dtype, ndim, batch, c_in, c_out, spatial);
     msd::Geom g;
-    if (need < 0 || dtype != MSD_F32 || ndim != 3 || c_in <= 0 || c_out > msd::group2d::kSlabOut3d ||
+    if (need < 0 || dtype != MSD_F32 || c_in <= 0 || c_out > (ndim == 3 ? msd::group2d::kSlabOut3d : msd::group2d::kSlabOut) ||
         make_geom("msd_conv_layer_workspace_bytes", dtype, ndim, batch, c_in, c_out, spatial, 1, false, &g) != MSD_OK)
         return need;
-    // (the pass of volume_layer_backward)
+    // (the pass of layer_backward_in_one_pass)
     const int64_t pass = msd::backward_k_mask_floats(g) + msd::group_pull_floats(g.B, (int64_t)g.D * g.H, g.W, g.C);
     return std::max(need, pass * (int64_t)sizeof(float));
 }
@@ -625,40 +625,53 @@ int msd_conv_relu_backward_kb(int dtype, int ndim, int64_t batch, int64_t c_in, 
 
 namespace {
 
-// All gradients of a 3D layer of one or two outputs in one pass over its input (msd_pull.hip).  *done is false (and nothing was
+// All gradients of a layer in one pass over its input (msd_pull.hip; up to seven outputs, two in 3D).  *done is false (and nothing was
 // launched) where that is not the faster way or not possible.
-int volume_layer_backward(const char *fn, bool relu, int64_t batch, int64_t c_in, int64_t c_out, const int64_t *spatial, int dilation,
+int layer_backward_in_one_pass(const char *fn, bool relu, int ndim, int64_t batch, int64_t c_in, int64_t c_out, const int64_t *spatial, int dilation,
                           const void *output, const int64_t *os, const void *grad_output, const int64_t *gs, const void *input,
                           const int64_t *xs, const void *kernel, void *grad_input, const int64_t *is, void *grad_kernel, void *grad_bias,
                           void *ws, int64_t ws_bytes, hipStream_t s, bool *done)
 {
     *done = false;
     msd::Geom g;
-    MSD_TRY(make_geom(fn, MSD_F32, 3, batch, c_in, c_out, spatial, dilation, true, &g));
+    MSD_TRY(make_geom(fn, MSD_F32, ndim, batch, c_in, c_out, spatial, dilation, true, &g));
     if (g_kernel_path != 0 || c_in <= 0 || !kernel) return MSD_OK;
-    // Forward and backward of a layer, us, with the operators one after the other and in one pass.  Two outputs: 64^3 over 2 / 32 channels
-    // 54, 49 / 118, 86; 40 x 61 x 75 over 16: 96, 60; 128^3 over 4 / 32: 207, 202 / 457, 327; 90 x 90 x 93 over 60: 469, 278.  One output
-    // leaves half of the matrix rows empty: 128^3 over 18 / 32 / 60: 193, 235 / 287, 281 / 507, 460; where launches and odd
-    // rows cost the operators more it pays from fewer channels on: 40 x 61 x 75 over 16: 65, 50; 61 x 93 x 75 over 12: 84, 71;
-    // 100 x 96 x 96 over 12 / 16: 111, 115 / 126, 116.
-    const bool small = batch * (int64_t)g.nvox <= (int64_t)1 << 20;
-    if (c_out == 1 && c_in < 32 && !(small && c_in >= (g.W % 4 != 0 ? 12 : 16))) return MSD_OK;
+    // Forward and backward of a layer, us, with the operators one after the other and in one pass.
+    const int64_t voxels = batch * (int64_t)g.nvox;
+    bool gains;
+    if (ndim == 2) {
+        // One pass wherever the weight gradient's row kernel does not reach (rows that are not whole groups of four, of more than
+        // 256 lanes): 333 x 477 over 8 / 32 channels 236, 40 / 307, 51; 1021 x 1023 over 32: 591, 142; 10 x 301 over 4: 36,
+        // 28.  Else many of a slab's rows have to be filled, and many channels to share the gather: three outputs, 256 x 256 over 5 / 20
+        // 33, 30 / 43, 35; 4 x 512 x 512 over 5 / 16: 107, 120 / 176, 135; 1024 x 1024 over 32: 264, 178; two, 128 x 128
+        // over 64: 57, 49; 2 x 512 x 512 over 24: 87, 95; 4 x 512 x 512 over 64: 304, 234; one over 64: 225, 217; 1024 x 1024
+        // over 32: 106, 137.
+        const bool no_rows = g.W % 4 != 0 && g.W > (g.W % 2 != 0 ? 256 : 512);
+        gains = no_rows || (c_out >= 3 ? c_in >= 12 || voxels <= (int64_t)1 << 17 : c_in >= (c_out == 2 ? 40 : 64));
+    } else {
+        // Two outputs: 64^3 over 2 / 32 channels 54, 49 / 118, 86; 40 x 61 x 75 over 16: 96, 60; 128^3 over 4 / 32: 207, 202 /
+        // 457, 327; 90 x 90 x 93 over 60: 469, 278.  One output leaves half of the matrix rows empty: 128^3 over 18 / 32 / 60:
+        // 193, 235 / 287, 281 / 507, 460; where launches and odd rows cost the operators more it pays from fewer channels
+        // on: 40 x 61 x 75 over 16: 65, 50; 61 x 93 x 75 over 12: 84, 71; 100 x 96 x 96 over 12 / 16: 111, 115 / 126, 116.
+        gains = c_out > 1 || c_in >= 32 || (voxels <= (int64_t)1 << 20 && c_in >= (g.W % 4 != 0 ? 12 : 16));
+    }
+    if (!gains) return MSD_OK;
     msd::View<const float> o{nullptr, 0, 0, 0, 0, 0}, gy, x;
     msd::View<float> gx;
-    if (relu) MSD_TRY(make_view(fn, "output", 3, output, os, &o));
-    MSD_TRY(make_view(fn, "grad_output", 3, grad_output, gs, &gy));
-    MSD_TRY(make_view(fn, "input", 3, input, xs, &x));
-    MSD_TRY(make_view(fn, "grad_input", 3, grad_input, is, &gx));
+    if (relu) MSD_TRY(make_view(fn, "output", ndim, output, os, &o));
+    MSD_TRY(make_view(fn, "grad_output", ndim, grad_output, gs, &gy));
+    MSD_TRY(make_view(fn, "input", ndim, input, xs, &x));
+    MSD_TRY(make_view(fn, "grad_input", ndim, grad_input, is, &gx));
     if (relu && (o.sx != 1 || gy.sx != 1)) return MSD_OK;
     const int64_t mask = relu ? msd::backward_k_mask_floats(g) : 0;
     const msd::View<const float> m =
         relu ? msd::View<const float>{(const float *)ws, (int64_t)g.Wd * g.nvox, (int64_t)g.nvox, (int64_t)g.H * g.W, (int64_t)g.W, 1} : gy;
-    if (!msd::layer_pull_supported_3d(g, x, m, gx) ||
+    if (!msd::layer_pull_supported(g, x, m, gx) ||
         ws_bytes < (mask + msd::group_pull_floats(g.B, (int64_t)g.D * g.H, g.W, g.C)) * (int64_t)sizeof(float))
         return MSD_OK;
     ProfileScope scope(3, s);
-    hipError_t e = relu ? msd::mask_gradient_3d(g, o, gy, (float *)ws, s) : hipSuccess;
-    if (e == hipSuccess) e = msd::layer_pull_3d(g, x, m, (const float *)kernel, gx, (float *)grad_kernel, (float *)grad_bias, (float *)ws + mask, s);
+    hipError_t e = relu ? msd::masked_gradient(g, o, gy, (float *)ws, s) : hipSuccess;
+    if (e == hipSuccess) e = msd::layer_pull(g, x, m, (const float *)kernel, gx, (float *)grad_kernel, (float *)grad_bias, (float *)ws + mask, s);
     if (e != hipSuccess) return hip_fail(fn, e);
     *done = true;
     return MSD_OK;
@@ -679,8 +692,8 @@ int msd_conv_layer_backward(int relu, int dtype, int ndim, int64_t batch, int64_
     const char *fn = "conv_layer_backward";
     if (!grad_input && !grad_kernel && !grad_bias) return fail(MSD_ERR_INVALID, "%s: no gradient buffer given", fn);
     bool done = false;
-    if (grad_input && grad_kernel && grad_bias && dtype == MSD_F32 && ndim == 3 && c_out <= 2 && workspace)
-        MSD_TRY(volume_layer_backward(fn, relu != 0, batch, c_in, c_out, spatial, dilation, output, output_strides, grad_output,
+    if (grad_input && grad_kernel && grad_bias && dtype == MSD_F32 && c_out <= msd::group2d::kSlabOut && workspace)
+        MSD_TRY(layer_backward_in_one_pass(fn, relu != 0, ndim, batch, c_in, c_out, spatial, dilation, output, output_strides, grad_output,
                                       grad_output_strides, input, input_strides, kernel, grad_input, grad_input_strides, grad_kernel,
                                       grad_bias, workspace, workspace_bytes, (hipStream_t)stream, &done));
     if (done) return MSD_OK;

@@ -15,7 +15,7 @@ bool fast_backward_kb_supported_3d(const Geom &g, bool relu, const View<const fl
     return bwdk::supported_nd<3>(g, relu, out, gy, x);
 }
 
-hipError_t mask_gradient_3d(const Geom &g, const View<const float> &out, const View<const float> &gy, float *m, hipStream_t s)
+hipError_t masked_gradient(const Geom &g, const View<const float> &out, const View<const float> &gy, float *m, hipStream_t s)
 {
     const int64_t total = (int64_t)g.B * g.Wd * g.nvox;
     const int blocks = (int)std::min<int64_t>((total + 255) / 256, 4096);
@@ -32,7 +32,7 @@ hipError_t fast_backward_kb_3d(const Geom &g, bool relu, const View<const float>
             relu ? View<const float>{ws, (int64_t)g.Wd * g.nvox, (int64_t)g.nvox, (int64_t)g.H * g.W, (int64_t)g.W, 1} : gy;
         if (fast_backward_k_only_supported_3d(g, m, x)) {
             if (relu) {
-                const hipError_t e = mask_gradient_3d(g, out, gy, ws, s);
+                const hipError_t e = masked_gradient(g, out, gy, ws, s);
                 if (e != hipSuccess) return e;
             }
             return fast_backward_k_only_3d(g, m, x, gk, gb, ws, s);

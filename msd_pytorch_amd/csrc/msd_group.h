@@ -91,11 +91,11 @@ hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::
                       const View<float> &grads, int first, const int *channels, float *const *gk, float *gb,
                       float *ws, bool reverse, hipStream_t s);
 
-// All three gradients of a single layer (g.Wd <= 2 outputs of dilation g.dil) over a volume without gaps, written and not added
-// to.  gy: the masked output gradient, without gaps in an image.  ws: group_pull_floats floats.
-bool layer_pull_supported_3d(const Geom &g, const View<const float> &x, const View<const float> &gy, const View<float> &gx);
-hipError_t layer_pull_3d(const Geom &g, const View<const float> &x, const View<const float> &gy, const float *k, const View<float> &gx,
-                         float *gk, float *gb, float *ws, hipStream_t s);
+// All three gradients of a single layer (of dilation g.dil; g.Wd outputs of one slab) over an image, or a volume without gaps,
+// written and not added to.  gy: the masked output gradient, rows as in x.  ws: group_pull_floats floats.
+bool layer_pull_supported(const Geom &g, const View<const float> &x, const View<const float> &gy, const View<float> &gx);
+hipError_t layer_pull(const Geom &g, const View<const float> &x, const View<const float> &gy, const float *k, const View<float> &gx,
+                      float *gk, float *gb, float *ws, hipStream_t s);
 
 // Completes the gradient of the `width` channels from `channel` on: adds what the outputs right
 // above them (`above`, their weights of these channels) contribute, and applies the ReLU mask.

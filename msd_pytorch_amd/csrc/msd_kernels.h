@@ -171,7 +171,7 @@ hipError_t fast_backward_kb_3d(const Geom &g, bool relu, const View<const float>
                                const View<const float> &x, float *gk, float *gb, float *ws, hipStream_t s);
 
 // The masked output gradient, without gaps: m[b][co][voxel].
-hipError_t mask_gradient_3d(const Geom &g, const View<const float> &out, const View<const float> &gy, float *m, hipStream_t s);
+hipError_t masked_gradient(const Geom &g, const View<const float> &out, const View<const float> &gy, float *m, hipStream_t s);
 inline bool fast_backward_kb_supported(const Geom &g, bool relu, const View<const float> &out,
                                        const View<const float> &gy, const View<const float> &x)
 {

@@ -1281,8 +1281,8 @@ bool group_pull_supported(const Geom &g, const View<const float> &x, const View<
 
 namespace {
 
-// gy: the outputs' gradients, channels gsc apart, rows as in x.  fresh: the gradients are written, not added to (volumes
-// without gaps, at most two outputs).
+// gy: the outputs' gradients, channels gsc apart, rows as in x.  fresh: the gradients are written, not added to (one slab;
+// images, volumes without gaps).
 hipError_t pull(const Geom &g, const View<const float> &x, const float *gy, int64_t gsb, int64_t gsc, const group2d::Outputs &out,
                 int update, int mask_from, const View<float> &grads, const int *channels, float *const *gk, float *gb, float *ws,
                 bool reverse, bool fresh, hipStream_t s)
@@ -1290,7 +1290,7 @@ hipError_t pull(const Geom &g, const View<const float> &x, const float *gy, int6
     using namespace group2d;
     const int per_slab = g.ndim == 3 ? kSlabOut3d : kSlabOut;
     const Form form = form_of(g, x);
-    if (out.n < 1 || out.n > 2 * per_slab || !group_pull_supported(g, x, grads) || (fresh && (form != kFlat || out.n > kSlabOut3d)))
+    if (out.n < 1 || out.n > 2 * per_slab || !group_pull_supported(g, x, grads) || (fresh && (form == kVolume || out.n > per_slab)))
         return hipErrorInvalidValue;
     const int slabs = out.n > per_slab ? 2 : 1;
     const int span = form == kFlat ? g.nvox : g.W, rows = g.nvox / span;
@@ -1310,7 +1310,7 @@ hipError_t pull(const Geom &g, const View<const float> &x, const float *gy, int6
     const int share = p.chunks.blocks <= 2 ? 4 : p.chunks.blocks <= 4 ? 2 : 1;
     auto launch = [&](auto f) {
         constexpr int N = decltype(f)::value;
-        if constexpr (N == kFlat) {
+        if constexpr (N != kVolume) {
             if (fresh) return share == 4 ? pull_launch<N, 1, 4, true>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s)
                                          : pull_launch<N, 1, 2, true>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
         }
@@ -1350,23 +1350,25 @@ hipError_t group_pull(const Geom &g, const View<const float> &x, const group2d::
                 reverse, false, s);
 }
 
-bool layer_pull_supported_3d(const Geom &g, const View<const float> &x, const View<const float> &gy, const View<float> &gx)
+bool layer_pull_supported(const Geom &g, const View<const float> &x, const View<const float> &gy, const View<float> &gx)
 {
     using namespace group2d;
-    return g.ndim == 3 && g.Wd <= kSlabOut3d && form_of(g, x) == kFlat && form_of(g, gy) == kFlat && gy.sx == 1 &&
-           gy.sc < ((int64_t)1 << 26) && group_pull_supported(g, x, gx);
+    const bool rows = g.ndim == 3 ? form_of(g, x) == kFlat && form_of(g, gy) == kFlat : x.sy == gy.sy;
+    return g.Wd <= (g.ndim == 3 ? kSlabOut3d : kSlabOut) && rows && gy.sx == 1 && gy.sc < ((int64_t)1 << 26) &&
+           group_pull_supported(g, x, gx);
 }
 
-hipError_t layer_pull_3d(const Geom &g, const View<const float> &x, const View<const float> &gy, const float *k, const View<float> &gx,
-                         float *gk, float *gb, float *ws, hipStream_t s)
+hipError_t layer_pull(const Geom &g, const View<const float> &x, const View<const float> &gy, const float *k, const View<float> &gx,
+                      float *gk, float *gb, float *ws, hipStream_t s)
 {
     group2d::Outputs out{};
-    int channels[group2d::kSlabOut3d];
-    float *gks[group2d::kSlabOut3d];
+    int channels[group2d::kSlabOut];
+    float *gks[group2d::kSlabOut];
+    const int64_t weights = (int64_t)g.C * (g.ndim == 3 ? 27 : group2d::kTaps);
     for (; out.n < g.Wd; out.n++) {
         out.dil[out.n] = g.dil;
-        out.k[out.n] = k + (int64_t)out.n * g.C * 27;
-        gks[out.n] = gk + (int64_t)out.n * g.C * 27;
+        out.k[out.n] = k + out.n * weights;
+        gks[out.n] = gk + out.n * weights;
         channels[out.n] = g.C;
     }
     return pull(g, x, gy.p, gy.sb, gy.sc, out, g.C, g.C, gx, channels, gks, gb, ws, false, true, s);

@@ -1,4 +1,4 @@
-"""All gradients of a 3D layer of one or two outputs in one pass over its input."""
+"""All gradients of a layer in one pass over its input (up to seven outputs, two in 3D)."""
 import pytest
 import torch
 
@@ -8,23 +8,29 @@ pytestmark = pytest.mark.gpu
 
 
 def gradients(x, w, b, g, dilation, relu):
-    from msd_pytorch_amd import conv3d
+    from msd_pytorch_amd import conv2d, conv3d
+    if x.dim() == 4:
+        fn = conv2d.conv2d_relu if relu else conv2d.conv2d
+    else:
+        fn = conv3d.conv3d_relu if relu else conv3d.conv3d
     leaves = [t.detach().clone().requires_grad_() for t in (x, w, b)]
     out = torch.empty_like(g)
-    y = (conv3d.conv3d_relu if relu else conv3d.conv3d)(*leaves, out, 1, dilation)
+    y = fn(*leaves, out, 1, dilation)
     return torch.autograd.grad(y, leaves, g)
 
 
 def problem(size, batch, c_in, c_out, seed=11):
     gen = torch.Generator().manual_seed(seed)
     x = torch.randn(batch, c_in, *size, generator=gen).cuda()
-    w = (torch.randn(c_out, c_in, 3, 3, 3, generator=gen) * (2.0 / (27 * c_in)) ** 0.5).cuda()
+    taps = [3] * len(size)
+    w = (torch.randn(c_out, c_in, *taps, generator=gen) * (2.0 / (3 ** len(size) * c_in)) ** 0.5).cuda()
     return x, w, (torch.randn(c_out, generator=gen) * 0.1).cuda(), torch.randn(batch, c_out, *size, generator=gen).cuda()
 
 
 # Blocks of 16 channels that four or two waves share, one and two chunks of the grid, channels at, below and past a
 # block; volumes of one segment of 32 voxels, of one more, of fewer than a tile, rows shorter than a segment; a
-# dilation of the volume's extent; images that end inside a tile.  Two outputs at any number of channels.
+# dilation of the volume's extent; images that end inside a tile.  Two outputs at any number of channels.  2D: odd rows
+# of more than 256 voxels and even ones of more than 512, one to seven outputs, from 64, 40 and 12 channels on, or small.
 CASES = [
     ((2, 4, 4), 1, 12, 1, 1),
     ((3, 1, 11), 2, 16, 1, 1),
@@ -37,6 +43,18 @@ CASES = [
     ((7, 6, 40), 2, 40, 2, 3),
     ((3, 5, 37), 1, 130, 2, 2),
     ((40, 33, 35), 1, 20, 2, 10),
+    ((3, 257), 2, 1, 1, 3),
+    ((9, 259), 1, 17, 2, 1),
+    ((5, 514), 2, 33, 1, 5),
+    ((7, 1021), 1, 7, 1, 2),
+    ((6, 32), 3, 64, 1, 6),
+    ((4, 45), 2, 40, 2, 1),
+    ((33, 35), 1, 3, 3, 10),
+    ((12, 70), 2, 12, 4, 12),
+    ((5, 96), 1, 70, 5, 2),
+    ((8, 50), 2, 20, 6, 3),
+    ((4, 33), 1, 1, 7, 1),
+    ((40, 64), 1, 130, 7, 7),
 ]
 
 
@@ -48,16 +66,21 @@ def test_layer_gradients(case, relu):
     got = gradients(*tensors, dilation, relu)
     # (double precision goes through the shape-generic kernels; a ReLU that is open in one precision only would show)
     want = gradients(*(t.double() for t in tensors), dilation, relu)
-    for a, b in zip(got, want):
+    for a, b in zip(got[:2], want[:2]):
         assert rel_err(a, b) <= 1e-5
+    # the bias gradient is a sum of terms of both signs, in chains and trees of fewer than 64 additions here: each
+    # rounds to 2^-24 of at most the sum of the terms' sizes
+    terms = tensors[3].double().abs().sum(dim=[0, *range(2, tensors[3].dim())])
+    assert bool(((got[2] - want[2]).abs() <= 64 * 2.0 ** -24 * terms).all())
 
 
 @pytest.mark.parametrize("where", ["input", "gradient", "weight"])
 @pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
-def test_values_without_bf16_parts(where, value):
+@pytest.mark.parametrize("size", [(5, 6, 37), (13, 259)], ids=str)
+def test_values_without_bf16_parts(size, where, value):
     from msd_pytorch_amd import _native
     lib = _native.load()
-    x, w, b, g = problem((5, 6, 37), 2, 33, 2, seed=13)
+    x, w, b, g = problem(size, 2, 33, 2, seed=13)
     x, w, g = x.abs() * 1e-3 + 1e-3, w.abs() * 1e-3 + 1e-4, g.abs() * 1e-3 + 1e-4      # (every ReLU open, sums of one sign)
     {"input": x, "gradient": g, "weight": w}[where].view(-1)[777 % (w.numel() if where == "weight" else g.numel())] = value
     found = []
