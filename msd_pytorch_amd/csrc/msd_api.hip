@@ -642,12 +642,13 @@ int layer_backward_in_one_pass(const char *fn, bool relu, int ndim, int64_t batc
     if (ndim == 2) {
         // One pass wherever the weight gradient's row kernel does not reach (rows that are not whole groups of four, of more than
         // 256 lanes): 333 x 477 over 8 / 32 channels 236, 40 / 307, 51; 1021 x 1023 over 32: 591, 142; 10 x 301 over 4: 36,
-        // 28.  Else many of a slab's rows have to be filled, and many channels to share the gather: three outputs, 256 x 256 over 5 / 20
-        // 33, 30 / 43, 35; 4 x 512 x 512 over 5 / 16: 107, 120 / 176, 135; 1024 x 1024 over 32: 264, 178; two, 128 x 128
+        // 28.  Else many of a slab's rows have to be filled, and many channels to share the gather: three outputs, 64 x 83 over 3: 24,
+        // 27; 256 x 256 over 5 / 20 33, 30 / 43, 35; 4 x 512 x 512 over 5 / 16: 107, 120 / 176, 135; 1024 x 1024 over 32: 264, 178; two, 128 x 128
         // over 64: 57, 49; 2 x 512 x 512 over 24: 87, 95; 4 x 512 x 512 over 64: 304, 234; one over 64: 225, 217; 1024 x 1024
         // over 32: 106, 137.
+        const bool middle = voxels >= (int64_t)1 << 14 && voxels <= (int64_t)1 << 17;
         const bool no_rows = g.W % 4 != 0 && g.W > (g.W % 2 != 0 ? 256 : 512);
-        gains = no_rows || (c_out >= 3 ? c_in >= 12 || voxels <= (int64_t)1 << 17 : c_in >= (c_out == 2 ? 40 : 64));
+        gains = no_rows || (c_out >= 3 ? c_in >= 12 || (middle && c_in >= 4) : c_in >= (c_out == 2 ? 40 : 64));
     } else {
         // Two outputs: 64^3 over 2 / 32 channels 54, 49 / 118, 86; 40 x 61 x 75 over 16: 96, 60; 128^3 over 4 / 32: 207, 202 /
         // 457, 327; 90 x 90 x 93 over 60: 469, 278.  One output leaves half of the matrix rows empty: 128^3 over 18 / 32 / 60:

@@ -124,6 +124,29 @@ def test_block_backward_of_volumes_in_groups(case, input_grad):
         check_block(3, size, c_in, width, depth, batch, dilations=dilations, seed=67, input_grad=input_grad)
 
 
+# Layers of one and two channels in one group: seven outputs above a layer of one, one output above a layer of two (3D: in a
+# volume with and without gaps), against the layers on their own.
+@pytest.mark.parametrize("size,widths,gap", [((9, 37), [1, 1, 2, 2, 2, 2, 2, 2], 0), ((4, 5, 37), [2, 1], 0), ((4, 5, 37), [2, 1], 3),
+                                             ((5, 4, 33), [1, 2, 1], 0)], ids=str)
+def test_backward_groups_of_mixed_widths(size, widths, gap):
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator().manual_seed(73)
+    c_in, channels = 3, 3 + sum(widths)
+    big = torch.randn(2, 2, channels, *size[:-1], size[-1] + gap, generator=gen).cuda()
+    stack, gradient = big[0][..., :size[-1]], big[1][..., :size[-1]]
+    reads = [c_in + sum(widths[:i]) for i in range(len(widths))]
+    weights = [torch.randn(w, c, *([3] * len(size)), generator=gen).cuda() * 0.1 for w, c in zip(widths, reads)]
+    found = []
+    for setting in (0, 1):
+        g = torch.empty_strided(gradient.shape, gradient.stride(), device="cuda").copy_(gradient)
+        gk, gb = [torch.zeros_like(w) for w in weights], torch.zeros(channels - c_in).cuda()
+        with tuning({"bwd.group": setting}):
+            cc.block_backward(stack, g, c_in, [1 + i % 4 for i in range(len(widths))], weights, gk, gb, True)
+        found.append((g[:, :c_in], gb, *gk))
+    for a, b in zip(*found):
+        assert rel_err(b, a) <= 1e-5
+
+
 # A volume without gaps is taken as one row, any other by its rows (of 32 voxels at least): the same gradients from
 # rows with gaps, from slices with gaps and from slices and rows in the other order.
 @pytest.mark.parametrize("layout", ["rows", "slices", "transposed"])

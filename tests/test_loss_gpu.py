@@ -84,7 +84,7 @@ def test_fused_loss_every_form_of_the_single_read_kernel(c_in, spatial, c_out, k
 # Planes that are no whole groups of four (two above 64 channels) voxels: of every remainder, of fewer voxels than a
 # group, one more and one less than a tile, the last lane's voxels moved left in a tile of its own.
 @pytest.mark.parametrize("kind", ["mse", "l1", "nll"])
-@pytest.mark.parametrize("c_in,c_out", [(7, 3), (33, 1), (70, 2), (101, 4)])
+@pytest.mark.parametrize("c_in,c_out", [(7, 3), (9, 2), (33, 1), (70, 2), (101, 4)])
 @pytest.mark.parametrize("spatial", [(1, 1), (1, 2), (1, 3), (1, 5), (3, 21), (1, 129), (5, 51), (1, 257), (2, 129), (7, 37), (31, 47)], ids=str)
 def test_fused_loss_of_odd_planes(spatial, c_in, c_out, kind):
     check_fused_loss(3, c_in, c_out, spatial, kind, torch.float32)
