@@ -26,11 +26,12 @@ HBM_PEAK_GBS = 8000.0
 # fp32 peak of MI355X (matrix cores, or packed vector instructions); plain (non-packed) vector
 # fp32, which the build rules leave to the forward kernel's multiply-adds, peaks at half of it
 FP32_PEAK_TFLOPS = 157.3
-PIPE = {"forward": "fp32 VALU, non-packed (78.6 TFLOP/s of the 157.3 peak); 2D layer groups: fp32 MFMA 16x16x4",
+PIPE = {"forward": "fp32 VALU, non-packed (78.6 TFLOP/s of the 157.3 peak); 2D layer groups: fp32 MFMA 16x16x4, "
+                   "of fourteen outputs bf16 MFMA 16x16x32 (six products of bf16 parts per fp32 product)",
         "backward_x": "fp32 VALU, non-packed (78.6 TFLOP/s of the 157.3 peak)",
         "backward_kb": "fp32 MFMA 16x16x4",
         "backward_xkb": "fp32 MFMA 16x16x4 (weight gradient) + fp32 VALU (input gradient), half of the flops each; "
-                        "2D layer groups: both on the MFMA"}
+                        "layer groups: both as six bf16 MFMA 16x16x32 products of bf16 parts per fp32 product"}
 
 # kernel families (as named in the profile summaries) whose HBM traffic belongs to a class
 FAMILIES = {"forward": ("fwd_lattice", "push_rows", "push_table", "push_split", "finish_rows"),

@@ -76,8 +76,8 @@ int msd_set_kernel_path(int path);
  * workgroups take every n-th row group), "block.fuse" (0/1: fused backward in the block),
  * "block.defer" (0/1: one reduction launch for many layers), "block.snake" (0/1: alternate
  * layers walk the channels in opposite directions), "fwd.class3d" (0/1: 3D forward tiles
- * numbered by residue class), "fwd.lattice3d" (24, 33 or 44: rows z x y of a 3D forward tile;
- * 0: chosen by the library), "block.pair" (0/1: the backward pass of a 2D block of one-channel
+ * numbered by residue class), "fwd.lattice3d" (24, 33 or 44: rows z x y of a 3D forward tile,
+ * 44 with all channels in one group; 0: chosen by the library), "block.pair" (0/1: the backward pass of a 2D block of one-channel
  * layers takes its layers two or three at a time), "block.triple" (0: never three at a time,
  * n > 0: three where the layers share at least n channels; 32 by default), "final.tiled" (0/1:
  * msd_final_forward_loss reads the stack once, through LDS tiles, where it can: fp32, up to 128
@@ -90,7 +90,10 @@ int msd_set_kernel_path(int path);
  * a 3D layer of one or two output channels runs on the weight-gradient-only form of the fused
  * backward kernel where that takes the shape; 0: on the separate weight-gradient kernels),
  * "bwdx.lean1" (0/1: a 3D backward_x over one input and one output channel runs on a kernel
- * of its own; 0: on the general one).
+ * of its own; 0: on the general one), "fwd.group" and "bwd.group" (0: the block's layers in no
+ * groups; n > 0: groups from n channels in front of, or below, them on; "fwd.group" from 1024 on: groups of
+ * up to fourteen outputs from n - 1024 channels on).  A value set for "block.pair" or "block.triple" (2D),
+ * "block.split3d" or "block.chainpair" (3D) takes the place of the backward groups.
  * Unknown keys return MSD_ERR_INVALID.
  */
 int msd_set_tuning(const char *key, int value);
