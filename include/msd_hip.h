@@ -91,9 +91,9 @@ int msd_set_kernel_path(int path);
  * backward kernel where that takes the shape; 0: on the separate weight-gradient kernels),
  * "bwdx.lean1" (0/1: a 3D backward_x over one input and one output channel runs on a kernel
  * of its own; 0: on the general one), "fwd.group" and "bwd.group" (0: the block's layers in no
- * groups; n > 0: groups from n channels in front of, or below, them on; "fwd.group" from 1024 on: groups of
- * up to fourteen outputs from n - 1024 channels on).  A value set for "block.pair" or "block.triple" (2D),
- * "block.split3d" or "block.chainpair" (3D) takes the place of the backward groups.
+ * groups; n > 0: groups from n channels in front of, or below, them on; the forward one from 1024 on: groups of
+ * up to fourteen outputs from n - 1024 channels on).  A value set for one of the block's pair, triple (2D),
+ * split3d and chainpair (3D) settings takes the place of the backward groups.
  * Unknown keys return MSD_ERR_INVALID.
  */
 int msd_set_tuning(const char *key, int value);
