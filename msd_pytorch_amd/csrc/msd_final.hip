@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <initializer_list>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -48,6 +49,25 @@ __device__ __forceinline__ void store_elems(T *p, const T (&d)[V])
         for (int i = 0; i < V; i++) v[i] = d[i];
         *reinterpret_cast<typename VecOf<T, V>::type *>(p) = v;
     }
+}
+
+// V floats at any multiple of four bytes (images of odd size: every channel begins elsewhere).  3 x 333 x 477, 35
+// channels, three labels: 66 us with one voxel per lane, the widest aligned access, 42 with four; 61 x 93 x 75, 21 channels: 35 and 15.
+template <int V> __device__ __forceinline__ void load_unaligned(uint64_t base, uint32_t byte_offset, float (&d)[V])
+{
+    typedef float vec_t __attribute__((ext_vector_type(V), aligned(4)));
+    typedef const __attribute__((address_space(1))) char *gbytes_t;
+    const vec_t v = *reinterpret_cast<const __attribute__((address_space(1))) vec_t *>(reinterpret_cast<gbytes_t>(base) + byte_offset);
+#pragma unroll
+    for (int i = 0; i < V; i++) d[i] = v[i];
+}
+template <int V> __device__ __forceinline__ void store_unaligned(float *p, const float (&d)[V])
+{
+    typedef float vec_t __attribute__((ext_vector_type(V), aligned(4)));
+    vec_t v;
+#pragma unroll
+    for (int i = 0; i < V; i++) v[i] = d[i];
+    *reinterpret_cast<vec_t *>(p) = v;
 }
 
 template <typename T>
@@ -167,6 +187,41 @@ __global__ __launch_bounds__(kFinalThreads) void final_backward_kernel(int64_t n
                 if (lane == 0 && o0 + o < c_out) part[((int64_t)(o0 + o) * C + c) * rows + row] = s;
             }
         }
+    }
+}
+
+// grad_input alone (fp32): nothing is read but the output gradients, all outputs at once, four voxels per lane at any
+// address; the last lane's are moved left (what they share with the lane before is written twice, the same).  Bound by the
+// stores.  3 x 333 x 477, three outputs to 35 channels: 41 us in launches of two outputs and of one with a voxel per
+// lane, 13 so; 1024 x 1024, four outputs to 101 channels: 71 and 64 (6.6 TB/s); 61 x 93 x 75, one to 21: 9.9 and 7.8.
+template <int MAXO>
+__global__ __launch_bounds__(kFinalThreads) void final_backward_write(int64_t nvox, int C, int c_out, const float *__restrict__ go,
+                                                                      int64_t gsb, int64_t gsc, const float *__restrict__ w,
+                                                                      float *__restrict__ gx, int64_t gxsb, int64_t gxsc)
+{
+    constexpr int V = 4;
+    const int64_t i = ((int64_t)blockIdx.x * kFinalThreads + threadIdx.x) * V;
+    if (i >= nvox) return;
+    const int64_t first = min(i, nvox - V);
+    typedef const __attribute__((address_space(4))) float *const_floats_t;
+    const const_floats_t wk = (const_floats_t)(uintptr_t)w;
+    float g[MAXO][V];
+#pragma unroll
+    for (int o = 0; o < MAXO; o++) {
+        load_unaligned<V>(reinterpret_cast<uint64_t>(go + blockIdx.y * gsb + min(o, c_out - 1) * gsc + first), 0, g[o]);
+    }
+    float *gp = gx + blockIdx.y * gxsb + first;
+#pragma unroll 4
+    for (int c = 0; c < C; c++) {
+        float r[V] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int o = 0; o < MAXO; o++) {
+            if (o >= c_out) break;                // uniform
+            const float wv = wk[(int64_t)o * C + c];
+#pragma unroll
+            for (int e = 0; e < V; e++) r[e] += wv * g[o][e];
+        }
+        store_unaligned<V>(gp + c * gxsc, r);
     }
 }
 
@@ -304,25 +359,6 @@ __global__ __launch_bounds__(kFinalThreads) void final_forward_loss_kernel(
 constexpr int kTiledWaves = 8;
 constexpr int kTiledThreads = kTiledWaves * kWave;
 constexpr int kTiledMaxChannels = 128;
-
-// V floats at any multiple of four bytes (images of odd size: every channel begins elsewhere).  3 x 333 x 477, 35
-// channels, three labels: 66 us with one voxel per lane, the widest aligned access, 42 with four; 61 x 93 x 75, 21 channels: 35 and 15.
-template <int V> __device__ __forceinline__ void load_unaligned(uint64_t base, uint32_t byte_offset, float (&d)[V])
-{
-    typedef float vec_t __attribute__((ext_vector_type(V), aligned(4)));
-    typedef const __attribute__((address_space(1))) char *gbytes_t;
-    const vec_t v = *reinterpret_cast<const __attribute__((address_space(1))) vec_t *>(reinterpret_cast<gbytes_t>(base) + byte_offset);
-#pragma unroll
-    for (int i = 0; i < V; i++) d[i] = v[i];
-}
-template <int V> __device__ __forceinline__ void store_unaligned(float *p, const float (&d)[V])
-{
-    typedef float vec_t __attribute__((ext_vector_type(V), aligned(4)));
-    vec_t v;
-#pragma unroll
-    for (int i = 0; i < V; i++) v[i] = d[i];
-    *reinterpret_cast<vec_t *>(p) = v;
-}
 
 template <int V, int MAXO, int KIND, int CC>
 __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
@@ -656,6 +692,17 @@ hipError_t final_backward(int64_t batch, int c_in, int c_out, int64_t nvox, cons
     const int64_t rows = (int64_t)grid.x * batch * (kFinalThreads / kWave);
     if (!gw && !gb) ws = nullptr;                 // no sums over voxels wanted: no partial sums, no second pass
     if (!ws && !gx) return hipSuccess;
+    if constexpr (std::is_same<T, float>::value) {
+        if (!ws && c_out <= 8 && nvox >= 4) {
+            const dim3 wgs((unsigned)(((nvox + 3) / 4 + kFinalThreads - 1) / kFinalThreads), (unsigned)batch, 1);
+#define MSD_FINAL_WRITE(OO)                                                                                             \
+    hipLaunchKernelGGL(final_backward_write<OO>, wgs, dim3(kFinalThreads), 0, s, nvox, c_in, c_out, go, gsb, gsc, w, gx, \
+                       gxsb, gxsc)
+            if (c_out > 4) MSD_FINAL_WRITE(8); else if (c_out > 2) MSD_FINAL_WRITE(4); else if (c_out > 1) MSD_FINAL_WRITE(2); else MSD_FINAL_WRITE(1);
+#undef MSD_FINAL_WRITE
+            return hipGetLastError();
+        }
+    }
     for (int o0 = 0; o0 < c_out;) {
         const int gwd = group_width(c_out - o0);
 #define MSD_FINAL_BWD(VV, OO)                                                                                        \

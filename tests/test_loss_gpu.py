@@ -90,6 +90,27 @@ def test_fused_loss_of_odd_planes(spatial, c_in, c_out, kind):
     check_fused_loss(3, c_in, c_out, spatial, kind, torch.float32)
 
 
+# grad_input alone: planes of every remainder modulo four, of fewer voxels than four, of more than a workgroup covers, one to
+# nine outputs (more than eight go in passes); an infinite weight meets its own output only.
+@pytest.mark.parametrize("c_out", [1, 2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("spatial", [(1, 3), (2, 2), (1, 5), (7, 9), (37, 53), (33, 32)], ids=str)
+def test_input_gradient_of_the_final_layer_alone(spatial, c_out):
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator().manual_seed(c_out)
+    g = torch.randn(2, c_out, *spatial, generator=gen).abs() + 0.1
+    w = torch.randn(c_out, 11, generator=gen)
+    w[c_out - 1, 4] = float("inf")
+    stack = torch.zeros(2, 13, *spatial).cuda()
+    gx = stack[:, 1:12]
+    cc.final_backward(None, g.cuda(), w.cuda(), gx, None, None)
+    want = (w.double()[None, :, :, None, None] * g.double()[:, :, None]).sum(1)
+    assert bool(torch.isposinf(gx[:, 4]).all()) and bool((stack[:, ::12] == 0).all())
+    keep = [c for c in range(11) if c != 4]
+    # (nine products and sums in single precision)
+    bound = 10 * 2.0 ** -24 * (w[:, keep].double().abs()[None, :, :, None, None] * g.double()[:, :, None]).sum(1)
+    assert bool(((gx[:, keep].cpu().double() - want[:, keep]).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("kind", ["mse", "l1", "nll"])
 @pytest.mark.parametrize("batch,c_in,c_out,spatial", CASES)
 def test_fused_loss_walking_the_stack_twice_matches_torch(batch, c_in, c_out, spatial, kind):
