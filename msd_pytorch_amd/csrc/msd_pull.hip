@@ -147,11 +147,6 @@ __device__ __forceinline__ void tile_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-__device__ __forceinline__ float part_value(const char *p)        // one bf16 in LDS
-{
-    return (float)*reinterpret_cast<const __bf16 *>(p);
-}
-
 // The sources of one voxel (or row) u of an axis of n through the outer taps of dilation d
 // (adjoint_sources): `up` is read by tap 0 where it lies inside and is otherwise the mirrored source of
 // tap 2, `down` the other way round, so that two loads hold all of them.
@@ -415,12 +410,11 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         // -A at every second voxel: the sums of the bf16 instruction are cut off towards minus infinity, which adds up
         // over an image where the gradients themselves cancel (bias gradients: an error of 2e-6 instead of 1.2e-7).
         // For the same reason x changes its sign with the voxel and from tile to tile.
-        const uint32_t odd = (uint32_t)v << 31;
+        const float factor = (v % 2 ? -1.f : 1.f) * (WHOLE ? 1.f : kSplitScale);
 #pragma unroll
         for (int j = 0; j < kLaneOut; j++)
 #pragma unroll
-            for (int t = 0; t < kTaps; t++)
-                val[j][t / 3][t % 3] = __uint_as_float(__float_as_uint(val[j][t / 3][t % 3]) ^ odd);
+            for (int t = 0; t < kTaps; t++) val[j][t / 3][t % 3] *= factor;
         // rows m of the lane (slot_of), eight at a time
         auto eight = [&](int i, float (&e8)[8]) {
 #pragma unroll
@@ -444,22 +438,19 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             float e8[8];
             eight(i, e8);
             Split8 s;
-            bad += split8(e8, s);
+            if constexpr (WHOLE) {
+                float scaled[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) scaled[e] = e8[e] * kSplitScale;
+                bad += split8(scaled, s);
+                put_whole(e8, s);
+            } else {
+                bad += split8(e8, s);
+            }
 #pragma unroll
             for (int k = 0; k < 3; k++) *reinterpret_cast<bf16x8_t *>(at + k * kPartBytes + (piece ^ 16 * i)) = s.p[k];
         }
-        const bool any = __any(bad != bad);
-        if (any) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float e8[8];
-                eight(i, e8);
-                Split8 s;
-                split_any(e8, s);
-#pragma unroll
-                for (int k = 0; k < 3; k++) *reinterpret_cast<bf16x8_t *>(at + k * kPartBytes + (piece ^ 16 * i)) = s.p[k];
-            }
-        }
+        const bool any = __any(taken_whole(bad));
         if (lane == 0) shared.bad_tile[wave] = any;
     };
 
@@ -489,17 +480,24 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         }
         return bits;
     };
-    // x in parts to the wave's own space; NaN where a value cannot be split
-    auto signed_x = [&](int i, int e, uint32_t sign) {
-        return __uint_as_float(__float_as_uint(xs[i][e]) ^ (sign ^ (uint32_t)(e % 2) << 31));
+    // x in parts to the wave's own space; not finite where a value cannot be split
+    // (factors for the even and the odd voxels, in registers of their own: a sign in the instruction doubles its size)
+    struct Factors {
+        uint32_t even, odd;
+        __device__ explicit Factors(float f, uint32_t sign = 0) : even(__float_as_uint(f) | sign), odd(even ^ 0x80000000u)
+        {
+            asm volatile("" : "+s"(even), "+s"(odd));
+        }
+        __device__ float of(int e) const { return __uint_as_float(e % 2 ? odd : even); }
     };
-    auto put_x = [&](uint32_t sign) {
+    auto put_x = [&](uint32_t sign_bit) {
+        const Factors factor(kSplitScale, sign_bit);
         float rest = 0.f;
 #pragma unroll
         for (int i = 0; i < kVec; i += 2) {
             float x8[8];
 #pragma unroll
-            for (int e = 0; e < 8; e++) x8[e] = signed_x(i + e / 4, e % 4, sign);
+            for (int e = 0; e < 8; e++) x8[e] = xs[i + e / 4][e % 4] * factor.of(e);
             Split8 s;
             rest += split8(x8, s);
             typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
@@ -512,13 +510,13 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         }
         return rest;
     };
-    // what the wave's own space holds for grad_input, added to it and masked
-    auto add_d = [&](uint32_t bits) {
+    // what the wave's own space holds for grad_input, in units of `unit`, added to it and masked
+    auto add_d = [&](uint32_t bits, const Factors unit) {
 #pragma unroll
         for (int i = 0; i < kVec; i++) {
             const f32x4_t d = *reinterpret_cast<const f32x4_t *>(own + (lc + kChannels * i) * kDRow + 16 * lv);
 #pragma unroll
-            for (int e = 0; e < 4; e++) gs[i][e] += e % 2 ? -d[e] : d[e];
+            for (int e = 0; e < 4; e++) gs[i][e] = __builtin_fmaf(d[e], unit.of(e), gs[i][e]);
         }
         if (ch0 + 16 > a.mask_from) {             // uniform
 #pragma unroll
@@ -530,7 +528,6 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
     constexpr int kK = kUnit / 32;                // steps of 32 voxels: the segments of the unit
     // False where a value cannot be split (and nothing is computed).
     auto compute = [&](int u, bool split, uint32_t sign_bit, const Unit &un, const Unit &next) {
-        const float sign = __uint_as_float(sign_bit | 0x3f800000u);
         uint32_t ll = (uint32_t)lane;
         if (G > 1 && P < 4) asm volatile("" : "+v"(ll));            // (no LDS addresses are kept over the tiles: registers)
         const uint32_t nn = ll % 16, qq = ll / 16 % 4;
@@ -566,7 +563,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         clear_skipped(un);
         const uint32_t bits = mask_of();
         const float rest = put_x(sign_bit);
-        const bool done = split && !__any(rest != rest);            // uniform
+        const bool done = split && !__any(taken_whole(rest));       // uniform
         __builtin_amdgcn_sched_barrier(0);        // (the scheduler would move the loads to where they are used)
         request(x, a.C, next, xs);
         __builtin_amdgcn_sched_barrier(0);
@@ -621,7 +618,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             if (r % kK == kK - 1) {
 #pragma unroll
                 for (int o = 0; o < 2; o++) {
-                    sums[r / kK * 2 + o] += sign * acc[o];
+                    sums[r / kK * 2 + o] += __uint_as_float(__float_as_uint(kSplitUnit) | sign_bit) * acc[o];
                     asm volatile("" : "+v"(sums[r / kK * 2 + o]));  // (here and not at the end of the tile: registers)
                 }
             }
@@ -664,12 +661,13 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                 __builtin_amdgcn_sched_barrier(0);
             }
             own_sync();
-            add_d(bits);
+            add_d(bits, Factors(kSplitUnit));
             own_sync();
         }
         return true;
     };
-    // The same with the fp32 instruction, for values that cannot be split among x, A or the weights.
+    // The same with the fp32 instruction, for values that cannot be split among x, A or the weights (A and the weights
+    // lie whole in the place of their parts).
     auto compute_whole = [&](int u, uint32_t sign_bit, const Unit &un) {
         const float sign = __uint_as_float(sign_bit | 0x3f800000u);
         clear_skipped(un);
@@ -681,13 +679,13 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         auto value = [&](uint32_t voxel, uint32_t m) {
             const char *const at = Au + (voxel / kSegment * G + m / kRows) * kSlabBytes + voxel % kSegment * kVoxelBytes +
                                    16 * (m % kRows / 8 ^ turn(voxel)) + m % 8 * 2;
-            return part_value(at) + part_value(at + kPartBytes) + part_value(at + 2 * kPartBytes);
+            return whole_value(*reinterpret_cast<const __bf16 *>(at), *reinterpret_cast<const __bf16 *>(at + kPartBytes));
         };
         own_sync();
 #pragma unroll
         for (int i = 0; i < kVec; i++)
             *reinterpret_cast<f32x4_t *>(own + (lc + kChannels * i) * kDRow + 16 * lv) =
-                f32x4_t{signed_x(i, 0, sign_bit), signed_x(i, 1, sign_bit), signed_x(i, 2, sign_bit), signed_x(i, 3, sign_bit)};
+                xs[i] * f32x4_t{sign, -sign, sign, -sign};
         own_sync();
 #pragma unroll
         for (int t = 0; t < kTiles; t++)
@@ -712,15 +710,15 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                     f32x4_t d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int e = 0; e < 8; e++) {
-                        const float we = (float)w[i][0][e] + (float)w[i][1][e] + (float)w[i][2][e];
-                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(value(16 * s + nn, 32 * i + 8 * qq + e), we, d, 0, 0, 0);
+                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(value(16 * s + nn, 32 * i + 8 * qq + e),
+                                                                 whole_value(w[i][0][e], w[i][1][e]), d, 0, 0, 0);
                     }
                     all += d;
                 }
                 *reinterpret_cast<f32x4_t *>(own + nn * kDRow + (16 * s + 4 * qq) * 4) = all;
             }
             own_sync();
-            add_d(bits);
+            add_d(bits, Factors(1.f));
         }
         own_sync();
     };
@@ -774,7 +772,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                     request_g(un);
                     clear_skipped(un);
                     const float rest = put_x(t.sign);
-                    if (split && !__any(rest != rest)) continue;    // (the first run has done it)
+                    if (split && !__any(taken_whole(rest))) continue;    // (the first run has done it)
                     compute_whole(u, t.sign, un);
                     store(un, true);
                 }
@@ -844,26 +842,28 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
         const int o = min(tid, a.out.n - 1), d = a.out.dil[o];
         shared.sources[tid] = Source{N == kVolume ? 4u * (uint32_t)(d * (int)a.sz) : 0u, 4u * (uint32_t)(d * (int)a.sy), 4u * (uint32_t)d, (uint32_t)o * ((uint32_t)a.gsc * 4u)};
     }
+    auto load_weights = [&](bool whole) {
+        int ch = ch0 + n, qq = q;
+        if (whole) asm volatile("" : "+v"(ch), "+v"(qq));       // (nothing of the first call is kept for the second)
+#pragma unroll
+        for (int step = 0; step < 2 * G; step++) {
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const Slot m = slot_of<N>(32 * step + 8 * qq + i);
+                const bool ok = m.tap >= 0 && m.output < a.out.n && ch < a.update;
+                const float k = a.out.k[ok ? m.output : 0][ok ? (int64_t)ch * kTaps + m.tap : 0];
+                v[i] = (ok ? k : 0.f) * (whole ? 1.f : kSplitScale);
+            }
+            Split8 s;
+            if (whole) put_whole(v, s);
+            else if (__any(taken_whole(split8(v, s)))) state.weights_split = false;
+#pragma unroll
+            for (int p = 0; p < 3; p++) state.w[step][p] = s.p[p];
+        }
+    };
     state.weights_split = true;
-#pragma unroll
-    for (int step = 0; step < 2 * G; step++) {
-        float v[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const Slot m = slot_of<N>(32 * step + 8 * q + i);
-            const bool ok = m.tap >= 0 && m.output < a.out.n && ch0 + n < a.update;
-            const float k = a.out.k[ok ? m.output : 0][ok ? (int64_t)(ch0 + n) * kTaps + m.tap : 0];
-            v[i] = ok ? k : 0.f;
-        }
-        Split8 s;
-        const float bad = split8(v, s);
-        if (__any(bad != bad)) {
-            split_any(v, s);
-            state.weights_split = false;
-        }
-#pragma unroll
-        for (int p = 0; p < 3; p++) state.w[step][p] = s.p[p];
-    }
+    load_weights(false);
     __syncthreads();
 
     float *const row = part + (int64_t)bid * (a.chunks.blocks * 1024 * G);
@@ -876,6 +876,7 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
     if (__builtin_amdgcn_readfirstlane(shared.bad_again) != 0) {    // uniform over the workgroup
         int tid2 = tid;
         asm volatile("" : "+v"(tid2));           // (nothing of the first run is kept for the second)
+        load_weights(true);
         pull_tiles<N, G, P, FRESH, true>(a, x, gy, gx, row, lds, shared, tid2, wave, blocks, c0, wgs, wg, state);
     }
 

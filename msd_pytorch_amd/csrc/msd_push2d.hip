@@ -245,8 +245,8 @@ struct SplitArgs {
 // is split, put and read before the second.
 __host__ __device__ __forceinline__ int channel_of(int q, int e) { return e < 4 ? 4 * q + e : 16 + 4 * q + e - 4; }
 
-// [step][tile of columns][part][lane (column n, q)]: eight channels each; bad[step]: weights without parts
-// among them.
+// [step][tile of columns][part][lane (column n, q)]: eight channels each; bad[step]: some of them have to be taken whole,
+// and all of the step's lie so.
 __global__ __launch_bounds__(kSlabs *kTiles *kWave) void push_table(const SplitArgs a, bf16x8_t *__restrict__ table, int *__restrict__ bad)
 {
     const int step = blockIdx.x, t = threadIdx.x / kWave, lane = threadIdx.x % kWave, i = lane % 16, q = lane / 16;
@@ -260,10 +260,12 @@ __global__ __launch_bounds__(kSlabs *kTiles *kWave) void push_table(const SplitA
         const float w = k[min(c, a.C - 1) * kTaps];
         v[e] = column && c < a.C ? w : 0.f;
     }
+    float scaled[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) scaled[e] = v[e] * kSplitScale;
     Split8 s;
-    const float rest = split8(v, s);
-    const int any = __syncthreads_or(rest != rest);
-    if (any) split_any(v, s);
+    const int any = __syncthreads_or(taken_whole(split8(scaled, s)));
+    if (any) put_whole(v, s);
     if (threadIdx.x == 0) bad[step] = any;
 #pragma unroll
     for (int p = 0; p < 3; p++) table[((step * kSlabs * kTiles + t) * 3 + p) * kWave + lane] = s.p[p];
@@ -403,7 +405,9 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
 #pragma unroll
                     for (int i = 4 * h; i < 4 * h + 4; i += 2) {
                         // -x at every second voxel: the sums of the bf16 instruction are cut off towards minus infinity
-                        const float v[8] = {xv[i][0], -xv[i][1], xv[i][2], -xv[i][3], xv[i + 1][0], -xv[i + 1][1], xv[i + 1][2], -xv[i + 1][3]};
+                        float v[8];
+#pragma unroll
+                        for (int e = 0; e < 8; e++) v[e] = xv[i + e / 4][e % 4] * (e % 2 ? -kSplitScale : kSplitScale);
                         Split8 s;
                         rest += split8(v, s);
 #pragma unroll
@@ -453,14 +457,14 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
                             for (int j = 0; j < 4; j++)
                                 one[j] = mfma_split(xa[j], w[t % 2], k == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : one[j], k);
 #pragma unroll
-                        for (int j = 0; j < 4; j++) acc[j][t] += one[j];
+                        for (int j = 0; j < 4; j++) acc[j][t] += kSplitUnit * one[j];
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
             }
             if (!real) continue;
-            if (!weights_split || __any(rest != rest)) {                           // uniform
-                // values without parts: all of the segment's sums again, with the fp32 instruction
+            if (!weights_split || __any(taken_whole(rest))) {                      // uniform
+                // values to be taken whole: all of the segment's sums again, with the fp32 instruction
 #pragma unroll
                 for (int j = 0; j < 4; j++)
 #pragma unroll
@@ -470,6 +474,7 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
 #pragma unroll 1
                 for (int c0 = 0; c0 < a.C; c0 += 4) {
                     const int c = c0 + (int)q;
+                    const bool whole = bad[c0 / kStepChannels] != 0;               // uniform
                     const int r = c % kStepChannels, at = (int)n + r % 16 / 4 * 16, e = r % 4 + r / 16 * 4;
                     float xj[4], wj[kTiles];
 #pragma unroll
@@ -481,7 +486,8 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
                     for (int t = 0; t < kTiles; t++) {
                         const __bf16 *const k = reinterpret_cast<const __bf16 *>(
                             table + ((int64_t)(min(c, a.C - 1) / kStepChannels * kSlabs + slab) * kTiles + t) * (3 * kWave) + at) + e;
-                        wj[t] = c < a.C ? (float)k[0] + (float)k[8 * kWave] + (float)k[16 * kWave] : 0.f;
+                        const float sum = (float)k[0] + (float)k[8 * kWave] + (float)k[16 * kWave];
+                        wj[t] = c < a.C ? (whole ? whole_value(k[0], k[8 * kWave]) : sum * (1.f / kSplitScale)) : 0.f;
                     }
 #pragma unroll
                     for (int j = 0; j < 4; j++)

@@ -10,9 +10,13 @@
 // product, and unlike that one they leave the vector pipe free (two vector instructions fit beside
 // each at no cost, beside the fp32 instruction none).
 //
-// Values that have no such sum (infinities, NaN, and the few finite ones above 3.39e38, which round
-// to an infinity) give a NaN in the rest of the split: callers look at that and take
-// v_mfma_f32_16x16x4_f32 for the product at hand (split_any keeps the parts addable: h + m + l is the value).
+// Values are taken 2^24 times as large: the lowest bit of an fp32 number, 2^-149, is then 2^-125, a normal bf16 number,
+// so that the sum is exact however small the value is.  Products come 2^48 times as large; where they are added to
+// what has been summed before, the same instruction takes that back.  (Without it values below 2^-110 lost their low
+// parts: products of values around 2^-122 were off by 1e-4 to 3e-3.)
+//
+// Values from 2^36 on (6.9e10), infinities and NaN are reported by split8: the sum of a few hundred products of such
+// values might not fit.  Callers take v_mfma_f32_16x16x4_f32 for the product at hand, on the values as they are.
 #pragma once
 
 #include "msd_common.h"
@@ -26,9 +30,14 @@ struct Split8 {
     bf16x8_t p[3];                                // high, middle, low part
 };
 
-// Returns a sum that is NaN where a value cannot be split.
+constexpr float kSplitScale = 0x1p24f;            // of a value, and what takes that of a product back
+constexpr float kSplitUnit = 0x1p-48f;
+
+// The parts of values that have been multiplied by kSplitScale.  Returns a sum that is not finite where one of them has
+// to be taken whole: 2^68 times a high part of 2^60 or more is an infinity.
 __device__ __forceinline__ float split8(const float (&v)[8], Split8 &s)
 {
+#pragma clang fp contract(off)                    // (the scale is multiplied once: as a part of each difference it costs more)
     typedef float f2_t __attribute__((ext_vector_type(2)));
     float bad = 0.f;
 #pragma unroll
@@ -41,7 +50,7 @@ __device__ __forceinline__ float split8(const float (&v)[8], Split8 &s)
         const f2_t mf = __builtin_convertvector(m, f2_t);
         const f2_t q{r[0] - mf[0], r[1] - mf[1]};
         const bf16x2_t l = __builtin_convertvector(q, bf16x2_t);
-        bad = __builtin_amdgcn_fdot2_f32_bf16(l, bf16x2_t{(__bf16)1.f, (__bf16)1.f}, bad, false);
+        bad = __builtin_amdgcn_fdot2_f32_bf16(h, bf16x2_t{(__bf16)0x1p68f, (__bf16)0x1p68f}, bad, false);
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             s.p[0][i + e] = h[e];
@@ -51,21 +60,22 @@ __device__ __forceinline__ float split8(const float (&v)[8], Split8 &s)
     }
     return bad;
 }
+__device__ __forceinline__ bool taken_whole(float bad) { return !__builtin_isfinite(bad); }
 
-// The parts of any value: those of a value that is not finite are itself and zeros, the high part is cut
-// off, not rounded, so that it stays finite where the value is.
-__device__ __forceinline__ void split_any(const float (&v)[8], Split8 &s)
+// Whole values in the place of their parts: the upper and the lower half of their bits.
+__device__ __forceinline__ void put_whole(const float (&v)[8], Split8 &s)
 {
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const float h = v[i] != v[i] ? v[i] : __uint_as_float(__float_as_uint(v[i]) & 0xffff0000u);
-        const bool finite = (__float_as_uint(h) & 0x7f800000u) != 0x7f800000u;
-        const float r = finite ? v[i] - h : 0.f;
-        const float m = __uint_as_float(__float_as_uint(r) & 0xffff0000u);
-        s.p[0][i] = (__bf16)h;
-        s.p[1][i] = (__bf16)m;
-        s.p[2][i] = (__bf16)(r - m);
+        const uint32_t bits = __float_as_uint(v[i]);
+        s.p[0][i] = __builtin_bit_cast(__bf16, (uint16_t)(bits >> 16));
+        s.p[1][i] = __builtin_bit_cast(__bf16, (uint16_t)bits);
+        s.p[2][i] = (__bf16)0.f;
     }
+}
+__device__ __forceinline__ float whole_value(__bf16 upper, __bf16 lower)
+{
+    return __uint_as_float((uint32_t)__builtin_bit_cast(uint16_t, upper) << 16 | __builtin_bit_cast(uint16_t, lower));
 }
 
 // acc += a b for the parts of a (rows, k) and b (k, columns).
