@@ -324,10 +324,14 @@ int msd_block_forward(int dtype, int ndim, int64_t batch, int64_t c_in, int dept
 /* The same with a workspace (msd_block_forward_workspace_bytes; less, or none, is accepted):
  * groups of layers then take the channels in front of them in one pass (2D, fp32; same sums in
  * another order).  It holds three planes per output channel of a group, so up to 21 channels of the
- * stack's size (large stacks: 42, and 13 KB per 32 channels; these groups take a workspace that begins at a multiple of
- * 16 bytes), while the call runs. */
+ * stack's size (large stacks: 42, and 24 KB per 32 channels; these groups take a workspace that begins at a multiple of
+ * 16 bytes), while the call runs.  The second query is for a block of these dilations (NULL: of any) and groups of at
+ * most `outputs` outputs: 14 for what the call can use, 7 for what it makes do with where that is not to be had. */
 int64_t msd_block_forward_workspace_bytes(int dtype, int ndim, int64_t batch, int64_t c_in, int depth,
                                           const int64_t *widths, const int64_t *spatial);
+int64_t msd_block_forward_workspace_bytes_of(int dtype, int ndim, int64_t batch, int64_t c_in, int depth,
+                                             const int64_t *widths, const int64_t *spatial, const int64_t *dilations,
+                                             int outputs);
 int msd_block_forward_ws(int dtype, int ndim, int64_t batch, int64_t c_in, int depth, const int64_t *widths,
                          const int64_t *spatial, const int64_t *dilations, void *stack, const int64_t *stack_strides,
                          const void *const *weights, const void *bias, void *workspace, int64_t workspace_bytes,

@@ -56,6 +56,7 @@ PROTOTYPES = {
     "msd_block_forward": (_c_int, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p, _i64p] + _VIEW
                           + [ctypes.POINTER(ctypes.c_void_p), _ptr, _ptr]),
     "msd_block_forward_workspace_bytes": (_c_i64, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p]),
+    "msd_block_forward_workspace_bytes_of": (_c_i64, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p, _i64p, _c_int]),
     "msd_block_forward_ws": (_c_int, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p, _i64p] + _VIEW
                              + [ctypes.POINTER(ctypes.c_void_p), _ptr] + _WS + [_ptr]),
     "msd_block_backward": (_c_int, [_c_int, _c_int, _c_i64, _c_i64, _c_int, _i64p, _i64p, _i64p] + _VIEW + _VIEW

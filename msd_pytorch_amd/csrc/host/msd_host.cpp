@@ -32,7 +32,7 @@ namespace py = pybind11;
 // The entry points, looked up in the library that the package has loaded.
 #define MSD_ENTRIES(X)                                                                                              \
     X(msd_last_error) X(msd_conv_forward) X(msd_conv_relu_forward) X(msd_conv_layer_backward) X(msd_conv_layer_workspace_bytes)  \
-    X(msd_block_forward_ws) X(msd_block_forward_workspace_bytes) X(msd_block_backward) X(msd_block_workspace_bytes) X(msd_final_forward)                     \
+    X(msd_block_forward_ws) X(msd_block_forward_workspace_bytes_of) X(msd_block_backward) X(msd_block_workspace_bytes) X(msd_final_forward)                     \
     X(msd_final_backward) X(msd_final_forward_loss) X(msd_final_workspace_bytes) X(msd_scale_fold) X(msd_adam_step)   \
     X(msd_label_check)
 struct Entries {
@@ -242,14 +242,20 @@ struct Block {
 
     void forward(const Tensor &stack, const Tensor &bias, void *stream) const
     {
-        const int64_t need = lib.msd_block_forward_workspace_bytes(dtype_of(stack), (int)stack.dim() - 2,
-                                                                   stack.size(0), c_in, (int)widths.size(),
-                                                                   widths.data(), stack.sizes().data() + 2);
         Tensor ws;
-        try {
-            if (need) ws = workspace(need, stack);
-        } catch (const c10::OutOfMemoryError &) {
-            // the block needs none: its layers then run one by one
+        int64_t need = 0;
+        for (const int outputs : {14, 7}) {
+            const int64_t bytes = lib.msd_block_forward_workspace_bytes_of(
+                dtype_of(stack), (int)stack.dim() - 2, stack.size(0), c_in, (int)widths.size(), widths.data(),
+                stack.sizes().data() + 2, dilations.data(), outputs);
+            if (bytes <= 0 || bytes == need) break;
+            need = bytes;
+            try {
+                ws = workspace(need, stack);
+                break;
+            } catch (const c10::OutOfMemoryError &) {
+                // groups of half as many layers, or none: the layers then run one by one
+            }
         }
         check(lib.msd_block_forward_ws(dtype_of(stack), (int)stack.dim() - 2, stack.size(0), c_in, (int)widths.size(),
                                        widths.data(), stack.sizes().data() + 2, dilations.data(), stack.data_ptr(),

@@ -1517,7 +1517,7 @@ int forward_group(const BlockArgs &a, int i, int64_t first, int most)
     int n = 0;
     int64_t outputs = 0, dmax = 0;
     while (i + n < a.depth && a.widths[i + n] <= 2 && outputs + a.widths[i + n] <= most) {
-        // (a query of the workspace does not know the dilations)
+        // (msd_block_forward_workspace_bytes does not know the dilations)
         if (a.dilations) dmax = a.dilations[i + n] > dmax ? a.dilations[i + n] : dmax;
         outputs += a.widths[i + n++];
     }
@@ -1539,13 +1539,14 @@ int64_t group_planes_bytes(const BlockArgs &a, int i, int n, int64_t first)
     return ((planes + 3) / 4 * 4 + msd::group_table_floats_2d(first)) * (int64_t)sizeof(float);
 }
 
-// Of the largest group that a block can form, whichever layer its groups start at.
-int64_t forward_group_bytes(const BlockArgs &a)
+// Of the largest group of at most `outputs` outputs that a block can form, whichever layer its groups start at.
+int64_t forward_group_bytes(const BlockArgs &a, int outputs)
 {
     if (a.ndim != 2 || !msd::group_rows_supported_2d(a.spatial[1])) return 0;
     int64_t first = a.c_in, bytes = 0;
     for (int i = 0; i < a.depth; i++) {
         for (const int most : {msd::group2d::kSlabOut, msd::group2d::kMaxOut}) {
+            if (most > outputs) continue;
             const int64_t n = group_planes_bytes(a, i, forward_group(a, i, first, most), first);
             bytes = n > bytes ? n : bytes;
         }
@@ -1620,11 +1621,18 @@ int block_group_forward(const char *fn, const BlockArgs &a, int i, int n, int64_
 int64_t msd_block_forward_workspace_bytes(int dtype, int ndim, int64_t batch, int64_t c_in, int depth,
                                           const int64_t *widths, const int64_t *spatial)
 {
+    return msd_block_forward_workspace_bytes_of(dtype, ndim, batch, c_in, depth, widths, spatial, nullptr, msd::group2d::kMaxOut);
+}
+
+int64_t msd_block_forward_workspace_bytes_of(int dtype, int ndim, int64_t batch, int64_t c_in, int depth,
+                                             const int64_t *widths, const int64_t *spatial, const int64_t *dilations,
+                                             int outputs)
+{
     if (!widths || !spatial || depth <= 0 || (ndim != 2 && ndim != 3) || batch <= 0 || c_in <= 0) return -1;
     for (int i = 0; i < depth; i++)
         if (widths[i] <= 0) return -1;
-    const BlockArgs a{dtype, ndim, depth, batch, c_in, 0, widths, spatial, nullptr, dtype == MSD_F32 ? 4u : 8u};
-    return forward_group_bytes(a);
+    const BlockArgs a{dtype, ndim, depth, batch, c_in, 0, widths, spatial, dilations, dtype == MSD_F32 ? 4u : 8u};
+    return forward_group_bytes(a, outputs);
 }
 
 int msd_block_forward(int dtype, int ndim, int64_t batch, int64_t c_in, int depth, const int64_t *widths,

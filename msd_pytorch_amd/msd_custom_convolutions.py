@@ -414,17 +414,21 @@ def block_forward(stack, c_in, dilations, bias, weights):
     dilations = _check_block(fn, stack, c_in, dilations, bias, weights)
     bias = bias.contiguous()
     head = _block_head(stack, c_in, dilations, weights)
-    need = _native.load().msd_block_forward_workspace_bytes(head[0], head[1], head[2], c_in, head[4], head[5], head[6])
-    if need < 0:
-        _fail(fn, "invalid block geometry")
-    ws = None
-    if need:
+    ws, need = None, 0
+    for outputs in (14, 7):
+        more = _native.load().msd_block_forward_workspace_bytes_of(*head, outputs)
+        if more < 0:
+            _fail(fn, "invalid block geometry")
+        if more == need:
+            break
+        need = int(more)
         try:
-            ws = torch.empty(int(need), dtype=torch.uint8, device=stack.device)
+            ws = torch.empty(need, dtype=torch.uint8, device=stack.device)
+            break
         except torch.cuda.OutOfMemoryError:
-            need = 0                # the block needs none: its layers then run one by one
-    _call("msd_block_forward_ws", stack.device, *head, *_view(stack), _ptr_array(weights),
-          ctypes.c_void_p(bias.data_ptr()), ctypes.c_void_p(ws.data_ptr() if need else 0), int(need), _stream(stack))
+            pass                    # groups of half as many layers, or none: the layers then run one by one
+    _call("msd_block_forward_ws", stack.device, *head, *_view(stack), _ptr_array(weights), ctypes.c_void_p(bias.data_ptr()),
+          ctypes.c_void_p(0 if ws is None else ws.data_ptr()), 0 if ws is None else need, _stream(stack))
 
 
 def block_backward(stack, grads, c_in, dilations, weights, grad_weights, grad_bias, need_input_grad):

@@ -145,3 +145,19 @@ def test_forward_workspace_holds_the_planes_of_the_largest_group(size, c_in, wid
         need = lib.msd_block_forward_workspace_bytes(0, 2, batch, c_in, depth, i64(*[width] * depth), i64(*size))
         assert need == 3 * outputs * batch * size[0] * size[1] * 4
     assert lib.msd_block_forward_workspace_bytes(1, 2, 1, c_in, depth, i64(*[width] * depth), i64(*size)) == 0
+
+
+def test_forward_workspace_of_dilations_and_of_smaller_groups():
+    """Groups of fourteen (large stacks) take dilations up to 16; the planes of groups of seven are asked for apart."""
+    lib = _native.load()
+    depth, plane = 30, 2048 * 2048 * 4
+
+    def need(dilations, outputs):
+        return lib.msd_block_forward_workspace_bytes_of(0, 2, 1, 60, depth, i64(*[1] * depth), i64(2048, 2048),
+                                                        dilations and i64(*dilations), outputs)
+
+    steps = (60 + depth - 1 + 31) // 32            # of 32 channels in front of a group, 24 KB of weights each
+    assert need(None, 14) == lib.msd_block_forward_workspace_bytes(0, 2, 1, 60, depth, i64(*[1] * depth), i64(2048, 2048))
+    assert 42 * plane < need([1] * depth, 14) <= 42 * plane + steps * 24592
+    assert need([1] * depth, 7) == need([17] * depth, 14) == need([17] * depth, 7) == 21 * plane
+    assert 42 * plane < need([17] + [1] * (depth - 1), 14)         # (the groups that do not start with that layer)

@@ -396,6 +396,47 @@ def test_a_forward_pass_that_has_no_room_for_the_planes_of_its_groups(gradients)
     assert rel_err(got, want) <= 1e-5
 
 
+@pytest.mark.parametrize("host", ["native", "python"])
+def test_a_forward_pass_with_room_for_groups_of_seven_only(host):
+    """Where the 42 planes of groups of fourteen are not to be had, the 21 of groups of seven are asked for."""
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    from test_knobs_gpu import tuning
+    gen = torch.Generator().manual_seed(7)
+    c_in, depth, size = 12, 14, (1024, 1024)
+    image = torch.rand(1, c_in, *size, generator=gen).cuda()
+    weights = [(torch.randn(1, c_in + i, 3, 3, generator=gen) * 0.1).cuda() for i in range(depth)]
+    bias, dilations = torch.zeros(depth).cuda(), [1 + i % 10 for i in range(depth)]
+    final_w, final_b = torch.randn(1, c_in + depth, 1, 1, generator=gen).cuda(), torch.zeros(1).cuda()
+
+    def result():
+        if host == "native":
+            from msd_pytorch_amd import _native
+            return _native.host().net_forward(image, bias, weights, dilations, final_w, final_b)
+        stack = torch.empty(1, c_in + depth, *size, device="cuda")
+        stack[:, :c_in] = image
+        cc.block_forward(stack, c_in, dilations, bias, weights)
+        return stack
+
+    with tuning({"fwd.group": 12}):
+        sevens = result()
+    with tuning({"fwd.group": 0}):
+        one_by_one = result()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    plane = size[0] * size[1] * 4
+    room = torch.cuda.memory_reserved() + plane * (c_in + depth + 2 + 30)
+    total, pool = torch.cuda.get_device_properties(0).total_memory, torch.cuda.MemPool()
+    torch.cuda.set_per_process_memory_fraction(room / total)
+    try:
+        with torch.cuda.use_mem_pool(pool), tuning({"fwd.group": 1024 + 12}):
+            got = result()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    got = got.clone()
+    assert not torch.equal(got, one_by_one)
+    assert torch.equal(got, sevens)
+
+
 @pytest.mark.filterwarnings("ignore:Using a target size")
 def test_a_target_of_another_shape_is_left_to_the_criterion():
     (model,) = _models("L2", 2, 3, 1, 1, 1)
