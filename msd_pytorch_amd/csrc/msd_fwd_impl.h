@@ -415,7 +415,7 @@ hipError_t pick(const Geom &g, const View<const float> &x, const float *k, const
                 const long t33 = (long)((rows_z + 2) / 3) * ((rows_y + 2) / 3);
                 const long t44 = (long)((rows_z + 3) / 4) * ((rows_y + 3) / 4);
                 const long waves = (long)g.dil * g.dil * g.B * ((g.W + kWave - 1) / kWave);     // per tile of a residue class
-                const int forced = knob(kKnobFwdLattice3d, 0);
+                const int forced = knob(kKnobFwdLattice3d, 0), split = knob(kKnobFwdSplit, -1);
                 if (forced == 44) return launch<3, RELU, 1, 1, 4, 4, true>(g, x, k, bias, out, s, sums);
                 if (forced == 33) return launch<3, RELU, 1, 1, 3, 3>(g, x, k, bias, out, s, sums);
                 if (forced == 24) return launch<3, RELU, 1, 1, 2, 4>(g, x, k, bias, out, s, sums);
@@ -423,16 +423,16 @@ hipError_t pick(const Geom &g, const View<const float> &x, const float *k, const
                 // instead of 3) but take twice the registers: where the input comes from memory and not
                 // from the 256 MB cache, the tiles of all channels at once fill the chip (four waves per SIMD) and are
                 // hardly more than half as many.  256^3 over 16 / 30 channels: 317, 297 / 602, 555; 192^3 over
-                // 20 / 45: 169, 165 / 403, 364; 128^3 over 30 (2048 waves): 69, 89.
+                // 20 / 45: 169, 165 / 403, 364; 128^3 over 30 (2048 waves): 69, 89.  (Not where the caller sets several groups.)
                 const bool streams = (double)g.B * g.C * g.nvox * sizeof(float) > 1.5 * kCacheResidentBytes;
-                if (streams && t44 * waves >= 4096 && t44 * 32 <= t24 * 17)
+                if (streams && split <= 1 && t44 * waves >= 4096 && t44 * 32 <= t24 * 17)
                     return launch<3, RELU, 1, 1, 4, 4, true>(g, x, k, bias, out, s, sums);
                 // The channels in one group where few of them leave the finishing step a large part and the tiles fill
                 // the chip without more waves (192^3 over 5 / 8 / 12 channels: 64, 50 / 80, 67 / 107, 99; over 20:
                 // 169, 175), in four where the tiles leave most of it idle (64^3 over 20 / 45: 18, 16 / 33, 23;
                 // 40 x 45 x 47 over 45: 27, 17; 61 x 93 x 75, 1500 waves, over 20: 25, 25; over 12: 18, 19).
                 const bool full = t24 * waves >= 7000;
-                const bool one = (full && g.C <= 12 && knob(kKnobFwdSplit, -1) < 0) || knob(kKnobFwdSplit, -1) == 1;
+                const bool one = (full && g.C <= 12 && split < 0) || split == 1;
                 const int groups = t24 * waves <= 1100 && g.C >= 12 ? 4 : 2;
                 // Lattices of 3 x 3 rows instead of 2 x 4 where they cover the residue classes
                 // with at least 1/16 fewer tiles (a partly filled lattice costs as much time as a

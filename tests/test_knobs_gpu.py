@@ -217,6 +217,23 @@ def test_channel_groups_of_the_3d_forward(cc, case):
         check_operator_problem(cc, shape, seed=5)
 
 
+def test_the_number_of_channel_groups_is_the_callers_in_large_volumes(cc):
+    """More than the caches hold: by default (and with one group set) one group, with two or four set that many."""
+    gen = torch.Generator().manual_seed(11)
+    x = torch.rand(1, 18, 200, 256, 128, generator=gen).cuda()
+    k, bias = (torch.randn(1, 18, 3, 3, 3, generator=gen) * 0.1).cuda(), torch.zeros(1).cuda()
+    found = {}
+    for split in (-1, 1, 2, 4):
+        found[split] = torch.empty(1, 1, 200, 256, 128, device="cuda")
+        with tuning({"fwd.split": split}):
+            cc.conv_relu_forward(x, k, bias, found[split], 1)
+    # (other groups add the channels up in another order)
+    assert torch.equal(found[-1], found[1])
+    assert not torch.equal(found[1], found[2]) and not torch.equal(found[2], found[4]) and not torch.equal(found[1], found[4])
+    for split in (2, 4):
+        assert rel_err(found[split], found[1]) <= 1e-5
+
+
 BLOCK_SETTINGS = [{"block.snake": 0}, {"block.snake": 1}, {"block.fuse": 0}, {"block.defer": 0},
                   {"xcd_remap": 0}, {"bwdk.interleave": 0}, {"fwd.class3d": 0}, {"fwd.lattice3d": 44},
                   {"block.pair": 0}, {"block.pair": 1}, {"block.pair": 1, "block.defer": 0},
