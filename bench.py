@@ -26,6 +26,8 @@ HBM_PEAK_GBS = 8000.0
 # fp32 peak of MI355X (matrix cores, or packed vector instructions); plain (non-packed) vector
 # fp32, which the build rules leave to the forward kernel's multiply-adds, peaks at half of it
 FP32_PEAK_TFLOPS = 157.3
+# fp32 products as six bf16 products of their parts: a sixth of the dense bf16 peak
+SPLIT_PEAK_TFLOPS = 2500.0 / 6
 PIPE = {"forward": "fp32 VALU, non-packed (78.6 TFLOP/s of the 157.3 peak); 2D layer groups: fp32 MFMA 16x16x4, "
                    "of fourteen outputs bf16 MFMA 16x16x32 (six products of bf16 parts per fp32 product)",
         "backward_x": "fp32 VALU, non-packed (78.6 TFLOP/s of the 157.3 peak)",
@@ -160,6 +162,15 @@ def grouped_layers(ndim, c_in, depth, width, voxels):
             backward[i - n + 1] = n
         i -= n if n >= 2 else 1
     return forward, backward
+
+
+def peak_tflops(c_in, depth, width, split):
+    """What the flops of a class could run at: those of the layers in `split` ({first layer: layers}) as bf16
+    parts, the others' on the fp32 pipes."""
+    layers = {j for i, n in split.items() for j in range(i, i + n)}
+    work = [c_in + width * i for i in range(depth)]
+    parts = sum(w for i, w in enumerate(work) if i in layers)
+    return sum(work) / (parts / SPLIT_PEAK_TFLOPS + (sum(work) - parts) / FP32_PEAK_TFLOPS)
 
 
 def algorithmic_work(name, fused, paired=False, triple_from=32, kpairs=False, chainpairs=False, groups=({}, {})):
@@ -403,9 +414,11 @@ def measure(name, args, lib, torch, steps=None, warmup=None, cpu=True):
                                                              kpairs=split3d,
                                                              chainpairs=split3d and tuned.get("block.chainpair") != "0")
         kernels = {}
+        split = {"forward": {i: n for i, n in forward.items() if n * width > 7}, "backward_xkb": backward}
         for cls, (ms, launches) in totals.items():
             if launches == 0:
                 continue
+            peak = peak_tflops(c_in, depth, width, split.get(cls, {}))
             per_step_s = ms / args.steps * 1e-3
             gbs = bytes_per_step[cls] / per_step_s / 1e9
             tfl = flops_per_step[cls] / per_step_s / 1e12
@@ -414,7 +427,8 @@ def measure(name, args, lib, torch, steps=None, warmup=None, cpu=True):
                             "algorithmic_GB_per_step": round(bytes_per_step[cls] / 1e9, 3),
                             "GBps": round(gbs, 1), "frac_hbm": round(gbs / HBM_PEAK_GBS, 4),
                             "algorithmic_GFLOP_per_step": round(flops_per_step[cls] / 1e9, 2),
-                            "TFLOPs": round(tfl, 2), "frac_fp32": round(tfl / FP32_PEAK_TFLOPS, 4),
+                            "TFLOPs": round(tfl, 2), "peak_TFLOPs": round(peak, 1),
+                            "frac_fp32": round(tfl / peak, 4),
                             "Mvoxel_per_s": round(nvox / per_step_s / 1e6, 2)}
             if cls == "backward_xkb" and (paired or backward):
                 # the same time priced with the bytes of one fused pass per layer, for comparison
@@ -436,7 +450,7 @@ def measure(name, args, lib, torch, steps=None, warmup=None, cpu=True):
         by_flops = dom["frac_fp32"] > dom["frac_hbm"]
         roof = {"bound": "mfma" if by_flops else "hbm", "kernel": dominant,
                 "achieved": dom["TFLOPs"] if by_flops else dom["GBps"],
-                "peak": FP32_PEAK_TFLOPS if by_flops else HBM_PEAK_GBS,
+                "peak": dom["peak_TFLOPs"] if by_flops else HBM_PEAK_GBS,
                 "unit": "TFLOP/s" if by_flops else "GB/s",
                 "frac": dom["frac_fp32"] if by_flops else dom["frac_hbm"],
                 # HBM-side bytes per launch (fetch + write counters of the committed rocprofv3
@@ -449,7 +463,7 @@ def measure(name, args, lib, torch, steps=None, warmup=None, cpu=True):
                 "algorithmic_flops_per_launch": round(flops_per_step[dominant] / dom["calls_per_step"]),
                 "avg_launch_us": dom["avg_call_us"],
                 "hbm": {"achieved_GBps": dom["GBps"], "peak_GBps": HBM_PEAK_GBS, "frac": dom["frac_hbm"]},
-                "fp32": {"achieved_TFLOPs": dom["TFLOPs"], "peak_TFLOPs": FP32_PEAK_TFLOPS, "frac": dom["frac_fp32"],
+                "fp32": {"achieved_TFLOPs": dom["TFLOPs"], "peak_TFLOPs": dom["peak_TFLOPs"], "frac": dom["frac_fp32"],
                          "pipe": PIPE[dominant]},
                 "timed": "HIP events on the launch stream around the library's operator launches "
                          "(msd_profile_enable; one pair per run of launches of one class), in a repeat of "
