@@ -405,7 +405,7 @@ int msd_final_forward_loss(int dtype, int loss_kind, int64_t batch, int64_t c_in
  * microseconds of idle stream to every launch).
  * msd_profile_read waits for the recorded events and returns, per class
  * {0 forward, 1 backward_x incl. the mask, 2 backward_k/bias, 3 fused backward_x +
- * backward_k/bias of the block backward pass}, the summed elapsed milliseconds and the
+ * backward_k/bias of the block backward pass and of msd_conv_layer_backward in one pass}, the summed elapsed milliseconds and the
  * number of calls since msd_profile_enable(1); ms and calls hold
  * MSD_PROFILE_CLASSES entries.  Not thread-safe; no counterpart in the reference.
  */

@@ -38,7 +38,7 @@ HBM_PEAK = 8.0e12
 
 # Launch-shape parameters each operator reads, with the values worth trying (the first value
 # listed is not special: the library's default is measured separately, with every parameter
-# unset).  {r} is the rank, 2 or 3.
+# unset).  {r} is the rank, 2 or 3.  (fwd.lattice3d of 44 is one channel group whatever fwd.split says.)
 SWEEP_GRID = {
     "forward": {
         2: {"fwd.vec2d": (1, 2, 4), "fwd.rows2d": (2, 3, 4, 5, 6), "fwd.split": (1, 2, 4)},

@@ -21,6 +21,11 @@ def bias_close(got, want, terms, tol=1e-4):
     return diff <= tol * max(want.abs().max().item(), floor)
 
 
+def same_specials(got, want):
+    """NaN, +inf and -inf in the same places."""
+    return all(torch.equal(f(got), f(want)) for f in (torch.isnan, torch.isposinf, torch.isneginf))
+
+
 def check_operator_problem(cc, shape, seed=7, plain=True):
     """conv_relu_forward and the three conv_relu_backward_* operators (accumulating), the plain
     operators (conv_forward, conv_backward_x, conv_backward_kb) and the three plain backward

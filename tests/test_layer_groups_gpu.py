@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from parity import check_block, rel_err
+from parity import check_block, rel_err, same_specials
 from test_knobs_gpu import tuning
 
 pytestmark = pytest.mark.gpu
@@ -177,7 +177,7 @@ def test_volumes_in_other_layouts(c_in, width, depth, layout):
 # What is no sum of three bf16 values takes the fp32 instruction: the same infinities and NaNs as from the
 # layers' own kernels, and the largest finite values (which round to an infinity in bf16) stay finite.
 @pytest.mark.parametrize("where", ["stack", "gradient", "weight"])
-@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38, -3.4028234e38])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4e38, -3.4028234e38])
 @pytest.mark.parametrize("depth", [6, 14])
 def test_values_without_bf16_parts(where, value, depth):
     from msd_pytorch_amd import msd_custom_convolutions as cc
@@ -198,8 +198,7 @@ def test_values_without_bf16_parts(where, value, depth):
         with tuning({"bwd.group": setting}):
             cc.block_backward(stack, grads, c_in, [1 + i % 4 for i in range(depth)], weights, gk, gb, True)
         found.append(torch.cat([grads[:, :c_in].flatten(), gb, *(k.flatten() for k in gk)]))
-    assert torch.equal(torch.isnan(found[0]), torch.isnan(found[1]))
-    assert torch.equal(torch.isinf(found[0]), torch.isinf(found[1]))
+    assert same_specials(found[1], found[0])
     finite = torch.isfinite(found[0])
     assert bool(finite.any())
     # (sums of up to 639 terms of one sign in another order, relative to the largest)
@@ -223,8 +222,7 @@ def test_an_infinity_meets_its_own_voxels_only():
             cc.block_backward(stack, gradient.clone(), c_in, [1, 2, 3, 1, 2, 3, 1, 2], weights, gk, gb, True)
         found.append(torch.cat([k.flatten() for k in gk]))
     assert torch.isinf(found[0]).any()
-    assert torch.equal(torch.isnan(found[0]), torch.isnan(found[1]))
-    assert torch.equal(torch.isinf(found[0]), torch.isinf(found[1]))
+    assert same_specials(found[1], found[0])
 
 
 @pytest.mark.parametrize("c_in", [4, 5, 6, 7, 129])
@@ -245,8 +243,7 @@ def test_an_infinity_in_front_of_a_forward_group_stays_one(c_in):
         found.append(stack)
     assert torch.isinf(found[0][:, c_in:]).any() and not torch.isnan(found[0]).any()
     finite = torch.isfinite(found[0])
-    assert torch.equal(torch.isinf(found[0]), torch.isinf(found[1]))
-    assert torch.equal(finite, torch.isfinite(found[1]))
+    assert same_specials(found[1], found[0])
     assert rel_err(found[1][finite], found[0][finite]) <= 1e-5
 
 
@@ -298,8 +295,7 @@ def test_values_without_bf16_parts_in_front_of_a_forward_group(where, value):
         with tuning({"fwd.group": setting}):
             cc.block_forward(stack, c_in, [1, 12, 3, 1, 2, 3, 1, 2, 3], torch.zeros(depth, device="cuda"), weights)
         found.append(stack[:, c_in:])
-    assert torch.equal(torch.isnan(found[0]), torch.isnan(found[1]))
-    assert torch.equal(torch.isinf(found[0]), torch.isinf(found[1]))
+    assert same_specials(found[1], found[0])
     finite = torch.isfinite(found[0])
     assert bool(finite.any()) and rel_err(found[1][finite], found[0][finite]) <= 1e-5
 
