@@ -221,7 +221,7 @@ struct Block {
     // kernels reads a short run of 16 channels at a time; where the channels lie a multiple of
     // kCamped bytes apart these runs meet in few of the memory's channels, so such planes are moved
     // apart by kApart bytes (from kFrom bytes on: smaller ones come from the caches).  1024 x 1024, 104
-    // channels, a pass of msd_pull2d.hip: 452 -> 372 us; a training step there, depth 100: 6.7 -> 6.3 ms;
+    // channels, a pass of msd_pull.hip: 452 -> 372 us; a training step there, depth 100: 6.7 -> 6.3 ms;
     // 2048 x 2048, two channels per layer, depth 200: 319 -> 272; a forward pass of 256^3, depth 30: 10.0 -> 9.6.
     // Distances of 128 to 66048 bytes did the same in 2D; 128^3, depth 50, gains 1 % with this one and loses 0.5 %
     // with 512 or 66048.  Planes of other sizes gain nothing (1000 x 1056: 396 us with and without).

@@ -362,7 +362,7 @@ void bwd_rows_fused(const Args a_, const float *__restrict__ gyp, const float *_
                 const uint32_t xch = (uint32_t)min(mj, g.C - 1 - cb0) * (uint32_t)xsc + xrow;
 #pragma unroll
                 for (int j = 0; j < NSS; j++)
-                    load_global_vec4_unaligned(xb, 4u * (xch + (uint32_t)min(kx + 16 * (h * NSS + j), g.W - 4)),
+                    load_global_vec_unaligned<4>(xb, 4u * (xch + (uint32_t)min(kx + 16 * (h * NSS + j), g.W - 4)),
                                                kk[j]);
             } else {
                 const uint32_t xch = (uint32_t)min(c0 + cb * kChanBlock + mj, g.C - 1) * (uint32_t)xsc + xrow;

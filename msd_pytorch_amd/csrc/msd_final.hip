@@ -51,16 +51,9 @@ __device__ __forceinline__ void store_elems(T *p, const T (&d)[V])
     }
 }
 
-// V floats at any multiple of four bytes (images of odd size: every channel begins elsewhere).  3 x 333 x 477, 35
-// channels, three labels: 66 us with one voxel per lane, the widest aligned access, 42 with four; 61 x 93 x 75, 21 channels: 35 and 15.
-template <int V> __device__ __forceinline__ void load_unaligned(uint64_t base, uint32_t byte_offset, float (&d)[V])
-{
-    typedef float vec_t __attribute__((ext_vector_type(V), aligned(4)));
-    typedef const __attribute__((address_space(1))) char *gbytes_t;
-    const vec_t v = *reinterpret_cast<const __attribute__((address_space(1))) vec_t *>(reinterpret_cast<gbytes_t>(base) + byte_offset);
-#pragma unroll
-    for (int i = 0; i < V; i++) d[i] = v[i];
-}
+// V floats to any multiple of four bytes, as load_global_vec_unaligned takes them (images of odd size: every channel begins
+// elsewhere).  3 x 333 x 477, 35 channels, three labels: 66 us with one voxel per lane, the widest aligned access, 42 with four;
+// 61 x 93 x 75, 21 channels: 35 and 15.
 template <int V> __device__ __forceinline__ void store_unaligned(float *p, const float (&d)[V])
 {
     typedef float vec_t __attribute__((ext_vector_type(V), aligned(4)));
@@ -208,7 +201,7 @@ __global__ __launch_bounds__(kFinalThreads) void final_backward_write(int64_t nv
     float g[MAXO][V];
 #pragma unroll
     for (int o = 0; o < MAXO; o++) {
-        load_unaligned<V>(reinterpret_cast<uint64_t>(go + blockIdx.y * gsb + min(o, c_out - 1) * gsc + first), 0, g[o]);
+        load_global_vec_unaligned<V>(reinterpret_cast<uint64_t>(go + blockIdx.y * gsb + min(o, c_out - 1) * gsc + first), 0, g[o]);
     }
     float *gp = gx + blockIdx.y * gxsb + first;
 #pragma unroll 4
@@ -413,7 +406,7 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
             float v[G][V];
 #pragma unroll
             for (int j = 0; j < G; j++)
-                load_unaligned<V>(xbase + (uint64_t)((int64_t)min((c0 + j) * kTiledWaves + wave, C - 1) * xsc * 4), xoff,
+                load_global_vec_unaligned<V>(xbase + (uint64_t)((int64_t)min((c0 + j) * kTiledWaves + wave, C - 1) * xsc * 4), xoff,
                                    v[j]);
 #pragma unroll
             for (int j = 0; j < G; j++) {
@@ -482,7 +475,7 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
             for (int o = 0; o < MAXO; o++) {
                 const bool keep = active && o < c_out;
                 float t[V];
-                load_unaligned<V>(reinterpret_cast<uint64_t>(static_cast<const float *>(target) + (int64_t)b * tsb +
+                load_global_vec_unaligned<V>(reinterpret_cast<uint64_t>(static_cast<const float *>(target) + (int64_t)b * tsb +
                                                              (int64_t)min(o, c_out - 1) * tsc), xoff, t);
                 const float bv = bias && o < c_out ? bk[o] : 0.f;
 #pragma unroll

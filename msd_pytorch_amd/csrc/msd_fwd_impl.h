@@ -91,9 +91,9 @@ __device__ __forceinline__ bool tile_origin(const Geom &g, const Lattice &lt, in
     return y0 < g.H && z0 < g.D;                 // false: empty tail of a residue class
 }
 
-// Output rows of a tile of `rows` that are finished together.  3D with one voxel per lane: the rows of half a tile take at
-// most 30 KB, which costs no resident workgroup (61 x 93 x 75, depth 20: 364 -> 358 us; 40 x 45 x 47, depth 30, in four groups:
-// 366 -> 323).  2D: one at a time (256 x 256, depth 10: half tiles are 3 us slower).
+// Output rows of a tile of `rows` that are finished together.  3D with one voxel per lane: half a tile of 2 x 4 or 3 x 3 rows
+// (at most 30 KB), six rows of one of 4 x 4 (at most 36 KB; its registers leave room for two workgroups of 512 lanes), which
+// costs no resident workgroup (61 x 93 x 75, depth 20: 364 -> 358 us; 40 x 45 x 47, depth 30, in four groups: 366 -> 323).  2D: one at a time (256 x 256, depth 10: half tiles are 3 us slower).
 constexpr int finish_batch(int ndim, int V, int rows) { return ndim == 2 || V > 1 ? 1 : rows <= 10 ? (rows + 1) / 2 : 6; }
 
 // ONE (3D): all channels in one group.  A channel's nine products are summed before they are added: in one chain over

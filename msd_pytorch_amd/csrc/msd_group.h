@@ -23,6 +23,22 @@ constexpr int kTiles = kRows / 16;
 constexpr int kChunk = 128;                       // channels whose weights are in LDS at a time
 
 // The outputs of a group: dilation, and weights of the channels from 0 on, of each.
+// Between LDS accesses of one wave: LDS executes them in order, only the compiler has to be kept from
+// reordering them.
+__device__ __forceinline__ void own_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// Between the LDS accesses of a workgroup (of LDS only: the loads and stores of memory stay in flight).
+__device__ __forceinline__ void lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 struct Outputs {
     int n;
     int dil[kMaxOut];

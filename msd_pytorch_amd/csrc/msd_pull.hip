@@ -131,22 +131,6 @@ __device__ __forceinline__ float load1(uint64_t base, uint32_t off)
     return d[0];
 }
 
-// Between LDS accesses of one wave: LDS executes them in order, only the compiler has to be kept from
-// reordering them.
-__device__ __forceinline__ void own_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-// Between the LDS accesses of a workgroup (of LDS only: the loads and stores of the units stay in flight).
-__device__ __forceinline__ void tile_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // The sources of one voxel (or row) u of an axis of n through the outer taps of dilation d
 // (adjoint_sources): `up` is read by tap 0 where it lies inside and is otherwise the mirrored source of
 // tap 2, `down` the other way round, so that two loads hold all of them.
@@ -203,9 +187,8 @@ template <int G> struct PullState {
 // The tiles of a workgroup.  True where units were left out that hold values which cannot be split: the second
 // run (WHOLE) takes these, with the fp32 instruction.  Apart, so that it keeps no registers in the first.
 template <int N, int G, int P, bool FRESH, bool WHOLE>
-__device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__restrict__ x, const float *gy, float *gx, float *row,
-                                           char *lds, PullShared &shared, int tid, int wave, int blocks, int c0, int wgs, int wg,
-                                           PullState<G> &state)
+__device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__restrict__ x, const float *gy, float *gx, char *lds,
+                                           PullShared &shared, int tid, int wave, int blocks, int c0, int wgs, int wg, PullState<G> &state)
 {
     using S = PullShape<G, P>;
     constexpr int kSegs = S::kSegs, kSteps = S::kSteps, kTiles = S::kTiles, kUnit = S::kUnit, kUnits = S::kUnits, kVec = S::kVec;
@@ -287,7 +270,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
 #pragma unroll
         for (int i = 0; i < kVec; i++) {
             float v4[4];
-            load_global_vec4_unaligned(base, min(at + (uint32_t)(kChannels * i) * plane, last) + un.at, v4);
+            load_global_vec_unaligned<4>(base, min(at + (uint32_t)(kChannels * i) * plane, last) + un.at, v4);
             d[i] = f32x4_t{v4[0], v4[1], v4[2], v4[3]};
         }
     };
@@ -791,7 +774,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         int round = 0;
         for (int tile = lb; tile < a.tiles; tile += wgs) {          // uniform over the workgroup
             gathered(here, round++);
-            tile_sync();
+            lds_sync();
             const Tile then = tile_of(tile + wgs);
             here = locate(then, segment);
             if (active) {
@@ -812,7 +795,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                 gather(then, here);
             }
             now = then;
-            tile_sync();
+            lds_sync();
         }
         return again;
     }
@@ -870,14 +853,14 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
 #pragma unroll
     for (int t = 0; t < kTiles; t++) state.sums[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     shared.bias_sums[tid] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    const bool again = pull_tiles<N, G, P, FRESH, false>(a, x, gy, gx, row, lds, shared, tid, wave, blocks, c0, wgs, wg, state);
+    const bool again = pull_tiles<N, G, P, FRESH, false>(a, x, gy, gx, lds, shared, tid, wave, blocks, c0, wgs, wg, state);
     if (lane == 0 && again) shared.bad_again = 1;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(shared.bad_again) != 0) {    // uniform over the workgroup
         int tid2 = tid;
         asm volatile("" : "+v"(tid2));           // (nothing of the first run is kept for the second)
         load_weights(true);
-        pull_tiles<N, G, P, FRESH, true>(a, x, gy, gx, row, lds, shared, tid2, wave, blocks, c0, wgs, wg, state);
+        pull_tiles<N, G, P, FRESH, true>(a, x, gy, gx, lds, shared, tid2, wave, blocks, c0, wgs, wg, state);
     }
 
     // the sums, of the waves that share a block through LDS

@@ -271,20 +271,6 @@ __global__ __launch_bounds__(kSlabs *kTiles *kWave) void push_table(const SplitA
     for (int p = 0; p < 3; p++) table[((step * kSlabs * kTiles + t) * 3 + p) * kWave + lane] = s.p[p];
 }
 
-// LDS accesses of one wave: executed in order, only the compiler has to be kept from reordering them.
-__device__ __forceinline__ void own_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-// Of a workgroup (of LDS only: the loads of x and the stores of z stay in flight).
-__device__ __forceinline__ void all_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 // A row of 16 bytes pieces lies at piece ^ turn(row): what is read transposed meets all banks once.
 __device__ __forceinline__ uint32_t turn(uint32_t row) { return row / 2 % 4 * 2 + row / 8 % 2; }
 
@@ -342,7 +328,7 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
             uint64_t base = image + (uint64_t)c * (uint64_t)(a.xsc * 4);
             asm volatile("" : "+s"(base));
             float v[4];
-            load_global_vec4_unaligned(base, min(lane_plane, (uint32_t)min(a.C - 1 - c, 3) * plane) + at, v);
+            load_global_vec_unaligned<4>(base, min(lane_plane, (uint32_t)min(a.C - 1 - c, 3) * plane) + at, v);
             xv[i] = f32x4_t{v[0], v[1], v[2], v[3]};
         }
     };
@@ -376,10 +362,10 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
             float rest = 0.f;
             for (int step = 0; step < steps; step++) {
                 if (!resident && step % kTableSteps == 0) {                        // uniform over the workgroup
-                    all_sync();
+                    lds_sync();
                     const int count = min(kTableSteps, steps - step) * kStepEntries;
                     for (int i = tid; i < count; i += kPushWaves * kWave) weights[i] = table[step * kStepEntries + i];
-                    all_sync();
+                    lds_sync();
                 }
                 const auto [id, n, q] = fresh();
                 // the lane at the row end has loaded voxels further left

@@ -102,15 +102,16 @@ __device__ __forceinline__ void load_global_vec(uint64_t base, uint32_t byte_off
         for (int i = 0; i < V; i++) d[i] = v[i];
     }
 }
-// Four consecutive floats at an address that is only known to be a multiple of four bytes.
-__device__ __forceinline__ void load_global_vec4_unaligned(uint64_t base, uint32_t byte_offset, float (&d)[4])
+// V consecutive floats at an address that is only known to be a multiple of four bytes.
+template <int V>
+__device__ __forceinline__ void load_global_vec_unaligned(uint64_t base, uint32_t byte_offset, float (&d)[V])
 {
-    typedef float vec_t __attribute__((ext_vector_type(4), aligned(4)));
+    typedef float vec_t __attribute__((ext_vector_type(V), aligned(4)));
     typedef const __attribute__((address_space(1))) char *gbytes_t;
     gbytes_t p = reinterpret_cast<gbytes_t>(base) + byte_offset;
     const vec_t v = *reinterpret_cast<const __attribute__((address_space(1))) vec_t *>(p);
 #pragma unroll
-    for (int i = 0; i < 4; i++) d[i] = v[i];
+    for (int i = 0; i < V; i++) d[i] = v[i];
 }
 template <int V>
 __device__ __forceinline__ void store_global_vec(uint64_t base, uint32_t byte_offset, const float (&d)[V])
