@@ -15,7 +15,7 @@
 // loop, as  out[x] = T_0[fold(x - dil)] + T_1[x] + T_2[fold(x + dil)]  through LDS.
 // The channel loop is therefore: one aligned V-wide load per input row, then
 // 3*V fused multiply-adds per (output row, tap row) pair, with wave-uniform
-// weights from scalar registers.
+// weights (copied from scalar to vector registers).
 //
 // The input channels are split over KS groups of lanes of the workgroup
 // (channel ci goes to group ci % KS), which multiplies the number of waves in
@@ -95,6 +95,16 @@ __device__ __forceinline__ bool tile_origin(const Geom &g, const Lattice &lt, in
 // (at most 30 KB), six rows of one of 4 x 4 (at most 36 KB; its registers leave room for two workgroups of 512 lanes), which
 // costs no resident workgroup (61 x 93 x 75, depth 20: 364 -> 358 us; 40 x 45 x 47, depth 30, in four groups: 366 -> 323).  2D: one at a time (256 x 256, depth 10: half tiles are 3 us slower).
 constexpr int finish_batch(int ndim, int V, int rows) { return ndim == 2 || V > 1 ? 1 : rows <= 10 ? (rows + 1) / 2 : 6; }
+
+// The channel loop's weights: a multiply-add of three vector registers issues in 2.4 cycles of a SIMD, one with a scalar
+// operand in 4.3, as does this copy, which eight (2 x 4 rows) or more multiply-adds share.  128^3 over 8 / 16 / 30 channels: 26.7, 23.0 / 40.8, 35.4 /
+// 68.8, 60.9 us; 61 x 93 x 75 over 20: 24.6, 19.9; 256^3 over 30: 559, 541 (the memory's).
+__device__ __forceinline__ float in_vector_register(float uniform)
+{
+    float copy;
+    asm volatile("v_mov_b32 %0, %1" : "=v"(copy) : "s"(uniform));   // (volatile: where it is written, and not all at once)
+    return copy;
+}
 
 // ONE (3D): all channels in one group.  A channel's nine products are summed before they are added: in one chain over
 // all channels the error would be a third larger than with two groups (as it is, it is a fifth smaller).
@@ -192,37 +202,42 @@ __global__ __launch_bounds__(NDIM == 3 ? 512 : 1024, (NDIM == 3 && V == 1 && WOU
             for (int my = 0; my < LY; my++) load_global_vec<V>(xz, offyx[my], xv[mz][my]);
         }
         if constexpr (WOUT == 1) __builtin_amdgcn_sched_barrier(0);
-        // output rows past the image edge (partial lattices) are skipped, uniformly per workgroup
+        // (rows past the image edge are formed as well: what they would save is less than the branches around them)
+        if constexpr (ONE) {
 #pragma unroll
-        for (int jz = 0; jz < RZ; jz++) {
-            if (jz >= nzv) break;
+            for (int r = 0; r < 3; r++) {
+                float wv[9];
 #pragma unroll
-            for (int jy = 0; jy < RY; jy++) {
-                if (jy >= nyv) break;
-                if constexpr (ONE) {
+                for (int t = 0; t < 9; t++) wv[t] = in_vector_register(w[0][t * 3 + r]);
 #pragma unroll
-                    for (int r = 0; r < 3; r++) {
-                        float one = xv[jz][jy][0] * w[0][r];
+                for (int jz = 0; jz < RZ; jz++)
 #pragma unroll
-                        for (int t = 1; t < 9; t++) one += xv[jz + t / 3][jy + t % 3][0] * w[0][t * 3 + r];
+                    for (int jy = 0; jy < RY; jy++) {
+                        float one = xv[jz][jy][0] * wv[0];
+#pragma unroll
+                        for (int t = 1; t < 9; t++) one += xv[jz + t / 3][jy + t % 3][0] * wv[t];
                         acc[0][jz][jy][r][0] += one;
                     }
-                    continue;
-                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
 #pragma unroll
-                for (int p = 0; p < NZ; p++)
+            for (int pq = 0; pq < NZ * 3; pq++)
 #pragma unroll
-                    for (int q = 0; q < 3; q++)
+                for (int co = 0; co < WOUT; co++) {
 #pragma unroll
-                        for (int co = 0; co < WOUT; co++)
+                    for (int r = 0; r < 3; r++) {
+                        const float wv = in_vector_register(w[co][pq * 3 + r]);
 #pragma unroll
-                            for (int r = 0; r < 3; r++) {
-                                const float wv = w[co][(p * 3 + q) * 3 + r];
+                        for (int jz = 0; jz < RZ; jz++)
+#pragma unroll
+                            for (int jy = 0; jy < RY; jy++)
 #pragma unroll
                                 for (int i = 0; i < V; i++)
-                                    acc[co][jz][jy][r][i] += xv[NDIM == 3 ? jz + p : 0][jy + q][i] * wv;
-                            }
-            }
+                                    acc[co][jz][jy][r][i] += xv[NDIM == 3 ? jz + pq / 3 : 0][jy + pq % 3][i] * wv;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);    // (no more copies ahead than there are registers for)
+                }
         }
     }
 
@@ -428,12 +443,14 @@ hipError_t pick(const Geom &g, const View<const float> &x, const float *k, const
                 if (streams && split <= 1 && t44 * waves >= 4096 && t44 * 32 <= t24 * 17)
                     return launch<3, RELU, 1, 1, 4, 4, true>(g, x, k, bias, out, s, sums);
                 // The channels in one group where few of them leave the finishing step a large part and the tiles fill
-                // the chip without more waves (192^3 over 5 / 8 / 12 channels: 64, 50 / 80, 67 / 107, 99; over 20:
-                // 169, 175), in four where the tiles leave most of it idle (64^3 over 20 / 45: 18, 16 / 33, 23;
-                // 40 x 45 x 47 over 45: 27, 17; 61 x 93 x 75, 1500 waves, over 20: 25, 25; over 12: 18, 19).
+                // the chip without more waves (192^3 over 4 / 12 channels: 57, 41 / 97, 94; over 20:
+                // 159, 166), in four, from two channels each, where the tiles leave most of it idle (64^3 over 8 / 20 / 45: 9.9, 8.7 /
+                // 15, 12 / 27, 19; 61 x 93 x 75, 1500 waves, over 12 / 20: 15.2, 16.7 / 20.7, 21.2), in eight where they leave nearly all of it
+                // (40 x 45 x 47 over 30: 12.7, 11.2; 32^3 over 10: 6.9, 6.5, over 4 in four: 6.2, 5.4; 64^3 over 20: 11.9, 12.1).
                 const bool full = t24 * waves >= 7000;
                 const bool one = (full && g.C <= 12 && split < 0) || split == 1;
-                const int groups = t24 * waves <= 1100 && g.C >= 12 ? 4 : 2;
+                const bool few = t24 * waves <= 400;
+                const int groups = t24 * waves > 1100 || g.C < (few ? 4 : 8) ? 2 : few && g.C >= 10 ? 8 : 4;
                 // Lattices of 3 x 3 rows instead of 2 x 4 where they cover the residue classes
                 // with at least 1/16 fewer tiles (a partly filled lattice costs as much time as a
                 // full one): at 128^3 dilations 3, 5, 9, 10, by 2 to 12 %.  Not at dilations 1
