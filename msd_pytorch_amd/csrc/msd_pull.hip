@@ -1209,6 +1209,9 @@ hipError_t pull_launch(const PullArgs &a, int wgs, const float *x, const float *
     return hipGetLastError();
 }
 
+// Blocks of a chunk, at most (one slab: 411 us over 100 channels, 463 with 8).
+int most_blocks(int slabs) { return slabs == 1 ? 4 : kWaves; }
+
 // As many workgroups as are resident, shared out over the chunks by their size.
 struct PullPlan {
     Chunks chunks;
@@ -1220,7 +1223,7 @@ PullPlan pull_plan(int64_t batch, int64_t rows, int64_t span, int64_t channels, 
     PullPlan p;
     const int nb = (int)((channels + 15) / 16);
     Chunks &c = p.chunks;
-    const int most = slabs == 1 ? 4 : kWaves;     // blocks of a chunk (one slab: 411 us over 100 channels, 463 with 8)
+    const int most = most_blocks(slabs);
     c.n = (nb + most - 1) / most;
     c.blocks = (nb + c.n - 1) / c.n;
     c.large = nb - c.n * (c.blocks - 1);
@@ -1242,6 +1245,27 @@ int64_t pull_floats(const PullPlan &p, int slabs)
     return (int64_t)p.wgs * slabs * (p.chunks.blocks * 1024 + kBiasColumns);
 }
 
+// Channels of a launch: those of one full chunk, where there are 2^18 voxels, else all of them.  A chunk of five to eight blocks takes nearly the
+// same time however many of its waves have a block (2048 x 2048, 14 outputs: 1.46, 1.54, 1.63, 1.61 ms over 5, 6, 7, 8), four 0.95, two 0.58
+// and one 0.44: full chunks and a small rest in a launch of its own take less than chunks of one size that share the chip (9 blocks: 2.75
+// ms as 5 + 4, 2.05 as 8 + 1).  Small images have too few tiles for launches one after the other.  Training step, two channels per layer, depth 100, us:
+// 256 x 256 2488, 2539; 384 x 384 3623, 3646; 512 x 512 4544, 4448; 1000 x 700 10526, 10286; depth 200: 2048 x 2048 88.1, 84.0 ms; depth 90: 100^3 35.5,
+// 33.7 ms.
+int64_t pull_channels(int64_t batch, int64_t rows, const PullPlan &p, int64_t channels, int slabs)
+{
+    const bool alone = batch * rows * p.segs >= (1 << 18) / kSegment;
+    return alone ? std::min<int64_t>(channels, 16 * most_blocks(slabs)) : channels;
+}
+// Floats of the largest of the launches.
+int64_t all_pull_floats(int64_t batch, int64_t rows, int64_t span, int64_t channels, int slabs)
+{
+    const PullPlan p = pull_plan(batch, rows, span, channels, slabs);
+    const int64_t step = pull_channels(batch, rows, p, channels, slabs), rest = channels % step;
+    int64_t most = std::max(pull_floats(p, slabs), pull_floats(pull_plan(batch, rows, span, step, slabs), slabs));
+    if (rest > 0) most = std::max(most, pull_floats(pull_plan(batch, rows, span, rest, slabs), slabs));
+    return most;
+}
+
 }  // namespace
 }  // namespace group2d
 
@@ -1249,7 +1273,7 @@ int64_t group_pull_floats(int64_t batch, int64_t rows, int64_t W, int64_t channe
 {
     using namespace group2d;
     // (volumes without gaps have fewer segments, and so no more workgroups)
-    return std::max(pull_floats(pull_plan(batch, rows, W, channels, 1), 1), pull_floats(pull_plan(batch, rows, W, channels, 2), 2));
+    return std::max(all_pull_floats(batch, rows, W, channels, 1), all_pull_floats(batch, rows, W, channels, 2));
 }
 
 bool group_pull_supported(const Geom &g, const View<const float> &x, const View<float> &gx)
@@ -1266,16 +1290,14 @@ bool group_pull_supported(const Geom &g, const View<const float> &x, const View<
 namespace {
 
 // gy: the outputs' gradients, channels gsc apart, rows as in x.  fresh: the gradients are written, not added to (one slab;
-// images, volumes without gaps).
-hipError_t pull(const Geom &g, const View<const float> &x, const float *gy, int64_t gsb, int64_t gsc, const group2d::Outputs &out,
-                int update, int mask_from, const View<float> &grads, const int *channels, float *const *gk, float *gb, float *ws,
-                bool reverse, bool fresh, hipStream_t s)
+// images, volumes without gaps).  gb: null where another launch forms the bias gradients.
+hipError_t pull_part(const Geom &g, const View<const float> &x, const float *gy, int64_t gsb, int64_t gsc, const group2d::Outputs &out,
+                     int update, int mask_from, const View<float> &grads, const int *channels, float *const *gk, float *gb, float *ws,
+                     bool reverse, bool fresh, hipStream_t s)
 {
     using namespace group2d;
     const int per_slab = g.ndim == 3 ? kSlabOut3d : kSlabOut;
     const Form form = form_of(g, x);
-    if (out.n < 1 || out.n > 2 * per_slab || !group_pull_supported(g, x, grads) || (fresh && (form == kVolume || out.n > per_slab)))
-        return hipErrorInvalidValue;
     const int slabs = out.n > per_slab ? 2 : 1;
     const int span = form == kFlat ? g.nvox : g.W, rows = g.nvox / span;
     const PullPlan p = pull_plan(g.B, rows, span, g.C, slabs);
@@ -1320,8 +1342,43 @@ hipError_t pull(const Geom &g, const View<const float> &x, const float *gy, int6
     sum.n = out.n;
     sum.fresh = fresh;
     sum.gb = gb;
-    hipLaunchKernelGGL(g.ndim == 3 ? sum_group<kVolume> : sum_group<kImage>, dim3(sum.columns / kWave + 1), dim3(1024), 0, s, sum, ws, bias_part);
+    // (the last workgroup takes the biases)
+    hipLaunchKernelGGL(g.ndim == 3 ? sum_group<kVolume> : sum_group<kImage>, dim3(sum.columns / kWave + (gb ? 1 : 0)), dim3(1024), 0, s, sum, ws, bias_part);
     return hipGetLastError();
+}
+
+hipError_t pull(const Geom &g, const View<const float> &x, const float *gy, int64_t gsb, int64_t gsc, const group2d::Outputs &out,
+                int update, int mask_from, const View<float> &grads, const int *channels, float *const *gk, float *gb, float *ws,
+                bool reverse, bool fresh, hipStream_t s)
+{
+    using namespace group2d;
+    const int per_slab = g.ndim == 3 ? kSlabOut3d : kSlabOut;
+    const Form form = form_of(g, x);
+    if (out.n < 1 || out.n > 2 * per_slab || !group_pull_supported(g, x, grads) || (fresh && (form == kVolume || out.n > per_slab)))
+        return hipErrorInvalidValue;
+    const int slabs = out.n > per_slab ? 2 : 1, taps = g.ndim == 3 ? 27 : group2d::kTaps;
+    const int span = form == kFlat ? g.nvox : g.W, rows = g.nvox / span;
+    const int step = (int)pull_channels(g.B, rows, pull_plan(g.B, rows, span, g.C, slabs), g.C, slabs);
+    for (int from = 0; from < g.C; from += step) {
+        Geom part = g;
+        View<const float> xp = x;
+        View<float> gp = grads;
+        Outputs op = out;
+        int reads[kMaxOut];
+        float *gkp[kMaxOut];
+        part.C = std::min(step, g.C - from);
+        xp.p += from * x.sc;
+        gp.p += from * grads.sc;
+        for (int o = 0; o < out.n; o++) {
+            reads[o] = std::max(channels[o] - from, 0);
+            if (from < update) op.k[o] += (int64_t)from * taps;      // (an output reads at least these; other weights are not needed)
+            gkp[o] = reads[o] > 0 ? gk[o] + (int64_t)from * taps : gk[o];
+        }
+        const hipError_t e = pull_part(part, xp, gy, gsb, gsc, op, std::min(std::max(update - from, 0), part.C), mask_from - from, gp, reads,
+                                       gkp, from == 0 ? gb : nullptr, ws, reverse, fresh, s);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace

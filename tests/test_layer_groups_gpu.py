@@ -65,6 +65,18 @@ def test_block_backward_in_layer_groups(case, input_grad):
         check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=43, input_grad=input_grad)
 
 
+# From 2^18 voxels on the channels go in launches of one chunk each (128 of them for more than seven outputs, 64 for fewer): a rest
+# of one channel and of several blocks, with and without gradients of the channels that the rest holds, several images, a volume.
+@pytest.mark.parametrize("input_grad", [True, False])
+@pytest.mark.parametrize("size, c_in, width, depth, batch", [
+    ((512, 513), 122, 1, 8, 1), ((260, 512), 128, 1, 10, 2), ((515, 512), 140, 2, 7, 1), ((512, 520), 250, 1, 8, 1),
+    ((512, 515), 70, 1, 6, 1), ((64, 66, 65), 130, 1, 4, 1), ((65, 64, 66), 64, 1, 2, 1)],
+    ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_backward_groups_over_several_chunks(size, c_in, width, depth, batch, input_grad):
+    check_block(len(size), size, c_in, width, depth, batch, dilations=[1 + 3 * i % 10 for i in range(depth)], seed=47,
+                input_grad=input_grad)
+
+
 # Groups of eight to fourteen outputs: two slabs of 64 matrix rows, the upper outputs' share of the lower
 # channels in one launch.  Blocks of 16 channels shared by four, two or one waves (1, 2 | 3, 4 | 5 to 8 blocks),
 # two chunks; tiles of four segments that end inside an image, also between two images; halves of 7 + 7, 7 + 1,
