@@ -984,8 +984,8 @@ __global__ __launch_bounds__(1024) void sum_group(const SumArgs a, const float *
 // in the group.
 //
 // One voxel per lane; the nine (27) values of each output come straight from the caches (a group's planes
-// were written or read by the launches before), with no LDS and no barrier: the launches are bound by
-// their ramp and by the vector cache.
+// were written or read by the launches before), not by way of LDS: the launches are bound by
+// their ramp, the vector cache and, with scalar weights, the multiply-adds.
 struct FinishArgs {
     int D, H, W, span, segs, items, dmax;         // (as in PullArgs, segments of 64)
     Divisor by_rows, by_voxels;
@@ -1078,13 +1078,23 @@ __device__ __forceinline__ void finish_fold(const FinishArgs &a, const FinishPla
 
 // The NOUT channels of one layer from the NQ outputs right above, and the channels' ReLU mask: with it
 // they are complete.
+//
+// Images with several outputs above take the weights through LDS into vector registers (see spread_back): 1000 x 1000, two channels
+// from 2 / 4 / 6 outputs 9.8, 8.6 / 13.7, 11.3 / 18.7, 15.3 us; 1024 x 1024, one from 6: 12.6, 12.3; 3 x 333 x 477: 8.9, 8.1.  One output
+// (4.8, 5.0) and volumes (128^3, one channel from 3: 37.3, 40.4) keep scalar ones.
 template <int N, int NQ, int NOUT>
 __global__ __launch_bounds__(256) void finish_back(const FinishArgs a, const float *__restrict__ act, float *g)
 {
     constexpr int kTaps = Gather<N>::kTaps;
     const int lb = block_for_xcd(blockIdx.x, gridDim.x, true);
-    const int it = lb * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    if (it >= a.items) return;                    // uniform over the wave
+    const int it0 = lb * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), it = min(it0, a.items - 1);
+    constexpr bool kStage = N == kImage && NQ > 1;
+    if (!kStage && it0 >= a.items) return;        // uniform over the wave
+    constexpr int kRow = (NOUT * kTaps + 3) / 4 * 4;                // an output's weights, in whole pieces of 16 bytes
+    __shared__ __attribute__((aligned(16))) float weights[kStage ? NQ * kRow : 4];
+    static_assert(!kStage || NQ * kRow <= 256, "a weight per thread");
+    float w = 0.f;
+    if constexpr (kStage) w = a.k[min((int)threadIdx.x / kRow, NQ - 1)][min((int)threadIdx.x % kRow, NOUT * kTaps - 1)];
     const FinishPlace p = finish_place<N>(a, it);
     const uint64_t img = reinterpret_cast<uint64_t>(g) + (uint64_t)p.img;
     const uint64_t ximg = reinterpret_cast<uint64_t>(act) + (uint64_t)p.img;
@@ -1098,6 +1108,11 @@ __global__ __launch_bounds__(256) void finish_back(const FinishArgs a, const flo
     float A[NQ][Gather<N>::kLines][3];
 #pragma unroll
     for (int o = 0; o < NQ; o++) finish_gather<N>(a, p, img + (uint64_t)(NOUT + o) * plane, a.dil[o], A[o]);
+    if constexpr (kStage) {
+        if (threadIdx.x < NQ * kRow) weights[threadIdx.x] = w;
+        __syncthreads();
+        if (it0 >= a.items) return;               // uniform over the wave
+    }
     if (!p.away) {
 #pragma unroll
         for (int o = 0; o < NQ; o++) finish_fold<N>(a, p, a.dil[o], A[o]);
@@ -1109,7 +1124,7 @@ __global__ __launch_bounds__(256) void finish_back(const FinishArgs a, const flo
         for (int o = 0; o < NQ; o++) {
             float one = 0.f;
 #pragma unroll
-            for (int t = 0; t < kTaps; t++) one += a.k[o][c * kTaps + t] * A[o][t / 3][t % 3];
+            for (int t = 0; t < kTaps; t++) one += (kStage ? weights[o * kRow + c * kTaps + t] : a.k[o][c * kTaps + t]) * A[o][t / 3][t % 3];
             all += one;
         }
         sum[c] += all;
