@@ -15,7 +15,7 @@
 // loop, as  out[x] = T_0[fold(x - dil)] + T_1[x] + T_2[fold(x + dil)]  through LDS.
 // The channel loop is therefore: one aligned V-wide load per input row, then
 // 3*V fused multiply-adds per (output row, tap row) pair, with wave-uniform
-// weights (copied from scalar to vector registers).
+// weights (read into scalar registers; COPY: copied from these to vector registers).
 //
 // The input channels are split over KS groups of lanes of the workgroup
 // (channel ci goes to group ci % KS), which multiplies the number of waves in
@@ -96,9 +96,9 @@ __device__ __forceinline__ bool tile_origin(const Geom &g, const Lattice &lt, in
 // costs no resident workgroup (61 x 93 x 75, depth 20: 364 -> 358 us; 40 x 45 x 47, depth 30, in four groups: 366 -> 323).  2D: one at a time (256 x 256, depth 10: half tiles are 3 us slower).
 constexpr int finish_batch(int ndim, int V, int rows) { return ndim == 2 || V > 1 ? 1 : rows <= 10 ? (rows + 1) / 2 : 6; }
 
-// The channel loop's weights: a multiply-add of three vector registers issues in 2.4 cycles of a SIMD, one with a scalar
-// operand in 4.3, as does this copy, which eight (2 x 4 rows) or more multiply-adds share.  128^3 over 8 / 16 / 30 channels: 26.7, 23.0 / 40.8, 35.4 /
-// 68.8, 60.9 us; 61 x 93 x 75 over 20: 24.6, 19.9; 256^3 over 30: 559, 541 (the memory's).
+// The channel loop's weights where COPY is set: a multiply-add of three vector registers issues in 2.4 cycles of a SIMD, one with a
+// scalar operand in 4.3, as does this copy, which the multiply-adds of all rows of the tile (and V voxels) share.  128^3 over 8 / 16 / 30
+// channels: 26.7, 23.0 / 40.8, 35.4 / 68.8, 60.9 us; 61 x 93 x 75 over 20: 24.6, 19.9; 256^3 over 30: 559, 541 (the memory's).
 __device__ __forceinline__ float in_vector_register(float uniform)
 {
     float copy;
@@ -106,9 +106,13 @@ __device__ __forceinline__ float in_vector_register(float uniform)
     return copy;
 }
 
+// COPY: the weights are multiplied by from vector registers, and rows past the image edge are formed as well (what they would
+// save in a full tile is less than the branches around them); else from scalar registers, and such rows are skipped
+// (copies_weights).
+//
 // ONE (3D): all channels in one group.  A channel's nine products are summed before they are added: in one chain over
 // all channels the error would be a third larger than with two groups (as it is, it is a fifth smaller).
-template <int NDIM, bool RELU, int WOUT, int V, int RZ, int RY, bool ONE = false>
+template <int NDIM, bool RELU, int WOUT, int V, int RZ, int RY, bool ONE, bool COPY>
 __global__ __launch_bounds__(NDIM == 3 ? 512 : 1024, (NDIM == 3 && V == 1 && WOUT == 1) ? (RZ * RY > 9 ? 4 : ONE ? 7 : 8) : 1) void fwd_lattice(Geom g, Lattice lt, int remap, View<const float> x,
                                                     const float *__restrict__ k, const float *__restrict__ bias,
                                                     View<float> out)
@@ -202,8 +206,36 @@ __global__ __launch_bounds__(NDIM == 3 ? 512 : 1024, (NDIM == 3 && V == 1 && WOU
             for (int my = 0; my < LY; my++) load_global_vec<V>(xz, offyx[my], xv[mz][my]);
         }
         if constexpr (WOUT == 1) __builtin_amdgcn_sched_barrier(0);
-        // (rows past the image edge are formed as well: what they would save is less than the branches around them)
-        if constexpr (ONE) {
+        if constexpr (!COPY) {
+            // output rows past the image edge (partial lattices) are skipped, uniformly per workgroup
+#pragma unroll
+            for (int jz = 0; jz < RZ; jz++) {
+                if (jz >= nzv) break;
+#pragma unroll
+                for (int jy = 0; jy < RY; jy++) {
+                    if (jy >= nyv) break;
+                    if constexpr (ONE) {
+#pragma unroll
+                        for (int r = 0; r < 3; r++) {
+                            float one = xv[jz][jy][0] * w[0][r];
+#pragma unroll
+                            for (int t = 1; t < 9; t++) one += xv[jz + t / 3][jy + t % 3][0] * w[0][t * 3 + r];
+                            acc[0][jz][jy][r][0] += one;
+                        }
+                        continue;
+                    }
+#pragma unroll
+                    for (int pq = 0; pq < NZ * 3; pq++)
+#pragma unroll
+                        for (int co = 0; co < WOUT; co++)
+#pragma unroll
+                            for (int r = 0; r < 3; r++)
+#pragma unroll
+                                for (int i = 0; i < V; i++)
+                                    acc[co][jz][jy][r][i] += xv[NDIM == 3 ? jz + pq / 3 : 0][jy + pq % 3][i] * w[co][pq * 3 + r];
+                }
+            }
+        } else if constexpr (ONE) {
 #pragma unroll
             for (int r = 0; r < 3; r++) {
                 float wv[9];
@@ -356,6 +388,18 @@ inline bool make_lattice(const Geom &g, int V, int rz, int ry, int ks_wanted, La
     return true;
 }
 
+// Whether the weights are copied: where some tile lies inside the image with all of its rows.  Images with fewer slices or rows per
+// residue class have none, and there the rows past the edge cost more than scalar operands do.  us, scalar operands and
+// copies, 30 channels: half of a tile's rows, 8 x 512 x 512 at dilation 8 83, 93, 3 x 512 x 512 at 3 39, 48; a third,
+// 256 x 8 x 256 at 8 27, 40; two thirds, 64 x 12 x 300 at 6 34.5, 33.9, 512 x 16 x 512 over 8 channels at 9 15 % more; two
+// outputs, 16 x 512 at 8 12.6, 15.5.  Where only some tiles are whole it is these that decide: 12 x 300 x 300 at 10 (0.56 of all
+// rows inside) 91, 82; 512 x 24 x 512 over 21 channels at 5 (0.66) 13 % less.
+inline bool copies_weights(const Geom &g, int rz, int ry)
+{
+    const int rows_y = (g.H + g.dil - 1) / g.dil, rows_z = g.ndim == 3 ? (g.D + g.dil - 1) / g.dil : 1;
+    return rows_z >= rz && rows_y >= ry;
+}
+
 template <int NDIM, bool RELU, int WOUT, int V, int RZ, int RY, bool ONE = false>
 hipError_t launch(const Geom &g, const View<const float> &x, const float *k, const float *bias,
                   const View<float> &out, hipStream_t s, const ForwardSums *sums, int groups = 2)
@@ -368,9 +412,15 @@ hipError_t launch(const Geom &g, const View<const float> &x, const float *k, con
     const int remap = knob(kKnobXcdRemap, 1);
     const dim3 grid(remap ? xcd_grid(lt.ntiles) : lt.ntiles, g.B, 1);
     const size_t lds = (size_t)lt.ks * finish_batch(NDIM, V, RZ * RY) * 3 * V * lt.lpr * sizeof(float);
-    hipLaunchKernelGGL((fwd_lattice<NDIM, RELU, WOUT, V, RZ, RY, ONE>), grid, dim3(lt.ks * lt.lpr), lds, s, g, lt, remap, x,
-                       k, bias, out);
-    return hipGetLastError();
+    auto with = [&](auto copy) {
+        hipLaunchKernelGGL((fwd_lattice<NDIM, RELU, WOUT, V, RZ, RY, ONE, decltype(copy)::value>), grid, dim3(lt.ks * lt.lpr), lds, s, g,
+                           lt, remap, x, k, bias, out);
+        return hipGetLastError();
+    };
+    // (3D with several voxels per lane: only by the setting)
+    if constexpr (NDIM == 2 || V == 1)
+        if (!copies_weights(g, RZ, RY)) return with(std::false_type{});
+    return with(std::true_type{});
 }
 
 // Largest V whose accesses are aligned in both views and that leaves at least

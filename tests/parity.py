@@ -142,3 +142,36 @@ def check_block(ndim, size, c_in, width, depth, batch, dilations=None, seed=0, i
     assert rel_err(bd.grad, want_gb) <= 1e-4, "grad_bias"
     worst = max((rel_err(a.grad, b), i) for i, (a, b) in enumerate(zip(wd, want_gw)))
     assert worst[0] <= 1e-4, "grad_weight of layer %d" % worst[1]
+
+
+def captured_kernels(run):
+    """The names (mangled) of the kernels that run() launches, in order: it is recorded into a graph and not executed."""
+    import ctypes
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    hip = ctypes.CDLL(path)
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    hip.hipKernelNameRefByPtr.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+
+    class Dim(ctypes.Structure):
+        _fields_ = [(c, ctypes.c_uint32) for c in "xyz"]
+
+    class KernelNode(ctypes.Structure):          # hipKernelNodeParams
+        _fields_ = [("block", Dim), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", Dim), ("params", ctypes.c_void_p),
+                    ("shared", ctypes.c_uint)]
+
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        run()
+    raw, count = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(count)) == 0
+    nodes = (ctypes.c_void_p * count.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(count)) == 0
+    names = []
+    for node in nodes:
+        kind, params = ctypes.c_int(), KernelNode()
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
+        if kind.value != 0:                      # (0: a kernel)
+            continue
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(params)) == 0
+        names.append(hip.hipKernelNameRefByPtr(params.func, None).decode())
+    return names

@@ -1,0 +1,58 @@
+"""How the forward kernel takes its weights: from vector registers, where it forms all rows of a tile, also those past the
+image edge, or from scalar registers, where it skips such rows."""
+import re
+
+import pytest
+import torch
+
+from cases import make_problem, problem_on
+from parity import captured_kernels, check_operator_problem
+from test_knobs_gpu import tuning
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def cc():
+    from msd_pytorch_amd import msd_custom_convolutions
+    return msd_custom_convolutions
+
+
+def forward_instances(cc, shape):
+    """The template arguments of each launch of fwd_lattice that a layer's forward pass makes, as numbers."""
+    p = problem_on(make_problem(shape, torch.float32), "cuda")
+    names = captured_kernels(lambda: cc.conv_relu_forward(p["x"], p["k"], p["bias"], p["y"], p["d"]))
+    found = [re.search(r"fwd_latticeI((?:L[ib]\d+E)+)E", n) for n in names]
+    return [[int(v) for v in re.findall(r"L[ib](\d+)E", m.group(1))] for m in found if m]
+
+
+# (settings, (B, C_in, C_out, spatial, dilation), copies): volumes and images with fewer slices or rows per residue class than a tile of
+# the instance has, and with exactly as many, for each tile and number of outputs; one channel group and several.
+THIN = [({}, s, c) for s, c in (
+    ((1, 5, 1, (2, 23, 70), 2), 0), ((1, 14, 1, (3, 20, 64), 2), 1), ((2, 9, 1, (23, 3, 40), 3), 0), ((1, 4, 1, (23, 6, 40), 2), 0),
+    ((1, 4, 1, (23, 7, 40), 2), 1), ((1, 30, 1, (8, 9, 130), 8), 0), ((1, 5, 2, (4, 33, 66), 4), 0), ((1, 5, 2, (5, 25, 66), 4), 1))]
+THIN += [({"fwd.lattice3d": m}, s, c) for m, s, c in (
+    (24, (1, 7, 1, (9, 3, 40), 3), 0), (33, (1, 7, 1, (6, 9, 40), 3), 0), (33, (1, 7, 1, (7, 9, 40), 3), 1), (44, (1, 7, 1, (6, 16, 40), 2), 0),
+    (44, (1, 20, 1, (16, 3, 65), 2), 0), (44, (1, 7, 1, (7, 16, 40), 2), 1))]
+THIN += [({"fwd.split": 1, "fwd.lattice3d": 0}, s, c) for s, c in (
+    ((1, 7, 1, (1, 12, 40), 1), 0), ((1, 7, 1, (27, 6, 40), 3), 0), ((1, 7, 1, (27, 7, 40), 3), 1))]
+THIN += [({"fwd.rows2d": r, "fwd.vec2d": v}, (2, 6, 1, (3 * r - 3, 256 if v == 4 else 128 if v == 2 else 70), 3), 0)
+         for r in (2, 3, 4, 5, 6) for v in (1, 2, 4)]
+THIN += [({"fwd.vec2d": v}, (1, 6, 2, (4, 256 if v == 4 else 128 if v == 2 else 71), 2), 0) for v in (1, 2, 4)]
+
+
+def _id(case):
+    settings, s, _ = case
+    return ",".join("%s=%d" % kv for kv in settings.items()) + "-B%d-C%d-w%d-%s-d%d" % (*s[:3], "x".join(map(str, s[3])), s[4])
+
+
+@pytest.mark.parametrize("case", THIN, ids=_id)
+def test_rows_past_the_edge_are_skipped_where_no_tile_is_whole(cc, case):
+    settings, shape, copies = case
+    with tuning(settings):
+        found = forward_instances(cc, shape)
+        assert len(found) == 1 and found[0][-1] == copies
+        tile = found[0][4:6]
+        rows = [1] * (3 - len(shape[3])) + [-(-n // shape[4]) for n in shape[3][:-1]]
+        assert copies == all(n >= t for n, t in zip(rows, tile))
+        check_operator_problem(cc, shape, seed=19)
