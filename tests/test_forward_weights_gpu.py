@@ -56,3 +56,23 @@ def test_rows_past_the_edge_are_skipped_where_no_tile_is_whole(cc, case):
         rows = [1] * (3 - len(shape[3])) + [-(-n // shape[4]) for n in shape[3][:-1]]
         assert copies == all(n >= t for n, t in zip(rows, tile))
         check_operator_problem(cc, shape, seed=19)
+
+
+# 2D: copies where waves share a SIMD.  Rows of the longest workgroups (16 waves) at each number of rows and voxels per lane;
+# rows of one wave in few and in many workgroups, of four waves (two channel groups) once and twice to a compute unit.
+IMAGES = [({"fwd.rows2d": r, "fwd.vec2d": v}, (1, 6, 1, (2 * r, {1: 1000, 2: 1022, 4: 2044}[v]), 2), int(r * v >= 4))
+          for r in (2, 3, 4, 5, 6) for v in (1, 2, 4)]
+IMAGES += [({}, s, c) for s, c in (
+    ((1, 5, 1, (64, 64), 1), 0), ((1, 5, 1, (256, 256), 3), 0), ((1, 5, 1, (512, 512), 1), 0), ((1, 2, 1, (1024, 40), 1), 0),
+    ((1, 12, 1, (1024, 256), 1), 0), ((1, 12, 1, (1024, 512), 1), 1), ((8, 3, 1, (260, 256), 3), 1), ((1, 6, 2, (9, 64), 2), 0),
+    ((1, 6, 2, (12, 128), 3), 0), ((1, 6, 2, (256, 256), 8), 0), ((1, 4, 2, (16, 512), 1), 0), ((3, 4, 2, (512, 512), 1), 1),
+    ((1, 4, 2, (9, 333), 1), 1), ((1, 6, 2, (12, 1022), 3), 1), ((1, 6, 2, (9, 2044), 2), 1))]
+
+
+@pytest.mark.parametrize("case", IMAGES, ids=_id)
+def test_images_copy_weights_where_waves_share_a_simd(cc, case):
+    settings, shape, copies = case
+    with tuning(settings):
+        found = forward_instances(cc, shape)
+        assert len(found) == 1 and found[0][-1] == copies
+        check_operator_problem(cc, shape, seed=23)
