@@ -1272,22 +1272,32 @@ int64_t pull_floats(const PullPlan &p, int slabs)
     return (int64_t)p.wgs * slabs * (p.chunks.blocks * 1024 + kBiasColumns);
 }
 
-// Channels of a launch: those of one full chunk, where there are 2^18 voxels, else all of them.  A chunk of five to eight blocks takes nearly the
-// same time however many of its waves have a block (2048 x 2048, 14 outputs: 1.46, 1.54, 1.63, 1.61 ms over 5, 6, 7, 8), four 0.95, two 0.58
-// and one 0.44: full chunks and a small rest in a launch of its own take less than chunks of one size that share the chip (9 blocks: 2.75
-// ms as 5 + 4, 2.05 as 8 + 1).  Small images have too few tiles for launches one after the other.  Training step, two channels per layer, depth 100, us:
-// 256 x 256 2488, 2539; 384 x 384 3623, 3646; 512 x 512 4544, 4448; 1000 x 700 10526, 10286; depth 200: 2048 x 2048 88.1, 84.0 ms; depth 90: 100^3 35.5,
-// 33.7 ms.
-int64_t pull_channels(int64_t batch, int64_t rows, const PullPlan &p, int64_t channels, int slabs)
+// Channels of a launch: those of one full chunk (128; one slab: 64) where chunks in launches of their own, which use the whole chip one after the
+// other, take less than chunks of about one size side by side, else all of them.
+// Two slabs: a chunk of five to eight blocks takes nearly the same time however many of its waves have a block (2048 x 2048, 14 outputs: 1.46, 1.54,
+// 1.63, 1.61 ms over 5, 6, 7, 8), four 0.95, two 0.58 and one 0.44, so that full chunks and a small rest gain (9 blocks: 2.75 ms as 5 + 4,
+// 2.05 as 8 + 1), a rest of five or more only in large images.  Time of a group of 14 (four in 3D), side by side 1, over 9 / 10 / 13 /
+// 16 blocks: 512 x 513 1.00 / 1.02 / 1.12 / 1.02; 724 x 724 0.94 / 0.96 / 1.09 / 0.96; 960 x 960 0.88 / 0.93 / 1.02 / 0.90; 1500 x 1021
+// 0.88 / 0.93 / 1.00 / 0.92; 94^3 over 9 / 10 / 13 0.87 / 0.87 / 0.98; over 13 / 14 / 15 1024 x 1024 1.02 / 0.97 / 1.02, 1448 x 1448 0.98 / 0.96 / 1.00,
+// 2048 x 2048 0.96 / 0.94 / 1.00, 128^3 0.93 / 1.00 / 1.01.
+// One slab: a chunk has at most four blocks, and its time goes with their number.  A launch per chunk gains where the chunks side by side would be of
+// unequal size, and only where gradients are written: a layer of three outputs (two in 3D) over 5 / 7 / 13 (unequal), 6 / 8 / 9
+// (equal) blocks 512 x 513 1.06 / 1.13 / 1.34, 1.22 / 1.25 / 1.30; 900 x 900 0.90 / 1.01 / 1.05, 1.05; 1024 x 1024 0.84 / 0.94 / 0.95, 1.01 /
+// 1.10 / 0.95; 128^3 0.81 / 0.88 / 0.88, 0.94 / 1.03 / 0.92; added to, a group of seven 1024 x 1024 1.05 / 1.09 / 0.97, 1.04 / 1.06 / 1.01.
+// Segments of a pass whose chunks have launches of their own (32 voxels each):
+constexpr int64_t kAloneSmallRest = 14000, kAloneAnyRest = 1 << 16, kAloneWritten = 28000;
+int64_t pull_channels(int64_t batch, int64_t rows, const PullPlan &p, int64_t channels, int slabs, bool fresh)
 {
-    const bool alone = batch * rows * p.segs >= (1 << 18) / kSegment;
-    return alone ? std::min<int64_t>(channels, 16 * most_blocks(slabs)) : channels;
+    const int64_t segments = batch * rows * p.segs, full = 16 * most_blocks(slabs);
+    const bool alone = slabs == 1 ? fresh && p.chunks.large < p.chunks.n && segments >= kAloneWritten
+                                  : segments >= (channels % full <= full / 2 ? kAloneSmallRest : kAloneAnyRest);
+    return alone ? std::min(channels, full) : channels;
 }
-// Floats of the largest of the launches.
+// Floats of the largest of the launches, whether the gradients are written or added to.
 int64_t all_pull_floats(int64_t batch, int64_t rows, int64_t span, int64_t channels, int slabs)
 {
     const PullPlan p = pull_plan(batch, rows, span, channels, slabs);
-    const int64_t step = pull_channels(batch, rows, p, channels, slabs), rest = channels % step;
+    const int64_t step = pull_channels(batch, rows, p, channels, slabs, true), rest = channels % step;
     int64_t most = std::max(pull_floats(p, slabs), pull_floats(pull_plan(batch, rows, span, step, slabs), slabs));
     if (rest > 0) most = std::max(most, pull_floats(pull_plan(batch, rows, span, rest, slabs), slabs));
     return most;
@@ -1385,7 +1395,7 @@ hipError_t pull(const Geom &g, const View<const float> &x, const float *gy, int6
         return hipErrorInvalidValue;
     const int slabs = out.n > per_slab ? 2 : 1, taps = g.ndim == 3 ? 27 : group2d::kTaps;
     const int span = form == kFlat ? g.nvox : g.W, rows = g.nvox / span;
-    const int step = (int)pull_channels(g.B, rows, pull_plan(g.B, rows, span, g.C, slabs), g.C, slabs);
+    const int step = (int)pull_channels(g.B, rows, pull_plan(g.B, rows, span, g.C, slabs), g.C, slabs, fresh);
     for (int from = 0; from < g.C; from += step) {
         Geom part = g;
         View<const float> xp = x;

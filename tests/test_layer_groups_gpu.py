@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from parity import check_block, rel_err, same_specials
+from parity import block_problem, captured_kernels, check_block, rel_err, same_specials
 from test_knobs_gpu import tuning
 
 pytestmark = pytest.mark.gpu
@@ -65,7 +65,7 @@ def test_block_backward_in_layer_groups(case, input_grad):
         check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=43, input_grad=input_grad)
 
 
-# From 2^18 voxels on the channels go in launches of one chunk each (128 of them for more than seven outputs, 64 for fewer): a rest
+# More channels than a chunk holds (128 of them for more than seven outputs, 64 for fewer): a rest
 # of one channel and of several blocks, with and without gradients of the channels that the rest holds, several images, a volume.
 @pytest.mark.parametrize("input_grad", [True, False])
 @pytest.mark.parametrize("size, c_in, width, depth, batch", [
@@ -75,6 +75,27 @@ def test_block_backward_in_layer_groups(case, input_grad):
 def test_backward_groups_over_several_chunks(size, c_in, width, depth, batch, input_grad):
     check_block(len(size), size, c_in, width, depth, batch, dilations=[1 + 3 * i % 10 for i in range(depth)], seed=47,
                 input_grad=input_grad)
+
+
+# The same where the chunks have launches of their own: from 14000 segments of 32 voxels on with a rest of at most four blocks, from
+# 65536 on with any; up to seven outputs (3D: two) stay in one launch.  Just below and just above.
+@pytest.mark.parametrize("input_grad", [True, False])
+@pytest.mark.parametrize("size, c_in, depth, batch, launches", [
+    ((600, 720), 136, 8, 1, 1), ((640, 704), 130, 8, 1, 2), ((320, 701), 180, 8, 2, 2), ((640, 704), 200, 8, 1, 1),
+    ((32760, 33), 195, 8, 1, 1), ((32770, 33), 195, 8, 1, 2), ((900, 1000), 70, 2, 1, 1), ((76, 76, 77), 130, 4, 1, 1), ((77, 77, 77), 130, 4, 1, 2)],
+    ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_backward_chunks_in_launches_of_their_own(size, c_in, depth, batch, launches, input_grad):
+    from msd_pytorch_amd.msd_block import msd_block
+    dilations = [1 + 3 * i % 10 for i in range(depth)]
+    x, dil, bias, ws, g = block_problem(len(size), size, c_in, 1, depth, batch, dilations, 47)
+    leaves = [t.cuda().requires_grad_() for t in (bias, *ws)]
+    xd, up = x.cuda().requires_grad_(input_grad), g.cuda()
+    torch.cuda.synchronize()
+    names = captured_kernels(lambda: torch.autograd.grad(msd_block(xd, dil, *leaves), leaves, up))
+    assert sum("pull_rows" in n for n in names) == launches
+    assert sum("sum_group" in n for n in names) == launches
+    del leaves, xd, up
+    check_block(len(size), size, c_in, 1, depth, batch, dilations=dilations, seed=47, input_grad=input_grad)
 
 
 # Groups of eight to fourteen outputs: two slabs of 64 matrix rows, the upper outputs' share of the lower

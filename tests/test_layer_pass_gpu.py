@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from parity import rel_err, same_specials
+from parity import captured_kernels, rel_err, same_specials
 
 pytestmark = pytest.mark.gpu
 
@@ -88,6 +88,32 @@ def test_layer_gradients(case, relu):
     # the bias gradient is a sum of terms of both signs, in chains and trees of fewer than 64 additions here: each
     # rounds to 2^-24 of at most the sum of the terms' sizes
     terms = tensors[3].double().abs().sum(dim=[0, *range(2, tensors[3].dim())])
+    assert bool(((got[2] - want[2]).abs() <= 64 * 2.0 ** -24 * terms).all())
+
+
+# More than the 64 channels of a chunk: side by side in one launch where they make chunks of one size or the image is small, one
+# launch after the other where they do not (two blocks, one block and one channel over).
+@pytest.mark.parametrize("size, batch, c_in, c_out, launches", [
+    ((512, 513), 1, 65, 3, 1), ((512, 513), 1, 130, 2, 1), ((900, 1000), 1, 65, 3, 2), ((450, 1001), 2, 97, 7, 2), ((900, 1000), 1, 96, 3, 1),
+    ((902, 999), 1, 193, 4, 4), ((98, 97, 97), 1, 65, 2, 2), ((48, 100, 97), 2, 160, 1, 3), ((97, 97, 98), 1, 90, 2, 1)],
+    ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_layer_gradients_over_several_chunks(size, batch, c_in, c_out, launches):
+    tensors = problem(size, batch, c_in, c_out, seed=17)
+    torch.cuda.synchronize()
+    names = captured_kernels(lambda: gradients(*tensors, 3, True))
+    assert sum("pull_rows" in n for n in names) == launches
+    got, in_one_pass = ran_in_one_pass(lambda: gradients(*tensors, 3, True))
+    assert in_one_pass
+    # (the ReLU as the forward pass in single precision found it: one that is open in one precision only would show)
+    from msd_pytorch_amd import conv2d, conv3d
+    x, w, b, g = tensors
+    open_relu = (conv2d.conv2d_relu if len(size) == 2 else conv3d.conv3d_relu)(x, w, b, torch.empty_like(g), 1, 3) > 0
+    want = gradients(x.double(), w.double(), b.double(), (g * open_relu).double(), 3, False)
+    for a, b in zip(got[:2], want[:2]):
+        assert rel_err(a, b) <= 1e-5
+    # the sums over voxels: chains of 1/256 of the tiles, then trees, as terms of both signs; each addition rounds to 2^-24 of at
+    # most the sum of the terms' sizes
+    terms = g.double().abs().sum(dim=[0, *range(2, g.dim())])
     assert bool(((got[2] - want[2]).abs() <= 64 * 2.0 ** -24 * terms).all())
 
 
