@@ -42,7 +42,7 @@ HBM_PEAK = 8.0e12
 SWEEP_GRID = {
     "forward": {
         2: {"fwd.vec2d": (1, 2, 4), "fwd.rows2d": (2, 3, 4, 5, 6), "fwd.split": (1, 2, 4)},
-        3: {"fwd.vec3d": (1, 2, 4), "fwd.lattice3d": (24, 33, 44), "fwd.split": (1, 2, 4), "fwd.class3d": (0, 1)},
+        3: {"fwd.vec3d": (1, 2, 4), "fwd.lattice3d": (24, 33, 44), "fwd.split": (1, 2, 4, 8), "fwd.class3d": (0, 1)},
     },
     "backward_x": {
         2: {"bwdx.vec2d": (1, 2, 4), "bwdx.unroll2d": (2, 4), "bwdx.min_blocks": (256, 1024, 4096)},

@@ -503,14 +503,9 @@ hipError_t pick(const Geom &g, const View<const float> &x, const float *k, const
                 if (streams && split <= 1 && t44 * waves >= 4096 && t44 * 32 <= t24 * 17)
                     return launch<3, RELU, 1, 1, 4, 4, true>(g, x, k, bias, out, s, sums);
                 // The channels in one group where few of them leave the finishing step a large part and the tiles fill
-                // the chip without more waves (192^3 over 4 / 12 channels: 57, 41 / 97, 94; over 20:
-                // 159, 166), in four, from two channels each, where the tiles leave most of it idle (64^3 over 8 / 20 / 45: 9.9, 8.7 /
-                // 15, 12 / 27, 19; 61 x 93 x 75, 1500 waves, over 12 / 20: 15.2, 16.7 / 20.7, 21.2), in eight where they leave nearly all of it
-                // (40 x 45 x 47 over 30: 12.7, 11.2; 32^3 over 10: 6.9, 6.5, over 4 in four: 6.2, 5.4; 64^3 over 20: 11.9, 12.1).
+                // the chip without more waves (192^3 over 4 / 12 channels: 57, 41 / 97, 94; over 20: 159, 166).
                 const bool full = t24 * waves >= 7000;
                 const bool one = (full && g.C <= 12 && split < 0) || split == 1;
-                const bool few = t24 * waves <= 400;
-                const int groups = t24 * waves > 1100 || g.C < (few ? 4 : 8) ? 2 : few && g.C >= 10 ? 8 : 4;
                 // Lattices of 3 x 3 rows instead of 2 x 4 where they cover the residue classes
                 // with at least 1/16 fewer tiles (a partly filled lattice costs as much time as a
                 // full one): at 128^3 dilations 3, 5, 9, 10, by 2 to 12 %.  Not at dilations 1
@@ -520,6 +515,15 @@ hipError_t pick(const Geom &g, const View<const float> &x, const float *k, const
                 if (one)
                     return square ? launch<3, RELU, 1, 1, 3, 3, true>(g, x, k, bias, out, s, sums)
                                   : launch<3, RELU, 1, 1, 2, 4, true>(g, x, k, bias, out, s, sums);
+                // In more than two groups where the workgroups of two leave most of the chip idle: by the waves of all tiles' rows
+                // and the channels that a group has left.  Two, four and eight groups: rows of one wave, 40 x 45 x 47 (240 waves) over 8 / 10 /
+                // 24 channels 8.3, 6.8, 6.8 / 8.9, 7.4, 7.0 / 13.0, 9.2, 8.2; 48^3 (288) over 4 / 16 / 40 1.16, 1 / 1.32, 1, 1.09 / 1.60, 1.05, 1
+                // times the best; 64^3 (512) over 40 1.5, 1, 1.06; 66 x 66 x 64 (561) over 6 / 8 1.03, 1 / 1.08, 1; 80 x 80 x 64 (800) over 8 / 12 / 16 1, 1.08 / 1, 1.03 / 1.07, 1; 120 x 120 x 64
+                // (1800) over 16 / 32 1, 1.05 / 1.01, 1.  Of two waves (eight groups would be more than 512 lanes): 30 x 60 x 100 (450) over
+                // 8 / 24 1.05, 1 / 1.28, 1; 40 x 61 x 75 (640) over 8 / 12 / 16 / 24 1, 1.12 / 1, 1.06 / 1, 1.04 / 1.02, 1; 61 x 93 x 75 (1488) over 20 1, 1.05.
+                const long row = (g.W + kWave - 1) / kWave, used = (square ? t33 : t24) * waves;
+                const int least = used <= 512 ? 4 : row > 1 ? 16 : used <= 700 ? 8 : 12;
+                const int groups = g.C >= (used <= 256 ? 9 : 32) && used <= 400 ? 8 : g.C >= least && used <= 1100 ? 4 : 2;
                 return square ? launch<3, RELU, 1, 1, 3, 3>(g, x, k, bias, out, s, sums, groups)
                               : launch<3, RELU, 1, 1, 2, 4>(g, x, k, bias, out, s, sums, groups);
             }

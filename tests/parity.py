@@ -145,7 +145,7 @@ def check_block(ndim, size, c_in, width, depth, batch, dilations=None, seed=0, i
 
 
 def captured_kernels(run):
-    """The names (mangled) of the kernels that run() launches, in order: it is recorded into a graph and not executed."""
+    """The kernels that run() launches, as (mangled name, lanes of a workgroup): it is recorded into a graph and not executed."""
     import ctypes
     path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
     hip = ctypes.CDLL(path)
@@ -166,12 +166,12 @@ def captured_kernels(run):
     assert hip.hipGraphGetNodes(raw, None, ctypes.byref(count)) == 0
     nodes = (ctypes.c_void_p * count.value)()
     assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(count)) == 0
-    names = []
+    found = []
     for node in nodes:
         kind, params = ctypes.c_int(), KernelNode()
         assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
         if kind.value != 0:                      # (0: a kernel)
             continue
         assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(params)) == 0
-        names.append(hip.hipKernelNameRefByPtr(params.func, None).decode())
-    return names
+        found.append((hip.hipKernelNameRefByPtr(params.func, None).decode(), params.block.x))
+    return found

@@ -1,5 +1,5 @@
-"""How the forward kernel takes its weights: from vector registers, where it forms all rows of a tile, also those past the
-image edge, or from scalar registers, where it skips such rows."""
+"""What the forward kernel is launched with.  How it takes its weights: from vector registers, where it forms all rows of a tile, also those past the
+image edge, or from scalar registers, where it skips such rows.  And in how many groups it takes the channels."""
 import re
 
 import pytest
@@ -19,11 +19,11 @@ def cc():
 
 
 def forward_instances(cc, shape):
-    """The template arguments of each launch of fwd_lattice that a layer's forward pass makes, as numbers."""
+    """Each launch of fwd_lattice that a layer's forward pass makes: its template arguments as numbers and the lanes of a workgroup."""
     p = problem_on(make_problem(shape, torch.float32), "cuda")
-    names = captured_kernels(lambda: cc.conv_relu_forward(p["x"], p["k"], p["bias"], p["y"], p["d"]))
-    found = [re.search(r"fwd_latticeI((?:L[ib]\d+E)+)E", n) for n in names]
-    return [[int(v) for v in re.findall(r"L[ib](\d+)E", m.group(1))] for m in found if m]
+    kernels = captured_kernels(lambda: cc.conv_relu_forward(p["x"], p["k"], p["bias"], p["y"], p["d"]))
+    found = [(re.search(r"fwd_latticeI((?:L[ib]\d+E)+)E", name), lanes) for name, lanes in kernels]
+    return [([int(v) for v in re.findall(r"L[ib](\d+)E", m.group(1))], lanes) for m, lanes in found if m]
 
 
 # (settings, (B, C_in, C_out, spatial, dilation), copies): volumes and images with fewer slices or rows per residue class than a tile of
@@ -50,9 +50,9 @@ def _id(case):
 def test_rows_past_the_edge_are_skipped_where_no_tile_is_whole(cc, case):
     settings, shape, copies = case
     with tuning(settings):
-        found = forward_instances(cc, shape)
-        assert len(found) == 1 and found[0][-1] == copies
-        tile = found[0][4:6]
+        (found, _), = forward_instances(cc, shape)
+        assert found[-1] == copies
+        tile = found[4:6]
         rows = [1] * (3 - len(shape[3])) + [-(-n // shape[4]) for n in shape[3][:-1]]
         assert copies == all(n >= t for n, t in zip(rows, tile))
         check_operator_problem(cc, shape, seed=19)
@@ -73,6 +73,26 @@ IMAGES += [({}, s, c) for s, c in (
 def test_images_copy_weights_where_waves_share_a_simd(cc, case):
     settings, shape, copies = case
     with tuning(settings):
-        found = forward_instances(cc, shape)
-        assert len(found) == 1 and found[0][-1] == copies
+        (found, _), = forward_instances(cc, shape)
+        assert found[-1] == copies
         check_operator_problem(cc, shape, seed=23)
+
+
+# 3D: channel groups by the waves of all tiles (in brackets) and the channels, on both sides of each line; a tile of 3 x 3 rows, several volumes.
+GROUPS = [((1, 3, 1, (16, 16, 32), 1), 2), ((1, 4, 1, (16, 16, 32), 1), 4), ((1, 8, 1, (16, 16, 32), 2), 4), ((1, 9, 1, (16, 16, 32), 1), 8),
+          ((1, 15, 1, (40, 45, 47), 5), 8),                                                     # (225 of 3 x 3 rows)
+          ((1, 9, 1, (34, 64, 40), 1), 4), ((1, 31, 1, (34, 64, 40), 1), 4), ((1, 32, 1, (34, 64, 40), 1), 8), ((2, 9, 1, (32, 32, 32), 2), 8),
+          ((1, 33, 1, (60, 60, 33), 1), 4),
+          ((3, 9, 1, (32, 32, 32), 2), 4),                                                      # (272, 256, 450, 384)
+          ((1, 7, 1, (66, 66, 33), 1), 2), ((1, 8, 1, (66, 66, 33), 1), 4), ((1, 11, 1, (80, 80, 34), 1), 2), ((1, 12, 1, (80, 80, 34), 1), 4),
+          ((1, 14, 1, (96, 96, 33), 1), 2),                                                     # (561, 800, 1152)
+          ((1, 4, 1, (30, 60, 70), 1), 4), ((1, 33, 1, (30, 60, 70), 1), 4), ((1, 15, 1, (36, 60, 65), 1), 2), ((1, 16, 1, (36, 60, 65), 1), 4),
+          ((1, 20, 1, (60, 93, 75), 1), 2)]                                                     # (rows of two waves: 450, 540, 1440)
+
+
+@pytest.mark.parametrize("case", GROUPS, ids=lambda c: _id(({}, c[0], 0)))
+def test_channel_groups_by_the_size_of_a_volume(cc, case):
+    shape, groups = case
+    (_, lanes), = forward_instances(cc, shape)
+    assert lanes == groups * -(-shape[3][-1] // 64) * 64
+    check_operator_problem(cc, shape, seed=29)

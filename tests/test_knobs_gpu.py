@@ -62,6 +62,9 @@ FORWARD_3D += [({"fwd.lattice3d": m}, s) for m in (24, 33, 44) for s in (VOL_A, 
 # (4 x 4 rows are one channel group whatever fwd.split says)
 FORWARD_3D += [({"fwd.lattice3d": m, "fwd.split": k}, VOL_E) for m in (24, 33) for k in (1, 4)]
 SPLIT = [({"fwd.split": k}, s) for k in (1, 2, 4) for s in (IMG_A, IMG_C, VOL_A, VOL_C)]
+# (eight: rows of one wave, volumes of two waves take four; more groups than channels)
+SPLIT += [({"fwd.split": 8}, s) for s in (IMG_A, IMG_C, VOL_A, VOL_E)]
+SPLIT += [({"fwd.split": 8}, (1, c, 1, (9, 8, w), 2)) for c, w in ((7, 40), (8, 64), (9, 33), (15, 40), (9, 65))]
 ORDER = [({"xcd_remap": r}, s) for r in (0, 1) for s in (IMG_B, IMG_D, VOL_A, VOL_D)]
 BACKWARD_K = [({"bwdk.vec2d": v}, s) for v in (1, 2, 4) for s in (IMG_A, IMG_B, IMG_C)]
 # ("bwdk.fused3d": 0 keeps a 3D layer of one or two output channels on the kernels that these
