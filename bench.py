@@ -40,19 +40,15 @@ FAMILIES = {"forward": ("fwd_lattice", "push_rows", "push_table", "push_split", 
             "backward_xkb": ("bwd_rows_fused", "bwd_one_channel", "pull_rows", "finish_back", "spread_back", "sum_group",
                              "reduce_columns"),
             "backward_kb": ("bwdk_rows", "bwdk_mfma"), "backward_x": ("relu_mask", "bwdx_rows", "bwdx_one_channel")}
-# families that are the further passes of an operator call or of a group of layers, not a call of their own
-SECOND_PASS = ("reduce_columns", "push_table", "finish_rows", "finish_back", "spread_back", "sum_group")
-
-
 def profiled_traffic(name, split3d=False):
     """HBM-side bytes per pass of the network for each kernel class, read from the committed
     rocprofv3 summary of this workload (profiles/bench_workload_<name>_*.txt, block "HBM-side
     bytes per pass": FETCH_SIZE + WRITE_SIZE per dispatch, scaled by what the same counters
     read for a 1 GiB device copy).  Counters cannot be read from inside this script.  The
     summary also holds how many dispatches of each family one pass of the network made when
-    the counters were taken (block "dispatches per pass"); a class whose main kernels are
-    launched another number of times now (the kernels or the grouping of layers changed since)
-    gets no figure.  Returns ({class: (bytes, dispatches of its main kernels or None)}, file
+    the counters were taken (block "dispatches per pass"); a class with a family that is
+    launched another number of times now (the kernels, the grouping of layers or the launches of
+    a group changed since) gets no figure.  Returns ({class: (bytes, {family: dispatches})}, file
     name) or ({}, None) when no summary is there."""
     import glob
     import re
@@ -85,9 +81,38 @@ def profiled_traffic(name, split3d=False):
     for cls, fams in families.items():
         found = [per_family[f] for f in fams if f in per_family]
         if found:
-            main = [dispatches[f] for f in fams if f in dispatches and f not in SECOND_PASS]
-            out[cls] = (sum(found), sum(main) if main else None)
+            out[cls] = (sum(found), {f: dispatches.get(f, 0) for f in fams})
     return out, os.path.relpath(files[0], ROOT)
+
+
+def launched_otherwise(profiled, names):
+    """The families that a summary counts another number of dispatches of than there are among the kernels `names`:
+    {family: (then, now)}."""
+    now = {family: sum(family in name for name in names) for family in profiled}
+    return {family: (then, now[family]) for family, then in profiled.items() if then != now[family]}
+
+
+def step_kernels(model, torch):
+    """The names of the kernels of one forward and backward pass, from a graph that is recorded and not run."""
+    from msd_pytorch_amd.benchmark_ops import recorded_kernels
+
+    def forget():                               # no autograd graph, and with it no gradient accumulator, of another stream
+        model.loss = model.output = None
+        model.optimizer.zero_grad(set_to_none=True)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    forget()
+    with torch.cuda.stream(side):
+        model.step_async(update=False)
+        forget()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=side):
+        model.step_async(update=False)
+    names = [name for name, _ in recorded_kernels(graph)]
+    forget()
+    return names
 
 
 WORKLOADS = {
@@ -443,8 +468,9 @@ def measure(name, args, lib, torch, steps=None, warmup=None, cpu=True):
         if split3d:
             result["config"]["backward"] = ("chain of backward_x launches (two layers per pass); weight gradients two "
                                             "layers per pass on a second stream (kernel classes timed on one stream)")
-        per_launch, profiled_calls = traffic.get(dominant, (None, None))
-        stale = per_launch is not None and profiled_calls is not None and profiled_calls != dom["calls_per_step"]
+        per_launch, profiled = traffic.get(dominant, (None, {}))
+        # (the step's own kernels, one by one: a call of a class may be any number of launches)
+        stale = launched_otherwise(profiled, step_kernels(model, torch)) if per_launch is not None else {}
         if stale:
             per_launch = None
         by_flops = dom["frac_fp32"] > dom["frac_hbm"]
@@ -457,8 +483,9 @@ def measure(name, args, lib, torch, steps=None, warmup=None, cpu=True):
                 # summary), to be compared with the algorithmic bytes per launch
                 "traffic": round(per_launch / dom["calls_per_step"]) if per_launch else None,
                 "traffic_source": source if per_launch else None,
-                **({"traffic_note": f"{source} was taken with {profiled_calls} launches of this class per step, "
-                                    f"this run makes {dom['calls_per_step']}: counters not comparable"} if stale else {}),
+                **({"traffic_note": f"{source} was taken with other launches of this class per step ("
+                                    + ", ".join(f"{f} {then}, now {now}" for f, (then, now) in sorted(stale.items()))
+                                    + "): counters not comparable"} if stale else {}),
                 "algorithmic_bytes_per_launch": round(bytes_per_step[dominant] / dom["calls_per_step"]),
                 "algorithmic_flops_per_launch": round(flops_per_step[dominant] / dom["calls_per_step"]),
                 "avg_launch_us": dom["avg_call_us"],

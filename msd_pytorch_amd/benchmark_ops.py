@@ -92,6 +92,40 @@ def _t_quantile_95(dof):
         return z + (z ** 3 + z) / (4 * dof) + (5 * z ** 5 + 16 * z ** 3 + 3 * z) / (96 * dof ** 2)
 
 
+def recorded_kernels(graph):
+    """The kernel nodes of a torch.cuda.CUDAGraph(keep_graph=True), in order of their making, as (mangled name, lanes of a
+    workgroup)."""
+    import ctypes
+    with open("/proc/self/maps") as maps:
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    hip.hipKernelNameRefByPtr.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+
+    class Dim(ctypes.Structure):
+        _fields_ = [(c, ctypes.c_uint32) for c in "xyz"]
+
+    class KernelNode(ctypes.Structure):          # hipKernelNodeParams
+        _fields_ = [("block", Dim), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", Dim),
+                    ("params", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+    def check(code):
+        if code != 0:
+            raise RuntimeError(f"recorded_kernels: HIP error {code}")
+
+    raw, count = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
+    check(hip.hipGraphGetNodes(raw, None, ctypes.byref(count)))
+    nodes = (ctypes.c_void_p * count.value)()
+    check(hip.hipGraphGetNodes(raw, nodes, ctypes.byref(count)))
+    found = []
+    for node in nodes:
+        kind, params = ctypes.c_int(), KernelNode()
+        check(hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)))
+        if kind.value == 0:                      # a kernel
+            check(hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(params)))
+            found.append((hip.hipKernelNameRefByPtr(params.func, None).decode(), params.block.x))
+    return found
+
+
 def fit_slope(counts, seconds):
     """Least-squares slope of seconds over counts and its 90 % confidence interval."""
     n = len(counts)

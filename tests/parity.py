@@ -146,32 +146,8 @@ def check_block(ndim, size, c_in, width, depth, batch, dilations=None, seed=0, i
 
 def captured_kernels(run):
     """The kernels that run() launches, as (mangled name, lanes of a workgroup): it is recorded into a graph and not executed."""
-    import ctypes
-    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
-    hip = ctypes.CDLL(path)
-    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
-    hip.hipKernelNameRefByPtr.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
-
-    class Dim(ctypes.Structure):
-        _fields_ = [(c, ctypes.c_uint32) for c in "xyz"]
-
-    class KernelNode(ctypes.Structure):          # hipKernelNodeParams
-        _fields_ = [("block", Dim), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", Dim), ("params", ctypes.c_void_p),
-                    ("shared", ctypes.c_uint)]
-
+    from msd_pytorch_amd.benchmark_ops import recorded_kernels
     graph = torch.cuda.CUDAGraph(keep_graph=True)
     with torch.cuda.graph(graph):
         run()
-    raw, count = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
-    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(count)) == 0
-    nodes = (ctypes.c_void_p * count.value)()
-    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(count)) == 0
-    found = []
-    for node in nodes:
-        kind, params = ctypes.c_int(), KernelNode()
-        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
-        if kind.value != 0:                      # (0: a kernel)
-            continue
-        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(params)) == 0
-        found.append((hip.hipKernelNameRefByPtr(params.func, None).decode(), params.block.x))
-    return found
+    return recorded_kernels(graph)

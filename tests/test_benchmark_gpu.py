@@ -26,3 +26,33 @@ def test_one_sweep_cell_and_one_table_line(tmp_path, capsys):
     rc = bo.main(["--ndim", "2", "--size", "128", "--channels", "3", "--dilations", "1", "--trials", "1"])
     assert rc == 0
     assert "forward" in capsys.readouterr().out
+
+
+def test_the_traffic_of_other_launches_is_not_quoted(monkeypatch):
+    """bench.py on its smallest workload: the step's kernels are the ones that its launches are compared by, and a summary taken with
+    another number of them gives no figure."""
+    import argparse
+
+    import torch
+
+    import bench
+    from msd_pytorch_amd import _native
+    args = argparse.Namespace(steps=2, warmup=1, graph=False, no_kernel_timing=False, tune=[], no_cpu_baseline=True)
+    lib = _native.load()
+    model = bench.make_model("A", torch)
+    x, target = bench.make_data("A", torch)
+    model.set_input(x)
+    model.set_target(target)
+    model.step_async(update=False)
+    names = bench.step_kernels(model, torch)
+    families = bench.FAMILIES["backward_xkb"]
+    now = {f: sum(f in n for n in names) for f in families}
+    assert now["pull_rows"] == now["sum_group"] == 1 and now["finish_back"] + now["spread_back"] == 9
+    assert torch.isfinite(model.step_async(update=False) or model.loss)          # (eager steps go on)
+    for extra, quoted in ((0, True), (1, False)):
+        profiled = {**now, "pull_rows": now["pull_rows"] + extra}
+        monkeypatch.setattr(bench, "profiled_traffic", lambda *a: ({c: (1e6, profiled if c == "backward_xkb" else {})
+                                                                    for c in bench.FAMILIES}, "a summary"))
+        roof = bench.measure("A", args, lib, torch, cpu=False)["roofline"]
+        assert roof["kernel"] == "backward_xkb"
+        assert (roof["traffic"] is not None) == quoted and ("traffic_note" in roof) != quoted

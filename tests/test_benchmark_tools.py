@@ -137,3 +137,11 @@ def test_algorithmic_bytes_of_the_paired_3d_chain():
     assert 0.5 < paired["backward_x"] / per_layer["backward_x"] < 0.55
     assert paired["backward_kb"] == per_layer["backward_kb"] and paired["forward"] == per_layer["forward"]
     assert flops["backward_x"] > 0
+
+
+def test_a_summary_of_other_launches_is_found_out():
+    import bench
+    # the launches of a pass over many channels: one call of its class, several kernels
+    names = ["_ZN3msd7group2d9pull_rowsILi2ELi2ELi1ELb0EEEvNS0_8PullArgsE"] * 2 + ["_ZN3msd7group2d9sum_groupILi2EEEv"] * 2
+    assert bench.launched_otherwise({"pull_rows": 2, "sum_group": 2, "spread_back": 0}, names) == {}
+    assert bench.launched_otherwise({"pull_rows": 1, "sum_group": 2, "spread_back": 1}, names) == {"pull_rows": (1, 2), "spread_back": (1, 0)}
