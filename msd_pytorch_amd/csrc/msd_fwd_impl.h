@@ -395,10 +395,12 @@ inline bool make_lattice(const Geom &g, int V, int rz, int ry, int ks_wanted, La
 // outputs, 16 x 512 at 8 12.6, 15.5.  Where only some tiles are whole it is these that decide: 12 x 300 x 300 at 10 (0.56 of all
 // rows inside) 91, 82; 512 x 24 x 512 over 21 channels at 5 (0.66) 13 % less.
 // 2D: a wave on its own does not issue faster without scalar operands, so several have to share a SIMD: two where
-// eight or more multiply-adds share a copy, three where four to seven do; with fewer they never gain.  One output, four rows: 2 waves of
+// eight or more multiply-adds share a copy, three where four to seven do, eight with fewer (four with three over up to ten channels: over more the
+// products outweigh what else the row takes).  One output, four rows: 2 waves of
 // a workgroup, 1024 x 40 over 30 / 60 channels 6.7, 7.0 / 10.1, 10.7; 8, 1024 x 256 over 11 / 70 5.4, 5.4 / 20.1, 20.4; 16, 1024 x 512
 // over 11 / 70 7.2, 7.0 / 25.3, 24.9; six rows, 1400 x 1000 over 30 31.2, 30.2; two rows, 64 x 64 / 256 x 256 / 512 x 512 over 60 7.9, 8.6 /
-// 9.0, 9.6 / 16.4, 17.0.  Two outputs, four voxels per lane: 2 and 4 waves, 256 x 256 / 512 x 512 over 30 16.5, 17.3 / 20.0, 20.7; 8,
+// 9.0, 9.6 / 16.4, 17.0; eight waves of a SIMD, 900 x 900 over 3 / 11 / 60 1 %, 2 %, 1 % less; three rows, four waves, 768 x 928
+// over 3 / 9 / 24 / 60 2 %, 1 % less, 1 %, 1 % more.  Two outputs, four voxels per lane: 2 and 4 waves, 256 x 256 / 512 x 512 over 30 16.5, 17.3 / 20.0, 20.7; 8,
 // 400 x 800 / 1024 x 1024 over 20 / 30 20.2, 17.8 / 39.5, 33.0.
 inline bool copies_weights(const Geom &g, const Lattice &lt, int rz, int ry, int V)
 {
@@ -407,7 +409,8 @@ inline bool copies_weights(const Geom &g, const Lattice &lt, int rz, int ry, int
     if (g.ndim == 3) return true;
     const int64_t workgroups = ((int64_t)lt.tiles_y * g.B + 255) / 256;       // of a compute unit
     const int64_t waves = workgroups * ((lt.ks * lt.lpr / kWave + 3) / 4);    // of a SIMD
-    return waves >= (ry * V >= 8 ? 2 : 3);
+    const int shared = ry * V;
+    return waves >= (shared >= 8 ? 2 : shared >= 4 ? 3 : shared == 3 && g.C <= 10 ? 4 : 8);
 }
 
 template <int NDIM, bool RELU, int WOUT, int V, int RZ, int RY, bool ONE = false>
@@ -427,9 +430,8 @@ hipError_t launch(const Geom &g, const View<const float> &x, const float *k, con
                            lt, remap, x, k, bias, out);
         return hipGetLastError();
     };
-    // (with less than four multiply-adds to a copy they never gain; 3D with several voxels per lane: only by the setting)
-    if constexpr (RZ * RY * V < 4) return with(std::false_type{});
-    else if constexpr (NDIM == 3 && V > 1) return with(std::true_type{});
+    // (3D with several voxels per lane: only by the setting)
+    if constexpr (NDIM == 3 && V > 1) return with(std::true_type{});
     else return copies_weights(g, lt, RZ, RY, V) ? with(std::true_type{}) : with(std::false_type{});
 }
 

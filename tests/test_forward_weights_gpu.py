@@ -60,11 +60,12 @@ def test_rows_past_the_edge_are_skipped_where_no_tile_is_whole(cc, case):
 
 # 2D: copies where waves share a SIMD.  Rows of the longest workgroups (16 waves) at each number of rows and voxels per lane;
 # rows of one wave in few and in many workgroups, of four waves (two channel groups) once and twice to a compute unit.
-IMAGES = [({"fwd.rows2d": r, "fwd.vec2d": v}, (1, 6, 1, (2 * r, {1: 1000, 2: 1022, 4: 2044}[v]), 2), int(r * v >= 4))
+IMAGES = [({"fwd.rows2d": r, "fwd.vec2d": v}, (1, 6, 1, (2 * r, {1: 1000, 2: 1022, 4: 2044}[v]), 2), int(r * v >= 3))
           for r in (2, 3, 4, 5, 6) for v in (1, 2, 4)]
 IMAGES += [({}, s, c) for s, c in (
     ((1, 5, 1, (64, 64), 1), 0), ((1, 5, 1, (256, 256), 3), 0), ((1, 5, 1, (512, 512), 1), 0), ((1, 2, 1, (1024, 40), 1), 0),
-    ((1, 12, 1, (1024, 256), 1), 0), ((1, 12, 1, (1024, 512), 1), 1), ((8, 3, 1, (260, 256), 3), 1), ((1, 6, 2, (9, 64), 2), 0),
+    ((1, 12, 1, (1024, 256), 1), 0), ((1, 12, 1, (1024, 512), 1), 1), ((1, 3, 1, (900, 900), 4), 1), ((1, 13, 1, (900, 837), 1), 1),
+    ((1, 10, 1, (700, 1000), 8), 1), ((1, 11, 1, (700, 1000), 8), 0), ((1, 4, 1, (500, 1000), 1), 0), ((8, 3, 1, (260, 256), 3), 1), ((1, 6, 2, (9, 64), 2), 0),
     ((1, 6, 2, (12, 128), 3), 0), ((1, 6, 2, (256, 256), 8), 0), ((1, 4, 2, (16, 512), 1), 0), ((3, 4, 2, (512, 512), 1), 1),
     ((1, 4, 2, (9, 333), 1), 1), ((1, 6, 2, (12, 1022), 3), 1), ((1, 6, 2, (9, 2044), 2), 1))]
 
