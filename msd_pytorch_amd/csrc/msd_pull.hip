@@ -1276,21 +1276,28 @@ int64_t pull_floats(const PullPlan &p, int slabs)
 // other, take less than chunks of about one size side by side, else all of them.
 // Two slabs: a chunk of five to eight blocks takes nearly the same time however many of its waves have a block (2048 x 2048, 14 outputs: 1.46, 1.54,
 // 1.63, 1.61 ms over 5, 6, 7, 8), four 0.95, two 0.58 and one 0.44, so that full chunks and a small rest gain (9 blocks: 2.75 ms as 5 + 4,
-// 2.05 as 8 + 1), a rest of five or more only in large images.  Time of a group of 14 (four in 3D), side by side 1, over 9 / 10 / 13 /
-// 16 blocks: 512 x 513 1.00 / 1.02 / 1.12 / 1.02; 724 x 724 0.94 / 0.96 / 1.09 / 0.96; 960 x 960 0.88 / 0.93 / 1.02 / 0.90; 1500 x 1021
-// 0.88 / 0.93 / 1.00 / 0.92; 94^3 over 9 / 10 / 13 0.87 / 0.87 / 0.98; over 13 / 14 / 15 1024 x 1024 1.02 / 0.97 / 1.02, 1448 x 1448 0.98 / 0.96 / 1.00,
-// 2048 x 2048 0.96 / 0.94 / 1.00, 128^3 0.93 / 1.00 / 1.01.
+// 2.05 as 8 + 1), a rest of six or more only in large images.  Time of a group of 14 (four in 3D), side by side 1, over 9 / 10 / 13 / 14 / 16 / 17
+// blocks: 512 x 513 0.97 / 0.99 / 1.03 / 1.13 / 1.14 / 1.02; 724 x 724 0.91 / 0.94 / 1.00 / 1.08 / 1.08 / 0.97; 960 x 960 0.85 / 0.89 / 0.95 / 1.04 / 1.05 / 0.92; 1500 x 1021
+// 0.86 / 0.89 / 0.95 / 1.02 / 1.02 / 0.93; 64 x 66 x 65 over 9 / 10 / 11 / 13 0.94 / 0.93 / 1.01 / 1.03; 94^3 over 9 / 10 / 13 / 14 0.88 / 0.88 / 0.97 / 1.04; over 13 / 14 / 16 1448 x 1448
+// 0.94 / 0.99 / 1.00, 2048 x 2048 0.94 / 1.00 / 0.98, 128^3 over 13 / 14 0.96 / 1.01.
 // One slab: a chunk has at most four blocks, and its time goes with their number.  A launch per chunk gains where the chunks side by side would be of
-// unequal size, and only where gradients are written: a layer of three outputs (two in 3D) over 5 / 7 / 13 (unequal), 6 / 8 / 9
-// (equal) blocks 512 x 513 1.06 / 1.13 / 1.34, 1.22 / 1.25 / 1.30; 900 x 900 0.90 / 1.01 / 1.05, 1.05; 1024 x 1024 0.84 / 0.94 / 0.95, 1.01 /
-// 1.10 / 0.95; 128^3 0.81 / 0.88 / 0.88, 0.94 / 1.03 / 0.92; added to, a group of seven 1024 x 1024 1.05 / 1.09 / 0.97, 1.04 / 1.06 / 1.01.
+// unequal size, five blocks most of all (4 + 1 for 3 + 2), the others only where gradients are written.  Side by side 1, a layer of three outputs (two
+// in 3D) over 5 / 7 / 13 (unequal), 6 / 8 / 9 (equal) blocks: 512 x 513 1.06 / 1.13 / 1.34, 1.22 / 1.25 / 1.30; 724 x 724 0.98 / 1.07 / 1.13, 1.12 /
+// 1.14 / 1.16; 900 x 900 0.90 / 1.01 / 1.05; 1024 x 1024 0.84 / 0.94 / 0.95, 1.01 / 1.10 / 0.95; 128^3 0.81 / 0.88 / 0.88, 0.94 / 1.03 / 0.92; added to, a group
+// of seven (two in 3D) over 5 / 7 / 11, 6 / 8 / 12: 724 x 724 1.03 / 1.09 / 1.16, 1.11 / 1.11 / 1.16; 1024 x 1024 0.90 / 1.00 / 1.04, 1.05 / 1.06 / 1.04; over
+// 5 / 7 / 11 100^3 0.91 / 1.00 / 1.00, 128^3 0.85 / 0.95 / 0.98.
 // Segments of a pass whose chunks have launches of their own (32 voxels each):
-constexpr int64_t kAloneSmallRest = 14000, kAloneAnyRest = 1 << 16, kAloneWritten = 28000;
+constexpr int64_t kAloneSmallRest = 14000, kAloneAnyRest = 1 << 16, kAloneOneSlab = 28000;
 int64_t pull_channels(int64_t batch, int64_t rows, const PullPlan &p, int64_t channels, int slabs, bool fresh)
 {
     const int64_t segments = batch * rows * p.segs, full = 16 * most_blocks(slabs);
-    const bool alone = slabs == 1 ? fresh && p.chunks.large < p.chunks.n && segments >= kAloneWritten
-                                  : segments >= (channels % full <= full / 2 ? kAloneSmallRest : kAloneAnyRest);
+    bool alone;
+    if (slabs == 1) {
+        const bool unequal = p.chunks.large < p.chunks.n, five = channels <= 5 * 16;
+        alone = unequal && (fresh || five) && segments >= (fresh && five ? kAloneSmallRest : kAloneOneSlab);
+    } else {
+        alone = segments >= (channels % full <= 5 * 16 ? kAloneSmallRest : kAloneAnyRest);
+    }
     return alone ? std::min(channels, full) : channels;
 }
 // Floats of the largest of the launches, whether the gradients are written or added to.

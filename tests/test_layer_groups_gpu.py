@@ -77,12 +77,12 @@ def test_backward_groups_over_several_chunks(size, c_in, width, depth, batch, in
                 input_grad=input_grad)
 
 
-# The same where the chunks have launches of their own: from 14000 segments of 32 voxels on with a rest of at most four blocks, from
-# 65536 on with any; up to seven outputs (3D: two) stay in one launch.  Just below and just above.
+# The same where the chunks have launches of their own: from 14000 segments of 32 voxels on with a rest of at most five blocks, from
+# 65536 on with any; up to seven outputs (3D: two) over five blocks from 28000 on, else in one launch.  Just below and just above.
 @pytest.mark.parametrize("input_grad", [True, False])
 @pytest.mark.parametrize("size, c_in, depth, batch, launches", [
-    ((600, 720), 136, 8, 1, 1), ((640, 704), 130, 8, 1, 2), ((320, 701), 180, 8, 2, 2), ((640, 704), 200, 8, 1, 1),
-    ((32760, 33), 195, 8, 1, 1), ((32770, 33), 195, 8, 1, 2), ((900, 1000), 70, 2, 1, 1), ((76, 76, 77), 130, 4, 1, 1), ((77, 77, 77), 130, 4, 1, 2)],
+    ((600, 720), 136, 8, 1, 1), ((640, 704), 130, 8, 1, 2), ((320, 701), 180, 8, 2, 2), ((640, 704), 201, 8, 1, 2), ((640, 704), 202, 8, 1, 1),
+    ((32760, 33), 205, 8, 1, 1), ((32770, 33), 205, 8, 1, 2), ((900, 1000), 70, 2, 1, 2), ((870, 1000), 70, 2, 1, 1), ((900, 1000), 100, 2, 1, 1), ((76, 76, 77), 130, 4, 1, 1), ((77, 77, 77), 130, 4, 1, 2)],
     ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_backward_chunks_in_launches_of_their_own(size, c_in, depth, batch, launches, input_grad):
     from msd_pytorch_amd.msd_block import msd_block

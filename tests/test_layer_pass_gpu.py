@@ -94,7 +94,7 @@ def test_layer_gradients(case, relu):
 # More than the 64 channels of a chunk: side by side in one launch where they make chunks of one size or the image is small, one
 # launch after the other where they do not (two blocks, one block and one channel over).
 @pytest.mark.parametrize("size, batch, c_in, c_out, launches", [
-    ((512, 513), 1, 65, 3, 1), ((512, 513), 1, 130, 2, 1), ((900, 1000), 1, 65, 3, 2), ((450, 1001), 2, 97, 7, 2), ((900, 1000), 1, 96, 3, 1),
+    ((512, 513), 1, 65, 3, 1), ((512, 513), 1, 130, 2, 1), ((700, 720), 1, 65, 3, 2), ((700, 720), 1, 97, 3, 1), ((900, 1000), 1, 65, 3, 2), ((450, 1001), 2, 97, 7, 2), ((900, 1000), 1, 96, 3, 1),
     ((902, 999), 1, 193, 4, 4), ((98, 97, 97), 1, 65, 2, 2), ((48, 100, 97), 2, 160, 1, 3), ((97, 97, 98), 1, 90, 2, 1)],
     ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_layer_gradients_over_several_chunks(size, batch, c_in, c_out, launches):
