@@ -1287,7 +1287,7 @@ int64_t pull_floats(const PullPlan &p, int slabs)
 // of seven (two in 3D) over 5 / 7 / 11, 6 / 8 / 12: 724 x 724 1.03 / 1.09 / 1.16, 1.11 / 1.11 / 1.16; 1024 x 1024 0.90 / 1.00 / 1.04, 1.05 / 1.06 / 1.04; over
 // 5 / 7 / 11 100^3 0.91 / 1.00 / 1.00, 128^3 0.85 / 0.95 / 0.98.
 // Segments of a pass whose chunks have launches of their own (32 voxels each):
-constexpr int64_t kAloneSmallRest = 14000, kAloneAnyRest = 1 << 16, kAloneOneSlab = 28000;
+constexpr int64_t kAloneTenBlocks = 1 << 13, kAloneSmallRest = 14000, kAloneAnyRest = 1 << 16, kAloneOneSlab = 28000;
 int64_t pull_channels(int64_t batch, int64_t rows, const PullPlan &p, int64_t channels, int slabs, bool fresh)
 {
     const int64_t segments = batch * rows * p.segs, full = 16 * most_blocks(slabs);
@@ -1296,7 +1296,7 @@ int64_t pull_channels(int64_t batch, int64_t rows, const PullPlan &p, int64_t ch
         const bool unequal = p.chunks.large < p.chunks.n, five = channels <= 5 * 16;
         alone = unequal && (fresh || five) && segments >= (fresh && five ? kAloneSmallRest : kAloneOneSlab);
     } else {
-        alone = segments >= (channels % full <= 5 * 16 ? kAloneSmallRest : kAloneAnyRest);
+        alone = segments >= (channels <= 10 * 16 ? kAloneTenBlocks : channels % full <= 5 * 16 ? kAloneSmallRest : kAloneAnyRest);
     }
     return alone ? std::min(channels, full) : channels;
 }
