@@ -4,35 +4,29 @@
 // voxel v, both gradients are matrix products with the same matrix:
 //     grad_input[c][v]  += sum_m k[m][c] * A[m][v],
 //     grad_kernel[c][m] += sum_v x[c][v] * A[m][v].
-// fp32 values are taken in three bf16 parts and six products (msd_split.h).  A workgroup of eight
-// waves owns a tile of eight segments of 32 voxels (four where a group has more than seven outputs) and
-// the 64 rows m of one slab (128 of two).  Each wave gathers a segment's A of one slab, splits it and
-// leaves it in LDS as [part][voxel][m]: the grad_input product reads it as it lies (lane = voxel, eight
-// rows m), the grad_kernel product through the transposing LDS read (ds_read_b64_tr_b16).  Behind a
-// barrier each wave takes its own block of 16 channels through both products, 64 voxels at a time; its
-// weights and its sums of grad_kernel stay in registers over all tiles, the sums leave as one row of
+// fp32 values are taken in three bf16 parts and six products (msd_split.h).  A workgroup owns a tile of two segments of 32 voxels
+// and the 128 rows m of two slabs (four segments where a group has at most seven outputs: one slab).  Four waves gather A
+// (each half a slab at the voxels of two segments, so that the outputs are the wave's own and a tap away from the edges is a scalar
+// address), split it and leave it in LDS as [part][voxel][m]: the grad_input product reads it as it lies (lane = voxel, eight
+// rows m), the grad_kernel product through the transposing LDS read (ds_read_b64_tr_b16).  At the same time four waves take the
+// tile before, which lies in a second buffer, through the one and four through the other product, a block of 16 channels at 32 voxels at a time; a
+// barrier per tile, and the buffers change.  Weights and sums stay in registers over all tiles, the sums leave as one row of
 // partial sums per workgroup.  x and grad_input go through a transposition in the wave's own part of LDS:
 // in the layout of the matrix cores a load touches 64 bytes of each of 16 channels, which memory
-// serves at 2.6-3.0 TB/s whatever else happens, four channels of 256 bytes at 4.0 (probed with loads and
-// stores alone, 64 channels of 1024 x 1024).
+// serves at 2.6-3.0 TB/s whatever else happens, whole lines at 4.0 (probed with loads and
+// stores alone, 64 channels of 1024 x 1024).  Five to eight blocks of two slabs: msd_pull_wide.h.
 //
-// 1024 x 1024, 14 outputs, us over the channels below: 4: 167, 20: 217, 45: 283, 70: 448, 95: 503, where two passes of
-// seven outputs on the fp32 instruction took 236 (20), 328 (48) and about 700 (95); seven outputs: 105 over 20 (118),
-// 411 over 100 (448).  Bound by the vector and matrix pipes together below about 60 channels (the split of A and
-// x is a third of the vector instructions; the waves of a workgroup are in the same phase, so that the two
-// pipes overlap little), above by memory (2.7 TB/s of channels that are read, and read and written).
-// A training step at 1024 x 1024, depth 100: 6.35 -> 5.33 ms; 4 x 512 x 512: 6.25 -> 4.99; 2048 x 2048, two
-// channels per layer, depth 200: 275 -> 194.
-//
-// Volumes (N = 3): two outputs of 27 taps in a slab's 64 rows, up to four in a group, the same tiles over the rows of all
-// slices or over a volume as one row.  128^3 over 1 to 46 channels: 335 us on average for four layers, and 80 for completing
-// their own channels, where the two streams of one and two layers per pass took 530; 61 x 93 x 75: 60 and 27
-// (168 one layer per pass).  Bound as above; every tile is taken to lie at an edge there (27 values folded along three axes
-// instead of 63 along two).
+// Bound by the issue of instructions: a SIMD issues a conversion, shift or select of a wave in 4.3 cycles and a matrix instruction
+// in 16.2, beside which there is room for two of the former, and a wave issues one instruction of any kind in 4.2 cycles.  With eight waves that all gathered and
+// then all multiplied, the two kinds of work did not meet and half of the waves were idle over few blocks.  us (with sum_group), eight
+// waves -> three kinds: 61 x 93 x 75, four outputs over 5 channels 69 -> 59; 128^3, four over 14 / 30 / 46 277 / 357 / 480 -> 254 / 335 / 455; 3 x 333 x
+// 477, 14 outputs over 19 90 -> 82; 1024 x 1024, 14 over 15 / 45 151 / 263 -> 140 / 258.
 //
 // Tried on the way: waves that walk the channels on their own tile (weights in LDS, loads in the matrix layout): 650 us
 // over 95 channels, 320 over 45; two workgroups of four waves per compute unit: 604 and 293; for 5 to 8 blocks
 // two chunks of at most 4: 588.  Any register spilt in the loop costs 10 % (its reload waits for all loads and stores).
+// Of the kinds: four waves that gather and four that do both products (128^3 over 14: 310), two teams that gather in turn (354), priorities by
+// kind (no gain), the next tile's loads spread among the split (271 for 250).
 #include "msd_group.h"
 #include "msd_split.h"
 
@@ -43,16 +37,17 @@ namespace msd {
 namespace group2d {
 namespace {
 
-constexpr int kWaves = 8;                         // of a workgroup; one workgroup per compute unit
-constexpr int kSegment = 32;                      // voxels of a row whose A a wave gathers
+constexpr int kSegment = 32;                      // voxels of a row that are gathered together
 constexpr int kVoxelBytes = 2 * 64;               // of a voxel's rows of a slab in LDS
 constexpr int kPartBytes = kSegment * kVoxelBytes;
 constexpr int kSlabBytes = 3 * kPartBytes;
 constexpr int kBiasColumns = 8;                   // per slab
 
 
-// LDS of a wave for a unit of voxels: 16 channels of x in three parts (the sums for grad_input take less)
-constexpr int unit_bytes(int voxels) { return 3 * 16 * (2 * voxels + 16); }
+// Bytes of a channel of a segment in a worker's own part of LDS: of x in one of its parts, of what is added to grad_input (16 apart in
+// the banks).
+constexpr int kXRow = 2 * kSegment + 16, kDRow = 4 * kSegment + 16;
+constexpr int kVec = 2, kLanes = kSegment / 4;    // 16-byte accesses per lane for a segment of 16 channels; lanes of a channel in one of them
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
@@ -68,7 +63,7 @@ template <int N> struct Gather {
     static constexpr int kLaneOut = kIsVolume ? 1 : 4;   // that a lane holds
 };
 
-// Row m of a slab's 64: the halves of 32 belong to the lanes h = 0 and 1 of the gather.  A lane holds
+// Row m of a slab's 64: the halves h = 0 and 1 of 32 are gathered apart.  A lane of a gatherer holds
 // whole outputs (the folds at the image's edges move values between an output's rows).  2D: three of nine
 // taps each, and of the seventh output, which both gather, five or four taps.  3D: one of 27.
 struct Slot {
@@ -154,53 +149,82 @@ __device__ __forceinline__ void fold(const Sides &s, float &tap0, float &tap2)
     tap2 = (s.down_in ? down : 0.f) + (s.up_in ? 0.f : up);
 }
 
-// What a workgroup of pull_rows keeps in LDS besides A and the waves' own space.
-struct Source {                                   // an output's place in bytes: its dilation in slices, rows and voxels, its plane
-    uint32_t slices, rows, voxels, plane;
+}  // namespace
+}  // namespace group2d
+}  // namespace msd
+#include "msd_pull_wide.h"
+namespace msd {
+namespace group2d {
+namespace {
+
+// The same with masks of bits: `and` and `add` of registers issue in half the cycles of a select.
+struct SideMasks {
+    uint32_t up, down, no_up, no_down;            // all bits where the source lies inside; where it does not
+    __device__ SideMasks(int u, int n, int d) : up(u + d < n ? ~0u : 0u), down(u >= d ? ~0u : 0u), no_up(~up), no_down(~down)
+    {
+        asm("" : "+v"(up), "+v"(down), "+v"(no_up), "+v"(no_down));                // (or they are selects again)
+    }
 };
+__device__ __forceinline__ float masked(float v, uint32_t bits) { return __uint_as_float(__float_as_uint(v) & bits); }
+__device__ __forceinline__ void fold(const SideMasks &s, float &tap0, float &tap2)
+{
+    const float up = tap0, down = tap2;
+    tap0 = masked(up, s.up) + masked(down, s.no_down);
+    tap2 = masked(down, s.down) + masked(up, s.no_up);
+}
+
+// What a workgroup of pull_rows keeps in LDS besides A and the waves' own space.
 struct PullShared {
-    Source sources[kMaxOut];
-    int bad_again, bad_tile[kWaves];
-    f32x4_t bias_sums[kWaves * kWave];                // of the lanes' outputs at their voxels (not in registers: there are none left)
+    int bad_again, bad_tile[2][4];                // (of a tile of A, by the waves that gather it)
 };
 
-// G slabs of rows; P waves share a block of 16 channels (the tile's voxels in as many parts).
+// G slabs of rows.  A workgroup is three kinds of four waves, one of each kind per SIMD: gatherers, which form A of a tile,
+// and those that take the tile before through the one and through the other product: kernel workers (grad_kernel) and input workers
+// (grad_input).  A is there twice.  P workers of a kind share a block of 16 channels (the tile's voxels in as many parts).
+enum Kind { kGatherer, kKernel, kInput };
+constexpr int kOfKind = 4;                        // waves
+constexpr int kPullThreads = 3 * kOfKind * kWave;
 template <int G, int P> struct PullShape {
-    static constexpr int kSegs = kWaves / G;             // segments of a tile
+    static constexpr int kSegs = kOfKind / G;            // segments of a tile
     static constexpr int kSteps = 2 * G;                 // of 32 rows m
     static constexpr int kTiles = 4 * G;                 // of 16 rows m
-    static constexpr int kUnit = kSegs * kSegment / P < 64 ? 32 : 64;      // voxels that a wave takes through the products at a time
-    static constexpr int kUnits = kSegs * kSegment / P / kUnit;
-    static constexpr int kVec = kUnit / 16;              // 16-byte accesses per lane for a unit of 16 channels
-    static constexpr int kLanes = kUnit / 4;             // lanes of a channel in one of them
-    static constexpr int kOwnBytes = unit_bytes(kUnit);
+    static constexpr int kUnits = kSegs / P;             // segments that a worker takes one after the other
+    static constexpr int kTileBytes = kSegs * G * kSlabBytes;
+    static constexpr int kXBytes = 16 * 3 * kXRow, kDBytes = 16 * kDRow;           // of a kernel, an input worker's own
+    static constexpr int kLds = 2 * kTileBytes + kOfKind * (kXBytes + kDBytes);
 };
 
-// What the kernel keeps for its life: the weights of rows 32 step + 8 q .. of channel n in parts, the sums of
-// grad_kernel.
+// What a wave keeps for its life: an input worker the weights of rows 32 step + 8 q .. of channel n in parts, a kernel worker its sums
+// of grad_kernel, a gatherer the sums of its outputs at its voxels (volumes: of one output, every fourth tile).  In the same registers:
+// what is declared is kept by all three.
 template <int G> struct PullState {
-    bf16x8_t w[2 * G][3];
+    f32x4_t kept[2 * G * 3];
     bool weights_split;
-    f32x4_t sums[4 * G];
+    __device__ f32x4_t &sums(int tile) { return kept[tile]; }
+    __device__ f32x4_t &bias() { return kept[0]; }
+    __device__ bf16x8_t weights(int step, int part) const { return __builtin_bit_cast(bf16x8_t, kept[step * 3 + part]); }
+    __device__ void set_weights(int step, int part, bf16x8_t w) { kept[step * 3 + part] = __builtin_bit_cast(f32x4_t, w); }
 };
 
 // The tiles of a workgroup.  True where units were left out that hold values which cannot be split: the second
 // run (WHOLE) takes these, with the fp32 instruction.  Apart, so that it keeps no registers in the first.
 template <int N, int G, int P, bool FRESH, bool WHOLE>
 __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__restrict__ x, const float *gy, float *gx, char *lds,
-                                           PullShared &shared, int tid, int wave, int blocks, int c0, int wgs, int wg, PullState<G> &state)
+                                           PullShared &shared, int kind, int number, int lane, int blocks, int c0, int wgs, int wg, PullState<G> &state)
 {
     using S = PullShape<G, P>;
-    constexpr int kSegs = S::kSegs, kSteps = S::kSteps, kTiles = S::kTiles, kUnit = S::kUnit, kUnits = S::kUnits, kVec = S::kVec;
-    constexpr int kLanes = S::kLanes, kOwnBytes = S::kOwnBytes;
+    constexpr int kSegs = S::kSegs, kSteps = S::kSteps, kTiles = S::kTiles, kUnits = S::kUnits;
     constexpr int kTaps = Gather<N>::kTaps, kLines = Gather<N>::kLines, kLaneOut = Gather<N>::kLaneOut, kSlabOut = Gather<N>::kOutputs;
-    const int lane = tid % kWave;
-    const int cb = wave / P, ch0 = c0 + cb * 16;  // the wave's block
-    const bool active = cb < blocks, update = ch0 < a.update;       // uniform
-    char *const A = lds;
-    char *const own = lds + kSegs * G * kSlabBytes + wave * kOwnBytes;
-    bf16x8_t(&w)[kSteps][3] = state.w;
-    f32x4_t(&sums)[kTiles] = state.sums;
+    const int cb = number / P, ch0 = c0 + cb * 16;                  // a worker's block
+    const int update_end = min(a.update, c0 + 16 * blocks);         // of the chunk
+    int buffer = 0;                               // of A: what is gathered, or taken through a product, next
+    char *A = lds;
+    auto turn_over = [&]() {
+        buffer = 1 - buffer;
+        A = lds + buffer * S::kTileBytes;
+    };
+    char *const own_x = lds + 2 * S::kTileBytes + number * S::kXBytes;             // a kernel worker's own
+    char *const own_d = lds + 2 * S::kTileBytes + kOfKind * S::kXBytes + number * S::kDBytes;      // an input worker's
 
     struct Tile {
         int first;                                // segment of its image
@@ -240,8 +264,8 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
     // The tiles: kSegs consecutive segments of an image each; every workgroup of an XCD works on neighbouring ones.
     const int lb = block_for_xcd(wg, wgs, wgs % kXcds == 0);
 
-    // ---- x and grad_input of a unit: lane (channel lane / kLanes of kVec x .., four voxels lane % kLanes)
-    const int lv = lane % kLanes, lc = lane / kLanes;               // voxels 4 lv .., channels lc + kRows4 i
+    // ---- x and grad_input of a unit, one segment: lane (channel lane / kLanes of kChannels, four voxels lane % kLanes)
+    const int lv = lane % kLanes, lc = lane / kLanes;               // voxels 4 lv .., channels lc + kChannels i
     constexpr int kChannels = kWave / kLanes;     // channels of one access
     const uint32_t lane_plane = (uint32_t)lc * plane;
     struct Unit {
@@ -250,14 +274,11 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         int skip;                                 // first of its four voxels that is its segment's own (0: all, 4: none)
     };
     auto unit_of = [&](const Tile &t, int u) {
-        const int first = ((wave % P) * kUnits + u) * (kUnit / kSegment);
-        const Place p0 = locate(t, first), p1 = locate(t, first + kUnit / kSegment - 1);
-        const int sel = lv / (kSegment / 4), v4 = lv % (kSegment / 4) * 4;
-        const uint32_t at0 = 4u * (uint32_t)(row_at(p0.z, p0.y) + p0.x0), at1 = 4u * (uint32_t)(row_at(p1.z, p1.y) + p1.x0);
+        const Place p = locate(t, number % P * kUnits + u);
         Unit un;
         un.img = t.img;
-        un.at = (sel ? at1 : at0) + 4u * (uint32_t)v4;
-        un.skip = min(max((sel ? p1.skip : p0.skip) - v4, 0), 4);
+        un.at = 4u * (uint32_t)(row_at(p.z, p.y) + p.x0 + 4 * lv);
+        un.skip = min(max(p.skip - 4 * lv, 0), 4);
         return un;
     };
     // channels from `limit` on: that channel before it again
@@ -274,96 +295,101 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             d[i] = f32x4_t{v4[0], v4[1], v4[2], v4[3]};
         }
     };
-    f32x4_t xs[kVec], gs[kVec];
-    auto request_g = [&](const Unit &un) {
-        if constexpr (FRESH) {
-#pragma unroll
-            for (int i = 0; i < kVec; i++) gs[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        } else {
-            request(gx, max(a.update, 1), un, gs);
-        }
-    };
 
-    // ---- the gather: lane (v, h) takes its outputs at voxel v of the wave's segment, 36 (27) values for 32 rows
-    // m.  Its loads are issued in the tile before, in front of that tile's last stores and requests (all of
-    // them retire in order: behind those it would wait for memory).
-    const int segment = wave / G, slab = wave % G;
-    const int v = lane % kSegment, h = lane / kSegment;
-    const uint32_t bias = 4u * (uint32_t)row_at(a.dmax, a.dmax);
+    // ---- the gather: a wave takes the 32 rows m of half h of one slab, 36 (27) values, at the voxels of two segments, so
+    // that the outputs and their dilations are the wave's own: away from the edges a tap is a scalar address.  The loads are
+    // issued in the tile before, in front of that tile's last stores and requests (all of them retire in order: behind
+    // those they would wait for memory).
+    const int pair = number / (2 * G), slab = number % (2 * G) / 2, h = number % 2;                // uniform
+    const int v = lane % kSegment, segment = 2 * pair + lane / kSegment;
     auto output_of = [&](int j) { return Gather<N>::kIsVolume ? h : j < 3 ? 3 * h + j : 6; };
-    auto source = [&](int j) {
-        int o = output_of(j);
-        asm volatile("" : "+v"(o));
-        return shared.sources[slab * kSlabOut + o];
-    };
-    // the lane's voxel (kImage, kVolume: y and z are uniform)
+    // (in registers: a scalar load in the loop is 400 cycles of waiting)
+    int dilation[kLaneOut];
+    uint32_t gplane[kLaneOut];                    // byte offset of the output's gradient
+#pragma unroll
+    for (int j = 0; j < kLaneOut; j++) {
+        const int o = min(slab * kSlabOut + output_of(j), a.out.n - 1);
+        dilation[j] = a.out.dil[o];
+        gplane[j] = (uint32_t)o * (uint32_t)(a.gsc * 4);
+        asm volatile("" : "+s"(dilation[j]), "+s"(gplane[j]));
+    }
+    // of the lane: its voxel, and how many voxels of its segment belong to the one before; of the wave: whether some have such, whether
+    // all voxels are away from the edges along x; along y and z
     struct Voxel {
-        int x, y, z;
+        int x, y, z, skip;
+        int skips, away_x, away_yz;               // (integers: a branch on a bool that is kept is made as if lanes could differ)
     };
-    auto voxel_of = [&](const Place &p) {
-        Voxel vx{p.x0 + v, p.y, p.z};
+    auto locate_pair = [&](const Tile &t) {
+        const Place p = locate(t, 2 * pair), p2 = locate(t, 2 * pair + 1);
+        const bool second = lane >= kSegment;
+        Voxel vx{(second ? p2.x0 : p.x0) + v, second ? p2.y : p.y, second ? p2.z : p.z, second ? p2.skip : p.skip, max(p.skip, p2.skip), 0, 0};
         if constexpr (N == kFlat) {
             const int row = a.by_voxels.of(vx.x);
             vx.x -= row * a.W;
             vx.z = a.by_rows.of(row);
             vx.y = row - vx.z * a.H;
+            vx.away_x = __all(vx.x >= a.dmax && vx.x + a.dmax < a.W) != 0;
+            vx.away_yz = __all(vx.y >= a.dmax && vx.y + a.dmax < a.H && vx.z >= a.dmax && vx.z + a.dmax < a.D) != 0;
+        } else {
+            vx.away_x = (min(p.x0, p2.x0) >= a.dmax) & (max(p.x0, p2.x0) + kSegment + a.dmax <= a.W);
+            vx.away_yz = (min(p.y, p2.y) >= a.dmax) & (max(p.y, p2.y) + a.dmax < a.H) &
+                         ((N == kImage) | ((min(p.z, p2.z) >= a.dmax) & (max(p.z, p2.z) + a.dmax < a.D)));
         }
+        vx.away_x = __builtin_amdgcn_readfirstlane(vx.away_x);
+        vx.away_yz = __builtin_amdgcn_readfirstlane(vx.away_yz);
         return vx;
     };
-    auto away = [&](const Place &p) {             // uniform: from all edges
-        return N != kFlat && p.x0 >= a.dmax && p.x0 + kSegment + a.dmax <= a.W && p.y >= a.dmax && p.y + a.dmax < a.H &&
-               (N == kImage || (p.z >= a.dmax && p.z + a.dmax < a.D));
-    };
     float val[kLaneOut][kLines][3];
-    auto gather = [&](const Tile &t, const Place &p) {
-        if (away(p)) {
-            const uint32_t u = (uint32_t)(p.x0 + v);
-            const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)(t.gimg + (int64_t)row_at(p.z, p.y) * 4) - bias;
+    auto gather = [&](const Tile &t, const Voxel &vx) {
+        const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)t.gimg;
 #pragma unroll
-            for (int j = 0; j < kLaneOut; j++) {
-                const Source o = source(j);
-                const uint32_t c = o.plane + bias + 4u * u;
+        for (int j = 0; j < kLaneOut; j++) {
+            const int d = dilation[j];
+            const uint64_t output = base + gplane[j];
+            const int up = min(vx.x + d, 2 * a.W - 1 - d - vx.x), down = max(vx.x - d, d - 1 - vx.x);
+            const int row = row_at(vx.z, vx.y);
+            uint32_t au = 4u * (uint32_t)(row + up), ah = 4u * (uint32_t)(row + vx.x), ad = 4u * (uint32_t)(row + down);
+            // (formed here: in the branch they may take registers that the other branch loads to, and wait for them)
+            if (N != kFlat) asm volatile("" : "+v"(au), "+v"(ah), "+v"(ad));
+            if (vx.away_yz != 0) {                    // uniform
 #pragma unroll
                 for (int l = 0; l < kLines; l++) {
-                    const uint32_t s = N == kImage || l / 3 == 1 ? c : l / 3 == 0 ? c + o.slices : c - o.slices;
-                    const uint32_t r = l % 3 == 0 ? s + o.rows : l % 3 == 1 ? s : s - o.rows;
-                    val[j][l][0] = load1(base, r + o.voxels);
-                    val[j][l][1] = load1(base, r);
-                    val[j][l][2] = load1(base, r - o.voxels);
+                    const uint64_t line = output + (uint64_t)((int64_t)row_at(N == kImage ? 0 : (1 - l / 3) * d, (1 - l % 3) * d) * 4);
+                    val[j][l][0] = load1(line, au);
+                    val[j][l][1] = load1(line, ah);
+                    val[j][l][2] = load1(line, ad);
                 }
-                __builtin_amdgcn_sched_barrier(0);    // (an output's addresses at a time: registers)
-            }
-        } else {
-            const uint64_t base = reinterpret_cast<uint64_t>(gy) + (uint64_t)t.gimg;
-            const Voxel vx = voxel_of(p);
-#pragma unroll
-            for (int j = 0; j < kLaneOut; j++) {
-                const Source o = source(j);
-                const int d = (int)(o.voxels / 4u);
-                const Sides sx = sides(vx.x, a.W, d), sy = sides(vx.y, a.H, d), sz = sides(vx.z, N == kImage ? 1 : a.D, N == kImage ? 0 : d);
+                asm volatile("; away" ::: "memory");  // (or the loads of both branches are one, at addresses that are kept for it)
+            } else {
+                const Sides sy = sides(vx.y, a.H, d), sz = sides(vx.z, N == kImage ? 1 : a.D, N == kImage ? 0 : d);
 #pragma unroll
                 for (int l = 0; l < kLines; l++) {
                     const int y = l % 3 == 0 ? sy.up : l % 3 == 1 ? vx.y : sy.down;
                     const int z = N == kImage || l / 3 == 1 ? vx.z : l / 3 == 0 ? sz.up : sz.down;
-                    const uint32_t r = o.plane + 4u * (uint32_t)row_at(z, y);
-                    val[j][l][0] = load1(base, r + 4u * (uint32_t)sx.up);
-                    val[j][l][1] = load1(base, r + 4u * (uint32_t)vx.x);
-                    val[j][l][2] = load1(base, r + 4u * (uint32_t)sx.down);
+                    const int at = row_at(z, y);
+                    val[j][l][0] = load1(output, 4u * (uint32_t)(at + up));
+                    val[j][l][1] = load1(output, 4u * (uint32_t)(at + vx.x));
+                    val[j][l][2] = load1(output, 4u * (uint32_t)(at + down));
                 }
-                __builtin_amdgcn_sched_barrier(0);
             }
+            __builtin_amdgcn_sched_barrier(0);        // (an output's addresses at a time: registers)
         }
     };
-    // round: number of the tile among the workgroup's, below 0 where its biases have been counted
-    auto gathered = [&](const Place &p, int round) {
-        if (!away(p)) {
-            const Voxel vx = voxel_of(p);
+    auto gathered = [&](const Voxel &vx) {
+        if (vx.away_x == 0) {                         // uniform
 #pragma unroll
             for (int j = 0; j < kLaneOut; j++) {
-                const int d = (int)(source(j).voxels / 4u);
-                const Sides sx = sides(vx.x, a.W, d), sy = sides(vx.y, a.H, d), sz = sides(vx.z, N == kImage ? 1 : a.D, N == kImage ? 0 : d);
+                const SideMasks sx(vx.x, a.W, dilation[j]);
 #pragma unroll
                 for (int l = 0; l < kLines; l++) fold(sx, val[j][l][0], val[j][l][2]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (vx.away_yz == 0) {                        // uniform
+#pragma unroll
+            for (int j = 0; j < kLaneOut; j++) {
+                const int d = dilation[j];
+                const SideMasks sy(vx.y, a.H, d), sz(vx.z, N == kImage ? 1 : a.D, N == kImage ? 0 : d);
 #pragma unroll
                 for (int l = 0; l < kLines; l += 3)
 #pragma unroll
@@ -377,18 +403,18 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (p.skip > 0 || a.out.n < G * kSlabOut) {                 // uniform
+        if (vx.skips > 0 || a.out.n < G * kSlabOut) { // uniform
 #pragma unroll
             for (int j = 0; j < kLaneOut; j++) {
-                const bool ok = v >= p.skip && slab * kSlabOut + output_of(j) < a.out.n;
+                const bool ok = v >= vx.skip && slab * kSlabOut + output_of(j) < a.out.n;
 #pragma unroll
                 for (int t = 0; t < kTaps; t++) val[j][t / 3][t % 3] = ok ? val[j][t / 3][t % 3] : 0.f;
             }
         }
-        if (round >= 0) {
+        if constexpr (!WHOLE) {                       // (the second run's have been counted)
             // (volumes: one value per lane, four chains of a quarter of the tiles)
-            if constexpr (N != kImage) reinterpret_cast<float *>(&shared.bias_sums[tid])[round % 4] += val[0][4 * (kLines / 9)][1];
-            else shared.bias_sums[tid] += f32x4_t{val[0][1][1], val[1][1][1], val[2][1][1], val[3][1][1]};
+            if constexpr (N != kImage) state.bias() = f32x4_t{state.bias()[1], state.bias()[2], state.bias()[3], state.bias()[0] + val[0][4 * (kLines / 9)][1]};
+            else state.bias() += f32x4_t{val[0][1][1], val[1][1][1], val[2][1][1], val[3][1][1]};
         }
         // -A at every second voxel: the sums of the bf16 instruction are cut off towards minus infinity, which adds up
         // over an image where the gradients themselves cancel (bias gradients: an error of 2e-6 instead of 1.2e-7).
@@ -398,7 +424,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         for (int j = 0; j < kLaneOut; j++)
 #pragma unroll
             for (int t = 0; t < kTaps; t++) val[j][t / 3][t % 3] *= factor;
-        // rows m of the lane (slot_of), eight at a time
+        // rows m of the wave (slot_of), eight at a time
         auto eight = [&](int i, float (&e8)[8]) {
 #pragma unroll
             for (int e = 0; e < 8; e++) {
@@ -434,14 +460,72 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             for (int k = 0; k < 3; k++) *reinterpret_cast<bf16x8_t *>(at + k * kPartBytes + (piece ^ 16 * i)) = s.p[k];
         }
         const bool any = __any(taken_whole(bad));
-        if (lane == 0) shared.bad_tile[wave] = any;
+        if (lane == 0) shared.bad_tile[buffer][number] = any;
     };
 
-    // ---- the products of a unit.  The wave's own space holds x as [part][channel][voxel], then what is added to
-    // grad_input as [channel][voxel]: loads and stores go by channel in whole lines, the matrix cores take 16
+    // ---- the products of a unit.  A worker's own space holds x as [block][part][channel][voxel], or what is added to grad_input
+    // as [block][channel][voxel]: loads and stores go by channel in whole lines, the matrix cores take 16
     // channels at once (loaded in that form, 64 bytes of 16 channels at a time, memory gives 2.6 to 3.0 TB/s instead of 4).
-    constexpr int kXRow = 2 * kUnit + 16, kDRow = 4 * kUnit + 16;   // bytes of a channel (16 apart in the banks)
-    const int first_seg = (wave % P) * kUnits * (kUnit / kSegment); // of the wave's first unit
+    const int first_seg = number % P * kUnits;    // of the wave's first unit
+    // (factors for the even and the odd voxels, in registers of their own: a sign in the instruction doubles its size)
+    struct Factors {
+        uint32_t even, odd;
+        __device__ explicit Factors(float f, uint32_t sign = 0) : even(__float_as_uint(f) | sign), odd(even ^ 0x80000000u)
+        {
+            asm volatile("" : "+v"(even), "+v"(odd));   // (a multiply-add with a scalar operand issues in twice the cycles)
+        }
+        __device__ float of(int e) const { return __uint_as_float(e % 2 ? odd : even); }
+    };
+    // Rows 16 t + n, voxels 8 q .. of segment j (the lane's address is that of voxel 8 q + n / 4 (+ 4), rows
+    // 4 (n % 4) .., which the read transposes).
+    auto read_rows = [&](uint32_t ll, int j, int t, bf16x8_t(&to)[3]) {
+        typedef short s16x4_t __attribute__((ext_vector_type(4)));
+        typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) s16x4_t *lds_tr_t;
+        const uint32_t nn = ll % 16, voxel = 8 * (ll / 16) + nn / 4;
+        const char *const tr = A + (j * G + t / 4) * kSlabBytes + voxel * kVoxelBytes + nn % 2 * 8;
+        const uint32_t piece = 16 * (nn % 4 / 2 ^ turn(voxel)), next = 16 * (nn % 4 / 2 ^ turn(voxel + 4));
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            const bf16x4_t lo = __builtin_bit_cast(
+                bf16x4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)(tr + p * kPartBytes + (piece ^ (uint32_t)(t % 4 * 32)))));
+            const bf16x4_t hi = __builtin_bit_cast(
+                bf16x4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)(tr + p * kPartBytes + 4 * kVoxelBytes + (next ^ (uint32_t)(t % 4 * 32)))));
+            to[p] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    };
+    // Voxels 16 s + n of segment j, rows 32 i + 8 q ..
+    auto read_voxels = [&](uint32_t ll, int j, int s, int i, bf16x8_t(&to)[3]) {
+        const uint32_t nn = ll % 16, qq = ll / 16;
+        const char *const vox = A + (j * G + i / 2) * kSlabBytes + nn * kVoxelBytes;
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+            to[p] = *reinterpret_cast<const bf16x8_t *>(vox + p * kPartBytes + s * 16 * kVoxelBytes + (16 * (qq ^ turn(nn)) ^ (uint32_t)(i % 2 * 64)));
+    };
+    // (no LDS addresses are kept over the tiles: registers)
+    auto fresh_lane = [&]() {
+        uint32_t ll = (uint32_t)lane;
+        asm volatile("" : "+v"(ll));
+        return ll & (kWave - 1);
+    };
+    // a value of A where it lies whole
+    auto whole_A = [&](int j, uint32_t voxel, uint32_t m) {
+        const char *const at = A + (j * G + m / kRows) * kSlabBytes + voxel * kVoxelBytes + 16 * (m % kRows / 8 ^ turn(voxel)) + m % 8 * 2;
+        return whole_value(*reinterpret_cast<const __bf16 *>(at), *reinterpret_cast<const __bf16 *>(at + kPartBytes));
+    };
+    // values of the tile at hand that can be split
+    auto tile_split = [&]() {
+        int bad = 0;
+#pragma unroll
+        for (int i = 0; i < kOfKind; i++) bad |= shared.bad_tile[buffer][i];
+        return __builtin_amdgcn_readfirstlane(bad) == 0;
+    };
+
+    // -- grad_kernel
+    f32x4_t xs[kVec];
+    auto request_x = [&](const Unit &un) {
+        request(x, a.C, un, xs);
+    };
     auto clear_skipped = [&](const Unit &un) {    // an infinity there belongs to the other segment
         if (__any(un.skip > 0)) {
 #pragma unroll
@@ -450,260 +534,111 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                 for (int e = 0; e < 4; e++) xs[i][e] = e >= un.skip ? xs[i][e] : 0.f;
         }
     };
-    // bit 4 i + e: the channel's gradient at voxel e is kept
-    auto mask_of = [&]() {
-        uint32_t bits = 0xffffu;
-        if (ch0 + 16 > a.mask_from) {             // uniform
-            bits = 0;
-#pragma unroll
-            for (int i = 0; i < kVec; i++)
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    bits |= ch0 + lc + kChannels * i < a.mask_from || 0.f < xs[i][e] ? 1u << (4 * i + e) : 0u;
-        }
-        return bits;
-    };
     // x in parts to the wave's own space; not finite where a value cannot be split
-    // (factors for the even and the odd voxels, in registers of their own: a sign in the instruction doubles its size)
-    struct Factors {
-        uint32_t even, odd;
-        __device__ explicit Factors(float f, uint32_t sign = 0) : even(__float_as_uint(f) | sign), odd(even ^ 0x80000000u)
-        {
-            asm volatile("" : "+s"(even), "+s"(odd));
-        }
-        __device__ float of(int e) const { return __uint_as_float(e % 2 ? odd : even); }
-    };
     auto put_x = [&](uint32_t sign_bit) {
         const Factors factor(kSplitScale, sign_bit);
-        float rest = 0.f;
+        float x8[8];
 #pragma unroll
-        for (int i = 0; i < kVec; i += 2) {
-            float x8[8];
+        for (int e = 0; e < 8; e++) x8[e] = xs[e / 4][e % 4] * factor.of(e);
+        Split8 s;
+        const float rest = split8(x8, s);
+        typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 #pragma unroll
-            for (int e = 0; e < 8; e++) x8[e] = xs[i + e / 4][e % 4] * factor.of(e);
-            Split8 s;
-            rest += split8(x8, s);
-            typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-#pragma unroll
-            for (int p = 0; p < 3; p++) {
-                char *const at = own + (p * 16 + lc + kChannels * i) * kXRow + 8 * lv;
-                *reinterpret_cast<bf16x4_t *>(at) = __builtin_shufflevector(s.p[p], s.p[p], 0, 1, 2, 3);
-                *reinterpret_cast<bf16x4_t *>(at + kChannels * kXRow) = __builtin_shufflevector(s.p[p], s.p[p], 4, 5, 6, 7);
-            }
+        for (int p = 0; p < 3; p++) {
+            char *const at = own_x + (p * 16 + lc) * kXRow + 8 * lv;
+            *reinterpret_cast<bf16x4_t *>(at) = __builtin_shufflevector(s.p[p], s.p[p], 0, 1, 2, 3);
+            *reinterpret_cast<bf16x4_t *>(at + kChannels * kXRow) = __builtin_shufflevector(s.p[p], s.p[p], 4, 5, 6, 7);
         }
         return rest;
     };
-    // what the wave's own space holds for grad_input, in units of `unit`, added to it and masked
-    auto add_d = [&](uint32_t bits, const Factors unit) {
-#pragma unroll
-        for (int i = 0; i < kVec; i++) {
-            const f32x4_t d = *reinterpret_cast<const f32x4_t *>(own + (lc + kChannels * i) * kDRow + 16 * lv);
-#pragma unroll
-            for (int e = 0; e < 4; e++) gs[i][e] = __builtin_fmaf(d[e], unit.of(e), gs[i][e]);
-        }
-        if (ch0 + 16 > a.mask_from) {             // uniform
-#pragma unroll
-            for (int i = 0; i < kVec; i++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) gs[i][e] = bits & 1u << (4 * i + e) ? gs[i][e] : 0.f;
-        }
-    };
-    constexpr int kK = kUnit / 32;                // steps of 32 voxels: the segments of the unit
     // False where a value cannot be split (and nothing is computed).
-    auto compute = [&](int u, bool split, uint32_t sign_bit, const Unit &un, const Unit &next) {
-        uint32_t ll = (uint32_t)lane;
-        if (G > 1 && P < 4) asm volatile("" : "+v"(ll));            // (no LDS addresses are kept over the tiles: registers)
-        const uint32_t nn = ll % 16, qq = ll / 16 % 4;
-        const char *const Au = A + (first_seg + u * kK) * G * kSlabBytes;
-        // rows 16 t + n, voxels 8 q .. of segment j (the lane's address is that of voxel 8 q + n / 4 (+ 4), rows
-        // 4 (n % 4) .., which the read transposes)
-        const uint32_t tr_voxel = 8 * qq + nn / 4;
-        const char *const tr = Au + tr_voxel * kVoxelBytes + nn % 2 * 8;
-        const uint32_t tr_piece = 16 * (nn % 4 / 2 ^ turn(tr_voxel)), tr_next = 16 * (nn % 4 / 2 ^ turn(tr_voxel + 4));
-        auto read_rows = [&](int j, int t, bf16x8_t(&to)[3]) {
-            typedef short s16x4_t __attribute__((ext_vector_type(4)));
-            typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-            typedef __attribute__((address_space(3))) s16x4_t *lds_tr_t;
-#pragma unroll
-            for (int p = 0; p < 3; p++) {
-                const char *const at = tr + (j * G + t / 4) * kSlabBytes + p * kPartBytes;
-                const bf16x4_t lo = __builtin_bit_cast(
-                    bf16x4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)(at + (tr_piece ^ (uint32_t)(t % 4 * 32)))));
-                const bf16x4_t hi = __builtin_bit_cast(
-                    bf16x4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr_t)(at + 4 * kVoxelBytes + (tr_next ^ (uint32_t)(t % 4 * 32)))));
-                to[p] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-            }
-        };
-        // voxels 16 s + n of the unit, rows 32 i + 8 q ..
-        const char *const vox = Au + nn * kVoxelBytes;
-        const uint32_t vox_piece = 16 * (qq ^ turn(nn));
-        auto read_voxels = [&](int s, int i, bf16x8_t(&to)[3]) {
-#pragma unroll
-            for (int p = 0; p < 3; p++)
-                to[p] = *reinterpret_cast<const bf16x8_t *>(vox + (s / 2 * G + i / 2) * kSlabBytes + p * kPartBytes +
-                                                            s % 2 * 16 * kVoxelBytes + (vox_piece ^ (uint32_t)(i % 2 * 64)));
-        };
+    auto kernel_unit = [&](int u, bool split, uint32_t sign_bit, const Unit &un, const Unit &next) {
         clear_skipped(un);
-        const uint32_t bits = mask_of();
+        own_sync();
         const float rest = put_x(sign_bit);
         const bool done = split && !__any(taken_whole(rest));       // uniform
         __builtin_amdgcn_sched_barrier(0);        // (the scheduler would move the loads to where they are used)
-        request(x, a.C, next, xs);
+        request_x(next);
         __builtin_amdgcn_sched_barrier(0);
         if (!done) return false;
         own_sync();
-        // Both products in stages of two chains of six matrix instructions, whose operands are read from LDS a
-        // stage ahead (where there are registers for it).
-        constexpr bool kAhead = G == 1 || P > 1;
-        bf16x8_t op[2][2][3], xp[kK][3];
-        constexpr int kRowStages = kTiles * kK / 2, kVoxelStages = kSteps * kK;
-        // stage r: tiles 2 (r / kK) and the next at segment r % kK
-        auto stage_rows = [&](int r, bf16x8_t(&to)[2][3]) {
+        const uint32_t ll = fresh_lane();
+        const Factors back(kSplitUnit, sign_bit);
+        // Stages of two chains of six matrix instructions, whose operands are read from LDS a stage ahead.
+        bf16x8_t op[2][2][3], xp[3];
+        auto stage = [&](int r) {
 #pragma unroll
-            for (int o = 0; o < 2; o++) read_rows(r % kK, r / kK * 2 + o, to[o]);
+            for (int o = 0; o < 2; o++) read_rows(ll, first_seg + u, 2 * r + o, op[r % 2][o]);
         };
-        // stage r: step r % kSteps at the voxels of segment r / kSteps
-        auto stage_voxels = [&](int r, bf16x8_t(&to)[2][3]) {
+        stage(0);
 #pragma unroll
-            for (int s = 0; s < 2; s++) read_voxels(r / kSteps * 2 + s, r % kSteps, to[s]);
-        };
-        f32x4_t acc[2];
-        bf16x8_t high[2];
-        stage_rows(0, op[0]);
+        for (int p = 0; p < 3; p++) xp[p] = *reinterpret_cast<const bf16x8_t *>(own_x + (p * 16 + ll % 16) * kXRow + ll / 16 * 16);
 #pragma unroll
-        for (int j = 0; j < kK; j++)
-#pragma unroll
-            for (int p = 0; p < 3; p++)
-                xp[j][p] = *reinterpret_cast<const bf16x8_t *>(own + (p * 16 + nn) * kXRow + (32 * j + 8 * qq) * 2);
-#pragma unroll
-        for (int r = 0; r < kRowStages; r++) {
-            if (!kAhead && r > 0) stage_rows(r, op[r % 2]);
-            if (kAhead && r + 1 < kRowStages) stage_rows(r + 1, op[(r + 1) % 2]);
-            if (kAhead && r + 1 == kRowStages) stage_voxels(0, op[(r + 1) % 2]);
+        for (int r = 0; r < kTiles / 2; r++) {
+            if (r + 1 < kTiles / 2) stage(r + 1);
             __builtin_amdgcn_sched_barrier(0);
-            // (the products of the high parts of both segments last: each instruction cuts its sum off at the size
-            // that it has reached)
+            f32x4_t acc[2];
 #pragma unroll
-            for (int k = 0; k < 5; k++)
+            for (int k = 0; k < 6; k++)
 #pragma unroll
-                for (int o = 0; o < 2; o++)
-                    acc[o] = mfma_split(op[r % 2][o], xp[r % kK], k == 0 && r % kK == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[o], k);
-            if (r % kK == kK - 1) {
+                for (int o = 0; o < 2; o++) acc[o] = mfma_split(op[r % 2][o], xp, k == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[o], k);
 #pragma unroll
-                for (int j = 0; j < kK; j++)
-#pragma unroll
-                    for (int o = 0; o < 2; o++)
-                        acc[o] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j == kK - 1 ? op[r % 2][o][0] : high[o], xp[j][0], acc[o], 0, 0, 0);
-            } else {
-#pragma unroll
-                for (int o = 0; o < 2; o++) high[o] = op[r % 2][o][0];
-            }
-            if (r % kK == kK - 1) {
-#pragma unroll
-                for (int o = 0; o < 2; o++) {
-                    sums[r / kK * 2 + o] += __uint_as_float(__float_as_uint(kSplitUnit) | sign_bit) * acc[o];
-                    asm volatile("" : "+v"(sums[r / kK * 2 + o]));  // (here and not at the end of the tile: registers)
-                }
+            for (int o = 0; o < 2; o++) {
+                state.sums(2 * r + o) += back.of(0) * acc[o];
+                asm volatile("" : "+v"(state.sums(2 * r + o)));                    // (here and not at the end of the tile: registers)
             }
             __builtin_amdgcn_sched_barrier(0);
-        }
-        if (update) {                             // uniform
-            // (x has been read: the wave's space is free for the sums)
-            f32x4_t d[2], all[2];
-#pragma unroll
-            for (int r = 0; r < kVoxelStages; r++) {
-                const int i = r % kSteps;
-                if (!kAhead) stage_voxels(r, op[(kRowStages + r) % 2]);
-                if (kAhead && r + 1 < kVoxelStages) stage_voxels(r + 1, op[(kRowStages + r + 1) % 2]);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int k = 0; k < 5; k++)
-#pragma unroll
-                    for (int s = 0; s < 2; s++)
-                        d[s] = mfma_split(op[(kRowStages + r) % 2][s], w[i], k == 0 && i % 2 == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : d[s], k);
-                if (i % 2 == 0) {
-#pragma unroll
-                    for (int s = 0; s < 2; s++) high[s] = op[(kRowStages + r) % 2][s][0];
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 2; j++)
-#pragma unroll
-                        for (int s = 0; s < 2; s++)
-                            d[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j ? op[(kRowStages + r) % 2][s][0] : high[s], w[i - 1 + j][0], d[s], 0, 0, 0);
-                }
-                // Summed slab by slab from zero and added to grad_input last: a chain of products that started from it
-                // would round each of them to its size.
-                if (i % 2 == 1) {
-#pragma unroll
-                    for (int s = 0; s < 2; s++) {
-                        all[s] = i == 1 ? d[s] : all[s] + d[s];
-                        if (i == kSteps - 1)
-                            *reinterpret_cast<f32x4_t *>(own + nn * kDRow + (16 * (r / kSteps * 2 + s) + 4 * qq) * 4) = all[s];
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            own_sync();
-            add_d(bits, Factors(kSplitUnit));
-            own_sync();
         }
         return true;
     };
-    // The same with the fp32 instruction, for values that cannot be split among x, A or the weights (A and the weights
-    // lie whole in the place of their parts).
-    auto compute_whole = [&](int u, uint32_t sign_bit, const Unit &un) {
+    // The same with the fp32 instruction, for values that cannot be split (A lies whole in the place of its parts).
+    auto kernel_whole = [&](int u, uint32_t sign_bit) {
         const float sign = __uint_as_float(sign_bit | 0x3f800000u);
-        clear_skipped(un);
-        const uint32_t bits = mask_of();
-        uint32_t ll = (uint32_t)lane;
-        asm volatile("" : "+v"(ll));
-        const uint32_t nn = ll % 16, qq = ll / 16 % 4;
-        const char *const Au = A + (first_seg + u * kK) * G * kSlabBytes;
-        auto value = [&](uint32_t voxel, uint32_t m) {
-            const char *const at = Au + (voxel / kSegment * G + m / kRows) * kSlabBytes + voxel % kSegment * kVoxelBytes +
-                                   16 * (m % kRows / 8 ^ turn(voxel)) + m % 8 * 2;
-            return whole_value(*reinterpret_cast<const __bf16 *>(at), *reinterpret_cast<const __bf16 *>(at + kPartBytes));
-        };
+        const uint32_t ll = fresh_lane(), nn = ll % 16, qq = ll / 16;
         own_sync();
 #pragma unroll
         for (int i = 0; i < kVec; i++)
-            *reinterpret_cast<f32x4_t *>(own + (lc + kChannels * i) * kDRow + 16 * lv) =
-                xs[i] * f32x4_t{sign, -sign, sign, -sign};
+            *reinterpret_cast<f32x4_t *>(own_x + (lc + kChannels * i) * kDRow + 16 * lv) = xs[i] * f32x4_t{sign, -sign, sign, -sign};
         own_sync();
 #pragma unroll
-        for (int t = 0; t < kTiles; t++)
-#pragma unroll
-            for (int j = 0; j < kK; j++) {
-                f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < kTiles; t++) {
+            f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-                for (int e = 0; e < 8; e++) {
-                    const uint32_t voxel = 32 * j + 8 * qq + (uint32_t)e;
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(value(voxel, 16 * t + nn),
-                                                               *reinterpret_cast<const float *>(own + nn * kDRow + 4 * voxel), acc, 0, 0, 0);
-                }
-                sums[t] += sign * acc;
+            for (int e = 0; e < 8; e++) {
+                const uint32_t voxel = 8 * qq + (uint32_t)e;
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(whole_A(first_seg + u, voxel, 16 * t + nn),
+                                                           *reinterpret_cast<const float *>(own_x + nn * kDRow + 4 * voxel), acc, 0, 0, 0);
             }
-        if (update) {
-            own_sync();
-#pragma unroll 1
-            for (int s = 0; s < kUnit / 16; s++) {
-                f32x4_t all = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int i = 0; i < kSteps; i++) {
-                    f32x4_t d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(value(16 * s + nn, 32 * i + 8 * qq + e),
-                                                                 whole_value(w[i][0][e], w[i][1][e]), d, 0, 0, 0);
-                    }
-                    all += d;
-                }
-                *reinterpret_cast<f32x4_t *>(own + nn * kDRow + (16 * s + 4 * qq) * 4) = all;
-            }
-            own_sync();
-            add_d(bits, Factors(1.f));
+            state.sums(t) += sign * acc;
         }
         own_sync();
+    };
+
+    // -- grad_input
+    f32x4_t gs[kVec];
+    auto request_g = [&](const Unit &un) {
+        if constexpr (FRESH) {
+#pragma unroll
+            for (int i = 0; i < kVec; i++) gs[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        } else {
+            request(gx, max(update_end, 1), un, gs);
+        }
+    };
+    // what the wave's own space holds for grad_input, in units of `unit`, added to it and masked with the activations m
+    const bool masks = ch0 + 16 > a.mask_from && ch0 < update_end;                 // uniform
+    auto add_d = [&](const f32x4_t (&m)[kVec], const Factors unit) {
+#pragma unroll
+        for (int i = 0; i < kVec; i++) {
+            const f32x4_t d = *reinterpret_cast<const f32x4_t *>(own_d + (lc + kChannels * i) * kDRow + 16 * lv);
+#pragma unroll
+            for (int e = 0; e < 4; e++) gs[i][e] = __builtin_fmaf(d[e], unit.of(e), gs[i][e]);
+        }
+        if (masks) {
+#pragma unroll
+            for (int i = 0; i < kVec; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) gs[i][e] = ch0 + lc + kChannels * i < a.mask_from || 0.f < m[i][e] ? gs[i][e] : 0.f;
+        }
     };
     auto store = [&](const Unit &un, bool all) {
         // Buffer stores, whose lanes past the end of the buffer store nothing: there is no branch around
@@ -712,13 +647,13 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         const uint64_t base = reinterpret_cast<uint64_t>(gx) + (uint64_t)un.img + (uint64_t)ch0 * plane;
         uint32_t at = lane_plane;
         asm volatile("" : "+v"(at));
-        const int end = un.skip == 0 && all ? a.update - ch0 : 0;
-        const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(base), 0, 0xfffffff0u, 0x00020000);
+        const int end = un.skip == 0 && all ? update_end - ch0 : 0;
+        const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(base), 0, 0xfffffff0u, 0x00020000);
 #pragma unroll
         for (int i = 0; i < kVec; i++) {
             typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
             const uint32_t plane_at = at + (uint32_t)(kChannels * i) * plane;
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, gs[i]), buffer,
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, gs[i]), to,
                                                    lc + kChannels * i < end ? plane_at + un.at : 0xffffffffu, 0, 0);
         }
         if (__any(un.skip % 4 != 0)) {            // some lanes own the last of their four voxels only
@@ -726,75 +661,173 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             for (int i = 0; i < kVec; i++)
 #pragma unroll
                 for (int e = 1; e < 4; e++)
-                    if (all && lc + kChannels * i < a.update - ch0 && un.skip > 0 && e >= un.skip)
+                    if (all && lc + kChannels * i < update_end - ch0 && un.skip > 0 && e >= un.skip)
                         reinterpret_cast<__attribute__((address_space(1))) float *>(base + (uint64_t)(lane_plane + (uint32_t)(kChannels * i) * plane) + un.at)[e] = gs[i][e];
         }
     };
-    // values of the tile at hand that can be split: A and the weights
-    auto tile_split = [&]() {
-        int bad = 0;
+    auto input_unit = [&](int u, const Unit &un) {
+        f32x4_t m[kVec];
+        if (masks) request(x, a.C, un, m);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t ll = fresh_lane(), nn = ll % 16, qq = ll / 16;
+        own_sync();                               // (what was there has been read)
+        // Stages of a step of rows at both halves of the voxels, read a stage ahead.
+        bf16x8_t op[2][2][3], high[2];
+        f32x4_t d[2], all[2];
+        auto stage = [&](int r) {
 #pragma unroll
-        for (int i = 0; i < kWaves; i++) bad |= shared.bad_tile[i];
-        return state.weights_split && __builtin_amdgcn_readfirstlane(bad) == 0;
+            for (int s = 0; s < 2; s++) read_voxels(ll, first_seg + u, s, r, op[r % 2][s]);
+        };
+        stage(0);
+#pragma unroll
+        for (int i = 0; i < kSteps; i++) {
+            if (i + 1 < kSteps) stage(i + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            const bf16x8_t w[3] = {state.weights(i, 0), state.weights(i, 1), state.weights(i, 2)};
+            // (the products of the high parts of a slab's two steps last: each instruction cuts its sum off at the size
+            // that it has reached)
+#pragma unroll
+            for (int k = 0; k < 5; k++)
+#pragma unroll
+                for (int s = 0; s < 2; s++) d[s] = mfma_split(op[i % 2][s], w, k == 0 && i % 2 == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : d[s], k);
+            if (i % 2 == 0) {
+#pragma unroll
+                for (int s = 0; s < 2; s++) high[s] = op[i % 2][s][0];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int s = 0; s < 2; s++)
+                        d[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j ? op[i % 2][s][0] : high[s], state.weights(i - 1 + j, 0), d[s], 0, 0, 0);
+                // Summed slab by slab from zero and added to grad_input last: a chain of products that started from it
+                // would round each of them to its size.
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    all[s] = i == 1 ? d[s] : all[s] + d[s];
+                    if (i == kSteps - 1) *reinterpret_cast<f32x4_t *>(own_d + nn * kDRow + (16 * s + 4 * qq) * 4) = all[s];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        own_sync();
+        add_d(m, Factors(kSplitUnit));
+    };
+    // (the weights lie whole in the place of their parts)
+    auto input_whole = [&](int u, const Unit &un) {
+        const uint32_t ll = fresh_lane(), nn = ll % 16, qq = ll / 16;
+        f32x4_t m[kVec];
+        if (masks) request(x, a.C, un, m);
+        own_sync();
+#pragma unroll 1
+        for (int s = 0; s < 2; s++) {
+            f32x4_t all = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < kSteps; i++) {
+                f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(whole_A(first_seg + u, 16 * s + nn, 32 * i + 8 * qq + e),
+                                                             whole_value(state.weights(i, 0)[e], state.weights(i, 1)[e]), d, 0, 0, 0);
+                all += d;
+            }
+            *reinterpret_cast<f32x4_t *>(own_d + nn * kDRow + (16 * s + 4 * qq) * 4) = all;
+        }
+        own_sync();
+        add_d(m, Factors(1.f));
     };
 
+    const bool kernel = cb < blocks && kind == kKernel, input = cb < blocks && ch0 < update_end && kind == kInput;     // uniform
     if constexpr (WHOLE) {
 #pragma unroll 1
         for (int tile = lb; tile < a.tiles; tile += wgs) {
             const Tile t = tile_of(tile);
-            const Place here = locate(t, segment);
-            gather(t, here);
-            gathered(here, -1);
+            if (kind == kGatherer) {
+                const Voxel here = locate_pair(t);
+                gather(t, here);
+                gathered(here);
+            }
             __syncthreads();
-            if (active) {
-                const bool split = tile_split();
+            const bool split = tile_split();
 #pragma unroll 1
-                for (int u = 0; u < kUnits; u++) {
-                    const Unit un = unit_of(t, u);
-                    request(x, a.C, un, xs);
-                    request_g(un);
+            for (int u = 0; u < kUnits; u++) {    // (what the first run has done is left out)
+                const Unit un = unit_of(t, u);
+                if (kernel) {
+                    request_x(un);
                     clear_skipped(un);
-                    const float rest = put_x(t.sign);
-                    if (split && !__any(taken_whole(rest))) continue;    // (the first run has done it)
-                    compute_whole(u, t.sign, un);
+                    own_sync();
+                    if (!split || __any(taken_whole(put_x(t.sign)))) kernel_whole(u, t.sign);
+                }
+                if (input && !(split && state.weights_split)) {
+                    request_g(un);
+                    input_whole(u, un);
                     store(un, true);
                 }
             }
             __syncthreads();
         }
         return false;
-    } else {
+    } else if (kind == kGatherer) {
+        // A tile is formed in the one buffer while the workers have the other; a barrier, and they change.
+        Voxel here = locate_pair(tile_of(lb));
+        gather(tile_of(lb), here);
+        for (int tile = lb; tile < a.tiles; tile += wgs) {          // uniform over the workgroup
+            gathered(here);
+            if (tile + wgs < a.tiles) {           // (the loads have the time of a tile to arrive)
+                const Tile then = tile_of(tile + wgs);
+                here = locate_pair(then);
+                gather(then, here);
+            }
+            turn_over();
+            lds_sync();
+        }
+        lds_sync();
+        return false;
+    } else if (kind == kKernel) {
+        bool again = false;                       // units were left to the second run
         Tile now = tile_of(lb);
         Unit un = unit_of(now, 0);
-        request(x, a.C, un, xs);
-        request_g(un);
-        bool again = false;                       // units were left to the second run
-        Place here = locate(now, segment);
-        gather(now, here);
-        int round = 0;
-        for (int tile = lb; tile < a.tiles; tile += wgs) {          // uniform over the workgroup
-            gathered(here, round++);
-            lds_sync();
-            const Tile then = tile_of(tile + wgs);
-            here = locate(then, segment);
-            if (active) {
+        if (kernel) request_x(un);
+        lds_sync();
+        for (int tile = lb; tile < a.tiles; tile += wgs) {
+            if (kernel) {
+                const Tile then = tile_of(tile + wgs);
                 const bool split = tile_split();
 #pragma unroll
                 for (int u = 0; u < kUnits; u++) {
                     const Unit next = u + 1 < kUnits ? unit_of(now, u + 1) : unit_of(then, 0);
-                    const bool done = compute(u, split, now.sign, un, next);
-                    again = again || !done;
-                    if (u + 1 == kUnits) gather(then, here);
-                    store(un, done);
+                    again = !kernel_unit(u, split, now.sign, un, next) || again;
+                    un = next;
+                }
+                now = then;
+            }
+            turn_over();
+            lds_sync();
+        }
+        return again;
+    } else {
+        bool again = false;
+        Tile now = tile_of(lb);
+        Unit un = unit_of(now, 0);
+        if (input) request_g(un);
+        lds_sync();
+        for (int tile = lb; tile < a.tiles; tile += wgs) {
+            if (input) {
+                const Tile then = tile_of(tile + wgs);
+                const bool split = tile_split() && state.weights_split;
+#pragma unroll
+                for (int u = 0; u < kUnits; u++) {
+                    const Unit next = u + 1 < kUnits ? unit_of(now, u + 1) : unit_of(then, 0);
+                    if (split) input_unit(u, un);
+                    store(un, split);
                     __builtin_amdgcn_sched_barrier(0);
                     request_g(next);
                     __builtin_amdgcn_sched_barrier(0);
                     un = next;
                 }
-            } else {
-                gather(then, here);
+                again = again || !split;
+                now = then;
             }
-            now = then;
+            turn_over();
             lds_sync();
         }
         return again;
@@ -803,10 +836,11 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
 
 // FRESH: grad_input is written, not added to.
 template <int N, int G, int P, bool FRESH = false>
-__global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, const float *__restrict__ x, const float *gy,
+__global__ __launch_bounds__(kPullThreads, 3) void pull_rows(const PullArgs a, const float *__restrict__ x, const float *gy,
                                                              float *gx, float *__restrict__ part, float *__restrict__ bias_part)
 {
-    constexpr int kSegs = PullShape<G, P>::kSegs, kTiles = PullShape<G, P>::kTiles;
+    using S = PullShape<G, P>;
+    constexpr int kTiles = S::kTiles;
     constexpr int kTaps = Gather<N>::kTaps, kLaneOut = Gather<N>::kLaneOut, kSlabOut = Gather<N>::kOutputs;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tid = threadIdx.x;
@@ -816,16 +850,15 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
     const int chunk = bid < big ? bid / a.chunks.wgs : a.chunks.large + (bid - big) / a.chunks.wgs_small;
     const int blocks = a.chunks.size(chunk), c0 = a.chunks.first_block(chunk) * 16;
     const int wgs = a.chunks.rows(chunk), wg = bid - a.chunks.first_wg(chunk);
-    const int cb = wave / P, ch0 = c0 + cb * 16;  // the wave's block
+    // (the workers of the two products that have no block are on different SIMDs)
+    const int kind = wave / kOfKind, number = (wave + (kind == kInput ? 2 : 0)) % kOfKind;
+    const int cb = number / P, ch0 = c0 + cb * 16;                  // a worker's block
     __shared__ PullShared shared;
     PullState<G> state;
 
     if (tid == 0) shared.bad_again = 0;
-    if (tid < G * kSlabOut) {
-        const int o = min(tid, a.out.n - 1), d = a.out.dil[o];
-        shared.sources[tid] = Source{N == kVolume ? 4u * (uint32_t)(d * (int)a.sz) : 0u, 4u * (uint32_t)(d * (int)a.sy), 4u * (uint32_t)d, (uint32_t)o * ((uint32_t)a.gsc * 4u)};
-    }
     auto load_weights = [&](bool whole) {
+        if (kind != kInput) return;               // uniform
         int ch = ch0 + n, qq = q;
         if (whole) asm volatile("" : "+v"(ch), "+v"(qq));       // (nothing of the first call is kept for the second)
 #pragma unroll
@@ -842,71 +875,72 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows(const PullArgs a, 
             if (whole) put_whole(v, s);
             else if (__any(taken_whole(split8(v, s)))) state.weights_split = false;
 #pragma unroll
-            for (int p = 0; p < 3; p++) state.w[step][p] = s.p[p];
+            for (int p = 0; p < 3; p++) state.set_weights(step, p, s.p[p]);
         }
     };
     state.weights_split = true;
+#pragma unroll
+    for (f32x4_t &v : state.kept) v = f32x4_t{0.f, 0.f, 0.f, 0.f};
     load_weights(false);
     __syncthreads();
 
     float *const row = part + (int64_t)bid * (a.chunks.blocks * 1024 * G);
-#pragma unroll
-    for (int t = 0; t < kTiles; t++) state.sums[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    shared.bias_sums[tid] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    const bool again = pull_tiles<N, G, P, FRESH, false>(a, x, gy, gx, lds, shared, tid, wave, blocks, c0, wgs, wg, state);
+    const bool again = pull_tiles<N, G, P, FRESH, false>(a, x, gy, gx, lds, shared, kind, number, lane, blocks, c0, wgs, wg, state);
     if (lane == 0 && again) shared.bad_again = 1;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(shared.bad_again) != 0) {    // uniform over the workgroup
-        int tid2 = tid;
-        asm volatile("" : "+v"(tid2));           // (nothing of the first run is kept for the second)
+        int lane2 = lane;
+        asm volatile("" : "+v"(lane2));          // (nothing of the first run is kept for the second)
         load_weights(true);
-        pull_tiles<N, G, P, FRESH, true>(a, x, gy, gx, lds, shared, tid2, wave, blocks, c0, wgs, wg, state);
+        pull_tiles<N, G, P, FRESH, true>(a, x, gy, gx, lds, shared, kind, number, lane2, blocks, c0, wgs, wg, state);
     }
 
     // the sums, of the waves that share a block through LDS
     constexpr int kBlock = 1024 * G;              // sums of a block of channels
     if constexpr (P == 1) {
-        if (cb < blocks) {
+        if (kind == kKernel && cb < blocks) {
 #pragma unroll
             for (int t = 0; t < kTiles; t++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) row[cb * kBlock + (t * 4 + r) * kWave + lane] = state.sums[t][r];
+                for (int r = 0; r < 4; r++) row[cb * kBlock + (t * 4 + r) * kWave + lane] = state.sums(t)[r];
         }
     } else {
         float *const red = reinterpret_cast<float *>(lds);
         __syncthreads();
+        if (kind == kKernel) {
 #pragma unroll
-        for (int t = 0; t < kTiles; t++)
+            for (int t = 0; t < kTiles; t++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) red[wave * kBlock + (t * 4 + r) * kWave + lane] = state.sums[t][r];
+                for (int r = 0; r < 4; r++) red[number * kBlock + (t * 4 + r) * kWave + lane] = state.sums(t)[r];
+        }
         __syncthreads();
-        for (int i = tid; i < kWaves / P * kBlock; i += kWaves * kWave) {
+        for (int i = tid; i < kOfKind / P * kBlock; i += kPullThreads) {
             const int b = i / kBlock;
             const float *const r = red + b * P * kBlock + i % kBlock;
             if (b < blocks) row[i] = P == 2 ? r[0] + r[kBlock] : (r[0] + r[kBlock]) + (r[2 * kBlock] + r[3 * kBlock]);
         }
     }
     if (chunk != 0) return;
-    const int v = lane % kSegment, h = lane / kSegment;
     // the bias gradients: the centre taps, over the lanes' voxels and the segments
-    f32x4_t bias_sum = shared.bias_sums[tid];
+    const int h = wave % 2;                       // (the waves' outputs: see the gather)
+    f32x4_t bias_sum = state.bias();
     if constexpr (N != kImage) bias_sum[0] = (bias_sum[0] + bias_sum[1]) + (bias_sum[2] + bias_sum[3]);
 #pragma unroll
     for (int j = 0; j < kLaneOut; j++)
 #pragma unroll
-        for (int off = kSegment / 2; off > 0; off >>= 1) bias_sum[j] += __shfl_down(bias_sum[j], off, kSegment);
-    float *const red = reinterpret_cast<float *>(lds);
+        for (int off = kWave / 2; off > 0; off >>= 1) bias_sum[j] += __shfl_down(bias_sum[j], off);
+    float *const red = reinterpret_cast<float *>(lds);              // [waves of a slab][slab][column]
     __syncthreads();
-    if (v == 0) {
+    if (lane == 0 && kind == kGatherer) {
 #pragma unroll
         for (int j = 0; j < kLaneOut; j++)
-            if (N != kImage || j < 3 || h == 0) red[wave * kBiasColumns + (N != kImage ? h : j < 3 ? 3 * h + j : 6)] = bias_sum[j];
+            if (N != kImage || j < 3 || h == 0) red[wave / 2 * kBiasColumns + (N != kImage ? h : j < 3 ? 3 * h + j : 6)] = bias_sum[j];
     }
     __syncthreads();
     if (tid < G * kBiasColumns && tid % kBiasColumns < kSlabOut) {
         float s = 0.f;
 #pragma unroll
-        for (int i = 0; i < kSegs; i++) s += red[i * G * kBiasColumns + tid];
+        for (int i = 0; i < kOfKind / (2 * G); i++) s += red[i * G * kBiasColumns + tid];
         bias_part[wg * (G * kBiasColumns) + tid] = s;
     }
 }
@@ -1224,20 +1258,20 @@ FinishArgs finish_args(const Geom &g, const View<const float> &x, const group2d:
     return a;
 }
 
-template <int N, int G, int P, bool FRESH = false>
-hipError_t pull_launch(const PullArgs &a, int wgs, const float *x, const float *gy, float *gx, float *part, float *bias_part,
-                       hipStream_t s)
+template <typename F>
+hipError_t pull_launch(F *kernel, int threads, int lds, LargeLds &large, const PullArgs &a, int wgs, const float *x, const float *gy, float *gx, float *part,
+                       float *bias_part, hipStream_t s)
 {
-    constexpr int kLds = kWaves * (kSlabBytes + PullShape<G, P>::kOwnBytes);
-    static LargeLds large;
-    const hipError_t e = large.allow(reinterpret_cast<const void *>(&pull_rows<N, G, P, FRESH>), kLds);
+    const hipError_t e = large.allow(reinterpret_cast<const void *>(kernel), lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((pull_rows<N, G, P, FRESH>), dim3(wgs), dim3(kWaves * kWave), kLds, s, a, x, gy, gx, part, bias_part);
+    hipLaunchKernelGGL(kernel, dim3(wgs), dim3(threads), lds, s, a, x, gy, gx, part, bias_part);
     return hipGetLastError();
 }
 
 // Blocks of a chunk, at most (one slab: 411 us over 100 channels, 463 with 8).
-int most_blocks(int slabs) { return slabs == 1 ? 4 : kWaves; }
+int most_blocks(int slabs) { return slabs == 1 ? 4 : 8; }
+// Blocks of a chunk that pull_rows takes; pull_rows_wide the others.
+constexpr int kNarrowBlocks = 4;
 
 // As many workgroups as are resident, shared out over the chunks by their size.
 struct PullPlan {
@@ -1255,7 +1289,7 @@ PullPlan pull_plan(int64_t batch, int64_t rows, int64_t span, int64_t channels, 
     c.blocks = (nb + c.n - 1) / c.n;
     c.large = nb - c.n * (c.blocks - 1);
     p.segs = (int)((span + kSegment - 1) / kSegment);
-    const int per_tile = kWaves / slabs;
+    const int per_tile = (c.blocks > kNarrowBlocks ? kWaves : kOfKind) / slabs;
     p.image_tiles = (int)((rows * p.segs + per_tile - 1) / per_tile);
     p.tiles = (int)batch * p.image_tiles;
     auto share = [&](int blocks) {
@@ -1356,22 +1390,29 @@ hipError_t pull_part(const Geom &g, const View<const float> &x, const float *gy,
     }
     float *const bias_part = ws + (int64_t)p.wgs * slabs * p.chunks.blocks * 1024;
     hipError_t e = hipErrorInvalidConfiguration;
-    // waves to a block: 4, 2 or 1
-    const int share = p.chunks.blocks <= 2 ? 4 : p.chunks.blocks <= 4 ? 2 : 1;
+    const int blocks = p.chunks.blocks;
     auto launch = [&](auto f) {
         constexpr int N = decltype(f)::value;
+        auto run = [&](auto g_, auto p_, auto fresh_) {
+            constexpr int G = decltype(g_)::value, P = decltype(p_)::value;
+            static LargeLds large;
+            return pull_launch(&pull_rows<N, G, P, decltype(fresh_)::value>, kPullThreads, PullShape<G, P>::kLds, large, a, p.wgs, x.p, gy, grads.p, ws,
+                               bias_part, s);
+        };
+        constexpr std::integral_constant<int, 1> one{};
+        constexpr std::integral_constant<int, 2> two{};
+        constexpr std::integral_constant<int, 4> four{};
         if constexpr (N != kVolume) {
-            if (fresh) return share == 4 ? pull_launch<N, 1, 4, true>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s)
-                                         : pull_launch<N, 1, 2, true>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
+            constexpr std::true_type yes{};
+            if (fresh) return blocks > 2 ? run(one, one, yes) : blocks > 1 ? run(one, two, yes) : run(one, four, yes);
         }
-        switch (slabs * 10 + share) {
-        case 14: return pull_launch<N, 1, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
-        case 12: return pull_launch<N, 1, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
-        case 24: return pull_launch<N, 2, 4>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
-        case 22: return pull_launch<N, 2, 2>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
-        case 21: return pull_launch<N, 2, 1>(a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
+        constexpr std::false_type no{};
+        if (slabs == 1) return blocks > 2 ? run(one, one, no) : blocks > 1 ? run(one, two, no) : run(one, four, no);
+        if (blocks > kNarrowBlocks) {
+            static LargeLds large;
+            return pull_launch(&pull_rows_wide<N>, kWaves * kWave, kWideLds, large, a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
         }
-        return hipErrorInvalidConfiguration;
+        return blocks > 2 ? run(two, one, no) : run(two, two, no);
     };
     switch (form) {
     case kImage: e = launch(std::integral_constant<int, kImage>{}); break;

@@ -127,6 +127,18 @@ def test_block_backward_in_groups_of_up_to_fourteen(case):
         check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=59)
 
 
+# Passes over one to four blocks of 16 channels, where a tile is gathered while the one before goes through the products: one, two or
+# three tiles for a workgroup, not the same number for all of them, workers without a block, rows that end inside a
+# tile; one slab of outputs and two.
+@pytest.mark.parametrize("size, batch", [((7, 64), 1), ((90, 200), 1), ((64, 257), 2), ((9, 17, 35), 1), ((12, 40, 72), 2)], ids=str)
+@pytest.mark.parametrize("c_in", [3, 20, 40, 60])
+@pytest.mark.parametrize("slabs", [1, 2])
+def test_backward_passes_over_few_blocks(size, batch, c_in, slabs):
+    depth = (5 if slabs == 1 else 9) if len(size) == 2 else 2 * slabs
+    with tuning({"bwd.group": 1}):
+        check_block(len(size), size, c_in, 1, depth, batch, dilations=[1 + 2 * i % 5 for i in range(depth)], seed=107)
+
+
 # Volumes: groups of up to four outputs, the same tiles over the rows of all slices.  Slices and rows
 # whose outer taps lie outside on both sides, dilations up to the volume, tiles that end inside a volume and between
 # two, every remainder modulo four, groups of 2, 3 and 4 outputs and a layer left over, two channels per layer, blocks
