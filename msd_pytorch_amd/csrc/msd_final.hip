@@ -10,6 +10,7 @@
 //             row of partial sums per wave and added in a fixed order by a second kernel,
 //             so the result does not depend on scheduling.
 // Output channels are handled in groups of at most MAXO per launch.
+#include "msd_group.h"
 #include "msd_kernels.h"
 #include "msd_rows.h"
 
@@ -340,34 +341,44 @@ __global__ __launch_bounds__(kFinalThreads) void final_forward_loss_kernel(
     }
 }
 
-// The same pass for up to 128 input channels with the stack read ONCE (fp32): a workgroup of
+// The same pass for up to 512 input channels with the stack read ONCE (fp32): a workgroup of
 // eight waves owns a tile of 64 * V voxels; lane l of every wave stands for the same V voxels
-// and wave w takes the channels c % 8 == w.  First walk: each wave loads its channels of the
-// tile (all requests issued before the first use), adds its share of the outputs and leaves
-// the values in LDS; the eight partial outputs meet in LDS, every wave forms the loss
+// and wave w takes the channels c % 8 == w.  First walk: each wave adds its channels' share of the outputs, leaves
+// the values in LDS and requests the next tile's in their place; the eight partial outputs meet in LDS, every wave forms the loss
 // gradient g of its lanes' voxels; second walk: each wave takes its channels back from LDS
 // and adds g * x to per-lane running sums, which live in registers over all tiles of the
 // workgroup (tile t, t + grid, ...) and are reduced over the lanes once at the end: one row
 // of partial sums per workgroup.  Same columns of `part` as the kernel above.
+//
+// Bound by memory where tiles are many (128^3, 51 channels, one output: 5.3 TB/s), else by the chain of a tile: first walk, LDS, loss,
+// LDS, second walk, beside which only the next tile's loads run.  Requested before the walk and not in the tile before, with scalar loads of the
+// weights between the channels (a round trip each), two voxels per lane above 64 channels and both walks reading memory
+// above 128, us: 1024 x 1024, 101 channels, four labels 182 -> 115; 4 x 512 x 512, 101, one output 110 -> 91; 3 x 333 x 477, 35, three labels
+// 42 -> 32; 1024 x 1024, 201 / 402 channels, one output 314 -> 201 / 652 -> 398 (2.1 / 4.2 TB/s); 256 x 256, 201: 92 -> 20.
 constexpr int kTiledWaves = 8;
 constexpr int kTiledThreads = kTiledWaves * kWave;
-constexpr int kTiledMaxChannels = 128;
+constexpr int kTiledMaxChannels = 512;
+
+// Workgroups per compute unit: their registers (the running sums, the next tile's values, targets) decide.
+template <int V, int MAXO, int KIND, int CC> constexpr int tiled_workgroups()
+{
+    return MAXO * CC + V * CC + (KIND == 2 ? 0 : 2 * MAXO * V) >= 96 ? 1 : 2;
+}
 
 template <int V, int MAXO, int KIND, int CC>
-__global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
+__global__ __launch_bounds__(kTiledThreads, (2 * tiled_workgroups<V, MAXO, KIND, CC>())) void final_forward_loss_tiled(
     int64_t nvox, int tiles_per_image, int total_tiles, int C, int c_out, const float *__restrict__ x, int64_t xsb,
     int64_t xsc, const float *__restrict__ w, const float *__restrict__ bias, const void *__restrict__ target,
     int64_t tsb, int64_t tsc, float *__restrict__ out, int64_t osb, int64_t osc, float *__restrict__ gout, int64_t gsb,
     int64_t gsc, float inv_n, int want_sums, float *__restrict__ part, int64_t rows)
 {
     extern __shared__ float lds_tile[];
-    // weights and bias are read-only for the whole kernel: addressed as constant memory they
-    // are wave-uniform scalar loads (as plain global loads next to the stores of the loop they
-    // would each take a vector register)
+    // the bias is read-only for the whole kernel: addressed as constant memory it is wave-uniform scalar loads (as plain
+    // global loads next to the stores of the loop it would take vector registers)
     typedef const __attribute__((address_space(4))) float *const_floats_t;
-    const const_floats_t wk = (const_floats_t)(uintptr_t)w;
     const const_floats_t bk = (const_floats_t)(uintptr_t)bias;
     constexpr int TV = kWave * V;                             // voxels of a tile
+    constexpr int kStep = 4;                                  // channels whose place the next tile's take
     float *red = lds_tile + (size_t)C * TV;                   // [wave][o][e][lane]; then g as [o][e][lane]
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
     float sw[MAXO][CC], sb[MAXO], lsum = 0.f;
@@ -377,111 +388,164 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
 #pragma unroll
         for (int cc = 0; cc < CC; cc++) sw[o][cc] = 0.f;
     }
-    // this wave's weights: w[o][c] for c = cc * 8 + wave (zero past the last channel)
-    for (int tile = blockIdx.x; tile < total_tiles; tile += gridDim.x) {
-        // new values as far as the compiler knows: the weights (scalar loads) and the channels'
-        // offsets are formed again per tile instead of being kept, and spilled, over the loop
-        asm volatile("" : "+s"(xsc), "+s"(C));
-        const int b = tile / tiles_per_image;
-        const int64_t i = (int64_t)(tile - b * tiles_per_image) * kWave + lane;
-        const int64_t nvec = (nvox + V - 1) / V;
-        const bool active = i < nvec;
+    const int64_t nvec = (nvox + V - 1) / V;
+    struct Place {
+        int b, skip;
+        bool active;
+        int64_t iv;
+    };
+    auto locate = [&](int tile) {
+        Place p;
+        p.b = tile / tiles_per_image;
+        const int64_t i = (int64_t)(tile - p.b * tiles_per_image) * kWave + lane;
+        p.active = i < nvec;
         // lanes past the end work on valid voxels and contribute zeros; the last lane's are moved left where there are fewer
         // than V, those below `skip` are the lane's before it
-        const int64_t iv = min((active ? i : nvec - 1) * V, nvox - V);
-        const int skip = active ? (int)(i * V - iv) : 0;
-        // a uniform base per channel plus one 32-bit lane offset: no address registers per request
-        const uint64_t xbase = reinterpret_cast<uint64_t>(x + (int64_t)b * xsb);
-        const uint32_t xoff = (uint32_t)iv * 4u;
+        p.iv = min((p.active ? i : nvec - 1) * V, nvox - V);
+        p.skip = p.active ? (int)(i * V - p.iv) : 0;
+        return p;
+    };
+    // a wave's channels cc * 8 + wave (past the last one that again)
+    float v[CC][V];
+    int count = (C - wave + kTiledWaves - 1) / kTiledWaves;   // of the wave's channels
+    float *const own = lds_tile + wave * TV + lane * V;       // what the wave itself stores and reads
+    uint64_t at = 0;                                          // of the channel that is asked for next: a uniform base, and a lane offset
+    uint32_t off = 0;
+    auto go_to = [&](const Place &p) {
+        at = reinterpret_cast<uint64_t>(x + (int64_t)p.b * xsb + (int64_t)min(wave, C - 1) * xsc);
+        off = (uint32_t)p.iv * 4u;
+    };
+    auto request = [&](int cc) {
+        load_global_vec_unaligned<V>(at, off, v[cc]);
+        at += cc + 1 < count ? (uint64_t)xsc * (4 * kTiledWaves) : 0;
+    };
+    go_to(locate(blockIdx.x));
+#pragma unroll
+    for (int cc = 0; cc < CC; cc++) request(cc);
+    // the wave's weights: lane cc has those of channel cc (scalar loads, one after the other between the channels, take longer than all else)
+    float weights[MAXO];
+#pragma unroll
+    for (int o = 0; o < MAXO; o++) weights[o] = w[(int64_t)min(o, c_out - 1) * C + min(lane * kTiledWaves + wave, C - 1)];
+    for (int tile = blockIdx.x; tile < total_tiles; tile += gridDim.x) {
+        // new values as far as the compiler knows: the channels' offsets are formed again per tile instead of being kept, and
+        // spilled, over the loop
+        asm volatile("" : "+s"(xsc), "+s"(count));
+        const Place here = locate(tile);
+        const int b = here.b, skip = here.skip;
+        const bool active = here.active;
+        const int64_t iv = here.iv;
+        // the targets, before the next tile's values (loads retire in order)
+        int64_t label = 0;
+        float t[MAXO][V];
+        if constexpr (KIND == 2) {
+            label = (static_cast<const int64_t *>(target) + (int64_t)b * tsb + iv)[min(wave, V - 1)];
+        } else {
+#pragma unroll
+            for (int o = 0; o < MAXO; o++)
+                load_global_vec_unaligned<V>(reinterpret_cast<uint64_t>(static_cast<const float *>(target) + (int64_t)b * tsb +
+                                                             (int64_t)min(o, c_out - 1) * tsc), (uint32_t)iv * 4u, t[o]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
         float acc[MAXO][V];
 #pragma unroll
         for (int o = 0; o < MAXO; o++)
 #pragma unroll
             for (int e = 0; e < V; e++) acc[o][e] = 0.f;
-        // channels in groups of G requests, all of a group issued before its first use: all of
-        // the wave's channels at once where the running sums leave the registers for it
-        constexpr int G = MAXO * CC + V * CC < 96 ? CC : (CC < 24 / V ? CC : 24 / V);
+        const bool more = tile + (int)gridDim.x < total_tiles;
+        go_to(locate(more ? tile + (int)gridDim.x : tile));
 #pragma unroll
-        for (int c0 = 0; c0 < CC; c0 += G) {
-            float v[G][V];
+        for (int cc = 0; cc < CC; cc++) {
+            if (cc < count) {                                 // uniform
 #pragma unroll
-            for (int j = 0; j < G; j++)
-                load_global_vec_unaligned<V>(xbase + (uint64_t)((int64_t)min((c0 + j) * kTiledWaves + wave, C - 1) * xsc * 4), xoff,
-                                   v[j]);
+                for (int o = 0; o < MAXO; o++) {
+                    const float wv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weights[o]), cc));
 #pragma unroll
-            for (int j = 0; j < G; j++) {
-                const int c = (c0 + j) * kTiledWaves + wave;  // uniform
-                if (c < C) {
-#pragma unroll
-                    for (int o = 0; o < MAXO; o++) {
-                        const float wv = wk[(int64_t)min(o, c_out - 1) * C + c];
-#pragma unroll
-                        for (int e = 0; e < V; e++) acc[o][e] += wv * v[j][e];
-                    }
-                    store_elems<float, V>(lds_tile + (size_t)c * TV + lane * V, v[j]);
+                    for (int e = 0; e < V; e++) acc[o][e] += wv * v[cc][e];
                 }
+                store_elems<float, V>(own + cc * kTiledWaves * TV, v[cc]);
+            }
+            if (cc % kStep == kStep - 1) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (more) {                                   // uniform
+#pragma unroll
+                    for (int j = cc + 1 - kStep; j <= cc; j++) request(j);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
 #pragma unroll
         for (int o = 0; o < MAXO; o++)
 #pragma unroll
             for (int e = 0; e < V; e++) red[((wave * MAXO + o) * V + e) * kWave + lane] = acc[o][e];
-        __syncthreads();
-        // the eight partial outputs in a fixed order (a loop that stays a loop: unrolled, all
-        // 8 * MAXO * V values would be requested at once and held in registers)
-#pragma unroll
-        for (int o = 0; o < MAXO; o++)
-#pragma unroll
-            for (int e = 0; e < V; e++) acc[o][e] = red[(o * V + e) * kWave + lane];
-#pragma unroll 1
-        for (int q = 1; q < kTiledWaves; q++) {
-            const float *rq = red + (size_t)q * MAXO * V * kWave + lane;
-#pragma unroll
-            for (int o = 0; o < MAXO; o++)
-#pragma unroll
-                for (int e = 0; e < V; e++) acc[o][e] += rq[(o * V + e) * kWave];
-        }
+        group2d::lds_sync();
         float g[MAXO][V];
         float tile_loss = 0.f;
         if constexpr (KIND == 2) {
             // the softmax is the expensive part: wave q forms it for element q of every lane's
-            // voxels only, and the waves exchange the results through LDS below
-            const int64_t *lab = static_cast<const int64_t *>(target) + (int64_t)b * tsb + iv;
+            // voxels only, and the waves exchange the results through LDS, in the place of the partial outputs that only it reads
+            float *gs = red, *ls = red + MAXO * V * kWave;    // [o][e][lane] each
+            if (wave < V) {                                   // uniform
+                float *const mine = red + wave * kWave + lane;
+                float a[MAXO];
+                // (the eight partial outputs in a fixed order)
 #pragma unroll
-            for (int e = 0; e < V; e++) {
-                if (wave != e) continue;                      // uniform
-                float m = acc[0][e] + (bias ? bk[0] : 0.f);
+                for (int o = 0; o < MAXO; o++) a[o] = mine[o * V * kWave];
+#pragma unroll
+                for (int q = 1; q < kTiledWaves; q++)
+#pragma unroll
+                    for (int o = 0; o < MAXO; o++) a[o] += mine[(q * MAXO + o) * V * kWave];
+                float m = a[0] + (bias ? bk[0] : 0.f);
 #pragma unroll
                 for (int o = 0; o < MAXO; o++) {
-                    acc[o][e] += bias && o < c_out ? bk[o] : 0.f;
-                    if (o < c_out) m = acc[o][e] > m ? acc[o][e] : m;
+                    a[o] += bias && o < c_out ? bk[o] : 0.f;
+                    if (o < c_out) m = a[o] > m ? a[o] : m;
                 }
                 float se = 0.f;
 #pragma unroll
                 for (int o = 0; o < MAXO; o++)
-                    if (o < c_out) se += exp(acc[o][e] - m);
+                    if (o < c_out) se += exp(a[o] - m);
                 const float lse = m + log(se);
-                const int64_t t = lab[e];
 #pragma unroll
                 for (int o = 0; o < MAXO; o++) {
-                    acc[o][e] -= lse;                         // log-probability
-                    const float pr = o < c_out ? exp(acc[o][e]) : 0.f;
-                    g[o][e] = active && o < c_out ? (pr - (t == o ? 1.f : 0.f)) * inv_n : 0.f;
-                    if (active && e >= skip && t == o) tile_loss -= acc[o][e];
+                    a[o] -= lse;                              // log-probability
+                    const float pr = o < c_out ? exp(a[o]) : 0.f;
+                    if (active && wave >= skip && label == o) tile_loss -= a[o];
+                    gs[(o * V + wave) * kWave + lane] = active && o < c_out ? (pr - (label == o ? 1.f : 0.f)) * inv_n : 0.f;
+                    ls[(o * V + wave) * kWave + lane] = a[o];
                 }
             }
+            group2d::lds_sync();
+#pragma unroll
+            for (int o = 0; o < MAXO; o++)
+#pragma unroll
+                for (int e = 0; e < V; e++) {
+                    g[o][e] = gs[(o * V + e) * kWave + lane];
+                    acc[o][e] = ls[(o * V + e) * kWave + lane];
+                }
+            // (tile_loss: each of the waves 0 .. V - 1 holds the terms of its element)
         } else {
+            // the eight partial outputs in a fixed order (a loop that stays a loop: unrolled, all
+            // 8 * MAXO * V values would be requested at once and held in registers)
+#pragma unroll
+            for (int o = 0; o < MAXO; o++)
+#pragma unroll
+                for (int e = 0; e < V; e++) acc[o][e] = red[(o * V + e) * kWave + lane];
+#pragma unroll 1
+            for (int q = 1; q < kTiledWaves; q++) {
+                const float *rq = red + (size_t)q * MAXO * V * kWave + lane;
+#pragma unroll
+                for (int o = 0; o < MAXO; o++)
+#pragma unroll
+                    for (int e = 0; e < V; e++) acc[o][e] += rq[(o * V + e) * kWave];
+            }
 #pragma unroll
             for (int o = 0; o < MAXO; o++) {
                 const bool keep = active && o < c_out;
-                float t[V];
-                load_global_vec_unaligned<V>(reinterpret_cast<uint64_t>(static_cast<const float *>(target) + (int64_t)b * tsb +
-                                                             (int64_t)min(o, c_out - 1) * tsc), xoff, t);
                 const float bv = bias && o < c_out ? bk[o] : 0.f;
 #pragma unroll
                 for (int e = 0; e < V; e++) {
                     acc[o][e] += bv;
-                    const float diff = acc[o][e] - t[e];
+                    const float diff = acc[o][e] - t[o][e];
                     if (KIND == 0) {
                         g[o][e] = keep ? 2.f * diff * inv_n : 0.f;
                         tile_loss += keep && e >= skip ? diff * diff : 0.f;
@@ -491,29 +555,6 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
                     }
                 }
             }
-        }
-        if constexpr (KIND == 2) {
-            // wave e wrote nothing of the other elements: log-probabilities and g through LDS
-            __syncthreads();                                  // all waves have read the partial outputs
-            float *gs = red, *ls = red + MAXO * V * kWave;    // [o][e][lane] each
-#pragma unroll
-            for (int e = 0; e < V; e++)
-                if (wave == e) {
-#pragma unroll
-                    for (int o = 0; o < MAXO; o++) {
-                        gs[(o * V + e) * kWave + lane] = g[o][e];
-                        ls[(o * V + e) * kWave + lane] = acc[o][e];
-                    }
-                }
-            __syncthreads();
-#pragma unroll
-            for (int o = 0; o < MAXO; o++)
-#pragma unroll
-                for (int e = 0; e < V; e++) {
-                    g[o][e] = gs[(o * V + e) * kWave + lane];
-                    acc[o][e] = ls[(o * V + e) * kWave + lane];
-                }
-            // (tile_loss: each of the waves 0 .. V - 1 holds the terms of its element)
         }
         if (wave == 0 || (KIND == 2 && wave < V)) lsum += tile_loss * inv_n;
         if (wave == 0) {                                      // uniform: one wave writes the outputs
@@ -540,12 +581,12 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
                 for (int e = 0; e < V; e++) sb[o] += g[o][e];
         }
         if (want_sums) {                                      // uniform
+            asm volatile("" : "+s"(count));
 #pragma unroll
             for (int cc = 0; cc < CC; cc++) {
-                const int c = cc * kTiledWaves + wave;
-                if (c < C) {
+                if (cc < count) {
                     float xv[V];
-                    load_elems<float, V>(lds_tile + (size_t)c * TV + lane * V, xv);   // what this wave stored itself
+                    load_elems<float, V>(own + cc * kTiledWaves * TV, xv);
 #pragma unroll
                     for (int o = 0; o < MAXO; o++)
 #pragma unroll
@@ -553,7 +594,7 @@ __global__ __launch_bounds__(kTiledThreads, 4) void final_forward_loss_tiled(
                 }
             }
         }
-        __syncthreads();                                      // `red` is rewritten by the next tile
+        group2d::lds_sync();                                  // `red` is rewritten by the next tile
     }
     const int64_t row = blockIdx.x;
     {
@@ -738,7 +779,12 @@ hipError_t allow_large_lds(const void *kernel, size_t bytes)
     return e;
 }
 
-constexpr size_t kTiledLdsLimit = 80 * 1024;     // two workgroups share the 160 KB of a CU
+// LDS of a tile, and of a workgroup: two share the 160 KB of a compute unit, or one has them.
+template <int V, int MAXO> constexpr size_t tiled_lds(int c_in)
+{
+    return ((size_t)c_in * kWave * V + (size_t)kTiledWaves * MAXO * V * kWave) * sizeof(float);
+}
+constexpr size_t kTiledLds = 160 * 1024;
 
 template <int V, int MAXO, int KIND, int CC>
 hipError_t launch_tiled(int64_t batch, int c_in, int c_out, int64_t nvox, const float *x, int64_t xsb, int64_t xsc,
@@ -749,13 +795,14 @@ hipError_t launch_tiled(int64_t batch, int c_in, int c_out, int64_t nvox, const 
     const int64_t tiles_per_image = ((nvox + V - 1) / V + kWave - 1) / kWave;
     const int64_t total = tiles_per_image * batch;
     if (total > INT32_MAX) return hipErrorInvalidConfiguration;
-    const size_t lds = ((size_t)c_in * kWave * V + (size_t)kTiledWaves * MAXO * V * kWave) * sizeof(float);
+    const size_t lds = tiled_lds<V, MAXO>(c_in);
     const void *fn = reinterpret_cast<const void *>(&final_forward_loss_tiled<V, MAXO, KIND, CC>);
     if (lds > 64 * 1024) {
-        const hipError_t e = allow_large_lds(fn, kTiledLdsLimit);
+        const hipError_t e = allow_large_lds(fn, kTiledLds);
         if (e != hipSuccess) return e;
     }
-    const int grid = (int)std::min<int64_t>(total, 512);      // two workgroups per CU, each walks its tiles
+    const int per_cu = lds * 2 <= kTiledLds ? tiled_workgroups<V, MAXO, KIND, CC>() : 1;
+    const int grid = (int)std::min<int64_t>(total, 256 * per_cu);                  // as many as are resident, each walks its tiles
     *rows = grid;
     hipLaunchKernelGGL((final_forward_loss_tiled<V, MAXO, KIND, CC>), dim3(grid), dim3(kTiledThreads), lds, s, nvox,
                        (int)tiles_per_image, (int)total, c_in, c_out, x, xsb, xsc, w, bias, target, tsb, tsc, out, osb,
@@ -763,8 +810,13 @@ hipError_t launch_tiled(int64_t batch, int c_in, int c_out, int64_t nvox, const 
     return hipGetLastError();
 }
 
-// The tiled kernel where it applies (fp32, up to 128 input and 4 output channels, a tile that
-// fits the LDS); *handled says whether it was launched.
+// Voxels from which 65 to 128 channels take four voxels per lane: tiles of 256 then are more than the 256 workgroups that are resident, of which
+// there are two per compute unit with two voxels and few outputs.  Two / four, us, 101 channels with one output, two, two labels, four labels:
+// 256 x 256 12.2 / 13.8, 17.6 / 18.2, 17.3 / 17.8, 25.4 / 26.4; 362 x 362 19.0 / 18.0, 24.1 / 22.6, 24.2 / 22.1, 35.0 / 31.0; 512 x 512
+// 25.7 / 25.2, 31.8 / 30.5, 30.8 / 30.0, 46.5 / 41.9.
+constexpr int64_t kTiledFourVoxels = 98304;
+
+// The tiled kernel where it applies (fp32, up to 256 input and 4 output channels, 512 and 2); *handled says whether it was launched.
 hipError_t final_forward_loss_tiled_try(int kind, int64_t batch, int c_in, int c_out, int64_t nvox, const float *x,
                                         int64_t xsb, int64_t xsc, const float *w, const float *bias,
                                         const void *target, int64_t tsb, int64_t tsc, float *out, int64_t osb,
@@ -774,36 +826,33 @@ hipError_t final_forward_loss_tiled_try(int kind, int64_t batch, int c_in, int c
     *handled = false;
     if (c_in > kTiledMaxChannels || c_out > 4 || !knob(kKnobFinalTiled, 1)) return hipSuccess;
     const int mo = c_out > 2 ? 4 : (c_out > 1 ? 2 : 1);
-    int v = 0;
-    for (int cand = 4; cand >= 2; cand /= 2) {
-        const size_t lds = ((size_t)c_in * kWave * cand + (size_t)kTiledWaves * mo * cand * kWave) * sizeof(float);
-        if (nvox >= cand && lds <= kTiledLdsLimit && (cand < 4 || c_in <= 64)) {
-            v = cand;
-            break;
-        }
-    }
-    if (v == 0) return hipSuccess;
-    const bool wide = c_in > 64;                              // sixteen channels per wave instead of eight
+    // channels per wave and voxels per lane: what LDS and registers hold
+    const int cc = c_in <= 64 ? 8 : c_in <= 128 ? 16 : c_in <= 256 ? 32 : 64;
+    const int v = cc == 64 ? 1 : cc == 32 || nvox < 4 || (cc == 16 && batch * nvox < kTiledFourVoxels) ? 2 : 4;
+    if (nvox < v || (cc == 64 && mo > 2)) return hipSuccess;
 #define MSD_TILED(VV, OO, KK, CCC)                                                                                    \
     return (*handled = true, launch_tiled<VV, OO, KK, CCC>(batch, c_in, c_out, nvox, x, xsb, xsc, w, bias, target, tsb, \
                                                           tsc, out, osb, osc, gout, gsb, gsc, inv_n, want, ws, rows, s))
-#define MSD_TILED_C(VV, OO, KK)                                  \
-    do {                                                         \
-        if (VV == 4 || !wide) MSD_TILED(VV, OO, KK, 8);          \
-        if constexpr (VV != 4) MSD_TILED(VV, OO, KK, 16);        \
+#define MSD_TILED_K(VV, OO, CCC)                                                                                      \
+    do {                                                                                                              \
+        if (kind == 0) MSD_TILED(VV, OO, 0, CCC); else if (kind == 1) MSD_TILED(VV, OO, 1, CCC);                      \
+        else MSD_TILED(VV, OO, 2, CCC);                                                                               \
     } while (0)
-#define MSD_TILED_K(VV, OO)                                                                     \
-    do {                                                                                        \
-        if (kind == 0) MSD_TILED_C(VV, OO, 0); else if (kind == 1) MSD_TILED_C(VV, OO, 1); else MSD_TILED_C(VV, OO, 2); \
+#define MSD_TILED_O(VV, CCC)                                                                                          \
+    do {                                                                                                              \
+        if (mo == 4) MSD_TILED_K(VV, 4, CCC); else if (mo == 2) MSD_TILED_K(VV, 2, CCC); else MSD_TILED_K(VV, 1, CCC); \
     } while (0)
-#define MSD_TILED_O(VV)                                                                         \
-    do {                                                                                        \
-        if (mo == 4) MSD_TILED_K(VV, 4); else if (mo == 2) MSD_TILED_K(VV, 2); else MSD_TILED_K(VV, 1); \
-    } while (0)
-    if (v == 4) MSD_TILED_O(4); else MSD_TILED_O(2);
+    if (cc == 64) {
+        if (mo == 2) MSD_TILED_K(1, 2, 64); else MSD_TILED_K(1, 1, 64);
+    } else if (cc == 32) {
+        MSD_TILED_O(2, 32);
+    } else if (cc == 16) {
+        if (v == 4) MSD_TILED_O(4, 16); else MSD_TILED_O(2, 16);
+    } else {
+        if (v == 4) MSD_TILED_O(4, 8); else MSD_TILED_O(2, 8);
+    }
 #undef MSD_TILED_O
 #undef MSD_TILED_K
-#undef MSD_TILED_C
 #undef MSD_TILED
     return hipSuccess;
 }

@@ -90,6 +90,19 @@ def test_fused_loss_of_odd_planes(spatial, c_in, c_out, kind):
     check_fused_loss(3, c_in, c_out, spatial, kind, torch.float32)
 
 
+# The single-read kernel's channels per wave (8, 16, 32, 64) at both ends of their ranges, with waves that have one channel less or none, and
+# above them the kernel that walks twice; planes of less than a tile, ragged, and of several tiles per workgroup in each form.  (Nine
+# voxels at least: the loss of a single one may be all but zero, while pre-activations of up to 0.3 sqrt(257) 3 = 14 are rounded to 2^-24 of
+# that, 8e-7, which is 1e-5 of a loss below 0.08.)
+@pytest.mark.parametrize("kind", ["mse", "l1", "nll"])
+@pytest.mark.parametrize("c_out", [1, 2, 4])
+@pytest.mark.parametrize("batch,c_in,spatial", [
+    (1, 3, (300, 301)), (1, 64, (5, 67)), (1, 65, (320, 331)), (1, 128, (320, 331)), (2, 128, (9, 13)), (9, 129, (1, 1)), (2, 129, (3, 43)),
+    (1, 201, (190, 201)), (3, 256, (7, 19)), (9, 257, (1, 1)), (2, 257, (5, 13)), (1, 402, (150, 151)), (3, 512, (11, 12)), (1, 513, (9, 15))], ids=str)
+def test_fused_loss_at_the_ends_of_the_forms(batch, c_in, spatial, c_out, kind):
+    check_fused_loss(batch, c_in, c_out, spatial, kind, torch.float32)
+
+
 # grad_input alone: planes of every remainder modulo four, of fewer voxels than four, of more than a workgroup covers, one to
 # nine outputs (more than eight go in passes); an infinite weight meets its own output only.
 @pytest.mark.parametrize("c_out", [1, 2, 3, 4, 5, 8, 9])
