@@ -211,28 +211,30 @@ __global__ __launch_bounds__(kMaxWaves *kWave) void push_rows(PushArgs a, const 
 // ---- More than seven outputs: two slabs of columns, fp32 values in bf16 parts (msd_split.h).
 //
 // A wave walks a row, or a part of one, in segments of 64 voxels and forms the columns of one slab; no
-// wave waits for another.  x arrives by channel in 256-byte pieces, is split and goes through the wave's
-// own part of LDS: the matrix cores take 16 voxels x 32 channels at once, read transposed
-// (ds_read_b64_tr_b16).  The shifts along x are taken as in push_rows, tile by tile of the columns, through the same
-// space; what a segment's outputs need of the segment before stays in registers, so that nothing is formed
-// twice.  Every channel is read once for up to fourteen outputs.
+// wave waits for another.  x arrives by channel in 256-byte pieces, four voxels of eight channels per lane: split, they are operands of the
+// matrix cores as they stand (voxel 4 n + j is row n of product j).  The shifts along x are taken as in push_rows, tile by tile of the
+// columns, through the wave's own part of LDS; what a segment's outputs need of the segment before stays in registers, so that nothing is formed
+// twice.  Every channel leaves memory once for up to fourteen outputs: the workgroups of the two slabs are neighbours on one XCD and
+// work on the same rows at the same time.
 //
-// Bound by latencies: eight waves per compute unit (their registers), each a chain of loads, split, LDS and matrix
-// instructions; the matrix part is a quarter of the time.  14 outputs at 2048 x 2048 over 20 / 45 / 90 / 120 channels: 512, 696,
-// 958, 1223 us, where two passes of push_rows take 485, 803, 1335 and 1526.  At 1024 x 1024 over 50: 206 (matrix
-// instructions cut to a sixth 200, x from the caches 163, without the shifts 112).  With a workgroup per row, its waves
-// side by side and barriers around each tile of the shifts: 194 there, but 2.3 ms at 2048 x 2048 over 120.
+// A workgroup has one slab, so that the weights of 256 channels lie in LDS at a time: with both slabs in one it were 128, and to load them
+// anew for every segment took 260 of the 1400 us over 131 channels.  Without them x is read through the L2 twice, which costs nothing
+// measurable.  2048 x 2048, 14 outputs, us, both slabs in a workgroup / one: over 16 / 58 / 100 / 128 channels 559 / 553, 743 / 730, 918 / 890, 939 / 904, over
+// 142 / 184 1390 / 1064, 1579 / 1247.  (x by way of a transposition in LDS instead of in the operands' own layout: the same times.)
+//
+// Bound by latencies: eight waves per compute unit (their registers), each a chain of loads, split and matrix
+// instructions; the matrix part is a quarter of the time.  With a workgroup per row, its waves
+// side by side and barriers around each tile of the shifts: 2.3 ms at 2048 x 2048 over 120.
 constexpr int kSlabs = 2;
 constexpr int kPushWaves = 8;                     // of a workgroup; one workgroup per compute unit
-constexpr int kPushTeams = kPushWaves / kSlabs;   // rows that a workgroup works on
 constexpr int kHalo = 16;                         // dilations up to here
 constexpr int kStepChannels = 32;
 constexpr int kTileBytes = 3 * kWave * 16;        // weights of 16 columns, a step
-constexpr int kTableSteps = 4;                    // steps whose weights are in LDS at a time
-constexpr int kTableBytes = kTableSteps * kSlabs * kTiles * kTileBytes;
+constexpr int kTableSteps = 8;                    // steps whose weights (of a slab) are in LDS at a time
+constexpr int kTableBytes = kTableSteps * kTiles * kTileBytes;
 constexpr int kLine = 2 * kHalo + kWave + 4;      // floats of a staged row (16 bytes apart in the banks)
-constexpr int kOwnBytes = kStaged * kLine * 4 + 16;                 // of a wave: staged rows, or 16 channels of x in parts
-static_assert(kOwnBytes >= 3 * 16 * 2 * kWave && kOwnBytes % 16 == 0, "x lies over the staged rows");
+constexpr int kOwnBytes = kStaged * kLine * 4 + 16;                 // of a wave: staged rows
+static_assert(kOwnBytes % 16 == 0, "16-byte accesses");
 constexpr int kSplitLds = kTableBytes + kPushWaves * kOwnBytes;
 
 struct SplitArgs {
@@ -241,9 +243,8 @@ struct SplitArgs {
     Outputs out;
 };
 
-// Channel (of the step's 32) that value e of the lanes q stands for: the first half of a step's channels
-// is split, put and read before the second.
-__host__ __device__ __forceinline__ int channel_of(int q, int e) { return e < 4 ? 4 * q + e : 16 + 4 * q + e - 4; }
+// Channel (of the step's 32) that value e of the lanes q stands for.
+__host__ __device__ __forceinline__ int channel_of(int q, int e) { return 4 * e + q; }
 
 // [step][tile of columns][part][lane (column n, q)]: eight channels each; bad[step]: some of them have to be taken whole,
 // and all of the step's lie so.
@@ -271,17 +272,15 @@ __global__ __launch_bounds__(kSlabs *kTiles *kWave) void push_table(const SplitA
     for (int p = 0; p < 3; p++) table[((step * kSlabs * kTiles + t) * 3 + p) * kWave + lane] = s.p[p];
 }
 
-// A row of 16 bytes pieces lies at piece ^ turn(row): what is read transposed meets all banks once.
-__device__ __forceinline__ uint32_t turn(uint32_t row) { return row / 2 % 4 * 2 + row / 8 % 2; }
-
 __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitArgs a, const float *__restrict__ x,
                                                                   const bf16x8_t *__restrict__ table, const int *__restrict__ bad,
                                                                   float *__restrict__ z)
 {
-    constexpr int kStepEntries = kSlabs * kTiles * 3 * kWave;
+    constexpr int kStepEntries = kTiles * 3 * kWave;
     extern __shared__ __attribute__((aligned(16))) char split_lds[];
     const int tid = threadIdx.x, lane = tid % kWave;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), slab = wave % kSlabs, team = wave / kSlabs;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave), slab = blockIdx.x / kXcds % kSlabs;
+    const int pair = blockIdx.x / (kSlabs * kXcds) * kXcds + blockIdx.x % kXcds, pairs = gridDim.x / kSlabs;      // of workgroups, on one XCD
     bf16x8_t *const weights = reinterpret_cast<bf16x8_t *>(split_lds);
     char *const own = split_lds + kTableBytes + wave * kOwnBytes;
     const int steps = (a.C + kStepChannels - 1) / kStepChannels;
@@ -315,13 +314,13 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
         p.end = min(p.to + kHalo, a.W);
         return p;
     };
-    // Loads: lane (channel q of four, voxels 4 n ..) of 64 voxels; past the row end its last four voxels, past
-    // the last channel that one again (its weights are zero).
+    // Loads: lane (channel q of four, voxels 4 n ..) of 64 voxels, which is what the matrix cores take: voxel 4 n + j is row n of product j.
+    // Past the row end its last four voxels, past the last channel that one again (its weights are zero).
     f32x4_t xv[8];
-    auto request = [&](const Item &p, int first, int step) {
+    auto image_of = [&](const Item &p) { return reinterpret_cast<uint64_t>(x) + (uint64_t)(((int64_t)p.b * a.xsb + (int64_t)p.y * a.xsy) * 4); };
+    auto request = [&](uint64_t image, int first, int step) {
         const Lane l = fresh();
         const uint32_t at = 4u * (uint32_t)min(first + 4 * (int)l.n, a.W - 4), lane_plane = l.q * plane;
-        const uint64_t image = reinterpret_cast<uint64_t>(x) + (uint64_t)(((int64_t)p.b * a.xsb + (int64_t)p.y * a.xsy) * 4);
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const int c = min(step * kStepChannels + 4 * i, a.C - 1);              // uniform
@@ -333,19 +332,24 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
         }
     };
     const bool resident = steps <= kTableSteps;   // the weights are in LDS once and for all
+    auto load_weights = [&](int step, int count) {
+#pragma unroll 2
+        for (int i = wave * kWave + (int)fresh().id; i < count * kStepEntries; i += kPushWaves * kWave)
+            weights[i] = table[((step + i / kStepEntries) * kSlabs + slab) * kStepEntries + i % kStepEntries];
+    };
     if (resident) {
-        for (int i = tid; i < steps * kStepEntries; i += kPushWaves * kWave) weights[i] = table[i];
+        load_weights(0, steps);
         __syncthreads();
     }
     // (workgroups whose table does not hold all weights meet at each part of it: all their waves take as many segments)
     const int most = (a.length + 2 * kHalo + kWave - 1) / kWave;
-    const int stride = gridDim.x * kPushTeams;
-    int it = blockIdx.x * kPushTeams + team;
+    const int stride = pairs * kPushWaves;
+    int it = pair * kPushWaves + wave;
     Item here = locate(it);
-    request(here, here.start, 0);
-    for (int it0 = blockIdx.x * kPushTeams; it0 < a.items; it0 += stride, it += stride) {
+    request(image_of(here), here.start, 0);
+    for (int it0 = pair * kPushWaves; it0 < a.items; it0 += stride, it += stride) {
         const Item next = locate(it + stride);
-        f32x4_t before[2][kTiles];                // the last 32 voxels of the segment before
+        f32x4_t before[2][kTiles];                // the last 32 voxels of the segment before: of lanes 32 + i, products 0 and 1 in lane i, 2 and 3 in theirs
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
@@ -363,8 +367,7 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
             for (int step = 0; step < steps; step++) {
                 if (!resident && step % kTableSteps == 0) {                        // uniform over the workgroup
                     lds_sync();
-                    const int count = min(kTableSteps, steps - step) * kStepEntries;
-                    for (int i = tid; i < count; i += kPushWaves * kWave) weights[i] = table[step * kStepEntries + i];
+                    load_weights(step, min(kTableSteps, steps - step));
                     lds_sync();
                 }
                 const auto [id, n, q] = fresh();
@@ -379,54 +382,24 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
                         xv[i][2] = over == 1 ? v[3] : v[2];
                     }
                 }
-                bf16x8_t xa[4][3];                // [16 voxels][part]: voxel n, channels channel_of(q, ..)
-                const uint32_t tr_row = 4 * q + n / 4;
-                const char *const tr = own + tr_row * (2 * kWave) + n % 2 * 8;
-                const uint32_t tr_piece = 16 * (n % 4 / 2 ^ turn(tr_row));
-                typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-                bf16x4_t low[4][3];
+                bf16x8_t xa[4][3];                // [voxels 4 n + j][part]: channels channel_of(q, ..)
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    own_sync();                   // (what was there has been read)
+                for (int j = 0; j < 4; j++) {
+                    // -x at every second voxel: the sums of the bf16 instruction are cut off towards minus infinity
+                    float v[8];
 #pragma unroll
-                    for (int i = 4 * h; i < 4 * h + 4; i += 2) {
-                        // -x at every second voxel: the sums of the bf16 instruction are cut off towards minus infinity
-                        float v[8];
+                    for (int e = 0; e < 8; e++) v[e] = xv[e][j] * (j % 2 ? -kSplitScale : kSplitScale);
+                    Split8 s;
+                    rest += split8(v, s);
 #pragma unroll
-                        for (int e = 0; e < 8; e++) v[e] = xv[i + e / 4][e % 4] * (e % 2 ? -kSplitScale : kSplitScale);
-                        Split8 s;
-                        rest += split8(v, s);
-#pragma unroll
-                        for (int k = 0; k < 2; k++) {
-                            const uint32_t channel = q + 4 * (uint32_t)(i % 4 + k);
-                            char *const at = own + channel * (2 * kWave) + 16 * (n / 2 ^ turn(channel)) + n % 2 * 8;
-#pragma unroll
-                            for (int p = 0; p < 3; p++)
-                                *reinterpret_cast<bf16x4_t *>(at + p * (16 * 2 * kWave)) =
-                                    k ? __builtin_shufflevector(s.p[p], s.p[p], 4, 5, 6, 7) : __builtin_shufflevector(s.p[p], s.p[p], 0, 1, 2, 3);
-                        }
-                    }
-                    own_sync();
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-#pragma unroll
-                        for (int p = 0; p < 3; p++) {
-                            typedef short s16x4_t __attribute__((ext_vector_type(4)));
-                            typedef __attribute__((address_space(3))) s16x4_t *lds_tr_t;
-                            const bf16x4_t r = __builtin_bit_cast(
-                                bf16x4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                              (lds_tr_t)(tr + p * (16 * 2 * kWave) + (tr_piece ^ (uint32_t)(32 * j)))));
-                            if (h == 0) low[j][p] = r;
-                            else xa[j][p] = __builtin_shufflevector(low[j][p], r, 0, 1, 2, 3, 4, 5, 6, 7);
-                        }
+                    for (int p = 0; p < 3; p++) xa[j][p] = s.p[p];
                 }
                 __builtin_amdgcn_sched_barrier(0);    // (the scheduler would move the loads to where they are used)
-                if (step + 1 < steps) request(here, first, step + 1);
-                else if (seg + 1 < segs) request(here, first + kWave, 0);
-                else request(next, next.start, 0);
+                const bool more = step + 1 < steps, row = more || seg + 1 < segs;
+                request(image_of(row ? here : next), more ? first : row ? first + kWave : next.start, more ? step + 1 : 0);
                 __builtin_amdgcn_sched_barrier(0);
                 if (real) {
-                    const bf16x8_t *const wt = weights + ((resident ? step : step % kTableSteps) * kSlabs + slab) * (kTiles * 3 * kWave) + id;
+                    const bf16x8_t *const wt = weights + (resident ? step : step % kTableSteps) * kStepEntries + id;
                     bf16x8_t w[2][3];
 #pragma unroll
                     for (int p = 0; p < 3; p++) w[0][p] = wt[p * kWave];
@@ -443,7 +416,7 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
                             for (int j = 0; j < 4; j++)
                                 one[j] = mfma_split(xa[j], w[t % 2], k == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : one[j], k);
 #pragma unroll
-                        for (int j = 0; j < 4; j++) acc[j][t] += kSplitUnit * one[j];
+                        for (int j = 0; j < 4; j++) acc[j][t] += (j % 2 ? -kSplitUnit : kSplitUnit) * one[j];
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
@@ -451,34 +424,25 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
             if (!real) continue;
             if (!weights_split || __any(taken_whole(rest))) {                      // uniform
                 // values to be taken whole: all of the segment's sums again, with the fp32 instruction
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-#pragma unroll
-                    for (int t = 0; t < kTiles; t++) acc[j][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
                 const float *const image = x + (int64_t)here.b * a.xsb + (int64_t)here.y * a.xsy;
-                const auto [id, n, q] = fresh();
+#pragma unroll
+                for (int t = 0; t < kTiles; t++) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) acc[j][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-                for (int c0 = 0; c0 < a.C; c0 += 4) {
-                    const int c = c0 + (int)q;
-                    const bool whole = bad[c0 / kStepChannels] != 0;               // uniform
-                    const int r = c % kStepChannels, at = (int)n + r % 16 / 4 * 16, e = r % 4 + r / 16 * 4;
-                    float xj[4], wj[kTiles];
+                    for (int c0 = 0; c0 < a.C; c0 += 4) {
+                        const auto [id, n, q] = fresh();
+                        const int c = c0 + (int)q, cc = min(c, a.C - 1), s = c0 / kStepChannels;   // (channel_of: step s, lanes q, value e)
+                        const __bf16 *const k = reinterpret_cast<const __bf16 *>(table + ((int64_t)(s * kSlabs + slab) * kTiles + t) * (3 * kWave) + id) +
+                                                c0 % kStepChannels / 4;
+                        const float w = bad[s] != 0 ? whole_value(k[0], k[8 * kWave])              // uniform
+                                                    : ((float)k[0] + (float)k[8 * kWave] + (float)k[16 * kWave]) * (1.f / kSplitScale);
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const float v = image[(int64_t)min(c, a.C - 1) * a.xsc + min(first + 16 * j + (int)n, a.W - 1)];
-                        xj[j] = c < a.C ? (n % 2 ? -v : v) : 0.f;
+                        for (int j = 0; j < 4; j++) {
+                            const float v = image[(int64_t)cc * a.xsc + min(first + 4 * (int)n + j, a.W - 1)];
+                            acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(c < a.C ? v : 0.f, c < a.C ? w : 0.f, acc[j][t], 0, 0, 0);
+                        }
                     }
-#pragma unroll
-                    for (int t = 0; t < kTiles; t++) {
-                        const __bf16 *const k = reinterpret_cast<const __bf16 *>(
-                            table + ((int64_t)(min(c, a.C - 1) / kStepChannels * kSlabs + slab) * kTiles + t) * (3 * kWave) + at) + e;
-                        const float sum = (float)k[0] + (float)k[8 * kWave] + (float)k[16 * kWave];
-                        wj[t] = c < a.C ? (whole ? whole_value(k[0], k[8 * kWave]) : sum * (1.f / kSplitScale)) : 0.f;
-                    }
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-#pragma unroll
-                        for (int t = 0; t < kTiles; t++) acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xj[j], wj[t], acc[j][t], 0, 0, 0);
                 }
             }
 
@@ -494,13 +458,15 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
 #pragma unroll
             for (int t = 0; t < kTiles; t++) {
                 if (kTriples * t >= triples_in) break;                             // uniform
-                float *const put = T + n * kLine + 4 * q + (n == 15 ? t * kLine : 0);                // (the last columns keep rows of their own)
-                auto stage = [&](int at, const f32x4_t &v) { *reinterpret_cast<f32x4_t *>(put + at) = f32x4_t{v[0], -v[1], v[2], -v[3]}; };
-                own_sync();                           // (x, or the tile before, has been read)
+                // acc[j][t][r] = Y[16 q + 4 r + j][16 t + n]
+                float *const put = T + n * kLine + (n == 15 ? t * kLine : 0);                        // (the last columns keep rows of their own)
+                own_sync();                           // (the tile before has been read)
 #pragma unroll
-                for (int j = 0; j < 2; j++) stage(16 * j, before[j][t]);
-#pragma unroll
-                for (int j = 0; j < 4; j++) stage(2 * kHalo + 16 * j, acc[j][t]);
+                for (int r = 0; r < 4; r++) {
+                    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+                    *reinterpret_cast<f32x2_t *>(put + 16 * (q % 2) + 4 * r + 2 * (q / 2)) = f32x2_t{before[0][t][r], before[1][t][r]};
+                    *reinterpret_cast<f32x4_t *>(put + 2 * kHalo + 16 * q + 4 * r) = f32x4_t{acc[0][t][r], acc[1][t][r], acc[2][t][r], acc[3][t][r]};
+                }
                 own_sync();
                 constexpr int kMost = kTriples + 1;
                 const int triples = t == kTiles - 1 ? kMost : kTriples;
@@ -538,7 +504,11 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
 #pragma unroll
             for (int j = 0; j < 2; j++)
 #pragma unroll
-                for (int t = 0; t < kTiles; t++) before[j][t] = acc[2 + j][t];
+                for (int t = 0; t < kTiles; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        before[j][t][r] = __uint_as_float(
+                            __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[j][t][r]), __float_as_uint(acc[j + 2][t][r]), false, false)[1]);
         }
         here = next;
     }
@@ -734,7 +704,7 @@ hipError_t group_push_split_2d(const Geom &g, const View<const float> &x, const 
     const int steps = (g.C + kStepChannels - 1) / kStepChannels;
     SplitArgs a{g.C, g.H, g.W, 0, 1, 0, x.sb, x.sc, x.sy, out};
     // Parts of a row: the waves that are resident take as few segments one after the other as can be.
-    const int64_t rows = (int64_t)g.B * g.H, slots = 256 * kPushTeams;
+    const int64_t rows = (int64_t)g.B * g.H, slots = 256 / kSlabs * kPushWaves;
     int64_t best = INT64_MAX;
     for (int parts = 1; parts <= 32; parts++) {
         const int length = ((g.W + parts - 1) / parts + 3) & ~3;
@@ -747,7 +717,7 @@ hipError_t group_push_split_2d(const Geom &g, const View<const float> &x, const 
         }
     }
     a.items = (int)(rows * a.parts);
-    const int blocks = (int)std::min<int64_t>(256, (a.items + kPushTeams - 1) / kPushTeams);
+    const int blocks = kSlabs * (int)std::min<int64_t>(256 / kSlabs, xcd_grid((a.items + kPushWaves - 1) / kPushWaves));
     bf16x8_t *const weights = reinterpret_cast<bf16x8_t *>(table);
     int *const bad = reinterpret_cast<int *>(table + (int64_t)steps * (kSlabs * kTiles * kTileBytes / 4));
     hipLaunchKernelGGL(push_table, dim3(steps), dim3(kSlabs * kTiles * kWave), 0, s, a, weights, bad);

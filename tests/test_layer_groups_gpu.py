@@ -321,6 +321,23 @@ def test_block_in_forward_groups_of_up_to_fourteen(case):
         check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=61)
 
 
+# As many channels as the table of weights holds at once, one step more and three parts of it; fewer rows than the workgroups of one XCD have
+# waves, one row, more rows than there are waves; rows in parts, of several segments, a last one of less than four voxels.
+@pytest.mark.parametrize("case", [
+    ((16, 70), 255, 1, 9, 1, [3, 16]),
+    ((17, 131), 257, 1, 14, 1, [1, 16, 7]),
+    ((1, 33), 300, 1, 10, 1, [1, 1]),
+    ((9, 1022), 520, 1, 8, 1, [9, 4]),
+    ((1030, 34), 260, 2, 5, 1, [2, 11]),
+    ((66, 67), 12, 2, 7, 2, [5, 16, 1]),
+], ids=lambda c: "x".join(map(str, c[0])) + "-c%d-w%d-d%d-B%d" % c[1:5])
+def test_forward_groups_of_fourteen_over_many_channels(case):
+    size, c_in, width, depth, batch, dilations = case
+    dilations = [dilations[i % len(dilations)] for i in range(depth)]
+    with tuning({"fwd.group": 1024}):
+        check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=67)
+
+
 @pytest.mark.parametrize("where", ["input", "weight"])
 @pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
 def test_values_without_bf16_parts_in_front_of_a_forward_group(where, value):
