@@ -1499,10 +1499,14 @@ constexpr int64_t kGroupChannels = 12, kGroupChannelsWide = 6;
 // Up to fourteen outputs instead of seven where the channels in front are at least this many voxels in all.  The pass
 // then moves them once and not twice (two channels per layer: 2.3 times, since sevens take six outputs), but the
 // upper layers of the group find up to 13 channels to add, and passes of seven have twice the waves.  Push and finish of
-// 14 outputs, us, sevens and fourteens: two channels per layer 1024 x 1024 over 60: 323, 339; over 180: 707, 613;
+// 14 outputs, us, sevens and fourteens (over 180 before a pass had the weights of 256 channels in LDS, now some 60 less): two channels per layer 1024 x 1024 over 60: 323, 339; over 180: 707, 613;
 // 2048 x 2048 over 24: 967, 959; over 60: 1426, 1185; over 120: 2180, 1663; one channel 1536 x 1536 over 80: 928, 913;
 // 2048 x 2048 over 45: 1127, 1253; over 90: 1657, 1507.
+// From 64 channels on two channels per layer gain from half as many voxels on.  Forward pass of a whole block of two channels per layer, ms, line at 2^27
+// / 2^26 from 64 channels on / 2^26 throughout: depth 100, 1024 x 1024 4.97 / 4.81 / 4.75, 1000 x 1001 5.10 / 4.85 / 4.87; depth 60, 4 x 512 x 512
+// 2.39 / 2.28 / 2.27, 1448 x 1448 4.72 / 4.68 / 4.79.
 constexpr int64_t kFourteenVoxels = (int64_t)1 << 28, kFourteenVoxelsWide = (int64_t)1 << 27;
+constexpr int64_t kFourteenManyWide = 64;
 
 // Number of layers from layer i on that form a group of the forward pass (0: none), of at most `most` outputs.
 // Knob: 0 < n < kFourteenKnob from n channels on, in sevens; from kFourteenKnob on: from n - kFourteenKnob channels on, in fourteens.
@@ -1522,7 +1526,8 @@ int forward_group(const BlockArgs &a, int i, int64_t first, int most)
         outputs += a.widths[i + n++];
     }
     if (outputs > msd::group2d::kSlabOut) {
-        const bool large = a.batch * a.spatial[0] * a.spatial[1] >= ((wide ? kFourteenVoxelsWide : kFourteenVoxels) + first - 1) / first;
+        const int64_t least = !wide ? kFourteenVoxels : first < kFourteenManyWide ? kFourteenVoxelsWide : kFourteenVoxelsWide / 2;
+        const bool large = a.batch * a.spatial[0] * a.spatial[1] >= (least + first - 1) / first;
         if (!(set < 0 ? large : force) || !msd::group_split_supported_2d(a.spatial[1], (int)dmax)) return 0;
     }
     return n >= 2 ? n : 0;
