@@ -220,7 +220,8 @@ __global__ __launch_bounds__(kMaxWaves *kWave) void push_rows(PushArgs a, const 
 // A workgroup has one slab, so that the weights of 256 channels lie in LDS at a time: with both slabs in one it were 128, and to load them
 // anew for every segment took 260 of the 1400 us over 131 channels.  Without them x is read through the L2 twice, which costs nothing
 // measurable.  2048 x 2048, 14 outputs, us, both slabs in a workgroup / one: over 16 / 58 / 100 / 128 channels 559 / 553, 743 / 730, 918 / 890, 939 / 904, over
-// 142 / 184 1390 / 1064, 1579 / 1247.  (x by way of a transposition in LDS instead of in the operands' own layout: the same times.)
+// 142 / 184 1390 / 1064, 1579 / 1247.  Above 256 the steps of one segment go up and the next one's down, so that a part of the table is
+// loaded once less per segment: over 268 / 324 / 380 2025 / 1914, 2250 / 2068, 2719 / 2449.  (x by way of a transposition in LDS instead of in the operands' own layout: the same times.)
 //
 // Bound by latencies: eight waves per compute unit (their registers), each a chain of loads, split and matrix
 // instructions; the matrix part is a quarter of the time.  With a workgroup per row, its waves
@@ -343,6 +344,9 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
     }
     // (workgroups whose table does not hold all weights meet at each part of it: all their waves take as many segments)
     const int most = (a.length + 2 * kHalo + kWave - 1) / kWave;
+    // (else one segment's steps go up, the next one's down: the part of the table that the one ends with is the other's first)
+    bool up = true;
+    int loaded = -1;
     const int stride = pairs * kPushWaves;
     int it = pair * kPushWaves + wave;
     Item here = locate(it);
@@ -364,10 +368,12 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
 #pragma unroll
                 for (int t = 0; t < kTiles; t++) acc[j][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
             float rest = 0.f;
-            for (int step = 0; step < steps; step++) {
-                if (!resident && step % kTableSteps == 0) {                        // uniform over the workgroup
+            for (int i = 0; i < steps; i++) {
+                const int step = up ? i : steps - 1 - i;
+                if (!resident && step / kTableSteps != loaded) {                   // uniform over the workgroup
+                    loaded = step / kTableSteps;
                     lds_sync();
-                    load_weights(step, min(kTableSteps, steps - step));
+                    load_weights(loaded * kTableSteps, min(kTableSteps, steps - loaded * kTableSteps));
                     lds_sync();
                 }
                 const auto [id, n, q] = fresh();
@@ -395,8 +401,8 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
                     for (int p = 0; p < 3; p++) xa[j][p] = s.p[p];
                 }
                 __builtin_amdgcn_sched_barrier(0);    // (the scheduler would move the loads to where they are used)
-                const bool more = step + 1 < steps, row = more || seg + 1 < segs;
-                request(image_of(row ? here : next), more ? first : row ? first + kWave : next.start, more ? step + 1 : 0);
+                const bool more = i + 1 < steps, row = more || seg + 1 < segs;
+                request(image_of(row ? here : next), more ? first : row ? first + kWave : next.start, more ? (up ? step + 1 : step - 1) : resident ? 0 : step);
                 __builtin_amdgcn_sched_barrier(0);
                 if (real) {
                     const bf16x8_t *const wt = weights + (resident ? step : step % kTableSteps) * kStepEntries + id;
@@ -421,6 +427,7 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
                     }
                 }
             }
+            up = resident || !up;
             if (!real) continue;
             if (!weights_split || __any(taken_whole(rest))) {                      // uniform
                 // values to be taken whole: all of the segment's sums again, with the fp32 instruction
