@@ -10,8 +10,8 @@
 // address), split it and leave it in LDS as [part][voxel][m]: the grad_input product reads it as it lies (lane = voxel, eight
 // rows m), the grad_kernel product through the transposing LDS read (ds_read_b64_tr_b16).  At the same time four waves take the
 // tile before, which lies in a second buffer, through the one and four through the other product, a block of 16 channels at 32 voxels at a time; a
-// barrier per tile, and the buffers change.  Weights and sums stay in registers over all tiles, the sums leave as one row of
-// partial sums per workgroup.  x and grad_input go through a transposition in the wave's own part of LDS:
+// barrier per tile, and the buffers change.  Weights and sums stay in registers over the tiles, the sums go to a second level in LDS
+// every 16 additions, and leave as one row of partial sums per workgroup, which sum_group adds in double precision.  x and grad_input go through a transposition in the wave's own part of LDS:
 // in the layout of the matrix cores a load touches 64 bytes of each of 16 channels, which memory
 // serves at 2.6-3.0 TB/s whatever else happens, whole lines at 4.0 (probed with loads and
 // stores alone, 64 channels of 1024 x 1024).  Five to eight blocks of two slabs: msd_pull_wide.h.
@@ -191,7 +191,9 @@ template <int G, int P> struct PullShape {
     static constexpr int kUnits = kSegs / P;             // segments that a worker takes one after the other
     static constexpr int kTileBytes = kSegs * G * kSlabBytes;
     static constexpr int kXBytes = 16 * 3 * kXRow, kDBytes = 16 * kDRow;           // of a kernel, an input worker's own
-    static constexpr int kLds = 2 * kTileBytes + kOfKind * (kXBytes + kDBytes);
+    static constexpr int kSumBytes = kTiles * kWave * 16;           // of a kernel worker's sums
+    static constexpr int kSumsAt = 2 * kTileBytes + kOfKind * (kXBytes + kDBytes);
+    static constexpr int kLds = kSumsAt + kOfKind * kSumBytes;
 };
 
 // What a wave keeps for its life: an input worker the weights of rows 32 step + 8 q .. of channel n in parts, a kernel worker its sums
@@ -201,7 +203,7 @@ template <int G> struct PullState {
     f32x4_t kept[2 * G * 3];
     bool weights_split;
     __device__ f32x4_t &sums(int tile) { return kept[tile]; }
-    __device__ f32x4_t &bias() { return kept[0]; }
+    __device__ f32x4_t &bias(int level) { return kept[level]; }
     __device__ bf16x8_t weights(int step, int part) const { return __builtin_bit_cast(bf16x8_t, kept[step * 3 + part]); }
     __device__ void set_weights(int step, int part, bf16x8_t w) { kept[step * 3 + part] = __builtin_bit_cast(f32x4_t, w); }
 };
@@ -225,6 +227,20 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
     };
     char *const own_x = lds + 2 * S::kTileBytes + number * S::kXBytes;             // a kernel worker's own
     char *const own_d = lds + 2 * S::kTileBytes + kOfKind * S::kXBytes + number * S::kDBytes;      // an input worker's
+    // Sums are added to a second level every so many tiles: a chain of n additions of terms of mixed sign rounds to about sqrt(n / 2)
+    // 2^-24 of what it comes to.  Errors of the weight gradients against 64 bits (2-norm), a chain over all tiles / in two levels: 192^3,
+    // four outputs over 30 / 46 channels 6.7 / 2.1, 6.8 / 2.0 e-7; 2048 x 2048, 14 outputs over 40 4.3 / 1.4; 1024 x 1024 2.2 / 1.1; 333 x 477
+    // 0.96 / 0.71.  Times are the same within 2 % (the branch in the loop over the tiles instead of around it: up to 6 % more).
+    constexpr int kChain = 16;                    // additions
+    const int chain = wgs * (kChain / kUnits), bias_chain = wgs * kChain * (N != kImage ? 4 : 1);      // tiles, of all workgroups
+    auto second_level = [&]() {                   // of a kernel worker
+        char *const at = lds + S::kSumsAt + number * S::kSumBytes + lane * 16;
+#pragma unroll
+        for (int t = 0; t < kTiles; t++) {
+            *reinterpret_cast<f32x4_t *>(at + t * kWave * 16) += state.sums(t);
+            state.sums(t) = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    };
 
     struct Tile {
         int first;                                // segment of its image
@@ -413,8 +429,9 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         }
         if constexpr (!WHOLE) {                       // (the second run's have been counted)
             // (volumes: one value per lane, four chains of a quarter of the tiles)
-            if constexpr (N != kImage) state.bias() = f32x4_t{state.bias()[1], state.bias()[2], state.bias()[3], state.bias()[0] + val[0][4 * (kLines / 9)][1]};
-            else state.bias() += f32x4_t{val[0][1][1], val[1][1][1], val[2][1][1], val[3][1][1]};
+            f32x4_t &bias = state.bias(0);
+            if constexpr (N != kImage) bias = f32x4_t{bias[1], bias[2], bias[3], bias[0] + val[0][4 * (kLines / 9)][1]};
+            else bias += f32x4_t{val[0][1][1], val[1][1][1], val[2][1][1], val[3][1][1]};
         }
         // -A at every second voxel: the sums of the bf16 instruction are cut off towards minus infinity, which adds up
         // over an image where the gradients themselves cancel (bias gradients: an error of 2e-6 instead of 1.2e-7).
@@ -739,8 +756,9 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
     const bool kernel = cb < blocks && kind == kKernel, input = cb < blocks && ch0 < update_end && kind == kInput;     // uniform
     if constexpr (WHOLE) {
 #pragma unroll 1
-        for (int tile = lb; tile < a.tiles; tile += wgs) {
+        for (int tile = lb, count = 0; tile < a.tiles; tile += wgs, count += kUnits) {
             const Tile t = tile_of(tile);
+            if (kernel && count % kChain == 0) second_level();      // uniform
             if (kind == kGatherer) {
                 const Voxel here = locate_pair(t);
                 gather(t, here);
@@ -770,15 +788,19 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         // A tile is formed in the one buffer while the workers have the other; a barrier, and they change.
         Voxel here = locate_pair(tile_of(lb));
         gather(tile_of(lb), here);
-        for (int tile = lb; tile < a.tiles; tile += wgs) {          // uniform over the workgroup
-            gathered(here);
-            if (tile + wgs < a.tiles) {           // (the loads have the time of a tile to arrive)
-                const Tile then = tile_of(tile + wgs);
-                here = locate_pair(then);
-                gather(then, here);
+        for (int tile = lb; tile < a.tiles;) {    // uniform over the workgroup
+            for (const int end = min(a.tiles, tile + bias_chain); tile < end; tile += wgs) {
+                gathered(here);
+                if (tile + wgs < a.tiles) {       // (the loads have the time of a tile to arrive)
+                    const Tile then = tile_of(tile + wgs);
+                    here = locate_pair(then);
+                    gather(then, here);
+                }
+                turn_over();
+                lds_sync();
             }
-            turn_over();
-            lds_sync();
+            state.bias(1) += state.bias(0);
+            state.bias(0) = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
         lds_sync();
         return false;
@@ -788,20 +810,23 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
         Unit un = unit_of(now, 0);
         if (kernel) request_x(un);
         lds_sync();
-        for (int tile = lb; tile < a.tiles; tile += wgs) {
-            if (kernel) {
-                const Tile then = tile_of(tile + wgs);
-                const bool split = tile_split();
+        for (int tile = lb; tile < a.tiles;) {
+            for (const int end = min(a.tiles, tile + chain); tile < end; tile += wgs) {
+                if (kernel) {
+                    const Tile then = tile_of(tile + wgs);
+                    const bool split = tile_split();
 #pragma unroll
-                for (int u = 0; u < kUnits; u++) {
-                    const Unit next = u + 1 < kUnits ? unit_of(now, u + 1) : unit_of(then, 0);
-                    again = !kernel_unit(u, split, now.sign, un, next) || again;
-                    un = next;
+                    for (int u = 0; u < kUnits; u++) {
+                        const Unit next = u + 1 < kUnits ? unit_of(now, u + 1) : unit_of(then, 0);
+                        again = !kernel_unit(u, split, now.sign, un, next) || again;
+                        un = next;
+                    }
+                    now = then;
                 }
-                now = then;
+                turn_over();
+                lds_sync();
             }
-            turn_over();
-            lds_sync();
+            second_level();
         }
         return again;
     } else {
@@ -881,6 +906,11 @@ __global__ __launch_bounds__(kPullThreads, 3) void pull_rows(const PullArgs a, c
     state.weights_split = true;
 #pragma unroll
     for (f32x4_t &v : state.kept) v = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    char *const sums2 = lds + S::kSumsAt + number * S::kSumBytes + lane * 16;      // a kernel worker's, second level
+    if (kind == kKernel) {
+#pragma unroll
+        for (int t = 0; t < kTiles; t++) *reinterpret_cast<f32x4_t *>(sums2 + t * kWave * 16) = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
     load_weights(false);
     __syncthreads();
 
@@ -897,6 +927,10 @@ __global__ __launch_bounds__(kPullThreads, 3) void pull_rows(const PullArgs a, c
 
     // the sums, of the waves that share a block through LDS
     constexpr int kBlock = 1024 * G;              // sums of a block of channels
+    if (kind == kKernel) {
+#pragma unroll
+        for (int t = 0; t < kTiles; t++) state.sums(t) += *reinterpret_cast<const f32x4_t *>(sums2 + t * kWave * 16);
+    }
     if constexpr (P == 1) {
         if (kind == kKernel && cb < blocks) {
 #pragma unroll
@@ -923,7 +957,7 @@ __global__ __launch_bounds__(kPullThreads, 3) void pull_rows(const PullArgs a, c
     if (chunk != 0) return;
     // the bias gradients: the centre taps, over the lanes' voxels and the segments
     const int h = wave % 2;                       // (the waves' outputs: see the gather)
-    f32x4_t bias_sum = state.bias();
+    f32x4_t bias_sum = state.bias(1);
     if constexpr (N != kImage) bias_sum[0] = (bias_sum[0] + bias_sum[1]) + (bias_sum[2] + bias_sum[3]);
 #pragma unroll
     for (int j = 0; j < kLaneOut; j++)
@@ -963,7 +997,7 @@ __global__ __launch_bounds__(1024) void sum_group(const SumArgs a, const float *
                                                   const float *__restrict__ bias_part)
 {
     constexpr int kTaps = Gather<N>::kTaps, kSlabOut = Gather<N>::kOutputs;
-    __shared__ float lds[16 * kWave];
+    __shared__ double lds[16 * kWave];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int col = blockIdx.x * kWave + lane, block = 1024 * a.slabs;
     const bool bias = (int)blockIdx.x * kWave >= a.columns;
@@ -980,25 +1014,25 @@ __global__ __launch_bounds__(1024) void sum_group(const SumArgs a, const float *
         p = part + (int64_t)a.chunks.first_wg(chunk) * a.stride + (blk - a.chunks.first_block(chunk)) * block + col % block;
         stride = a.stride;
     }
-    float part_sum[4] = {0.f, 0.f, 0.f, 0.f};     // (short chains, then trees: these are the largest sums)
+    double part_sum[4] = {0., 0., 0., 0.};        // (these are the largest sums)
     for (int r = wave; r < rows; r += 128) {
         float v[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) v[i] = p[min(r + 16 * i, rows - 1) * stride];
 #pragma unroll
-        for (int i = 0; i < 8; i++) part_sum[i % 4] += r + 16 * i < rows ? v[i] : 0.f;
+        for (int i = 0; i < 8; i++) part_sum[i % 4] += r + 16 * i < rows ? (double)v[i] : 0.;
     }
     lds[wave * kWave + lane] = (part_sum[0] + part_sum[1]) + (part_sum[2] + part_sum[3]);
     __syncthreads();
     if (wave != 0) return;
-    float tree[16];
+    double tree[16];
 #pragma unroll
     for (int w = 0; w < 16; w++) tree[w] = lds[w * kWave + lane];
 #pragma unroll
     for (int w = 8; w > 0; w /= 2)
 #pragma unroll
         for (int i = 0; i < w; i++) tree[i] += tree[i + w];
-    const float s = tree[0];
+    const float s = (float)tree[0];
     if (bias) {
         const int o = lane / kBiasColumns * kSlabOut + lane % kBiasColumns;
         if (lane < a.slabs * kBiasColumns && lane % kBiasColumns < kSlabOut && o < a.n) a.gb[o] = a.fresh ? s : a.gb[o] + s;

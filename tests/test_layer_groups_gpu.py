@@ -139,6 +139,54 @@ def test_backward_passes_over_few_blocks(size, batch, c_in, slabs):
         check_block(len(size), size, c_in, 1, depth, batch, dilations=[1 + 2 * i % 5 for i in range(depth)], seed=107)
 
 
+def exact_weight_gradients(x, g, dilations):
+    """[output, channel, tap] in 64 bits: sum over v of x[c][reflected(v + dilation (tap - 1))] g[o][v]."""
+    size = x.shape[2:]
+    found = []
+    for o, d in enumerate(dilations):
+        source = []
+        for n in size:
+            at = torch.arange(n, device=x.device) + d * torch.arange(-1, 2, device=x.device)[:, None]
+            at = torch.where(at < 0, -1 - at, at)
+            source.append(torch.where(at >= n, 2 * n - 1 - at, at))
+        taps = []
+        for tap in range(3 ** len(size)):
+            h = g[:, o].double()                   # what each voxel of x meets
+            for axis in range(len(size)):
+                k = tap // 3 ** (len(size) - 1 - axis) % 3
+                h = torch.zeros_like(h).index_add_(axis + 1, source[axis][k], h)
+            taps.append(torch.stack([(x[:, c].double() * h).sum() for c in range(x.shape[1])]))
+        found.append(torch.stack(taps, 1))
+    return torch.stack(found)
+
+
+# Sums over millions of voxels: chains of 16 additions, of a sixteenth of the units of 32 voxels that a worker of one of 256 workgroups has
+# (two workers share a block where there are one or two), and some 32 levels below and above them.  An addition of terms of mixed sign rounds to 0.6
+# 2^-24 of its sum (the rms of half a unit in the last place), of which n in a chain come to sqrt(n / 2).  1.3: x is of one sign, so that
+# some partial sums are larger.
+@pytest.mark.parametrize("size, c_in, outputs, workers", [
+    ((2048, 2048), 25, 14, 2), ((2048, 2048), 40, 14, 1), ((3000, 4096), 25, 7, 2), ((192, 192, 192), 30, 4, 2), ((192, 192, 192), 46, 4, 1)],
+    ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_weight_gradients_over_many_voxels(size, c_in, outputs, workers):
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator(device="cuda").manual_seed(83)
+    stack = torch.rand(1, c_in + outputs, *size, device="cuda", generator=gen)
+    stack[:, c_in:] = 1                            # every ReLU open
+    gradient = torch.randn(1, c_in + outputs, *size, device="cuda", generator=gen)
+    dilations = [1 + i % 10 for i in range(outputs)]
+    weights = [torch.randn(1, c_in + i, *[3] * len(size), device="cuda", generator=gen) * 0.1 for i in range(outputs)]
+    for w in weights:
+        w[:, c_in:] = 0                            # (the outputs' gradients are what they are given as)
+    want = exact_weight_gradients(stack[:, :c_in], gradient[:, c_in:], dilations)
+    gk, gb = [torch.zeros_like(w) for w in weights], torch.zeros(outputs, device="cuda")
+    with tuning({"bwd.group": 1}):
+        cc.block_backward(stack, gradient, c_in, dilations, weights, gk, gb, True)
+    got = torch.stack([k[0, :c_in].reshape(c_in, -1) for k in gk])
+    units = torch.Size(size).numel() / 32 / 256 / workers
+    bound = 1.3 * 0.6 * 2.0 ** -24 * (16 / 2 + units / 16 / 2 + 32 / 2) ** 0.5
+    assert float((got - want).norm() / want.norm()) <= bound
+
+
 # Volumes: groups of up to four outputs, the same tiles over the rows of all slices.  Slices and rows
 # whose outer taps lie outside on both sides, dilations up to the volume, tiles that end inside a volume and between
 # two, every remainder modulo four, groups of 2, 3 and 4 outputs and a layer left over, two channels per layer, blocks
