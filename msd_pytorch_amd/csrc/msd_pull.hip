@@ -14,7 +14,7 @@
 // every 16 additions, and leave as one row of partial sums per workgroup, which sum_group adds in double precision.  x and grad_input go through a transposition in the wave's own part of LDS:
 // in the layout of the matrix cores a load touches 64 bytes of each of 16 channels, which memory
 // serves at 2.6-3.0 TB/s whatever else happens, whole lines at 4.0 (probed with loads and
-// stores alone, 64 channels of 1024 x 1024).  Five to eight blocks of two slabs: msd_pull_wide.h.
+// stores alone, 64 channels of 1024 x 1024).  Five to eight blocks of two slabs, and three and four of one slab in large images: msd_pull_wide.h.
 //
 // Bound by the issue of instructions: a SIMD issues a conversion, shift or select of a wave in 4.3 cycles and a matrix instruction
 // in 16.2, beside which there is room for two of the former, and a wave issues one instruction of any kind in 4.2 cycles.  With eight waves that all gathered and
@@ -50,7 +50,6 @@ constexpr int kXRow = 2 * kSegment + 16, kDRow = 4 * kSegment + 16;
 constexpr int kVec = 2, kLanes = kSegment / 4;    // 16-byte accesses per lane for a segment of 16 channels; lanes of a channel in one of them
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
 
 // What the kernels run over.  kFlat: a volume whose voxels lie without gaps, as one row: segments cross the
 // ends of the rows, every lane has a row of its own.
@@ -1304,16 +1303,23 @@ hipError_t pull_launch(F *kernel, int threads, int lds, LargeLds &large, const P
 
 // Blocks of a chunk, at most (one slab: 411 us over 100 channels, 463 with 8).
 int most_blocks(int slabs) { return slabs == 1 ? 4 : 8; }
-// Blocks of a chunk that pull_rows takes; pull_rows_wide the others.
-constexpr int kNarrowBlocks = 4;
+// Blocks of a chunk of two slabs that pull_rows takes; pull_rows_wide the others, and three and four of one slab from as many segments of 32 voxels
+// on.  There the eight waves of the latter are faster, which all gather a tile twice as large and then all multiply.  Backward pass of seven outputs
+// (3D: two) with all launches, pull_rows to pull_rows_wide 1, over 40 / 48 / 60 channels: 724 x 724 0.95 / 0.94 / 1.07, 800 x 800 1.01 / 1.05 / 1.12, 1024 x
+// 1000 1.04 / 1.02 / 1.01, 2048 x 2048 1.13 / 1.04 / 1.05; 100^3 1.02 / 0.96 / 0.99, 113^3 1.02 / 0.97 / 1.01, 128^3 1.09 / 1.07 / 1.12; a
+// layer of three outputs 724 x 724 0.96 / 0.95 / 0.96, 900 x 900 1.00 / 1.03 / 1.04, 2048 x 2048 1.09 / 1.12 / 1.10; of one in 3D 100^3 0.96 / 1.00 / 1.00,
+// 128^3 1.02 / 1.07 / 1.08.  (Loads requested two and four units ahead, or gathered two tiles ahead, change nothing in pull_rows.)
+constexpr int kNarrowBlocks = 4, kNarrowOneSlab = 2;
+constexpr int64_t kWideImage = 20000, kWideVolume = 50000;
 
 // As many workgroups as are resident, shared out over the chunks by their size.
 struct PullPlan {
     Chunks chunks;
     int segs, wgs, image_tiles, tiles;
+    bool wide;                                    // pull_rows_wide
 };
 
-PullPlan pull_plan(int64_t batch, int64_t rows, int64_t span, int64_t channels, int slabs)
+PullPlan pull_plan(int64_t batch, int64_t rows, int64_t span, int64_t channels, int slabs, int64_t wide_from)
 {
     PullPlan p;
     const int nb = (int)((channels + 15) / 16);
@@ -1323,7 +1329,8 @@ PullPlan pull_plan(int64_t batch, int64_t rows, int64_t span, int64_t channels, 
     c.blocks = (nb + c.n - 1) / c.n;
     c.large = nb - c.n * (c.blocks - 1);
     p.segs = (int)((span + kSegment - 1) / kSegment);
-    const int per_tile = (c.blocks > kNarrowBlocks ? kWaves : kOfKind) / slabs;
+    p.wide = slabs == 1 ? c.blocks > kNarrowOneSlab && batch * rows * p.segs >= wide_from : c.blocks > kNarrowBlocks;
+    const int per_tile = (p.wide ? kWaves : kOfKind) / slabs;
     p.image_tiles = (int)((rows * p.segs + per_tile - 1) / per_tile);
     p.tiles = (int)batch * p.image_tiles;
     auto share = [&](int blocks) {
@@ -1371,10 +1378,11 @@ int64_t pull_channels(int64_t batch, int64_t rows, const PullPlan &p, int64_t ch
 // Floats of the largest of the launches, whether the gradients are written or added to.
 int64_t all_pull_floats(int64_t batch, int64_t rows, int64_t span, int64_t channels, int slabs)
 {
-    const PullPlan p = pull_plan(batch, rows, span, channels, slabs);
+    // (either kernel has as many workgroups where it is chosen by the voxels: fewer than tiles)
+    const PullPlan p = pull_plan(batch, rows, span, channels, slabs, kWideImage);
     const int64_t step = pull_channels(batch, rows, p, channels, slabs, true), rest = channels % step;
-    int64_t most = std::max(pull_floats(p, slabs), pull_floats(pull_plan(batch, rows, span, step, slabs), slabs));
-    if (rest > 0) most = std::max(most, pull_floats(pull_plan(batch, rows, span, rest, slabs), slabs));
+    int64_t most = std::max(pull_floats(p, slabs), pull_floats(pull_plan(batch, rows, span, step, slabs, kWideImage), slabs));
+    if (rest > 0) most = std::max(most, pull_floats(pull_plan(batch, rows, span, rest, slabs, kWideImage), slabs));
     return most;
 }
 
@@ -1412,7 +1420,7 @@ hipError_t pull_part(const Geom &g, const View<const float> &x, const float *gy,
     const Form form = form_of(g, x);
     const int slabs = out.n > per_slab ? 2 : 1;
     const int span = form == kFlat ? g.nvox : g.W, rows = g.nvox / span;
-    const PullPlan p = pull_plan(g.B, rows, span, g.C, slabs);
+    const PullPlan p = pull_plan(g.B, rows, span, g.C, slabs, g.ndim == 3 ? kWideVolume : kWideImage);
     PullArgs a{g.C, update, mask_from, g.D, g.H, g.W, span, p.segs, rows * p.segs, p.tiles, p.image_tiles, Divisor((uint32_t)p.segs),
                Divisor((uint32_t)p.image_tiles), Divisor((uint32_t)g.H), Divisor((uint32_t)g.W), reverse, 0, p.chunks,
                x.sb, x.sc, x.sz, x.sy, gsb, gsc, out};
@@ -1433,19 +1441,22 @@ hipError_t pull_part(const Geom &g, const View<const float> &x, const float *gy,
             return pull_launch(&pull_rows<N, G, P, decltype(fresh_)::value>, kPullThreads, PullShape<G, P>::kLds, large, a, p.wgs, x.p, gy, grads.p, ws,
                                bias_part, s);
         };
+        auto run_wide = [&](auto g_, auto p_, auto fresh_) {
+            constexpr int G = decltype(g_)::value, P = decltype(p_)::value;
+            static LargeLds large;
+            return pull_launch(&pull_rows_wide<N, G, P, decltype(fresh_)::value>, kWaves * kWave, WideShape<G, P>::kLds, large, a, p.wgs, x.p, gy, grads.p,
+                               ws, bias_part, s);
+        };
         constexpr std::integral_constant<int, 1> one{};
         constexpr std::integral_constant<int, 2> two{};
         constexpr std::integral_constant<int, 4> four{};
         if constexpr (N != kVolume) {
             constexpr std::true_type yes{};
-            if (fresh) return blocks > 2 ? run(one, one, yes) : blocks > 1 ? run(one, two, yes) : run(one, four, yes);
+            if (fresh) return p.wide ? run_wide(one, two, yes) : blocks > 2 ? run(one, one, yes) : blocks > 1 ? run(one, two, yes) : run(one, four, yes);
         }
         constexpr std::false_type no{};
-        if (slabs == 1) return blocks > 2 ? run(one, one, no) : blocks > 1 ? run(one, two, no) : run(one, four, no);
-        if (blocks > kNarrowBlocks) {
-            static LargeLds large;
-            return pull_launch(&pull_rows_wide<N>, kWaves * kWave, kWideLds, large, a, p.wgs, x.p, gy, grads.p, ws, bias_part, s);
-        }
+        if (slabs == 1) return p.wide ? run_wide(one, two, no) : blocks > 2 ? run(one, one, no) : blocks > 1 ? run(one, two, no) : run(one, four, no);
+        if (p.wide) return run_wide(two, one, no);
         return blocks > 2 ? run(two, one, no) : run(two, two, no);
     };
     switch (form) {
@@ -1477,7 +1488,7 @@ hipError_t pull(const Geom &g, const View<const float> &x, const float *gy, int6
         return hipErrorInvalidValue;
     const int slabs = out.n > per_slab ? 2 : 1, taps = g.ndim == 3 ? 27 : group2d::kTaps;
     const int span = form == kFlat ? g.nvox : g.W, rows = g.nvox / span;
-    const int step = (int)pull_channels(g.B, rows, pull_plan(g.B, rows, span, g.C, slabs), g.C, slabs, fresh);
+    const int step = (int)pull_channels(g.B, rows, pull_plan(g.B, rows, span, g.C, slabs, kWideImage), g.C, slabs, fresh);
     for (int from = 0; from < g.C; from += step) {
         Geom part = g;
         View<const float> xp = x;

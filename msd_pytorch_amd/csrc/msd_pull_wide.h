@@ -1,9 +1,10 @@
-// pull_rows_wide: pull_rows (msd_pull.hip, which includes this where its own helpers are declared) for two slabs over five to eight blocks of
-// 16 channels, of which every wave has one.
+// pull_rows_wide: pull_rows (msd_pull.hip, which includes this where its own helpers are declared) with eight waves that all gather and then all
+// multiply: two slabs over five to eight blocks of 16 channels, of which every wave has one, and one slab over three and four, of which
+// every wave has half of one, in large images.
 //
-// A workgroup of eight waves owns a tile of four segments of 32 voxels and the 128 rows m of two slabs.  Each wave gathers a segment's A of one slab, splits
-// it and leaves it in LDS; behind a barrier each wave takes its own block through both products, 64 voxels at a time.  Over fewer blocks
-// waves would be idle in the products, and pull_rows is faster; over these the three kinds of waves of pull_rows
+// A workgroup owns a tile of four segments of 32 voxels and the 128 rows m of two slabs, or of eight segments and one slab.  Each wave gathers a segment's A of
+// one slab, splits it and leaves it in LDS; behind a barrier each wave takes its own block through both products, 64 voxels at a time.  Over fewer
+// blocks waves would be idle in the products, and pull_rows is faster; over five to eight of two slabs the three kinds of waves of pull_rows
 // would need two blocks each, for which there are no registers (1024 x 1024, 14 outputs over 87 channels: 430 us; three kinds of waves with two blocks and
 // registers spilt 528; these eight waves with the gather and the products of pull_rows 442).
 #pragma once
@@ -14,7 +15,11 @@ namespace {
 
 constexpr int kWaves = 8;                         // of a workgroup; one workgroup per compute unit
 
+// LDS of a wave for a unit of voxels: 16 channels of x in three parts (the sums for grad_input take less)
+constexpr int unit_bytes(int voxels) { return 3 * 16 * (2 * voxels + 16); }
+
 // What a workgroup keeps in LDS besides A and the waves' own space.
+// What a workgroup of pull_rows_wide keeps in LDS besides A and the waves' own space.
 struct Source {                                   // an output's place in bytes: its dilation in slices, rows and voxels, its plane
     uint32_t slices, rows, voxels, plane;
 };
@@ -24,36 +29,43 @@ struct WideShared {
     f32x4_t bias_sums[kWaves * kWave];                // of the lanes' outputs at their voxels (not in registers: there are none left)
 };
 
-constexpr int kWideSlabs = 2, kWideSteps = 2 * kWideSlabs, kWideTiles = 4 * kWideSlabs;        // of 32 rows m, of 16
-constexpr int kWideSegs = kWaves / kWideSlabs;    // segments of a tile
-constexpr int kWideUnit = 64, kWideUnits = kWideSegs * kSegment / kWideUnit;       // voxels that a wave takes through the products at a time
-constexpr int kWideXRow = 2 * kWideUnit + 16, kWideDRow = 4 * kWideUnit + 16;      // bytes of a channel (16 apart in the banks)
-constexpr int kWideOwn = 3 * 16 * kWideXRow;      // of a wave: 16 channels of x in three parts (the sums for grad_input take less)
-constexpr int kWideLds = kWideSegs * kWideSlabs * kSlabBytes + kWaves * kWideOwn;
+// G slabs of rows; P waves share a block of 16 channels (the tile's voxels in as many parts).
+template <int G, int P> struct WideShape {
+    static_assert(G * P == 2, "a block per wave and two slabs, or half a block and one");
+    static constexpr int kSegs = kWaves / G;             // segments of a tile
+    static constexpr int kSteps = 2 * G;                 // of 32 rows m
+    static constexpr int kTiles = 4 * G;                 // of 16 rows m
+    static constexpr int kUnit = 64;                     // voxels that a wave takes through the products at a time
+    static constexpr int kUnits = kSegs * kSegment / P / kUnit;
+    static constexpr int kVec = kUnit / 16;              // 16-byte accesses per lane for a unit of 16 channels
+    static constexpr int kLanes = kUnit / 4;             // lanes of a channel in one of them
+    static constexpr int kOwnBytes = unit_bytes(kUnit);
+    static constexpr int kLds = kSegs * G * kSlabBytes + kWaves * kOwnBytes;
+};
 
 // What the kernel keeps for its life: the weights of rows 32 step + 8 q .. of channel n in parts, the sums of
 // grad_kernel.
-struct WideState {
-    bf16x8_t w[kWideSteps][3];
+template <int G> struct WideState {
+    bf16x8_t w[2 * G][3];
     bool weights_split;
-    f32x4_t sums[kWideTiles];
+    f32x4_t sums[4 * G];
 };
 
 // The tiles of a workgroup.  True where units were left out that hold values which cannot be split: the second
 // run (WHOLE) takes these, with the fp32 instruction.  Apart, so that it keeps no registers in the first.
-template <int N, bool WHOLE>
+template <int N, int G, int P, bool FRESH, bool WHOLE>
 __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__restrict__ x, const float *gy, float *gx, char *lds,
-                                           WideShared &shared, int tid, int wave, int blocks, int c0, int wgs, int wg, WideState &state)
+                                           WideShared &shared, int tid, int wave, int blocks, int c0, int wgs, int wg, WideState<G> &state)
 {
-    constexpr int G = kWideSlabs, kSegs = kWideSegs, kSteps = kWideSteps, kTiles = kWideTiles, kUnit = kWideUnit, kUnits = kWideUnits;
-    constexpr int kVec = kUnit / 16, kLanes = kUnit / 4;            // 16-byte accesses per lane for a unit of 16 channels; lanes of a channel
-    constexpr int kXRow = kWideXRow, kDRow = kWideDRow;
+    using S = WideShape<G, P>;
+    constexpr int kSegs = S::kSegs, kSteps = S::kSteps, kTiles = S::kTiles, kUnit = S::kUnit, kUnits = S::kUnits, kVec = S::kVec;
+    constexpr int kLanes = S::kLanes, kOwnBytes = S::kOwnBytes;
     constexpr int kTaps = Gather<N>::kTaps, kLines = Gather<N>::kLines, kLaneOut = Gather<N>::kLaneOut, kSlabOut = Gather<N>::kOutputs;
     const int lane = tid % kWave;
-    const int cb = wave, ch0 = c0 + cb * 16;      // the wave's block
+    const int cb = wave / P, ch0 = c0 + cb * 16;  // the wave's block
     const bool active = cb < blocks, update = ch0 < a.update;       // uniform
     char *const A = lds;
-    char *const own = lds + kSegs * G * kSlabBytes + wave * kWideOwn;
+    char *const own = lds + kSegs * G * kSlabBytes + wave * kOwnBytes;
     bf16x8_t(&w)[kSteps][3] = state.w;
     f32x4_t(&sums)[kTiles] = state.sums;
 
@@ -105,7 +117,7 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
         int skip;                                 // first of its four voxels that is its segment's own (0: all, 4: none)
     };
     auto unit_of = [&](const Tile &t, int u) {
-        const int first = u * (kUnit / kSegment);
+        const int first = ((wave % P) * kUnits + u) * (kUnit / kSegment);
         const Place p0 = locate(t, first), p1 = locate(t, first + kUnit / kSegment - 1);
         const int sel = lv / (kSegment / 4), v4 = lv % (kSegment / 4) * 4;
         const uint32_t at0 = 4u * (uint32_t)(row_at(p0.z, p0.y) + p0.x0), at1 = 4u * (uint32_t)(row_at(p1.z, p1.y) + p1.x0);
@@ -131,7 +143,12 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
     };
     f32x4_t xs[kVec], gs[kVec];
     auto request_g = [&](const Unit &un) {
-        request(gx, max(a.update, 1), un, gs);
+        if constexpr (FRESH) {
+#pragma unroll
+            for (int i = 0; i < kVec; i++) gs[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        } else {
+            request(gx, max(a.update, 1), un, gs);
+        }
     };
 
     // ---- the gather: lane (v, h) takes its outputs at voxel v of the wave's segment, 36 (27) values for 32 rows
@@ -290,6 +307,8 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
     // ---- the products of a unit.  The wave's own space holds x as [part][channel][voxel], then what is added to
     // grad_input as [channel][voxel]: loads and stores go by channel in whole lines, the matrix cores take 16
     // channels at once (loaded in that form, 64 bytes of 16 channels at a time, memory gives 2.6 to 3.0 TB/s instead of 4).
+    constexpr int kXRow = 2 * kUnit + 16, kDRow = 4 * kUnit + 16;   // bytes of a channel (16 apart in the banks)
+    const int first_seg = (wave % P) * kUnits * (kUnit / kSegment); // of the wave's first unit
     auto clear_skipped = [&](const Unit &un) {    // an infinity there belongs to the other segment
         if (__any(un.skip > 0)) {
 #pragma unroll
@@ -360,9 +379,9 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
     // False where a value cannot be split (and nothing is computed).
     auto compute = [&](int u, bool split, uint32_t sign_bit, const Unit &un, const Unit &next) {
         uint32_t ll = (uint32_t)lane;
-        asm volatile("" : "+v"(ll));              // (no LDS addresses are kept over the tiles: registers)
+        if (G > 1) asm volatile("" : "+v"(ll));                     // (no LDS addresses are kept over the tiles: registers)
         const uint32_t nn = ll % 16, qq = ll / 16 % 4;
-        const char *const Au = A + u * kK * G * kSlabBytes;
+        const char *const Au = A + (first_seg + u * kK) * G * kSlabBytes;
         // rows 16 t + n, voxels 8 q .. of segment j (the lane's address is that of voxel 8 q + n / 4 (+ 4), rows
         // 4 (n % 4) .., which the read transposes)
         const uint32_t tr_voxel = 8 * qq + nn / 4;
@@ -400,8 +419,10 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
         __builtin_amdgcn_sched_barrier(0);
         if (!done) return false;
         own_sync();
-        // Both products in stages of two chains of six matrix instructions.
-        bf16x8_t op[2][3], xp[kK][3];
+        // Both products in stages of two chains of six matrix instructions, whose operands are read from LDS a
+        // stage ahead (where there are registers for it).
+        constexpr bool kAhead = G == 1;
+        bf16x8_t op[2][2][3], xp[kK][3];
         constexpr int kRowStages = kTiles * kK / 2, kVoxelStages = kSteps * kK;
         // stage r: tiles 2 (r / kK) and the next at segment r % kK
         auto stage_rows = [&](int r, bf16x8_t(&to)[2][3]) {
@@ -415,6 +436,7 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
         };
         f32x4_t acc[2];
         bf16x8_t high[2];
+        stage_rows(0, op[0]);
 #pragma unroll
         for (int j = 0; j < kK; j++)
 #pragma unroll
@@ -422,7 +444,9 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
                 xp[j][p] = *reinterpret_cast<const bf16x8_t *>(own + (p * 16 + nn) * kXRow + (32 * j + 8 * qq) * 2);
 #pragma unroll
         for (int r = 0; r < kRowStages; r++) {
-            stage_rows(r, op);
+            if (!kAhead && r > 0) stage_rows(r, op[r % 2]);
+            if (kAhead && r + 1 < kRowStages) stage_rows(r + 1, op[(r + 1) % 2]);
+            if (kAhead && r + 1 == kRowStages) stage_voxels(0, op[(r + 1) % 2]);
             __builtin_amdgcn_sched_barrier(0);
             // (the products of the high parts of both segments last: each instruction cuts its sum off at the size
             // that it has reached)
@@ -430,16 +454,16 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
             for (int k = 0; k < 5; k++)
 #pragma unroll
                 for (int o = 0; o < 2; o++)
-                    acc[o] = mfma_split(op[o], xp[r % kK], k == 0 && r % kK == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[o], k);
+                    acc[o] = mfma_split(op[r % 2][o], xp[r % kK], k == 0 && r % kK == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : acc[o], k);
             if (r % kK == kK - 1) {
 #pragma unroll
                 for (int j = 0; j < kK; j++)
 #pragma unroll
                     for (int o = 0; o < 2; o++)
-                        acc[o] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j == kK - 1 ? op[o][0] : high[o], xp[j][0], acc[o], 0, 0, 0);
+                        acc[o] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j == kK - 1 ? op[r % 2][o][0] : high[o], xp[j][0], acc[o], 0, 0, 0);
             } else {
 #pragma unroll
-                for (int o = 0; o < 2; o++) high[o] = op[o][0];
+                for (int o = 0; o < 2; o++) high[o] = op[r % 2][o][0];
             }
             if (r % kK == kK - 1) {
 #pragma unroll
@@ -456,22 +480,23 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
 #pragma unroll
             for (int r = 0; r < kVoxelStages; r++) {
                 const int i = r % kSteps;
-                stage_voxels(r, op);
+                if (!kAhead) stage_voxels(r, op[(kRowStages + r) % 2]);
+                if (kAhead && r + 1 < kVoxelStages) stage_voxels(r + 1, op[(kRowStages + r + 1) % 2]);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int k = 0; k < 5; k++)
 #pragma unroll
                     for (int s = 0; s < 2; s++)
-                        d[s] = mfma_split(op[s], w[i], k == 0 && i % 2 == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : d[s], k);
+                        d[s] = mfma_split(op[(kRowStages + r) % 2][s], w[i], k == 0 && i % 2 == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : d[s], k);
                 if (i % 2 == 0) {
 #pragma unroll
-                    for (int s = 0; s < 2; s++) high[s] = op[s][0];
+                    for (int s = 0; s < 2; s++) high[s] = op[(kRowStages + r) % 2][s][0];
                 } else {
 #pragma unroll
                     for (int j = 0; j < 2; j++)
 #pragma unroll
                         for (int s = 0; s < 2; s++)
-                            d[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j ? op[s][0] : high[s], w[i - 1 + j][0], d[s], 0, 0, 0);
+                            d[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j ? op[(kRowStages + r) % 2][s][0] : high[s], w[i - 1 + j][0], d[s], 0, 0, 0);
                 }
                 // Summed slab by slab from zero and added to grad_input last: a chain of products that started from it
                 // would round each of them to its size.
@@ -500,7 +525,7 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
         uint32_t ll = (uint32_t)lane;
         asm volatile("" : "+v"(ll));
         const uint32_t nn = ll % 16, qq = ll / 16 % 4;
-        const char *const Au = A + u * kK * G * kSlabBytes;
+        const char *const Au = A + (first_seg + u * kK) * G * kSlabBytes;
         auto value = [&](uint32_t voxel, uint32_t m) {
             const char *const at = Au + (voxel / kSegment * G + m / kRows) * kSlabBytes + voxel % kSegment * kVoxelBytes +
                                    16 * (m % kRows / 8 ^ turn(voxel)) + m % 8 * 2;
@@ -643,11 +668,12 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
     }
 }
 
-template <int N>
+// FRESH: grad_input is written, not added to.
+template <int N, int G, int P, bool FRESH = false>
 __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows_wide(const PullArgs a, const float *__restrict__ x, const float *gy,
                                                              float *gx, float *__restrict__ part, float *__restrict__ bias_part)
 {
-    constexpr int G = kWideSlabs, kSegs = kWideSegs, kTiles = kWideTiles;
+    constexpr int kSegs = WideShape<G, P>::kSegs, kTiles = WideShape<G, P>::kTiles;
     constexpr int kTaps = Gather<N>::kTaps, kLaneOut = Gather<N>::kLaneOut, kSlabOut = Gather<N>::kOutputs;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tid = threadIdx.x;
@@ -657,9 +683,9 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows_wide(const PullArg
     const int chunk = bid < big ? bid / a.chunks.wgs : a.chunks.large + (bid - big) / a.chunks.wgs_small;
     const int blocks = a.chunks.size(chunk), c0 = a.chunks.first_block(chunk) * 16;
     const int wgs = a.chunks.rows(chunk), wg = bid - a.chunks.first_wg(chunk);
-    const int cb = wave, ch0 = c0 + cb * 16;      // the wave's block
+    const int cb = wave / P, ch0 = c0 + cb * 16;  // the wave's block
     __shared__ WideShared shared;
-    WideState state;
+    WideState<G> state;
 
     if (tid == 0) shared.bad_again = 0;
     if (tid < G * kSlabOut) {
@@ -694,21 +720,38 @@ __global__ __launch_bounds__(kWaves *kWave, 2) void pull_rows_wide(const PullArg
 #pragma unroll
     for (int t = 0; t < kTiles; t++) state.sums[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     shared.bias_sums[tid] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    const bool again = wide_tiles<N, false>(a, x, gy, gx, lds, shared, tid, wave, blocks, c0, wgs, wg, state);
+    const bool again = wide_tiles<N, G, P, FRESH, false>(a, x, gy, gx, lds, shared, tid, wave, blocks, c0, wgs, wg, state);
     if (lane == 0 && again) shared.bad_again = 1;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(shared.bad_again) != 0) {    // uniform over the workgroup
         int tid2 = tid;
         asm volatile("" : "+v"(tid2));           // (nothing of the first run is kept for the second)
         load_weights(true);
-        wide_tiles<N, true>(a, x, gy, gx, lds, shared, tid2, wave, blocks, c0, wgs, wg, state);
+        wide_tiles<N, G, P, FRESH, true>(a, x, gy, gx, lds, shared, tid2, wave, blocks, c0, wgs, wg, state);
     }
 
-    if (cb < blocks) {
+    // the sums, of the waves that share a block through LDS
+    constexpr int kBlock = 1024 * G;              // sums of a block of channels
+    if constexpr (P == 1) {
+        if (cb < blocks) {
+#pragma unroll
+            for (int t = 0; t < kTiles; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) row[cb * kBlock + (t * 4 + r) * kWave + lane] = state.sums[t][r];
+        }
+    } else {
+        float *const red = reinterpret_cast<float *>(lds);
+        __syncthreads();
 #pragma unroll
         for (int t = 0; t < kTiles; t++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) row[cb * 1024 * G + (t * 4 + r) * kWave + lane] = state.sums[t][r];
+            for (int r = 0; r < 4; r++) red[wave * kBlock + (t * 4 + r) * kWave + lane] = state.sums[t][r];
+        __syncthreads();
+        for (int i = tid; i < kWaves / P * kBlock; i += kWaves * kWave) {
+            const int b = i / kBlock;
+            const float *const r = red + b * P * kBlock + i % kBlock;
+            if (b < blocks) row[i] = r[0] + r[kBlock];
+        }
     }
     if (chunk != 0) return;
     const int v = lane % kSegment, h = lane / kSegment;

@@ -187,6 +187,35 @@ def test_weight_gradients_over_many_voxels(size, c_in, outputs, workers):
     assert float((got - want).norm() / want.norm()) <= bound
 
 
+# One slab of outputs over three and four blocks: from 20000 segments of 32 voxels on (volumes 50000) the eight waves that gather and multiply in
+# turn.  Just below and just above, rows that end inside a segment, rows with gaps, two images, a block without its last channels and
+# a chunk of two blocks beside one of three; against the layers on their own.
+@pytest.mark.parametrize("size, batch, c_in, gap, wide", [
+    ((799, 800), 1, 40, 0, False), ((801, 799), 1, 40, 0, True), ((400, 830), 2, 62, 3, True), ((801, 800), 1, 75, 0, True),
+    ((801, 798), 1, 31, 0, False), ((100, 160, 99), 1, 47, 0, False), ((100, 161, 101), 1, 47, 0, True), ((100, 125, 99), 1, 33, 1, True),
+    ((50, 124, 100), 2, 33, 1, False)], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_one_slab_over_three_and_four_blocks(size, batch, c_in, gap, wide):
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator(device="cuda").manual_seed(89)
+    both = torch.randn(2, batch, c_in + 2, *size[:-1], size[-1] + gap, device="cuda", generator=gen)
+    stack, gradient = both[0][..., :size[-1]], both[1][..., :size[-1]]
+    weights = [torch.randn(1, c_in + i, *[3] * len(size), device="cuda", generator=gen) * 0.1 for i in range(2)]
+
+    def run(setting):
+        g = torch.empty_strided(gradient.shape, gradient.stride(), device="cuda").copy_(gradient)
+        gk, gb = [torch.zeros_like(w) for w in weights], torch.zeros(2, device="cuda")
+        with tuning({"bwd.group": setting}):
+            cc.block_backward(stack, g, c_in, [3, 7], weights, gk, gb, True)
+        return g[:, :c_in], gb, *gk
+
+    torch.cuda.synchronize()
+    passes = [name for name, _ in captured_kernels(lambda: run(1)) if "pull_rows" in name]
+    assert len(passes) == 1 and ("pull_rows_wide" in passes[0]) == wide
+    found = [run(setting) for setting in (0, 1)]
+    for a, b in zip(*found):
+        assert rel_err(b, a) <= 1e-5
+
+
 # Volumes: groups of up to four outputs, the same tiles over the rows of all slices.  Slices and rows
 # whose outer taps lie outside on both sides, dilations up to the volume, tiles that end inside a volume and between
 # two, every remainder modulo four, groups of 2, 3 and 4 outputs and a layer left over, two channels per layer, blocks
