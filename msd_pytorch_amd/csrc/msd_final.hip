@@ -358,6 +358,14 @@ __global__ __launch_bounds__(kFinalThreads) void final_forward_loss_kernel(
 constexpr int kTiledWaves = 8;
 constexpr int kTiledThreads = kTiledWaves * kWave;
 constexpr int kTiledMaxChannels = 512;
+constexpr int kTiledChain = 32;                   // tiles of a workgroup, at most (see launch_tiled)
+
+template <int V> __device__ __forceinline__ float sum_of(const float (&v)[V])
+{
+    if constexpr (V == 4) return (v[0] + v[1]) + (v[2] + v[3]);
+    else if constexpr (V == 2) return v[0] + v[1];
+    else return v[0];
+}
 
 // Workgroups per compute unit: their registers (the running sums, the next tile's values, targets) decide.
 template <int V, int MAXO, int KIND, int CC> constexpr int tiled_workgroups()
@@ -576,9 +584,7 @@ __global__ __launch_bounds__(kTiledThreads, (2 * tiled_workgroups<V, MAXO, KIND,
         }
         if (wave == 0) {
 #pragma unroll
-            for (int o = 0; o < MAXO; o++)
-#pragma unroll
-                for (int e = 0; e < V; e++) sb[o] += g[o][e];
+            for (int o = 0; o < MAXO; o++) sb[o] += sum_of(g[o]);
         }
         if (want_sums) {                                      // uniform
             asm volatile("" : "+s"(count));
@@ -588,9 +594,12 @@ __global__ __launch_bounds__(kTiledThreads, (2 * tiled_workgroups<V, MAXO, KIND,
                     float xv[V];
                     load_elems<float, V>(own + cc * kTiledWaves * TV, xv);
 #pragma unroll
-                    for (int o = 0; o < MAXO; o++)
+                    for (int o = 0; o < MAXO; o++) {
+                        float tile_sum = g[o][0] * xv[0];
 #pragma unroll
-                        for (int e = 0; e < V; e++) sw[o][cc] += g[o][e] * xv[e];
+                        for (int e = 1; e < V; e++) tile_sum += g[o][e] * xv[e];
+                        sw[o][cc] += tile_sum;
+                    }
                 }
             }
         }
@@ -636,18 +645,19 @@ __global__ __launch_bounds__(256) void final_reduce_kernel(const T *__restrict__
                                                            int64_t nb, T *__restrict__ gw, T *__restrict__ gb,
                                                            T *__restrict__ loss)
 {
-    __shared__ T wave_sum[256 / kWave];
+    __shared__ double wave_sum[256 / kWave];
     const int64_t col = blockIdx.x;
     const T *p = part + col * rows;
-    T s = T(0);
+    double s = 0.;                                // (these are the largest sums)
     for (int64_t r = threadIdx.x; r < rows; r += 256) s += p[r];
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) s += __shfl_down(s, off, kWave);
     if (threadIdx.x % kWave == 0) wave_sum[threadIdx.x / kWave] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
-        T total = wave_sum[0];
-        for (int w = 1; w < 256 / kWave; w++) total += wave_sum[w];
+        double sum = wave_sum[0];
+        for (int w = 1; w < 256 / kWave; w++) sum += wave_sum[w];
+        const T total = (T)sum;
         if (col < nw) {
             if (gw) gw[col] = total;
         } else if (col < nw + nb) {
@@ -802,7 +812,10 @@ hipError_t launch_tiled(int64_t batch, int c_in, int c_out, int64_t nvox, const 
         if (e != hipSuccess) return e;
     }
     const int per_cu = lds * 2 <= kTiledLds ? tiled_workgroups<V, MAXO, KIND, CC>() : 1;
-    const int grid = (int)std::min<int64_t>(total, 256 * per_cu);                  // as many as are resident, each walks its tiles
+    // As many workgroups as are resident, or whole rounds of them: a lane adds once per tile, and in a longer chain of additions the sums
+    // would round to more than those of the kernel that walks twice (chains of 16 rows and trees at 1024 x 1024).
+    const int64_t resident = 256 * per_cu, rounds = (total + kTiledChain * resident - 1) / (kTiledChain * resident);
+    const int grid = (int)std::min<int64_t>(total, rounds * resident);
     *rows = grid;
     hipLaunchKernelGGL((final_forward_loss_tiled<V, MAXO, KIND, CC>), dim3(grid), dim3(kTiledThreads), lds, s, nvox,
                        (int)tiles_per_image, (int)total, c_in, c_out, x, xsb, xsc, w, bias, target, tsb, tsc, out, osb,

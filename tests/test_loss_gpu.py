@@ -103,6 +103,26 @@ def test_fused_loss_at_the_ends_of_the_forms(batch, c_in, spatial, c_out, kind):
     check_fused_loss(batch, c_in, c_out, spatial, kind, torch.float32)
 
 
+# The parameter gradients as sums over millions of voxels, from the gradients that the pass itself wrote: a lane adds once per tile and for at most
+# 32 tiles, about 14 levels of trees stand around that, and the rows of all workgroups are added in double precision.  An addition of terms of
+# mixed sign rounds to 0.6 2^-24 of its sum (the rms of half a unit in the last place), of which n in a chain come to sqrt(n / 2).
+# 1.4: x is of one sign, so that some partial sums are larger.
+@pytest.mark.parametrize("c_in,c_out,spatial,kind", [(11, 4, (2048, 4096), "mse"), (5, 3, (4096, 4096), "l1"), (201, 2, (2048, 3000), "mse"), (402, 1, (2048, 3000), "mse")], ids=str)
+def test_fused_loss_sums_over_many_voxels(c_in, c_out, spatial, kind):
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator(device="cuda").manual_seed(c_in)
+    x = torch.rand(1, c_in, *spatial, device="cuda", generator=gen)
+    w = torch.randn(c_out, c_in, device="cuda", generator=gen) * 0.1
+    # (a target around the output: terms of mixed sign)
+    target = torch.stack([sum(w[o, c] * x[:, c] for c in range(c_in)) for o in range(c_out)], 1)
+    target += torch.randn(target.shape, device="cuda", generator=gen)
+    gw = torch.empty_like(w)
+    _, _, g = cc.final_forward_loss(x, w, None, kind, target, gw)
+    want = torch.stack([torch.stack([(x[:, c].double() * g[:, o].double()).sum() for c in range(c_in)]) for o in range(c_out)])
+    bound = 1.4 * 0.6 * 2.0 ** -24 * (32 / 2 + 14 / 2) ** 0.5
+    assert float((gw - want).norm() / want.norm()) <= bound
+
+
 # grad_input alone: planes of every remainder modulo four, of fewer voxels than four, of more than a workgroup covers, one to
 # nine outputs (more than eight go in passes); an infinite weight meets its own output only.
 @pytest.mark.parametrize("c_out", [1, 2, 3, 4, 5, 8, 9])
