@@ -828,6 +828,13 @@ hipError_t launch_tiled(int64_t batch, int c_in, int c_out, int64_t nvox, const 
 // 256 x 256 12.2 / 13.8, 17.6 / 18.2, 17.3 / 17.8, 25.4 / 26.4; 362 x 362 19.0 / 18.0, 24.1 / 22.6, 24.2 / 22.1, 35.0 / 31.0; 512 x 512
 // 25.7 / 25.2, 31.8 / 30.5, 30.8 / 30.0, 46.5 / 41.9.
 constexpr int64_t kTiledFourVoxels = 98304;
+// Three and four outputs whose targets are values: with four voxels per lane and eight channels per wave they need 134 registers, and there is one workgroup per
+// compute unit.  Up to 32 channels a wave has four of them (105 registers, two workgroups), 33 to 64 take two voxels per lane from as many voxels on,
+// and below so few that tiles of 256 leave most of the chip idle.
+// us, kernel before the pipelined one / eight channels, four voxels / these, three outputs: over 11 channels 512 x 512 30.0 / 33.6 / 24.6, 1024 x 1024 65.9 / 82.8 / 50.5,
+// 2048 x 2048 231 / 276 / 154; over 40 512 x 512 36.3 / 37.6 / 35.3, 1024 x 1024 79.9 / 94.4 / 78.0; over 64 200 x 200 24.6 / 23.1 / 24.2, 333 x 477 35.2 / 35.2 /
+// 32.4, 1024 x 1024 118 / 105 / 91; 100 x 120 20.5 / 22.0 / 20.9.
+constexpr int64_t kTiledTwoVoxels = 65536, kTiledFewVoxels = 16384;
 
 // The tiled kernel where it applies (fp32, up to 256 input and 4 output channels, 512 and 2); *handled says whether it was launched.
 hipError_t final_forward_loss_tiled_try(int kind, int64_t batch, int c_in, int c_out, int64_t nvox, const float *x,
@@ -840,8 +847,10 @@ hipError_t final_forward_loss_tiled_try(int kind, int64_t batch, int c_in, int c
     if (c_in > kTiledMaxChannels || c_out > 4 || !knob(kKnobFinalTiled, 1)) return hipSuccess;
     const int mo = c_out > 2 ? 4 : (c_out > 1 ? 2 : 1);
     // channels per wave and voxels per lane: what LDS and registers hold
-    const int cc = c_in <= 64 ? 8 : c_in <= 128 ? 16 : c_in <= 256 ? 32 : 64;
-    const int v = cc == 64 ? 1 : cc == 32 || nvox < 4 || (cc == 16 && batch * nvox < kTiledFourVoxels) ? 2 : 4;
+    const bool targets = kind != 2 && mo == 4;               // of four outputs, in registers too
+    const int cc = targets && c_in <= 32 ? 4 : c_in <= 64 ? 8 : c_in <= 128 ? 16 : c_in <= 256 ? 32 : 64;
+    const int v = cc == 64 ? 1 : cc == 32 || nvox < 4 || (cc == 16 && batch * nvox < kTiledFourVoxels) ||
+                  (cc == 8 && targets && (batch * nvox >= kTiledTwoVoxels || batch * nvox < kTiledFewVoxels)) ? 2 : 4;
     if (nvox < v || (cc == 64 && mo > 2)) return hipSuccess;
 #define MSD_TILED(VV, OO, KK, CCC)                                                                                    \
     return (*handled = true, launch_tiled<VV, OO, KK, CCC>(batch, c_in, c_out, nvox, x, xsb, xsc, w, bias, target, tsb, \
@@ -861,6 +870,10 @@ hipError_t final_forward_loss_tiled_try(int kind, int64_t batch, int c_in, int c
         MSD_TILED_O(2, 32);
     } else if (cc == 16) {
         if (v == 4) MSD_TILED_O(4, 16); else MSD_TILED_O(2, 16);
+    } else if (cc == 4) {
+        if (v == 4 && kind == 0) MSD_TILED(4, 4, 0, 4);
+        if (v == 4) MSD_TILED(4, 4, 1, 4);
+        if (kind == 0) MSD_TILED(2, 4, 0, 4); else MSD_TILED(2, 4, 1, 4);
     } else {
         if (v == 4) MSD_TILED_O(4, 8); else MSD_TILED_O(2, 8);
     }

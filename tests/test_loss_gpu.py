@@ -103,6 +103,17 @@ def test_fused_loss_at_the_ends_of_the_forms(batch, c_in, spatial, c_out, kind):
     check_fused_loss(batch, c_in, c_out, spatial, kind, torch.float32)
 
 
+# Three and four outputs with targets that are values: four channels per wave up to 32 channels, above them two voxels per lane from 65536 voxels
+# on and below 16384; just below and above, planes that are no whole groups of the lanes' voxels, fewer than four voxels, waves without a channel.
+@pytest.mark.parametrize("kind", ["mse", "l1"])
+@pytest.mark.parametrize("c_out", [3, 4])
+@pytest.mark.parametrize("batch,c_in,spatial", [
+    (3, 1, (1, 3)), (1, 5, (37, 53)), (9, 7, (1, 2)), (2, 25, (300, 301)), (1, 32, (255, 257)), (1, 32, (700, 300)), (1, 33, (255, 257)), (1, 33, (257, 255)),
+    (1, 40, (256, 256)), (1, 40, (128, 128)), (1, 41, (127, 129)), (2, 64, (181, 183)), (4, 57, (3, 43))], ids=str)
+def test_fused_loss_of_three_and_four_outputs_with_values(batch, c_in, spatial, c_out, kind):
+    check_fused_loss(batch, c_in, c_out, spatial, kind, torch.float32)
+
+
 # The parameter gradients as sums over millions of voxels, from the gradients that the pass itself wrote: a lane adds once per tile and for at most
 # 32 tiles, about 14 levels of trees stand around that, and the rows of all workgroups are added in double precision.  An addition of terms of
 # mixed sign rounds to 0.6 2^-24 of its sum (the rms of half a unit in the last place), of which n in a chain come to sqrt(n / 2).
