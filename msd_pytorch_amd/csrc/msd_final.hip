@@ -836,6 +836,9 @@ constexpr int64_t kTiledFourVoxels = 98304;
 // 32.4, 1024 x 1024 118 / 105 / 91; 100 x 120 20.5 / 22.0 / 20.9.
 constexpr int64_t kTiledTwoVoxels = 65536, kTiledFewVoxels = 16384;
 
+// Voxels of a plane whose byte offsets fit the 32 bits that the tiled kernel's loads take beside a channel's base.
+constexpr int64_t kTiledMaxVoxels = (int64_t)1 << 30;
+
 // The tiled kernel where it applies (fp32, up to 256 input and 4 output channels, 512 and 2); *handled says whether it was launched.
 hipError_t final_forward_loss_tiled_try(int kind, int64_t batch, int c_in, int c_out, int64_t nvox, const float *x,
                                         int64_t xsb, int64_t xsc, const float *w, const float *bias,
@@ -844,7 +847,7 @@ hipError_t final_forward_loss_tiled_try(int kind, int64_t batch, int c_in, int c
                                         float *ws, int64_t *rows, hipStream_t s, bool *handled)
 {
     *handled = false;
-    if (c_in > kTiledMaxChannels || c_out > 4 || !knob(kKnobFinalTiled, 1)) return hipSuccess;
+    if (c_in > kTiledMaxChannels || c_out > 4 || nvox > kTiledMaxVoxels || !knob(kKnobFinalTiled, 1)) return hipSuccess;
     const int mo = c_out > 2 ? 4 : (c_out > 1 ? 2 : 1);
     // channels per wave and voxels per lane: what LDS and registers hold
     const bool targets = kind != 2 && mo == 4;               // of four outputs, in registers too

@@ -134,6 +134,29 @@ def test_fused_loss_sums_over_many_voxels(c_in, c_out, spatial, kind):
     assert float((gw - want).norm() / want.norm()) <= bound
 
 
+# A plane of more than 2^30 voxels, whose byte offsets need more than 32 bits (one plane stands for all channels): the kernel that walks twice.
+@pytest.mark.parametrize("c_in", [3, 129])
+def test_fused_loss_of_a_plane_of_more_than_four_gigabytes(c_in):
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator(device="cuda").manual_seed(c_in)
+    x = torch.rand(1, 1, 2, (1 << 29) + 1000, device="cuda", generator=gen)
+    w, b = torch.rand(1, c_in, device="cuda", generator=gen), torch.rand(1, device="cuda", generator=gen)
+    target = torch.zeros_like(x)
+    gw = torch.empty_like(w)
+    out, loss, g = cc.final_forward_loss(x.expand(-1, c_in, -1, -1), w, b, "mse", target, gw)
+    scale, n = w.double().sum(), x.numel()
+    for part in (slice(0, 1000), slice(-5000, None)):
+        want = scale * x.view(-1)[part].double() + b.double()
+        assert rel_err(out.view(-1)[part], want) <= 1e-5
+        assert rel_err(g.view(-1)[part], 2 * want / n) <= 1e-5
+    squares = sums = 0.
+    for xs in x.view(-1).split(1 << 27):
+        want = scale * xs.double() + b.double()
+        squares, sums = squares + float((want ** 2).sum()), sums + float((want * xs).sum())
+    assert abs(loss.item() - squares / n) <= 1e-5 * squares / n
+    assert float((gw.double() - 2 * sums / n).abs().max()) <= 1e-4 * 2 * sums / n
+
+
 # grad_input alone: planes of every remainder modulo four, of fewer voxels than four, of more than a workgroup covers, one to
 # nine outputs (more than eight go in passes); an infinite weight meets its own output only.
 @pytest.mark.parametrize("c_out", [1, 2, 3, 4, 5, 8, 9])
