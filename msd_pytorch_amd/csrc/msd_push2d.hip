@@ -220,8 +220,10 @@ __global__ __launch_bounds__(kMaxWaves *kWave) void push_rows(PushArgs a, const 
 // A workgroup has one slab, so that the weights of 256 channels lie in LDS at a time: with both slabs in one it were 128, and to load them
 // anew for every segment took 260 of the 1400 us over 131 channels.  Without them x is read through the L2 twice, which costs nothing
 // measurable.  2048 x 2048, 14 outputs, us, both slabs in a workgroup / one: over 16 / 58 / 100 / 128 channels 559 / 553, 743 / 730, 918 / 890, 939 / 904, over
-// 142 / 184 1390 / 1064, 1579 / 1247.  Above 256 the steps of one segment go up and the next one's down, so that a part of the table is
-// loaded once less per segment: over 268 / 324 / 380 2025 / 1914, 2250 / 2068, 2719 / 2449.  (x by way of a transposition in LDS instead of in the operands' own layout: the same times.)
+// 142 / 184 1390 / 1064, 1579 / 1247.  Above 256 the steps of one segment of a row go up and the next one's down, so that a part of the table is
+// loaded once less per segment: over 268 / 324 / 380 2025 / 1914, 2250 / 2068, 2719 / 2449.  Every row (or part of one) begins upwards: the order in which a
+// voxel's channels are added goes with its place in the row, as the sign does that its values are taken with, and not with the row or the image of a
+// batch (rows of an odd number of segments load one part more; the times are the same).  (x by way of a transposition in LDS instead of in the operands' own layout: the same times.)
 //
 // Bound by latencies: eight waves per compute unit (their registers), each a chain of loads, split and matrix
 // instructions; the matrix part is a quarter of the time.  With a workgroup per row, its waves
@@ -342,10 +344,10 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
         load_weights(0, steps);
         __syncthreads();
     }
-    // (workgroups whose table does not hold all weights meet at each part of it: all their waves take as many segments)
-    const int most = (a.length + 2 * kHalo + kWave - 1) / kWave;
-    // (else one segment's steps go up, the next one's down: the part of the table that the one ends with is the other's first)
-    bool up = true;
+    // (workgroups whose table does not hold all weights meet at each part of it: all their waves take as many segments, of a row without
+    // parts no more than it has)
+    const int most = ((a.parts > 1 ? a.length + 2 * kHalo : a.W) + kWave - 1) / kWave;
+    bool up;                                      // the segment's steps go up: the part of the table that one ends with is the next one's first
     int loaded = -1;
     const int stride = pairs * kPushWaves;
     int it = pair * kPushWaves + wave;
@@ -358,6 +360,7 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int t = 0; t < kTiles; t++) before[j][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        up = true;
         const int segs = resident ? (here.end - here.start + kWave - 1) / kWave : most;
         for (int seg = 0; seg < segs; seg++) {
             const int first = here.start + seg * kWave;
@@ -402,7 +405,7 @@ __global__ __launch_bounds__(kPushWaves *kWave, 2) void push_split(const SplitAr
                 }
                 __builtin_amdgcn_sched_barrier(0);    // (the scheduler would move the loads to where they are used)
                 const bool more = i + 1 < steps, row = more || seg + 1 < segs;
-                request(image_of(row ? here : next), more ? first : row ? first + kWave : next.start, more ? (up ? step + 1 : step - 1) : resident ? 0 : step);
+                request(image_of(row ? here : next), more ? first : row ? first + kWave : next.start, more ? (up ? step + 1 : step - 1) : resident || !row ? 0 : step);
                 __builtin_amdgcn_sched_barrier(0);
                 if (real) {
                     const bf16x8_t *const wt = weights + (resident ? step : step % kTableSteps) * kStepEntries + id;

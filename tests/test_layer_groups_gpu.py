@@ -415,6 +415,22 @@ def test_forward_groups_of_fourteen_over_many_channels(case):
         check_block(2, size, c_in, width, depth, batch, dilations=dilations, seed=67)
 
 
+# Where the weights of a pass are loaded in parts, the order of the additions changes from segment to segment of a row, but the same rows
+# give the same bits at every place of a batch: more rows than there are waves, of an odd and an even number of segments.
+@pytest.mark.parametrize("width", [100, 150])
+@pytest.mark.parametrize("c_in", [200, 260])
+def test_the_place_in_a_batch_does_not_change_a_forward_group(c_in, width):
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator().manual_seed(97)
+    depth = 9
+    stack = torch.empty(5, c_in + depth, 300, width, device="cuda")
+    stack[:, :c_in] = torch.randn(c_in, 300, width, generator=gen).cuda()
+    weights = [(torch.randn(1, c_in + i, 3, 3, generator=gen) * 0.05).cuda() for i in range(depth)]
+    with tuning({"fwd.group": 1024}):
+        cc.block_forward(stack, c_in, [1 + i % 4 for i in range(depth)], torch.zeros(depth, device="cuda"), weights)
+    assert all(torch.equal(image, stack[0]) for image in stack[1:])
+
+
 @pytest.mark.parametrize("where", ["input", "weight"])
 @pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
 def test_values_without_bf16_parts_in_front_of_a_forward_group(where, value):
