@@ -330,6 +330,50 @@ def test_values_without_bf16_parts(where, value, depth):
     assert float(((a - b).abs() / a.abs().clamp_min(1e-30)).max()) <= 1e-4
 
 
+# The same where a workgroup walks several tiles and only one or two of them, not the first (in either buffer) holds such a value, so that some of its units are
+# left to the second run and some are not: passes over one to four blocks of channels of two slabs and of one, over five and six (all waves alike), one slab in a
+# large image, volumes with and without gaps.  The rest of all gradients is compared as well: grad_input is added to in place, by one run or the other.
+@pytest.mark.parametrize("where", ["stack", "gradient", "weight"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
+@pytest.mark.parametrize("size, gap, c_in, depth, at", [
+    ((160, 320), 0, 4, 14, 0.4), ((160, 321), 0, 20, 14, 0.9), ((160, 320), 0, 40, 14, 0.7), ((320, 330), 3, 60, 14, 0.35), ((400, 320), 0, 80, 14, 0.3),
+    ((400, 320), 0, 90, 9, 0.9), ((320, 320), 0, 10, 6, 0.4), ((320, 320), 0, 30, 6, 0.7), ((320, 333), 0, 50, 6, 0.6), ((650, 1000), 0, 40, 2, 0.5),
+    ((16, 40, 65), 0, 10, 4, 0.4), ((16, 40, 65), 0, 30, 4, 0.7), ((16, 40, 65), 0, 50, 4, 0.8), ((16, 50, 65), 3, 50, 4, 0.4), ((32, 60, 65), 0, 70, 4, 0.6),
+    ((32, 60, 65), 2, 70, 3, 0.3), ((20, 60, 65), 0, 20, 2, 0.6), ((30, 60, 65), 1, 40, 2, 0.5)],
+    ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_values_without_bf16_parts_in_some_tiles(size, gap, c_in, depth, at, value, where):
+    from msd_pytorch_amd import msd_custom_convolutions as cc
+    gen = torch.Generator(device="cuda").manual_seed(31)
+    taps = [3] * len(size)
+
+    def some(scale, least):
+        big = torch.rand(1, c_in + depth, *size[:-1], size[-1] + gap, device="cuda", generator=gen)
+        return (big * scale + least)[..., :size[-1]]
+
+    stack, gradient = some(1, 0.1), some(1e-3, 0)              # every ReLU open
+    weights = [torch.rand(1, c_in + i, *taps, device="cuda", generator=gen) * 1e-3 + 1e-4 for i in range(depth)]
+    voxel = [int(at * n) for n in size[:-1]] + [size[-1] // 2]
+    if where == "stack":
+        stack[(0, c_in // 2, *voxel)] = value
+    elif where == "gradient":
+        gradient[(0, c_in, *voxel)] = value          # (the lowest layer: it stays where it is)
+    else:
+        weights[depth - 1][(0, c_in - 1, *[1] * len(size))] = value
+    found = []
+    for setting in (0, 1):
+        grads = torch.empty_strided(gradient.shape, gradient.stride(), device="cuda").copy_(gradient)
+        gk, gb = [torch.zeros_like(w) for w in weights], torch.zeros(depth, device="cuda")
+        with tuning({"bwd.group": setting}):
+            cc.block_backward(stack, grads, c_in, [1 + i % 4 for i in range(depth)], weights, gk, gb, True)
+        found.append(torch.cat([grads[:, :c_in].flatten(), gb, *(k.flatten() for k in gk)]))
+    assert same_specials(found[1], found[0])
+    finite = torch.isfinite(found[0])
+    assert bool(finite.any())
+    # (sums of terms of one sign: chains of at most some thousand additions, relative to the largest)
+    a, b = found[0][finite].double(), found[1][finite].double()
+    assert float(((a - b).abs() / a.abs().clamp_min(1e-30)).max()) <= 1e-4
+
+
 def test_an_infinity_meets_its_own_voxels_only():
     """The last tile of a row repeats voxels of the one before (here 8 to 31): what they hold counts once."""
     from msd_pytorch_amd import msd_custom_convolutions as cc
