@@ -1,4 +1,4 @@
-// pull_rows_wide: pull_rows (msd_pull.hip, which includes this where its own helpers are declared) with eight waves that all gather and then all
+// pull_rows_wide: pull_rows (msd_pull.hip) with eight waves that all gather and then all
 // multiply: two slabs over five to eight blocks of 16 channels, of which every wave has one, and one slab over three and four, of which
 // every wave has half of one, in large images.
 //
@@ -8,6 +8,8 @@
 // would need two blocks each, for which there are no registers (1024 x 1024, 14 outputs over 87 channels: 430 us; three kinds of waves with two blocks and
 // registers spilt 528; these eight waves with the gather and the products of pull_rows 442).
 #pragma once
+
+#include "msd_pull_common.h"
 
 namespace msd {
 namespace group2d {
@@ -69,38 +71,8 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
     bf16x8_t(&w)[kSteps][3] = state.w;
     f32x4_t(&sums)[kTiles] = state.sums;
 
-    struct Tile {
-        int first;                                // segment of its image
-        int64_t img, gimg;                        // byte offsets of the image, of the outputs' gradients
-        uint32_t sign;                            // of x in this tile
-    };
-    struct Place {
-        int x0, skip, y, z;                       // first voxel, voxels that belong to the segment before, row, slice
-        bool valid;
-    };
-    // (past the last tile that one again)
-    auto tile_of = [&](int tile) {
-        Tile t;
-        const int it0 = min(tile, a.tiles - 1), it = a.reverse ? a.tiles - 1 - it0 : it0;
-        const int b = a.by_tiles.of(it);
-        t.first = (it - b * a.image_tiles) * kSegs;
-        t.img = (int64_t)b * a.sb * 4;
-        t.gimg = (int64_t)b * a.gsb * 4;
-        t.sign = (uint32_t)it << 31;
-        return t;
-    };
-    auto locate = [&](const Tile &t, int segment) {
-        Place p;
-        p.valid = t.first + segment < a.items;
-        const int it = min(t.first + segment, a.items - 1);
-        p.y = a.by_segs.of(it);
-        const int own0 = (it - p.y * a.segs) * kSegment;
-        p.z = N == kVolume ? a.by_rows.of(p.y) : 0;
-        p.y -= N == kVolume ? p.z * a.H : 0;
-        p.x0 = min(own0, a.span - kSegment);         // (the last segment of a row overlaps the one before)
-        p.skip = p.valid ? own0 - p.x0 : kSegment;
-        return p;
-    };
+    auto tile_of = [&](int tile) { return tile_at<kSegs>(a, tile); };
+    auto locate = [&](const Tile &t, int segment) { return place_at<N>(a, t, segment); };
     const uint32_t plane = (uint32_t)a.sc * 4u;
     auto row_at = [&](int z, int y) { return (Gather<N>::kIsVolume ? z * (int)a.sz : 0) + y * (int)a.sy; };
 
@@ -111,11 +83,6 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
     const int lv = lane % kLanes, lc = lane / kLanes;               // voxels 4 lv .., channels lc + kRows4 i
     constexpr int kChannels = kWave / kLanes;     // channels of one access
     const uint32_t lane_plane = (uint32_t)lc * plane;
-    struct Unit {
-        int64_t img;                              // byte offset of the image
-        uint32_t at;                              // the lane's of (row, voxel)
-        int skip;                                 // first of its four voxels that is its segment's own (0: all, 4: none)
-    };
     auto unit_of = [&](const Tile &t, int u) {
         const int first = ((wave % P) * kUnits + u) * (kUnit / kSegment);
         const Place p0 = locate(t, first), p1 = locate(t, first + kUnit / kSegment - 1);
@@ -127,20 +94,7 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
         un.skip = min(max((sel ? p1.skip : p0.skip) - v4, 0), 4);
         return un;
     };
-    // channels from `limit` on: that channel before it again
-    auto request = [&](const float *from, int limit, const Unit &un, f32x4_t (&d)[kVec]) {
-        uint64_t base = reinterpret_cast<uint64_t>(from) + (uint64_t)un.img + (uint64_t)min(ch0, limit - 1) * plane;
-        asm volatile("" : "+s"(base));           // (scalar base, 32-bit lane offsets)
-        const uint32_t last = (uint32_t)min(max(limit - 1 - ch0, 0), 15) * plane;
-        uint32_t at = lane_plane;
-        asm volatile("" : "+v"(at));             // (nothing of this is kept over the tiles)
-#pragma unroll
-        for (int i = 0; i < kVec; i++) {
-            float v4[4];
-            load_global_vec_unaligned<4>(base, min(at + (uint32_t)(kChannels * i) * plane, last) + un.at, v4);
-            d[i] = f32x4_t{v4[0], v4[1], v4[2], v4[3]};
-        }
-    };
+    auto request = [&](const float *from, int limit, const Unit &un, f32x4_t (&d)[kVec]) { request_unit(from, ch0, limit, plane, lane_plane, un, d); };
     f32x4_t xs[kVec], gs[kVec];
     auto request_g = [&](const Unit &un) {
         if constexpr (FRESH) {
@@ -265,28 +219,13 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
         for (int j = 0; j < kLaneOut; j++)
 #pragma unroll
             for (int t = 0; t < kTaps; t++) val[j][t / 3][t % 3] *= factor;
-        // rows m of the lane (slot_of), eight at a time
-        auto eight = [&](int i, float (&e8)[8]) {
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const int s = 8 * i + e;
-                if (s < 27) {
-                    e8[e] = val[s / kTaps][s % kTaps / 3][s % 3];
-                } else if constexpr (N != kImage) {
-                    e8[e] = 0.f;
-                } else {
-                    const int t0 = s - 27, t1 = s - 22;
-                    e8[e] = h ? (t1 < kTaps ? val[3][t1 / 3 % 3][t1 % 3] : 0.f) : val[3][t0 / 3][t0 % 3];
-                }
-            }
-        };
         char *const at = A + (segment * G + slab) * kSlabBytes + v * kVoxelBytes;
         const uint32_t piece = 16 * (4 * (uint32_t)h ^ turn((uint32_t)v));
         float bad = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             float e8[8];
-            eight(i, e8);
+            eight_rows<N>(val, h, i, e8);
             Split8 s;
             if constexpr (WHOLE) {
                 float scaled[8];
@@ -309,14 +248,6 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
     // channels at once (loaded in that form, 64 bytes of 16 channels at a time, memory gives 2.6 to 3.0 TB/s instead of 4).
     constexpr int kXRow = 2 * kUnit + 16, kDRow = 4 * kUnit + 16;   // bytes of a channel (16 apart in the banks)
     const int first_seg = (wave % P) * kUnits * (kUnit / kSegment); // of the wave's first unit
-    auto clear_skipped = [&](const Unit &un) {    // an infinity there belongs to the other segment
-        if (__any(un.skip > 0)) {
-#pragma unroll
-            for (int i = 0; i < kVec; i++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) xs[i][e] = e >= un.skip ? xs[i][e] : 0.f;
-        }
-    };
     // bit 4 i + e: the channel's gradient at voxel e is kept
     auto mask_of = [&]() {
         uint32_t bits = 0xffffu;
@@ -410,7 +341,7 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
                 to[p] = *reinterpret_cast<const bf16x8_t *>(vox + (s / 2 * G + i / 2) * kSlabBytes + p * kPartBytes +
                                                             s % 2 * 16 * kVoxelBytes + (vox_piece ^ (uint32_t)(i % 2 * 64)));
         };
-        clear_skipped(un);
+        clear_skipped(un, xs);
         const uint32_t bits = mask_of();
         const float rest = put_x(sign_bit);
         const bool done = split && !__any(taken_whole(rest));       // uniform
@@ -520,7 +451,7 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
     // lie whole in the place of their parts).
     auto compute_whole = [&](int u, uint32_t sign_bit, const Unit &un) {
         const float sign = __uint_as_float(sign_bit | 0x3f800000u);
-        clear_skipped(un);
+        clear_skipped(un, xs);
         const uint32_t bits = mask_of();
         uint32_t ll = (uint32_t)lane;
         asm volatile("" : "+v"(ll));
@@ -572,31 +503,7 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
         }
         own_sync();
     };
-    auto store = [&](const Unit &un, bool all) {
-        // Buffer stores, whose lanes past the end of the buffer store nothing: there is no branch around
-        // them.  (Loads and stores retire through one in-order counter, and a store that may be skipped turns the
-        // wait for the next unit's values, requested before it, into one for the store itself.)
-        const uint64_t base = reinterpret_cast<uint64_t>(gx) + (uint64_t)un.img + (uint64_t)ch0 * plane;
-        uint32_t at = lane_plane;
-        asm volatile("" : "+v"(at));
-        const int end = un.skip == 0 && all ? a.update - ch0 : 0;
-        const __amdgpu_buffer_rsrc_t buffer = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(base), 0, 0xfffffff0u, 0x00020000);
-#pragma unroll
-        for (int i = 0; i < kVec; i++) {
-            typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-            const uint32_t plane_at = at + (uint32_t)(kChannels * i) * plane;
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, gs[i]), buffer,
-                                                   lc + kChannels * i < end ? plane_at + un.at : 0xffffffffu, 0, 0);
-        }
-        if (__any(un.skip % 4 != 0)) {            // some lanes own the last of their four voxels only
-#pragma unroll
-            for (int i = 0; i < kVec; i++)
-#pragma unroll
-                for (int e = 1; e < 4; e++)
-                    if (all && lc + kChannels * i < a.update - ch0 && un.skip > 0 && e >= un.skip)
-                        reinterpret_cast<__attribute__((address_space(1))) float *>(base + (uint64_t)(lane_plane + (uint32_t)(kChannels * i) * plane) + un.at)[e] = gs[i][e];
-        }
-    };
+    auto store = [&](const Unit &un, bool all) { store_unit(gx, ch0, a.update, plane, lane_plane, lc, un, gs, all); };
     // values of the tile at hand that can be split: A and the weights
     auto tile_split = [&]() {
         int bad = 0;
@@ -620,7 +527,7 @@ __device__ __forceinline__ bool wide_tiles(const PullArgs &a, const float *__res
                     const Unit un = unit_of(t, u);
                     request(x, a.C, un, xs);
                     request_g(un);
-                    clear_skipped(un);
+                    clear_skipped(un, xs);
                     const float rest = put_x(t.sign);
                     if (split && !__any(taken_whole(rest))) continue;    // (the first run has done it)
                     compute_whole(u, t.sign, un);
