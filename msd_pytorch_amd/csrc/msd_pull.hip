@@ -114,16 +114,24 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
     // Sums are added to a second level every so many tiles: a chain of n additions of terms of mixed sign rounds to about sqrt(n / 2)
     // 2^-24 of what it comes to.  Errors of the weight gradients against 64 bits (2-norm), a chain over all tiles / in two levels: 192^3,
     // four outputs over 30 / 46 channels 6.7 / 2.1, 6.8 / 2.0 e-7; 2048 x 2048, 14 outputs over 40 4.3 / 1.4; 1024 x 1024 2.2 / 1.1; 333 x 477
-    // 0.96 / 0.71.  Times are the same within 2 % (the branch in the loop over the tiles instead of around it: up to 6 % more).
+    // 0.96 / 0.71.  Times are the same
+    // within 2 %.  (With a branch in the loop over the tiles instead of around it, or with the second level cleared before the loop and added behind the second run, 3 to 6 % more over
+    // 33 to 64 channels: the compiler then orders the loops of all kinds of waves otherwise.)
     constexpr int kChain = 16;                    // additions
     const int chain = wgs * (kChain / kUnits), bias_chain = wgs * kChain * (N != kImage ? 4 : 1);      // tiles, of all workgroups
-    auto second_level = [&]() {                   // of a kernel worker
+    bool two_levels = false;
+    auto second_level = [&](bool back) {          // of a kernel worker; back: all of it is in the registers again
         char *const at = lds + S::kSumsAt + number * S::kSumBytes + lane * 16;
 #pragma unroll
         for (int t = 0; t < kTiles; t++) {
-            *reinterpret_cast<f32x4_t *>(at + t * kWave * 16) += state.sums(t);
-            state.sums(t) = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            f32x4_t &sum = *reinterpret_cast<f32x4_t *>(at + t * kWave * 16);
+            if (two_levels) state.sums(t) += sum;             // uniform
+            if (!back) {
+                sum = state.sums(t);
+                state.sums(t) = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            }
         }
+        two_levels = true;
     };
 
     auto tile_of = [&](int tile) { return tile_at<kSegs>(a, tile); };
@@ -547,7 +555,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
 #pragma unroll 1
         for (int tile = lb, count = 0; tile < a.tiles; tile += wgs, count += kUnits) {
             const Tile t = tile_of(tile);
-            if (kernel && count % kChain == 0) second_level();      // uniform
+            if (kernel && count > 0 && count % kChain == 0) second_level(false);   // uniform
             if (kind == kGatherer) {
                 const Voxel here = locate_pair(t);
                 gather(t, here);
@@ -572,6 +580,7 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
             }
             __syncthreads();
         }
+        if (kernel && two_levels) second_level(true);
         return false;
     } else if (kind == kGatherer) {
         // A tile is formed in the one buffer while the workers have the other; a barrier, and they change.
@@ -615,8 +624,9 @@ __device__ __forceinline__ bool pull_tiles(const PullArgs &a, const float *__res
                 turn_over();
                 lds_sync();
             }
-            second_level();
+            if (tile < a.tiles) second_level(false);
         }
+        if (two_levels) second_level(true);
         return again;
     } else {
         bool again = false;
@@ -695,11 +705,6 @@ __global__ __launch_bounds__(kPullThreads, 3) void pull_rows(const PullArgs a, c
     state.weights_split = true;
 #pragma unroll
     for (f32x4_t &v : state.kept) v = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    char *const sums2 = lds + S::kSumsAt + number * S::kSumBytes + lane * 16;      // a kernel worker's, second level
-    if (kind == kKernel) {
-#pragma unroll
-        for (int t = 0; t < kTiles; t++) *reinterpret_cast<f32x4_t *>(sums2 + t * kWave * 16) = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
     load_weights(false);
     __syncthreads();
 
@@ -716,10 +721,6 @@ __global__ __launch_bounds__(kPullThreads, 3) void pull_rows(const PullArgs a, c
 
     // the sums, of the waves that share a block through LDS
     constexpr int kBlock = 1024 * G;              // sums of a block of channels
-    if (kind == kKernel) {
-#pragma unroll
-        for (int t = 0; t < kTiles; t++) state.sums(t) += *reinterpret_cast<const f32x4_t *>(sums2 + t * kWave * 16);
-    }
     if constexpr (P == 1) {
         if (kind == kKernel && cb < blocks) {
 #pragma unroll
