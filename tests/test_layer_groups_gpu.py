@@ -187,11 +187,13 @@ def test_weight_gradients_over_many_voxels(size, c_in, outputs, workers):
     assert float((got - want).norm() / want.norm()) <= bound
 
 
-# One slab of outputs over three and four blocks: from 20000 segments of 32 voxels on (volumes 50000) the eight waves that gather and multiply in
-# turn.  Just below and just above, rows that end inside a segment, rows with gaps, two images, a block without its last channels and
+# One slab of outputs over three and four blocks: from 20000 segments of 32 voxels on (volumes 50000, 25000 with chunks side by side) for each 256
+# workgroups of a chunk the eight waves that gather and multiply in turn.  Just below and just above, rows that end inside a segment, rows with gaps, two images, a block without its last channels and
 # a chunk of two blocks beside one of three; against the layers on their own.
 @pytest.mark.parametrize("size, batch, c_in, gap, wide", [
     ((799, 800), 1, 40, 0, False), ((801, 799), 1, 40, 0, True), ((400, 830), 2, 62, 3, True), ((801, 800), 1, 75, 0, True),
+    ((595, 640), 1, 75, 0, False), ((605, 640), 1, 75, 0, True), ((400, 520), 1, 130, 0, True),
+    ((78, 76, 80), 1, 70, 0, False), ((80, 77, 80), 1, 70, 0, True), ((80, 100, 60), 1, 65, 1, True),
     ((801, 798), 1, 31, 0, False), ((100, 160, 99), 1, 47, 0, False), ((100, 161, 101), 1, 47, 0, True), ((100, 125, 99), 1, 33, 1, True),
     ((50, 124, 100), 2, 33, 1, False)], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_one_slab_over_three_and_four_blocks(size, batch, c_in, gap, wide):
