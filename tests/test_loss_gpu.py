@@ -42,7 +42,7 @@ CASES = [
     (2, 6, 4, (3, 5, 7)),
     (1, 5, 8, (9, 11)),
     (1, 9, 2, (8, 12)),
-    # more than 64 and more than 128 input channels (sixteen channels per wave; the walk-twice kernel),
+    # more than 64 and more than 128 input channels (sixteen and 32 channels per wave),
     # several tiles per workgroup and a ragged last tile
     (1, 70, 4, (24, 50)),
     (2, 101, 4, (130, 258)),
@@ -61,16 +61,15 @@ def test_fused_loss_matches_torch(batch, c_in, c_out, spatial, kind, dtype):
     check_fused_loss(batch, c_in, c_out, spatial, kind, dtype)
 
 
-# One small case per compiled form of the single-read kernel: voxels per lane (4: plane size a
-# multiple of four and at most 64 channels; 2: even planes otherwise; 1: odd planes) x channels
-# per wave and pass (8 up to 64 channels, 16 above) x output channels (1, 2, 3 or 4) x loss.
+# Small planes through the single-read kernel, in whole groups of a lane's voxels and not (four voxels up to 64 channels, two
+# above), eight and sixteen channels per wave (four with three outputs whose targets are values) x output channels x loss.
 SINGLE_READ_FORMS = [
     # (c_in, spatial)
-    (20, (8, 16)),      # 4 voxels, 8 channels
-    (20, (6, 7)),       # 2 voxels, 8 channels
-    (20, (5, 7)),       # 1 voxel,  8 channels
-    (70, (6, 8)),       # 2 voxels, 16 channels
-    (70, (5, 7)),       # 1 voxel,  16 channels
+    (20, (8, 16)),      # 4 voxels, 4 or 8 channels: whole groups
+    (20, (6, 7)),       # a remainder of two
+    (20, (5, 7)),       # a remainder of three
+    (70, (6, 8)),       # 2 voxels, 16 channels: whole groups
+    (70, (5, 7)),       # a remainder of one
 ]
 
 
