@@ -341,7 +341,8 @@ def test_values_without_bf16_parts(where, value, depth):
     ((160, 320), 0, 4, 14, 0.4), ((160, 321), 0, 20, 14, 0.9), ((160, 320), 0, 40, 14, 0.7), ((320, 330), 3, 60, 14, 0.35), ((400, 320), 0, 80, 14, 0.3),
     ((400, 320), 0, 90, 9, 0.9), ((320, 320), 0, 10, 6, 0.4), ((320, 320), 0, 30, 6, 0.7), ((320, 333), 0, 50, 6, 0.6), ((650, 1000), 0, 40, 2, 0.5),
     ((16, 40, 65), 0, 10, 4, 0.4), ((16, 40, 65), 0, 30, 4, 0.7), ((16, 40, 65), 0, 50, 4, 0.8), ((16, 50, 65), 3, 50, 4, 0.4), ((32, 60, 65), 0, 70, 4, 0.6),
-    ((32, 60, 65), 2, 70, 3, 0.3), ((20, 60, 65), 0, 20, 2, 0.6), ((30, 60, 65), 1, 40, 2, 0.5)],
+    ((32, 60, 65), 2, 70, 3, 0.3), ((20, 60, 65), 0, 20, 2, 0.6), ((30, 60, 65), 1, 40, 2, 0.5),
+    ((30, 60, 65), 1, 20, 2, 0.7)],
     ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_values_without_bf16_parts_in_some_tiles(size, gap, c_in, depth, at, value, where):
     from msd_pytorch_amd import msd_custom_convolutions as cc
