@@ -1499,9 +1499,11 @@ constexpr int64_t kGroupChannels = 12, kGroupChannelsWide = 6;
 // Up to fourteen outputs instead of seven where the channels in front are at least this many voxels in all.  The pass
 // then moves them once and not twice (two channels per layer: 2.3 times, since sevens take six outputs), but the
 // upper layers of the group find up to 13 channels to add, and passes of seven have twice the waves.  Push and finish of
-// 14 outputs, us, sevens and fourteens (over 180 before a pass had the weights of 256 channels in LDS, now some 60 less): two channels per layer 1024 x 1024 over 60: 323, 339; over 180: 707, 613;
-// 2048 x 2048 over 24: 967, 959; over 60: 1426, 1185; over 120: 2180, 1663; one channel 1536 x 1536 over 80: 928, 913;
-// 2048 x 2048 over 45: 1127, 1253; over 90: 1657, 1507.
+// 14 outputs, us, sevens and fourteens: two channels per layer 1024 x 1024 over 45: 275, 258; over 64: 341, 268; over 180: 709, 450; 1448 x 1448 over 45: 530, 553;
+// over 64: 634, 559; 2048 x 2048 over 24: 789, 870; over 45: 1055, 968; over 120: 1961, 1348; one channel 1024 x 1024 over 45: 255, 294; over 90: 359, 340; over
+// 180: 563, 474; 1448 x 1448 over 90: 702, 725; over 120: 812, 817; over 140: 977, 908; 1536 x 1536 over 90: 824, 776; over 140: 1166, 979; 2048 x 2048
+// over 45: 948, 1088; over 64: 1110, 1157; over 90: 1358, 1284.  (The lines are those of passes with the weights of 128 channels in LDS; with 256, 1024 x 1024 would gain from 90
+// channels on, 1536 x 1536 from 64, while 2048 x 2048 over 64, on the line, loses 4 %.)
 // From 64 channels on two channels per layer gain from half as many voxels on.  Forward pass of a whole block of two channels per layer, ms, line at 2^27
 // / 2^26 from 64 channels on / 2^26 throughout: depth 100, 1024 x 1024 4.97 / 4.81 / 4.75, 1000 x 1001 5.10 / 4.85 / 4.87; depth 60, 4 x 512 x 512
 // 2.39 / 2.28 / 2.27, 1448 x 1448 4.72 / 4.68 / 4.79.

@@ -350,11 +350,11 @@ __global__ __launch_bounds__(kFinalThreads) void final_forward_loss_kernel(
 // workgroup (tile t, t + grid, ...) and are reduced over the lanes once at the end: one row
 // of partial sums per workgroup.  Same columns of `part` as the kernel above.
 //
-// Bound by memory where tiles are many (128^3, 51 channels, one output: 5.3 TB/s), else by the chain of a tile: first walk, LDS, loss,
+// Bound by memory where tiles are many (128^3, 51 channels, one output: 92 us, 4.7 TB/s), else by the chain of a tile: first walk, LDS, loss,
 // LDS, second walk, beside which only the next tile's loads run.  Requested before the walk and not in the tile before, with scalar loads of the
 // weights between the channels (a round trip each), two voxels per lane above 64 channels and both walks reading memory
-// above 128, us: 1024 x 1024, 101 channels, four labels 182 -> 115; 4 x 512 x 512, 101, one output 110 -> 91; 3 x 333 x 477, 35, three labels
-// 42 -> 32; 1024 x 1024, 201 / 402 channels, one output 314 -> 201 / 652 -> 398 (2.1 / 4.2 TB/s); 256 x 256, 201: 92 -> 20.
+// above 128, us: 1024 x 1024, 101 channels, four labels 185 -> 123; 4 x 512 x 512, 101, one output 111 -> 90; 3 x 333 x 477, 35, three labels
+// 40 -> 31; 1024 x 1024, 201 / 402 channels, one output 329 -> 214 / 686 -> 454 (3.9 / 3.7 TB/s); 256 x 256, 201: 89 -> 21.
 constexpr int kTiledWaves = 8;
 constexpr int kTiledThreads = kTiledWaves * kWave;
 constexpr int kTiledMaxChannels = 512;

@@ -16,11 +16,12 @@
 // serves at 2.6-3.0 TB/s whatever else happens, whole lines at 4.0 (probed with loads and
 // stores alone, 64 channels of 1024 x 1024).  Five to eight blocks of two slabs, and three and four of one slab in large images: msd_pull_wide.h.
 //
-// Bound by the issue of instructions: a SIMD issues a conversion, shift or select of a wave in 4.3 cycles and a matrix instruction
-// in 16.2, beside which there is room for two of the former, and a wave issues one instruction of any kind in 4.2 cycles.  With eight waves that all gathered and
-// then all multiplied, the two kinds of work did not meet and half of the waves were idle over few blocks.  us (with sum_group), eight
-// waves -> three kinds: 61 x 93 x 75, four outputs over 5 channels 69 -> 59; 128^3, four over 14 / 30 / 46 277 / 357 / 480 -> 254 / 335 / 455; 3 x 333 x
-// 477, 14 outputs over 19 90 -> 82; 1024 x 1024, 14 over 15 / 45 151 / 263 -> 140 / 258.
+// Bound by waiting and issue together, not by one pipe.  Counters at 1024 x 1024, 14 outputs with 28 / 33 / 58 channels in the pass, and at 128^3, four with 17 / 33 / 49: the
+// matrix cores are busy 21 / 24 / 31 and 23 / 27 / 36 % of the time, vector instructions take 44 / 37 / 41 and 49 / 43 / 48 % of the SIMDs' cycles (at four
+// each), and waves spend 42 / 57 / 44 and 39 / 54 / 40 % of theirs waiting for loads, LDS and the barrier and 28 / 19 / 30 and 31 / 20 / 31 % for a turn to issue; eight waves that
+// all gathered and then all multiplied: matrix cores 19 / 26 / 30 and 21 / 26 / 32 %.  (Loads requested two and four units ahead, and gathered two tiles
+// ahead, change nothing.)  us, eight waves -> three kinds: 61 x 93 x 75, four outputs, 8 channels 62 -> 54; 128^3, four with 17 / 33 / 49 325 / 440 / 501 -> 299 / 426 /
+// 455; 3 x 333 x 477, 14 with 32 92 -> 82; 1024 x 1024, 14 with 17 / 28 / 33 / 58 167 / 169 / 220 / 263 -> 157 / 159 / 228 / 258.
 //
 // Tried on the way: waves that walk the channels on their own tile (weights in LDS, loads in the matrix layout): 650 us
 // over 95 channels, 320 over 45; two workgroups of four waves per compute unit: 604 and 293; for 5 to 8 blocks
@@ -1092,7 +1093,7 @@ hipError_t pull_launch(F *kernel, int threads, int lds, LargeLds &large, const P
     return hipGetLastError();
 }
 
-// Blocks of a chunk, at most (one slab: 411 us over 100 channels, 463 with 8).
+// Blocks of a chunk, at most (one slab, when all had eight waves: 411 us over 100 channels, 463 with 8).
 int most_blocks(int slabs) { return slabs == 1 ? 4 : 8; }
 // Blocks of a chunk of two slabs that pull_rows takes; pull_rows_wide the others, and three and four of one slab from so many segments of 32 voxels on,
 // for each 256 workgroups of the chunk.  There the eight waves of the latter are faster, which all gather a tile twice as large and then all multiply.  Backward pass of
@@ -1101,7 +1102,7 @@ int most_blocks(int slabs) { return slabs == 1 ? 4 : 8; }
 // layer of three outputs 724 x 724 0.96 / 0.95 / 0.96, 900 x 900 1.00 / 1.03 / 1.03, 2048 x 2048 1.09 / 1.12 / 1.10; of one in 3D 100^3 0.96 / 1.00 / 1.00,
 // 128^3 1.02 / 1.07 / 1.10.  Chunks side by side have fewer workgroups each (60 channels below seven outputs are five blocks, 3 + 2); over 64 / 70 / 100 / 130 512 x
 // 512 1.02 / 0.97 / 0.99 / 1.06, 680 x 700 1.03 / 1.02 / 1.03 / 1.00; 61 x 93 x 75 1.02 / 0.93 / 1.02 / 1.02, 80^3 1.10 / 1.08 / 1.03 / 1.03, 90^3 1.14 / 1.08 /
-// 1.00 / 1.00.  (Loads requested two and four units ahead, or gathered two tiles ahead, change nothing in pull_rows.)
+// 1.00 / 1.00.
 constexpr int kNarrowBlocks = 4, kNarrowOneSlab = 2;
 constexpr int64_t kWideImage = 20000, kWideVolume = 50000, kWideVolumeChunks = 25000;
 
@@ -1143,18 +1144,17 @@ int64_t pull_floats(const PullPlan &p, int slabs)
 
 // Channels of a launch: those of one full chunk (128; one slab: 64) where chunks in launches of their own, which use the whole chip one after the
 // other, take less than chunks of about one size side by side, else all of them.
-// Two slabs: a chunk of five to eight blocks takes nearly the same time however many of its waves have a block (2048 x 2048, 14 outputs: 1.46, 1.54,
-// 1.63, 1.61 ms over 5, 6, 7, 8), four 0.95, two 0.58 and one 0.44, so that full chunks and a small rest gain (9 blocks: 2.75 ms as 5 + 4,
-// 2.05 as 8 + 1), a rest of six or more only in large images.  Time of a group of 14 (four in 3D), side by side 1, over 9 / 10 / 13 / 14 / 16 / 17
-// blocks: 512 x 513 0.97 / 0.99 / 1.03 / 1.13 / 1.14 / 1.02; 724 x 724 0.91 / 0.94 / 1.00 / 1.08 / 1.08 / 0.97; 960 x 960 0.85 / 0.89 / 0.95 / 1.04 / 1.05 / 0.92; 1500 x 1021
-// 0.86 / 0.89 / 0.95 / 1.02 / 1.02 / 0.93; 64 x 66 x 65 over 9 / 10 / 11 / 13 0.94 / 0.93 / 1.01 / 1.03; 94^3 over 9 / 10 / 13 / 14 0.88 / 0.88 / 0.97 / 1.04; over 13 / 14 / 16 1448 x 1448
-// 0.94 / 0.99 / 1.00, 2048 x 2048 0.94 / 1.00 / 0.98, 128^3 over 13 / 14 0.96 / 1.01.
+// Two slabs: a chunk of five to eight blocks takes 1.36, 1.54, 1.66 and 1.79 ms (2048 x 2048, 14 outputs), three 0.85 and one or two 0.56, so that full
+// chunks and a small rest gain, a rest of six or more only in large images.  Time of a group of 14 (four in 3D) with all launches, side by side 1, over 9 / 10 / 13 / 14 / 16 / 17
+// blocks: 512 x 513 0.95 / 0.97 / 1.05 / 1.12 / 1.11 / 0.94; 724 x 724 0.93 / 0.92 / 1.01 / 1.07 / 1.06 / 0.92; 960 x 960 0.90 / 0.89 / 0.99 / 1.03 / 1.02 / 0.87; 1500 x 1021
+// 0.89 / 0.90 / 0.98 / 1.02 / 1.02 / 0.80; 64 x 66 x 65 over 9 / 10 / 11 / 13 0.91 / 0.91 / 0.86 / 1.02; 94^3 over 9 / 10 / 13 / 14 0.90 / 0.90 / 0.99 / 1.04; over 13 / 14 / 16 1448 x 1448
+// 0.97 / 1.03 / 1.02, 2048 x 2048 0.94 / 1.00 / 1.00, 128^3 over 13 / 14 0.96 / 1.01.
 // One slab: a chunk has at most four blocks, and its time goes with their number.  A launch per chunk gains where the chunks side by side would be of
 // unequal size, five blocks most of all (4 + 1 for 3 + 2), the others only where gradients are written.  Side by side 1, a layer of three outputs (two
-// in 3D) over 5 / 7 / 13 (unequal), 6 / 8 / 9 (equal) blocks: 512 x 513 1.06 / 1.13 / 1.34, 1.22 / 1.25 / 1.30; 724 x 724 0.98 / 1.07 / 1.13, 1.12 /
-// 1.14 / 1.16; 900 x 900 0.90 / 1.01 / 1.05; 1024 x 1024 0.84 / 0.94 / 0.95, 1.01 / 1.10 / 0.95; 128^3 0.81 / 0.88 / 0.88, 0.94 / 1.03 / 0.92; added to, a group
-// of seven (two in 3D) over 5 / 7 / 11, 6 / 8 / 12: 724 x 724 1.03 / 1.09 / 1.16, 1.11 / 1.11 / 1.16; 1024 x 1024 0.90 / 1.00 / 1.04, 1.05 / 1.06 / 1.04; over
-// 5 / 7 / 11 100^3 0.91 / 1.00 / 1.00, 128^3 0.85 / 0.95 / 0.98.
+// in 3D) over 5 / 7 / 13 (unequal), 6 / 8 / 9 (equal) blocks: 512 x 513 0.93 / 1.07 / 1.23, 1.11 / 1.22 / 1.21; 724 x 724 0.98 / 1.13 / 1.17, 1.10 /
+// 1.17 / 1.14; 900 x 900 0.89 / 1.01 / 1.04, 1.03 / 1.08 / 1.04; 1024 x 1024 0.80 / 0.92 / 0.93, 0.98 / 1.06 / 0.93; over 5 / 7, 6 / 9 80^3 0.92 / 1.09, 1.07 / 1.10, 128^3 0.78 / 0.91,
+// 0.95 / 0.92; added to, a group of seven (two in 3D) over 5 / 7 / 11, 6 / 8 / 12: 724 x 724 0.99 / 1.02 / 1.04, 1.05 / 1.03 / 1.05; 1024 x 1024 0.91 / 0.99 / 0.98, 1.02 / 1.07 / 1.04;
+// over 5 / 7 / 11 100^3 0.88 / 1.00 / 0.98, 128^3 0.86 / 0.96 / 0.94.
 // Segments of a pass whose chunks have launches of their own (32 voxels each):
 constexpr int64_t kAloneTenBlocks = 1 << 13, kAloneSmallRest = 14000, kAloneAnyRest = 1 << 16, kAloneOneSlab = 28000;
 int64_t pull_channels(int64_t batch, int64_t rows, const PullPlan &p, int64_t channels, int slabs, bool fresh)

@@ -20,7 +20,6 @@ constexpr int kWaves = 8;                         // of a workgroup; one workgro
 // LDS of a wave for a unit of voxels: 16 channels of x in three parts (the sums for grad_input take less)
 constexpr int unit_bytes(int voxels) { return 3 * 16 * (2 * voxels + 16); }
 
-// What a workgroup keeps in LDS besides A and the waves' own space.
 // What a workgroup of pull_rows_wide keeps in LDS besides A and the waves' own space.
 struct Source {                                   // an output's place in bytes: its dilation in slices, rows and voxels, its plane
     uint32_t slices, rows, voxels, plane;
