@@ -1095,16 +1095,20 @@ hipError_t pull_launch(F *kernel, int threads, int lds, LargeLds &large, const P
 
 // Blocks of a chunk, at most (one slab, when all had eight waves: 411 us over 100 channels, 463 with 8).
 int most_blocks(int slabs) { return slabs == 1 ? 4 : 8; }
-// Blocks of a chunk of two slabs that pull_rows takes; pull_rows_wide the others, and three and four of one slab from so many segments of 32 voxels on,
-// for each 256 workgroups of the chunk.  There the eight waves of the latter are faster, which all gather a tile twice as large and then all multiply.  Backward pass of
-// seven outputs (3D: two) with all launches, pull_rows to pull_rows_wide 1, over 40 / 48 / 60 channels below them: 724 x 724 0.95 / 0.94 / 1.09, 800 x 800 1.00 / 1.05 / 1.12,
-// 1024 x 1000 1.04 / 1.01 / 1.00, 2048 x 2048 1.13 / 1.05 / 1.05; 100^3 1.01 / 0.96 / 0.97, 113^3 1.02 / 0.95 / 1.02, 128^3 1.07 / 1.04 / 1.09; a
-// layer of three outputs 724 x 724 0.96 / 0.95 / 0.96, 900 x 900 1.00 / 1.03 / 1.03, 2048 x 2048 1.09 / 1.12 / 1.10; of one in 3D 100^3 0.96 / 1.00 / 1.00,
-// 128^3 1.02 / 1.07 / 1.10.  Chunks side by side have fewer workgroups each (60 channels below seven outputs are five blocks, 3 + 2); over 64 / 70 / 100 / 130 512 x
+// Blocks of a chunk of two slabs that pull_rows takes; pull_rows_wide the others, and three and four of one slab in large images.  There the eight waves of the
+// latter are faster, which all gather a tile twice as large and then all multiply.  Volumes, and images whose gradients are written: from so many values of x and of the outputs'
+// gradients on, which with grad_input fill 240 MB of the 256 MB cache, behind which the units of 32 voxels wait longer.  pull_rows to pull_rows_wide 1, a layer of one output: 80^3 over 60 / 64
+// channels (31.2, 33.3 million values) 0.95 / 1.13; 80 x 81 x 83 over 56 / 60 / 64 (30.7, 32.8, 35.0) 0.92 / 1.00 / 1.03; 90^3 over 41 / 48 (30.6, 35.7) 0.94 / 1.06; 90 x 100 x 101 over 33 / 36 / 41 /
+// 48 (30.9, 33.6, 38.2, 44.5) 0.95 / 1.02 / 1.07 / 1.15; 100^3 over 33 / 48 / 64 0.97 / 1.13 / 1.12; 108^3 1.01 / 1.18 / 1.15; two outputs 80^3 over 56 / 60 (29.7, 31.7) 0.96 / 1.08; three 512 x 513 over 64 (17.6) 0.86; 724 x
+// 724 over 56 / 64 (30.9, 35.1) 0.95 / 1.02; 700 x 801 over 52 / 56 / 60 (30.8, 33.1, 35.3) 1.00 / 1.02 / 1.05; two outputs, added to, 90^3 over 36 / 44 / 60 0.92 / 0.97 / 0.98; 90 x 100 x 101
+// 0.98 / 1.05 / 1.03; 113^3 1.00 / 1.03 / 1.01.
+// Other images: from so many segments of 32 voxels on, for each 256 workgroups of the chunk.  Seven outputs, added to, over 36 / 44 / 52 / 60 channels: 512 x 513 0.94 / 0.93 / 0.90 /
+// 0.89; 724 x 724 0.96 / 0.95 / 0.93 / 0.96; 700 x 801 0.99 / 0.98 / 0.95 / 0.97; over 40 / 48 / 60 below them 800 x 800 1.00 / 1.05 / 1.12, 1024 x 1000 1.04 / 1.01 / 1.00, 2048 x
+// 2048 1.13 / 1.05 / 1.05.  Chunks side by side have fewer workgroups each (60 channels below seven outputs are five blocks, 3 + 2); over 64 / 70 / 100 / 130 512 x
 // 512 1.02 / 0.97 / 0.99 / 1.06, 680 x 700 1.03 / 1.02 / 1.03 / 1.00; 61 x 93 x 75 1.02 / 0.93 / 1.02 / 1.02, 80^3 1.10 / 1.08 / 1.03 / 1.03, 90^3 1.14 / 1.08 /
 // 1.00 / 1.00.
 constexpr int kNarrowBlocks = 4, kNarrowOneSlab = 2;
-constexpr int64_t kWideImage = 20000, kWideVolume = 50000, kWideVolumeChunks = 25000;
+constexpr int64_t kWideImage = 20000, kWideValues = 30 << 20;
 
 // As many workgroups as are resident, shared out over the chunks by their size.
 struct PullPlan {
@@ -1113,7 +1117,7 @@ struct PullPlan {
     bool wide;                                    // pull_rows_wide
 };
 
-PullPlan pull_plan(int64_t batch, int64_t rows, int64_t span, int64_t channels, int slabs, bool volume)
+PullPlan pull_plan(int64_t batch, int64_t rows, int64_t span, int64_t channels, int slabs, bool volume = false, int outputs = 0)
 {
     PullPlan p;
     const int nb = (int)((channels + 15) / 16);
@@ -1123,8 +1127,8 @@ PullPlan pull_plan(int64_t batch, int64_t rows, int64_t span, int64_t channels, 
     c.blocks = (nb + c.n - 1) / c.n;
     c.large = nb - c.n * (c.blocks - 1);
     p.segs = (int)((span + kSegment - 1) / kSegment);
-    const int64_t wide_from = !volume ? kWideImage : c.n == 1 ? kWideVolume : kWideVolumeChunks;
-    p.wide = slabs == 1 ? c.blocks > kNarrowOneSlab && batch * rows * p.segs * nb >= wide_from * c.blocks : c.blocks > kNarrowBlocks;
+    const bool large = (outputs > 0 && batch * rows * span * (channels + outputs) >= kWideValues) || (!volume && batch * rows * p.segs * nb >= kWideImage * c.blocks);
+    p.wide = slabs == 1 ? c.blocks > kNarrowOneSlab && large : c.blocks > kNarrowBlocks;
     const int per_tile = (p.wide ? kWaves : kOfKind) / slabs;
     p.image_tiles = (int)((rows * p.segs + per_tile - 1) / per_tile);
     p.tiles = (int)batch * p.image_tiles;
@@ -1173,10 +1177,10 @@ int64_t pull_channels(int64_t batch, int64_t rows, const PullPlan &p, int64_t ch
 int64_t all_pull_floats(int64_t batch, int64_t rows, int64_t span, int64_t channels, int slabs)
 {
     // (either kernel has as many workgroups where it is chosen by the voxels: fewer than tiles)
-    const PullPlan p = pull_plan(batch, rows, span, channels, slabs, false);
+    const PullPlan p = pull_plan(batch, rows, span, channels, slabs);
     const int64_t step = pull_channels(batch, rows, p, channels, slabs, true), rest = channels % step;
-    int64_t most = std::max(pull_floats(p, slabs), pull_floats(pull_plan(batch, rows, span, step, slabs, false), slabs));
-    if (rest > 0) most = std::max(most, pull_floats(pull_plan(batch, rows, span, rest, slabs, false), slabs));
+    int64_t most = std::max(pull_floats(p, slabs), pull_floats(pull_plan(batch, rows, span, step, slabs), slabs));
+    if (rest > 0) most = std::max(most, pull_floats(pull_plan(batch, rows, span, rest, slabs), slabs));
     return most;
 }
 
@@ -1214,7 +1218,7 @@ hipError_t pull_part(const Geom &g, const View<const float> &x, const float *gy,
     const Form form = form_of(g, x);
     const int slabs = out.n > per_slab ? 2 : 1;
     const int span = form == kFlat ? g.nvox : g.W, rows = g.nvox / span;
-    const PullPlan p = pull_plan(g.B, rows, span, g.C, slabs, g.ndim == 3);
+    const PullPlan p = pull_plan(g.B, rows, span, g.C, slabs, g.ndim == 3, g.ndim == 3 || fresh ? out.n : 0);
     PullArgs a{g.C, update, mask_from, g.D, g.H, g.W, span, p.segs, rows * p.segs, p.tiles, p.image_tiles, Divisor((uint32_t)p.segs),
                Divisor((uint32_t)p.image_tiles), Divisor((uint32_t)g.H), Divisor((uint32_t)g.W), reverse, 0, p.chunks,
                x.sb, x.sc, x.sz, x.sy, gsb, gsc, out};
@@ -1282,7 +1286,7 @@ hipError_t pull(const Geom &g, const View<const float> &x, const float *gy, int6
         return hipErrorInvalidValue;
     const int slabs = out.n > per_slab ? 2 : 1, taps = g.ndim == 3 ? 27 : group2d::kTaps;
     const int span = form == kFlat ? g.nvox : g.W, rows = g.nvox / span;
-    const int step = (int)pull_channels(g.B, rows, pull_plan(g.B, rows, span, g.C, slabs, false), g.C, slabs, fresh);
+    const int step = (int)pull_channels(g.B, rows, pull_plan(g.B, rows, span, g.C, slabs), g.C, slabs, fresh);
     for (int from = 0; from < g.C; from += step) {
         Geom part = g;
         View<const float> xp = x;

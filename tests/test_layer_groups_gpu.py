@@ -187,15 +187,15 @@ def test_weight_gradients_over_many_voxels(size, c_in, outputs, workers):
     assert float((got - want).norm() / want.norm()) <= bound
 
 
-# One slab of outputs over three and four blocks: from 20000 segments of 32 voxels on (volumes 50000, 25000 with chunks side by side) for each 256
-# workgroups of a chunk the eight waves that gather and multiply in turn.  Just below and just above, rows that end inside a segment, rows with gaps, two images, a block without its last channels and
-# a chunk of two blocks beside one of three; against the layers on their own.
+# One slab of outputs over three and four blocks: images from 20000 segments of 32 voxels on for each 256 workgroups of a chunk, volumes from 30 x 2^20 values of
+# the channels and the outputs on, take the eight waves that gather and multiply in turn.  Just below and just above, rows that end inside a segment, rows with gaps, two images, a block without its
+# last channels and a chunk of two blocks beside one of three; against the layers on their own.
 @pytest.mark.parametrize("size, batch, c_in, gap, wide", [
     ((799, 800), 1, 40, 0, False), ((801, 799), 1, 40, 0, True), ((400, 830), 2, 62, 3, True), ((801, 800), 1, 75, 0, True),
     ((595, 640), 1, 75, 0, False), ((605, 640), 1, 75, 0, True), ((400, 520), 1, 130, 0, True),
-    ((78, 76, 80), 1, 70, 0, False), ((80, 77, 80), 1, 70, 0, True), ((80, 100, 60), 1, 65, 1, True),
-    ((801, 798), 1, 31, 0, False), ((100, 160, 99), 1, 47, 0, False), ((100, 161, 101), 1, 47, 0, True), ((100, 125, 99), 1, 33, 1, True),
-    ((50, 124, 100), 2, 33, 1, False)], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+    ((70, 76, 80), 1, 70, 0, False), ((72, 76, 80), 1, 70, 0, True), ((80, 100, 60), 1, 65, 1, True),
+    ((801, 798), 1, 31, 0, False), ((63, 100, 99), 1, 47, 0, False), ((64, 100, 99), 1, 47, 0, True), ((70, 125, 99), 1, 33, 1, False), ((100, 125, 99), 1, 33, 1, True),
+    ((35, 124, 100), 2, 33, 1, False), ((36, 124, 100), 2, 33, 1, True)], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_one_slab_over_three_and_four_blocks(size, batch, c_in, gap, wide):
     from msd_pytorch_amd import msd_custom_convolutions as cc
     gen = torch.Generator(device="cuda").manual_seed(89)
@@ -215,6 +215,33 @@ def test_one_slab_over_three_and_four_blocks(size, batch, c_in, gap, wide):
     assert len(passes) == 1 and ("pull_rows_wide" in passes[0]) == wide
     found = [run(setting) for setting in (0, 1)]
     for a, b in zip(*found):
+        assert rel_err(b, a) <= 1e-5
+
+
+# The same of a layer of its own, whose gradients are written: by the values in images too.
+@pytest.mark.parametrize("size, batch, c_in, outputs, wide", [
+    ((660, 801), 1, 56, 3, False), ((672, 801), 1, 56, 3, True), ((300, 396), 4, 63, 3, False), ((300, 398), 4, 63, 3, True),
+    ((77, 100, 99), 1, 40, 1, False), ((78, 100, 99), 1, 40, 1, True), ((58, 101, 80), 1, 64, 2, False), ((61, 101, 80), 1, 64, 2, True), ((25, 99, 181), 2, 33, 2, False),
+    ((25, 99, 182), 2, 33, 2, True)],
+    ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_a_layer_over_three_and_four_blocks(size, batch, c_in, outputs, wide):
+    from msd_pytorch_amd import conv2d, conv3d
+    gen = torch.Generator(device="cuda").manual_seed(101)
+    fn = conv2d.conv2d_relu if len(size) == 2 else conv3d.conv3d_relu
+    x = torch.randn(batch, c_in, *size, device="cuda", generator=gen).requires_grad_()
+    w = (torch.randn(outputs, c_in, *[3] * len(size), device="cuda", generator=gen) * 0.1).requires_grad_()
+    b = torch.zeros(outputs, device="cuda").requires_grad_()
+    g = torch.randn(batch, outputs, *size, device="cuda", generator=gen)
+
+    def run(x, w, b, *leaves):
+        y = fn(x, w, b, torch.empty(batch, outputs, *size, device="cuda"), 1, 3)
+        return torch.autograd.grad(y, leaves, g)
+
+    found = run(x, w, b, x, w, b)
+    torch.cuda.synchronize()
+    passes = [name for name, _ in captured_kernels(lambda: run(x, w, b, x, w, b)) if "pull_rows" in name]
+    assert len(passes) == 1 and ("pull_rows_wide" in passes[0]) == wide
+    for a, b in zip(run(x, w.detach(), b.detach(), x) + run(x.detach(), w, b, w, b), found):       # (one gradient at a time: the operators of their own)
         assert rel_err(b, a) <= 1e-5
 
 
